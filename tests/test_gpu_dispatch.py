@@ -1,0 +1,111 @@
+"""The native dispatch (csrc/host/snnf_dispatch.cpp): a call of a known signature returns bit for bit what the first call (the
+Python implementation) returned, counts the same statistics, follows in-place weight updates and replaced weight tensors, and
+calls it does not take (strided inputs, another backend) still run."""
+import pytest
+import torch
+
+from helpers import DEV, gen, q
+
+pytestmark = pytest.mark.gpu
+LIF = (1.0, 0.0, 2.0, False)
+
+
+def _operands(dtype, seed=3):
+    g = gen(seed)
+    spikes = lambda *s: (torch.rand(*s, generator=g) < 0.3).to(DEV, dtype)
+    weights = lambda *s: q(torch.randn(*s, generator=g) * 0.4, dtype).to(DEV, dtype)
+    return g, spikes, weights
+
+
+def _calls(dtype, zero):
+    """name -> (call, weight) of every operator that the native dispatch implements, smallest shapes with a remainder."""
+    S = torch.ops.snn_custom
+    g, spikes, weights = _operands(dtype)
+    xs = [spikes(2, 24, 7, 9) for _ in range(4)]
+    rs = [spikes(2, 40, 7, 9) for _ in range(4)]
+    seq = torch.randn(4, 2, 24, 7, 9, generator=g).to(DEV, dtype)
+    rows = spikes(4, 5, 40)
+    w3, w1, wd, b40, b24 = weights(40, 24, 3, 3), weights(40, 24, 1, 1), weights(24, 1, 3, 3), weights(40), weights(24)
+    wl, bl, wt, bt = weights(33, 40), weights(33), weights(11, 24), weights(11)
+    same, one = ([1, 1], [1, 1], [1, 1]), ([1, 1], [0, 0], [1, 1])
+    v1 = torch.rand(2, 24, 7, 9, generator=g).to(DEV, dtype)
+    return {
+        "lif_forward_state": (lambda: S.lif_forward_state(xs[0], v1, *LIF), None),
+        "fused_conv_lif_state": (lambda: S.fused_conv_lif_state(xs[0], w3, b40, zero, *same, 1, *LIF), w3),
+        "fused_temporal_conv_lif_state": (lambda: S.fused_temporal_conv_lif_state(xs, w3, b40, zero, *same, 1, *LIF), w3),
+        "fused_temporal_pointwise_conv_lif_state": (lambda: S.fused_temporal_pointwise_conv_lif_state(xs, w1, b40, zero, *one, 1, *LIF), w1),
+        "fused_temporal_depthwise_conv_lif_state": (lambda: S.fused_temporal_depthwise_conv_lif_state(xs, wd, b24, zero, *same, 24, *LIF), wd),
+        "fused_temporal_conv_add_lif_state": (lambda: S.fused_temporal_conv_add_lif_state(xs, rs, w3, b40, zero, *same, 1, *LIF), w3),
+        "fused_temporal_lif_state": (lambda: S.fused_temporal_lif_state(seq, zero, *LIF), None),
+        "fused_temporal_lif_avgpool_linear": (lambda: S.fused_temporal_lif_avgpool_linear(seq, zero, wt, bt, *LIF), wt),
+        "fused_temporal_linear_lif_state": (lambda: S.fused_temporal_linear_lif_state(list(rows.unbind(0)), wl, bl, zero, *LIF), wl),
+        "fused_temporal_linear_lif_state_packed": (lambda: S.fused_temporal_linear_lif_state_packed(rows, wl, None, zero, *LIF), wl),
+    }
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("host_state", [False, True])
+def test_known_signature_equals_first_call(hip_ops, dtype, host_state):
+    from triton_snn_fusion_amd import _dispatch
+    zero = torch.zeros(()) if host_state else torch.zeros((), device=DEV)
+    native = _dispatch.module()
+    for name, (call, weight) in _calls(dtype, zero).items():
+        native.forget_plans()
+        hip_ops.reset_fused_op_call_stats()
+        first = call()
+        once = hip_ops.get_fused_op_call_stats()
+        before = sum(native.hits())
+        again = [call() for _ in range(2)]
+        assert name == "lif_forward_state" or sum(native.hits()) == before + 2, name      # ran natively
+        for out in again:
+            assert all(torch.equal(a, b) and a.dtype == b.dtype for a, b in zip(out, first)), name
+        three = hip_ops.get_fused_op_call_stats()
+        assert three["total"] == 3 * once["total"] and three["triton"] == 3 * once["triton"] and three["fallback"] == 0, name
+        for key in ("kernel_temporal_configs", "temporal_conv_lif_runtime_by_signature"):
+            assert set(three[key]) == set(once[key]), name
+        assert three["kernel_temporal_configs"] == {k: 3 * n for k, n in once["kernel_temporal_configs"].items()}, name
+        if weight is not None:                              # an update in place is seen by the next call
+            weight.mul_(-1.0)
+            flipped = call()
+            hip_ops.configure_fused_op("hip", strict_triton=True, verbose=True)      # the Python implementation
+            expected = call()
+            hip_ops.configure_fused_op("hip", strict_triton=True)
+            assert all(torch.equal(a, b) for a, b in zip(flipped, expected)), name
+
+
+def test_calls_off_the_fast_path(hip_ops):
+    """Strided inputs of a signature that is known contiguous, a tensor state, and the eager backend."""
+    _, spikes, weights = _operands(torch.bfloat16)
+    S = torch.ops.snn_custom
+    zero = torch.zeros((), device=DEV)
+    xs = [spikes(2, 24, 7, 9) for _ in range(3)]
+    w, b = weights(40, 24, 3, 3), weights(40)
+    args = (w, b, zero, [1, 1], [1, 1], [1, 1], 1, *LIF)
+    ref = S.fused_temporal_conv_lif_state(xs, *args)
+    S.fused_temporal_conv_lif_state(xs, *args)
+    strided = [x.permute(0, 1, 3, 2).contiguous().permute(0, 1, 3, 2) for x in xs]
+    out = S.fused_temporal_conv_lif_state(strided, *args)
+    assert all(torch.equal(a, c) for a, c in zip(out, ref))
+    two = S.fused_temporal_conv_lif_state(xs[:2], *args)
+    rest = [S.fused_temporal_conv_lif_state(xs[2:], w, b, two[1], [1, 1], [1, 1], [1, 1], 1, *LIF) for _ in range(2)]
+    assert all(torch.equal(a, c) for a, c in zip(rest[0], rest[1]))
+    assert torch.equal(rest[0][0][0], ref[0][2]) and torch.equal(rest[0][1], ref[1])
+    hip_ops.configure_fused_op("torch")
+    eager = S.fused_temporal_conv_lif_state(xs, *args)
+    assert hip_ops.get_fused_op_call_stats()["fallback"] == 1
+    assert float((eager[0] != ref[0]).float().mean()) < 1e-2
+
+
+def test_weights_of_dead_tensors_are_given_back(hip_ops):
+    _, spikes, weights = _operands(torch.bfloat16)
+    S = torch.ops.snn_custom
+    zero = torch.zeros((), device=DEV)
+    xs = [spikes(1, 8, 5, 5)]
+    outs = []
+    for i in range(4):                                      # the allocator hands a dead weight's address to the next one
+        w, b = weights(16, 8, 3, 3), weights(16)
+        outs.append(S.fused_temporal_conv_lif_state(xs, w, b, zero, [1, 1], [1, 1], [1, 1], 1, *LIF)[1])
+        ref = torch.nn.functional.conv2d(xs[0].float(), w.float(), b.float(), padding=1) / 2
+        fired = ref >= 1.0
+        assert float((outs[-1] - torch.where(fired, torch.zeros_like(ref), ref)).abs().max()) < 1e-4   # bf16 products are exact, 73 of them added in float32: 73 * 2^-24 * |sum| < 1e-4
+        del w, b

@@ -80,7 +80,8 @@ class SnnfError(RuntimeError):
 
 
 def library_available() -> bool:
-    return LIB_PATH.exists()
+    """Both halves of the native build: the kernels and the dispatch module in front of them."""
+    return LIB_PATH.exists() and (LIB_PATH.parent / "_snnf_dispatch.so").exists()
 
 
 def lib() -> ctypes.CDLL:

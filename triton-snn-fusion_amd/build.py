@@ -3,7 +3,8 @@
     python triton-snn-fusion_amd/build.py [--jobs N] [--keep-objects]
 
 hipcc cross-compiles gfx950 code objects without a GPU, so this runs on any host that has ROCm installed. The shared
-library is written to triton-snn-fusion_amd/lib/libsnnf.so, next to the Python modules that load it through ctypes.
+library is written to triton-snn-fusion_amd/lib/libsnnf.so, next to the Python modules that load it through ctypes; the
+host-side dispatch module (csrc/host/snnf_dispatch.cpp, g++ against PyTorch's headers) to lib/_snnf_dispatch.so.
 """
 from __future__ import annotations
 
@@ -23,6 +24,8 @@ INCLUDE_DIR = REPO_ROOT / "include"
 LIB_DIR = PKG_DIR / "lib"
 OBJ_DIR = CSRC_DIR / "_obj"
 LIB_PATH = LIB_DIR / "libsnnf.so"
+DISPATCH_SOURCE = CSRC_DIR / "host" / "snnf_dispatch.cpp"
+DISPATCH_PATH = LIB_DIR / "_snnf_dispatch.so"
 
 OFFLOAD_ARCH = "gfx950"
 
@@ -88,8 +91,30 @@ def _compile_one(hipcc: str, src: Path):
     return obj, len(allowed), unexpected
 
 
+def build_dispatch(verbose: bool = True) -> Path:
+    """Compiles the host-side dispatch module (plain C++ against PyTorch's headers, no GPU code) and links it to libsnnf.so."""
+    import sysconfig
+    import torch
+    root = Path(torch.__file__).resolve().parent
+    tmp = DISPATCH_PATH.with_suffix(".so.tmp")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-unused-function", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           "-DTORCH_EXTENSION_NAME=_snnf_dispatch", "-DTORCH_API_INCLUDE_EXTENSION_H", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-I{INCLUDE_DIR}"]
+    for include in (root / "include", root / "include" / "torch" / "csrc" / "api" / "include", Path("/opt/rocm/include"), Path(sysconfig.get_paths()["include"])):
+        cmd += ["-isystem", str(include)]
+    cmd += [str(DISPATCH_SOURCE), "-o", str(tmp), f"-L{root / 'lib'}", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-ltorch_python",
+            f"-L{LIB_DIR}", "-lsnnf", "-Wl,-rpath,$ORIGIN"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"dispatch module failed to build:\n{' '.join(cmd)}\n{proc.stdout}\n{proc.stderr}")
+    os.replace(tmp, DISPATCH_PATH)
+    if verbose:
+        print(f"[build] wrote {DISPATCH_PATH} ({DISPATCH_PATH.stat().st_size} bytes)", flush=True)
+    return DISPATCH_PATH
+
+
 def build_library(jobs: int = 4, keep_objects: bool = False, verbose: bool = True, allow_new_warnings: bool = False) -> Path:
-    """Compiles every csrc/*.hip for gfx950 and links lib/libsnnf.so. Always recompiles."""
+    """Compiles every csrc/*.hip for gfx950 and links lib/libsnnf.so, then the dispatch module on top of it. Always recompiles."""
     hipcc = _hipcc()
     OBJ_DIR.mkdir(parents=True, exist_ok=True)
     LIB_DIR.mkdir(parents=True, exist_ok=True)
@@ -117,6 +142,7 @@ def build_library(jobs: int = 4, keep_objects: bool = False, verbose: bool = Tru
         shutil.rmtree(OBJ_DIR, ignore_errors=True)
     if verbose:
         print(f"[build] wrote {LIB_PATH} ({LIB_PATH.stat().st_size} bytes)", flush=True)
+    build_dispatch(verbose=verbose)
     return LIB_PATH
 
 

@@ -36,7 +36,9 @@ import torch.fx as fx
 import torch.nn as nn
 import torch.nn.functional as F
 
-from .runtime.hip_pool_backend import pool_config
+from .runtime import hip_blocked_backend as B
+from .runtime.hip_convlif_backend import run_hip_conv_bias_frames
+from .runtime.hip_pool_backend import pool_config, run_hip_pool2d
 from .workloads import fold_bn_into_conv_params
 
 
@@ -601,7 +603,6 @@ def rewrite_temporal_to_fused(gm: fx.GraphModule, stats: Optional[RewriteStats] 
 def pooled_frames(x_seq: torch.Tensor, is_max: bool, kernel: int, stride: int, padding: int) -> torch.Tensor:
     """Pooling of a [T, N, C, H, W] sequence: the HIP pooling kernel on the GPU, the framework's pooling on CPU tensors."""
     if x_seq.is_cuda:
-        from .runtime.hip_pool_backend import run_hip_pool2d
         return run_hip_pool2d(x_seq, is_max, kernel, stride, padding)
     flat = x_seq.flatten(0, 1)
     y = F.max_pool2d(flat, kernel, stride, padding) if is_max else F.avg_pool2d(flat, kernel, stride, padding)
@@ -612,9 +613,8 @@ def conv_bias_frames(x_seq: torch.Tensor, weight: torch.Tensor, bias: torch.Tens
     """LIF-free convolution + folded BatchNorm of a [T, N, C, H, W] sequence: the matrix kernel's neuron-free mode where
     it takes the layer, the framework's convolution otherwise."""
     if x_seq.is_cuda:
-        from .runtime.hip_convlif_backend import run_hip_temporal_conv_bias
         try:
-            return run_hip_temporal_conv_bias(list(x_seq.unbind(0)), weight, bias, stride, padding)
+            return run_hip_conv_bias_frames(x_seq, weight, bias, stride, padding)
         except RuntimeError as exc:
             if "unsupported" not in str(exc):
                 raise
@@ -749,7 +749,6 @@ def blocked_input(frames, T: int, shared: bool, spikes: bool = False):
     """Graph input side: one analog frame [N, C, H, W] shared by all T steps (read as it is when it has at most 8 channels),
     or a dense [T, N, C, H, W] tensor (or the list of its T steps), into the channel-blocked layout; `spikes`: the tensor is
     the spike output of a fused operator (zeros and ones) and goes into the bit-packed layout."""
-    from .runtime import hip_blocked_backend as B
     if shared:
         return B.input_frame(frames, T)
     if isinstance(frames, (list, tuple)):
@@ -760,7 +759,6 @@ def blocked_input(frames, T: int, shared: bool, spikes: bool = False):
 def blocked_residual(frames):
     """A dense [T, N, C, H, W] tensor (or the list of its steps) as a residual operand: no conversion, the kernel reads
     dense residuals as they are."""
-    from .runtime import hip_blocked_backend as B
     if isinstance(frames, (list, tuple)):
         frames = torch.stack(list(frames))
     return B.from_dense(frames, B.NCHW)
@@ -768,7 +766,6 @@ def blocked_residual(frames):
 
 def blocked_conv_lif(x, weight, bias, stride, padding, lif, residual, out_layout: int):
     """Conv + folded BN (+ residual) + LIF over the T steps of a `Blocked` value, or without a neuron when `lif` is None."""
-    from .runtime import hip_blocked_backend as B
     out, _ = B.conv_lif_blocked_or_dense(x, weight, bias, stride, padding, lif, residual=residual, out_layout=out_layout)
     return out
 
@@ -776,7 +773,6 @@ def blocked_conv_lif(x, weight, bias, stride, padding, lif, residual, out_layout
 def blocked_conv_lif_shortcut(x, weight, bias, padding, lif, shortcut_x, shortcut_weight, shortcut_bias, shortcut_stride, out_layout: int):
     """The second convolution of a residual block with the block's 1x1 projection shortcut accumulated in the same launch
     (LIF(conv(x) + conv1x1(shortcut_x))); the two convolutions one after the other where the kernel does not take the pair."""
-    from .runtime import hip_blocked_backend as B
     try:
         out, _ = B.conv_lif_blocked_shortcut(x, weight, bias, padding, shortcut_x, shortcut_weight, shortcut_bias, shortcut_stride, lif,
                                              out_layout=out_layout)
@@ -792,7 +788,6 @@ def blocked_conv_lif_shortcut(x, weight, bias, padding, lif, shortcut_x, shortcu
 def blocked_conv_lif_avgpool(x, weight, bias, stride, padding, lif):
     """Conv + folded BN + LIF and the 2x2 / 2 average pool of its spikes in one launch; the two one after the other where the
     kernel does not take the layer in that form."""
-    from .runtime import hip_blocked_backend as B
     try:
         out, _ = B.conv_lif_blocked_avgpool(x, weight, bias, stride, padding, lif)
         return out
@@ -806,7 +801,6 @@ def blocked_conv_lif_pool_linear(x, weight, bias, stride, padding, lif, residual
     """The network's last convolution with the tail's neuron in its epilogue (bit-packed spikes out), then average pool and
     classifier on those spikes, summed over T and scaled (1 / T: the mean over the timesteps): [N, K]. Where a kernel does
     not take the layer in this form, the convolution writes its sums dense and the LIF -> pool -> Linear operator follows."""
-    from .runtime import hip_blocked_backend as B
     try:
         spikes, _ = B.conv_lif_blocked(x, weight, bias, stride, padding, lif, residual=residual, out_layout=B.BITS)
         return B.spike_pool_linear(spikes, fc_weight, fc_bias, scale)
@@ -820,7 +814,6 @@ def blocked_conv_lif_pool_linear(x, weight, bias, stride, padding, lif, residual
 
 
 def blocked_pool(x, is_max: bool, kernel: int, stride: int, padding: int):
-    from .runtime import hip_blocked_backend as B
     try:
         return B.pool_blocked(x, is_max, kernel, stride, padding)
     except RuntimeError as exc:
@@ -831,7 +824,6 @@ def blocked_pool(x, is_max: bool, kernel: int, stride: int, padding: int):
 
 
 def blocked_to_dense(x):
-    from .runtime import hip_blocked_backend as B
     return B.to_dense(x)
 
 
@@ -860,7 +852,6 @@ def propagate_internal_layouts(gm: fx.GraphModule) -> int:
     it is a fused (residual) convolution from the scalar-zero membrane with nobody reading its final membrane, a
     `conv_bias_frames` / `pooled_frames` call, or the sum of a LIF-free convolution and a stack (folded into that
     convolution as its residual); everything else keeps reading dense tensors, converted once where needed."""
-    from .runtime import hip_blocked_backend as B
     S = torch.ops.snn_custom
     conv_ops = {S.fused_temporal_conv_lif_state: False, S.fused_temporal_conv_lif_state.default: False,
                 S.fused_temporal_conv_add_lif_state: True, S.fused_temporal_conv_add_lif_state.default: True}

@@ -22,7 +22,7 @@ from typing import Dict, Optional, Sequence, Tuple
 
 import torch
 
-from .. import _lib
+from .. import _dispatch, _lib
 from .hip_convlif_backend import _as_pair, _packed_weight
 from .hip_convlif_backend import last_conv_plan as _library_conv_plan
 
@@ -30,7 +30,12 @@ NCHW, C8, BITS = _lib.SNNF_LAYOUT_NCHW, _lib.SNNF_LAYOUT_C8, _lib.SNNF_LAYOUT_BI
 LAYOUT_NAMES = {NCHW: "nchw", C8: "c8", BITS: "bits"}
 
 
-@dataclass
+# Calls whose signature has been seen run from the native dispatch module (csrc/host/snnf_dispatch.cpp): an entry point hands it
+# the call first, runs the call itself when it is not known, and then hands it over once more with what it learnt (these bits).
+_ROUTE_PLANE, _ALLOCATE_V, _RETURN_V = 1, 2, 4
+
+
+@dataclass(slots=True)
 class Blocked:
     """T x N frames of [C, H, W] in one of the layouts. `data` is [T, N, C, H, W] (NCHW), [T, N, C8, H, W, 8] (C8) in the
     activation dtype, or [T, N, C8, H, W] uint8 (BITS). `shared`: every timestep is the same frame (data holds one)."""
@@ -111,10 +116,15 @@ def to_dense(x: Blocked) -> torch.Tensor:
 def pool_blocked(x: Blocked, is_max: bool, kernel: int, stride: int, padding: int, out_layout: Optional[int] = None) -> Blocked:
     """Max (2x2 or 3x3, stride 2) or average (2x2 / 2) pooling of every frame. Max pooling keeps the layout (BITS: a bitwise
     OR); average pooling of BITS yields C8 (quarters)."""
-    if x.layout == NCHW:
-        raise RuntimeError("unsupported_layout: pool_blocked takes C8 or BITS tensors (dense ones go to snnf_pool2d)")
     if out_layout is None:
         out_layout = x.layout if is_max else C8
+    native = _dispatch.module()
+    call = (x.data, x.layout, x.shared, x.T, x.N, x.C, x.H, x.W, x.dtype, kernel, stride, padding, is_max, out_layout)
+    known = native.blocked_pool(*call, -1)
+    if known is not None:
+        return Blocked(known[0], out_layout, x.T, x.N, x.C, known[2], known[3], x.dtype, x.shared)
+    if x.layout == NCHW:
+        raise RuntimeError("unsupported_layout: pool_blocked takes C8 or BITS tensors (dense ones go to snnf_pool2d)")
     ho = (x.H + 2 * padding - kernel) // stride + 1
     wo = (x.W + 2 * padding - kernel) // stride + 1
     frames_t = int(x.data.shape[0])
@@ -123,6 +133,7 @@ def pool_blocked(x: Blocked, is_max: bool, kernel: int, stride: int, padding: in
     _lib.check("snnf_pool2d_blocked", _lib.lib().snnf_pool2d_blocked(
         x.data.data_ptr(), x.layout, out.data.data_ptr(), out_layout, frames_t * x.N, x.C, x.H, x.W, int(kernel), int(stride),
         int(padding), 1 if is_max else 0, _lib.dtype_code(x.dtype), _lib.current_stream(x.data.device)))
+    native.blocked_pool(*call, 0)
     return out
 
 
@@ -198,14 +209,19 @@ def input_frame(frame: torch.Tensor, T: int) -> Blocked:
 # BITS frame its bits, so the frames are the matrix rows as they lie in memory.
 # ---------------------------------------------------------------------------------------------------------------
 _PLANE_MATRIX_CACHE: "OrderedDict" = OrderedDict()
-_LAST_PLANE_MATRIX: Optional[Dict] = None      # set by the most recent convolution of this module when it ran as a matrix product
+_LAST_PLANE_MATRIX: Optional[tuple] = None      # set by the most recent convolution of this module when it ran as a matrix product
 
 
 def last_conv_plan() -> Dict:
     """What ran the most recent convolution launched through this module: the library planner's answer (kernel family,
     tile, waves, ...: hip_convlif_backend.last_conv_plan), or {"kernel": "plane_matrix", ...} for a layer on a plane of a few
     pixels that went through the Linear + LIF kernel."""
-    return dict(_LAST_PLANE_MATRIX) if _LAST_PLANE_MATRIX is not None else _library_conv_plan()
+    if _LAST_PLANE_MATRIX is None:
+        return _library_conv_plan()
+    window, rows, fin, fout, bits_in = _LAST_PLANE_MATRIX
+    return {"kernel": "plane_matrix", "window": window, "rows": rows, "features_in": fin, "features_out": fout, "x": "bits" if bits_in else "c8"}
+
+
 _PLANE_MATRIX_LIMIT = 16
 PLANE_MATRIX_MAX_PIXELS = 4
 PLANE_MATRIX_MAX_ELEMENTS = 4096 * 4096
@@ -263,8 +279,7 @@ def _conv_lif_plane_matrix(x: Blocked, weight: torch.Tensor, bias: torch.Tensor,
     matrix, bias_row = _plane_matrix(weight, bias, x.H, x.W, ph, pw)
     out = empty_blocked(BITS, x.T, x.N, cout, x.H, x.W, x.dtype, x.data.device)
     bits_in = x.layout == BITS
-    _LAST_PLANE_MATRIX = {"kernel": "plane_matrix", "window": x.T, "rows": x.N, "features_in": fin, "features_out": fout,
-                          "x": "bits" if bits_in else "c8"}
+    _LAST_PLANE_MATRIX = (x.T, x.N, fin, fout, bits_in)
     lib = _lib.lib()
     workspace = _split_workspace(lib, x.data.device, x.T, x.N, fin, fout)
     _lib.check("snnf_linear_lif_bits", lib.snnf_linear_lif_bits(
@@ -280,6 +295,19 @@ def conv_lif_blocked(x: Blocked, weight: torch.Tensor, bias: Optional[torch.Tens
     """Dense convolution + bias (+ residual) + LIF over the T steps of `x` (C8 or BITS), or without a neuron when `lif` is
     None (output C8 or NCHW). Returns (Blocked output, final membrane [N, Cout, Ho, Wo] fp32 or None). The membrane is
     only written when asked for (`want_v`) or when the timesteps take more than one window of the kernel."""
+    call = None
+    r = residual
+    if v_init is None and bias is not None and (r is None or (r.dtype == x.dtype and not r.shared)):
+        native = _dispatch.module()
+        call = (x.data, x.layout, x.shared, x.T, x.N, x.C, x.H, x.W, x.dtype, weight, bias, stride, padding, lif,
+                *((None, 0, 0, 0, 0) if r is None else (r.data, r.layout, r.C, r.H, r.W)), out_layout, want_v)
+        known = native.blocked_conv(*call, -1)
+        if known is not None:
+            global _LAST_PLANE_MATRIX
+            data, cout, ho, wo, route, v = known
+            plane = x.H * x.W
+            _LAST_PLANE_MATRIX = (x.T, x.N, x.C * plane, cout * plane, x.layout == BITS) if route & _ROUTE_PLANE else None
+            return Blocked(data, out_layout, x.T, x.N, cout, ho, wo, x.dtype), v
     if x.layout not in (C8, BITS) and not _is_input_frame(x):
         raise RuntimeError("unsupported_layout: conv_lif_blocked takes inputs in C8 or BITS layout (or one dense frame of at most 8 channels)")
     if weight.dim() != 4 or int(weight.shape[1]) != x.C:
@@ -294,7 +322,10 @@ def conv_lif_blocked(x: Blocked, weight: torch.Tensor, bias: Optional[torch.Tens
     if bias is None:
         bias = torch.zeros(cout, dtype=weight.dtype, device=weight.device)
     if _runs_as_plane_matrix(x, cout, kh, kw, sh, sw, ph, pw, lif, residual, out_layout, v_init, want_v):
-        return _conv_lif_plane_matrix(x, weight, bias, ph, pw, lif), None
+        out = _conv_lif_plane_matrix(x, weight, bias, ph, pw, lif)
+        if call is not None:
+            native.blocked_conv(*call, _ROUTE_PLANE)
+        return out, None
     if _TUNED is None:
         load_tuned_plans()
     _forget_plane_matrix()
@@ -323,10 +354,14 @@ def conv_lif_blocked(x: Blocked, weight: torch.Tensor, bias: Optional[torch.Tens
             _lib.ptr(v_buffer), 1 if neuron else 0, v_th, v_reset, tau, _lib.current_stream(dev))
 
     status = launch(v_out)
+    learnt = 0 if v_out is None else _ALLOCATE_V | _RETURN_V
     if status != 0 and neuron and v_out is None and b"v_out is required" in _lib.lib().snnf_last_error():
         _NEEDS_MEMBRANE_BUFFER.add(layer)            # refused before anything was enqueued
         status = launch(torch.empty((x.N, cout, ho, wo), dtype=torch.float32, device=dev))
+        learnt = _ALLOCATE_V
     _lib.check("snnf_conv_lif_blocked", status)
+    if call is not None:
+        native.blocked_conv(*call, learnt)
     return out, v_out
 
 
@@ -339,6 +374,16 @@ def conv_lif_blocked_shortcut(x: Blocked, weight: torch.Tensor, bias: Optional[t
     Raises RuntimeError("unsupported_shortcut: ...") for layers the kernel does not take in this form (the caller then
     runs the shortcut as a convolution of its own and hands its output to conv_lif_blocked as the residual).
     Returns (Blocked output, final membrane or None)."""
+    call = None
+    if bias is not None and shortcut_bias is not None and shortcut_x.dtype == x.dtype:
+        native = _dispatch.module()
+        s = shortcut_x
+        call = (x.data, x.layout, x.shared, x.T, x.N, x.C, x.H, x.W, x.dtype, weight, bias, padding, lif,
+                s.data, s.layout, s.shared, s.T, s.N, s.C, s.H, s.W, shortcut_weight, shortcut_bias, shortcut_stride, out_layout, want_v)
+        known = native.blocked_shortcut(*call, -1)
+        if known is not None:
+            _forget_plane_matrix()
+            return Blocked(known[0], out_layout, x.T, x.N, known[1], x.H, x.W, x.dtype), known[5]
     if x.layout != BITS or shortcut_x.layout != BITS:
         raise RuntimeError("unsupported_shortcut: both inputs must be bit-packed")
     if weight.dim() != 4 or shortcut_weight.dim() != 4 or int(weight.shape[1]) != x.C or int(shortcut_weight.shape[1]) != shortcut_x.C or \
@@ -369,6 +414,8 @@ def conv_lif_blocked_shortcut(x: Blocked, weight: torch.Tensor, bias: Optional[t
         x.step_pointers(), shortcut_x.step_pointers(), x.T, x.N, x.C, x.H, x.W, _lib.dtype_code(x.dtype), packed.data_ptr(), cout, kh, kw,
         ph, pw, shortcut_x.C, shortcut_x.H, shortcut_x.W, ssh, ssw, packed_sc.data_ptr(), None, out.data.data_ptr(), out_layout,
         out.step_stride_bytes(), _lib.ptr(v_out), 1 if neuron else 0, v_th, v_reset, tau, _lib.current_stream(dev)))
+    if call is not None:
+        native.blocked_shortcut(*call, 0 if v_out is None else _ALLOCATE_V | _RETURN_V)
     return out, v_out
 
 
@@ -379,6 +426,14 @@ def conv_lif_blocked_avgpool(x: Blocked, weight: torch.Tensor, bias: Optional[to
     `pool_blocked(conv_lif_blocked(...), False, 2, 2, 0)` without the spikes ever being stored (bit for bit where both launches
     share K among waves in the same way; this form plans patches of even extents, which can change the summation order). Raises
     RuntimeError("unsupported_pool: ...") where the kernel does not take the layer in this form."""
+    call = None
+    if bias is not None:
+        native = _dispatch.module()
+        call = (x.data, x.layout, x.shared, x.T, x.N, x.C, x.H, x.W, x.dtype, weight, bias, stride, padding, lif, want_v)
+        known = native.blocked_avgpool(*call, -1)
+        if known is not None:
+            _forget_plane_matrix()
+            return Blocked(known[0], C8, x.T, x.N, known[1], known[2], known[3], x.dtype), known[5]
     if x.layout not in (C8, BITS) and not _is_input_frame(x):
         raise RuntimeError("unsupported_layout: conv_lif_blocked_avgpool takes inputs in C8 or BITS layout (or one dense frame of at most 8 channels)")
     if weight.dim() != 4 or int(weight.shape[1]) != x.C:
@@ -403,6 +458,8 @@ def conv_lif_blocked_avgpool(x: Blocked, weight: torch.Tensor, bias: Optional[to
     _lib.check("snnf_conv_lif_blocked_avgpool", _lib.lib().snnf_conv_lif_blocked_avgpool(
         x.step_pointers(), x.layout, x.T, x.N, x.C, x.H, x.W, _lib.dtype_code(x.dtype), packed.data_ptr(), cout, kh, kw, sh, sw, ph, pw,
         out.data.data_ptr(), out.step_stride_bytes(), _lib.ptr(v_out), float(lif[0]), float(lif[1]), float(lif[2]), _lib.current_stream(dev)))
+    if call is not None:
+        native.blocked_avgpool(*call, 0 if v_out is None else _ALLOCATE_V | _RETURN_V)
     return out, v_out
 
 
@@ -410,6 +467,11 @@ def spike_pool_linear(x: Blocked, fc_weight: torch.Tensor, fc_bias: Optional[tor
     """scale * sum_t (fc_weight . mean_hw(spikes_t) + fc_bias) of bit-packed spikes: [N, K] in the activation dtype. What is
     left of the LIF -> average pool -> Linear tail when the network's last neuron has fired inside the convolution in front of
     it; `scale = 1 / T` gives the mean over the timesteps."""
+    native = _dispatch.module()
+    call = (x.data, x.layout, x.shared, x.T, x.N, x.C, x.H, x.W, x.dtype, fc_weight, fc_bias, scale)
+    known = native.blocked_head(*call, -1)
+    if known is not None:
+        return known
     if x.layout != BITS or x.shared:
         raise RuntimeError("unsupported_layout: spike_pool_linear takes bit-packed spikes, one frame per timestep")
     if fc_weight.dim() != 2 or int(fc_weight.shape[1]) != x.C or fc_weight.dtype != x.dtype or (fc_bias is not None and fc_bias.dtype != x.dtype):
@@ -419,6 +481,7 @@ def spike_pool_linear(x: Blocked, fc_weight: torch.Tensor, fc_bias: Optional[tor
     _lib.check("snnf_spike_pool_linear", _lib.lib().snnf_spike_pool_linear(
         x.step_pointers(), x.T, x.N, x.C, x.H, x.W, w.data_ptr(), _lib.ptr(fc_bias), int(w.shape[0]), _lib.dtype_code(x.dtype),
         out.data_ptr(), float(scale), _lib.current_stream(x.data.device)))
+    native.blocked_head(*call, 0)
     return out
 
 

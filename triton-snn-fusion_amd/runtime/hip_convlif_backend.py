@@ -24,7 +24,7 @@ from typing import Dict, List, Optional, Sequence, Tuple
 
 import torch
 
-from .. import _lib
+from .. import _dispatch, _lib
 
 
 @dataclass
@@ -293,6 +293,9 @@ _PACK_CACHE_LIMIT = 512
 
 def clear_packed_weight_cache() -> None:
     _PACK_CACHE.clear()
+    native = _dispatch.loaded()
+    if native is not None:
+        native.forget_weights()
 
 
 def _packed_weight(weight: torch.Tensor, bias: Optional[torch.Tensor], x_dtype: torch.dtype) -> torch.Tensor:
@@ -403,6 +406,16 @@ def run_hip_temporal_conv_bias(xs: Sequence[torch.Tensor], weight, bias, stride,
         _lib.step_pointers(steps), _lib.step_pointers(res) if res is not None else None, T, n, cin, h, w,
         _lib.dtype_code(first.dtype), packed.data_ptr(), cout, kh, kw, sh, sw, ph, pw,
         out.data_ptr(), int(out.stride(0)), _lib.current_stream(first.device)))
+    return out
+
+
+def run_hip_conv_bias_frames(x_seq: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, stride, padding) -> torch.Tensor:
+    """run_hip_temporal_conv_bias of the T frames of one [T, N, C, H, W] tensor."""
+    native = _dispatch.module()
+    out = native.dense_conv_bias(x_seq, weight, bias, stride, padding, -1)
+    if out is None:
+        out = run_hip_temporal_conv_bias(list(x_seq.unbind(0)), weight, bias, stride, padding)
+        native.dense_conv_bias(x_seq, weight, bias, stride, padding, 0)
     return out
 
 

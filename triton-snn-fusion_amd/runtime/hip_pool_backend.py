@@ -9,7 +9,7 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
-from .. import _lib
+from .. import _dispatch, _lib
 
 
 def pool_config(module: nn.Module):
@@ -34,6 +34,10 @@ def pool_config(module: nn.Module):
 
 def run_hip_pool2d(x: torch.Tensor, is_max: bool, kernel: int, stride: int, padding: int) -> torch.Tensor:
     """Pools the last two dimensions of a contiguous [..., H, W] tensor; returns [..., Ho, Wo] in the same dtype."""
+    native = _dispatch.module() if x.is_cuda else None
+    known = None if native is None else native.dense_pool(x, is_max, kernel, stride, padding, -1)
+    if known is not None:
+        return known
     if not x.is_cuda or x.dtype not in (torch.float32, torch.bfloat16, torch.float16) or x.dim() < 3:
         raise RuntimeError("unsupported_device: snnf_pool2d needs an fp32 / bf16 / fp16 tensor [..., H, W] on the GPU")
     xc = x if x.is_contiguous() else x.contiguous()
@@ -45,4 +49,5 @@ def run_hip_pool2d(x: torch.Tensor, is_max: bool, kernel: int, stride: int, padd
     y = torch.empty(tuple(xc.shape[:-2]) + (ho, wo), dtype=xc.dtype, device=xc.device)
     _lib.check("snnf_pool2d", _lib.lib().snnf_pool2d(xc.data_ptr(), y.data_ptr(), planes, h, w, kernel, stride, padding,
                                                      1 if is_max else 0, _lib.dtype_code(xc.dtype), _lib.current_stream(xc.device)))
+    native.dense_pool(x, is_max, kernel, stride, padding, 0)
     return y

@@ -14,7 +14,9 @@ is never papered over: it raises even in non-strict mode.
 """
 from __future__ import annotations
 
+import copy
 import os
+import threading
 from collections import Counter
 from dataclasses import dataclass
 from typing import Any, Callable, Dict, List, Optional, Sequence, Tuple
@@ -22,8 +24,10 @@ from typing import Any, Callable, Dict, List, Optional, Sequence, Tuple
 import torch
 import torch.nn.functional as F
 
-from .. import _lib
+from .. import _dispatch, _lib
+from .hip_blocked_backend import _plane_matrix
 from .hip_convlif_backend import (
+    _packed_weight,
     check_triton_support,
     classify_conv_lif_config,
     get_autotune_best_config,
@@ -38,6 +42,7 @@ from .hip_convlif_backend import (
 from .hip_temporal_lif_avgpool_linear_backend import run_triton_fused_temporal_lif_avgpool_linear
 from .hip_temporal_lif_backend import run_hip_lif_forward_state, run_triton_fused_temporal_lif_state
 from .hip_temporal_linear_lif_backend import (
+    _split_workspace,
     run_triton_fused_temporal_linear_lif_state,
     run_triton_fused_temporal_linear_lif_state_packed,
     run_triton_fused_temporal_linear_lif_state_packed_out,
@@ -98,32 +103,75 @@ def configure_fused_op(backend: str = "torch", strict_triton: bool = False, verb
     _CONFIG.strict_triton = bool(strict_triton)
     _CONFIG.verbose = bool(verbose)
     _CONFIG.use_triton_autotune = bool(use_triton_autotune)
+    native = _dispatch.loaded()
+    if native is not None:
+        # Verbose calls report what they do, from the Python implementations.
+        native.enable(backend in NATIVE_BACKENDS and not _CONFIG.verbose)
 
 
 def reset_fused_op_call_stats() -> None:
     _CALL_STATS.clear()
     _CALL_STATS.update(_fresh_stats())
     _FALLBACK_REASON_STATS.clear()
+    native = _dispatch.loaded()
+    if native is not None:
+        native.reset_hits()
+
+
+def _all_call_stats() -> Dict[str, Any]:
+    """The counters of the Python implementations plus what the natively dispatched calls of known signatures add."""
+    stats = copy.deepcopy(_CALL_STATS)
+    native = _dispatch.loaded()
+    for events, hits in zip(_SIGNATURE_EVENTS, native.hits() if native is not None else ()):
+        if hits:
+            for event in events:
+                _count(stats, event, hits)
+    return stats
 
 
 def get_fused_op_call_stats() -> Dict[str, Any]:
-    out = {key: dict(value) if isinstance(value, dict) else value for key, value in _CALL_STATS.items()}
+    out = _all_call_stats()
     out["fallback_reasons"] = dict(_FALLBACK_REASON_STATS)
     return out
 
 
 def get_kernel_temporal_configs() -> Dict[str, int]:
-    return dict(_CALL_STATS.get("kernel_temporal_configs", {}))
+    return _all_call_stats().get("kernel_temporal_configs", {})
+
+
+# What a call adds to the statistics, as events: ("count", key), ("table", table, key) and ("signature", entry). While the first
+# call of a signature runs, its thread keeps them: each natively dispatched call of that signature adds the same.
+_SIGNATURE_EVENTS: List[tuple] = []
+_LEARNING = threading.local()
+
+
+def _count(stats: Dict[str, Any], event: tuple, amount: int = 1) -> None:
+    if event[0] == "count":
+        stats[event[1]] = stats.get(event[1], 0) + amount
+    elif event[0] == "table":
+        table = stats.setdefault(event[1], {})
+        table[event[2]] = table.get(event[2], 0) + amount
+    else:
+        entry = stats.setdefault("temporal_conv_lif_runtime_by_signature", {}).setdefault(
+            event[1], {"total": 0, "triton": 0, "fallback": 0, "fallback_reasons": {}})
+        entry["total"] += amount
+        entry["triton"] += amount
+
+
+def _record(event: tuple) -> None:
+    _count(_CALL_STATS, event)
+    events = getattr(_LEARNING, "events", None)
+    if events is not None:
+        events.append(event)
 
 
 def _bump(*keys: str) -> None:
     for key in keys:
-        _CALL_STATS[key] = _CALL_STATS.get(key, 0) + 1
+        _record(("count", key))
 
 
-def _bump_table(name: str, key: str, amount: int = 1) -> None:
-    table = _CALL_STATS.setdefault(name, {})
-    table[key] = table.get(key, 0) + amount
+def _bump_table(name: str, key: str) -> None:
+    _record(("table", name, key))
 
 
 # -----------------------------------------------------------------------------------------------------------------
@@ -242,12 +290,12 @@ def _format_conv_signature_key(x, weight, stride, padding, dilation, groups) -> 
 
 def _record_temporal_conv_signature(kind: str, signature: str, status: str, reasons=None) -> None:
     entry_key = f"{kind}:{signature}"
-    table = _CALL_STATS.setdefault("temporal_conv_lif_runtime_by_signature", {})
-    entry = table.setdefault(entry_key, {"total": 0, "triton": 0, "fallback": 0, "fallback_reasons": {}})
-    entry["total"] += 1
     if status == "triton":
-        entry["triton"] += 1
+        _record(("signature", entry_key))
     else:
+        table = _CALL_STATS.setdefault("temporal_conv_lif_runtime_by_signature", {})
+        entry = table.setdefault(entry_key, {"total": 0, "triton": 0, "fallback": 0, "fallback_reasons": {}})
+        entry["total"] += 1
         entry["fallback"] += 1
         for reason_key in _fallback_reason_keys(reasons):
             entry["fallback_reasons"][reason_key] = entry["fallback_reasons"].get(reason_key, 0) + 1
@@ -895,6 +943,35 @@ OPERATORS: Dict[str, Tuple[str, Callable, Optional[Callable], Callable]] = {
 }
 
 
+def _slow_dispatch(name: str, args: list, learn: bool) -> tuple:
+    """A GPU call the native dispatch does not know: (result, index of what a call of this signature counts or None). `learn`:
+    the call is one the native dispatch could take over, if it turns out to run on the kernels."""
+    impl = OPERATORS[name.partition("::")[2]][1]
+    if not learn:
+        return impl(*args), None
+    outer, _LEARNING.events = getattr(_LEARNING, "events", None), []
+    try:
+        result = impl(*args)
+    finally:
+        events, _LEARNING.events = tuple(_LEARNING.events), outer
+    if ("count", "triton") not in events or ("count", "fallback") in events:
+        return result, None
+    try:
+        return result, _SIGNATURE_EVENTS.index(events)
+    except ValueError:
+        _SIGNATURE_EVENTS.append(events)
+        return result, len(_SIGNATURE_EVENTS) - 1
+
+
+# Operators that csrc/host/snnf_dispatch.cpp implements for GPU tensors, with the implementations above behind it.
+NATIVE_DISPATCH = (
+    "lif_forward_state", "fused_conv_lif_state", "fused_temporal_conv_lif_state", "fused_temporal_pointwise_conv_lif_state",
+    "fused_temporal_depthwise_conv_lif_state", "fused_temporal_conv_lif_state_depthwise", "fused_temporal_conv_add_lif_state",
+    "fused_temporal_conv_add_lif_state_depthwise", "fused_temporal_lif_state", "fused_temporal_lif_avgpool_linear",
+    "fused_temporal_lif_tail", "fused_temporal_linear_lif_state", "fused_temporal_linear_lif_state_packed",
+)
+
+
 def register_snn_custom_ops() -> None:
     """Defines and implements the `snn_custom` library once per process (a second definition is ignored, like the
     reference's try/except around registration, runtime/snn_custom_ops.py:1964-2076)."""
@@ -907,13 +984,18 @@ def register_snn_custom_ops() -> None:
         pass
     try:
         impl_lib = torch.library.Library("snn_custom", "IMPL")
+        native = _dispatch.available()
         for name, (_, gpu_impl, cpu_impl, meta_impl) in OPERATORS.items():
             impl_lib.impl(name, cpu_impl if cpu_impl is not None else gpu_impl, "CPU")
-            impl_lib.impl(name, gpu_impl, "CUDA")
+            if not (native and name in NATIVE_DISPATCH):      # without a build GPU calls raise with the build instruction
+                impl_lib.impl(name, gpu_impl, "CUDA")
             impl_lib.impl(name, meta_impl, "Meta")
         TORCH_LIBRARY_HANDLES.append(impl_lib)
     except RuntimeError:
-        pass
+        return
+    if native:
+        _dispatch.connect(_slow_dispatch, _packed_weight, _plane_matrix,
+                          lambda device, T, M, fin, fout: _split_workspace(_lib.lib(), device, T, M, fin, fout))
 
 
 register_snn_custom_ops()
