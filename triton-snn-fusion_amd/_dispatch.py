@@ -2,6 +2,7 @@
 whose signature has been seen run from C++; everything else runs the Python implementations, which this module hands it."""
 from __future__ import annotations
 
+import importlib
 import importlib.machinery
 import importlib.util
 from typing import Callable, Optional
@@ -29,6 +30,8 @@ def module():
         loaded = importlib.util.module_from_spec(spec)
         loader.exec_module(loaded)
         _MODULE = loaded
+        # The operator layer connects the extension (`connect` below) when it is imported: whoever loads the extension imports it.
+        importlib.import_module(".runtime.snn_custom_ops", __package__)
     return _MODULE
 
 

@@ -47,7 +47,7 @@ constexpr size_t kMaxWeights = 512;
 // Signatures and plans
 // ------------------------------------------------------------------------------------------------------------------
 struct Key {
-    std::array<int64_t, 48> v;
+    std::array<int64_t, 64> v;
     int n = 0;
     bool plain = true;                     // false: something about the call keeps it off the fast path
 
@@ -826,6 +826,10 @@ bool proceed(Attempt& key, const Args& a, int64_t learnt) {
 }
 
 PyObject* guarded(PyObject* (*body)(Args&), PyObject* const* args, Py_ssize_t n, Py_ssize_t expected) {
+    if (g_pack == nullptr) {
+        PyErr_SetString(PyExc_RuntimeError, "snnf dispatch: not connected to the Python implementations");
+        return nullptr;
+    }
     if (n != expected) {
         PyErr_SetString(PyExc_TypeError, "snnf dispatch: wrong number of arguments");
         return nullptr;
@@ -1110,7 +1114,8 @@ PYBIND11_MODULE(_snnf_dispatch, m) {
         keep(&g_plane, std::move(plane));
         keep(&g_workspace, std::move(workspace));
     });
-    m.def("enable", [](bool on) { g_enabled.store(on); });
+    m.def("connected", [] { return g_pack != nullptr; });
+    m.def("enable", [](bool on) { g_enabled.store(on && g_pack != nullptr); });
     m.def("hits", [] {
         std::lock_guard<std::mutex> lock(g_mutex);
         return g_hits;
