@@ -243,6 +243,26 @@ int snnf_conv_lif(const void* const* xs, const void* const* residuals, int T,
                   void* spikes, int64_t spike_step_stride, void* v_out,
                   float v_threshold, float v_reset, float tau, void* stream);
 
+/*
+ * snnf_conv_lif with a caller-owned workspace, which lets the library bring the inputs into the channel-blocked layout
+ * first and run the kernel of that layout on them. The reference has no counterpart (its Triton kernel reads NCHW,
+ * kernels/benchmark_conv_lif_temporal_general.py:629-676). Results are those of snnf_conv_lif up to the order of the fp32
+ * additions.
+ *   snnf_conv_lif_workspace_bytes : bytes with which this shape takes that route (0: the call is snnf_conv_lif).
+ *   workspace : NULL (then this is snnf_conv_lif), or device memory, 16-byte aligned, contents undefined before and after.
+ *               A smaller workspace than asked for is not used. Calls that share a workspace must not overlap in time.
+ */
+size_t snnf_conv_lif_workspace_bytes(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW,
+                                     int stride_h, int stride_w, int pad_h, int pad_w, int v_dtype, int has_residual);
+int snnf_conv_lif_ws(const void* const* xs, const void* const* residuals, int T,
+                     int N, int Cin, int H, int W, int x_dtype,
+                     const void* packed_weight, int Cout, int KH, int KW,
+                     int stride_h, int stride_w, int pad_h, int pad_w,
+                     const void* v_init, int v_dtype,
+                     void* spikes, int64_t spike_step_stride, void* v_out,
+                     float v_threshold, float v_reset, float tau,
+                     void* workspace, size_t workspace_bytes, void* stream);
+
 /* Convolution + bias (+ residual) WITHOUT a neuron: out[t] = conv2d(xs[t]) + b (+ residuals[t]) in the activation dtype,
  * for T independent frames, with the same packed weight and matrix kernel as snnf_conv_lif. No fused operator of the
  * reference corresponds to it: its rewrite leaves LIF-free Conv+BN nodes (the 1x1 downsample shortcuts of a ResNet,
@@ -402,7 +422,9 @@ int snnf_conv_blocked_tune(int T, int N, int Cin, int H, int W, int Cout, int KH
                            int pad_h, int pad_w, int shared_frame, int patch_cols, int stage_groups, int k_waves);
 
 /* Describes what the most recent snnf_conv_lif / snnf_conv_bias call on this thread selected: kernel family, timesteps per launch, tile
- * and wave decomposition, LDS bytes, grid ("key=value" pairs, empty before the first call). Plays the role of the
+ * and wave decomposition, LDS bytes, grid ("key=value" pairs, empty before the first call). A layer that snnf_conv_lif_ws brought
+ * into the channel-blocked layout says route=c8: "kernel" is then the family that snnf_conv_lif runs it on, the rest describes
+ * the blocked launch. Plays the role of the
  * reference's get_autotune_best_config (kernels/benchmark_conv_lif_temporal_general.py:1332-1369), whose result the
  * operator layer publishes as kernel_temporal_config (runtime/snn_custom_ops.py:341-353): selection here is a
  * deterministic planner, and this is how a host reads its decision. The pointer stays valid for the thread's lifetime. */

@@ -1,0 +1,70 @@
+"""snnf_conv_lif_ws: layers on dense tensors that are brought into the channel-blocked layout first, against the CPU oracle and
+against snnf_conv_lif on the same operands, at the edges of the transposing copy (planes of 8 k pixels, of 4 k, ragged ones, one
+pixel; channel counts of a whole and of a part of a group; inputs that start at an odd element) and of the timestep windows."""
+import pytest
+import torch
+
+from helpers import DEV, LIF, check, dev, gen, q, spikes
+from oracle import snn_oracle as O
+
+pytestmark = pytest.mark.gpu
+BF16, F16, F32 = torch.bfloat16, torch.float16, torch.float32
+
+CASES = [  # (Cin, Cout, H, W, k, stride, T, N, dtype, residual, tensor v_init, elements the inputs start behind an aligned address)
+    (9, 17, 8, 8, 3, 1, 4, 2, BF16, False, False, 0),         # one channel in the second group; 16-byte runs of pixels
+    (12, 64, 6, 6, 3, 1, 4, 3, F16, True, True, 0),           # a plane of 4 k pixels
+    (20, 40, 5, 7, 3, 1, 3, 2, BF16, True, True, 0),          # 35 pixels: the last run holds three
+    (23, 33, 1, 1, 1, 1, 4, 5, BF16, False, True, 0),         # one pixel
+    (33, 30, 9, 5, 5, 1, 1, 1, F16, False, False, 0),         # one timestep
+    (30, 24, 8, 12, 3, 2, 16, 2, BF16, True, False, 0),       # the longest call, several windows
+    (44, 20, 7, 9, 3, 2, 5, 2, BF16, False, True, 1),         # inputs at an odd element, a last window of one step
+    (36, 24, 8, 8, 3, 1, 4, 2, BF16, False, False, 4),        # a plane of 8 k pixels at an 8-byte address
+    (128, 72, 7, 7, 3, 1, 4, 3, F16, True, True, 0),          # whole groups, the matrix kernel's masked variant
+    (300, 64, 3, 3, 3, 1, 6, 1, BF16, True, False, 0),        # K shared by the waves of a workgroup
+]
+
+
+@pytest.mark.parametrize("Cin,Cout,H,W,k,s,T,N,dtype,residual,tensor_v,shift", CASES)
+def test_conv_through_the_blocked_layout(snnf_lib, Cin, Cout, H, W, k, s, T, N, dtype, residual, tensor_v, shift):
+    from triton_snn_fusion_amd import _lib
+    from triton_snn_fusion_amd.runtime import hip_convlif_backend as CB
+    g = gen(4000 + Cin + Cout + H)
+    p = k // 2
+    Ho, Wo = (H + 2 * p - k) // s + 1, (W + 2 * p - k) // s + 1
+    xs = [q(torch.randn(N, Cin, H, W, generator=g), dtype) if t % 2 else spikes((N, Cin, H, W), 0.25, g) for t in range(T)]
+    w, b = q(torch.randn(Cout, Cin, k, k, generator=g) * 2.0 * (2.0 / (Cin * k * k)) ** 0.5, dtype), q(torch.randn(Cout, generator=g) * 0.1, dtype)
+    rs = [q(torch.randn(N, Cout, Ho, Wo, generator=g) * 0.3, dtype) for _ in range(T)] if residual else None
+    v0 = torch.randn(N, Cout, Ho, Wo, generator=g) * 0.3 if tensor_v else torch.tensor(0.0)
+    ref = O.temporal_conv_lif(xs, w, b, v0, (s, s), (p, p), (1, 1), 1, *LIF, residuals=rs)
+    dx = []
+    for x in xs:
+        room = torch.zeros(x.numel() + shift, device=DEV, dtype=dtype)
+        room[shift:].copy_(x.flatten())
+        dx.append(room[shift:].view(x.shape))
+    dr = [dev(r, dtype) for r in rs] if residual else None
+    dv = dev(v0, F32) if tensor_v else None
+    packed = CB._packed_weight(dev(w, dtype), dev(b, dtype), dtype)
+    code = _lib.dtype_code(dtype)
+    nbytes = snnf_lib.snnf_conv_lif_workspace_bytes(T, N, Cin, H, W, code, Cout, k, k, s, s, p, p, 0, int(residual))
+    assert nbytes == T * N * -(-Cin // 8) * H * W * 16
+    results = {}
+    for name, given in (("blocked", nbytes), ("dense", 0), ("short", nbytes - 1)):     # a workspace that is too small is not used
+        workspace = torch.full((nbytes,), 255, dtype=torch.uint8, device=DEV)          # NaN patterns
+        sp, v = torch.empty(T, N, Cout, Ho, Wo, device=DEV, dtype=dtype), torch.empty(N, Cout, Ho, Wo, device=DEV)
+        _lib.check(name, snnf_lib.snnf_conv_lif_ws(
+            _lib.step_pointers(dx), _lib.step_pointers(dr) if residual else None, T, N, Cin, H, W, code, packed.data_ptr(), Cout, k, k, s, s, p, p,
+            _lib.ptr(dv), 0, sp.data_ptr(), int(sp.stride(0)), v.data_ptr(), *LIF, workspace.data_ptr(), given, _lib.current_stream(sp.device)))
+        assert (CB.last_conv_plan().get("route") == "c8") == (name == "blocked"), CB.last_conv_plan()
+        check(sp, v, ref, what=f"{name} {Cin}->{Cout} {H}x{W}")
+        results[name] = (sp, v)
+    assert torch.equal(results["short"][0], results["dense"][0]) and torch.equal(results["short"][1], results["dense"][1])
+
+
+def test_layers_that_stay_on_the_dense_kernels(snnf_lib):
+    bf16, f32 = 1, 0
+    asks = snnf_lib.snnf_conv_lif_workspace_bytes
+    assert asks(4, 16, 64, 56, 56, bf16, 64, 3, 3, 1, 1, 1, 1, f32, 0) == 0          # whole tiles
+    assert asks(4, 16, 128, 56, 56, bf16, 256, 1, 1, 1, 1, 0, 0, f32, 0) == 0        # pointwise
+    assert asks(4, 8, 20, 9, 9, f32, 24, 3, 3, 1, 1, 1, 1, f32, 0) == 0              # float32 tensors
+    assert asks(1, 8, 20, 9, 9, bf16, 24, 3, 3, 1, 1, 1, 1, bf16, 0) == 0            # 16-bit membrane
+    assert asks(17, 8, 20, 9, 9, bf16, 24, 3, 3, 1, 1, 1, 1, f32, 0) == 0            # more timesteps than one launch takes

@@ -52,6 +52,9 @@ SIGNATURES = {
     "snnf_conv_pack_weight": (_i, [_vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _sz, _vp]),
     "snnf_conv_lif": (_i, [_pp, _pp, _i, _i, _i, _i, _i, _i, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _i, _vp, _i64,
                            _vp, _f, _f, _f, _vp]),
+    "snnf_conv_lif_workspace_bytes": (_sz, [_i] * 15),
+    "snnf_conv_lif_ws": (_i, [_pp, _pp, _i, _i, _i, _i, _i, _i, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _i, _vp, _i64,
+                              _vp, _f, _f, _f, _vp, _sz, _vp]),
     "snnf_layout_bytes": (_sz, [_i, _i64, _i, _i, _i, _i]),
     "snnf_layout_convert": (_i, [_vp, _i, _vp, _i, _i64, _i, _i, _i, _i, _vp]),
     "snnf_pool2d_blocked": (_i, [_vp, _i, _vp, _i, _i64, _i, _i, _i, _i, _i, _i, _i, _i, _vp]),

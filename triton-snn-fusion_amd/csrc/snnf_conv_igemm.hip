@@ -246,6 +246,37 @@ char* conv_plan_buffer() {
 extern "C" const char* snnf_conv_last_plan(void) { return snnf::conv_plan_buffer(); }
 
 namespace snnf {
+// What snnf_conv_lif runs a layer of 16-bit activations and an fp32 membrane on, whatever its neuron, when every operand is 16-byte
+// aligned and the steps have inputs of their own.
+DenseFamily dense_family(int T, int N, int Cin, int H, int W, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w, int x_dtype) {
+    const bool pointwise = KH == 1 && KW == 1 && stride_h == 1 && stride_w == 1 && pad_h == 0 && pad_w == 0;
+    if (pointwise && Cin % 8 == 0) return DenseFamily::kPointwise;
+    ConvGeom g = {};
+    g.N = N; g.Cin = Cin; g.Cout = Cout; g.KH = KH; g.KW = KW;
+    g.H = pointwise ? 1 : H; g.W = pointwise ? H * W : W;
+    g.sh = stride_h; g.sw = stride_w; g.ph = pad_h; g.pw = pad_w;
+    g.Ho = (g.H + 2 * pad_h - KH) / stride_h + 1;
+    g.Wo = (g.W + 2 * pad_w - KW) / stride_w + 1;
+    const PackGeom pg = make_pack_geom(Cout, Cin, KH, KW, false);
+    g.CK = pg.CK; g.nchunks = pg.nchunks; g.npairs = pg.npairs; g.nchunks_r = pg.nchunks_r;
+    while ((8 << g.groups_log2) < pg.CK) ++g.groups_log2;
+    g.pitch = pg.CK * 2 + 16;
+    const int64_t plane = static_cast<int64_t>(g.Ho) * g.Wo;
+    const int vec = plane % 8 == 0 ? 8 : (plane % 4 == 0 ? 4 : 0);
+    if (Cin % 8 == 0 || Cin < 8) {
+        for (int tt = T >= 3 ? 4 : T; tt >= 1; tt >>= 1) {
+            MmPlan p = {};
+            if (!plan_mm(g, tt, (g.W % 2 == 0 || g.W >= 3) ? LOAD_PAIR32 : LOAD_2X16, vec, 8, p)) continue;
+            if (Cout % 64 == 0 && p.all_full && p.run >= 4) return DenseFamily::kMatrixWhole;
+            if (tt < 4) return DenseFamily::kMatrixMasked;
+        }
+    }
+    const double flops = 2.0 * T * N * plane * Cout * Cin * KH * KW;
+    const double bytes = 2.0 * (static_cast<double>(T) * N * Cin * H * W + static_cast<double>(T) * N * Cout * plane) + 4.0 * N * Cout * plane;
+    Plan pl = {};
+    return flops / bytes < 200.0 && plan(g, 1, 0, g.W % 2 == 0 ? LOAD_PAIR32 : LOAD_2X16, vec == 8, pl) ? DenseFamily::kTimeOuter : DenseFamily::kTInM;
+}
+
 namespace {
 // Shared body of snnf_conv_lif and snnf_conv_bias. `analog_out`: no neuron - the convolution output (+ bias, + residual)
 // is written in the activation dtype where the spikes would go, and no membrane is read or written.

@@ -77,6 +77,33 @@ std::map<TunedKey, TunedPlan>& tuned_plans() {
     return plans;
 }
 
+size_t c8_step_bytes(int N, int Cin, int H, int W) { return static_cast<size_t>(N) * ((Cin + 7) / 8) * H * W * 16; }
+
+// Whether a layer on dense tensors is brought into C8 and run on the blocked kernel (two launches) or stays on the dense kernels.
+// Measured (bf16, us, dense / this route). Channel counts that are no multiple of 8 only have the four-wave kernels on dense
+// tensors, which assemble every channel group from scalar loads: 230 -> 144 at 11 x 83 stride 2 651 / 34, 167 -> 64 at 23 x 91
+// 765 / 86, 41 -> 88 at 44^2 57 / 24, 135 -> 144 at 9^2 stride 2 and T = 1 55 / 18; they always move. Layers that the
+// matrix kernel runs in its masked variant (planes or channels its tiles do not divide) go in windows of two timesteps there and
+// pay a pass over the weights per window: 512 -> 512 at 7^2 x 16 54 / 36, 352 -> 224 at 17 x 25 with a residual 47 / 32, 88 -> 176 at
+// 43^2 68 / 44, 80 -> 16 at 10^2 50 / 26; with few products per output the extra launch, and the residual's short loads, outweigh that:
+// 72 -> 104 at 27 x 35 with a residual 55 / 76, 32 -> 480 at 7^2 21 / 29. One or two timesteps are one window there:
+// 104 -> 168 at 23^2, T = 2, residual 42 / 57, 64 -> 80 at 46 x 17, T = 2 15 / 24, but 344 -> 16 at 20 x 37, 5x5, T = 2 108 / 79.
+// Whole tiles stay: 64 -> 64 at 56^2 x 16 38 / 54, 128 -> 128 at 28^2 x 16 41 / 42, 256 -> 256 at 14^2 x 16 35 / 34.
+bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w,
+                         int v_dtype, bool residual, DenseFamily& family) {
+    if (x_dtype != SNNF_BF16 && x_dtype != SNNF_F16) return false;
+    if (v_dtype != SNNF_F32 || T < 1 || T > SNNF_MAX_T_PER_LAUNCH || N < 1 || Cin < 1 || H < 1 || W < 1 || Cout < 1 || KH < 1 || KW < 1 ||
+        stride_h < 1 || stride_w < 1 || pad_h < 0 || pad_w < 0 || H + 2 * pad_h < KH || W + 2 * pad_w < KW) return false;
+    const int K = Cin * KH * KW;
+    family = dense_family(T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, x_dtype);
+    switch (family) {
+        case DenseFamily::kTInM:
+        case DenseFamily::kTimeOuter: return true;
+        case DenseFamily::kMatrixMasked: return T <= 2 ? K >= 2304 : K >= (residual ? 1152 : 432);
+        default: return false;
+    }
+}
+
 bool valid_layout(int layout) { return layout == SNNF_LAYOUT_NCHW || layout == SNNF_LAYOUT_C8 || layout == SNNF_LAYOUT_BITS; }
 
 // A projection shortcut whose sums join the main convolution's accumulators: a pointwise convolution (stride s, no padding)
@@ -87,7 +114,18 @@ struct Shortcut {
     const void* packed_weight;
 };
 
+// A call on dense tensors that runs here: its inputs, which are brought into C8 first, and the kernel family of the dense route.
+struct DenseRoute {
+    const void* const* xs;
+    DenseFamily family;
+};
+const char* family_name(DenseFamily f) {
+    return f == DenseFamily::kTInM ? "t_in_m" : (f == DenseFamily::kTimeOuter ? "time_outer" : (f == DenseFamily::kPointwise ? "pointwise" : "matrix"));
+}
+
 }  // namespace
+
+int launch_steps_to_c8(const StepPtrs& xs, int T, void* dst, int N, int C, int H, int W, hipStream_t stream);   // snnf_layout.hip
 
 char* conv_plan_buffer();   // the thread's plan text (snnf_conv_igemm.hip), shared with snnf_conv_last_plan()
 
@@ -96,7 +134,7 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
                           int N, int Cin, int H, int W, int x_dtype, const void* packed_weight, int Cout, int KH,
                           int KW, int stride_h, int stride_w, int pad_h, int pad_w, const void* v_init, void* out,
                           int out_layout, int64_t out_step_stride, void* v_out, int neuron, float v_threshold,
-                          float v_reset, float tau, void* stream, const Shortcut* sc, bool pool2 = false);
+                          float v_reset, float tau, void* stream, const Shortcut* sc, bool pool2 = false, const DenseRoute* dense = nullptr);
 }  // namespace
 
 }  // namespace snnf
@@ -148,13 +186,49 @@ extern "C" int snnf_conv_lif_blocked_avgpool(const void* const* xs, int x_layout
                                        v_reset, tau, stream, nullptr, true);
 }
 
+extern "C" size_t snnf_conv_lif_workspace_bytes(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h,
+                                                int stride_w, int pad_h, int pad_w, int v_dtype, int residual) {
+    using namespace snnf;
+    DenseFamily family;
+    if (!takes_blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residual != 0, family)) return 0;
+    return static_cast<size_t>(T) * c8_step_bytes(N, Cin, H, W);
+}
+
+extern "C" int snnf_conv_lif_ws(const void* const* xs, const void* const* residuals, int T, int N, int Cin, int H, int W, int x_dtype,
+                                const void* packed_weight, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w,
+                                const void* v_init, int v_dtype, void* spikes, int64_t spike_step_stride, void* v_out, float v_threshold,
+                                float v_reset, float tau, void* workspace, size_t workspace_bytes, void* stream) {
+    using namespace snnf;
+    DenseFamily family = DenseFamily::kTInM;
+    bool blocked = xs != nullptr && workspace != nullptr && v_out != nullptr && aligned_to(workspace, 16) && spike_step_stride >= 0 &&
+                   takes_blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residuals != nullptr, family);
+    bool shared = T > 1;
+    for (int t = 0; blocked && t < T; ++t) {
+        blocked = xs[t] != nullptr;
+        shared = shared && xs[t] == xs[0];
+    }
+    blocked = blocked && !shared;       // one frame for all timesteps is convolved once on the dense kernels too
+    const size_t step = blocked ? c8_step_bytes(N, Cin, H, W) : 0;
+    if (blocked && workspace_bytes >= step * T) {
+        const void* inner[SNNF_MAX_T_PER_LAUNCH];
+        for (int t = 0; t < T; ++t) inner[t] = static_cast<const char*>(workspace) + t * step;
+        const DenseRoute route = {xs, family};
+        const int rc = conv_lif_blocked_impl("snnf_conv_lif", inner, SNNF_LAYOUT_C8, residuals, SNNF_LAYOUT_NCHW, T, N, Cin, H, W, x_dtype, packed_weight,
+                                             Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_init, spikes, SNNF_LAYOUT_NCHW, spike_step_stride * 2, v_out,
+                                             1, v_threshold, v_reset, tau, stream, nullptr, false, &route);
+        if (rc != SNNF_ERR_UNSUPPORTED) return rc;
+    }
+    return snnf_conv_lif(xs, residuals, T, N, Cin, H, W, x_dtype, packed_weight, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_init, v_dtype, spikes,
+                         spike_step_stride, v_out, v_threshold, v_reset, tau, stream);
+}
+
 namespace snnf {
 namespace {
 int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, const void* const* residuals, int res_layout, int T,
                           int N, int Cin, int H, int W, int x_dtype, const void* packed_weight, int Cout, int KH,
                           int KW, int stride_h, int stride_w, int pad_h, int pad_w, const void* v_init, void* out,
                           int out_layout, int64_t out_step_stride, void* v_out, int neuron, float v_threshold,
-                          float v_reset, float tau, void* stream, const Shortcut* sc, bool pool2) {
+                          float v_reset, float tau, void* stream, const Shortcut* sc, bool pool2, const DenseRoute* dense) {
     if (xs == nullptr || packed_weight == nullptr || out == nullptr)
         return fail(SNNF_ERR_INVALID_ARGUMENT, "%s: xs, packed_weight and out must be non-null", who);
     if (T < 1 || N < 1 || Cin < 1 || H < 1 || W < 1 || Cout < 1 || KH < 1 || KW < 1 || stride_h < 1 || stride_w < 1 || pad_h < 0 || pad_w < 0)
@@ -364,11 +438,16 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
                           L.lif.v_threshold >= 1e-30f && L.lif.v_threshold <= 1e30f &&   // its multiples by 2^t stay normal numbers
                           v_init == nullptr && windows == 1 && Cout % 8 == 0;
     snprintf(snnf::conv_plan_buffer(), 256,
-             "kernel=blocked variant=%d window=%d launches=1 tile=%dx%dx%d halo=%dx%d waves=8x1x%d oc_tiles=%d px_tiles=%d "
-             "stage_chunks=%d run=0 lds=%zu grid=%d tuned=%d shortcut_stages=%d",
-             (wk_log2 > 0 ? 50 : 40) + tt + (fast_epi ? 20 : 0), shared ? T : tt, g.PI, g.PR, g.PC, g.RR, g.RC, 1 << wk_log2, oc_tiles, g.n_patches, g.G,
-             L.lds_bytes, grid, (tuned_patch ? 1 : 0) + (tuned_split ? 2 : 0), g.sc_stages);
+             "kernel=%s variant=%d window=%d launches=%d tile=%dx%dx%d halo=%dx%d waves=8x1x%d oc_tiles=%d px_tiles=%d "
+             "stage_chunks=%d run=0 lds=%zu grid=%d tuned=%d shortcut_stages=%d%s",
+             dense != nullptr ? family_name(dense->family) : "blocked", (wk_log2 > 0 ? 50 : 40) + tt + (fast_epi ? 20 : 0), shared ? T : tt, dense != nullptr ? 2 : 1, g.PI, g.PR, g.PC, g.RR, g.RC, 1 << wk_log2, oc_tiles, g.n_patches, g.G,
+             L.lds_bytes, grid, (tuned_patch ? 1 : 0) + (tuned_split ? 2 : 0), g.sc_stages, dense != nullptr ? " route=c8" : "");
     L.fast_epilogue = fast_epi;
+    if (dense != nullptr) {   // the plan stands: bring the dense inputs into the C8 buffers behind `xs`
+        StepPtrs from = {};
+        for (int t = 0; t < T; ++t) from.p[t] = dense->xs[t];
+        if (const int rc = launch_steps_to_c8(from, T, const_cast<void*>(xs[0]), N, Cin, H, W, L.stream); rc != SNNF_OK) return rc;
+    }
     if (pool2) {
         if (!fast_epi || windows != 1 || (tt != 4 && !shared))
             return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_pool: the pooled output needs the usual neuron (tau 2, hard reset to 0) and the four steps in one window", who);

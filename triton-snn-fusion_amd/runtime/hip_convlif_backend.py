@@ -367,10 +367,14 @@ def _launch(kernel_key: str, steps: Sequence[torch.Tensor], residuals: Optional[
             float(v_threshold), float(v_reset), float(tau), stream))
     else:
         packed = _packed_weight(weight, bias, first.dtype)
-        _lib.check("snnf_conv_lif", lib.snnf_conv_lif(
+        # Scratch for the inputs in the channel-blocked layout where the library asks for it; the caching allocator hands the block
+        # out again in the order of the stream the kernels run on.
+        nbytes = int(lib.snnf_conv_lif_workspace_bytes(T, n, cin, h, w, x_code, cout, kh, kw, sh, sw, ph, pw, v_code, 1 if rs is not None else 0))
+        workspace = torch.empty(nbytes, dtype=torch.uint8, device=first.device) if nbytes else None
+        _lib.check("snnf_conv_lif", lib.snnf_conv_lif_ws(
             xs, rs, T, n, cin, h, w, x_code, packed.data_ptr(), cout, kh, kw, sh, sw, ph, pw,
             _lib.ptr(vi), v_code, spikes.data_ptr(), step_stride, v_out.data_ptr(),
-            float(v_threshold), float(v_reset), float(tau), stream))
+            float(v_threshold), float(v_reset), float(tau), _lib.ptr(workspace), nbytes, stream))
 
 
 def run_hip_temporal_conv_bias(xs: Sequence[torch.Tensor], weight, bias, stride, padding,
