@@ -64,7 +64,29 @@ def test_layers_that_stay_on_the_dense_kernels(snnf_lib):
     bf16, f32 = 1, 0
     asks = snnf_lib.snnf_conv_lif_workspace_bytes
     assert asks(4, 16, 64, 56, 56, bf16, 64, 3, 3, 1, 1, 1, 1, f32, 0) == 0          # whole tiles
+    assert asks(4, 16, 256, 14, 14, bf16, 256, 3, 3, 1, 1, 1, 1, f32, 0) == 0        # ... of a deep layer with many outputs
+    assert asks(4, 2, 256, 14, 14, bf16, 256, 3, 3, 1, 1, 1, 1, f32, 0) > 0          # ... with few
     assert asks(4, 16, 128, 56, 56, bf16, 256, 1, 1, 1, 1, 0, 0, f32, 0) == 0        # pointwise
     assert asks(4, 8, 20, 9, 9, f32, 24, 3, 3, 1, 1, 1, 1, f32, 0) == 0              # float32 tensors
     assert asks(1, 8, 20, 9, 9, bf16, 24, 3, 3, 1, 1, 1, 1, bf16, 0) == 0            # 16-bit membrane
     assert asks(17, 8, 20, 9, 9, bf16, 24, 3, 3, 1, 1, 1, 1, f32, 0) == 0            # more timesteps than one launch takes
+
+
+@pytest.mark.parametrize("Cin,Cout,H,W,N,waves,groups", [
+    (128, 96, 8, 8, 1, "8x1x8", 2),        # few tiles: short stages, so that eight waves share K
+    (72, 64, 9, 7, 2, "8x1x4", 2),         # nine channel groups: the last stage holds one
+    (128, 64, 32, 40, 13, "8x1x2", 4),     # 520 tiles: four waves each would be a second round
+    (128, 64, 32, 40, 26, "8x1x1", 4),     # 1040 tiles: two waves each would be a second round
+])
+def test_waves_that_share_a_tile(snnf_lib, Cin, Cout, H, W, N, waves, groups):
+    from triton_snn_fusion_amd.runtime import hip_blocked_backend as B
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the shapes sit at the edges of 256 compute units")
+    g = gen(4500 + N)
+    x = torch.stack([spikes((N, Cin, H, W), 0.25, g) for _ in range(4)])
+    w, b = q(torch.randn(Cout, Cin, 3, 3, generator=g) * 2.0 * (2.0 / (Cin * 9)) ** 0.5, BF16), q(torch.randn(Cout, generator=g) * 0.1, BF16)
+    ref = O.temporal_conv_lif(list(x), w, b, torch.tensor(0.0), (1, 1), (1, 1), (1, 1), 1, *LIF)
+    out, v = B.conv_lif_blocked(B.from_dense(dev(x, BF16), B.BITS), dev(w, BF16), dev(b, BF16), [1, 1], [1, 1], LIF, out_layout=B.BITS, want_v=True)
+    plan = B.last_conv_plan()
+    assert (plan["waves"], int(plan["stage_chunks"])) == (waves, groups), plan
+    check(B.to_dense(out), v, ref, what=f"{Cin}->{Cout} {H}x{W} x {N}")

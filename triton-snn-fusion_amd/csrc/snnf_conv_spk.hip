@@ -62,6 +62,11 @@ bool plan_spk(const SpkGeom& g0, int tt, SpkPlan& best, int only_pc = 0, int onl
         // Wide patches store longer runs of a row; stages of 4 slots move in one batch.
         double score = eff / (1.0 + 0.08 * (halo - 1.0)) * (1.0 + 0.004 * std::min(pc, 16));
         if (G * region > 256) score *= 0.97;
+        // Waves own whole tiles: a launch of a little more than one round of waves takes as long as one of two. 88 -> 176 channels at
+        // 43^2 x 5 is 1980 tiles of 4 x 8 pixels (31 us) or 2205 of 4 x 7 (53 us) on 2048 waves. Among patches of several rounds the fewer
+        // tiles win (256 -> 256 at 14^2 x 128: 3584 of 2 x 14 99 us, 4096 of 4 x 8 103 us).
+        const int64_t tiles = static_cast<int64_t>(img_groups) * patches_x * patches_y * oc_tiles, slots = static_cast<int64_t>(cus) * kSpkWaves;
+        if (tiles > slots) score *= 0.6;
         if (score > best.score) best = SpkPlan{pr, pc, pi, rr, rc, region, G, patches_x, patches_y, img_groups, score};
     }
     return best.score > 0.0;
@@ -85,21 +90,26 @@ size_t c8_step_bytes(int N, int Cin, int H, int W) { return static_cast<size_t>(
 // 765 / 86, 41 -> 88 at 44^2 57 / 24, 135 -> 144 at 9^2 stride 2 and T = 1 55 / 18; they always move. Layers that the
 // matrix kernel runs in its masked variant (planes or channels its tiles do not divide) go in windows of two timesteps there and
 // pay a pass over the weights per window: 512 -> 512 at 7^2 x 16 54 / 36, 352 -> 224 at 17 x 25 with a residual 47 / 32, 88 -> 176 at
-// 43^2 68 / 44, 80 -> 16 at 10^2 50 / 26; with few products per output the extra launch, and the residual's short loads, outweigh that:
-// 72 -> 104 at 27 x 35 with a residual 55 / 76, 32 -> 480 at 7^2 21 / 29. One or two timesteps are one window there:
-// 104 -> 168 at 23^2, T = 2, residual 42 / 57, 64 -> 80 at 46 x 17, T = 2 15 / 24, but 344 -> 16 at 20 x 37, 5x5, T = 2 108 / 79.
-// Whole tiles stay: 64 -> 64 at 56^2 x 16 38 / 54, 128 -> 128 at 28^2 x 16 41 / 42, 256 -> 256 at 14^2 x 16 35 / 34.
+// 43^2 68 / 44, 72 -> 104 at 27 x 35, T = 6, with a residual 54 / 49, 80 -> 16 at 10^2 50 / 26; with few products per output the extra
+// launch and the 2-byte accesses of the dense output outweigh that: 32 -> 480 at 7^2 21 / 29, 24 -> 256 at 10 x 44, 5x5, with a
+// residual 27 / 33, 16 -> 96 at 25^2 with a residual 32 / 51. One or two timesteps are one window there: 16 -> 136 at 70^2 stride 2, T = 2
+// 31 / 47, 104 -> 168 at 23^2, T = 2, residual 42 / 57, but 344 -> 16 at 20 x 37, 5x5, T = 2 108 / 79, 304 -> 208 at 15^2, T = 1 28 / 21.
+// Whole tiles stay (64 -> 64 at 56^2 x 16 38 / 54, 128 -> 128 at 28^2 x 16 41 / 43, 256 -> 256 at 14^2 x 16 with a residual 37 / 40) but for
+// deep layers of few outputs and no residual, whose K the blocked kernel shares among more waves: 256 -> 256 at 14^2 x 2 27 / 22, at 6^2 x 8 33 / 23,
+// 512 -> 512 at 2^2 x 64 37 / 29 (at 8^2 x 64, a million outputs, 256 -> 256 36 / 39).
 bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w,
                          int v_dtype, bool residual, DenseFamily& family) {
     if (x_dtype != SNNF_BF16 && x_dtype != SNNF_F16) return false;
     if (v_dtype != SNNF_F32 || T < 1 || T > SNNF_MAX_T_PER_LAUNCH || N < 1 || Cin < 1 || H < 1 || W < 1 || Cout < 1 || KH < 1 || KW < 1 ||
         stride_h < 1 || stride_w < 1 || pad_h < 0 || pad_w < 0 || H + 2 * pad_h < KH || W + 2 * pad_w < KW) return false;
-    const int K = Cin * KH * KW;
+    const int64_t K = static_cast<int64_t>(Cin) * KH * KW;
+    const int64_t out = static_cast<int64_t>(N) * Cout * ((H + 2 * pad_h - KH) / stride_h + 1) * ((W + 2 * pad_w - KW) / stride_w + 1);
     family = dense_family(T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, x_dtype);
     switch (family) {
         case DenseFamily::kTInM:
         case DenseFamily::kTimeOuter: return true;
-        case DenseFamily::kMatrixMasked: return T <= 2 ? K >= 2304 : K >= (residual ? 1152 : 432);
+        case DenseFamily::kMatrixMasked: return T <= 2 ? K >= 1152 : K >= (residual ? 640 : 432);
+        case DenseFamily::kMatrixWhole: return T >= 3 && K >= 2304 && out <= 262144 && !residual;
         default: return false;
     }
 }
@@ -334,6 +344,14 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     if (!planned)
         return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_shape: no patch of this layer fits a wave's LDS region (kernel %dx%d, stride %dx%d)",
                     who, KH, KW, stride_h, stride_w);
+    if (!tuned_patch && !g.tap_pairs) {
+        // Few tiles: stages of fewer channel groups where that lets more waves share a tile's K (128 -> 256 at 8^2, one image: stages
+        // of 4 groups on 4 waves 13.4 us, of 2 groups on 8 waves 11.9 us; 64 -> 128 at 16^2 13.3 / 11.7).
+        const int64_t tiles = static_cast<int64_t>(pl.img_groups) * pl.patches_x * pl.patches_y * ((Cout + 63) / 64);
+        int share = 1;
+        while (share < kSpkWaves && tiles * share * 2 <= static_cast<int64_t>(compute_units()) * kSpkWaves) share *= 2;
+        while (pl.G > 2 && (g.C8in + pl.G - 1) / pl.G < share) pl.G >>= 1;
+    }
     const int windows = shared ? 1 : (T + tt - 1) / tt;
     if (neuron && windows > 1 && v_out == nullptr)
         return fail(SNNF_ERR_INVALID_ARGUMENT, "%s: v_out is required when the timesteps take %d windows of %d (it carries the membrane between them)",
@@ -348,11 +366,11 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     g.lds_wave_bytes = tt * (g.IT + 1) * 16;
     const int oc_tiles = (Cout + 63) / 64;
     g.n_items = g.n_patches * oc_tiles;
-    // Split K over waves of a workgroup while the layer has fewer items than the machine has SIMDs (one wave each) and
-    // every wave still gets at least one stage.
+    // K is shared by as many waves of a workgroup (up to eight, whole stages each) as keep the layer's tiles in one round of waves:
+    // 64 -> 64 at 56^2 x 12 is 1176 tiles, 20.2 us unsplit and 27.9 us when two waves share each (2352 of 2048 waves).
     const int cus = compute_units();
     int wk_log2 = 0;
-    while (wk_log2 < 3 && static_cast<int64_t>(g.n_items) << wk_log2 < static_cast<int64_t>(cus) * 6 && g.nstages >= (2 << wk_log2)) ++wk_log2;
+    while (wk_log2 < 3 && static_cast<int64_t>(g.n_items) << (wk_log2 + 1) <= static_cast<int64_t>(cus) * kSpkWaves && g.nstages >= (2 << wk_log2)) ++wk_log2;
     bool tuned_split = false;
     if (tuned.k_waves > 0) {
         int want = 0;
