@@ -277,6 +277,14 @@ int snnf_conv_bias(const void* const* xs, const void* const* residuals /* nullab
                    int stride_h, int stride_w, int pad_h, int pad_w,
                    void* out, int64_t out_step_stride, void* stream);
 
+/* snnf_conv_bias with a workspace of snnf_conv_lif_workspace_bytes(..., SNNF_F32, ...) bytes, as snnf_conv_lif_ws; accepts what
+ * snnf_conv_bias accepts. */
+int snnf_conv_bias_ws(const void* const* xs, const void* const* residuals /* nullable */, int T,
+                      int N, int Cin, int H, int W, int x_dtype,
+                      const void* packed_weight, int Cout, int KH, int KW,
+                      int stride_h, int stride_w, int pad_h, int pad_w,
+                      void* out, int64_t out_step_stride, void* workspace, size_t workspace_bytes, void* stream);
+
 /* 2-D pooling of `planes` independent H x W planes (NCHW with planes = N * C, or T * N * C for a spike sequence):
  * max 3x3 stride 2, max 2x2 stride 2 (padding <= kernel / 2, padded positions never win) and average 2x2 stride 2
  * (no padding), floor output size. No fused operator of the reference corresponds to it: pooling layers stay ordinary

@@ -90,3 +90,21 @@ def test_waves_that_share_a_tile(snnf_lib, Cin, Cout, H, W, N, waves, groups):
     plan = B.last_conv_plan()
     assert (plan["waves"], int(plan["stage_chunks"])) == (waves, groups), plan
     check(B.to_dense(out), v, ref, what=f"{Cin}->{Cout} {H}x{W} x {N}")
+
+
+@pytest.mark.parametrize("Cin,Cout,H,W,k,s,T,N,residual", [(128, 72, 7, 7, 3, 1, 4, 3, True), (256, 40, 6, 7, 3, 2, 5, 2, False), (480, 24, 9, 9, 1, 2, 1, 2, False)])
+def test_convolution_without_a_neuron(snnf_lib, Cin, Cout, H, W, k, s, T, N, residual):
+    """Against float64 sums rounded once to bf16: half a unit in the last place (2^-8 relative) and the float32 sums' own error."""
+    from triton_snn_fusion_amd.runtime import hip_convlif_backend as CB
+    g = gen(4700 + Cin)
+    p = k // 2
+    Ho, Wo = (H + 2 * p - k) // s + 1, (W + 2 * p - k) // s + 1
+    xs = [q(torch.randn(N, Cin, H, W, generator=g), BF16) for _ in range(T)]
+    w, b = q(torch.randn(Cout, Cin, k, k, generator=g) * (1.0 / (Cin * k * k)) ** 0.5, BF16), q(torch.randn(Cout, generator=g) * 0.1, BF16)
+    rs = [q(torch.randn(N, Cout, Ho, Wo, generator=g), BF16) for _ in range(T)] if residual else None
+    out = CB.run_hip_temporal_conv_bias([dev(x, BF16) for x in xs], dev(w, BF16), dev(b, BF16), [s, s], [p, p],
+                                        [dev(r, BF16) for r in rs] if residual else None)
+    want = k == 3 or T > 2
+    assert (CB.last_conv_plan().get("route") == "c8") == want, CB.last_conv_plan()
+    ref = torch.stack([torch.nn.functional.conv2d(x.double(), w.double(), b.double(), s, p) + (rs[t].double() if residual else 0) for t, x in enumerate(xs)])
+    assert torch.all((out.double().cpu() - ref).abs() <= ref.abs() * 2.0 ** -8 + 1e-4)

@@ -1056,10 +1056,16 @@ PyObject* dense_conv_bias(Args& a) {
     packed_steps(*x, T, steps);
     const Tensor packed = packed_weight(*w, *b, x->scalar_type());
     Tensor out = empty({T, N, cout, ho, wo}, x->scalar_type(), *x);
-    if (snnf_conv_bias(steps, nullptr, static_cast<int>(T), static_cast<int>(N), static_cast<int>(x->size(2)), static_cast<int>(H), static_cast<int>(W),
-                       code_of(x->scalar_type()), packed.data_ptr(), static_cast<int>(cout), static_cast<int>(kh), static_cast<int>(kw),
-                       static_cast<int>(sh), static_cast<int>(sw), static_cast<int>(ph), static_cast<int>(pw), out.data_ptr(), out.stride(0),
-                       stream_of(*x)) != 0)
+    const size_t bytes = snnf_conv_lif_workspace_bytes(static_cast<int>(T), static_cast<int>(N), static_cast<int>(x->size(2)), static_cast<int>(H),
+                                                       static_cast<int>(W), code_of(x->scalar_type()), static_cast<int>(cout), static_cast<int>(kh),
+                                                       static_cast<int>(kw), static_cast<int>(sh), static_cast<int>(sw), static_cast<int>(ph),
+                                                       static_cast<int>(pw), SNNF_F32, 0);
+    Tensor workspace;
+    if (bytes > 0) workspace = empty({static_cast<int64_t>(bytes)}, at::kByte, *x);
+    if (snnf_conv_bias_ws(steps, nullptr, static_cast<int>(T), static_cast<int>(N), static_cast<int>(x->size(2)), static_cast<int>(H), static_cast<int>(W),
+                          code_of(x->scalar_type()), packed.data_ptr(), static_cast<int>(cout), static_cast<int>(kh), static_cast<int>(kw),
+                          static_cast<int>(sh), static_cast<int>(sw), static_cast<int>(ph), static_cast<int>(pw), out.data_ptr(), out.stride(0),
+                          bytes > 0 ? workspace.data_ptr() : nullptr, bytes, stream_of(*x)) != 0)
         return none();
     return THPVariable_Wrap(out);
 }

@@ -204,32 +204,55 @@ extern "C" size_t snnf_conv_lif_workspace_bytes(int T, int N, int Cin, int H, in
     return static_cast<size_t>(T) * c8_step_bytes(N, Cin, H, W);
 }
 
+namespace snnf {
+namespace {
+// The blocked route of a call on dense tensors: SNNF_ERR_UNSUPPORTED (nothing enqueued) when it does not apply.
+int run_blocked_route(const void* const* xs, const void* const* residuals, int T, int N, int Cin, int H, int W, int x_dtype, const void* packed_weight,
+                      int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w, const void* v_init, int v_dtype, void* out,
+                      int64_t out_step_stride, void* v_out, int neuron, float v_threshold, float v_reset, float tau, void* workspace,
+                      size_t workspace_bytes, void* stream) {
+    DenseFamily family = DenseFamily::kTInM;
+    if (xs == nullptr || workspace == nullptr || (neuron && v_out == nullptr) || !aligned_to(workspace, 16) || out_step_stride < 0 ||
+        !takes_blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residuals != nullptr, family))
+        return SNNF_ERR_UNSUPPORTED;
+    // Without a neuron the dense route has the matrix kernel only; what it refuses stays refused.
+    if (!neuron && family != DenseFamily::kMatrixMasked && family != DenseFamily::kMatrixWhole) return SNNF_ERR_UNSUPPORTED;
+    const size_t step = c8_step_bytes(N, Cin, H, W);
+    if (workspace_bytes < step * T) return SNNF_ERR_UNSUPPORTED;
+    bool shared = T > 1;
+    const void* inner[SNNF_MAX_T_PER_LAUNCH];
+    for (int t = 0; t < T; ++t) {
+        if (xs[t] == nullptr) return SNNF_ERR_UNSUPPORTED;
+        shared = shared && xs[t] == xs[0];
+        inner[t] = static_cast<const char*>(workspace) + t * step;
+    }
+    if (shared) return SNNF_ERR_UNSUPPORTED;       // one frame for all timesteps is convolved once on the dense kernels too
+    const DenseRoute route = {xs, family};
+    return conv_lif_blocked_impl(neuron ? "snnf_conv_lif" : "snnf_conv_bias", inner, SNNF_LAYOUT_C8, residuals, SNNF_LAYOUT_NCHW, T, N, Cin, H, W, x_dtype,
+                                 packed_weight, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_init, out, SNNF_LAYOUT_NCHW, out_step_stride * 2, v_out,
+                                 neuron, v_threshold, v_reset, tau, stream, nullptr, false, &route);
+}
+}  // namespace
+}  // namespace snnf
+
 extern "C" int snnf_conv_lif_ws(const void* const* xs, const void* const* residuals, int T, int N, int Cin, int H, int W, int x_dtype,
                                 const void* packed_weight, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w,
                                 const void* v_init, int v_dtype, void* spikes, int64_t spike_step_stride, void* v_out, float v_threshold,
                                 float v_reset, float tau, void* workspace, size_t workspace_bytes, void* stream) {
-    using namespace snnf;
-    DenseFamily family = DenseFamily::kTInM;
-    bool blocked = xs != nullptr && workspace != nullptr && v_out != nullptr && aligned_to(workspace, 16) && spike_step_stride >= 0 &&
-                   takes_blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residuals != nullptr, family);
-    bool shared = T > 1;
-    for (int t = 0; blocked && t < T; ++t) {
-        blocked = xs[t] != nullptr;
-        shared = shared && xs[t] == xs[0];
-    }
-    blocked = blocked && !shared;       // one frame for all timesteps is convolved once on the dense kernels too
-    const size_t step = blocked ? c8_step_bytes(N, Cin, H, W) : 0;
-    if (blocked && workspace_bytes >= step * T) {
-        const void* inner[SNNF_MAX_T_PER_LAUNCH];
-        for (int t = 0; t < T; ++t) inner[t] = static_cast<const char*>(workspace) + t * step;
-        const DenseRoute route = {xs, family};
-        const int rc = conv_lif_blocked_impl("snnf_conv_lif", inner, SNNF_LAYOUT_C8, residuals, SNNF_LAYOUT_NCHW, T, N, Cin, H, W, x_dtype, packed_weight,
-                                             Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_init, spikes, SNNF_LAYOUT_NCHW, spike_step_stride * 2, v_out,
-                                             1, v_threshold, v_reset, tau, stream, nullptr, false, &route);
-        if (rc != SNNF_ERR_UNSUPPORTED) return rc;
-    }
+    const int rc = snnf::run_blocked_route(xs, residuals, T, N, Cin, H, W, x_dtype, packed_weight, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_init,
+                                           v_dtype, spikes, spike_step_stride, v_out, 1, v_threshold, v_reset, tau, workspace, workspace_bytes, stream);
+    if (rc != SNNF_ERR_UNSUPPORTED) return rc;
     return snnf_conv_lif(xs, residuals, T, N, Cin, H, W, x_dtype, packed_weight, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_init, v_dtype, spikes,
                          spike_step_stride, v_out, v_threshold, v_reset, tau, stream);
+}
+
+extern "C" int snnf_conv_bias_ws(const void* const* xs, const void* const* residuals, int T, int N, int Cin, int H, int W, int x_dtype,
+                                 const void* packed_weight, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w, void* out,
+                                 int64_t out_step_stride, void* workspace, size_t workspace_bytes, void* stream) {
+    const int rc = snnf::run_blocked_route(xs, residuals, T, N, Cin, H, W, x_dtype, packed_weight, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, nullptr,
+                                           SNNF_F32, out, out_step_stride, nullptr, 0, 1.0f, 0.0f, 2.0f, workspace, workspace_bytes, stream);
+    if (rc != SNNF_ERR_UNSUPPORTED) return rc;
+    return snnf_conv_bias(xs, residuals, T, N, Cin, H, W, x_dtype, packed_weight, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, out, out_step_stride, stream);
 }
 
 namespace snnf {

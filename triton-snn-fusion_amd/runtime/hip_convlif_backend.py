@@ -406,10 +406,13 @@ def run_hip_temporal_conv_bias(xs: Sequence[torch.Tensor], weight, bias, stride,
         bias = torch.zeros(cout, dtype=weight.dtype, device=weight.device)
     out = torch.empty((T, n, cout, ho, wo), dtype=first.dtype, device=first.device)
     packed = _packed_weight(weight, bias, first.dtype)
-    _lib.check("snnf_conv_bias", _lib.lib().snnf_conv_bias(
+    lib, x_code = _lib.lib(), _lib.dtype_code(first.dtype)
+    nbytes = int(lib.snnf_conv_lif_workspace_bytes(T, n, cin, h, w, x_code, cout, kh, kw, sh, sw, ph, pw, _lib.SNNF_F32, 1 if res is not None else 0))
+    workspace = torch.empty(nbytes, dtype=torch.uint8, device=first.device) if nbytes else None
+    _lib.check("snnf_conv_bias", lib.snnf_conv_bias_ws(
         _lib.step_pointers(steps), _lib.step_pointers(res) if res is not None else None, T, n, cin, h, w,
-        _lib.dtype_code(first.dtype), packed.data_ptr(), cout, kh, kw, sh, sw, ph, pw,
-        out.data_ptr(), int(out.stride(0)), _lib.current_stream(first.device)))
+        x_code, packed.data_ptr(), cout, kh, kw, sh, sw, ph, pw,
+        out.data_ptr(), int(out.stride(0)), _lib.ptr(workspace), nbytes, _lib.current_stream(first.device)))
     return out
 
 
