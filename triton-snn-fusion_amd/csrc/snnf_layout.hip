@@ -62,59 +62,39 @@ __global__ __launch_bounds__(kThreads) void layout_convert_kernel(const void* __
 }
 
 // The T dense tensors of an operator call -> one C8 tensor [T][N][C8][HW][8], 16-bit elements moved as they are. Bound by HBM. A
-// thread owns PX consecutive pixels of a channel group: 8 loads of 2 PX bytes, PX stores of 16 bytes that lie side by side (one
-// pixel per thread, as in layout_convert_kernel, moves 2 bytes per load: 25.7 MB of [4, 16, 64, 56, 56] took 16.4 us). PX = 8 needs planes
-// of a multiple of 8 pixels and 16-byte aligned tensors; PX = 4 takes any plane, its loads are then only 2-byte aligned, and the
-// last pixels of a plane that is no multiple of 4 are read one by one.
-template <int PX>
+// thread owns two neighbouring pixels of a channel group: 8 loads of 4 bytes (2-byte aligned where a plane is odd, whose last pixel
+// is read by itself) and two 16-byte stores side by side, so that a wave's loads cover 256 bytes of a channel and its stores 2 KB.
+// 279 MB ([4, 17, 479, 33, 65]) in 64 us = 4.4 TB/s; with four pixels per thread (loads of 8 bytes, stores 64 bytes apart) 99 us. At
+// [4, 16, 64, 56, 56] (51 MB) two, four and eight pixels per thread take 12, 15 and 16 us, one (layout_convert_kernel) 16.4 us.
 __global__ __launch_bounds__(kThreads) void steps_to_c8_kernel(const StepPtrs xs, uint16_t* __restrict__ dst, uint32_t items, int C, int C8, uint32_t HW,
-                                                               FastDiv d_runs, FastDiv d_C8, int64_t step_elems) {
+                                                               FastDiv d_pairs, FastDiv d_C8, int64_t step_elems) {
     const uint32_t item = blockIdx.x * kThreads + threadIdx.x;
     if (item >= items) return;
-    const uint32_t plane = static_cast<uint32_t>(fast_div(static_cast<int>(item), d_runs));
-    const uint32_t px = (item - plane * d_runs.d) * PX;
+    const uint32_t plane = static_cast<uint32_t>(fast_div(static_cast<int>(item), d_pairs));
+    const uint32_t px = (item - plane * d_pairs.d) * 2;
     const uint32_t n = static_cast<uint32_t>(fast_div(static_cast<int>(plane), d_C8));
     const uint32_t c0 = (plane - n * C8) * 8;
     const uint16_t* __restrict__ src = static_cast<const uint16_t*>(sk_kernarg_ptr(0, static_cast<int>(blockIdx.y))) + (static_cast<int64_t>(n) * C + c0) * HW + px;
     uint16_t* __restrict__ out = dst + static_cast<int64_t>(blockIdx.y) * step_elems + (static_cast<int64_t>(plane) * HW + px) * 8;
     const int chans = min(8, C - static_cast<int>(c0));
-    uint32_t v[8][PX / 2];
-    const uint32_t left = HW - px;
-    if (PX == 8 || left >= PX) {
+    const bool both = px + 1 < HW;
+    uint32_t v[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            if (j < chans) {
-                if constexpr (PX == 8) {
-                    const Pack<uint32_t, 4> w = *reinterpret_cast<const Pack<uint32_t, 4>*>(src + j * HW);
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) v[j][k] = w.v[k];
-                } else {
-                    __builtin_memcpy(v[j], src + j * HW, 2 * PX);
-                }
-            } else {
-#pragma unroll
-                for (int k = 0; k < PX / 2; ++k) v[j][k] = 0u;
-            }
+    for (int j = 0; j < 8; ++j) {
+        v[j] = 0u;
+        if (j < chans) {
+            if (both) __builtin_memcpy(&v[j], src + j * HW, 4);
+            else v[j] = src[j * HW];
         }
-    } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-#pragma unroll
-            for (int k = 0; k < PX / 2; ++k) {
-                const uint32_t a = j < chans && 2u * k < left ? src[j * HW + 2 * k] : 0u;
-                const uint32_t b = j < chans && 2u * k + 1u < left ? src[j * HW + 2 * k + 1] : 0u;
-                v[j][k] = a | (b << 16);
-            }
     }
+    Pack<uint32_t, 4> g;
 #pragma unroll
-    for (int p = 0; p < PX; ++p) {
-        if (PX == 8 || static_cast<uint32_t>(p) < left) {
-            Pack<uint32_t, 4> g;
+    for (int k = 0; k < 4; ++k) g.v[k] = __builtin_amdgcn_perm(v[2 * k + 1], v[2 * k], 0x05040100u);
+    *reinterpret_cast<Pack<uint32_t, 4>*>(out) = g;
+    if (both) {
 #pragma unroll
-            for (int k = 0; k < 4; ++k)
-                g.v[k] = __builtin_amdgcn_perm(v[2 * k + 1][p / 2], v[2 * k][p / 2], (p & 1) ? 0x07060302u : 0x05040100u);
-            *reinterpret_cast<Pack<uint32_t, 4>*>(out + p * 8) = g;
-        }
+        for (int k = 0; k < 4; ++k) g.v[k] = __builtin_amdgcn_perm(v[2 * k + 1], v[2 * k], 0x07060302u);
+        *reinterpret_cast<Pack<uint32_t, 4>*>(out + 8) = g;
     }
 }
 
@@ -262,16 +242,11 @@ int pool_typed(const void* x, int xl, void* y, int yl, int64_t frames, int C, in
 int launch_steps_to_c8(const StepPtrs& xs, int T, void* dst, int N, int C, int H, int W, hipStream_t stream) {
     const int C8 = (C + 7) / 8;
     const int64_t HW = static_cast<int64_t>(H) * W;
-    bool wide = HW % 8 == 0;
-    for (int t = 0; t < T; ++t) wide = wide && aligned_to(xs.p[t], 16);
-    const int px = wide ? 8 : 4;
-    const int64_t runs = (HW + px - 1) / px, items = runs * N * C8;
+    const int64_t pairs = (HW + 1) / 2, items = pairs * N * C8;
     if (items >= (1LL << 30)) return fail(SNNF_ERR_UNSUPPORTED, "snnf_conv_lif: unsupported_shape: too many elements for the blocked copy");
     const dim3 grid(static_cast<unsigned>((items + kThreads - 1) / kThreads), static_cast<unsigned>(T));
-    const FastDiv d_runs = make_fast_div(static_cast<int>(runs)), d_C8 = make_fast_div(C8);
-    const int64_t step = static_cast<int64_t>(N) * C8 * HW * 8;
-    if (wide) steps_to_c8_kernel<8><<<grid, kThreads, 0, stream>>>(xs, static_cast<uint16_t*>(dst), static_cast<uint32_t>(items), C, C8, static_cast<uint32_t>(HW), d_runs, d_C8, step);
-    else steps_to_c8_kernel<4><<<grid, kThreads, 0, stream>>>(xs, static_cast<uint16_t*>(dst), static_cast<uint32_t>(items), C, C8, static_cast<uint32_t>(HW), d_runs, d_C8, step);
+    steps_to_c8_kernel<<<grid, kThreads, 0, stream>>>(xs, static_cast<uint16_t*>(dst), static_cast<uint32_t>(items), C, C8, static_cast<uint32_t>(HW),
+                                                       make_fast_div(static_cast<int>(pairs)), make_fast_div(C8), static_cast<int64_t>(N) * C8 * HW * 8);
     return check_launch("snnf_conv_lif");
 }
 
