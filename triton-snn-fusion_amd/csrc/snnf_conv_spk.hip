@@ -85,21 +85,22 @@ std::map<TunedKey, TunedPlan>& tuned_plans() {
 size_t c8_step_bytes(int N, int Cin, int H, int W) { return static_cast<size_t>(N) * ((Cin + 7) / 8) * H * W * 16; }
 
 // Whether a layer on dense tensors is brought into C8 and run on the blocked kernel (two launches) or stays on the dense kernels.
-// Measured (bf16, us, dense / this route). Channel counts that are no multiple of 8 only have the four-wave kernels on dense
-// tensors, which assemble every channel group from scalar loads: 230 -> 144 at 11 x 83 stride 2 651 / 34, 167 -> 64 at 23 x 91
-// 765 / 86, 41 -> 88 at 44^2 57 / 24, 135 -> 144 at 9^2 stride 2 and T = 1 55 / 18; they move, but for large 1x1 layers, which are
-// memory traffic (421 -> 288 at 100^2, T = 8, 342 MB: 352 / 440; 99 -> 130 at 40^2 28 / 23). Layers that the
-// matrix kernel runs in its masked variant (planes or channels its tiles do not divide) go in windows of two timesteps there and
-// pay a pass over the weights per window: 512 -> 512 at 7^2 x 16 54 / 36, 352 -> 224 at 17 x 25 with a residual 47 / 32, 88 -> 176 at
-// 43^2 68 / 44, 72 -> 104 at 27 x 35, T = 6, with a residual 54 / 49, 80 -> 16 at 10^2 50 / 26; with few products per output the extra
-// launch and the 2-byte accesses of the dense output outweigh that: 32 -> 480 at 7^2 21 / 29, 24 -> 256 at 10 x 44, 5x5, with a
-// residual 27 / 33, 16 -> 96 at 25^2 with a residual 32 / 51. One or two timesteps are one window there: 16 -> 136 at 70^2 stride 2, T = 2
-// 31 / 47, 104 -> 168 at 23^2, T = 2, residual 42 / 57, but 344 -> 16 at 20 x 37, 5x5, T = 2 108 / 79, 304 -> 208 at 15^2, T = 1 28 / 21.
-// More than four timesteps are several windows here as well, over which few channels do not pay: 40 -> 16 at 24 x 59, 5x5, T = 5
-// 41 / 55, 48 -> 16 at 66 x 103, 7x7, T = 8 80 / 99, but 56 -> 184 at 17^2, 7x7, T = 5 63 / 47, 72 -> 184 at 7^2, T = 8 134 / 54.
-// Whole tiles stay (64 -> 64 at 56^2 x 16 38 / 54, 128 -> 128 at 28^2 x 16 41 / 43, 256 -> 256 at 14^2 x 16 with a residual 37 / 40) but for
-// deep layers of few outputs and no residual, whose K the blocked kernel shares among more waves: 256 -> 256 at 14^2 x 2 27 / 22, at 6^2 x 8 33 / 23,
-// 512 -> 512 at 2^2 x 64 37 / 29 (at 8^2 x 64, a million outputs, 256 -> 256 36 / 39).
+// Measured (bf16, T = 4 unless said, us, dense / this route). Channel counts that are no multiple of 8 only have the four-wave kernels
+// on dense tensors, which assemble every channel group from scalar loads: 230 -> 144 at 11 x 83 stride 2 650 / 32, 167 -> 64 at
+// 23 x 91, T = 3 763 / 76, 41 -> 88 at 44^2 57 / 25, 135 -> 144 at 9^2 stride 2, T = 1 56 / 13; they move, but for large 1x1 layers, which
+// are memory traffic (421 -> 288 at 100^2, T = 8, 342 MB: 356 / 416; 99 -> 130 at 40^2 28 / 23). Layers that the matrix kernel runs in
+// its masked variant (planes or channels its tiles do not divide) go in windows of two timesteps there and pay a pass over the
+// weights per window: 512 -> 512 at 7^2 x 16 56 / 34, 352 -> 224 at 17 x 25 with a residual 47 / 30, 88 -> 176 at 43^2 68 / 41, 72 -> 104 at
+// 27 x 35, T = 6, with a residual 54 / 48, 80 -> 16 at 10^2, T = 3 50 / 20; with few products per output the extra launch and the
+// 2-byte accesses of the dense output outweigh that: 24 -> 256 at 10 x 44, 5x5, with a residual 27 / 32, 16 -> 96 at 25^2 with a residual
+// 32 / 49. One or two timesteps are one window there: 16 -> 136 at 70^2 stride 2, T = 2 31 / 46, 104 -> 168 at 23^2, T = 2, residual 41 / 53,
+// but 344 -> 16 at 20 x 37, 5x5, T = 2 106 / 71, 304 -> 208 at 15^2, T = 1 27 / 19. More than four timesteps are several windows here as
+// well, over which few channels do not pay: 40 -> 16 at 24 x 59, 5x5, T = 5 41 / 56, 48 -> 16 at 66 x 103, 7x7, T = 8 80 / 95, but 56 -> 184 at
+// 17^2, 7x7, T = 5 63 / 46, 72 -> 184 at 7^2, T = 8 134 / 39.
+// Whole tiles stay (64 -> 64 at 56^2 x 16 37 / 50, 128 -> 128 at 28^2 x 16 40 / 40 and with a residual 42 / 50, 256 -> 256 at 14^2 x 16 with a
+// residual 37 / 39, at 8^2 x 64 36 / 37) but for deep layers, whose K the blocked kernel shares among more waves: 512 -> 512 at 4^2 x 16
+// 36 / 30 and with a residual 36 / 31, at 4^2 x 64 49 / 39, at 2^2 x 64 37 / 29; of 256 channels those with few outputs: 14^2 x 4
+// 28 / 23 (T = 1 15 / 14, T = 6 53 / 39), 6^2 x 16 33 / 23, 256 -> 512 at 4^2 x 64 29 / 27.
 bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w,
                          int v_dtype, bool residual, DenseFamily& family) {
     if (x_dtype != SNNF_BF16 && x_dtype != SNNF_F16) return false;
@@ -113,7 +114,7 @@ bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int C
         case DenseFamily::kTInM:
         case DenseFamily::kTimeOuter: return !pointwise || static_cast<int64_t>(T) * N * (Cin + Cout) * H * W <= (1 << 25);
         case DenseFamily::kMatrixMasked: return T > 4 && Cin < 56 ? false : T <= 2 ? K >= 1152 : K >= (residual ? 640 : 432);
-        case DenseFamily::kMatrixWhole: return T >= 3 && K >= 2304 && out <= 262144 && !residual;
+        case DenseFamily::kMatrixWhole: return K >= 4608 || (K >= 2304 && out <= (1 << 19) && !residual);
         default: return false;
     }
 }
