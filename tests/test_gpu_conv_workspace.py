@@ -72,13 +72,17 @@ def test_layers_that_stay_on_the_dense_kernels(snnf_lib):
     assert asks(17, 8, 20, 9, 9, bf16, 24, 3, 3, 1, 1, 1, 1, f32, 0) == 0            # more timesteps than one launch takes
 
 
-@pytest.mark.parametrize("Cin,Cout,H,W,N,waves,groups", [
-    (128, 96, 8, 8, 1, "8x1x8", 2),        # few tiles: short stages, so that eight waves share K
-    (72, 64, 9, 7, 2, "8x1x4", 2),         # nine channel groups: the last stage holds one
-    (128, 64, 32, 40, 13, "8x1x2", 4),     # 520 tiles: four waves each would be a second round
-    (128, 64, 32, 40, 26, "8x1x1", 4),     # 1040 tiles: two waves each would be a second round
+@pytest.mark.parametrize("Cin,Cout,H,W,N,waves,groups,tiles", [
+    (128, 96, 8, 8, 1, "8x1x8", 2, 3),        # few tiles: short stages, so that eight waves share K; tiles of 32 channels
+    (128, 40, 8, 8, 1, "8x1x8", 2, 2),        # ... the last of them with 8
+    (32, 40, 5, 5, 1, "8x1x2", 2, 2),         # ... two waves each
+    (64, 32, 5, 5, 1, "8x1x4", 2, 1),         # ... no more than one tile of channels
+    (256, 96, 32, 16, 8, "8x1x8", 4, 2),      # 256 tiles of 64 channels on eight waves: 384 of 32 would be a second round
+    (72, 64, 9, 7, 2, "8x1x4", 2, 2),         # nine channel groups: the last stage holds one
+    (128, 64, 32, 40, 13, "8x1x2", 4, 1),     # 520 tiles: four waves each would be a second round
+    (128, 64, 32, 40, 26, "8x1x1", 4, 1),     # 1040 tiles: two waves each would be a second round
 ])
-def test_waves_that_share_a_tile(snnf_lib, Cin, Cout, H, W, N, waves, groups):
+def test_waves_that_share_a_tile(snnf_lib, Cin, Cout, H, W, N, waves, groups, tiles):
     from triton_snn_fusion_amd.runtime import hip_blocked_backend as B
     if torch.cuda.get_device_properties(0).multi_processor_count != 256:
         pytest.skip("the shapes sit at the edges of 256 compute units")
@@ -88,7 +92,7 @@ def test_waves_that_share_a_tile(snnf_lib, Cin, Cout, H, W, N, waves, groups):
     ref = O.temporal_conv_lif(list(x), w, b, torch.tensor(0.0), (1, 1), (1, 1), (1, 1), 1, *LIF)
     out, v = B.conv_lif_blocked(B.from_dense(dev(x, BF16), B.BITS), dev(w, BF16), dev(b, BF16), [1, 1], [1, 1], LIF, out_layout=B.BITS, want_v=True)
     plan = B.last_conv_plan()
-    assert (plan["waves"], int(plan["stage_chunks"])) == (waves, groups), plan
+    assert (plan["waves"], int(plan["stage_chunks"]), int(plan["oc_tiles"])) == (waves, groups, tiles), plan
     check(B.to_dense(out), v, ref, what=f"{Cin}->{Cout} {H}x{W} x {N}")
 
 

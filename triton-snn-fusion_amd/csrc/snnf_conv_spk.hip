@@ -392,7 +392,7 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     g.IT = g.G * g.region;
     g.JT = (g.IT + 63) / 64;
     g.lds_wave_bytes = tt * (g.IT + 1) * 16;
-    const int oc_tiles = (Cout + 63) / 64;
+    int oc_tiles = (Cout + 63) / 64;
     g.n_items = g.n_patches * oc_tiles;
     // K is shared by as many waves of a workgroup (up to eight, whole stages each) as keep the layer's tiles in one round of waves:
     // 64 -> 64 at 56^2 x 12 is 1176 tiles, 20.2 us unsplit and 27.9 us when two waves share each (2352 of 2048 waves).
@@ -409,6 +409,13 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
         }
     }
     g.wk_log2 = wk_log2;
+    // Tiles of 32 channels where even those fit one round of waves: 256 -> 256 at 14^2 x 4 (112 tiles of 64 channels on eight waves each)
+    // 13.9 -> 10.0 us, 512 -> 512 at 7^2 x 8 19.8 -> 13.9, at 4^2 x 32 22.2 -> 17.6. At twice the tiles they would make a second round.
+    if (tt == 4 && wk_log2 > 0 && !tuned_split && Cout > 32 && static_cast<int64_t>(g.n_patches) * ((Cout + 31) / 32) << wk_log2 <= static_cast<int64_t>(cus) * kSpkWaves) {
+        g.narrow = 1;
+        oc_tiles = (Cout + 31) / 32;
+        g.n_items = g.n_patches * oc_tiles;
+    }
     const int tiles_per_block = kSpkWaves >> wk_log2;
     // Workgroups that are resident together: one per compute unit, or two where a wave needs at most a quarter of a SIMD's
     // registers (one timestep's accumulators) and two staging areas fit the LDS. The tiles are dealt evenly over as many

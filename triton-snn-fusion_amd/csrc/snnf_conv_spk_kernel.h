@@ -67,7 +67,8 @@ struct SpkGeom {
     int hg_log2;                 // log2 of the k-slot pairs per tap and stage (G / 2; 0 with tap pairs)
     int pair_tap_stride;         // packed pairs between consecutive taps of one group pair (gpc / 2; 1 with tap pairs)
     int wk_log2;                 // split-K: waves per tile
-    int n_items, iters;          // (patch, 64-channel tile) pairs; loop trips per wave
+    int n_items, iters;          // (patch, channel tile) pairs; loop trips per wave
+    int narrow;                  // tiles of 32 output channels instead of 64
     int in_layout, res_layout, out_layout;   // snnf_layout codes; res_layout < 0: no residual
     int analog_out;              // no neuron: the sums themselves are written (C8 or NCHW)
     int pool2;                   // the POOL variants: the spikes leave as their 2x2 averages (quarters, C8, half the plane)
@@ -143,7 +144,10 @@ __device__ __forceinline__ sk_u32x4 sk_expand_bits(uint32_t byte) {
     return d;
 }
 
-template <typename XT, int TT, int IN, bool SK, bool FAST, bool SC = false, bool POOL = false>
+// NARROW: tiles of 32 output channels (one weight fragment) for launches of few tiles that share K among waves: twice the workgroups,
+// each with half the matrix instructions and half the weights in its chain of steps, which is what such a launch lasts (512 -> 512 at
+// 4^2, one image: 288 steps on eight waves, 19.1 -> 12.6 us; 64 -> 64 at 56^2 11.7 -> 8.7 us).
+template <typename XT, int TT, int IN, bool SK, bool FAST, bool SC = false, bool POOL = false, bool NARROW = false>
 __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_eu(TT == 1 ? 4 : 2, TT == 1 ? 4 : 2))) void conv_spk_kernel(
     const StepPtrs xs, const StepPtrs residuals, const SpkGeom g, const uint16_t* __restrict__ wpacked,
     const float* __restrict__ bias, const float* __restrict__ v_init, unsigned char* __restrict__ out,
@@ -172,6 +176,9 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
     static_assert(!SC || (IN == SNNF_LAYOUT_BITS && TT == 4), "the shortcut variants take bit-packed inputs, four timesteps at a time");
     static_assert(!POOL || (FAST && (TT == 4 || TT == 1)), "the pooled output belongs to the straight-line epilogue of four steps");
     static_assert(IN != SNNF_LAYOUT_NCHW || TT == 1, "a dense input is one frame for all timesteps");
+    static_assert(!NARROW || (SK && TT == 4), "narrow tiles are for launches that share K among waves");
+    constexpr int NF = NARROW ? 1 : 2;         // 32-channel weight fragments of a tile
+    constexpr int TG = 4 * NF;                 // channel groups of 8 of a tile
     constexpr bool F16 = dtype_of<XT>::value == SNNF_F16;
     constexpr uint32_t ONE = F16 ? 0x3c00u : 0x3f80u;
     constexpr int kResTable = static_cast<int>(sizeof(StepPtrs));
@@ -305,10 +312,10 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
         const bool lane_in_patch = pi < g.PI;
         const uint32_t lane_b = lane_in_patch ? static_cast<uint32_t>(((pi * g.RR + prow * g.sh) * g.RC + pcol * g.sw) * 16) : 0u;
 
-        const int ocf0 = oc_tile * 2;
+        const int ocf0 = oc_tile * NF;
         // With K split over two waves the second one computes the tile's two 32-channel fragments in swapped places: each wave
         // then finishes the fragment in its accumulators' first half (fragment wk) and hands over the second half.
-        const int swap_f = (SK && WK == 2) ? wk : 0;
+        const int swap_f = (SK && !NARROW && WK == 2) ? wk : 0;
         const int64_t w_frag0 = min(ocf0 + swap_f, g.nocf - 1);
         const int64_t w_frag1 = min(ocf0 + 1 - swap_f, g.nocf - 1);
 
@@ -324,30 +331,30 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             // The accumulators start from the bias: register 4 q + k of fragment f is channel 64 oc_tile + 32 f + 8 q + 4 half + k.
             // With K split over waves only the first one adds it. The bias is requested here and copied into the accumulators
             // after the first stage's activations have been requested, so that both round trips to memory overlap.
-            sk_f32x16 acc[TT][2];
-            sk_f32x4 bias4[2][4];
+            sk_f32x16 acc[TT][NF];
+            sk_f32x4 bias4[NF][4];
             {
                 const int nbias = g.nocf * 32;               // bias values behind the packed weight (zero beyond Cout)
 #pragma unroll
-                for (int f = 0; f < 2; ++f)
+                for (int f = 0; f < NF; ++f)
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
-                        const int ch0 = oc_tile * 64 + f * 32 + q * 8 + 4 * half;
+                        const int ch0 = oc_tile * (32 * NF) + f * 32 + q * 8 + 4 * half;
                         bias4[f][q] = sk_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
                         if (ch0 < nbias && (!SK || wk == 0)) bias4[f][q] = *reinterpret_cast<const sk_f32x4*>(bias + ch0);
                     }
                 if constexpr (SC) {
-                    sk_f32x4 more[2][4];
+                    sk_f32x4 more[NF][4];
 #pragma unroll
-                    for (int f = 0; f < 2; ++f)
+                    for (int f = 0; f < NF; ++f)
 #pragma unroll
                         for (int q = 0; q < 4; ++q) {
-                            const int ch0 = oc_tile * 64 + f * 32 + q * 8 + 4 * half;
+                            const int ch0 = oc_tile * (32 * NF) + f * 32 + q * 8 + 4 * half;
                             more[f][q] = sk_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
                             if (ch0 < nbias && (!SK || wk == 0)) more[f][q] = *reinterpret_cast<const sk_f32x4*>(bias2 + ch0);
                         }
 #pragma unroll
-                    for (int f = 0; f < 2; ++f)
+                    for (int f = 0; f < NF; ++f)
 #pragma unroll
                         for (int q = 0; q < 4; ++q) bias4[f][q] += more[f][q];
                 }
@@ -506,7 +513,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             int oc_e = oc_tile;
             asm volatile("" : "+s"(oc_e));
 #pragma unroll
-            for (int f = 0; f < 2; ++f)
+            for (int f = 0; f < NF; ++f)
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
 #pragma unroll
@@ -534,14 +541,14 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     const unsigned char* __restrict__ pa1 = reinterpret_cast<const unsigned char*>(wp + w_frag1 * fs + static_cast<int64_t>(pbase) * (kFragBytes / 2));
                     const Pack<uint32_t, 2>* __restrict__ tb = second ? table + 2 * (nst + 4) : table;
                     const int nst_s = second ? hg : nst;
-                    sk_u32x4 wa[4][2];
+                    sk_u32x4 wa[4][NF];
                     sk_u32x4 wb[2][TT];
                     uint32_t bo[4];
                     // Requests the weight fragments of the step described by table entry `e` and notes where its activations are.
                     auto req_a = [&](int slot, const Pack<uint32_t, 2>& e) __attribute__((always_inline)) {
                         const uint32_t voff = lane16 + e.v[0];
                         wa[slot][0] = *reinterpret_cast<const sk_u32x4*>(pa0 + voff);
-                        wa[slot][1] = *reinterpret_cast<const sk_u32x4*>(pa1 + voff);
+                        if constexpr (!NARROW) wa[slot][1] = *reinterpret_cast<const sk_u32x4*>(pa1 + voff);
                         bo[slot] = e.v[1];
                     };
                     auto read_b = [&](int slot, uint32_t boff) __attribute__((always_inline)) {
@@ -552,7 +559,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
 #pragma unroll
                         for (int t = 0; t < TT; ++t) {
                             acc[t][0] = sk_mfma<F16>(wa[sa][0], wb[sb][t], acc[t][0]);
-                            acc[t][1] = sk_mfma<F16>(wa[sa][1], wb[sb][t], acc[t][1]);
+                            if constexpr (!NARROW) acc[t][1] = sk_mfma<F16>(wa[sa][1], wb[sb][t], acc[t][1]);
                         }
                     };
                     req_a(0, tb[0]);
@@ -572,6 +579,20 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     // would run dry while they issue.
                     auto step_order = [&]() __attribute__((always_inline)) {
                         constexpr int kMfma = 0x008, kValu = 0x002, kVmemRead = 0x020, kDsRead = 0x100;
+                        if constexpr (NARROW) {
+                            __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(kValu, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(kVmemRead, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(kDsRead, 2, 0);
+                            __builtin_amdgcn_sched_group_barrier(kValu, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(kDsRead, 2, 0);
+                            __builtin_amdgcn_sched_group_barrier(kValu, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+                            __builtin_amdgcn_sched_barrier(0);
+                            return;
+                        }
                         __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
                         __builtin_amdgcn_sched_group_barrier(kValu, 1, 0);
                         __builtin_amdgcn_sched_group_barrier(kVmemRead, 2, 0);
@@ -633,7 +654,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             }
 
             // ---- epilogue. Accumulator register 4 q + k of fragment f holds channel 32 f + 8 q + 4 half + k of the lane's
-            // pixel: a "quad" (f, q) is the lane's half of channel group j8 = 8 oc_tile + 4 f + q. One quad at a time: its bias
+            // pixel: a "quad" (f, q) is the lane's half of channel group j8 = TG oc_tile + 4 f + q. One quad at a time: its bias
             // and membrane (4 + 4 registers) live across its timesteps; a lane's addresses are 32-bit offsets from uniform bases.
             if constexpr (!SK) {
                 if (wave < 4) __builtin_amdgcn_s_setprio(0);
@@ -1013,10 +1034,10 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                         const unsigned char* res_ptr[TT];
 #pragma unroll
                         for (int tw = 0; tw < TT; ++tw)
-                            res_ptr[tw] = static_cast<const unsigned char*>(sk_kernarg_ptr(kResTable, min(tw, t_count - 1))) + static_cast<int64_t>(oc_e) * 8 * po;
+                            res_ptr[tw] = static_cast<const unsigned char*>(sk_kernarg_ptr(kResTable, min(tw, t_count - 1))) + static_cast<int64_t>(oc_e) * TG * po;
                         auto req_res = [&](auto fq_tag) __attribute__((always_inline)) {
                             constexpr int fq = decltype(fq_tag)::value;
-                            const uint32_t off = lane_bits + static_cast<uint32_t>(min(fq, g.C8out - 1 - oc_e * 8) * po);
+                            const uint32_t off = lane_bits + static_cast<uint32_t>(min(fq, g.C8out - 1 - oc_e * TG) * po);
 #pragma unroll
                             for (int tw = 0; tw < TT; ++tw) rb[fq][tw] = res_ptr[tw][off];
                         };
@@ -1036,8 +1057,8 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
 #pragma unroll
                         for (int tw = 0; tw < TT; ++tw)
 #pragma unroll
-                            for (int k = 0; k < 4; ++k) xq[tw][k] = acc[tw][fq >> 2][4 * (fq & 3) + k];
-                        fast_quad(oc_e * 8 + fq, xq, rb[fq], with_res);
+                            for (int k = 0; k < 4; ++k) xq[tw][k] = acc[tw][(fq >> 2) % NF][4 * (fq & 3) + k];
+                        fast_quad(oc_e * TG + fq, xq, rb[fq], with_res);
                     };
                     do_quad(std::integral_constant<int, 0>{});
                     do_quad(std::integral_constant<int, 1>{});
@@ -1054,7 +1075,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                         float xq[TT][4];
 #define SNNF_SPK_COPY_QUAD(F, Q)                                          \
     _Pragma("unroll") for (int tw = 0; tw < TT; ++tw)                     \
-        _Pragma("unroll") for (int k = 0; k < 4; ++k) xq[tw][k] = acc[tw][F][4 * (Q) + k]
+        _Pragma("unroll") for (int k = 0; k < 4; ++k) xq[tw][k] = acc[tw][(F) % NF][4 * (Q) + k]
                         switch (fq) {
                             case 0: SNNF_SPK_COPY_QUAD(0, 0); break;
                             case 1: SNNF_SPK_COPY_QUAD(0, 1); break;
@@ -1066,7 +1087,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                             default: SNNF_SPK_COPY_QUAD(1, 3); break;
                         }
 #undef SNNF_SPK_COPY_QUAD
-                        general_quad(oc_e * 8 + fq, xq);
+                        general_quad(oc_e * TG + fq, xq);
                     }
                 }
             } else {
@@ -1074,10 +1095,10 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                 float* __restrict__ part = reinterpret_cast<float*>(lds + kSpkHeaderBytes);      // [wave][e 0..3][tw][lane][4]
 #define SNNF_SPK_PARK_QUAD(E, F)                                                                                                 \
     _Pragma("unroll") for (int tw = 0; tw < TT; ++tw) {                                                                          \
-        const sk_f32x4 four = {acc[tw][F][4 * (E)], acc[tw][F][4 * (E) + 1], acc[tw][F][4 * (E) + 2], acc[tw][F][4 * (E) + 3]};  \
+        const sk_f32x4 four = {acc[tw][(F) % NF][4 * (E)], acc[tw][(F) % NF][4 * (E) + 1], acc[tw][(F) % NF][4 * (E) + 2], acc[tw][(F) % NF][4 * (E) + 3]};  \
         *reinterpret_cast<sk_f32x4*>(part + (((wave * 4 + (E)) * TT + tw) * 64 + lane) * 4) = four;                             \
     }
-                if (WK == 2) {
+                if (!NARROW && WK == 2) {
                     // Two waves per tile: wave wk finishes the four quads of fragment wk, which sit in the first half of its
                     // accumulators (the second wave computes the fragments in swapped places). It hands its sums of the other
                     // fragment to its partner and adds the partner's sums to its own, which never leave their registers: one exchange.
@@ -1089,7 +1110,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     if constexpr (FAST) {   // the residual bytes of the first quad travel while the workgroup meets
                         if (g.res_layout >= 0 && TT > 1) {
 #pragma unroll
-                            for (int tw = 0; tw < TT; ++tw) rb[tw] = fast_res(min(tw, t_count - 1), oc_e * 8 + 4 * wk);
+                            for (int tw = 0; tw < TT; ++tw) rb[tw] = fast_res(min(tw, t_count - 1), oc_e * TG + 4 * wk);
                         }
                     }
                     __syncthreads();
@@ -1097,7 +1118,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     int lane_x = lane;                   // opaque: the addresses below are computed here, not ahead of the matrix loop
                     asm volatile("" : "+v"(lane_x));
                     for (int e = 0; e < 4; ++e) {
-                        const int j8 = oc_e * 8 + 4 * wk + e;
+                        const int j8 = oc_e * TG + 4 * wk + e;
                         sk_f32x4 theirs[TT];
 #pragma unroll
                         for (int tw = 0; tw < TT; ++tw)
@@ -1105,7 +1126,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                         float xq[TT][4];
 #define SNNF_SPK_COPY_QUAD(F, Q)                                          \
     _Pragma("unroll") for (int tw = 0; tw < TT; ++tw)                     \
-        _Pragma("unroll") for (int k = 0; k < 4; ++k) xq[tw][k] = acc[tw][F][4 * (Q) + k]
+        _Pragma("unroll") for (int k = 0; k < 4; ++k) xq[tw][k] = acc[tw][(F) % NF][4 * (Q) + k]
                         switch (e) {
                             case 0: SNNF_SPK_COPY_QUAD(0, 0); break;
                             case 1: SNNF_SPK_COPY_QUAD(0, 1); break;
@@ -1131,7 +1152,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                 // More waves per tile: four quads per round for all TT timesteps; quad 4 r + e of round r is finished by wave
                 // (4 r + e) mod WK of the tile, which adds the WK partial sums in a fixed order and then runs that quad's timesteps
                 // like the unsplit kernel.
-                for (int r = 0; r < 2; ++r) {
+                for (int r = 0; r < NF; ++r) {
                     __syncthreads();   // the previous round's sums are consumed (first round: every wave is done with its staging region)
                     if (r == 0) {
                         SNNF_SPK_PARK_QUAD(0, 0) SNNF_SPK_PARK_QUAD(1, 0) SNNF_SPK_PARK_QUAD(2, 0) SNNF_SPK_PARK_QUAD(3, 0)
@@ -1147,12 +1168,12 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     if constexpr (FAST) {
                         if (e_first < 4 && g.res_layout >= 0 && TT > 1) {
 #pragma unroll
-                            for (int tw = 0; tw < TT; ++tw) rb[tw] = fast_res(min(tw, t_count - 1), oc_e * 8 + 4 * r + e_first);
+                            for (int tw = 0; tw < TT; ++tw) rb[tw] = fast_res(min(tw, t_count - 1), oc_e * TG + 4 * r + e_first);
                         }
                     }
                     __syncthreads();
                     for (int e_own = e_first; e_own < 4; e_own += WK) {
-                        const int j8 = oc_e * 8 + 4 * r + e_own;
+                        const int j8 = oc_e * TG + 4 * r + e_own;
                         float xq[TT][4];
                         {
                             // The partial sums of the tile's waves, all timesteps of a wave (of two waves) in flight together (WK is a power
@@ -1208,6 +1229,10 @@ int launch_conv_spk_variant(const SpkLaunch& L) {
                                                                         static_cast<unsigned char*>(L.out), L.v_out, L.lif, L.wpacked2, L.bias2);
         return check_launch("snnf_conv_lif_blocked");
     };
+    if constexpr (TT == 4) {
+        if (L.g.narrow)
+            return L.fast_epilogue ? run(conv_spk_kernel<XT, 4, IN, true, true, false, false, true>) : run(conv_spk_kernel<XT, 4, IN, true, false, false, false, true>);
+    }
     if (L.fast_epilogue) return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, IN, true, true>) : run(conv_spk_kernel<XT, TT, IN, false, true>);
     return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, IN, true, false>) : run(conv_spk_kernel<XT, TT, IN, false, false>);
 }
@@ -1221,6 +1246,7 @@ int launch_conv_spk_pooled(const SpkLaunch& L, int tt) {
                                                                         static_cast<unsigned char*>(L.out), L.v_out, L.lif, L.wpacked2, L.bias2);
         return check_launch("snnf_conv_lif_blocked_avgpool");
     };
+    if (tt == 4 && L.g.narrow) return run(conv_spk_kernel<XT, 4, IN, true, true, false, true, true>);
     if (tt == 4) return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, 4, IN, true, true, false, true>) : run(conv_spk_kernel<XT, 4, IN, false, true, false, true>);
     return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, 1, IN, true, true, false, true>) : run(conv_spk_kernel<XT, 1, IN, false, true, false, true>);
 }
@@ -1250,6 +1276,7 @@ int launch_conv_spk_shortcut(const SpkLaunch& L) {
         return check_launch("snnf_conv_lif_blocked_shortcut");
     };
     constexpr int B = SNNF_LAYOUT_BITS;
+    if (L.g.narrow) return L.fast_epilogue ? run(conv_spk_kernel<XT, 4, B, true, true, true, false, true>) : run(conv_spk_kernel<XT, 4, B, true, false, true, false, true>);
     if (L.fast_epilogue) return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, 4, B, true, true, true>) : run(conv_spk_kernel<XT, 4, B, false, true, true>);
     return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, 4, B, true, false, true>) : run(conv_spk_kernel<XT, 4, B, false, false, true>);
 }
