@@ -112,3 +112,19 @@ def test_convolution_without_a_neuron(snnf_lib, Cin, Cout, H, W, k, s, T, N, res
     assert (CB.last_conv_plan().get("route") == "c8") == want, CB.last_conv_plan()
     ref = torch.stack([torch.nn.functional.conv2d(x.double(), w.double(), b.double(), s, p) + (rs[t].double() if residual else 0) for t, x in enumerate(xs)])
     assert torch.all((out.double().cpu() - ref).abs() <= ref.abs() * 2.0 ** -8 + 1e-4)
+
+
+@pytest.mark.parametrize("Cin,Cout,H,W,N,grid", [(16, 64, 8, 8, 3, 6), (16, 64, 40, 40, 46, 256), (16, 64, 56, 56, 16, 196)])
+def test_tiles_spread_over_compute_units(snnf_lib, Cin, Cout, H, W, N, grid):
+    """Six tiles on six workgroups; 2300 tiles in two rounds of 256 workgroups (144 full ones would leave 112 units idle); 1568 in
+    one round of 196 full workgroups."""
+    from triton_snn_fusion_amd.runtime import hip_blocked_backend as B
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the shapes sit at the edges of 256 compute units")
+    g = gen(4800 + N)
+    x = torch.stack([spikes((N, Cin, H, W), 0.25, g) for _ in range(4)])
+    w, b = q(torch.randn(Cout, Cin, 3, 3, generator=g) * 2.0 * (2.0 / (Cin * 9)) ** 0.5, BF16), q(torch.randn(Cout, generator=g) * 0.1, BF16)
+    ref = O.temporal_conv_lif(list(x), w, b, torch.tensor(0.0), (1, 1), (1, 1), (1, 1), 1, *LIF)
+    out, v = B.conv_lif_blocked(B.from_dense(dev(x, BF16), B.BITS), dev(w, BF16), dev(b, BF16), [1, 1], [1, 1], LIF, out_layout=B.BITS, want_v=True)
+    assert int(B.last_conv_plan()["grid"]) == grid, B.last_conv_plan()
+    check(B.to_dense(out), v, ref, what=f"{Cin}->{Cout} {H}x{W} x {N}")

@@ -424,7 +424,11 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     const int resident = cus * ((tt == 1 && 2 * (lds_bytes + 1024) <= kMaxLds) ? 2 : 1);
     const int blocks = (g.n_items + tiles_per_block - 1) / tiles_per_block;
     g.iters = (blocks + resident - 1) / resident;
-    const int grid = (blocks + g.iters - 1) / g.iters;
+    int grid = (blocks + g.iters - 1) / g.iters;
+    // Workgroups full of waves that leave a quarter of the compute units idle in every round, or half of them in the only one: a workgroup
+    // on every unit, some of its waves idle in the last round (128 -> 128 at 28^2 x 40, 140 workgroups 55.5 us, 256 workgroups 45.1; 64 -> 64
+    // at 24^2, one image, 18 and 36 workgroups 8.5 / 7.5). Fuller rounds stay even: 256 -> 256 at 14^2 x 128, 224 workgroups 100 us, 256 105.
+    if (g.iters > 1 ? grid * 4 < resident * 3 : grid * 2 <= cus) grid = std::min(g.n_items, g.iters > 1 ? resident : cus);
     g.d_ppx = make_fast_div(g.PR * g.PC);
     g.d_PC = make_fast_div(g.PC);
     g.d_region = make_fast_div(g.region);
