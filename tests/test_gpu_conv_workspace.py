@@ -128,3 +128,17 @@ def test_tiles_spread_over_compute_units(snnf_lib, Cin, Cout, H, W, N, grid):
     out, v = B.conv_lif_blocked(B.from_dense(dev(x, BF16), B.BITS), dev(w, BF16), dev(b, BF16), [1, 1], [1, 1], LIF, out_layout=B.BITS, want_v=True)
     assert int(B.last_conv_plan()["grid"]) == grid, B.last_conv_plan()
     check(B.to_dense(out), v, ref, what=f"{Cin}->{Cout} {H}x{W} x {N}")
+
+
+@pytest.mark.parametrize("T,out", [(1, "bits"), (2, "bits"), (1, "c8"), (2, "nchw")])
+def test_narrow_tiles_of_short_windows(snnf_lib, T, out):
+    """One and two timesteps on tiles of 32 channels, straight-line and general epilogue, a last tile of 8 channels."""
+    from triton_snn_fusion_amd.runtime import hip_blocked_backend as B
+    layout = {"bits": B.BITS, "c8": B.C8, "nchw": B.NCHW}[out]
+    g = gen(4900 + T)
+    x = torch.stack([spikes((2, 128, 9, 7), 0.25, g) for _ in range(T)])
+    w, b = q(torch.randn(40, 128, 3, 3, generator=g) * 2.0 * (2.0 / 1152) ** 0.5, BF16), q(torch.randn(40, generator=g) * 0.1, BF16)
+    ref = O.temporal_conv_lif(list(x), w, b, torch.tensor(0.0), (1, 1), (1, 1), (1, 1), 1, *LIF)
+    got, v = B.conv_lif_blocked(B.from_dense(dev(x, BF16), B.BITS), dev(w, BF16), dev(b, BF16), [1, 1], [1, 1], LIF, out_layout=layout, want_v=True)
+    assert int(B.last_conv_plan()["oc_tiles"]) == 2, B.last_conv_plan()
+    check(B.to_dense(got), v, ref, what=f"T={T} {out}")

@@ -411,7 +411,7 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     g.wk_log2 = wk_log2;
     // Tiles of 32 channels where even those fit one round of waves: 256 -> 256 at 14^2 x 4 (112 tiles of 64 channels on eight waves each)
     // 13.9 -> 10.0 us, 512 -> 512 at 7^2 x 8 19.8 -> 13.9, at 4^2 x 32 22.2 -> 17.6. At twice the tiles they would make a second round.
-    if (tt == 4 && wk_log2 > 0 && !tuned_split && Cout > 32 && static_cast<int64_t>(g.n_patches) * ((Cout + 31) / 32) << wk_log2 <= static_cast<int64_t>(cus) * kSpkWaves) {
+    if ((tt == 4 || (!pool2 && x_layout != SNNF_LAYOUT_NCHW)) && wk_log2 > 0 && !tuned_split && Cout > 32 && static_cast<int64_t>(g.n_patches) * ((Cout + 31) / 32) << wk_log2 <= static_cast<int64_t>(cus) * kSpkWaves) {
         g.narrow = 1;
         oc_tiles = (Cout + 31) / 32;
         g.n_items = g.n_patches * oc_tiles;

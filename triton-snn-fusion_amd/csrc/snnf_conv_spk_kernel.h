@@ -146,7 +146,7 @@ __device__ __forceinline__ sk_u32x4 sk_expand_bits(uint32_t byte) {
 
 // NARROW: tiles of 32 output channels (one weight fragment) for launches of few tiles that share K among waves: twice the workgroups,
 // each with half the matrix instructions and half the weights in its chain of steps, which is what such a launch lasts (512 -> 512 at
-// 4^2, one image: 288 steps on eight waves, 19.1 -> 12.6 us; 64 -> 64 at 56^2 11.7 -> 8.7 us).
+// 4^2, one image: 288 steps on eight waves, 19.1 -> 12.6 us; 64 -> 64 at 56^2 11.7 -> 8.7 us; of one timestep 512 -> 512 at 4^2 10.8 -> 7.5).
 template <typename XT, int TT, int IN, bool SK, bool FAST, bool SC = false, bool POOL = false, bool NARROW = false>
 __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_eu(TT == 1 ? 4 : 2, TT == 1 ? 4 : 2))) void conv_spk_kernel(
     const StepPtrs xs, const StepPtrs residuals, const SpkGeom g, const uint16_t* __restrict__ wpacked,
@@ -176,7 +176,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
     static_assert(!SC || (IN == SNNF_LAYOUT_BITS && TT == 4), "the shortcut variants take bit-packed inputs, four timesteps at a time");
     static_assert(!POOL || (FAST && (TT == 4 || TT == 1)), "the pooled output belongs to the straight-line epilogue of four steps");
     static_assert(IN != SNNF_LAYOUT_NCHW || TT == 1, "a dense input is one frame for all timesteps");
-    static_assert(!NARROW || (SK && TT == 4), "narrow tiles are for launches that share K among waves");
+    static_assert(!NARROW || (SK && IN != SNNF_LAYOUT_NCHW), "narrow tiles are for launches that share K among waves");
     constexpr int NF = NARROW ? 1 : 2;         // 32-channel weight fragments of a tile
     constexpr int TG = 4 * NF;                 // channel groups of 8 of a tile
     constexpr bool F16 = dtype_of<XT>::value == SNNF_F16;
@@ -583,13 +583,17 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                             __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
                             __builtin_amdgcn_sched_group_barrier(kValu, 1, 0);
                             __builtin_amdgcn_sched_group_barrier(kVmemRead, 1, 0);
-                            __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
-                            __builtin_amdgcn_sched_group_barrier(kDsRead, 2, 0);
-                            __builtin_amdgcn_sched_group_barrier(kValu, 1, 0);
-                            __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
-                            __builtin_amdgcn_sched_group_barrier(kDsRead, 2, 0);
-                            __builtin_amdgcn_sched_group_barrier(kValu, 1, 0);
-                            __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+                            if constexpr (TT >= 2) {
+                                __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+                                __builtin_amdgcn_sched_group_barrier(kDsRead, 2, 0);
+                                __builtin_amdgcn_sched_group_barrier(kValu, 1, 0);
+                            }
+                            if constexpr (TT >= 4) {
+                                __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+                                __builtin_amdgcn_sched_group_barrier(kDsRead, 2, 0);
+                                __builtin_amdgcn_sched_group_barrier(kValu, 1, 0);
+                                __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+                            }
                             __builtin_amdgcn_sched_barrier(0);
                             return;
                         }
@@ -1229,10 +1233,8 @@ int launch_conv_spk_variant(const SpkLaunch& L) {
                                                                         static_cast<unsigned char*>(L.out), L.v_out, L.lif, L.wpacked2, L.bias2);
         return check_launch("snnf_conv_lif_blocked");
     };
-    if constexpr (TT == 4) {
-        if (L.g.narrow)
-            return L.fast_epilogue ? run(conv_spk_kernel<XT, 4, IN, true, true, false, false, true>) : run(conv_spk_kernel<XT, 4, IN, true, false, false, false, true>);
-    }
+    if (L.g.narrow)
+        return L.fast_epilogue ? run(conv_spk_kernel<XT, TT, IN, true, true, false, false, true>) : run(conv_spk_kernel<XT, TT, IN, true, false, false, false, true>);
     if (L.fast_epilogue) return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, IN, true, true>) : run(conv_spk_kernel<XT, TT, IN, false, true>);
     return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, IN, true, false>) : run(conv_spk_kernel<XT, TT, IN, false, false>);
 }
