@@ -109,3 +109,37 @@ def test_weights_of_dead_tensors_are_given_back(hip_ops):
         fired = ref >= 1.0
         assert float((outs[-1] - torch.where(fired, torch.zeros_like(ref), ref)).abs().max()) < 1e-4   # bf16 products are exact, 73 of them added in float32: 73 * 2^-24 * |sum| < 1e-4
         del w, b
+
+
+def _one_step_views(x):
+    """The one step of `x` ([1, N, ...]) as contiguous tensors whose first stride is not the size of a step: the time axis moved to
+    the front of a batch-first tensor, and every fourth of a sequence of four."""
+    other = torch.full_like(x, 7.0)
+    views = [torch.stack([x[0]], dim=1).transpose(0, 1), torch.cat([x, other, other, other])[::4]]
+    for v in views:
+        assert v.shape == x.shape and v.is_contiguous() and v.stride(0) != x.stride(0)
+    return views
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_one_step_whose_first_stride_means_nothing(hip_ops, dtype):
+    """A size-1 time axis may have any stride in a contiguous tensor: no size of anything follows from it."""
+    from triton_snn_fusion_amd.runtime import hip_convlif_backend as CB
+    S = torch.ops.snn_custom
+    g, spikes, weights = _operands(dtype)
+    zero = torch.zeros((), device=DEV)
+    seq, rows = torch.randn(1, 3, 16, 5, 8, generator=g).to(DEV, dtype), spikes(1, 5, 40)
+    wt, bt, wl, wc, bc = weights(11, 16), weights(11), weights(33, 40), weights(24, 16, 3, 3), weights(24)
+    calls = {
+        "scan": (seq, lambda x: S.fused_temporal_lif_state(x, zero, *LIF)),
+        "scan from a state": (seq, lambda x: S.fused_temporal_lif_state(x, seq[0] * 0.5, *LIF)),
+        "tail": (seq, lambda x: S.fused_temporal_lif_avgpool_linear(x, zero, wt, bt, *LIF)),
+        "linear": (rows, lambda x: S.fused_temporal_linear_lif_state_packed(x, wl, None, zero, *LIF)),
+        "convolution without a neuron": (seq, lambda x: (CB.run_hip_conv_bias_frames(x, wc, bc, [1, 1], [1, 1]),)),
+        "convolution": (seq, lambda x: S.fused_temporal_conv_lif_state([x[0]], wc, bc, zero, [1, 1], [1, 1], [1, 1], 1, *LIF)),
+    }
+    for name, (x, call) in calls.items():
+        want = call(x)
+        for view in [x] + _one_step_views(x):
+            for _ in range(2):
+                assert all(torch.equal(a, b) for a, b in zip(call(view), want)), (name, view.stride())

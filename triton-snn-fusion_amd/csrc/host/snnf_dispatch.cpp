@@ -414,6 +414,8 @@ bool step_call(const Call& c, Attempt& key, Pair* out) {
     return true;
 }
 
+// Where the T steps of a contiguous tensor start. Of a single step `stride(0)` says nothing: a size-1 dimension of a contiguous
+// tensor may have any stride, so the size of a step is always the product of its extents.
 void packed_steps(const Tensor& x, int64_t T, const void** steps) {
     const char* base = static_cast<const char*>(x.data_ptr());
     const int64_t bytes = x.stride(0) * static_cast<int64_t>(x.element_size());
@@ -431,7 +433,7 @@ bool scan_call(const Call& c, Attempt& key, Pair* out) {
     const Membrane m = add_membrane(key, x, v, shape);
     add_lif(key, c, 2);
     if (!key.known()) return false;
-    const int64_t T = x.size(0), n = x.stride(0);
+    const int64_t T = x.size(0), n = c10::multiply_integers(shape);
     const void* steps[kMaxSteps];
     packed_steps(x, T, steps);
     const Lif lif = c.lif(2);
