@@ -143,3 +143,31 @@ def test_one_step_whose_first_stride_means_nothing(hip_ops, dtype):
         for view in [x] + _one_step_views(x):
             for _ in range(2):
                 assert all(torch.equal(a, b) for a, b in zip(call(view), want)), (name, view.stride())
+
+
+@pytest.mark.parametrize("strict", [False, True])
+def test_a_host_operand_next_to_gpu_operands_stays_off_the_kernels(hip_ops, strict):
+    """One GPU operand brings a call to the dispatch; an input in host memory runs on the eager operators, or is refused as it is
+    without the dispatch, whether or not the same call on the GPU is known."""
+    hip_ops.configure_fused_op("hip", strict_triton=strict)
+    S = torch.ops.snn_custom
+    g = gen(8)
+    host = torch.randn(3, 16, 5, 8, generator=g)
+    device_zero, device_v = torch.zeros((), device=DEV), torch.rand(3, 16, 5, 8, generator=g).to(DEV)
+    S.lif_forward_state(host.to(DEV), device_v, *LIF)
+    want = hip_ops.lif_forward_state_torch(host, device_zero, *LIF)       # a state on another device: the step starts from zeros
+    for state in (device_zero, device_v):
+        got = S.lif_forward_state(host, state, *LIF)
+        assert all(a.device.type == "cpu" and torch.equal(a, b) for a, b in zip(got, want))
+    xs = [(torch.rand(2, 16, 5, 8, generator=g) < 0.3).float() for _ in range(4)]
+    w, b = torch.randn(24, 16, 3, 3, generator=g), torch.randn(24, generator=g)
+    args = ([1, 1], [1, 1], [1, 1], 1, *LIF)
+    for _ in range(2):
+        S.fused_temporal_conv_lif_state([x.to(DEV) for x in xs], w.to(DEV), b.to(DEV), device_zero, *args)
+        S.fused_temporal_lif_state(torch.stack(xs).to(DEV), device_zero, *LIF)
+    hip_ops.reset_fused_op_call_stats()
+    hip_ops.configure_fused_op("hip")
+    spikes, v = S.fused_temporal_lif_state(torch.stack(xs), device_zero, *LIF)
+    assert spikes.device.type == v.device.type == "cpu"
+    assert torch.equal(S.fused_temporal_conv_lif_state(xs, w, b, device_zero, *args)[0], S.fused_temporal_conv_lif_state(xs, w, b, torch.zeros(()), *args)[0])
+    assert hip_ops.get_fused_op_call_stats()["triton"] == 0

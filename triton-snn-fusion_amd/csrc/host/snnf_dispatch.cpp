@@ -378,8 +378,6 @@ void call_python(const c10::OperatorHandle& op, Stack* stack, const Key* learn) 
     torch::jit::push(*stack, std::move(first), std::move(second));
 }
 
-bool is_gpu(const IValue& v) { return v.isTensor() && v.toTensor().defined() && v.toTensor().is_cuda(); }
-
 struct Call {
     Stack* stack;
     size_t base;
@@ -399,7 +397,9 @@ bool step_call(const Call& c, Attempt& key, Pair* out) {
     const Tensor x = c.at(0).toTensor(), v = c.at(1).toTensor();
     const Lif lif = c.lif(2);
     int code;
-    if (!dtype_code(x.scalar_type(), &code) || !x.is_contiguous() || x.numel() == 0 || lif.tau == 0.0) return false;
+    // One GPU operand is enough for a call to arrive here: a state on the GPU does not make the input one.
+    key.tensor(x);
+    if (!key.plain || !dtype_code(x.scalar_type(), &code) || x.numel() == 0 || lif.tau == 0.0) return false;
     const Membrane m = membrane_of(x, v);
     // A state of another shape, device or dtype starts from zeros.
     const bool continues = v.dim() != 0 && v.sizes() == x.sizes() && v.device() == x.device() && v.scalar_type() == m.dtype;
