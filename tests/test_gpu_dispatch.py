@@ -171,3 +171,38 @@ def test_a_host_operand_next_to_gpu_operands_stays_off_the_kernels(hip_ops, stri
     assert spikes.device.type == v.device.type == "cpu"
     assert torch.equal(S.fused_temporal_conv_lif_state(xs, w, b, device_zero, *args)[0], S.fused_temporal_conv_lif_state(xs, w, b, torch.zeros(()), *args)[0])
     assert hip_ops.get_fused_op_call_stats()["triton"] == 0
+
+
+def test_inference_weights_of_a_known_signature(hip_ops):
+    """Weights made under inference mode have no version counter, so nothing is packed for them: the operators fall back (and raise in
+    strict mode), the internal layouts refuse, whether or not the call is known with ordinary weights."""
+    from triton_snn_fusion_amd.runtime import hip_blocked_backend as B
+    S = torch.ops.snn_custom
+    _, spikes, weights = _operands(torch.bfloat16)
+    zero = torch.zeros((), device=DEV)
+    xs = [spikes(2, 24, 7, 9) for _ in range(4)]
+    bits = B.from_dense(torch.stack(xs))
+    w, b = weights(40, 24, 3, 3), weights(40)
+    with torch.inference_mode():
+        wi, bi = w.clone(), b.clone()
+    rest = (zero, [1, 1], [1, 1], [1, 1], 1, *LIF)
+    for _ in range(2):
+        S.fused_temporal_conv_lif_state(xs, w, b, *rest)
+        B.conv_lif_blocked(bits, w, b, [1, 1], [1, 1], LIF[:3])
+    for weight, bias in ((wi, bi), (wi, b), (w, bi)):
+        for _ in range(2):
+            hip_ops.configure_fused_op("hip", strict_triton=True)
+            with pytest.raises(RuntimeError, match="Inference tensors"):
+                S.fused_temporal_conv_lif_state(xs, weight, bias, *rest)
+            with pytest.raises(RuntimeError, match="Inference tensors"):
+                B.conv_lif_blocked(bits, weight, bias, [1, 1], [1, 1], LIF[:3])
+            hip_ops.configure_fused_op("hip")
+            hip_ops.reset_fused_op_call_stats()
+            got = S.fused_temporal_conv_lif_state(xs, weight, bias, *rest)
+            want = hip_ops.fused_temporal_conv_lif_state_torch(xs, weight, bias, *rest)
+            assert all(torch.equal(a, c) for a, c in zip(got, want))
+            assert hip_ops.get_fused_op_call_stats()["fallback"] == 1
+    with torch.inference_mode():        # ordinary weights, activations that are inference tensors
+        for _ in range(2):
+            got = S.fused_temporal_conv_lif_state([x.clone() for x in xs], w, b, *rest)
+        assert hip_ops.get_fused_op_call_stats()["triton"] == 2

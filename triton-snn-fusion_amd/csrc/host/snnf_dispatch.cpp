@@ -63,13 +63,14 @@ struct Key {
         add(t.dim());
         for (int64_t d : t.sizes()) add(d);
     }
-    // A GPU operand that the kernels read in place.
+    // A GPU operand that the kernels read in place. Inference tensors have signatures of their own: as weights they have no version by
+    // which a packed copy could be known to be current, and the Python implementations refuse to pack them.
     void tensor(const Tensor& t) {
         if (!t.defined() || !t.is_cuda() || !t.is_contiguous()) {
             plain = false;
             return;
         }
-        add((static_cast<int64_t>(t.scalar_type()) << 8) | t.device().index());
+        add((static_cast<int64_t>(t.scalar_type()) << 16) | (t.is_inference() ? 1 << 8 : 0) | t.device().index());
         sizes(t);
     }
     bool operator==(const Key& o) const { return n == o.n && std::memcmp(v.data(), o.v.data(), n * sizeof(int64_t)) == 0; }
@@ -162,7 +163,7 @@ std::list<WeightKey> g_weight_ages;        // most recently used in front
 py::object* g_pack = nullptr;              // _packed_weight(weight, bias, dtype)
 py::object* g_plane = nullptr;             // _plane_matrix(weight, bias, H, W, ph, pw)
 
-int64_t version_of(const Tensor& t) { return t.is_inference() ? 0 : static_cast<int64_t>(t._version()); }
+int64_t version_of(const Tensor& t) { return static_cast<int64_t>(t._version()); }
 
 // Tensors that leave the table are released by the caller after the mutex: freeing one can need the interpreter lock.
 using Released = std::vector<Tensor>;
