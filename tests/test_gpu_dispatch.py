@@ -206,3 +206,56 @@ def test_inference_weights_of_a_known_signature(hip_ops):
         for _ in range(2):
             got = S.fused_temporal_conv_lif_state([x.clone() for x in xs], w, b, *rest)
         assert hip_ops.get_fused_op_call_stats()["triton"] == 2
+
+
+@pytest.mark.parametrize("error", [torch.OutOfMemoryError, "SnnfError", KeyboardInterrupt])
+def test_what_a_known_call_throws(hip_ops, monkeypatch, error):
+    """An error on the native route (here: the weight cannot be packed) is answered by the Python implementation: the type of the
+    exception, the counted fallback and the eager result are what they are without the dispatch. An interrupt passes through."""
+    from triton_snn_fusion_amd import _dispatch, _lib
+    from triton_snn_fusion_amd.runtime import hip_blocked_backend as B, hip_convlif_backend as CB, hip_temporal_linear_lif_backend as NB
+    S = torch.ops.snn_custom
+    _, spikes, weights = _operands(torch.bfloat16)
+    zero = torch.zeros((), device=DEV)
+    xs = [spikes(2, 24, 7, 9) for _ in range(4)]
+    bits = B.from_dense(torch.stack(xs))
+    w, b = weights(40, 24, 3, 3), weights(40)
+    conv = lambda: S.fused_temporal_conv_lif_state(xs, w, b, zero, [1, 1], [1, 1], [1, 1], 1, *LIF)
+    blocked = lambda: B.conv_lif_blocked(bits, w, b, [1, 1], [1, 1], LIF[:3], want_v=True)
+    bias = lambda: CB.run_hip_conv_bias_frames(torch.stack(xs), w, b, [1, 1], [1, 1])
+    want = conv(), blocked()[1], bias()
+    eager = hip_ops.fused_temporal_conv_lif_state_torch(xs, w, b, zero, [1, 1], [1, 1], [1, 1], 1, *LIF)
+    raised = (lambda: _lib.SnnfError("snnf_conv_pack_weight", -1, "planted")) if error == "SnnfError" else lambda: error("planted")
+    kind = _lib.SnnfError if error == "SnnfError" else error
+    tried = []
+
+    def pack(*args):
+        tried.append(args)
+        raise raised()
+
+    native = _dispatch.module()
+    try:
+        native.connect(hip_ops._slow_dispatch, pack, B._plane_matrix,
+                       lambda device, T, M, fin, fout: NB._split_workspace(_lib.lib(), device, T, M, fin, fout))
+        native.forget_weights()
+        if kind is KeyboardInterrupt:
+            for call in (conv, blocked, bias):
+                with pytest.raises(KeyboardInterrupt):
+                    call()
+            assert len(tried) == 3
+            return
+        got = conv(), blocked()[1], bias()              # the Python implementations pack the weight
+        assert len(tried) == 3 and torch.equal(got[1], want[1]) and torch.equal(got[2], want[2])
+        assert all(torch.equal(a, c) for a, c in zip(got[0], want[0]))
+        for module in (CB, B):
+            monkeypatch.setattr(module, "_packed_weight", pack)
+        for call in (conv, blocked, bias):              # strict
+            with pytest.raises(kind, match="planted"):
+                call()
+        hip_ops.configure_fused_op("hip")
+        hip_ops.reset_fused_op_call_stats()
+        assert all(torch.equal(a, c) for a, c in zip(conv(), eager))
+        stats = hip_ops.get_fused_op_call_stats()
+        assert (stats["total"], stats["triton"], stats["fallback"]) == (1, 0, 1)
+    finally:
+        hip_ops.connect_native_dispatch()

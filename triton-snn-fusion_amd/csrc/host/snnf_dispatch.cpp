@@ -8,8 +8,9 @@
 // judged, refused and counted, and this file remembers a signature that ran natively together with the statistics it
 // added. Later calls of the signature are a hash look-up, two allocations and the C ABI call (measured, batch-1 neuron
 // step: 12.3 -> 5 us per call).
-// A call whose signature is unknown, whose tensors are not plain contiguous GPU tensors, or whose entry point returns an
-// error goes through the Python implementation, which raises or falls back as it always did.
+// A call whose signature is unknown, whose tensors are not plain contiguous GPU tensors, whose entry point returns an error, or
+// that throws on its way (no memory, a weight that cannot be packed) goes through the Python implementation, which raises or
+// falls back as it always did.
 //
 // State: the plan table (bounded; cleared when full), the hit counters, the packed weights of live weight tensors. All under
 // one mutex: operator calls arrive without the interpreter lock and from any thread. The mutex is never held while the
@@ -393,6 +394,20 @@ void add_lif(Key& key, const Call& c, size_t i) {
 
 using Pair = std::pair<Tensor, Tensor>;
 
+// A native route that throws ends there, with nothing handed out: the Python implementation then runs the call, and raises what
+// there is to raise, of the type that it always had, or counts a fallback. Only what is no error (an interrupt) leaves here.
+template <typename Body>
+auto run_native(Body&& body) -> decltype(body()) {
+    try {
+        return body();
+    } catch (py::error_already_set& e) {
+        py::gil_scoped_acquire gil;
+        if (!e.matches(PyExc_Exception)) throw;
+    } catch (const std::exception&) {
+    }
+    return {};
+}
+
 // Each operator builds its signature and, when that is known to run natively, enqueues the kernels and returns true.
 bool step_call(const Call& c, Attempt& key, Pair* out) {
     const Tensor x = c.at(0).toTensor(), v = c.at(1).toTensor();
@@ -655,11 +670,13 @@ void dispatch(const c10::OperatorHandle& op, Stack* stack) {
     bool ran = false;
     if (g_enabled.load(std::memory_order_relaxed)) {
         attempt.add(static_cast<int64_t>(OP));
-        if constexpr (OP == kStep) ran = step_call(c, attempt, &out);      // counts nothing, and its conditions are few: no plan
-        else if constexpr (OP == kScan) ran = scan_call(c, attempt, &out);
-        else if constexpr (OP == kTail) ran = tail_call(c, attempt, &out);
-        else if constexpr (OP == kLinear || OP == kLinearPacked) ran = linear_call(c, attempt, OP == kLinearPacked, &out);
-        else ran = conv_call(c, attempt, OP, &out);
+        ran = run_native([&]() -> bool {
+            if constexpr (OP == kStep) return step_call(c, attempt, &out);      // counts nothing, and its conditions are few: no plan
+            else if constexpr (OP == kScan) return scan_call(c, attempt, &out);
+            else if constexpr (OP == kTail) return tail_call(c, attempt, &out);
+            else if constexpr (OP == kLinear || OP == kLinearPacked) return linear_call(c, attempt, OP == kLinearPacked, &out);
+            else return conv_call(c, attempt, OP, &out);
+        });
     }
     if (!ran) return call_python(op, stack, attempt.worth_learning() ? &attempt : nullptr);
     count(attempt.plan);
@@ -844,10 +861,13 @@ PyObject* guarded(PyObject* (*body)(Args&), PyObject* const* args, Py_ssize_t n,
         return nullptr;
     }
     try {
-        Args a{args, n};
-        return body(a);
-    } catch (const std::exception& e) {
-        PyErr_SetString(PyExc_RuntimeError, e.what());
+        PyObject* answer = run_native([&] {
+            Args a{args, n};
+            return body(a);
+        });
+        return answer != nullptr || PyErr_Occurred() ? answer : none();
+    } catch (py::error_already_set& e) {
+        e.restore();
         return nullptr;
     }
 }

@@ -972,6 +972,12 @@ NATIVE_DISPATCH = (
 )
 
 
+def connect_native_dispatch() -> None:
+    """Hands the Python implementations to the native dispatch: what it does not know, weight packing, workspaces."""
+    _dispatch.connect(_slow_dispatch, _packed_weight, _plane_matrix,
+                      lambda device, T, M, fin, fout: _split_workspace(_lib.lib(), device, T, M, fin, fout))
+
+
 def register_snn_custom_ops() -> None:
     """Defines and implements the `snn_custom` library once per process (a second definition is ignored, like the
     reference's try/except around registration, runtime/snn_custom_ops.py:1964-2076)."""
@@ -994,8 +1000,7 @@ def register_snn_custom_ops() -> None:
     except RuntimeError:
         return
     if native:
-        _dispatch.connect(_slow_dispatch, _packed_weight, _plane_matrix,
-                          lambda device, T, M, fin, fout: _split_workspace(_lib.lib(), device, T, M, fin, fout))
+        connect_native_dispatch()
 
 
 register_snn_custom_ops()
