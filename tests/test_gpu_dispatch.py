@@ -259,3 +259,52 @@ def test_what_a_known_call_throws(hip_ops, monkeypatch, error):
         assert (stats["total"], stats["triton"], stats["fallback"]) == (1, 0, 1)
     finally:
         hip_ops.connect_native_dispatch()
+
+
+def test_other_threads_run_while_a_known_call_allocates_and_launches(hip_ops):
+    """With the interpreter's own switching off, another thread gets on only when a call gives the interpreter lock back."""
+    import sys
+    import threading
+    import time
+    from triton_snn_fusion_amd.runtime import hip_blocked_backend as B, hip_convlif_backend as CB, hip_pool_backend as PB
+    _, spikes, weights = _operands(torch.bfloat16)
+    dense = torch.stack([spikes(2, 24, 8, 8) for _ in range(4)])
+    bits, half = B.from_dense(dense), B.from_dense(torch.stack([spikes(2, 48, 16, 16) for _ in range(4)]))
+    x16 = B.from_dense(torch.stack([spikes(2, 32, 8, 8) for _ in range(4)]))
+    w, b, wsc, bsc, w16, fc = weights(40, 24, 3, 3), weights(40), weights(40, 48, 1, 1), weights(40), weights(40, 32, 3, 3), weights(10, 24)
+    one = [1, 1]
+    calls = {
+        "convolution": lambda: B.conv_lif_blocked(bits, w, b, one, one, LIF[:3]),
+        "with a shortcut": lambda: B.conv_lif_blocked_shortcut(x16, w16, b, one, half, wsc, bsc, [2, 2], LIF[:3]),
+        "with a pool": lambda: B.conv_lif_blocked_avgpool(bits, w, b, one, one, LIF[:3]),
+        "pool": lambda: B.pool_blocked(bits, True, 2, 2, 0),
+        "classifier": lambda: B.spike_pool_linear(bits, fc, None),
+        "convolution without a neuron": lambda: CB.run_hip_conv_bias_frames(dense, w, b, one, one),
+        "dense pool": lambda: PB.run_hip_pool2d(dense, True, 2, 2, 0),
+    }
+    progress, stop = [0], threading.Event()
+
+    def other():
+        while not stop.is_set():
+            progress[0] += 1
+            time.sleep(0)
+
+    interval = sys.getswitchinterval()
+    thread = threading.Thread(target=other, daemon=True)
+    try:
+        thread.start()
+        for name, call in calls.items():
+            kept = [call() for _ in range(3)]              # known, the weight packed; nothing is freed meanwhile
+            sys.setswitchinterval(1000.0)
+            time.sleep(0.02)                               # the other thread's next wait is one without an end
+            before = progress[0]
+            while progress[0] == before and len(kept) < 1000:
+                kept.append(call())
+            after = progress[0]
+            sys.setswitchinterval(interval)
+            torch.cuda.synchronize()
+            assert after > before, name
+    finally:
+        sys.setswitchinterval(interval)
+        stop.set()
+        thread.join()

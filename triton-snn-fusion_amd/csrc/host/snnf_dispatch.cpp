@@ -701,9 +701,9 @@ TORCH_LIBRARY_IMPL(snn_custom, CUDA, m) {
 }
 
 // ------------------------------------------------------------------------------------------------------------------
-// Internal layouts (hip_blocked_backend.py): plain functions, called with the interpreter lock held. Each takes what the Python
-// entry point has in hand and returns the result, or None for a call that is not known: the Python entry point then runs it
-// and, when it ran, calls again with what it learnt in the last argument.
+// Internal layouts (hip_blocked_backend.py): plain functions, called with the interpreter lock held, which they give back while they
+// allocate and launch. Each takes what the Python entry point has in hand and returns the result, or None for a call that is not
+// known: the Python entry point then runs it and, when it ran, calls again with what it learnt in the last argument.
 // ------------------------------------------------------------------------------------------------------------------
 enum Blocked { kBlockedConv = 100, kBlockedShortcut, kBlockedAvgPool, kBlockedPool, kBlockedHead, kDenseConvBias, kDensePool };
 enum Learnt { kRoutePlane = 1, kAllocateV = 2, kReturnV = 4 };     // the last argument; -1: run
@@ -712,6 +712,8 @@ struct Args {
     PyObject* const* v;
     Py_ssize_t n;
     bool fine = true;
+    std::array<Tensor, 8> held;
+    int n_held = 0;
 
     int64_t number(Py_ssize_t i) {
         const long long x = PyLong_AsLongLong(v[i]);
@@ -729,12 +731,14 @@ struct Args {
         }
         return x;
     }
+    // The tensors are held here: the kernels are launched without the interpreter lock.
     const Tensor* tensor(Py_ssize_t i) {
-        if (!THPVariable_Check(v[i])) {
+        if (!THPVariable_Check(v[i]) || n_held == static_cast<int>(held.size())) {
             fine = false;
             return nullptr;
         }
-        return &THPVariable_Unpack(v[i]);
+        held[n_held] = THPVariable_Unpack(v[i]);
+        return &held[n_held++];
     }
     // a pair of numbers, or one number for both
     void pair(Py_ssize_t i, int64_t* a, int64_t* b) {
@@ -820,6 +824,13 @@ Tensor empty_frames(int layout, int64_t T, int64_t N, int64_t C, int64_t H, int6
 int64_t step_bytes(const Tensor& t) { return t.stride(0) * static_cast<int64_t>(t.element_size()); }
 
 PyObject* none() { Py_RETURN_NONE; }
+
+// Runs `body` without the interpreter lock: other Python threads go on while it allocates and launches.
+template <typename Body>
+bool unlocked(Body&& body) {
+    py::gil_scoped_release nogil;
+    return body();
+}
 
 // The answer of a convolution or pool: (output data, channels, Ho, Wo, route, membrane or None).
 PyObject* frames_answer(const Tensor& out, int64_t channels, int64_t ho, int64_t wo, int route, const Tensor& v) {
@@ -908,33 +919,36 @@ PyObject* blocked_conv(Args& a) {
     if (!proceed(key, a, learnt)) return none();
     const int64_t cout = w->size(0), kh = w->size(2), kw = w->size(3);
     const int64_t ho = (x.H + 2 * ph - kh) / sh + 1, wo = (x.W + 2 * pw - kw) / sw + 1;
-    const hipStream_t stream = stream_of(*x.data);
     const int route = key.plan.route;
-    Tensor out = empty_frames(out_layout, x.T, x.N, cout, ho, wo, dtype, *x.data), v;
-    int status;
-    if (route & kRoutePlane) {
-        Tensor matrix, row;
-        plane_matrix(*w, *b, x.H, x.W, ph, pw, &matrix, &row);
-        const int64_t fin = static_cast<int64_t>(x.C) * x.H * x.W, fout = cout * x.H * x.W;
-        const Workspace space = split_workspace(*x.data, stream, x.T, x.N, fin, fout);
-        const bool bits = x.layout == SNNF_LAYOUT_BITS;
-        status = snnf_linear_lif_bits(x.steps, bits ? 1 : 0, x.T, x.N, static_cast<int>(fin), bits ? fin / 8 : fin, code_of(dtype), matrix.data_ptr(),
-                                      row.data_ptr(), static_cast<int>(fout), nullptr, out.data_ptr(), step_bytes(out), nullptr,
-                                      static_cast<float>(lif.v_threshold), static_cast<float>(lif.v_reset), static_cast<float>(lif.tau),
-                                      space.data, space.bytes, stream);
-    } else {
-        const Tensor packed = packed_weight(*w, *b, dtype);
-        const void* rs[kMaxSteps];
-        if (residual) packed_steps(*r, x.T, rs);
-        if (route & kAllocateV) v = empty({x.N, cout, ho, wo}, at::kFloat, *x.data);
-        status = snnf_conv_lif_blocked(x.steps, x.layout, residual ? rs : nullptr, res_layout, x.T, x.N, x.C, x.H, x.W, code_of(dtype),
-                                       packed.data_ptr(), static_cast<int>(cout), static_cast<int>(kh), static_cast<int>(kw),
-                                       static_cast<int>(sh), static_cast<int>(sw), static_cast<int>(ph), static_cast<int>(pw), nullptr,
-                                       out.data_ptr(), out_layout, step_bytes(out), v.defined() ? v.data_ptr() : nullptr, neuron ? 1 : 0,
-                                       static_cast<float>(lif.v_threshold), static_cast<float>(lif.v_reset), static_cast<float>(lif.tau), stream);
-    }
-    if (status != 0) return none();
-    return frames_answer(out, cout, ho, wo, route, route & kReturnV ? v : Tensor());
+    Tensor out, v;
+    const bool ran = unlocked([&] {
+        const hipStream_t stream = stream_of(*x.data);
+        out = empty_frames(out_layout, x.T, x.N, cout, ho, wo, dtype, *x.data);
+        int status;
+        if (route & kRoutePlane) {
+            Tensor matrix, row;
+            plane_matrix(*w, *b, x.H, x.W, ph, pw, &matrix, &row);
+            const int64_t fin = static_cast<int64_t>(x.C) * x.H * x.W, fout = cout * x.H * x.W;
+            const Workspace space = split_workspace(*x.data, stream, x.T, x.N, fin, fout);
+            const bool bits = x.layout == SNNF_LAYOUT_BITS;
+            status = snnf_linear_lif_bits(x.steps, bits ? 1 : 0, x.T, x.N, static_cast<int>(fin), bits ? fin / 8 : fin, code_of(dtype), matrix.data_ptr(),
+                                          row.data_ptr(), static_cast<int>(fout), nullptr, out.data_ptr(), step_bytes(out), nullptr,
+                                          static_cast<float>(lif.v_threshold), static_cast<float>(lif.v_reset), static_cast<float>(lif.tau),
+                                          space.data, space.bytes, stream);
+        } else {
+            const Tensor packed = packed_weight(*w, *b, dtype);
+            const void* rs[kMaxSteps];
+            if (residual) packed_steps(*r, x.T, rs);
+            if (route & kAllocateV) v = empty({x.N, cout, ho, wo}, at::kFloat, *x.data);
+            status = snnf_conv_lif_blocked(x.steps, x.layout, residual ? rs : nullptr, res_layout, x.T, x.N, x.C, x.H, x.W, code_of(dtype),
+                                           packed.data_ptr(), static_cast<int>(cout), static_cast<int>(kh), static_cast<int>(kw),
+                                           static_cast<int>(sh), static_cast<int>(sw), static_cast<int>(ph), static_cast<int>(pw), nullptr,
+                                           out.data_ptr(), out_layout, step_bytes(out), v.defined() ? v.data_ptr() : nullptr, neuron ? 1 : 0,
+                                           static_cast<float>(lif.v_threshold), static_cast<float>(lif.v_reset), static_cast<float>(lif.tau), stream);
+        }
+        return status == 0;
+    });
+    return ran ? frames_answer(out, cout, ho, wo, route, route & kReturnV ? v : Tensor()) : none();
 }
 
 // data, layout, shared, T, N, C, H, W, dtype, weight, bias, padding, lif, shortcut: data, layout, shared, T, N, C, H, W, weight, bias,
@@ -965,17 +979,19 @@ PyObject* blocked_shortcut(Args& a) {
     if (!proceed(key, a, learnt)) return none();
     const int64_t cout = w->size(0);
     const int route = key.plan.route;
-    const Tensor packed = packed_weight(*w, *b, dtype), packed_sc = packed_weight(*sw_, *sb, dtype);
-    Tensor out = empty_frames(out_layout, x.T, x.N, cout, x.H, x.W, dtype, *x.data), v;
-    if (route & kAllocateV) v = empty({x.N, cout, x.H, x.W}, at::kFloat, *x.data);
-    if (snnf_conv_lif_blocked_shortcut(x.steps, s.steps, x.T, x.N, x.C, x.H, x.W, code_of(dtype), packed.data_ptr(), static_cast<int>(cout),
-                                       static_cast<int>(w->size(2)), static_cast<int>(w->size(3)), static_cast<int>(ph), static_cast<int>(pw), s.C,
-                                       s.H, s.W, static_cast<int>(ssh), static_cast<int>(ssw), packed_sc.data_ptr(), nullptr, out.data_ptr(),
-                                       out_layout, step_bytes(out), v.defined() ? v.data_ptr() : nullptr, neuron ? 1 : 0,
-                                       static_cast<float>(lif.v_threshold), static_cast<float>(lif.v_reset), static_cast<float>(lif.tau),
-                                       stream_of(*x.data)) != 0)
-        return none();
-    return frames_answer(out, cout, x.H, x.W, route, route & kReturnV ? v : Tensor());
+    Tensor out, v;
+    const bool ran = unlocked([&] {
+        const Tensor packed = packed_weight(*w, *b, dtype), packed_sc = packed_weight(*sw_, *sb, dtype);
+        out = empty_frames(out_layout, x.T, x.N, cout, x.H, x.W, dtype, *x.data);
+        if (route & kAllocateV) v = empty({x.N, cout, x.H, x.W}, at::kFloat, *x.data);
+        return snnf_conv_lif_blocked_shortcut(x.steps, s.steps, x.T, x.N, x.C, x.H, x.W, code_of(dtype), packed.data_ptr(), static_cast<int>(cout),
+                                              static_cast<int>(w->size(2)), static_cast<int>(w->size(3)), static_cast<int>(ph), static_cast<int>(pw), s.C,
+                                              s.H, s.W, static_cast<int>(ssh), static_cast<int>(ssw), packed_sc.data_ptr(), nullptr, out.data_ptr(),
+                                              out_layout, step_bytes(out), v.defined() ? v.data_ptr() : nullptr, neuron ? 1 : 0,
+                                              static_cast<float>(lif.v_threshold), static_cast<float>(lif.v_reset), static_cast<float>(lif.tau),
+                                              stream_of(*x.data)) == 0;
+    });
+    return ran ? frames_answer(out, cout, x.H, x.W, route, route & kReturnV ? v : Tensor()) : none();
 }
 
 // data, layout, shared, T, N, C, H, W, dtype, weight, bias, stride, padding, lif, want_v, learnt
@@ -1004,16 +1020,18 @@ PyObject* blocked_avgpool(Args& a) {
     const int64_t cout = w->size(0), kh = w->size(2), kw = w->size(3);
     const int64_t ho = (x.H + 2 * ph - kh) / sh + 1, wo = (x.W + 2 * pw - kw) / sw + 1;
     const int route = key.plan.route;
-    const Tensor packed = packed_weight(*w, *b, dtype);
-    Tensor out = empty_frames(SNNF_LAYOUT_C8, x.T, x.N, cout, ho / 2, wo / 2, dtype, *x.data), v;
-    if (route & kAllocateV) v = empty({x.N, cout, ho, wo}, at::kFloat, *x.data);
-    if (snnf_conv_lif_blocked_avgpool(x.steps, x.layout, x.T, x.N, x.C, x.H, x.W, code_of(dtype), packed.data_ptr(), static_cast<int>(cout),
-                                      static_cast<int>(kh), static_cast<int>(kw), static_cast<int>(sh), static_cast<int>(sw), static_cast<int>(ph),
-                                      static_cast<int>(pw), out.data_ptr(), step_bytes(out), v.defined() ? v.data_ptr() : nullptr,
-                                      static_cast<float>(lif.v_threshold), static_cast<float>(lif.v_reset), static_cast<float>(lif.tau),
-                                      stream_of(*x.data)) != 0)
-        return none();
-    return frames_answer(out, cout, ho / 2, wo / 2, route, route & kReturnV ? v : Tensor());
+    Tensor out, v;
+    const bool ran = unlocked([&] {
+        const Tensor packed = packed_weight(*w, *b, dtype);
+        out = empty_frames(SNNF_LAYOUT_C8, x.T, x.N, cout, ho / 2, wo / 2, dtype, *x.data);
+        if (route & kAllocateV) v = empty({x.N, cout, ho, wo}, at::kFloat, *x.data);
+        return snnf_conv_lif_blocked_avgpool(x.steps, x.layout, x.T, x.N, x.C, x.H, x.W, code_of(dtype), packed.data_ptr(), static_cast<int>(cout),
+                                             static_cast<int>(kh), static_cast<int>(kw), static_cast<int>(sh), static_cast<int>(sw), static_cast<int>(ph),
+                                             static_cast<int>(pw), out.data_ptr(), step_bytes(out), v.defined() ? v.data_ptr() : nullptr,
+                                             static_cast<float>(lif.v_threshold), static_cast<float>(lif.v_reset), static_cast<float>(lif.tau),
+                                             stream_of(*x.data)) == 0;
+    });
+    return ran ? frames_answer(out, cout, ho / 2, wo / 2, route, route & kReturnV ? v : Tensor()) : none();
 }
 
 // data, layout, shared, T, N, C, H, W, dtype, kernel, stride, padding, is_max, out layout, learnt
@@ -1027,12 +1045,14 @@ PyObject* blocked_pool(Args& a) {
     for (int64_t v : {static_cast<int64_t>(dtype), k, s, p, is_max, out_layout}) key.add(v);
     if (!proceed(key, a, learnt)) return none();
     const int64_t frames = x.data->size(0), ho = (x.H + 2 * p - k) / s + 1, wo = (x.W + 2 * p - k) / s + 1;
-    Tensor out = empty_frames(static_cast<int>(out_layout), frames, x.N, x.C, ho, wo, dtype, *x.data);
-    if (snnf_pool2d_blocked(x.data->data_ptr(), x.layout, out.data_ptr(), static_cast<int>(out_layout), frames * x.N, x.C, x.H, x.W,
-                            static_cast<int>(k), static_cast<int>(s), static_cast<int>(p), is_max != 0 ? 1 : 0, code_of(dtype),
-                            stream_of(*x.data)) != 0)
-        return none();
-    return frames_answer(out, x.C, ho, wo, 0, Tensor());
+    Tensor out;
+    const bool ran = unlocked([&] {
+        out = empty_frames(static_cast<int>(out_layout), frames, x.N, x.C, ho, wo, dtype, *x.data);
+        return snnf_pool2d_blocked(x.data->data_ptr(), x.layout, out.data_ptr(), static_cast<int>(out_layout), frames * x.N, x.C, x.H, x.W,
+                                   static_cast<int>(k), static_cast<int>(s), static_cast<int>(p), is_max != 0 ? 1 : 0, code_of(dtype),
+                                   stream_of(*x.data)) == 0;
+    });
+    return ran ? frames_answer(out, x.C, ho, wo, 0, Tensor()) : none();
 }
 
 // data, layout, shared, T, N, C, H, W, dtype, weight, bias | None, scale, learnt
@@ -1053,11 +1073,13 @@ PyObject* blocked_head(Args& a) {
     key.add(static_cast<int64_t>(biased));
     if (biased) key.tensor(*b);
     if (!proceed(key, a, learnt)) return none();
-    Tensor out = empty({x.N, w->size(0)}, dtype, *x.data);
-    if (snnf_spike_pool_linear(x.steps, x.T, x.N, x.C, x.H, x.W, w->data_ptr(), biased ? b->data_ptr() : nullptr, static_cast<int>(w->size(0)),
-                               code_of(dtype), out.data_ptr(), static_cast<float>(scale), stream_of(*x.data)) != 0)
-        return none();
-    return THPVariable_Wrap(out);
+    Tensor out;
+    const bool ran = unlocked([&] {
+        out = empty({x.N, w->size(0)}, dtype, *x.data);
+        return snnf_spike_pool_linear(x.steps, x.T, x.N, x.C, x.H, x.W, w->data_ptr(), biased ? b->data_ptr() : nullptr, static_cast<int>(w->size(0)),
+                                      code_of(dtype), out.data_ptr(), static_cast<float>(scale), stream_of(*x.data)) == 0;
+    });
+    return ran ? THPVariable_Wrap(out) : none();
 }
 
 // x [T, N, C, H, W] dense, weight, bias, stride, padding, learnt: the convolution without a neuron
@@ -1077,20 +1099,22 @@ PyObject* dense_conv_bias(Args& a) {
     const int64_t ho = (H + 2 * ph - kh) / sh + 1, wo = (W + 2 * pw - kw) / sw + 1;
     const void* steps[kMaxSteps];
     packed_steps(*x, T, steps);
-    const Tensor packed = packed_weight(*w, *b, x->scalar_type());
-    Tensor out = empty({T, N, cout, ho, wo}, x->scalar_type(), *x);
-    const size_t bytes = snnf_conv_lif_workspace_bytes(static_cast<int>(T), static_cast<int>(N), static_cast<int>(x->size(2)), static_cast<int>(H),
-                                                       static_cast<int>(W), code_of(x->scalar_type()), static_cast<int>(cout), static_cast<int>(kh),
-                                                       static_cast<int>(kw), static_cast<int>(sh), static_cast<int>(sw), static_cast<int>(ph),
-                                                       static_cast<int>(pw), SNNF_F32, 0);
-    Tensor workspace;
-    if (bytes > 0) workspace = empty({static_cast<int64_t>(bytes)}, at::kByte, *x);
-    if (snnf_conv_bias_ws(steps, nullptr, static_cast<int>(T), static_cast<int>(N), static_cast<int>(x->size(2)), static_cast<int>(H), static_cast<int>(W),
-                          code_of(x->scalar_type()), packed.data_ptr(), static_cast<int>(cout), static_cast<int>(kh), static_cast<int>(kw),
-                          static_cast<int>(sh), static_cast<int>(sw), static_cast<int>(ph), static_cast<int>(pw), out.data_ptr(), out.stride(0),
-                          bytes > 0 ? workspace.data_ptr() : nullptr, bytes, stream_of(*x)) != 0)
-        return none();
-    return THPVariable_Wrap(out);
+    Tensor out;
+    const bool ran = unlocked([&] {
+        const Tensor packed = packed_weight(*w, *b, x->scalar_type());
+        out = empty({T, N, cout, ho, wo}, x->scalar_type(), *x);
+        const size_t bytes = snnf_conv_lif_workspace_bytes(static_cast<int>(T), static_cast<int>(N), static_cast<int>(x->size(2)), static_cast<int>(H),
+                                                           static_cast<int>(W), code_of(x->scalar_type()), static_cast<int>(cout), static_cast<int>(kh),
+                                                           static_cast<int>(kw), static_cast<int>(sh), static_cast<int>(sw), static_cast<int>(ph),
+                                                           static_cast<int>(pw), SNNF_F32, 0);
+        Tensor workspace;
+        if (bytes > 0) workspace = empty({static_cast<int64_t>(bytes)}, at::kByte, *x);
+        return snnf_conv_bias_ws(steps, nullptr, static_cast<int>(T), static_cast<int>(N), static_cast<int>(x->size(2)), static_cast<int>(H), static_cast<int>(W),
+                                 code_of(x->scalar_type()), packed.data_ptr(), static_cast<int>(cout), static_cast<int>(kh), static_cast<int>(kw),
+                                 static_cast<int>(sh), static_cast<int>(sw), static_cast<int>(ph), static_cast<int>(pw), out.data_ptr(), out.stride(0),
+                                 bytes > 0 ? workspace.data_ptr() : nullptr, bytes, stream_of(*x)) == 0;
+    });
+    return ran ? THPVariable_Wrap(out) : none();
 }
 
 // x [..., H, W] dense, is_max, kernel, stride, padding, learnt
@@ -1107,11 +1131,13 @@ PyObject* dense_pool(Args& a) {
     c10::SmallVector<int64_t, 6> shape(x->sizes().begin(), x->sizes().end());
     shape[shape.size() - 2] = ho;
     shape[shape.size() - 1] = wo;
-    Tensor out = empty(shape, x->scalar_type(), *x);
-    if (snnf_pool2d(x->data_ptr(), out.data_ptr(), x->numel() / (H * W), static_cast<int>(H), static_cast<int>(W), static_cast<int>(k), static_cast<int>(s),
-                    static_cast<int>(p), is_max != 0 ? 1 : 0, code_of(x->scalar_type()), stream_of(*x)) != 0)
-        return none();
-    return THPVariable_Wrap(out);
+    Tensor out;
+    const bool ran = unlocked([&] {
+        out = empty(shape, x->scalar_type(), *x);
+        return snnf_pool2d(x->data_ptr(), out.data_ptr(), x->numel() / (H * W), static_cast<int>(H), static_cast<int>(W), static_cast<int>(k), static_cast<int>(s),
+                           static_cast<int>(p), is_max != 0 ? 1 : 0, code_of(x->scalar_type()), stream_of(*x)) == 0;
+    });
+    return ran ? THPVariable_Wrap(out) : none();
 }
 
 PyObject* py_conv(PyObject*, PyObject* const* args, Py_ssize_t n) { return guarded(blocked_conv, args, n, 22); }
