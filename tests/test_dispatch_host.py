@@ -2,8 +2,10 @@
 internal-layout call of a known signature packs its weight through them)."""
 import subprocess
 import sys
+import weakref
 
 import pytest
+import torch
 
 from conftest import ROOT
 
@@ -14,3 +16,10 @@ def test_extension_is_connected_by_whoever_loads_it(snnf_lib, first):
             "from triton_snn_fusion_amd import _dispatch\nassert _dispatch.module().connected()\n")
     done = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=120)
     assert done.returncode == 0, done.stderr[-2000:]
+
+
+def test_internal_layout_tensors_take_attributes_and_weak_references():
+    from triton_snn_fusion_amd.runtime import hip_blocked_backend as B
+    x = B.Blocked(torch.empty(0), B.BITS, 1, 1, 8, 2, 2, torch.bfloat16)
+    x.note = "a host program's own mark"
+    assert weakref.ref(x)() is x and x.note

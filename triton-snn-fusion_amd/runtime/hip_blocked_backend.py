@@ -35,7 +35,7 @@ LAYOUT_NAMES = {NCHW: "nchw", C8: "c8", BITS: "bits"}
 _ROUTE_PLANE, _ALLOCATE_V, _RETURN_V = 1, 2, 4
 
 
-@dataclass(slots=True)
+@dataclass
 class Blocked:
     """T x N frames of [C, H, W] in one of the layouts. `data` is [T, N, C, H, W] (NCHW), [T, N, C8, H, W, 8] (C8) in the
     activation dtype, or [T, N, C8, H, W] uint8 (BITS). `shared`: every timestep is the same frame (data holds one)."""
