@@ -2,6 +2,8 @@
 internal-layout call of a known signature packs its weight through them)."""
 import subprocess
 import sys
+import threading
+import time
 import weakref
 
 import pytest
@@ -23,3 +25,36 @@ def test_internal_layout_tensors_take_attributes_and_weak_references():
     x = B.Blocked(torch.empty(0), B.BITS, 1, 1, 8, 2, 2, torch.bfloat16)
     x.note = "a host program's own mark"
     assert weakref.ref(x)() is x and x.note
+
+
+def test_two_threads_that_learn_at_once_file_their_own_statistics(monkeypatch):
+    """The index that a first call hands to the native dispatch names the events of that call, whatever another thread files meanwhile."""
+    from triton_snn_fusion_amd.runtime import snn_custom_ops as ops
+
+    class Slow(list):
+        def append(self, item):
+            super().append(item)
+            time.sleep(0.05)                                # room for the other thread
+
+    filed = Slow()
+    monkeypatch.setattr(ops, "_SIGNATURE_EVENTS", filed)
+    start = threading.Barrier(2)
+
+    def implementation(key):
+        start.wait()
+        ops._bump("triton", key)
+        return ()
+
+    answers = {}
+    for name in ("a", "b"):
+        monkeypatch.setitem(ops.OPERATORS, name, ("", implementation, None, None))
+    threads = [threading.Thread(target=lambda n=n: answers.update({n: ops._slow_dispatch(f"snn_custom::{n}", [f"counter_{n}"], True)[1]})) for n in ("a", "b")]
+    try:
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join(10)
+    finally:
+        ops.reset_fused_op_call_stats()
+    assert len(filed) == 2
+    assert all(("count", f"counter_{n}") in filed[answers[n]] for n in ("a", "b")), (answers, list(filed))

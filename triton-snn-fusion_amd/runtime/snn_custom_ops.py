@@ -142,6 +142,7 @@ def get_kernel_temporal_configs() -> Dict[str, int]:
 # What a call adds to the statistics, as events: ("count", key), ("table", table, key) and ("signature", entry). While the first
 # call of a signature runs, its thread keeps them: each natively dispatched call of that signature adds the same.
 _SIGNATURE_EVENTS: List[tuple] = []
+_SIGNATURE_EVENTS_LOCK = threading.Lock()      # calls arrive from any thread: an index belongs to the events filed under it
 _LEARNING = threading.local()
 
 
@@ -956,11 +957,10 @@ def _slow_dispatch(name: str, args: list, learn: bool) -> tuple:
         events, _LEARNING.events = tuple(_LEARNING.events), outer
     if ("count", "triton") not in events or ("count", "fallback") in events:
         return result, None
-    try:
+    with _SIGNATURE_EVENTS_LOCK:
+        if events not in _SIGNATURE_EVENTS:
+            _SIGNATURE_EVENTS.append(events)
         return result, _SIGNATURE_EVENTS.index(events)
-    except ValueError:
-        _SIGNATURE_EVENTS.append(events)
-        return result, len(_SIGNATURE_EVENTS) - 1
 
 
 # Operators that csrc/host/snnf_dispatch.cpp implements for GPU tensors, with the implementations above behind it.
