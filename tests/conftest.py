@@ -14,9 +14,9 @@ def pytest_configure(config):
 
 @pytest.fixture(scope="session")
 def snnf_lib():
-    """The built libsnnf.so (built here only when no library is present)."""
-    from triton_snn_fusion_amd import _lib
-    if not _lib.library_available():
+    """The built libsnnf.so and the dispatch module in front of it (built here only when one of them is not there)."""
+    from triton_snn_fusion_amd import _dispatch, _lib
+    if not _dispatch.available():
         from triton_snn_fusion_amd import build
         build.build_library()
     return _lib.lib()

@@ -308,3 +308,24 @@ def test_other_threads_run_while_a_known_call_allocates_and_launches(hip_ops):
         sys.setswitchinterval(interval)
         stop.set()
         thread.join()
+
+
+def test_internal_layouts_without_the_extension(hip_ops, monkeypatch):
+    """The internal-layout entry points, the neuron-free convolution and the dense pool on their Python implementations alone."""
+    from triton_snn_fusion_amd import _dispatch
+    from triton_snn_fusion_amd.runtime import hip_blocked_backend as B, hip_convlif_backend as CB, hip_pool_backend as PB
+    _, spikes, weights = _operands(torch.float16)
+    dense = torch.stack([spikes(2, 24, 8, 8) for _ in range(4)])
+    w, b, fc, one = weights(40, 24, 3, 3), weights(40), weights(10, 24), [1, 1]
+    x = B.from_dense(dense)
+
+    def run():
+        out, v = B.conv_lif_blocked(x, w, b, one, one, LIF[:3], want_v=True)
+        pooled, _ = B.conv_lif_blocked_avgpool(x, w, b, one, one, LIF[:3])
+        return [out.data, v, pooled.data, B.pool_blocked(x, True, 2, 2, 0).data, B.spike_pool_linear(x, fc, None),
+                CB.run_hip_conv_bias_frames(dense, w, b, one, one), PB.run_hip_pool2d(dense, True, 2, 2, 0)]
+
+    run()
+    known = run()
+    monkeypatch.setattr(_dispatch, "_MODULE", _dispatch._Absent())
+    assert all(torch.equal(a, c) for a, c in zip(run(), known))

@@ -84,8 +84,7 @@ class SnnfError(RuntimeError):
 
 
 def library_available() -> bool:
-    """Both halves of the native build: the kernels and the dispatch module in front of them."""
-    return LIB_PATH.exists() and (LIB_PATH.parent / "_snnf_dispatch.so").exists()
+    return LIB_PATH.exists()
 
 
 def lib() -> ctypes.CDLL:

@@ -988,12 +988,12 @@ def register_snn_custom_ops() -> None:
         TORCH_LIBRARY_HANDLES.append(def_lib)
     except RuntimeError:
         pass
+    native = _dispatch.load() is not None
     try:
         impl_lib = torch.library.Library("snn_custom", "IMPL")
-        native = _dispatch.available()
         for name, (_, gpu_impl, cpu_impl, meta_impl) in OPERATORS.items():
             impl_lib.impl(name, cpu_impl if cpu_impl is not None else gpu_impl, "CPU")
-            if not (native and name in NATIVE_DISPATCH):      # without a build GPU calls raise with the build instruction
+            if not (native and name in NATIVE_DISPATCH):
                 impl_lib.impl(name, gpu_impl, "CUDA")
             impl_lib.impl(name, meta_impl, "Meta")
         TORCH_LIBRARY_HANDLES.append(impl_lib)
