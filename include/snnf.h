@@ -248,7 +248,8 @@ int snnf_conv_lif(const void* const* xs, const void* const* residuals, int T,
  * first and run the kernel of that layout on them. The reference has no counterpart (its Triton kernel reads NCHW,
  * kernels/benchmark_conv_lif_temporal_general.py:629-676). Results are those of snnf_conv_lif up to the order of the fp32
  * additions.
- *   snnf_conv_lif_workspace_bytes : bytes with which this shape takes that route (0: the call is snnf_conv_lif).
+ *   snnf_conv_lif_workspace_bytes : bytes with which this shape takes that route (0: the call is snnf_conv_lif). A call whose
+ *               timesteps all read one frame never takes it and needs none.
  *   workspace : NULL (then this is snnf_conv_lif), or device memory, 16-byte aligned, contents undefined before and after.
  *               A smaller workspace than asked for is not used. Calls that share a workspace must not overlap in time.
  */
@@ -277,8 +278,9 @@ int snnf_conv_bias(const void* const* xs, const void* const* residuals /* nullab
                    int stride_h, int stride_w, int pad_h, int pad_w,
                    void* out, int64_t out_step_stride, void* stream);
 
-/* snnf_conv_bias with a workspace of snnf_conv_lif_workspace_bytes(..., SNNF_F32, ...) bytes, as snnf_conv_lif_ws; accepts what
- * snnf_conv_bias accepts. */
+/* snnf_conv_bias with a workspace, as snnf_conv_lif_ws; accepts what snnf_conv_bias accepts. */
+size_t snnf_conv_bias_workspace_bytes(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW,
+                                      int stride_h, int stride_w, int pad_h, int pad_w, int has_residual);
 int snnf_conv_bias_ws(const void* const* xs, const void* const* residuals /* nullable */, int T,
                       int N, int Cin, int H, int W, int x_dtype,
                       const void* packed_weight, int Cout, int KH, int KW,

@@ -142,3 +142,26 @@ def test_narrow_tiles_of_short_windows(snnf_lib, T, out):
     got, v = B.conv_lif_blocked(B.from_dense(dev(x, BF16), B.BITS), dev(w, BF16), dev(b, BF16), [1, 1], [1, 1], LIF, out_layout=layout, want_v=True)
     assert int(B.last_conv_plan()["oc_tiles"]) == 2, B.last_conv_plan()
     check(B.to_dense(got), v, ref, what=f"T={T} {out}")
+
+
+def test_one_frame_for_all_timesteps_takes_no_scratch_memory(hip_ops):
+    """The operator, on its first call and once it is known, and the neuron-free convolution allocate their outputs and nothing else;
+    with a frame per timestep the scratch of the blocked route comes on top."""
+    from triton_snn_fusion_amd.runtime import hip_convlif_backend as CB
+    S = torch.ops.snn_custom
+    g = gen(4950)
+    frames = [dev(spikes((8, 72, 33, 33), 0.25, g), BF16) for _ in range(4)]
+    w, b = dev(torch.randn(40, 72, 3, 3, generator=g), BF16), dev(torch.randn(40, generator=g), BF16)
+    zero = torch.zeros((), device=DEV)
+    operator = lambda xs: S.fused_temporal_conv_lif_state(xs, w, b, zero, [1, 1], [1, 1], [1, 1], 1, *LIF, False)
+    neuron_free = lambda xs: CB.run_hip_temporal_conv_bias(xs, w, b, [1, 1], [1, 1])
+    scratch = 4 * 8 * 9 * 33 * 33 * 16
+    for call, outputs in ((operator, (4 * 2 + 4) * 8 * 40 * 33 * 33), (neuron_free, 4 * 2 * 8 * 40 * 33 * 33)):
+        call(frames)                                            # packs the weight
+        for xs, extra in (([frames[0]] * 4, 0), (frames, scratch)):
+            for _ in range(3):
+                torch.cuda.reset_peak_memory_stats()
+                before = torch.cuda.memory_stats()["requested_bytes.all.current"]
+                out = call(xs)
+                assert torch.cuda.memory_stats()["requested_bytes.all.peak"] - before == outputs + extra
+                del out

@@ -400,3 +400,36 @@ def test_float32_state_next_to_16_bit_activations_both_rules():
     s_c, m_c = ops.lif_forward_state_torch(x, v16, *lif, False)
     want_s, want_m = ops._lif_step_torch(x, v16, x.dtype, *lif, False)
     assert m_c.dtype == torch.bfloat16 and torch.equal(s_c, want_s) and torch.equal(m_c, want_m)
+
+
+@pytest.mark.parametrize("shape,asked", [
+    ((16, 64, 20, 128, 128, 24, 3, 3, 1, 1, 1, 1), True),
+    ((16, 64, 20, 1024, 1024, 24, 3, 3, 1, 1, 1, 1), False),    # more than 2^27 groups of channels per timestep: 32-bit offsets
+    ((4, 1, 20, 40, 40, 24, 31, 31, 1, 1, 15, 15), False),      # more matrix steps than the kernel's table holds
+    ((2, 32, 170, 128, 264, 269, 5, 5, 4, 4, 1, 1), False),     # no patch of such a stride fits a wave's LDS region
+    ((8, 3, 414, 62, 62, 384, 13, 1, 2, 2, 7, 0), False),       # padding of more than half the kernel
+    ((16, 600, 20, 200, 200, 300, 3, 3, 1, 1, 1, 1), False),    # 2^31 output groups over all timesteps
+])
+def test_scratch_is_asked_for_only_where_it_is_used(snnf_lib, shape, asked):
+    """What the planner of the blocked kernel refuses at launch asks for no scratch memory, with and without a neuron."""
+    T, N, Cin, H, W, *rest = shape
+    need = T * N * -(-Cin // 8) * H * W * 16 if asked else 0
+    for residual in (0, 1):
+        for _ in range(2):                                      # planned, and remembered
+            assert snnf_lib.snnf_conv_lif_workspace_bytes(T, N, Cin, H, W, _lib.SNNF_BF16, *rest, _lib.SNNF_F32, residual) == need
+            # without a neuron only layers of the matrix kernel run at all: whole groups of eight channels
+            assert snnf_lib.snnf_conv_bias_workspace_bytes(T, N, Cin, H, W, _lib.SNNF_BF16, *rest, residual) == 0
+    assert snnf_lib.snnf_conv_bias_workspace_bytes(4, 16, 512, 7, 7, _lib.SNNF_BF16, 512, 3, 3, 1, 1, 1, 1, 0) == 4 * 16 * 64 * 49 * 16
+
+
+def test_a_tuned_plan_is_seen_by_a_remembered_route(snnf_lib):
+    """A 7x7 layer whose planned stages of four channel groups hold more steps than the table, and stages of two do not."""
+    layer = (2, 2, 372, 5, 5, 384, 7, 7, 1, 1, 3, 3)
+    asks = lambda: snnf_lib.snnf_conv_lif_workspace_bytes(*layer[:5], _lib.SNNF_BF16, *layer[5:], _lib.SNNF_F32, 0)
+    before = asks()
+    try:
+        assert snnf_lib.snnf_conv_blocked_tune(*layer, 0, 0, 2, 0) == 0
+        tuned = asks()
+    finally:
+        snnf_lib.snnf_conv_blocked_tune(*layer, 0, 0, 0, 0)
+    assert (before, tuned, asks()) == (0, 2 * 2 * 47 * 25 * 16, 0)

@@ -67,6 +67,7 @@ SIGNATURES = {
     "snnf_spike_pool_linear": (_i, [_pp, _i, _i, _i, _i, _i, _vp, _vp, _i, _i, _vp, _f, _vp]),
     "snnf_linear_lif_bits": (_i, [_pp, _i, _i, _i, _i, _i64, _i, _vp, _vp, _i, _vp, _vp, _i64, _vp, _f, _f, _f, _vp, _sz, _vp]),
     "snnf_pool2d": (_i, [_vp, _vp, _i64, _i, _i, _i, _i, _i, _i, _i, _vp]),
+    "snnf_conv_bias_workspace_bytes": (_sz, [_i] * 14),
     "snnf_conv_bias_ws": (_i, [_pp, _pp, _i, _i, _i, _i, _i, _i, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _i64, _vp, _sz, _vp]),
     "snnf_conv_bias": (_i, [_pp, _pp, _i, _i, _i, _i, _i, _i, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _i64, _vp]),
 }

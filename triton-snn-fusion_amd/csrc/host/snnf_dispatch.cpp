@@ -438,6 +438,13 @@ void packed_steps(const Tensor& x, int64_t T, const void** steps) {
     for (int64_t t = 0; t < T; ++t) steps[t] = base + t * bytes;
 }
 
+// Whether all of several timesteps read the same tensor: such a convolution runs once, on the dense kernels, without scratch memory.
+bool one_frame(const void* const* steps, int64_t T) {
+    for (int64_t t = 1; t < T; ++t)
+        if (steps[t] != steps[0]) return false;
+    return T > 1;
+}
+
 bool scan_call(const Call& c, Attempt& key, Pair* out) {
     const Tensor x = c.at(0).toTensor(), v = c.at(1).toTensor();
     key.tensor(x);
@@ -644,9 +651,10 @@ bool conv_call(const Call& c, Attempt& key, Op op, Pair* out) {
                                     static_cast<float>(lif.v_threshold), static_cast<float>(lif.v_reset), static_cast<float>(lif.tau), stream);
     } else {
         const Tensor packed = packed_weight(w, b, x.scalar_type());
-        const size_t bytes = snnf_conv_lif_workspace_bytes(static_cast<int>(T), N, cin, H, W, code_of(x.scalar_type()), static_cast<int>(shape[1]),
-                                                           static_cast<int>(kh), static_cast<int>(kw), static_cast<int>(sh), static_cast<int>(sw),
-                                                           static_cast<int>(ph), static_cast<int>(pw), wm.code(), residual ? 1 : 0);
+        const size_t bytes = one_frame(steps, T) ? 0
+            : snnf_conv_lif_workspace_bytes(static_cast<int>(T), N, cin, H, W, code_of(x.scalar_type()), static_cast<int>(shape[1]), static_cast<int>(kh),
+                                            static_cast<int>(kw), static_cast<int>(sh), static_cast<int>(sw), static_cast<int>(ph), static_cast<int>(pw),
+                                            wm.code(), residual ? 1 : 0);
         Tensor workspace;
         if (bytes > 0) workspace = empty({static_cast<int64_t>(bytes)}, at::kByte, x);
         status = snnf_conv_lif_ws(steps, residuals, static_cast<int>(T), N, cin, H, W, code_of(x.scalar_type()), packed.data_ptr(),
@@ -1103,10 +1111,10 @@ PyObject* dense_conv_bias(Args& a) {
     const bool ran = unlocked([&] {
         const Tensor packed = packed_weight(*w, *b, x->scalar_type());
         out = empty({T, N, cout, ho, wo}, x->scalar_type(), *x);
-        const size_t bytes = snnf_conv_lif_workspace_bytes(static_cast<int>(T), static_cast<int>(N), static_cast<int>(x->size(2)), static_cast<int>(H),
-                                                           static_cast<int>(W), code_of(x->scalar_type()), static_cast<int>(cout), static_cast<int>(kh),
-                                                           static_cast<int>(kw), static_cast<int>(sh), static_cast<int>(sw), static_cast<int>(ph),
-                                                           static_cast<int>(pw), SNNF_F32, 0);
+        const size_t bytes = snnf_conv_bias_workspace_bytes(static_cast<int>(T), static_cast<int>(N), static_cast<int>(x->size(2)), static_cast<int>(H),
+                                                            static_cast<int>(W), code_of(x->scalar_type()), static_cast<int>(cout), static_cast<int>(kh),
+                                                            static_cast<int>(kw), static_cast<int>(sh), static_cast<int>(sw), static_cast<int>(ph),
+                                                            static_cast<int>(pw), 0);
         Tensor workspace;
         if (bytes > 0) workspace = empty({static_cast<int64_t>(bytes)}, at::kByte, *x);
         return snnf_conv_bias_ws(steps, nullptr, static_cast<int>(T), static_cast<int>(N), static_cast<int>(x->size(2)), static_cast<int>(H), static_cast<int>(W),

@@ -105,7 +105,7 @@ bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int C
                          int v_dtype, bool residual, DenseFamily& family) {
     if (x_dtype != SNNF_BF16 && x_dtype != SNNF_F16) return false;
     if (v_dtype != SNNF_F32 || T < 1 || T > SNNF_MAX_T_PER_LAUNCH || N < 1 || Cin < 1 || H < 1 || W < 1 || Cout < 1 || KH < 1 || KW < 1 ||
-        stride_h < 1 || stride_w < 1 || pad_h < 0 || pad_w < 0 || H + 2 * pad_h < KH || W + 2 * pad_w < KW) return false;
+        stride_h < 1 || stride_w < 1 || pad_h < 0 || pad_w < 0 || H + 2 * pad_h < KH || W + 2 * pad_w < KW || 2 * pad_h > KH || 2 * pad_w > KW) return false;
     const bool pointwise = KH == 1 && KW == 1 && stride_h == 1 && stride_w == 1 && pad_h == 0 && pad_w == 0;
     const int64_t K = static_cast<int64_t>(Cin) * KH * KW;
     const int64_t out = static_cast<int64_t>(N) * Cout * ((H + 2 * pad_h - KH) / stride_h + 1) * ((W + 2 * pad_w - KW) / stride_w + 1);
@@ -128,6 +128,219 @@ struct Shortcut {
     int Cin, H, W, stride_h, stride_w;
     const void* packed_weight;
 };
+
+// What a launch of the blocked kernel depends on, without its pointers.
+struct BlockedCall {
+    int T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w;
+    int x_layout, res_layout, out_layout;              // res_layout: -1 without a residual
+    int64_t out_step_stride;
+    bool shared, neuron, has_v_init, has_v_out, pool2;
+    const Shortcut* shortcut;
+};
+
+struct BlockedPlan {
+    SpkGeom g = {};
+    SpkPlan patch = {};
+    PackGeom pg = {}, pg2 = {};                        // of the weight, and of the shortcut's
+    int tt = 0, windows = 0, wk_log2 = 0, oc_tiles = 0, grid = 0;
+    size_t lds_bytes = 0;
+    bool tuned_patch = false, tuned_split = false;
+};
+
+// Everything that decides whether and how the kernel runs a call; nothing is enqueued.
+int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
+    const int T = c.T, N = c.N, Cin = c.Cin, H = c.H, W = c.W, Cout = c.Cout, KH = c.KH, KW = c.KW;
+    const int stride_h = c.stride_h, stride_w = c.stride_w, pad_h = c.pad_h, pad_w = c.pad_w;
+    const bool shared = c.shared, neuron = c.neuron, pool2 = c.pool2;
+    const Shortcut* sc = c.shortcut;
+    SpkGeom& g = p.g;
+    g.N = N; g.Cin = Cin; g.H = H; g.W = W; g.Cout = Cout; g.KH = KH; g.KW = KW;
+    g.sh = stride_h; g.sw = stride_w; g.ph = pad_h; g.pw = pad_w;
+    g.Ho = (H + 2 * pad_h - KH) / stride_h + 1;
+    g.Wo = (W + 2 * pad_w - KW) / stride_w + 1;
+    g.C8in = (Cin + 7) / 8;
+    g.C8out = (Cout + 7) / 8;
+    const int64_t in_items = static_cast<int64_t>(N) * g.C8in * H * W;
+    const int64_t out_elems = static_cast<int64_t>(N) * g.C8out * 8 * g.Ho * g.Wo;
+    if (in_items >= (1LL << 27) || out_elems >= (1LL << 30) || static_cast<int64_t>(T) * N * g.C8out * g.Ho * g.Wo >= (1LL << 31))
+        return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_shape: tensor too large for 32-bit offsets", who);
+    if (c.out_layout == SNNF_LAYOUT_BITS && (c.out_step_stride < 0 || c.out_step_stride >= (1LL << 31) / T))
+        return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_shape: bit-packed output beyond 2 GiB", who);
+    const PackGeom& pg = p.pg = make_pack_geom(Cout, Cin, KH, KW, false);
+    g.gpc = pg.CK / 8;
+    g.npairs = pg.npairs;
+    g.nocf = pg.nocf;
+    g.tap_pairs = pg.CK == 8 ? 1 : 0;
+    g.taps = KH * KW;
+    g.frag_stride = static_cast<int64_t>(pg.nchunks) * pg.npairs * (kFragBytes / 2);
+    g.T = T;
+    g.shared_x = shared ? 1 : 0;
+    g.in_layout = c.x_layout;
+    g.res_layout = c.res_layout;
+    g.out_layout = c.out_layout;
+    g.analog_out = neuron ? 0 : 1;
+    g.out_step_stride = c.out_step_stride;
+
+    // Timesteps side by side: 4 (2 for T == 2, 1 for a single step or a shared frame), fewer when the halo does not fit.
+    int& tt = p.tt;
+    tt = shared || T == 1 ? 1 : (T == 2 ? 2 : 4);
+    TunedPlan tuned = {0, 0, 0};
+    {
+        const TunedKey key = {T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, shared ? 1 : 0};
+        std::lock_guard<std::mutex> lock(tuned_mutex);
+        const auto it = tuned_plans().find(key);
+        if (it != tuned_plans().end()) tuned = it->second;
+    }
+    SpkPlan& pl = p.patch;
+    if (pool2 && (!neuron || T != 4 || (g.Ho & 1) || (g.Wo & 1) || c.res_layout >= 0 || c.has_v_init || Cout % 8 != 0))
+        return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_pool: needs four timesteps, a neuron from the zero membrane, no residual, an even %dx%d output plane and whole channel groups",
+                    who, g.Ho, g.Wo);
+    bool planned = (tuned.patch_cols > 0 || tuned.stage_groups > 0) && plan_spk(g, tt, pl, tuned.patch_cols, tuned.stage_groups, pool2);
+    p.tuned_patch = planned;
+    for (; !planned && tt >= 1; tt >>= 1) {
+        planned = plan_spk(g, tt, pl, 0, 0, pool2);
+        if (planned) break;
+        if (pool2) break;   // the pooled store covers the four steps of one window
+    }
+    if (!planned)
+        return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_shape: no patch of this layer fits a wave's LDS region (kernel %dx%d, stride %dx%d)",
+                    who, KH, KW, stride_h, stride_w);
+    if (!p.tuned_patch && !g.tap_pairs) {
+        // Few tiles: stages of fewer channel groups where that lets more waves share a tile's K (128 -> 256 at 8^2, one image: stages
+        // of 4 groups on 4 waves 13.4 us, of 2 groups on 8 waves 11.9 us; 64 -> 128 at 16^2 13.3 / 11.7).
+        const int64_t tiles = static_cast<int64_t>(pl.img_groups) * pl.patches_x * pl.patches_y * ((Cout + 63) / 64);
+        int share = 1;
+        while (share < kSpkWaves && tiles * share * 2 <= static_cast<int64_t>(compute_units()) * kSpkWaves) share *= 2;
+        while (pl.G > 2 && (g.C8in + pl.G - 1) / pl.G < share) pl.G >>= 1;
+    }
+    p.windows = shared ? 1 : (T + tt - 1) / tt;
+    if (neuron && p.windows > 1 && !c.has_v_out)
+        return fail(SNNF_ERR_INVALID_ARGUMENT, "%s: v_out is required when the timesteps take %d windows of %d (it carries the membrane between them)",
+                    who, p.windows, tt);
+    g.PR = pl.PR; g.PC = pl.PC; g.PI = pl.PI; g.RR = pl.RR; g.RC = pl.RC; g.region = pl.region; g.G = pl.G;
+    g.patches_x = pl.patches_x;
+    g.patches_img = pl.patches_x * pl.patches_y;
+    g.n_patches = pl.img_groups * g.patches_img;
+    g.nstages = (g.C8in + g.G - 1) / g.G;
+    g.IT = g.G * g.region;
+    g.JT = (g.IT + 63) / 64;
+    g.lds_wave_bytes = tt * (g.IT + 1) * 16;
+    int& oc_tiles = p.oc_tiles;
+    oc_tiles = (Cout + 63) / 64;
+    g.n_items = g.n_patches * oc_tiles;
+    // K is shared by as many waves of a workgroup (up to eight, whole stages each) as keep the layer's tiles in one round of waves:
+    // 64 -> 64 at 56^2 x 12 is 1176 tiles, 20.2 us unsplit and 27.9 us when two waves share each (2352 of 2048 waves).
+    const int cus = compute_units();
+    int& wk_log2 = p.wk_log2;
+    while (wk_log2 < 3 && static_cast<int64_t>(g.n_items) << (wk_log2 + 1) <= static_cast<int64_t>(cus) * kSpkWaves && g.nstages >= (2 << wk_log2)) ++wk_log2;
+    if (tuned.k_waves > 0) {
+        int want = 0;
+        while ((1 << want) < tuned.k_waves) ++want;
+        if (g.nstages >= (1 << want)) {
+            wk_log2 = want;
+            p.tuned_split = true;
+        }
+    }
+    g.wk_log2 = wk_log2;
+    // Tiles of 32 channels where even those fit one round of waves: 256 -> 256 at 14^2 x 4 (112 tiles of 64 channels on eight waves each)
+    // 13.9 -> 10.0 us, 512 -> 512 at 7^2 x 8 19.8 -> 13.9, at 4^2 x 32 22.2 -> 17.6. At twice the tiles they would make a second round.
+    if ((tt == 4 || (!pool2 && c.x_layout != SNNF_LAYOUT_NCHW)) && wk_log2 > 0 && !p.tuned_split && Cout > 32 && static_cast<int64_t>(g.n_patches) * ((Cout + 31) / 32) << wk_log2 <= static_cast<int64_t>(cus) * kSpkWaves) {
+        g.narrow = 1;
+        oc_tiles = (Cout + 31) / 32;
+        g.n_items = g.n_patches * oc_tiles;
+    }
+    const int tiles_per_block = kSpkWaves >> wk_log2;
+    // Workgroups that are resident together: one per compute unit, or two where a wave needs at most a quarter of a SIMD's
+    // registers (one timestep's accumulators) and two staging areas fit the LDS. The tiles are dealt evenly over as many
+    // rounds as that takes.
+    p.lds_bytes = std::max(kSpkHeaderBytes + static_cast<size_t>(kSpkWaves) * g.lds_wave_bytes, wk_log2 > 0 ? kSpkHeaderBytes + kSpkPartialBytes : size_t{0});
+    const int resident = cus * ((tt == 1 && 2 * (p.lds_bytes + 1024) <= kMaxLds) ? 2 : 1);
+    const int blocks = (g.n_items + tiles_per_block - 1) / tiles_per_block;
+    g.iters = (blocks + resident - 1) / resident;
+    int& grid = p.grid;
+    grid = (blocks + g.iters - 1) / g.iters;
+    // Workgroups full of waves that leave a quarter of the compute units idle in every round, or half of them in the only one: a workgroup
+    // on every unit, some of its waves idle in the last round (128 -> 128 at 28^2 x 40, 140 workgroups 55.5 us, 256 workgroups 45.1; 64 -> 64
+    // at 24^2, one image, 18 and 36 workgroups 8.5 / 7.5). Fuller rounds stay even: 256 -> 256 at 14^2 x 128, 224 workgroups 100 us, 256 105.
+    if (g.iters > 1 ? grid * 4 < resident * 3 : grid * 2 <= cus) grid = std::min(g.n_items, g.iters > 1 ? resident : cus);
+    g.d_ppx = make_fast_div(g.PR * g.PC);
+    g.d_PC = make_fast_div(g.PC);
+    g.d_region = make_fast_div(g.region);
+    g.d_rrrc = make_fast_div(g.RR * g.RC);
+    g.d_RC = make_fast_div(g.RC);
+    g.d_n_patches = make_fast_div(g.n_patches);
+    g.d_patches_img = make_fast_div(g.patches_img);
+    g.d_patches_x = make_fast_div(g.patches_x);
+    g.d_gpc = make_fast_div(g.gpc);
+    const int hg = g.tap_pairs ? 1 : g.G / 2;
+    const int nst = g.tap_pairs ? g.npairs : g.taps * hg;
+    g.kw_mul = (KW & (KW - 1)) == 0 ? 65536 / KW : 65536 / KW + 1;
+    for (int tap = 0; tap < KH * KW; ++tap)
+        if (((tap * g.kw_mul) >> 16) != tap / KW)
+            return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_kernel: kernel %dx%d too large", who, KH, KW);
+    g.gpc_log2 = 0;
+    while ((1 << g.gpc_log2) < g.gpc) ++g.gpc_log2;
+    g.hg_log2 = 0;
+    while ((1 << g.hg_log2) < hg) ++g.hg_log2;
+    g.pair_tap_stride = g.tap_pairs ? 1 : g.gpc / 2;
+    if (nst > kSpkMaxSteps)
+        return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_kernel: %d matrix steps per stage exceed %d (kernel %dx%d)", who, nst, kSpkMaxSteps, KH, KW);
+    if (sc != nullptr) {
+        PackGeom& pg2 = p.pg2;
+        pg2 = make_pack_geom(Cout, sc->Cin, 1, 1, false);
+        const int gpc2 = pg2.CK / 8;
+        if (tt != 4 || g.tap_pairs || gpc2 % g.G != 0 || nst + 4 + hg + 4 > kSpkMaxSteps + 4)
+            return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_shortcut: this layer's plan (window %d, %d channel groups per stage, %d steps) has no room for a shortcut",
+                        who, tt, g.G, nst);
+        g.sc_C8 = sc->Cin / 8;
+        g.sc_stages = (g.sc_C8 + g.G - 1) / g.G;
+        g.sc_H = sc->H; g.sc_W = sc->W; g.sc_sh = sc->stride_h; g.sc_sw = sc->stride_w;
+        g.sc_gpc_log2 = 0;
+        while ((1 << g.sc_gpc_log2) < gpc2) ++g.sc_gpc_log2;
+        g.sc_npairs = pg2.npairs;
+        g.sc_frag_stride = static_cast<int64_t>(pg2.nchunks) * pg2.npairs * (kFragBytes / 2);
+    }
+    g.d_hg = make_fast_div(hg);
+    g.d_nst = make_fast_div(nst);
+    g.d_KW = make_fast_div(KW);
+    return SNNF_OK;
+}
+
+// Whether a layer takes the blocked route: where the rule sends it there and the kernel then runs it. A layer that the planner refuses
+// (offsets, a kernel of too many steps, no patch that fits) gets no scratch memory asked for. Without a neuron the dense route has the
+// matrix kernel only; what it refuses stays refused. The answer depends on the layer and the table of tuned plans alone and is
+// kept per layer: it is asked for twice per call.
+using RouteKey = std::array<int, 14>;
+struct Route { bool taken; DenseFamily family; };
+std::mutex routes_mutex;
+std::map<RouteKey, Route>& routes() {
+    static std::map<RouteKey, Route> known;
+    return known;
+}
+constexpr size_t kMaxRoutes = 4096;
+
+Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w,
+                    int v_dtype, bool residual, bool neuron) {
+    if ((x_dtype != SNNF_BF16 && x_dtype != SNNF_F16) || v_dtype != SNNF_F32) return {false, DenseFamily::kTInM};
+    const RouteKey key = {T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, residual ? 1 : 0, neuron ? 1 : 0};
+    {
+        std::lock_guard<std::mutex> lock(routes_mutex);
+        const auto it = routes().find(key);
+        if (it != routes().end()) return it->second;
+    }
+    Route route = {false, DenseFamily::kTInM};
+    route.taken = takes_blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residual, route.family) &&
+                  (neuron || route.family == DenseFamily::kMatrixMasked || route.family == DenseFamily::kMatrixWhole);
+    if (route.taken) {
+        BlockedPlan plan;
+        route.taken = plan_blocked("snnf_conv_lif_workspace_bytes", BlockedCall{T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, SNNF_LAYOUT_C8,
+                                   residual ? SNNF_LAYOUT_NCHW : -1, SNNF_LAYOUT_NCHW, 0, false, neuron, false, neuron, false, nullptr}, plan) == SNNF_OK;
+    }
+    std::lock_guard<std::mutex> lock(routes_mutex);
+    if (routes().size() >= kMaxRoutes) routes().clear();
+    routes()[key] = route;
+    return route;
+}
 
 // A call on dense tensors that runs here: its inputs, which are brought into C8 first, and the kernel family of the dense route.
 struct DenseRoute {
@@ -161,9 +374,13 @@ extern "C" int snnf_conv_blocked_tune(int T, int N, int Cin, int H, int W, int C
         return fail(SNNF_ERR_INVALID_ARGUMENT, "snnf_conv_blocked_tune: patch_cols=%d stage_groups=%d k_waves=%d out of range", patch_cols,
                     stage_groups, k_waves);
     const TunedKey key = {T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, shared_frame ? 1 : 0};
-    std::lock_guard<std::mutex> lock(tuned_mutex);
-    if (patch_cols == 0 && stage_groups == 0 && k_waves == 0) tuned_plans().erase(key);
-    else tuned_plans()[key] = TunedPlan{patch_cols, stage_groups, k_waves};
+    {
+        std::lock_guard<std::mutex> lock(tuned_mutex);
+        if (patch_cols == 0 && stage_groups == 0 && k_waves == 0) tuned_plans().erase(key);
+        else tuned_plans()[key] = TunedPlan{patch_cols, stage_groups, k_waves};
+    }
+    std::lock_guard<std::mutex> lock(routes_mutex);
+    routes().clear();
     return SNNF_OK;
 }
 
@@ -204,8 +421,14 @@ extern "C" int snnf_conv_lif_blocked_avgpool(const void* const* xs, int x_layout
 extern "C" size_t snnf_conv_lif_workspace_bytes(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h,
                                                 int stride_w, int pad_h, int pad_w, int v_dtype, int residual) {
     using namespace snnf;
-    DenseFamily family;
-    if (!takes_blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residual != 0, family)) return 0;
+    if (!blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residual != 0, true).taken) return 0;
+    return static_cast<size_t>(T) * c8_step_bytes(N, Cin, H, W);
+}
+
+extern "C" size_t snnf_conv_bias_workspace_bytes(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h,
+                                                 int stride_w, int pad_h, int pad_w, int residual) {
+    using namespace snnf;
+    if (!blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, SNNF_F32, residual != 0, false).taken) return 0;
     return static_cast<size_t>(T) * c8_step_bytes(N, Cin, H, W);
 }
 
@@ -216,12 +439,9 @@ int run_blocked_route(const void* const* xs, const void* const* residuals, int T
                       int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w, const void* v_init, int v_dtype, void* out,
                       int64_t out_step_stride, void* v_out, int neuron, float v_threshold, float v_reset, float tau, void* workspace,
                       size_t workspace_bytes, void* stream) {
-    DenseFamily family = DenseFamily::kTInM;
-    if (xs == nullptr || workspace == nullptr || (neuron && v_out == nullptr) || !aligned_to(workspace, 16) || out_step_stride < 0 ||
-        !takes_blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residuals != nullptr, family))
-        return SNNF_ERR_UNSUPPORTED;
-    // Without a neuron the dense route has the matrix kernel only; what it refuses stays refused.
-    if (!neuron && family != DenseFamily::kMatrixMasked && family != DenseFamily::kMatrixWhole) return SNNF_ERR_UNSUPPORTED;
+    if (xs == nullptr || workspace == nullptr || (neuron && v_out == nullptr) || !aligned_to(workspace, 16) || out_step_stride < 0) return SNNF_ERR_UNSUPPORTED;
+    const Route taken = blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residuals != nullptr, neuron != 0);
+    if (!taken.taken) return SNNF_ERR_UNSUPPORTED;
     const size_t step = c8_step_bytes(N, Cin, H, W);
     if (workspace_bytes < step * T) return SNNF_ERR_UNSUPPORTED;
     bool shared = T > 1;
@@ -232,7 +452,7 @@ int run_blocked_route(const void* const* xs, const void* const* residuals, int T
         inner[t] = static_cast<const char*>(workspace) + t * step;
     }
     if (shared) return SNNF_ERR_UNSUPPORTED;       // one frame for all timesteps is convolved once on the dense kernels too
-    const DenseRoute route = {xs, family};
+    const DenseRoute route = {xs, taken.family};
     return conv_lif_blocked_impl(neuron ? "snnf_conv_lif" : "snnf_conv_bias", inner, SNNF_LAYOUT_C8, residuals, SNNF_LAYOUT_NCHW, T, N, Cin, H, W, x_dtype,
                                  packed_weight, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_init, out, SNNF_LAYOUT_NCHW, out_step_stride * 2, v_out,
                                  neuron, v_threshold, v_reset, tau, stream, nullptr, false, &route);
@@ -321,154 +541,12 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
             if (sc->xs[t] == nullptr) return fail(SNNF_ERR_INVALID_ARGUMENT, "%s: shortcut_xs[%d] is null", who, t);
     }
 
-    SpkGeom g = {};
-    g.N = N; g.Cin = Cin; g.H = H; g.W = W; g.Cout = Cout; g.KH = KH; g.KW = KW;
-    g.sh = stride_h; g.sw = stride_w; g.ph = pad_h; g.pw = pad_w;
-    g.Ho = (H + 2 * pad_h - KH) / stride_h + 1;
-    g.Wo = (W + 2 * pad_w - KW) / stride_w + 1;
-    g.C8in = (Cin + 7) / 8;
-    g.C8out = (Cout + 7) / 8;
-    const int64_t in_items = static_cast<int64_t>(N) * g.C8in * H * W;
-    const int64_t out_elems = static_cast<int64_t>(N) * g.C8out * 8 * g.Ho * g.Wo;
-    if (in_items >= (1LL << 27) || out_elems >= (1LL << 30) || static_cast<int64_t>(T) * N * g.C8out * g.Ho * g.Wo >= (1LL << 31))
-        return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_shape: tensor too large for 32-bit offsets", who);
-    if (out_layout == SNNF_LAYOUT_BITS && (out_step_stride < 0 || out_step_stride >= (1LL << 31) / T))
-        return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_shape: bit-packed output beyond 2 GiB", who);
-    const PackGeom pg = make_pack_geom(Cout, Cin, KH, KW, false);
-    g.gpc = pg.CK / 8;
-    g.npairs = pg.npairs;
-    g.nocf = pg.nocf;
-    g.tap_pairs = pg.CK == 8 ? 1 : 0;
-    g.taps = KH * KW;
-    g.frag_stride = static_cast<int64_t>(pg.nchunks) * pg.npairs * (kFragBytes / 2);
-    g.T = T;
-    g.shared_x = shared ? 1 : 0;
-    g.in_layout = x_layout;
-    g.res_layout = residuals != nullptr ? res_layout : -1;
-    g.out_layout = out_layout;
-    g.analog_out = neuron ? 0 : 1;
-    g.out_step_stride = out_step_stride;
-
-    // Timesteps side by side: 4 (2 for T == 2, 1 for a single step or a shared frame), fewer when the halo does not fit.
-    int tt = shared || T == 1 ? 1 : (T == 2 ? 2 : 4);
-    TunedPlan tuned = {0, 0, 0};
-    {
-        const TunedKey key = {T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, shared ? 1 : 0};
-        std::lock_guard<std::mutex> lock(tuned_mutex);
-        const auto it = tuned_plans().find(key);
-        if (it != tuned_plans().end()) tuned = it->second;
-    }
-    SpkPlan pl = {};
-    if (pool2 && (!neuron || T != 4 || (g.Ho & 1) || (g.Wo & 1) || residuals != nullptr || v_init != nullptr || Cout % 8 != 0))
-        return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_pool: needs four timesteps, a neuron from the zero membrane, no residual, an even %dx%d output plane and whole channel groups",
-                    who, g.Ho, g.Wo);
-    bool planned = (tuned.patch_cols > 0 || tuned.stage_groups > 0) && plan_spk(g, tt, pl, tuned.patch_cols, tuned.stage_groups, pool2);
-    const bool tuned_patch = planned;
-    for (; !planned && tt >= 1; tt >>= 1) {
-        planned = plan_spk(g, tt, pl, 0, 0, pool2);
-        if (planned) break;
-        if (pool2) break;   // the pooled store covers the four steps of one window
-    }
-    if (!planned)
-        return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_shape: no patch of this layer fits a wave's LDS region (kernel %dx%d, stride %dx%d)",
-                    who, KH, KW, stride_h, stride_w);
-    if (!tuned_patch && !g.tap_pairs) {
-        // Few tiles: stages of fewer channel groups where that lets more waves share a tile's K (128 -> 256 at 8^2, one image: stages
-        // of 4 groups on 4 waves 13.4 us, of 2 groups on 8 waves 11.9 us; 64 -> 128 at 16^2 13.3 / 11.7).
-        const int64_t tiles = static_cast<int64_t>(pl.img_groups) * pl.patches_x * pl.patches_y * ((Cout + 63) / 64);
-        int share = 1;
-        while (share < kSpkWaves && tiles * share * 2 <= static_cast<int64_t>(compute_units()) * kSpkWaves) share *= 2;
-        while (pl.G > 2 && (g.C8in + pl.G - 1) / pl.G < share) pl.G >>= 1;
-    }
-    const int windows = shared ? 1 : (T + tt - 1) / tt;
-    if (neuron && windows > 1 && v_out == nullptr)
-        return fail(SNNF_ERR_INVALID_ARGUMENT, "%s: v_out is required when the timesteps take %d windows of %d (it carries the membrane between them)",
-                    who, windows, tt);
-    g.PR = pl.PR; g.PC = pl.PC; g.PI = pl.PI; g.RR = pl.RR; g.RC = pl.RC; g.region = pl.region; g.G = pl.G;
-    g.patches_x = pl.patches_x;
-    g.patches_img = pl.patches_x * pl.patches_y;
-    g.n_patches = pl.img_groups * g.patches_img;
-    g.nstages = (g.C8in + g.G - 1) / g.G;
-    g.IT = g.G * g.region;
-    g.JT = (g.IT + 63) / 64;
-    g.lds_wave_bytes = tt * (g.IT + 1) * 16;
-    int oc_tiles = (Cout + 63) / 64;
-    g.n_items = g.n_patches * oc_tiles;
-    // K is shared by as many waves of a workgroup (up to eight, whole stages each) as keep the layer's tiles in one round of waves:
-    // 64 -> 64 at 56^2 x 12 is 1176 tiles, 20.2 us unsplit and 27.9 us when two waves share each (2352 of 2048 waves).
-    const int cus = compute_units();
-    int wk_log2 = 0;
-    while (wk_log2 < 3 && static_cast<int64_t>(g.n_items) << (wk_log2 + 1) <= static_cast<int64_t>(cus) * kSpkWaves && g.nstages >= (2 << wk_log2)) ++wk_log2;
-    bool tuned_split = false;
-    if (tuned.k_waves > 0) {
-        int want = 0;
-        while ((1 << want) < tuned.k_waves) ++want;
-        if (g.nstages >= (1 << want)) {
-            wk_log2 = want;
-            tuned_split = true;
-        }
-    }
-    g.wk_log2 = wk_log2;
-    // Tiles of 32 channels where even those fit one round of waves: 256 -> 256 at 14^2 x 4 (112 tiles of 64 channels on eight waves each)
-    // 13.9 -> 10.0 us, 512 -> 512 at 7^2 x 8 19.8 -> 13.9, at 4^2 x 32 22.2 -> 17.6. At twice the tiles they would make a second round.
-    if ((tt == 4 || (!pool2 && x_layout != SNNF_LAYOUT_NCHW)) && wk_log2 > 0 && !tuned_split && Cout > 32 && static_cast<int64_t>(g.n_patches) * ((Cout + 31) / 32) << wk_log2 <= static_cast<int64_t>(cus) * kSpkWaves) {
-        g.narrow = 1;
-        oc_tiles = (Cout + 31) / 32;
-        g.n_items = g.n_patches * oc_tiles;
-    }
-    const int tiles_per_block = kSpkWaves >> wk_log2;
-    // Workgroups that are resident together: one per compute unit, or two where a wave needs at most a quarter of a SIMD's
-    // registers (one timestep's accumulators) and two staging areas fit the LDS. The tiles are dealt evenly over as many
-    // rounds as that takes.
-    const size_t lds_bytes = std::max(kSpkHeaderBytes + static_cast<size_t>(kSpkWaves) * g.lds_wave_bytes, wk_log2 > 0 ? kSpkHeaderBytes + kSpkPartialBytes : size_t{0});
-    const int resident = cus * ((tt == 1 && 2 * (lds_bytes + 1024) <= kMaxLds) ? 2 : 1);
-    const int blocks = (g.n_items + tiles_per_block - 1) / tiles_per_block;
-    g.iters = (blocks + resident - 1) / resident;
-    int grid = (blocks + g.iters - 1) / g.iters;
-    // Workgroups full of waves that leave a quarter of the compute units idle in every round, or half of them in the only one: a workgroup
-    // on every unit, some of its waves idle in the last round (128 -> 128 at 28^2 x 40, 140 workgroups 55.5 us, 256 workgroups 45.1; 64 -> 64
-    // at 24^2, one image, 18 and 36 workgroups 8.5 / 7.5). Fuller rounds stay even: 256 -> 256 at 14^2 x 128, 224 workgroups 100 us, 256 105.
-    if (g.iters > 1 ? grid * 4 < resident * 3 : grid * 2 <= cus) grid = std::min(g.n_items, g.iters > 1 ? resident : cus);
-    g.d_ppx = make_fast_div(g.PR * g.PC);
-    g.d_PC = make_fast_div(g.PC);
-    g.d_region = make_fast_div(g.region);
-    g.d_rrrc = make_fast_div(g.RR * g.RC);
-    g.d_RC = make_fast_div(g.RC);
-    g.d_n_patches = make_fast_div(g.n_patches);
-    g.d_patches_img = make_fast_div(g.patches_img);
-    g.d_patches_x = make_fast_div(g.patches_x);
-    g.d_gpc = make_fast_div(g.gpc);
-    const int hg = g.tap_pairs ? 1 : g.G / 2;
-    const int nst = g.tap_pairs ? g.npairs : g.taps * hg;
-    g.kw_mul = (KW & (KW - 1)) == 0 ? 65536 / KW : 65536 / KW + 1;
-    for (int tap = 0; tap < KH * KW; ++tap)
-        if (((tap * g.kw_mul) >> 16) != tap / KW)
-            return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_kernel: kernel %dx%d too large", who, KH, KW);
-    g.gpc_log2 = 0;
-    while ((1 << g.gpc_log2) < g.gpc) ++g.gpc_log2;
-    g.hg_log2 = 0;
-    while ((1 << g.hg_log2) < hg) ++g.hg_log2;
-    g.pair_tap_stride = g.tap_pairs ? 1 : g.gpc / 2;
-    if (nst > kSpkMaxSteps)
-        return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_kernel: %d matrix steps per stage exceed %d (kernel %dx%d)", who, nst, kSpkMaxSteps, KH, KW);
-    PackGeom pg2 = {};
-    if (sc != nullptr) {
-        pg2 = make_pack_geom(Cout, sc->Cin, 1, 1, false);
-        const int gpc2 = pg2.CK / 8;
-        if (tt != 4 || g.tap_pairs || gpc2 % g.G != 0 || nst + 4 + hg + 4 > kSpkMaxSteps + 4)
-            return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_shortcut: this layer's plan (window %d, %d channel groups per stage, %d steps) has no room for a shortcut",
-                        who, tt, g.G, nst);
-        g.sc_C8 = sc->Cin / 8;
-        g.sc_stages = (g.sc_C8 + g.G - 1) / g.G;
-        g.sc_H = sc->H; g.sc_W = sc->W; g.sc_sh = sc->stride_h; g.sc_sw = sc->stride_w;
-        g.sc_gpc_log2 = 0;
-        while ((1 << g.sc_gpc_log2) < gpc2) ++g.sc_gpc_log2;
-        g.sc_npairs = pg2.npairs;
-        g.sc_frag_stride = static_cast<int64_t>(pg2.nchunks) * pg2.npairs * (kFragBytes / 2);
-    }
-    g.d_hg = make_fast_div(hg);
-    g.d_nst = make_fast_div(nst);
-    g.d_KW = make_fast_div(KW);
+    BlockedPlan p;
+    if (const int rc = plan_blocked(who, BlockedCall{T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, x_layout,
+                                                     residuals != nullptr ? res_layout : -1, out_layout, out_step_stride, shared, neuron != 0,
+                                                     v_init != nullptr, v_out != nullptr, pool2, sc}, p); rc != SNNF_OK)
+        return rc;
+    const SpkGeom& g = p.g;
 
     SpkLaunch L = {};
     for (int t = 0; t < T; ++t) {
@@ -478,27 +556,27 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     }
     if (sc != nullptr) {
         L.wpacked2 = static_cast<const uint16_t*>(sc->packed_weight);
-        L.bias2 = reinterpret_cast<const float*>(L.wpacked2 + packed_weight_elems(pg2));
+        L.bias2 = reinterpret_cast<const float*>(L.wpacked2 + packed_weight_elems(p.pg2));
     }
     L.g = g;
     L.wpacked = static_cast<const uint16_t*>(packed_weight);
-    L.bias = reinterpret_cast<const float*>(L.wpacked + packed_weight_elems(pg));
+    L.bias = reinterpret_cast<const float*>(L.wpacked + packed_weight_elems(p.pg));
     L.v_init = neuron ? static_cast<const float*>(v_init) : nullptr;
     L.out = out;
     L.v_out = neuron ? static_cast<float*>(v_out) : nullptr;
     L.lif = make_lif_params(v_threshold, v_reset, tau);
-    L.grid = grid;
-    L.lds_bytes = lds_bytes;
+    L.grid = p.grid;
+    L.lds_bytes = p.lds_bytes;
     L.stream = as_stream(stream);
     const bool fast_epi = neuron && (out_layout == SNNF_LAYOUT_BITS || pool2) && (residuals == nullptr || res_layout == SNNF_LAYOUT_BITS) &&
                           L.lif.charge_mode == CHARGE_SCALE && L.lif.inv_tau == 0.5f && L.lif.v_reset == 0.0f &&
                           L.lif.v_threshold >= 1e-30f && L.lif.v_threshold <= 1e30f &&   // its multiples by 2^t stay normal numbers
-                          v_init == nullptr && windows == 1 && Cout % 8 == 0;
+                          v_init == nullptr && p.windows == 1 && Cout % 8 == 0;
     snprintf(snnf::conv_plan_buffer(), 256,
              "kernel=%s variant=%d window=%d launches=%d tile=%dx%dx%d halo=%dx%d waves=8x1x%d oc_tiles=%d px_tiles=%d "
              "stage_chunks=%d run=0 lds=%zu grid=%d tuned=%d shortcut_stages=%d%s",
-             dense != nullptr ? family_name(dense->family) : "blocked", (wk_log2 > 0 ? 50 : 40) + tt + (fast_epi ? 20 : 0), shared ? T : tt, dense != nullptr ? 2 : 1, g.PI, g.PR, g.PC, g.RR, g.RC, 1 << wk_log2, oc_tiles, g.n_patches, g.G,
-             L.lds_bytes, grid, (tuned_patch ? 1 : 0) + (tuned_split ? 2 : 0), g.sc_stages, dense != nullptr ? " route=c8" : "");
+             dense != nullptr ? family_name(dense->family) : "blocked", (p.wk_log2 > 0 ? 50 : 40) + p.tt + (fast_epi ? 20 : 0), shared ? T : p.tt, dense != nullptr ? 2 : 1, g.PI, g.PR, g.PC, g.RR, g.RC, 1 << p.wk_log2, p.oc_tiles, g.n_patches, g.G,
+             L.lds_bytes, p.grid, (p.tuned_patch ? 1 : 0) + (p.tuned_split ? 2 : 0), g.sc_stages, dense != nullptr ? " route=c8" : "");
     L.fast_epilogue = fast_epi;
     if (dense != nullptr) {   // the plan stands: bring the dense inputs into the C8 buffers behind `xs`
         StepPtrs from = {};
@@ -506,16 +584,16 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
         if (const int rc = launch_steps_to_c8(from, T, const_cast<void*>(xs[0]), N, Cin, H, W, L.stream); rc != SNNF_OK) return rc;
     }
     if (pool2) {
-        if (!fast_epi || windows != 1 || (tt != 4 && !shared))
+        if (!fast_epi || p.windows != 1 || (p.tt != 4 && !shared))
             return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_pool: the pooled output needs the usual neuron (tau 2, hard reset to 0) and the four steps in one window", who);
         L.g.pool2 = 1;
         if (x_layout == SNNF_LAYOUT_NCHW) return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_frame(L, true) : launch_conv_spk_f16_frame(L, true);
-        return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_pooled(L, tt) : launch_conv_spk_f16_pooled(L, tt);
+        return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_pooled(L, p.tt) : launch_conv_spk_f16_pooled(L, p.tt);
     }
     if (sc != nullptr) return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_shortcut(L) : launch_conv_spk_f16_shortcut(L);
     if (x_layout == SNNF_LAYOUT_NCHW) return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_frame(L, false) : launch_conv_spk_f16_frame(L, false);
-    if (x_layout == SNNF_LAYOUT_BITS) return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_bits(L, tt) : launch_conv_spk_f16_bits(L, tt);
-    return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_c8(L, tt) : launch_conv_spk_f16_c8(L, tt);
+    if (x_layout == SNNF_LAYOUT_BITS) return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_bits(L, p.tt) : launch_conv_spk_f16_bits(L, p.tt);
+    return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_c8(L, p.tt) : launch_conv_spk_f16_c8(L, p.tt);
 }
 
 }  // namespace

@@ -341,6 +341,11 @@ def _v_init_pointer(v_init, out_shape, v_dtype, device):
     return v_init if v_init.is_contiguous() else v_init.contiguous()
 
 
+def _one_frame(pointers) -> bool:
+    """Whether all of several timesteps read the same tensor (convolved once, on the dense kernels)."""
+    return len(pointers) > 1 and len(set(pointers)) == 1
+
+
 def _launch(kernel_key: str, steps: Sequence[torch.Tensor], residuals: Optional[Sequence[torch.Tensor]], weight, bias,
             v_init, stride, padding, v_threshold, v_reset, tau, spikes: torch.Tensor, v_out: torch.Tensor) -> None:
     """Enqueues the HIP kernel(s) for one fused conv+LIF call. `steps` are T contiguous [N, C, H, W] tensors."""
@@ -367,9 +372,11 @@ def _launch(kernel_key: str, steps: Sequence[torch.Tensor], residuals: Optional[
             float(v_threshold), float(v_reset), float(tau), stream))
     else:
         packed = _packed_weight(weight, bias, first.dtype)
-        # Scratch for the inputs in the channel-blocked layout where the library asks for it; the caching allocator hands the block
-        # out again in the order of the stream the kernels run on.
-        nbytes = int(lib.snnf_conv_lif_workspace_bytes(T, n, cin, h, w, x_code, cout, kh, kw, sh, sw, ph, pw, v_code, 1 if rs is not None else 0))
+        # Scratch for the inputs in the channel-blocked layout where the library asks for it (one frame for all timesteps needs none);
+        # the caching allocator hands the block out again in the order of the stream the kernels run on.
+        nbytes = 0
+        if not _one_frame(xs):
+            nbytes = int(lib.snnf_conv_lif_workspace_bytes(T, n, cin, h, w, x_code, cout, kh, kw, sh, sw, ph, pw, v_code, 1 if rs is not None else 0))
         workspace = torch.empty(nbytes, dtype=torch.uint8, device=first.device) if nbytes else None
         _lib.check("snnf_conv_lif", lib.snnf_conv_lif_ws(
             xs, rs, T, n, cin, h, w, x_code, packed.data_ptr(), cout, kh, kw, sh, sw, ph, pw,
@@ -406,11 +413,13 @@ def run_hip_temporal_conv_bias(xs: Sequence[torch.Tensor], weight, bias, stride,
         bias = torch.zeros(cout, dtype=weight.dtype, device=weight.device)
     out = torch.empty((T, n, cout, ho, wo), dtype=first.dtype, device=first.device)
     packed = _packed_weight(weight, bias, first.dtype)
-    lib, x_code = _lib.lib(), _lib.dtype_code(first.dtype)
-    nbytes = int(lib.snnf_conv_lif_workspace_bytes(T, n, cin, h, w, x_code, cout, kh, kw, sh, sw, ph, pw, _lib.SNNF_F32, 1 if res is not None else 0))
+    lib, x_code, pointers = _lib.lib(), _lib.dtype_code(first.dtype), _lib.step_pointers(steps)
+    nbytes = 0
+    if not _one_frame(pointers):
+        nbytes = int(lib.snnf_conv_bias_workspace_bytes(T, n, cin, h, w, x_code, cout, kh, kw, sh, sw, ph, pw, 1 if res is not None else 0))
     workspace = torch.empty(nbytes, dtype=torch.uint8, device=first.device) if nbytes else None
     _lib.check("snnf_conv_bias", lib.snnf_conv_bias_ws(
-        _lib.step_pointers(steps), _lib.step_pointers(res) if res is not None else None, T, n, cin, h, w,
+        pointers, _lib.step_pointers(res) if res is not None else None, T, n, cin, h, w,
         x_code, packed.data_ptr(), cout, kh, kw, sh, sw, ph, pw,
         out.data_ptr(), int(out.stride(0)), _lib.ptr(workspace), nbytes, _lib.current_stream(first.device)))
     return out
