@@ -47,7 +47,7 @@ def test_conv_through_the_blocked_layout(snnf_lib, Cin, Cout, H, W, k, s, T, N, 
     code = _lib.dtype_code(dtype)
     nbytes = snnf_lib.snnf_conv_lif_workspace_bytes(T, N, Cin, H, W, code, Cout, k, k, s, s, p, p, 0, int(residual))
     assert nbytes == T * N * -(-Cin // 8) * H * W * 16
-    results = {}
+    results, families = {}, {}
     for name, given in (("blocked", nbytes), ("dense", 0), ("short", nbytes - 1)):     # a workspace that is too small is not used
         workspace = torch.full((nbytes,), 255, dtype=torch.uint8, device=DEV)          # NaN patterns
         sp, v = torch.empty(T, N, Cout, Ho, Wo, device=DEV, dtype=dtype), torch.empty(N, Cout, Ho, Wo, device=DEV)
@@ -57,6 +57,8 @@ def test_conv_through_the_blocked_layout(snnf_lib, Cin, Cout, H, W, k, s, T, N, 
         assert (CB.last_conv_plan().get("route") == "c8") == (name == "blocked"), CB.last_conv_plan()
         check(sp, v, ref, what=f"{name} {Cin}->{Cout} {H}x{W}")
         results[name] = (sp, v)
+        families[name] = CB.last_conv_plan()["kernel"]
+    assert shift or families["blocked"] == families["dense"], families      # the rule knows which kernel the layer leaves
     assert torch.equal(results["short"][0], results["dense"][0]) and torch.equal(results["short"][1], results["dense"][1])
 
 

@@ -246,35 +246,147 @@ char* conv_plan_buffer() {
 extern "C" const char* snnf_conv_last_plan(void) { return snnf::conv_plan_buffer(); }
 
 namespace snnf {
-// What snnf_conv_lif runs a layer of 16-bit activations and an fp32 membrane on, whatever its neuron, when every operand is 16-byte
-// aligned and the steps have inputs of their own.
-DenseFamily dense_family(int T, int N, int Cin, int H, int W, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w, int x_dtype) {
-    const bool pointwise = KH == 1 && KW == 1 && stride_h == 1 && stride_w == 1 && pad_h == 0 && pad_w == 0;
-    if (pointwise && Cin % 8 == 0) return DenseFamily::kPointwise;
+namespace {
+constexpr int kMaxTT = 4;                // timesteps accumulated side by side, at most
+
+bool is_pointwise(int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w) {
+    return KH == 1 && KW == 1 && stride_h == 1 && stride_w == 1 && pad_h == 0 && pad_w == 0;
+}
+
+// The geometry of a layer as the dense kernels see it. A pointwise convolution has no spatial structure: each image is one row of
+// H * W pixels.
+ConvGeom layer_geom(int N, int Cin, int H, int W, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w, const PackGeom& pg) {
     ConvGeom g = {};
     g.N = N; g.Cin = Cin; g.Cout = Cout; g.KH = KH; g.KW = KW;
-    g.H = pointwise ? 1 : H; g.W = pointwise ? H * W : W;
     g.sh = stride_h; g.sw = stride_w; g.ph = pad_h; g.pw = pad_w;
+    const bool pointwise = is_pointwise(KH, KW, stride_h, stride_w, pad_h, pad_w);
+    g.H = pointwise ? 1 : H;
+    g.W = pointwise ? H * W : W;
     g.Ho = (g.H + 2 * pad_h - KH) / stride_h + 1;
     g.Wo = (g.W + 2 * pad_w - KW) / stride_w + 1;
-    const PackGeom pg = make_pack_geom(Cout, Cin, KH, KW, false);
     g.CK = pg.CK; g.nchunks = pg.nchunks; g.npairs = pg.npairs; g.nchunks_r = pg.nchunks_r;
     while ((8 << g.groups_log2) < pg.CK) ++g.groups_log2;
     g.pitch = pg.CK * 2 + 16;
-    const int64_t plane = static_cast<int64_t>(g.Ho) * g.Wo;
-    const int vec = plane % 8 == 0 ? 8 : (plane % 4 == 0 ? 4 : 0);
-    if (Cin % 8 == 0 || Cin < 8) {
-        for (int tt = T >= 3 ? 4 : T; tt >= 1; tt >>= 1) {
-            MmPlan p = {};
-            if (!plan_mm(g, tt, (g.W % 2 == 0 || g.W >= 3) ? LOAD_PAIR32 : LOAD_2X16, vec, 8, p)) continue;
-            if (Cout % 64 == 0 && p.all_full && p.run >= 4) return DenseFamily::kMatrixWhole;
-            if (tt < 4) return DenseFamily::kMatrixMasked;
+    return g;
+}
+
+// What the choice of a kernel depends on beside the geometry.
+struct ChoiceInput {
+    int T, xsize;
+    bool all_shared;                     // every timestep reads the same tensor
+    bool analog_out;                     // no neuron
+    bool x_rowbits;                      // row-packed spikes in: only the pointwise kernel reads them
+    bool usual_neuron, v_f32;            // charge by a scale and hard reset; membrane in fp32
+    bool vec_ok, vec4_ok;                // runs of 8 / 4 output pixels may be accessed as vectors
+    bool pair_aligned;                   // pixel pairs of a row may be loaded as 4 bytes
+};
+
+struct Choice {
+    bool planned = false, mm_kernel = false, pw_kernel = false, time_outer = false;
+    int window = 0;                      // timesteps per launch
+    Plan pl = {};
+    MmPlan mp = {};
+    int load_mode = 0, mm_load_mode = 0;
+};
+
+// Kernel choice. Layers whose arithmetic intensity is far below the matrix-core / HBM ridge (about 300 flop/byte)
+// run the time-outer kernel (small footprint, two workgroups per CU, membrane resident for any T); the others
+// accumulate up to 4 timesteps side by side so that each weight fragment load feeds 4x the matrix work.
+Choice choose_kernel(const ConvGeom& g, const ChoiceInput& c) {
+    Choice r;
+    Plan& pl = r.pl;
+    MmPlan& mp = r.mp;
+    int& window = r.window;
+    bool &planned = r.planned, &pw_kernel = r.pw_kernel, &mm_kernel = r.mm_kernel, &time_outer = r.time_outer;
+    const int T = c.T, N = g.N, Cin = g.Cin, Cout = g.Cout, xsize = c.xsize;
+    const bool all_shared = c.all_shared, vec_ok = c.vec_ok;
+    const bool pointwise = is_pointwise(g.KH, g.KW, g.sh, g.sw, g.ph, g.pw);
+    const int load_mode = r.load_mode = xsize == 4 ? LOAD_2XF32 : (c.pair_aligned ? LOAD_PAIR32 : LOAD_2X16);
+    // The matrix kernel also pairs the pixels of planes of odd width (2 columns or more): 4-byte loads at 2-byte alignment.
+    const int mm_load_mode = r.mm_load_mode = (xsize == 2 && g.W % 2 == 1 && g.W >= 3) ? LOAD_PAIR32 : load_mode;
+    const double out_plane = static_cast<double>(g.Ho) * g.Wo, in_plane = static_cast<double>(g.H) * g.W;
+    const double flops = 2.0 * (all_shared ? 1 : T) * N * out_plane * Cout * Cin * g.KH * g.KW;
+    const double bytes = static_cast<double>(xsize) * ((all_shared ? 1 : T) * static_cast<double>(N) * Cin * in_plane +
+                                                       static_cast<double>(T) * N * Cout * out_plane) +
+                         4.0 * N * Cout * out_plane;
+    // Dense layers whose input channels fill whole groups of 8 (or fit a single group) go to the 8-wave matrix kernel
+    // whatever their intensity (its per-tile cost is the lower one); pointwise layers stay with the pointwise kernel unless
+    // they are compute bound (deep 512 -> 512 layers: an image is then one row of H * W pixels to the matrix kernel).
+    // Measured on 1x1 layers of more than one channel chunk (T = 4, us on the pointwise / the matrix kernel): 256 -> 256 at 28^2
+    // x 32 images (128 MB) 79 / 55, 256 -> 512 at 28^2 x 16 (103 MB) 78 / 51, 192 -> 64 at 28^2 x 32 (58 MB) 57 / 32, 384 -> 96 at
+    // 14^2 x 32 (26 MB) 42 / 36, 1024 -> 64 at 8^2 x 8 56 / 54, but 256 -> 128 at 56^2 x 32 (360 MB) 90 / 139: the pointwise
+    // kernel keeps the layers that are mostly memory traffic.
+    const bool pointwise_to_matrix = !c.x_rowbits && pointwise && (flops / bytes >= 200.0 || (Cin > 128 && bytes < 200.0e6));
+    // A neuron-free pointwise layer (snnf_conv_bias) has no other kernel to go to: the pointwise kernel always runs a neuron.
+    const bool matrix_candidate = (!pointwise || pointwise_to_matrix || (c.analog_out && !c.x_rowbits)) && (Cin % 8 == 0 || Cin < 8);
+    if (matrix_candidate) {
+        // 8-wave matrix kernel: the largest window of 4, 2 or 1 timesteps whose halo tiles fit LDS.
+        // One analog frame for all T: a single stage of input (TT = 1), up to 16 LIF steps per launch.
+        int w2 = 1;
+        while (!all_shared && w2 < T && w2 < kMaxTT) w2 *= 2;
+        const bool fast_layer = Cout % 64 == 0 && c.v_f32 && c.usual_neuron;
+        const int vec = vec_ok ? 8 : (c.vec4_ok ? 4 : 0);
+        for (; w2 >= 1 && !mm_kernel; w2 >>= 1) {
+            MmPlan p8 = {}, p4 = {};
+            const bool ok8 = plan_mm(g, w2, mm_load_mode, vec, 8, p8);
+            // One shared frame: a single short matrix stage, then T steps of epilogue per tile. Two 4-wave workgroups per
+            // CU (fast variant only) overlap one's epilogue with the other's loads and matrix work; measured 15 % faster on
+            // a 7x7/2 stem, slower on every layer with a deep matrix loop.
+            const bool ok4 = all_shared && fast_layer && plan_mm(g, w2, mm_load_mode, vec, 4, p4) && p4.all_full && p4.run >= 4;
+            if (!ok8 && !ok4) continue;
+            mp = ok4 ? p4 : p8;
+            // The masked variant with 4 timesteps of accumulators spills registers (and every reload then waits behind
+            // the activation prefetch): it runs windows of 2.
+            const bool fast_plan = fast_layer && mp.all_full && mp.run >= 4;
+            if (w2 == 4 && !fast_plan) continue;
+            mm_kernel = planned = true;
+            window = w2;
+        }
+        if (mm_kernel && all_shared) window = T < SNNF_MAX_T_PER_LAUNCH ? T : SNNF_MAX_T_PER_LAUNCH;
+        if (mm_kernel) {
+            pl.TH = mp.TH; pl.TW = mp.TW; pl.tiles_x = mp.tiles_x; pl.tiles_y = mp.tiles_y; pl.NR = mp.NR; pl.WT = mp.WT;
+            pl.wm_log2 = mp.wm_log2; pl.wn_log2 = mp.wn_log2; pl.oc_tiles = mp.oc_tiles; pl.lds_bytes = mp.lds_bytes;
         }
     }
-    const double flops = 2.0 * T * N * plane * Cout * Cin * KH * KW;
-    const double bytes = 2.0 * (static_cast<double>(T) * N * Cin * H * W + static_cast<double>(T) * N * Cout * plane) + 4.0 * N * Cout * plane;
-    Plan pl = {};
-    return flops / bytes < 200.0 && plan(g, 1, 0, g.W % 2 == 0 ? LOAD_PAIR32 : LOAD_2X16, vec == 8, pl) ? DenseFamily::kTimeOuter : DenseFamily::kTInM;
+    if (c.analog_out && !mm_kernel) return r;
+    // Everything else: the time-outer kernels for a shared frame or a low intensity, the 4-wave T-in-M kernel otherwise.
+    time_outer = !mm_kernel && (all_shared || c.x_rowbits || flops / bytes < 200.0);
+    if (time_outer && pointwise && Cin % 8 == 0 && static_cast<int64_t>(Cout) * g.Wo < (1LL << 30)) {
+        // Pointwise kernel: flat tiles of 64 pixels x 128 output channels, no planning needed.
+        pw_kernel = planned = true;
+        window = T < SNNF_MAX_T_PER_LAUNCH ? T : SNNF_MAX_T_PER_LAUNCH;
+        pl.TH = 1; pl.TW = 64; pl.tiles_x = (g.Wo + 63) / 64; pl.tiles_y = N; pl.NR = 1; pl.WT = 64;
+        pl.wm_log2 = 0; pl.wn_log2 = 2; pl.oc_tiles = (Cout + 127) / 128;
+        pl.lds_bytes = 0;
+    } else if (time_outer) {
+        planned = plan(g, 1, 0, load_mode, vec_ok, pl);
+        window = T < SNNF_MAX_T_PER_LAUNCH ? T : SNNF_MAX_T_PER_LAUNCH;
+        if (!planned) time_outer = false;
+    }
+    if (!time_outer && !mm_kernel) {
+        // Timesteps per launch: as many (<= 4) as fit LDS side by side; a shared analog frame needs one tile for any window.
+        window = T < kMaxTT ? T : kMaxTT;
+        int w2 = 1;
+        while (w2 < window) w2 *= 2;
+        window = w2;
+        while (true) {
+            planned = plan(g, all_shared ? 1 : window, window, load_mode, vec_ok, pl);
+            if (planned || window == 1) break;
+            window >>= 1;
+        }
+    }
+    return r;
+}
+}  // namespace
+
+// The kernel that snnf_conv_lif chooses for a layer of 16-bit activations, an fp32 membrane and the usual neuron, when every operand is
+// 16-byte aligned and the steps have inputs of their own.
+DenseFamily dense_family(int T, int N, int Cin, int H, int W, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w) {
+    const ConvGeom g = layer_geom(N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, make_pack_geom(Cout, Cin, KH, KW, false));
+    const int64_t plane = static_cast<int64_t>(g.Ho) * g.Wo;
+    const Choice c = choose_kernel(g, ChoiceInput{T, 2, false, false, false, true, true, plane % 8 == 0, plane % 4 == 0, g.W % 2 == 0});
+    if (c.mm_kernel) return Cout % 64 == 0 && c.mp.all_full && c.mp.run >= 4 ? DenseFamily::kMatrixWhole : DenseFamily::kMatrixMasked;
+    return c.pw_kernel ? DenseFamily::kPointwise : (c.time_outer ? DenseFamily::kTimeOuter : DenseFamily::kTInM);
 }
 
 namespace {
@@ -309,23 +421,9 @@ int conv_lif_impl(const void* const* xs, const void* const* residuals, int T, in
     if (static_cast<int64_t>(N) * Cin * H * W >= (1LL << 30) || static_cast<int64_t>(N) * Cout * Ho_real * Wo_real >= (1LL << 31))
         return fail(SNNF_ERR_UNSUPPORTED, "snnf_conv_lif: unsupported_shape: more than 2^30 input elements per timestep");
 
-    ConvGeom g = {};
-    g.N = N; g.Cin = Cin; g.Cout = Cout; g.KH = KH; g.KW = KW;
-    g.sh = stride_h; g.sw = stride_w; g.ph = pad_h; g.pw = pad_w;
-    const bool pointwise = KH == 1 && KW == 1 && stride_h == 1 && stride_w == 1 && pad_h == 0 && pad_w == 0;
-    if (pointwise) {
-        // A pointwise convolution has no spatial structure: treat each image as one row of H * W pixels.
-        g.H = 1; g.W = H * W;
-    } else {
-        g.H = H; g.W = W;
-    }
-    g.Ho = (g.H + 2 * pad_h - KH) / stride_h + 1;
-    g.Wo = (g.W + 2 * pad_w - KW) / stride_w + 1;
+    const bool pointwise = is_pointwise(KH, KW, stride_h, stride_w, pad_h, pad_w);
     const PackGeom pg = make_pack_geom(Cout, Cin, KH, KW, x_dtype == SNNF_F32);
-    g.CK = pg.CK; g.nchunks = pg.nchunks; g.npairs = pg.npairs; g.nchunks_r = pg.nchunks_r;
-    g.groups_log2 = 0;
-    while ((8 << g.groups_log2) < pg.CK) ++g.groups_log2;
-    g.pitch = pg.CK * 2 + 16;
+    ConvGeom g = layer_geom(N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, pg);
     g.spike_step_stride = spike_step_stride;
     g.v_is_f32 = v_dtype == SNNF_F32 ? 1 : 0;
     g.analog_out = analog_out ? 1 : 0;
@@ -333,7 +431,6 @@ int conv_lif_impl(const void* const* xs, const void* const* residuals, int T, in
     const LifParams lif = make_lif_params(v_threshold, v_reset, tau);
     hipStream_t hs = as_stream(stream);
 
-    constexpr int kMaxTT = 4;
     bool all_shared = T > 1;
     bool pair_aligned = xsize == 2 && (g.W % 2 == 0);
     // 8 consecutive output pixels start 16-byte aligned whenever their first pixel offset is a multiple of 8.
@@ -348,24 +445,6 @@ int conv_lif_impl(const void* const* xs, const void* const* residuals, int T, in
         if (residuals != nullptr) vec_ok = vec_ok && aligned_to(residuals[t], 16);
         if (residuals != nullptr) vec4_ok = vec4_ok && aligned_to(residuals[t], 8);
     }
-    const int load_mode = xsize == 4 ? LOAD_2XF32 : (pair_aligned ? LOAD_PAIR32 : LOAD_2X16);
-    // The matrix kernel also pairs the pixels of planes of odd width (2 columns or more): 4-byte loads at 2-byte alignment.
-    const int mm_load_mode = (xsize == 2 && g.W % 2 == 1 && g.W >= 3) ? LOAD_PAIR32 : load_mode;
-
-    // Kernel choice. Layers whose arithmetic intensity is far below the matrix-core / HBM ridge (about 300 flop/byte)
-    // run the time-outer kernel (small footprint, two workgroups per CU, membrane resident for any T); the others
-    // accumulate up to 4 timesteps side by side so that each weight fragment load feeds 4x the matrix work.
-    const double flops = 2.0 * (all_shared ? 1 : T) * N * static_cast<double>(Ho_real) * Wo_real * Cout * Cin * KH * KW;
-    const double bytes = static_cast<double>(xsize) * ((all_shared ? 1 : T) * static_cast<double>(N) * Cin * H * W +
-                                                       static_cast<double>(T) * N * Cout * Ho_real * Wo_real) +
-                         4.0 * N * Cout * Ho_real * Wo_real;
-    // Dense layers whose input channels fill whole groups of 8 (or fit a single group) go to the 8-wave matrix kernel
-    // whatever their intensity (its per-tile cost is the lower one); pointwise layers stay with the pointwise kernel unless
-    // they are compute bound (deep 512 -> 512 layers: an image is then one row of H * W pixels to the matrix kernel).
-    // Measured on 1x1 layers of more than one channel chunk (T = 4, us on the pointwise / the matrix kernel): 256 -> 256 at 28^2
-    // x 32 images (128 MB) 79 / 55, 256 -> 512 at 28^2 x 16 (103 MB) 78 / 51, 192 -> 64 at 28^2 x 32 (58 MB) 57 / 32, 384 -> 96 at
-    // 14^2 x 32 (26 MB) 42 / 36, 1024 -> 64 at 8^2 x 8 56 / 54, but 256 -> 128 at 56^2 x 32 (360 MB) 90 / 139: the pointwise
-    // kernel keeps the layers that are mostly memory traffic.
     // Row-packed spikes in (`x_rowbits`): xs[t] are [N][Cin][H * W / 8] bytes; only the pointwise kernel's fast variant reads them.
     if (x_rowbits) {
         const bool fast_neuron = lif.charge_mode == CHARGE_SCALE && !lif.soft_reset;
@@ -379,49 +458,15 @@ int conv_lif_impl(const void* const* xs, const void* const* residuals, int T, in
         return fail(SNNF_ERR_UNSUPPORTED, "snnf_pwconv_lif_rowbits: row-packed output needs row-packed input");
     }
     g.bits_out = out_rowbits ? 1 : 0;
-    const bool pointwise_to_matrix = !x_rowbits && pointwise && (flops / bytes >= 200.0 || (Cin > 128 && bytes < 200.0e6));
-    // A neuron-free pointwise layer (snnf_conv_bias) has no other kernel to go to: the pointwise kernel always runs a neuron.
-    const bool matrix_candidate = (!pointwise || pointwise_to_matrix || (analog_out && !x_rowbits)) && (Cin % 8 == 0 || Cin < 8);
-    int window = 0;
-    Plan pl = {};
-    bool planned = false;
-    bool pw_kernel = false;
-    bool mm_kernel = false;
-    MmPlan mp = {};
-    if (matrix_candidate) {
-        // 8-wave matrix kernel: the largest window of 4, 2 or 1 timesteps whose halo tiles fit LDS.
-        // One analog frame for all T: a single stage of input (TT = 1), up to 16 LIF steps per launch.
-        int w2 = 1;
-        while (!all_shared && w2 < T && w2 < kMaxTT) w2 *= 2;
-        const bool fast_layer = Cout % 64 == 0 && v_dtype == SNNF_F32 && lif.charge_mode == CHARGE_SCALE && !lif.soft_reset;
-        const int vec = vec_ok ? 8 : (vec4_ok ? 4 : 0);
-        for (; w2 >= 1 && !mm_kernel; w2 >>= 1) {
-            MmPlan p8 = {}, p4 = {};
-            const bool ok8 = plan_mm(g, w2, mm_load_mode, vec, 8, p8);
-            // One shared frame: a single short matrix stage, then T steps of epilogue per tile. Two 4-wave workgroups per
-            // CU (fast variant only) overlap one's epilogue with the other's loads and matrix work; measured 15 % faster on
-            // a 7x7/2 stem, slower on every layer with a deep matrix loop.
-            const bool ok4 = all_shared && fast_layer && plan_mm(g, w2, mm_load_mode, vec, 4, p4) && p4.all_full && p4.run >= 4;
-            if (!ok8 && !ok4) continue;
-            mp = ok4 ? p4 : p8;
-            // The masked variant with 4 timesteps of accumulators spills registers (and every reload then waits behind
-            // the activation prefetch): it runs windows of 2.
-            const bool fast_plan = fast_layer && mp.all_full && mp.run >= 4;
-            if (w2 == 4 && !fast_plan) continue;
-            mm_kernel = planned = true;
-            window = w2;
-        }
-        if (mm_kernel && all_shared) window = T < SNNF_MAX_T_PER_LAUNCH ? T : SNNF_MAX_T_PER_LAUNCH;
-        if (mm_kernel) {
-            pl.TH = mp.TH; pl.TW = mp.TW; pl.tiles_x = mp.tiles_x; pl.tiles_y = mp.tiles_y; pl.NR = mp.NR; pl.WT = mp.WT;
-            pl.wm_log2 = mp.wm_log2; pl.wn_log2 = mp.wn_log2; pl.oc_tiles = mp.oc_tiles; pl.lds_bytes = mp.lds_bytes;
-        }
-    }
+    const bool usual_neuron = lif.charge_mode == CHARGE_SCALE && !lif.soft_reset;
+    const Choice choice = choose_kernel(g, ChoiceInput{T, xsize, all_shared, analog_out, x_rowbits, usual_neuron, v_dtype == SNNF_F32, vec_ok, vec4_ok, pair_aligned});
+    const bool planned = choice.planned, mm_kernel = choice.mm_kernel, pw_kernel = choice.pw_kernel, time_outer = choice.time_outer;
+    const int window = choice.window, load_mode = choice.load_mode, mm_load_mode = choice.mm_load_mode;
+    const MmPlan& mp = choice.mp;
+    const Plan& pl = choice.pl;
     if (analog_out && !mm_kernel)
         return fail(SNNF_ERR_UNSUPPORTED, "snnf_conv_bias: unsupported_shape: only layers the 8-wave matrix kernel takes "
                     "(Cin %% 8 == 0 or Cin < 8, tiles that fit LDS)");
-    // Everything else: the time-outer kernels for a shared frame or a low intensity, the 4-wave T-in-M kernel otherwise.
-    bool time_outer = !mm_kernel && (all_shared || x_rowbits || flops / bytes < 200.0);
     // Pointwise kernel: where the weight fragments live (registers only in the fast variant) and the LDS that takes.
     auto pw_config = [&](bool allow_regs, ConvGeom& gg) -> size_t {
         const size_t xb = static_cast<size_t>(64) * gg.pitch;
@@ -441,30 +486,6 @@ int conv_lif_impl(const void* const* xs, const void* const* residuals, int T, in
         }
         return bytes;
     };
-    if (time_outer && pointwise && Cin % 8 == 0 && static_cast<int64_t>(Cout) * g.Wo < (1LL << 30)) {
-        // Pointwise kernel: flat tiles of 64 pixels x 128 output channels, no planning needed.
-        pw_kernel = planned = true;
-        window = T < SNNF_MAX_T_PER_LAUNCH ? T : SNNF_MAX_T_PER_LAUNCH;
-        pl.TH = 1; pl.TW = 64; pl.tiles_x = (g.Wo + 63) / 64; pl.tiles_y = N; pl.NR = 1; pl.WT = 64;
-        pl.wm_log2 = 0; pl.wn_log2 = 2; pl.oc_tiles = (Cout + 127) / 128;
-        pl.lds_bytes = 0;
-    } else if (time_outer) {
-        planned = plan(g, 1, 0, load_mode, vec_ok, pl);
-        window = T < SNNF_MAX_T_PER_LAUNCH ? T : SNNF_MAX_T_PER_LAUNCH;
-        if (!planned) time_outer = false;
-    }
-    if (!time_outer && !mm_kernel) {
-        // Timesteps per launch: as many (<= 4) as fit LDS side by side; a shared analog frame needs one tile for any window.
-        window = T < kMaxTT ? T : kMaxTT;
-        int w2 = 1;
-        while (w2 < window) w2 *= 2;
-        window = w2;
-        while (true) {
-            planned = plan(g, all_shared ? 1 : window, window, load_mode, vec_ok, pl);
-            if (planned || window == 1) break;
-            window >>= 1;
-        }
-    }
     if (!planned)
         return fail(SNNF_ERR_UNSUPPORTED, "snnf_conv_lif: unsupported_shape: no activation tile fits LDS (W=%d, kernel %dx%d, stride %dx%d)",
                     W, KH, KW, stride_h, stride_w);
