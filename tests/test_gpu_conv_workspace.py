@@ -54,7 +54,8 @@ def test_conv_through_the_blocked_layout(snnf_lib, Cin, Cout, H, W, k, s, T, N, 
         _lib.check(name, snnf_lib.snnf_conv_lif_ws(
             _lib.step_pointers(dx), _lib.step_pointers(dr) if residual else None, T, N, Cin, H, W, code, packed.data_ptr(), Cout, k, k, s, s, p, p,
             _lib.ptr(dv), 0, sp.data_ptr(), int(sp.stride(0)), v.data_ptr(), *LIF, workspace.data_ptr(), given, _lib.current_stream(sp.device)))
-        assert (CB.last_conv_plan().get("route") == "c8") == (name == "blocked"), CB.last_conv_plan()
+        plan = CB.last_conv_plan()
+        assert (plan.get("route") == "c8") == (plan.get("ran") == "blocked") == (name == "blocked"), plan
         check(sp, v, ref, what=f"{name} {Cin}->{Cout} {H}x{W}")
         results[name] = (sp, v)
         families[name] = CB.last_conv_plan()["kernel"]
@@ -95,6 +96,7 @@ def test_waves_that_share_a_tile(snnf_lib, Cin, Cout, H, W, N, waves, groups, ti
     out, v = B.conv_lif_blocked(B.from_dense(dev(x, BF16), B.BITS), dev(w, BF16), dev(b, BF16), [1, 1], [1, 1], LIF, out_layout=B.BITS, want_v=True)
     plan = B.last_conv_plan()
     assert (plan["waves"], int(plan["stage_chunks"]), int(plan["oc_tiles"])) == (waves, groups, tiles), plan
+    assert plan["oc_tiles"] == -(-Cout // plan["oc_tile"])
     check(B.to_dense(out), v, ref, what=f"{Cin}->{Cout} {H}x{W} x {N}")
 
 

@@ -532,9 +532,23 @@ def test_dense_conv_lif_shapes_outside_the_matrix_and_pointwise_kernels(hip_ops,
         sp, v = S.fused_temporal_conv_add_lif_state(dx, [dev(r, dtype) for r in rs], dw, db, dv, *geo, *lif, False)
     else:
         sp, v = S.fused_temporal_conv_lif_state(dx, dw, db, dv, *geo, *lif, False)
-    assert last_conv_plan()["kernel"] == family, last_conv_plan()
+    plan = last_conv_plan()
+    assert plan["kernel"] == family, plan
     check(sp, v, ref, v_threshold=lif[0], v_dtype=vdtype, what=f"{family} {Cin}->{Cout} k{k} s{stride} {H}x{W}")
     _no_fallback(hip_ops, 1)
+    if "ran" in plan:       # the operator brought the layer into the blocked layout: the family's kernel itself, through its own entry point
+        from triton_snn_fusion_amd import _lib
+        from triton_snn_fusion_amd.runtime import hip_convlif_backend as CB
+        packed, lib = CB._packed_weight(dw, db, dtype), _lib.lib()
+        dr, dv = [dev(r, dtype) for r in rs] if residual else None, dev(v0, F32) if tensor_v else None
+        sp, v = torch.empty_like(sp), torch.empty(N, Cout, Ho, Wo, device=DEV)
+        _lib.check("snnf_conv_lif", lib.snnf_conv_lif(
+            _lib.step_pointers(dx), _lib.step_pointers(dr) if residual else None, T, N, Cin, H, W, _lib.dtype_code(dtype),
+            packed.data_ptr(), Cout, k, k, stride, stride, pad, pad, _lib.ptr(dv), _lib.SNNF_F32, sp.data_ptr(),
+            int(sp.stride(0)), v.data_ptr(), *lif, _lib.current_stream(sp.device)))
+        plan = last_conv_plan()
+        assert plan["kernel"] == family and "ran" not in plan, plan
+        check(sp, v, ref, v_threshold=lif[0], v_dtype=F32, what=f"{family} alone {Cin}->{Cout} k{k} s{stride} {H}x{W}")
 
 
 def test_planes_of_four_pixels_with_several_images_per_tile(hip_ops):

@@ -75,10 +75,11 @@ def test_random_dense_conv_lif_cases(hip_ops, seed, cases):
         sp, v = op(*args, dev(w, dtype), dev(b, dtype), v_dev, [s, s], [p, p], [1, 1], groups, *lif, False)
         assert sp.dtype == dtype and v.dtype == vdtype
         check(sp, v, ref, v_threshold=lif[0], v_dtype=vdtype, what=what, max_rate=2e-4)
-        kernels["depthwise" if depthwise else CB.last_conv_plan()["kernel"]] += 1
+        plan = {} if depthwise else CB.last_conv_plan()
+        kernels["depthwise" if depthwise else plan.get("ran", plan["kernel"])] += 1      # what ran, not the family that the layer belongs to
     print(dict(kernels), flush=True)
     assert hip_ops.get_fused_op_call_stats()["fallback"] == 0
-    assert set(kernels) >= {"matrix", "pointwise", "time_outer", "t_in_m", "depthwise"}, kernels   # the sweep reaches every family
+    assert set(kernels) >= {"matrix", "pointwise", "time_outer", "t_in_m", "depthwise", "blocked"}, kernels   # the sweep reaches every family
 
 
 @pytest.mark.parametrize("seed,cases", [(12, 400)])

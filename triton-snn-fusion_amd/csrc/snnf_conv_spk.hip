@@ -576,10 +576,10 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
                           L.lif.v_threshold >= 1e-30f && L.lif.v_threshold <= 1e30f &&   // its multiples by 2^t stay normal numbers
                           v_init == nullptr && p.windows == 1 && Cout % 8 == 0;
     snprintf(snnf::conv_plan_buffer(), 256,
-             "kernel=%s variant=%d window=%d launches=%d tile=%dx%dx%d halo=%dx%d waves=8x1x%d oc_tiles=%d px_tiles=%d "
+             "kernel=%s variant=%d window=%d launches=%d tile=%dx%dx%d halo=%dx%d waves=8x1x%d oc_tiles=%d oc_tile=%d px_tiles=%d "
              "stage_chunks=%d run=0 lds=%zu grid=%d tuned=%d shortcut_stages=%d%s",
-             dense != nullptr ? family_name(dense->family) : "blocked", (p.wk_log2 > 0 ? 50 : 40) + p.tt + (fast_epi ? 20 : 0), shared ? T : p.tt, dense != nullptr ? 2 : 1, g.PI, g.PR, g.PC, g.RR, g.RC, 1 << p.wk_log2, p.oc_tiles, g.n_patches, g.G,
-             L.lds_bytes, p.grid, (p.tuned_patch ? 1 : 0) + (p.tuned_split ? 2 : 0), g.sc_stages, dense != nullptr ? " route=c8" : "");
+             dense != nullptr ? family_name(dense->family) : "blocked", (p.wk_log2 > 0 ? 50 : 40) + p.tt + (fast_epi ? 20 : 0), shared ? T : p.tt, dense != nullptr ? 2 : 1, g.PI, g.PR, g.PC, g.RR, g.RC, 1 << p.wk_log2, p.oc_tiles, g.narrow ? 32 : 64, g.n_patches, g.G,
+             L.lds_bytes, p.grid, (p.tuned_patch ? 1 : 0) + (p.tuned_split ? 2 : 0), g.sc_stages, dense != nullptr ? " route=c8 ran=blocked" : "");
     L.fast_epilogue = fast_epi;
     if (dense != nullptr) {   // the plan stands: bring the dense inputs into the C8 buffers behind `xs`
         StepPtrs from = {};

@@ -242,7 +242,8 @@ def get_autotune_best_config(kernel_key: str, residual_add: bool = False, T: int
 
 def last_conv_plan() -> Dict:
     """What the planner selected for this thread's most recent matrix-core convolution launch (snnf_conv_last_plan):
-    kernel family, timesteps per launch, tile and wave decomposition, LDS bytes and grid, as a dict."""
+    kernel family, timesteps per launch, tile and wave decomposition, LDS bytes and grid, as a dict. `ran` is there when another
+    kernel than the family's ran (the blocked one, for a layer that was brought into its layout)."""
     text = _lib.lib().snnf_conv_last_plan().decode("ascii", "replace")
     plan: Dict = {}
     for item in text.split():
