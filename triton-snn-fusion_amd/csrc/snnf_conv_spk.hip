@@ -97,10 +97,14 @@ size_t c8_step_bytes(int N, int Cin, int H, int W) { return static_cast<size_t>(
 // but 344 -> 16 at 20 x 37, 5x5, T = 2 106 / 71, 304 -> 208 at 15^2, T = 1 27 / 19. More than four timesteps are several windows here as
 // well, over which few channels do not pay: 40 -> 16 at 24 x 59, 5x5, T = 5 41 / 56, 48 -> 16 at 66 x 103, 7x7, T = 8 80 / 95, but 56 -> 184 at
 // 17^2, 7x7, T = 5 63 / 46, 72 -> 184 at 7^2, T = 8 134 / 39.
-// Whole tiles stay (64 -> 64 at 56^2 x 16 37 / 50, 128 -> 128 at 28^2 x 16 40 / 40 and with a residual 42 / 50, 256 -> 256 at 14^2 x 16 with a
-// residual 37 / 39, at 8^2 x 64 36 / 37) but for deep layers, whose K the blocked kernel shares among more waves: 512 -> 512 at 4^2 x 16
-// 36 / 30 and with a residual 36 / 31, at 4^2 x 64 49 / 39, at 2^2 x 64 37 / 29; of 256 channels those with few outputs: 14^2 x 4
-// 28 / 23 (T = 1 15 / 14, T = 6 53 / 39), 6^2 x 16 33 / 23, 256 -> 512 at 4^2 x 64 29 / 27.
+// Whole tiles stay (64 -> 64 at 56^2 x 16 37 / 50, 128 -> 128 at 28^2 x 16 41 / 41 and with a residual 42 / 50, 192 -> 192 at 8^2 x 64 31 / 35,
+// 256 -> 256 at 8^2 x 64 37 / 37, at 14^2 x 16 with a residual 38 / 39) but for deep layers, whose K the blocked kernel shares among more
+// waves. The line, K = 2304 for few outputs and no residual and K = 4608 for any, is on the safe side: of 197 layers measured behind it, 64 to
+// 640 channels, 3x3 to 7x7, one to eight timesteps, none loses (512 -> 512 with a residual at 8^2 x 64 89 / 89, 128 -> 128 5x5 at 16^2 x 16
+// 30 / 29, 64 -> 128 7x7 at 16^2 x 16 28 / 26, 96 -> 64 5x5 at 16^2 x 16 25 / 21, 256 -> 256 at 14^2 x 4 29 / 18, 320 -> 320 34 / 27, 384 -> 384
+// 37 / 28 (T = 1 21 / 16, T = 6 71 / 47), 448 -> 448 42 / 32, 512 -> 512 46 / 33 there and 37 / 21 at 4^2 x 16). In front of it some would
+// gain as well: 320 to 448 channels with more outputs (at 14^2 x 16 60 / 55, 70 / 61, 79 / 67), and layers of few outputs with less depth or with a
+// residual (128 -> 128 at 14^2 x 4 20 / 14, 384 -> 384 with a residual at 8^2 x 4 37 / 22).
 bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w,
                          int v_dtype, bool residual, DenseFamily& family) {
     if (x_dtype != SNNF_BF16 && x_dtype != SNNF_F16) return false;
