@@ -7,7 +7,7 @@
 // there -, so the first call of a signature runs the Python implementation, which stays the only place where calls are
 // judged, refused and counted, and this file remembers a signature that ran natively together with the statistics it
 // added. Later calls of the signature are a hash look-up, two allocations and the C ABI call (measured, batch-1 neuron
-// step: 12.3 -> 5 us per call).
+// step: 12.2 -> 5.9 us per call).
 // A call whose signature is unknown, whose tensors are not plain contiguous GPU tensors, whose entry point returns an error, or
 // that throws on its way (no memory, a weight that cannot be packed) goes through the Python implementation, which raises or
 // falls back as it always did.
