@@ -248,11 +248,14 @@ int snnf_conv_lif(const void* const* xs, const void* const* residuals, int T,
  * first and run the kernel of that layout on them. The reference has no counterpart (its Triton kernel reads NCHW,
  * kernels/benchmark_conv_lif_temporal_general.py:629-676). Results are those of snnf_conv_lif up to the order of the fp32
  * additions.
- *   snnf_conv_lif_workspace_bytes : bytes with which this shape takes that route (0: the call is snnf_conv_lif). A call whose
+ *   snnf_conv_lif_scratch_bytes : bytes with which this call takes that route (0: the call is snnf_conv_lif). A call whose
  *               timesteps all read one frame never takes it and needs none.
+ *   snnf_conv_lif_workspace_bytes : the same for 16-bit activations beside an fp32 membrane, 0 for every other call.
  *   workspace : NULL (then this is snnf_conv_lif), or device memory, 16-byte aligned, contents undefined before and after.
  *               A smaller workspace than asked for is not used. Calls that share a workspace must not overlap in time.
  */
+size_t snnf_conv_lif_scratch_bytes(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW,
+                                   int stride_h, int stride_w, int pad_h, int pad_w, int v_dtype, int has_residual);
 size_t snnf_conv_lif_workspace_bytes(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW,
                                      int stride_h, int stride_w, int pad_h, int pad_w, int v_dtype, int has_residual);
 int snnf_conv_lif_ws(const void* const* xs, const void* const* residuals, int T,

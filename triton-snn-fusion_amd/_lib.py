@@ -53,6 +53,7 @@ SIGNATURES = {
     "snnf_conv_lif": (_i, [_pp, _pp, _i, _i, _i, _i, _i, _i, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _i, _vp, _i64,
                            _vp, _f, _f, _f, _vp]),
     "snnf_conv_lif_workspace_bytes": (_sz, [_i] * 15),
+    "snnf_conv_lif_scratch_bytes": (_sz, [_i] * 15),
     "snnf_conv_lif_ws": (_i, [_pp, _pp, _i, _i, _i, _i, _i, _i, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _i, _vp, _i64,
                               _vp, _f, _f, _f, _vp, _sz, _vp]),
     "snnf_layout_bytes": (_sz, [_i, _i64, _i, _i, _i, _i]),

@@ -652,7 +652,7 @@ bool conv_call(const Call& c, Attempt& key, Op op, Pair* out) {
     } else {
         const Tensor packed = packed_weight(w, b, x.scalar_type());
         const size_t bytes = one_frame(steps, T) ? 0
-            : snnf_conv_lif_workspace_bytes(static_cast<int>(T), N, cin, H, W, code_of(x.scalar_type()), static_cast<int>(shape[1]), static_cast<int>(kh),
+            : snnf_conv_lif_scratch_bytes(static_cast<int>(T), N, cin, H, W, code_of(x.scalar_type()), static_cast<int>(shape[1]), static_cast<int>(kh),
                                             static_cast<int>(kw), static_cast<int>(sh), static_cast<int>(sw), static_cast<int>(ph), static_cast<int>(pw),
                                             wm.code(), residual ? 1 : 0);
         Tensor workspace;

@@ -201,6 +201,6 @@ int launch_conv_mm_w4_f16(const ConvLaunch& L, int tt, int load_mode);
 
 // The kernels behind snnf_conv_lif (snnf_conv_igemm.hip).
 enum class DenseFamily { kTInM, kTimeOuter, kMatrixMasked, kMatrixWhole, kPointwise };
-DenseFamily dense_family(int T, int N, int Cin, int H, int W, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w);
+DenseFamily dense_family(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w);
 
 }  // namespace snnf

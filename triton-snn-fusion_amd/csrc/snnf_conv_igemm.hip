@@ -379,12 +379,12 @@ Choice choose_kernel(const ConvGeom& g, const ChoiceInput& c) {
 }
 }  // namespace
 
-// The kernel that snnf_conv_lif chooses for a layer of 16-bit activations, an fp32 membrane and the usual neuron, when every operand is
+// The kernel that snnf_conv_lif chooses for a layer of activations of `x_dtype`, an fp32 membrane and the usual neuron, when every operand is
 // 16-byte aligned and the steps have inputs of their own.
-DenseFamily dense_family(int T, int N, int Cin, int H, int W, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w) {
-    const ConvGeom g = layer_geom(N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, make_pack_geom(Cout, Cin, KH, KW, false));
+DenseFamily dense_family(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w) {
+    const ConvGeom g = layer_geom(N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, make_pack_geom(Cout, Cin, KH, KW, x_dtype == SNNF_F32));
     const int64_t plane = static_cast<int64_t>(g.Ho) * g.Wo;
-    const Choice c = choose_kernel(g, ChoiceInput{T, 2, false, false, false, true, true, plane % 8 == 0, plane % 4 == 0, g.W % 2 == 0});
+    const Choice c = choose_kernel(g, ChoiceInput{T, dtype_size(x_dtype), false, false, false, true, true, plane % 8 == 0, plane % 4 == 0, g.W % 2 == 0});
     if (c.mm_kernel) return Cout % 64 == 0 && c.mp.all_full && c.mp.run >= 4 ? DenseFamily::kMatrixWhole : DenseFamily::kMatrixMasked;
     return c.pw_kernel ? DenseFamily::kPointwise : (c.time_outer ? DenseFamily::kTimeOuter : DenseFamily::kTInM);
 }

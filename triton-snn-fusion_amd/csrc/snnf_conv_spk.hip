@@ -34,7 +34,7 @@ bool plan_spk(const SpkGeom& g0, int tt, SpkPlan& best, int only_pc = 0, int onl
         // fewer tiles than half the compute units; a tile's K is shared by the eight waves of a workgroup at that size, so tiles
         // are workgroups (512 -> 512 on 2 x 2 planes at batch 64: 64 workgroups of 8 images 24.1 us, 128 of 4 images 21.3 us,
         // 256 of 2 images 22.6 us, single images 34.7 us).
-        const int oc_tiles = (g0.Cout + 63) / 64;
+        const int oc_tiles = g0.narrow ? (g0.Cout + 31) / 32 : (g0.Cout + 63) / 64;
         if (pi > 1 && ((g0.N + pi - 1) / pi) * oc_tiles * 2 < cus) pi >>= 1;
         const int rr = (pr - 1) * g0.sh + g0.KH;
         const int rc = (pc - 1) * g0.sw + g0.KW;
@@ -84,6 +84,23 @@ std::map<TunedKey, TunedPlan>& tuned_plans() {
 
 size_t c8_step_bytes(int N, int Cin, int H, int W) { return static_cast<size_t>(N) * ((Cin + 7) / 8) * H * W * 16; }
 
+// The workspace of a call on the blocked route: the C8 steps; of fp32 tensors the steps of their low terms and the flags behind them.
+struct RouteSpace {
+    size_t step, lo, flags, flag_stride, total;        // bytes; offsets of the low terms and of the flags
+};
+RouteSpace route_space(int T, int N, int Cin, int H, int W, bool split) {
+    RouteSpace r = {};
+    r.step = c8_step_bytes(N, Cin, H, W);
+    r.total = r.step * T;
+    if (split) {
+        r.lo = r.total;
+        r.flags = 2 * r.total;
+        r.flag_stride = (r.step / 16 + 255) / 256 * 4;   // one byte per 64 items, in whole dwords
+        r.total = r.flags + r.flag_stride * T;
+    }
+    return r;
+}
+
 // Whether a layer on dense tensors is brought into C8 and run on the blocked kernel (two launches) or stays on the dense kernels.
 // Measured (bf16, T = 4 unless said, us, dense / this route). Channel counts that are no multiple of 8 only have the four-wave kernels
 // on dense tensors, which assemble every channel group from scalar loads: 230 -> 144 at 11 x 83 stride 2 650 / 32, 167 -> 64 at
@@ -107,7 +124,7 @@ size_t c8_step_bytes(int N, int Cin, int H, int W) { return static_cast<size_t>(
 // residual (128 -> 128 at 14^2 x 4 20 / 14, 384 -> 384 with a residual at 8^2 x 4 37 / 22).
 bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w,
                          int v_dtype, bool residual, DenseFamily& family) {
-    if (x_dtype != SNNF_BF16 && x_dtype != SNNF_F16) return false;
+    if (x_dtype != SNNF_BF16 && x_dtype != SNNF_F16 && x_dtype != SNNF_F32) return false;
     if (v_dtype != SNNF_F32 || T < 1 || T > SNNF_MAX_T_PER_LAUNCH || N < 1 || Cin < 1 || H < 1 || W < 1 || Cout < 1 || KH < 1 || KW < 1 ||
         stride_h < 1 || stride_w < 1 || pad_h < 0 || pad_w < 0 || H + 2 * pad_h < KH || W + 2 * pad_w < KW || 2 * pad_h > KH || 2 * pad_w > KW) return false;
     const bool pointwise = KH == 1 && KW == 1 && stride_h == 1 && stride_w == 1 && pad_h == 0 && pad_w == 0;
@@ -115,8 +132,15 @@ bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int C
     const int64_t out = static_cast<int64_t>(N) * Cout * ((H + 2 * pad_h - KH) / stride_h + 1) * ((W + 2 * pad_w - KW) / stride_w + 1);
     // 1x1 layers of whole channel groups are mostly memory traffic and stay (128 -> 256 at 56^2 x 32: 68 us on the pointwise kernel, 79 here
     // even on bit-packed spikes), and so do those of a single group, which have next to no products.
-    if (pointwise && (Cin % 8 == 0 || Cin < 8)) return false;
-    family = dense_family(T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w);
+    if (x_dtype != SNNF_F32 && pointwise && (Cin % 8 == 0 || Cin < 8)) return false;
+    family = dense_family(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w);
+    // fp32 tensors (two bf16 terms each) run here at three times the speed of the dense kernels over 180 measured layers (us, dense / here):
+    // 64 -> 64 at 32^2 x 8 35 / 20, at 56^2 x 16 100 / 73, 512 -> 512 at 7^2 x 4 with a residual 125 / 29, 240 -> 32 at 60 x 74, T = 3 212 / 72,
+    // 41 -> 72 at 8 x 14 x 15 191 / 20, 122 -> 111 at 15^2, 5x5, T = 5 1068 / 36, 3 -> 64 at 32^2 x 64 34 / 31, 128 -> 256 1x1 at 28^2 x 8 135 / 27.
+    // Only 1x1 layers with few products per output stay, where those are many: the copy and the elementwise outputs are their time
+    // (64 -> 256 at 56^2 x 16, T = 1 with a residual 66 / 82, 64 -> 128 at 112^2 x 4 80 / 90, 32 -> 192 at 56^2 x 16 116 / 124; but
+    // 64 -> 128 at 28^2 x 8 79 / 25, 128 -> 256 at 56^2 x 16 281 / 192, 64 -> 64 at 112^2 x 8 128 / 98).
+    if (x_dtype == SNNF_F32) return !(family == DenseFamily::kPointwise && Cin <= 64 && Cout >= 96 && T * out >= (1 << 22));
     switch (family) {
         case DenseFamily::kTInM:
         case DenseFamily::kTimeOuter: return !pointwise || static_cast<int64_t>(T) * N * (Cin + Cout) * H * W <= (1 << 25);
@@ -143,6 +167,7 @@ struct BlockedCall {
     int64_t out_step_stride;
     bool shared, neuron, has_v_init, has_v_out, pool2;
     const Shortcut* shortcut;
+    bool split;                                        // fp32 tensors as two bf16 terms
 };
 
 struct BlockedPlan {
@@ -173,13 +198,15 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
         return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_shape: tensor too large for 32-bit offsets", who);
     if (c.out_layout == SNNF_LAYOUT_BITS && (c.out_step_stride < 0 || c.out_step_stride >= (1LL << 31) / T))
         return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_shape: bit-packed output beyond 2 GiB", who);
-    const PackGeom& pg = p.pg = make_pack_geom(Cout, Cin, KH, KW, false);
+    const PackGeom& pg = p.pg = make_pack_geom(Cout, Cin, KH, KW, c.split);
     g.gpc = pg.CK / 8;
     g.npairs = pg.npairs;
     g.nocf = pg.nocf;
     g.tap_pairs = pg.CK == 8 ? 1 : 0;
     g.taps = KH * KW;
     g.frag_stride = static_cast<int64_t>(pg.nchunks) * pg.npairs * (kFragBytes / 2);
+    g.w_lo_offset = static_cast<int64_t>(pg.nchunks_r) * pg.npairs * (kFragBytes / 2);   // part 1 of the weight (kSplitParts)
+    g.narrow = c.split ? 1 : 0;
     g.T = T;
     g.shared_x = shared ? 1 : 0;
     g.in_layout = c.x_layout;
@@ -192,7 +219,7 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
     int& tt = p.tt;
     tt = shared || T == 1 ? 1 : (T == 2 ? 2 : 4);
     TunedPlan tuned = {0, 0, 0};
-    {
+    if (!c.split) {   // (measured on 16-bit activations)
         const TunedKey key = {T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, shared ? 1 : 0};
         std::lock_guard<std::mutex> lock(tuned_mutex);
         const auto it = tuned_plans().find(key);
@@ -215,7 +242,7 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
     if (!p.tuned_patch && !g.tap_pairs) {
         // Few tiles: stages of fewer channel groups where that lets more waves share a tile's K (128 -> 256 at 8^2, one image: stages
         // of 4 groups on 4 waves 13.4 us, of 2 groups on 8 waves 11.9 us; 64 -> 128 at 16^2 13.3 / 11.7).
-        const int64_t tiles = static_cast<int64_t>(pl.img_groups) * pl.patches_x * pl.patches_y * ((Cout + 63) / 64);
+        const int64_t tiles = static_cast<int64_t>(pl.img_groups) * pl.patches_x * pl.patches_y * (g.narrow ? (Cout + 31) / 32 : (Cout + 63) / 64);
         int share = 1;
         while (share < kSpkWaves && tiles * share * 2 <= static_cast<int64_t>(compute_units()) * kSpkWaves) share *= 2;
         while (pl.G > 2 && (g.C8in + pl.G - 1) / pl.G < share) pl.G >>= 1;
@@ -233,7 +260,7 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
     g.JT = (g.IT + 63) / 64;
     g.lds_wave_bytes = tt * (g.IT + 1) * 16;
     int& oc_tiles = p.oc_tiles;
-    oc_tiles = (Cout + 63) / 64;
+    oc_tiles = g.narrow ? (Cout + 31) / 32 : (Cout + 63) / 64;
     g.n_items = g.n_patches * oc_tiles;
     // K is shared by as many waves of a workgroup (up to eight, whole stages each) as keep the layer's tiles in one round of waves:
     // 64 -> 64 at 56^2 x 12 is 1176 tiles, 20.2 us unsplit and 27.9 us when two waves share each (2352 of 2048 waves).
@@ -251,7 +278,7 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
     g.wk_log2 = wk_log2;
     // Tiles of 32 channels where even those fit one round of waves: 256 -> 256 at 14^2 x 4 (112 tiles of 64 channels on eight waves each)
     // 13.9 -> 10.0 us, 512 -> 512 at 7^2 x 8 19.8 -> 13.9, at 4^2 x 32 22.2 -> 17.6. At twice the tiles they would make a second round.
-    if ((tt == 4 || (!pool2 && c.x_layout != SNNF_LAYOUT_NCHW)) && wk_log2 > 0 && !p.tuned_split && Cout > 32 && static_cast<int64_t>(g.n_patches) * ((Cout + 31) / 32) << wk_log2 <= static_cast<int64_t>(cus) * kSpkWaves) {
+    if (!c.split && (tt == 4 || (!pool2 && c.x_layout != SNNF_LAYOUT_NCHW)) && wk_log2 > 0 && !p.tuned_split && Cout > 32 && static_cast<int64_t>(g.n_patches) * ((Cout + 31) / 32) << wk_log2 <= static_cast<int64_t>(cus) * kSpkWaves) {
         g.narrow = 1;
         oc_tiles = (Cout + 31) / 32;
         g.n_items = g.n_patches * oc_tiles;
@@ -317,7 +344,7 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
 // (offsets, a kernel of too many steps, no patch that fits) gets no scratch memory asked for. Without a neuron the dense route has the
 // matrix kernel only; what it refuses stays refused. The answer depends on the layer and the table of tuned plans alone and is
 // kept per layer: it is asked for twice per call.
-using RouteKey = std::array<int, 14>;
+using RouteKey = std::array<int, 15>;
 struct Route { bool taken; DenseFamily family; };
 std::mutex routes_mutex;
 std::map<RouteKey, Route>& routes() {
@@ -328,8 +355,9 @@ constexpr size_t kMaxRoutes = 4096;
 
 Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w,
                     int v_dtype, bool residual, bool neuron) {
-    if ((x_dtype != SNNF_BF16 && x_dtype != SNNF_F16) || v_dtype != SNNF_F32) return {false, DenseFamily::kTInM};
-    const RouteKey key = {T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, residual ? 1 : 0, neuron ? 1 : 0};
+    if (!valid_dtype(x_dtype) || v_dtype != SNNF_F32) return {false, DenseFamily::kTInM};
+    const bool split = x_dtype == SNNF_F32;
+    const RouteKey key = {T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, residual ? 1 : 0, neuron ? 1 : 0, split ? 1 : 0};
     {
         std::lock_guard<std::mutex> lock(routes_mutex);
         const auto it = routes().find(key);
@@ -337,11 +365,11 @@ Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, 
     }
     Route route = {false, DenseFamily::kTInM};
     route.taken = takes_blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residual, route.family) &&
-                  (neuron || route.family == DenseFamily::kMatrixMasked || route.family == DenseFamily::kMatrixWhole);
+                  (neuron || (!split && (route.family == DenseFamily::kMatrixMasked || route.family == DenseFamily::kMatrixWhole)));
     if (route.taken) {
         BlockedPlan plan;
         route.taken = plan_blocked("snnf_conv_lif_workspace_bytes", BlockedCall{T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, SNNF_LAYOUT_C8,
-                                   residual ? SNNF_LAYOUT_NCHW : -1, SNNF_LAYOUT_NCHW, 0, false, neuron, false, neuron, false, nullptr}, plan) == SNNF_OK;
+                                   residual ? SNNF_LAYOUT_NCHW : -1, SNNF_LAYOUT_NCHW, 0, false, neuron, false, neuron, false, nullptr, split}, plan) == SNNF_OK;
     }
     std::lock_guard<std::mutex> lock(routes_mutex);
     if (routes().size() >= kMaxRoutes) routes().clear();
@@ -353,6 +381,7 @@ Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, 
 struct DenseRoute {
     const void* const* xs;
     DenseFamily family;
+    RouteSpace space;
 };
 const char* family_name(DenseFamily f) {
     return f == DenseFamily::kTInM ? "t_in_m" : (f == DenseFamily::kTimeOuter ? "time_outer" : (f == DenseFamily::kPointwise ? "pointwise" : "matrix"));
@@ -361,6 +390,8 @@ const char* family_name(DenseFamily f) {
 }  // namespace
 
 int launch_steps_to_c8(const StepPtrs& xs, int T, void* dst, int N, int C, int H, int W, hipStream_t stream);   // snnf_layout.hip
+int launch_steps_to_c8_split(const StepPtrs& xs, int T, void* dst, void* flags, int64_t lo_offset, int64_t flag_stride, int N, int C, int H, int W,
+                             hipStream_t stream);
 
 char* conv_plan_buffer();   // the thread's plan text (snnf_conv_igemm.hip), shared with snnf_conv_last_plan()
 
@@ -427,16 +458,22 @@ extern "C" int snnf_conv_lif_blocked_avgpool(const void* const* xs, int x_layout
 
 extern "C" size_t snnf_conv_lif_workspace_bytes(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h,
                                                 int stride_w, int pad_h, int pad_w, int v_dtype, int residual) {
+    if (x_dtype != SNNF_BF16 && x_dtype != SNNF_F16) return 0;
+    return snnf_conv_lif_scratch_bytes(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residual);
+}
+
+extern "C" size_t snnf_conv_lif_scratch_bytes(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h,
+                                              int stride_w, int pad_h, int pad_w, int v_dtype, int residual) {
     using namespace snnf;
     if (!blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residual != 0, true).taken) return 0;
-    return static_cast<size_t>(T) * c8_step_bytes(N, Cin, H, W);
+    return route_space(T, N, Cin, H, W, x_dtype == SNNF_F32).total;
 }
 
 extern "C" size_t snnf_conv_bias_workspace_bytes(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h,
                                                  int stride_w, int pad_h, int pad_w, int residual) {
     using namespace snnf;
     if (!blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, SNNF_F32, residual != 0, false).taken) return 0;
-    return static_cast<size_t>(T) * c8_step_bytes(N, Cin, H, W);
+    return route_space(T, N, Cin, H, W, x_dtype == SNNF_F32).total;
 }
 
 namespace snnf {
@@ -449,19 +486,19 @@ int run_blocked_route(const void* const* xs, const void* const* residuals, int T
     if (xs == nullptr || workspace == nullptr || (neuron && v_out == nullptr) || !aligned_to(workspace, 16) || out_step_stride < 0) return SNNF_ERR_UNSUPPORTED;
     const Route taken = blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residuals != nullptr, neuron != 0);
     if (!taken.taken) return SNNF_ERR_UNSUPPORTED;
-    const size_t step = c8_step_bytes(N, Cin, H, W);
-    if (workspace_bytes < step * T) return SNNF_ERR_UNSUPPORTED;
+    const RouteSpace space = route_space(T, N, Cin, H, W, x_dtype == SNNF_F32);
+    if (workspace_bytes < space.total) return SNNF_ERR_UNSUPPORTED;
     bool shared = T > 1;
     const void* inner[SNNF_MAX_T_PER_LAUNCH];
     for (int t = 0; t < T; ++t) {
         if (xs[t] == nullptr) return SNNF_ERR_UNSUPPORTED;
         shared = shared && xs[t] == xs[0];
-        inner[t] = static_cast<const char*>(workspace) + t * step;
+        inner[t] = static_cast<const char*>(workspace) + t * space.step;
     }
     if (shared) return SNNF_ERR_UNSUPPORTED;       // one frame for all timesteps is convolved once on the dense kernels too
-    const DenseRoute route = {xs, taken.family};
+    const DenseRoute route = {xs, taken.family, space};
     return conv_lif_blocked_impl(neuron ? "snnf_conv_lif" : "snnf_conv_bias", inner, SNNF_LAYOUT_C8, residuals, SNNF_LAYOUT_NCHW, T, N, Cin, H, W, x_dtype,
-                                 packed_weight, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_init, out, SNNF_LAYOUT_NCHW, out_step_stride * 2, v_out,
+                                 packed_weight, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_init, out, SNNF_LAYOUT_NCHW, out_step_stride * dtype_size(x_dtype), v_out,
                                  neuron, v_threshold, v_reset, tau, stream, nullptr, false, &route);
 }
 }  // namespace
@@ -501,7 +538,8 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
                     T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w);
     if (T > SNNF_MAX_T_PER_LAUNCH)
         return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_temporal_length: T=%d exceeds %d", who, T, SNNF_MAX_T_PER_LAUNCH);
-    if (x_dtype != SNNF_BF16 && x_dtype != SNNF_F16)
+    const bool split = dense != nullptr && x_dtype == SNNF_F32;
+    if (x_dtype != SNNF_BF16 && x_dtype != SNNF_F16 && !split)
         return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_dtype: the internal layouts hold bf16 or fp16 activations", who);
     if (x_layout != SNNF_LAYOUT_C8 && x_layout != SNNF_LAYOUT_BITS && x_layout != SNNF_LAYOUT_NCHW)
         return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_layout: inputs must be in C8 or BITS layout (or one dense frame of at most 8 channels)", who);
@@ -516,7 +554,7 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
         return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_padding: padding %dx%d too large for kernel %dx%d", who, pad_h, pad_w, KH, KW);
     // Bytes a tensor in a layout is accessed by: bit-packed tensors by single bytes, blocked inputs by 16-byte groups, blocked
     // outputs and residuals by 4 channels (8 bytes), dense tensors by elements.
-    auto need_align = [](int layout, bool as_input) -> size_t { return layout == SNNF_LAYOUT_BITS ? 1 : (layout == SNNF_LAYOUT_C8 ? (as_input ? 16 : 8) : 2); };
+    auto need_align = [x_dtype](int layout, bool as_input) -> size_t { return layout == SNNF_LAYOUT_BITS ? 1 : (layout == SNNF_LAYOUT_C8 ? (as_input ? 16 : 8) : static_cast<size_t>(dtype_size(x_dtype))); };
     if (!aligned_to(packed_weight, 16) || !aligned_to(out, need_align(out_layout, false)) || (out_step_stride % need_align(out_layout, false)) != 0 ||
         (v_init != nullptr && !aligned_to(v_init, 4)) || (v_out != nullptr && !aligned_to(v_out, 4)))
         return fail(SNNF_ERR_INVALID_ARGUMENT, "%s: packed_weight, out (and its step stride) or a membrane pointer is misaligned", who);
@@ -551,7 +589,7 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     BlockedPlan p;
     if (const int rc = plan_blocked(who, BlockedCall{T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, x_layout,
                                                      residuals != nullptr ? res_layout : -1, out_layout, out_step_stride, shared, neuron != 0,
-                                                     v_init != nullptr, v_out != nullptr, pool2, sc}, p); rc != SNNF_OK)
+                                                     v_init != nullptr, v_out != nullptr, pool2, sc, split}, p); rc != SNNF_OK)
         return rc;
     const SpkGeom& g = p.g;
 
@@ -568,9 +606,10 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     L.g = g;
     L.wpacked = static_cast<const uint16_t*>(packed_weight);
     L.bias = reinterpret_cast<const float*>(L.wpacked + packed_weight_elems(p.pg));
-    L.v_init = neuron ? static_cast<const float*>(v_init) : nullptr;
+    L.v_init = neuron ? v_init : nullptr;
     L.out = out;
-    L.v_out = neuron ? static_cast<float*>(v_out) : nullptr;
+    L.v_out = neuron ? v_out : nullptr;
+    L.v_carry = static_cast<float*>(L.v_out);
     L.lif = make_lif_params(v_threshold, v_reset, tau);
     L.grid = p.grid;
     L.lds_bytes = p.lds_bytes;
@@ -578,17 +617,31 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     const bool fast_epi = neuron && (out_layout == SNNF_LAYOUT_BITS || pool2) && (residuals == nullptr || res_layout == SNNF_LAYOUT_BITS) &&
                           L.lif.charge_mode == CHARGE_SCALE && L.lif.inv_tau == 0.5f && L.lif.v_reset == 0.0f &&
                           L.lif.v_threshold >= 1e-30f && L.lif.v_threshold <= 1e30f &&   // its multiples by 2^t stay normal numbers
-                          v_init == nullptr && p.windows == 1 && Cout % 8 == 0;
+                          v_init == nullptr && (p.windows == 1 || p.tt == 4) && Cout % 8 == 0;
+    // Dense tensors around the neuron: no range limit on the threshold, any reset potential, initial membrane, windows and channels.
+    const bool dense_epi = neuron && x_layout == SNNF_LAYOUT_C8 && out_layout == SNNF_LAYOUT_NCHW && (residuals == nullptr || res_layout == SNNF_LAYOUT_NCHW) &&
+                           L.lif.charge_mode == CHARGE_SCALE && L.lif.inv_tau == 0.5f && !L.lif.soft_reset && L.v_out != nullptr && !shared;
     snprintf(snnf::conv_plan_buffer(), 256,
              "kernel=%s variant=%d window=%d launches=%d tile=%dx%dx%d halo=%dx%d waves=8x1x%d oc_tiles=%d oc_tile=%d px_tiles=%d "
              "stage_chunks=%d run=0 lds=%zu grid=%d tuned=%d shortcut_stages=%d%s",
-             dense != nullptr ? family_name(dense->family) : "blocked", (p.wk_log2 > 0 ? 50 : 40) + p.tt + (fast_epi ? 20 : 0), shared ? T : p.tt, dense != nullptr ? 2 : 1, g.PI, g.PR, g.PC, g.RR, g.RC, 1 << p.wk_log2, p.oc_tiles, g.narrow ? 32 : 64, g.n_patches, g.G,
+             dense != nullptr ? family_name(dense->family) : "blocked", (p.wk_log2 > 0 ? 50 : 40) + p.tt + (fast_epi ? 20 : (dense_epi ? 40 : 0)), shared ? T : p.tt, dense != nullptr ? 2 : 1, g.PI, g.PR, g.PC, g.RR, g.RC, 1 << p.wk_log2, p.oc_tiles, g.narrow ? 32 : 64, g.n_patches, g.G,
              L.lds_bytes, p.grid, (p.tuned_patch ? 1 : 0) + (p.tuned_split ? 2 : 0), g.sc_stages, dense != nullptr ? " route=c8 ran=blocked" : "");
     L.fast_epilogue = fast_epi;
+    L.multi_window = p.windows > 1;
+    L.dense_epilogue = dense_epi;
     if (dense != nullptr) {   // the plan stands: bring the dense inputs into the C8 buffers behind `xs`
         StepPtrs from = {};
         for (int t = 0; t < T; ++t) from.p[t] = dense->xs[t];
-        if (const int rc = launch_steps_to_c8(from, T, const_cast<void*>(xs[0]), N, Cin, H, W, L.stream); rc != SNNF_OK) return rc;
+        char* const base = static_cast<char*>(const_cast<void*>(xs[0]));
+        if (split) {
+            L.g.lo_offset = static_cast<int64_t>(dense->space.lo);
+            L.g.flag_stride = static_cast<int64_t>(dense->space.flag_stride);
+            L.lo_flags = reinterpret_cast<const unsigned char*>(base + dense->space.flags);
+            if (const int rc = launch_steps_to_c8_split(from, T, base, base + dense->space.flags, L.g.lo_offset, L.g.flag_stride, N, Cin, H, W, L.stream); rc != SNNF_OK)
+                return rc;
+            return launch_conv_spk_f32(L, p.tt);
+        }
+        if (const int rc = launch_steps_to_c8(from, T, base, N, Cin, H, W, L.stream); rc != SNNF_OK) return rc;
     }
     if (pool2) {
         if (!fast_epi || p.windows != 1 || (p.tt != 4 && !shared))

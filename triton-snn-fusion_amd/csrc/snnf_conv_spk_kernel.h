@@ -82,6 +82,11 @@ struct SpkGeom {
     int sc_C8, sc_H, sc_W, sc_sh, sc_sw;
     int sc_gpc_log2, sc_npairs;  // channel groups (log2) and k-slot pairs per packed chunk of the second weight
     int64_t sc_frag_stride;
+    // fp32 tensors (SPLIT): the low bf16 terms of the activations lie `lo_offset` bytes behind the high ones, those of the weights
+    // `w_lo_offset` elements behind. One byte per 64 items of the C8 tensor tells whether any of them has a low term; only those are written.
+    int64_t lo_offset, w_lo_offset;
+    int64_t flag_stride;         // bytes of the flags of one timestep (a multiple of 4)
+    int v16;                     // v_init and v_out hold the activation dtype; the windows in between pass v_carry on
     FastDiv d_ppx, d_PC, d_region, d_rrrc, d_RC, d_n_patches, d_patches_img, d_patches_x, d_gpc, d_hg, d_nst, d_KW;
 };
 
@@ -91,17 +96,21 @@ struct SpkLaunch {
     SpkGeom g;
     const uint16_t* wpacked;
     const float* bias;
-    const float* v_init;
+    const void* v_init;
     void* out;
-    float* v_out;
+    void* v_out;
+    float* v_carry;             // the membrane between the windows of a call (v_out itself where that is fp32)
     LifParams lif;
     const uint16_t* wpacked2;   // packed weight and bias of the shortcut (sc_stages > 0), else null
     const float* bias2;
+    const unsigned char* lo_flags;   // SPLIT: see SpkGeom::lo_offset
     int grid;
     size_t lds_bytes;
     hipStream_t stream;
+    bool dense_epilogue;  // straight-line epilogue with dense spikes (and residual): a neuron of tau 2 with a hard reset, dense tensors around it
+    bool multi_window;    // ... with more than one window
     bool fast_epilogue;   // the straight-line epilogue applies: bit-packed output, no or a bit-packed residual, the usual neuron
-                          // (tau 2, hard reset to 0), zero initial membrane, one window, whole channel groups
+                          // (tau 2, hard reset to 0), zero initial membrane, whole channel groups
 };
 
 template <bool F16>
@@ -147,11 +156,17 @@ __device__ __forceinline__ sk_u32x4 sk_expand_bits(uint32_t byte) {
 // NARROW: tiles of 32 output channels (one weight fragment) for launches of few tiles that share K among waves: twice the workgroups,
 // each with half the matrix instructions and half the weights in its chain of steps, which is what such a launch lasts (512 -> 512 at
 // 4^2, one image: 288 steps on eight waves, 19.1 -> 12.6 us; 64 -> 64 at 56^2 11.7 -> 8.7 us; of one timestep 512 -> 512 at 4^2 10.8 -> 7.5).
-template <typename XT, int TT, int IN, bool SK, bool FAST, bool SC = false, bool POOL = false, bool NARROW = false>
+// MULTI: the straight-line epilogue of calls of several windows, which pass the membrane on through memory (a variant of its own: the
+// loads of that membrane cost the calls of one window 3 to 5 %).
+// SPLIT (XT = float): fp32 tensors as two bf16 terms. The tile is a narrow one whose two weight fragments are the high and the low terms
+// of the same 32 channels, both multiplied with the high terms of the activations; stages of the low activation terms follow where the
+// tile's halo has any (spikes, averages of spikes and 8-bit pixels have none).
+template <typename XT, int TT, int IN, bool SK, bool FAST, bool SC = false, bool POOL = false, bool NARROW = false, bool DENSE = false, bool MULTI = false>
 __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_eu(TT == 1 ? 4 : 2, TT == 1 ? 4 : 2))) void conv_spk_kernel(
     const StepPtrs xs, const StepPtrs residuals, const SpkGeom g, const uint16_t* __restrict__ wpacked,
-    const float* __restrict__ bias, const float* __restrict__ v_init, unsigned char* __restrict__ out,
-    float* __restrict__ v_out, const LifParams lif, const uint16_t* __restrict__ wpacked2, const float* __restrict__ bias2) {
+    const float* __restrict__ bias, const void* __restrict__ v_init, unsigned char* __restrict__ out,
+    void* __restrict__ v_out_any, const LifParams lif, const uint16_t* __restrict__ wpacked2, const float* __restrict__ bias2,
+    float* v_carry, const unsigned char* __restrict__ lo_flags) {
     extern __shared__ __align__(16) unsigned char lds[];
     // ---- every cache line of the kernel arguments is touched once, in one round trip: the compiler loads the arguments
     // where they are used, all over the prologue, and each of those loads then hits the scalar cache instead of waiting
@@ -160,15 +175,15 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
         auto ka = __builtin_amdgcn_kernarg_segment_ptr();
         // The explicit arguments are two step tables, the geometry, five pointers and the neuron: the last dword that is
         // touched must lie inside them (what follows is the hidden-argument area, which the compiler may leave out).
-        constexpr size_t kExplicitArgBytes = 2 * sizeof(StepPtrs) + sizeof(SpkGeom) + 7 * sizeof(void*) + sizeof(LifParams);
+        constexpr size_t kExplicitArgBytes = 2 * sizeof(StepPtrs) + sizeof(SpkGeom) + 9 * sizeof(void*) + sizeof(LifParams);
         static_assert(0x2c0 + 4 <= kExplicitArgBytes, "argument prefetch reads past the explicit kernel arguments");
-        static_assert(kExplicitArgBytes <= 0x300, "argument prefetch does not cover the last cache line of the arguments");
-        uint32_t d0, d1, d2, d3, d4, d5, d6, d7, d8, d9, d10;
+        static_assert(0x300 + 4 <= kExplicitArgBytes && kExplicitArgBytes <= 0x340, "argument prefetch does not end in the last cache line of the arguments");
+        uint32_t d0, d1, d2, d3, d4, d5, d6, d7, d8, d9, d10, d11;
         asm volatile(
-            "s_load_dword %0, %11, 0x40\n\ts_load_dword %1, %11, 0x80\n\ts_load_dword %2, %11, 0xc0\n\ts_load_dword %3, %11, 0x100\n\t"
-            "s_load_dword %4, %11, 0x140\n\ts_load_dword %5, %11, 0x180\n\ts_load_dword %6, %11, 0x1c0\n\ts_load_dword %7, %11, 0x200\n\t"
-            "s_load_dword %8, %11, 0x240\n\ts_load_dword %9, %11, 0x280\n\ts_load_dword %10, %11, 0x2c0\n\ts_waitcnt lgkmcnt(0)"
-            : "=&s"(d0), "=&s"(d1), "=&s"(d2), "=&s"(d3), "=&s"(d4), "=&s"(d5), "=&s"(d6), "=&s"(d7), "=&s"(d8), "=&s"(d9), "=&s"(d10)
+            "s_load_dword %0, %12, 0x40\n\ts_load_dword %1, %12, 0x80\n\ts_load_dword %2, %12, 0xc0\n\ts_load_dword %3, %12, 0x100\n\t"
+            "s_load_dword %4, %12, 0x140\n\ts_load_dword %5, %12, 0x180\n\ts_load_dword %6, %12, 0x1c0\n\ts_load_dword %7, %12, 0x200\n\t"
+            "s_load_dword %8, %12, 0x240\n\ts_load_dword %9, %12, 0x280\n\ts_load_dword %10, %12, 0x2c0\n\ts_load_dword %11, %12, 0x300\n\ts_waitcnt lgkmcnt(0)"
+            : "=&s"(d0), "=&s"(d1), "=&s"(d2), "=&s"(d3), "=&s"(d4), "=&s"(d5), "=&s"(d6), "=&s"(d7), "=&s"(d8), "=&s"(d9), "=&s"(d10), "=&s"(d11)
             : "s"(ka));
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -176,7 +191,12 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
     static_assert(!SC || (IN == SNNF_LAYOUT_BITS && TT == 4), "the shortcut variants take bit-packed inputs, four timesteps at a time");
     static_assert(!POOL || (FAST && (TT == 4 || TT == 1)), "the pooled output belongs to the straight-line epilogue of four steps");
     static_assert(IN != SNNF_LAYOUT_NCHW || TT == 1, "a dense input is one frame for all timesteps");
-    static_assert(!NARROW || (SK && IN != SNNF_LAYOUT_NCHW), "narrow tiles are for launches that share K among waves");
+    constexpr bool SPLIT = std::is_same<XT, float>::value;
+    static_assert(!NARROW || ((SK || SPLIT) && IN != SNNF_LAYOUT_NCHW), "narrow tiles are for launches that share K among waves, and for fp32");
+    static_assert(!SPLIT || (NARROW && IN == SNNF_LAYOUT_C8 && !FAST && !SC && !POOL), "fp32 tensors: narrow tiles on two C8 tensors, dense tensors out");
+    static_assert(!MULTI || (FAST && !POOL), "several windows belong to the straight-line epilogue");
+    static_assert(!DENSE || (IN == SNNF_LAYOUT_C8 && !FAST && !SC && !POOL), "the dense epilogue belongs to calls on dense tensors");
+    float* const v_out = static_cast<float*>(v_out_any);
     constexpr int NF = NARROW ? 1 : 2;         // 32-channel weight fragments of a tile
     constexpr int TG = 4 * NF;                 // channel groups of 8 of a tile
     constexpr bool F16 = dtype_of<XT>::value == SNNF_F16;
@@ -375,7 +395,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             // the sampled positions.
             auto batch_decode = [&](int s, int jb, int lane_s, int (&idx)[4]) __attribute__((always_inline)) -> uint32_t {
                 const bool second = SC && s >= g.nstages;
-                const int gg0 = (second ? s - g.nstages : s) * g.G;
+                const int gg0 = ((SC || SPLIT) && s >= g.nstages ? s - g.nstages : s) * g.G;
                 const int c8 = second ? g.sc_C8 : g.C8in;
                 const int base_u = second ? ((n0 * g.sc_C8 + gg0) * g.sc_H + ih_lo * g.sc_sh) * g.sc_W + iw_lo * g.sc_sw
                                    : IN == SNNF_LAYOUT_NCHW ? ((n0 * g.Cin + gg0 * 8) * g.H + ih_lo) * g.W + iw_lo
@@ -479,6 +499,16 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                             for (int t = 0; t < TT; ++t) {
                                 const int ts = t0 + t < nsteps_t ? t0 + t : t0;
                                 const unsigned char* __restrict__ src = static_cast<const unsigned char*>(sk_kernarg_ptr(0, ts));
+                                uint32_t ok_t = ok_bits;
+                                if constexpr (SPLIT) {
+                                    if (s >= g.nstages) {   // low terms: items without any were not written
+                                        src += g.lo_offset;
+                                        const unsigned char* __restrict__ flags_t = lo_flags + static_cast<int64_t>(ts) * g.flag_stride;
+#pragma unroll
+                                        for (int j = 0; j < 4; ++j)
+                                            if (flags_t[idx[j] >> 6] == 0) ok_t &= ~(1u << j);
+                                    }
+                                }
                                 sk_u32x4 raw[4];
 #pragma unroll
                                 for (int j = 0; j < 4; ++j) raw[j] = *reinterpret_cast<const sk_u32x4*>(src + static_cast<int64_t>(idx[j]) * 16);
@@ -486,7 +516,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                                 for (int j = 0; j < 4; ++j) {
                                     sk_u32x4 d;
 #pragma unroll
-                                    for (int k = 0; k < 4; ++k) d[k] = ((ok_bits >> j) & 1u) ? raw[j][k] : 0u;
+                                    for (int k = 0; k < 4; ++k) d[k] = ((ok_t >> j) & 1u) ? raw[j][k] : 0u;
                                     *reinterpret_cast<sk_u32x4*>(wlds + t * tile_t + min((jb + j) * 64 + lane_s, g.IT) * 16) = d;
                                 }
                             }
@@ -502,7 +532,18 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             // sets, activation fragments one step ahead through two.
             const int s_first = SK ? wk : 0;
             const int s_step = SK ? WK : 1;
-            const int nstages_all = SC ? g.nstages + g.sc_stages : g.nstages;
+            int nstages_all = SC ? g.nstages + g.sc_stages : g.nstages;
+            if constexpr (SPLIT) {
+                // Stages of low terms only where the tile's images have any in this window (their flags are one range of bytes per step).
+                const int image_items = g.C8in * g.H * g.W;
+                const int w0 = (n0 * image_items) >> 8, w1 = (min(n0 + g.PI, g.N) * image_items - 1) >> 8;   // dwords of four flags
+                uint32_t any = 0;
+                for (int t = t0; t < min(t0 + TT, nsteps_t); ++t) {
+                    const uint32_t* __restrict__ flags_t = reinterpret_cast<const uint32_t*>(lo_flags + static_cast<int64_t>(t) * g.flag_stride);
+                    for (int w = w0 + lane; w <= w1; w += 64) any |= flags_t[w];
+                }
+                if (__ballot(any != 0u) != 0ull) nstages_all = 2 * g.nstages;
+            }
             if constexpr (PRE) {
                 if (have && s_first < nstages_all) stage_req(s_first);
             }
@@ -531,24 +572,26 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                 const unsigned char* __restrict__ bl = wlds + lane_b;
                 for (int stage = s_first; stage < nstages_all; stage += s_step) {
                     const bool second = SC && stage >= g.nstages;     // a stage of the shortcut
-                    const int gg0 = (second ? stage - g.nstages : stage) * g.G;
+                    const bool low = SPLIT && stage >= g.nstages;     // a stage of low activation terms: against the high weight terms alone
+                    const int gg0 = (second || low ? stage - g.nstages : stage) * g.G;
                     const int gpc_l2 = second ? g.sc_gpc_log2 : g.gpc_log2;
                     const int chunk = gg0 >> gpc_l2;
                     const int pbase = chunk * (second ? g.sc_npairs : g.npairs) + ((gg0 - (chunk << gpc_l2)) >> 1);   // pair of (tap 0, the stage's first two groups)
                     const uint16_t* __restrict__ wp = second ? wpacked2 : wpacked;
                     const int64_t fs = second ? g.sc_frag_stride : g.frag_stride;
                     const unsigned char* __restrict__ pa0 = reinterpret_cast<const unsigned char*>(wp + w_frag0 * fs + static_cast<int64_t>(pbase) * (kFragBytes / 2));
-                    const unsigned char* __restrict__ pa1 = reinterpret_cast<const unsigned char*>(wp + w_frag1 * fs + static_cast<int64_t>(pbase) * (kFragBytes / 2));
+                    const unsigned char* __restrict__ pa1 = reinterpret_cast<const unsigned char*>(wp + (SPLIT ? w_frag0 * fs + g.w_lo_offset : w_frag1 * fs) + static_cast<int64_t>(pbase) * (kFragBytes / 2));
                     const Pack<uint32_t, 2>* __restrict__ tb = second ? table + 2 * (nst + 4) : table;
                     const int nst_s = second ? hg : nst;
-                    sk_u32x4 wa[4][NF];
+                    constexpr int WF = SPLIT ? 2 : NF;    // weight fragments of a step: two of 32 channels, or the two terms of one
+                    sk_u32x4 wa[4][WF];
                     sk_u32x4 wb[2][TT];
                     uint32_t bo[4];
                     // Requests the weight fragments of the step described by table entry `e` and notes where its activations are.
                     auto req_a = [&](int slot, const Pack<uint32_t, 2>& e) __attribute__((always_inline)) {
                         const uint32_t voff = lane16 + e.v[0];
                         wa[slot][0] = *reinterpret_cast<const sk_u32x4*>(pa0 + voff);
-                        if constexpr (!NARROW) wa[slot][1] = *reinterpret_cast<const sk_u32x4*>(pa1 + voff);
+                        if constexpr (WF == 2) wa[slot][1] = *reinterpret_cast<const sk_u32x4*>(pa1 + voff);
                         bo[slot] = e.v[1];
                     };
                     auto read_b = [&](int slot, uint32_t boff) __attribute__((always_inline)) {
@@ -560,6 +603,12 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                         for (int t = 0; t < TT; ++t) {
                             acc[t][0] = sk_mfma<F16>(wa[sa][0], wb[sb][t], acc[t][0]);
                             if constexpr (!NARROW) acc[t][1] = sk_mfma<F16>(wa[sa][1], wb[sb][t], acc[t][1]);
+                        }
+                        if constexpr (SPLIT) {
+                            if (!low) {
+#pragma unroll
+                                for (int t = 0; t < TT; ++t) acc[t][0] = sk_mfma<F16>(wa[sa][1], wb[sb][t], acc[t][0]);
+                            }
                         }
                     };
                     req_a(0, tb[0]);
@@ -579,6 +628,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     // would run dry while they issue.
                     auto step_order = [&]() __attribute__((always_inline)) {
                         constexpr int kMfma = 0x008, kValu = 0x002, kVmemRead = 0x020, kDsRead = 0x100;
+                        if constexpr (SPLIT) return;
                         if constexpr (NARROW) {
                             __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
                             __builtin_amdgcn_sched_group_barrier(kValu, 1, 0);
@@ -663,7 +713,10 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             if constexpr (!SK) {
                 if (wave < 4) __builtin_amdgcn_s_setprio(0);
             }
-            const float* __restrict__ v_src = t0 == 0 ? v_init : v_out;   // later windows continue from the stored membrane
+            const bool first_window = t0 == 0, last_window = t0 + TT >= nsteps_t;
+            const void* v_src = first_window ? v_init : v_carry;          // later windows continue from the stored membrane
+            void* const v_dst = last_window ? v_out_any : v_carry;
+            const bool v_src16 = !SPLIT && g.v16 && first_window, v_dst16 = !SPLIT && g.v16 && last_window;
             const int t_count = g.shared_x ? g.T : min(TT, g.T - t0);      // LIF steps of this window
             // (Made opaque here: everything derived from the lane's pixel offset is then computed after the matrix loop instead of
             // before it, where the compiler would otherwise park two dozen store addresses in registers or scratch memory.)
@@ -683,19 +736,32 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     v[k] = 0.0f;
                 }
                 if (v_src != nullptr && !g.analog_out && px_ok) {
-                    const float* __restrict__ vp = v_src + static_cast<int64_t>(j8) * 8 * po;
+                    if (v_src16) {
+                        const XT* vp = static_cast<const XT*>(v_src) + static_cast<int64_t>(j8) * 8 * po;
 #pragma unroll
-                    for (int k = 0; k < 4; ++k)
-                        if ((chm >> k) & 1u) v[k] = vp[lane_nchw + static_cast<uint32_t>(k * po)];
+                        for (int k = 0; k < 4; ++k)
+                            if ((chm >> k) & 1u) v[k] = to_float(vp[lane_nchw + static_cast<uint32_t>(k * po)]);
+                    } else {
+                        const float* vp = static_cast<const float*>(v_src) + static_cast<int64_t>(j8) * 8 * po;
+#pragma unroll
+                        for (int k = 0; k < 4; ++k)
+                            if ((chm >> k) & 1u) v[k] = vp[lane_nchw + static_cast<uint32_t>(k * po)];
+                    }
                 }
             };
             // The residual of a quad at timestep `ta`, raw (two registers in any layout), and its addition to the quad's sums.
-            auto res_load = [&](int ta, int j8, uint32_t (&raw)[2]) __attribute__((always_inline)) {
-                raw[0] = 0u;
-                raw[1] = 0u;
+            constexpr int RW = SPLIT ? 4 : 2;     // registers of a residual quad
+            auto res_load = [&](int ta, int j8, uint32_t (&raw)[RW]) __attribute__((always_inline)) {
+#pragma unroll
+                for (int k = 0; k < RW; ++k) raw[k] = 0u;
                 if (g.res_layout < 0 || !(j8 < g.C8out && px_ok)) return;
                 const unsigned char* __restrict__ res_t = static_cast<const unsigned char*>(sk_kernarg_ptr(kResTable, ta));
-                if (g.res_layout == SNNF_LAYOUT_BITS) {
+                if constexpr (SPLIT) {
+                    const float* __restrict__ rp = reinterpret_cast<const float*>(res_t) + static_cast<int64_t>(j8) * 8 * po;
+                    const int ch0 = j8 * 8 + 4 * half_e;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) raw[k] = ch0 + k < g.Cout ? __float_as_uint(rp[lane_nchw + static_cast<uint32_t>(k * po)]) : 0u;
+                } else if (g.res_layout == SNNF_LAYOUT_BITS) {
                     raw[0] = (res_t + static_cast<int64_t>(j8) * po)[lane_bits];
                 } else if (g.res_layout == SNNF_LAYOUT_C8) {
                     const Pack<uint32_t, 2> r2 = *reinterpret_cast<const Pack<uint32_t, 2>*>(reinterpret_cast<const XT*>(res_t) + static_cast<int64_t>(j8) * po * 8 + lane_c8);
@@ -711,23 +777,26 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     raw[1] = e[2] | (e[3] << 16);
                 }
             };
-            auto res_add = [&](const uint32_t (&raw)[2], float (&x)[4]) __attribute__((always_inline)) {
+            auto res_add = [&](const uint32_t (&raw)[RW], float (&x)[4]) __attribute__((always_inline)) {
                 if (g.res_layout < 0) return;
-                if (g.res_layout == SNNF_LAYOUT_BITS) {
+                if constexpr (SPLIT) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) x[k] += __uint_as_float(raw[k]);
+                } else if (g.res_layout == SNNF_LAYOUT_BITS) {
 #pragma unroll
                     for (int k = 0; k < 4; ++k) x[k] += ((raw[0] >> (4 * half_e + k)) & 1u) ? 1.0f : 0.0f;
                 } else {
 #pragma unroll
                     for (int k = 0; k < 4; ++k) {
                         const uint32_t bits = (raw[k >> 1] >> (16 * (k & 1))) & 0xffffu;
-                        x[k] += to_float(XT{static_cast<uint16_t>(bits)});
+                        if constexpr (!SPLIT) x[k] += to_float(XT{static_cast<uint16_t>(bits)});
                     }
                 }
             };
             // Store of 4 channel values of the lane's pixel at timestep `ta` in a dense layout (C8: one 8-byte store).
             auto quad_store_dense = [&](int ta, int j8, const Pack<XT, 4>& o, uint32_t chm) __attribute__((always_inline)) {
                 unsigned char* __restrict__ out_t = out + static_cast<int64_t>(ta) * g.out_step_stride;
-                if (g.out_layout == SNNF_LAYOUT_C8) {
+                if (!SPLIT && g.out_layout == SNNF_LAYOUT_C8) {
                     *reinterpret_cast<Pack<XT, 4>*>(reinterpret_cast<XT*>(out_t) + static_cast<int64_t>(j8) * po * 8 + lane_c8) = o;
                 } else {
                     XT* __restrict__ op = reinterpret_cast<XT*>(out_t) + static_cast<int64_t>(j8) * 8 * po;
@@ -738,7 +807,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             };
             // One step of a quad at absolute timestep `ta`: x = sums (bias included) (+ residual), then the neuron (its spikes are the
             // returned nibble) or, without a neuron, x itself written to the dense output.
-            auto quad_step = [&](int ta, int j8, const float (&x_in)[4], const uint32_t (&res_raw)[2], float (&v)[4], uint32_t chm) __attribute__((always_inline)) -> uint32_t {
+            auto quad_step = [&](int ta, int j8, const float (&x_in)[4], const uint32_t (&res_raw)[RW], float (&v)[4], uint32_t chm) __attribute__((always_inline)) -> uint32_t {
                 const bool grp_ok = j8 < g.C8out && px_ok;
                 float x[4];
 #pragma unroll
@@ -800,17 +869,25 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                 }
             };
             auto quad_end = [&](int j8, const float (&v)[4], uint32_t chm) __attribute__((always_inline)) {
-                if (v_out != nullptr && !g.analog_out && px_ok) {
-                    float* __restrict__ vp = v_out + static_cast<int64_t>(j8) * 8 * po;
+                if (v_dst != nullptr && !g.analog_out && px_ok) {
+                    if (v_dst16) {
+                        XT* vp = static_cast<XT*>(v_dst) + static_cast<int64_t>(j8) * 8 * po;
 #pragma unroll
-                    for (int k = 0; k < 4; ++k)
-                        if ((chm >> k) & 1u) vp[lane_nchw + static_cast<uint32_t>(k * po)] = v[k];
+                        for (int k = 0; k < 4; ++k)
+                            if ((chm >> k) & 1u) vp[lane_nchw + static_cast<uint32_t>(k * po)] = from_float<XT>(v[k]);
+                    } else {
+                        float* vp = static_cast<float*>(v_dst) + static_cast<int64_t>(j8) * 8 * po;
+#pragma unroll
+                        for (int k = 0; k < 4; ++k)
+                            if ((chm >> k) & 1u) vp[lane_nchw + static_cast<uint32_t>(k * po)] = v[k];
+                    }
                 }
             };
 
+            const int tb = MULTI ? t0 : 0;   // the straight-line epilogue's first step
             // FAST: the layer as it runs inside a network - bit-packed output, no or a bit-packed residual, the usual neuron
             // (tau = 2, hard reset to 0, a threshold whose power-of-two multiples are normal numbers), zero initial membrane,
-            // one window, whole channel groups. Straight-line code.
+            // whole channel groups. Straight-line code.
             // The membrane is kept scaled, S_t = 2^t v_t: a step is then S += 2^(t-1) x (every scaling is exact, so S_t / 2^t
             // is bit for bit the (v + x) / 2 of the general path), a comparison against 2^t v_th and a select, and the carry of
             // the comparison is shifted into the quad's word of quiet (not fired) bits: four instructions per neuron step.
@@ -875,13 +952,13 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     }
                 }
             };
-            // The same for exactly the four steps 0..3 (the usual window), without a condition per step: the lower half
+            // The same for exactly the four steps of a whole window, without a condition per step: the lower half
             // stores steps 0 and 2, the upper half steps 1 and 3.
             auto fast_store4 = [&](int j8, uint32_t quiet) __attribute__((always_inline)) {
                 const uint32_t fired = ~quiet;
                 const auto both = __builtin_amdgcn_permlane32_swap(fired, fired, false, false);
                 if (j8 < g.C8out && px_ok) {
-                    unsigned char* __restrict__ ob = out + static_cast<int64_t>(j8) * po;
+                    unsigned char* __restrict__ ob = out + static_cast<int64_t>(j8) * po + static_cast<int64_t>(tb) * g.out_step_stride;
                     const uint32_t first = lane_bits + (half_e ? static_cast<uint32_t>(g.out_step_stride) : 0u);
                     const uint32_t sh = half_e ? 8u : 12u;
                     ob[first] = static_cast<unsigned char>(((both[0] >> sh) & 15u) | (((both[1] >> sh) & 15u) << 4));
@@ -922,9 +999,18 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     *reinterpret_cast<Pack<XT, 4>*>(out + static_cast<int64_t>(step) * g.out_step_stride + static_cast<int64_t>(off) * 2) = q4;
                 }
             };
+            // A quad's membrane from the window before.
+            auto fast_v0 = [&](int j8, float (&v0)[4]) __attribute__((always_inline)) {
+                if (MULTI && t0 > 0) {
+                    const float* vp = v_out + static_cast<int64_t>(min(j8, g.C8out - 1)) * 8 * po;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) v0[k] = vp[lane_nchw + static_cast<uint32_t>(k * po)];
+                }
+            };
             // All steps of one quad whose sums are xq[tw][k]: residual, LIF, bit-packed store, optional membrane store.
-            auto fast_quad = [&](int j8, const float (&xq)[TT][4], const uint32_t (&rb)[TT], bool with_res) __attribute__((always_inline)) {
-                float S[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            // `v0`: the membrane the window starts from (a later window's is what the one before stored, zero in the first).
+            auto fast_quad = [&](int j8, const float (&xq)[TT][4], const uint32_t (&rb)[TT], bool with_res, const float (&v0)[4]) __attribute__((always_inline)) {
+                float S[4] = {v0[0], v0[1], v0[2], v0[3]};
                 if constexpr (TT == 1) {
                     if (t_count == 4 && !with_res) {
                         // The usual stem: one frame, four steps, no residual. Straight-line.
@@ -941,10 +1027,10 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                                 float x[4];
 #pragma unroll
                                 for (int k = 0; k < 4; ++k) x[k] = xq[0][k];
-                                if (with_res) fast_add_res(fast_res(ta0 + i, j8), x);
+                                if (with_res) fast_add_res(fast_res(tb + ta0 + i, j8), x);
                                 fast_step4(x, ta0 + i, S, quiet);
                             }
-                            fast_store(ta0, cnt, j8, quiet);
+                            fast_store(tb + ta0, cnt, j8, quiet);
                         }
                     }
                 } else {
@@ -968,7 +1054,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                             if constexpr (POOL) fast_store4_pooled(j8, quiet);
                             else fast_store4(j8, quiet);
                         } else {
-                            fast_store(0, TT, j8, quiet);
+                            fast_store(tb, TT, j8, quiet);
                         }
                     } else {
 #pragma unroll
@@ -981,7 +1067,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                                 fast_step4(x, tw, S, quiet);
                             }
                         }
-                        fast_store(0, t_count, j8, quiet);
+                        fast_store(tb, t_count, j8, quiet);
                     }
                 }
                 if (v_out != nullptr && px_ok && j8 < g.C8out) {
@@ -990,6 +1076,102 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
 #pragma unroll
                     for (int k = 0; k < 4; ++k) vp[lane_nchw + static_cast<uint32_t>(k * po)] = S[k] * unscale;
                 }
+            };
+            // DENSE: dense spikes (and residual) around the usual neuron (tau 2, hard reset), any number of windows and channels. A lane's
+            // pixel is one element of a channel plane, so spikes, residual and membrane move as single elements, 32 lanes side by side.
+            // What that costs is the segments of a patch's rows, not the instructions: 25.7 MB of spikes in patches of 4 x 8 pixels take
+            // 12 us in single elements and in runs of 16 bytes alike. The residual (and the membrane of a previous window) of a
+            // quad is requested one quad ahead: waited for in turn it cost 28 us on 64 -> 64 at 56^2 x 16 (67 -> 39 us without).
+            using DT = typename std::conditional<SPLIT, uint32_t, uint16_t>::type;     // an element's bits
+            struct DenseIn { uint32_t res[TT][4]; uint32_t v[4]; };
+            auto dense_request = [&](int j8_any, DenseIn& in) __attribute__((always_inline)) {
+                const int j8 = min(j8_any, g.C8out - 1);
+                const int left = g.Cout - (j8 * 8 + 4 * half_e);     // channels of this lane's quad, and beyond
+                auto get = [&](auto ragged_tag) __attribute__((always_inline)) {
+                    constexpr bool RAGGED = decltype(ragged_tag)::value;
+                    // Lanes without a pixel read pixel 0 of image 0; channels beyond the last are not read.
+                    if (RAGGED || left > 0) {
+                        if (g.res_layout >= 0) {
+#pragma unroll
+                            for (int tw = 0; tw < TT; ++tw) {
+                                const DT* __restrict__ rp = static_cast<const DT*>(sk_kernarg_ptr(kResTable, min(t0 + tw, g.T - 1))) + static_cast<int64_t>(j8) * 8 * po;
+#pragma unroll
+                                for (int k = 0; k < 4; ++k)
+                                    if (!RAGGED || k < left) in.res[tw][k] = rp[lane_nchw + static_cast<uint32_t>(k * po)];
+                            }
+                        }
+                        if (v_src != nullptr) {
+                            if (v_src16) {
+                                const uint16_t* vp = static_cast<const uint16_t*>(v_src) + static_cast<int64_t>(j8) * 8 * po;
+#pragma unroll
+                                for (int k = 0; k < 4; ++k)
+                                    if (!RAGGED || k < left) in.v[k] = vp[lane_nchw + static_cast<uint32_t>(k * po)];
+                            } else {
+                                const uint32_t* vp = static_cast<const uint32_t*>(v_src) + static_cast<int64_t>(j8) * 8 * po;
+#pragma unroll
+                                for (int k = 0; k < 4; ++k)
+                                    if (!RAGGED || k < left) in.v[k] = vp[lane_nchw + static_cast<uint32_t>(k * po)];
+                            }
+                        }
+                    }
+                };
+                if (g.res_layout >= 0 || v_src != nullptr) {
+                    if (g.Cout & 3) get(std::true_type{});
+                    else get(std::false_type{});
+                }
+            };
+            auto dense_quad = [&](int j8, const float (&xq)[TT][4], const DenseIn& in) __attribute__((always_inline)) {
+                if (j8 >= g.C8out) return;
+                const int left = g.Cout - (j8 * 8 + 4 * half_e);
+                float v[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[k] = 0.0f;
+                if (v_src != nullptr) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        if constexpr (SPLIT) v[k] = __uint_as_float(in.v[k]);
+                        else v[k] = v_src16 ? to_float(XT{static_cast<uint16_t>(in.v[k])}) : __uint_as_float(in.v[k]);
+                    }
+                }
+                auto run = [&](auto ragged_tag) __attribute__((always_inline)) {
+                    constexpr bool RAGGED = decltype(ragged_tag)::value;
+                    if (px_ok && left > 0) {
+#pragma unroll
+                        for (int tw = 0; tw < TT; ++tw) {
+                            if (tw < t_count) {
+                                DT* __restrict__ op = reinterpret_cast<DT*>(out + static_cast<int64_t>(t0 + tw) * g.out_step_stride) + static_cast<int64_t>(j8) * 8 * po;
+#pragma unroll
+                                for (int k = 0; k < 4; ++k) {
+                                    float x = xq[tw][k];
+                                    if (g.res_layout >= 0) {
+                                        if constexpr (SPLIT) x += __uint_as_float(in.res[tw][k]);
+                                        else x += to_float(XT{static_cast<uint16_t>(in.res[tw][k])});
+                                    }
+                                    const float h = (v[k] + x) * 0.5f;
+                                    const bool fired = h >= lif.v_threshold;
+                                    v[k] = fired ? lif.v_reset : h;
+                                    const DT spike = fired ? static_cast<DT>(SPLIT ? 0x3f800000u : ONE) : DT{0};
+                                    if (!RAGGED || k < left) op[lane_nchw + static_cast<uint32_t>(k * po)] = spike;
+                                }
+                            }
+                        }
+                        if (v_dst16) {
+                            if constexpr (!SPLIT) {
+                                XT* vp = static_cast<XT*>(v_dst) + static_cast<int64_t>(j8) * 8 * po;
+#pragma unroll
+                                for (int k = 0; k < 4; ++k)
+                                    if (!RAGGED || k < left) vp[lane_nchw + static_cast<uint32_t>(k * po)] = from_float<XT>(v[k]);
+                            }
+                        } else {
+                            float* vp = static_cast<float*>(v_dst) + static_cast<int64_t>(j8) * 8 * po;
+#pragma unroll
+                            for (int k = 0; k < 4; ++k)
+                                if (!RAGGED || k < left) vp[lane_nchw + static_cast<uint32_t>(k * po)] = v[k];
+                        }
+                    }
+                };
+                if (g.Cout & 3) run(std::true_type{});
+                else run(std::false_type{});
             };
             // All steps of one quad, any layouts and neuron (the general path).
             auto general_quad = [&](int j8, const float (&xq)[TT][4]) __attribute__((always_inline)) {
@@ -1002,7 +1184,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                         const int cnt = min(8, t_count - ta0);
                         uint32_t nibw = 0;
                         for (int i = 0; i < cnt; ++i) {
-                            uint32_t rr[2];
+                            uint32_t rr[RW];
                             res_load(t0 + ta0 + i, j8, rr);
                             nibw |= quad_step(t0 + ta0 + i, j8, xq[0], rr, v, chm) << (4 * i);
                         }
@@ -1010,7 +1192,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                         else if (!g.analog_out) quad_store_spikes(t0 + ta0, cnt, j8, nibw, chm);
                     }
                 } else {
-                    uint32_t rr[TT][2];
+                    uint32_t rr[TT][RW];
 #pragma unroll
                     for (int tw = 0; tw < TT; ++tw) res_load(min(t0 + tw, g.T - 1), j8, rr[tw]);
                     uint32_t nibw = 0;
@@ -1030,15 +1212,24 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     // one round trip to memory for the whole epilogue. The fence keeps the compiler from sinking each request
                     // to its use, where every one of them would be waited for in turn.
                     uint32_t rb[8][TT];
+                    float v0[8][4];
 #pragma unroll
-                    for (int fq = 0; fq < 8; ++fq)
+                    for (int fq = 0; fq < 8; ++fq) {
 #pragma unroll
                         for (int tw = 0; tw < TT; ++tw) rb[fq][tw] = 0u;
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) v0[fq][k] = 0.0f;
+                    }
+                    if (MULTI && t0 > 0) {
+#pragma unroll
+                        for (int fq = 0; fq < 8; ++fq) fast_v0(oc_e * TG + fq, v0[fq]);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
                     if (with_res && TT > 1) {
                         const unsigned char* res_ptr[TT];
 #pragma unroll
                         for (int tw = 0; tw < TT; ++tw)
-                            res_ptr[tw] = static_cast<const unsigned char*>(sk_kernarg_ptr(kResTable, min(tw, t_count - 1))) + static_cast<int64_t>(oc_e) * TG * po;
+                            res_ptr[tw] = static_cast<const unsigned char*>(sk_kernarg_ptr(kResTable, tb + min(tw, t_count - 1))) + static_cast<int64_t>(oc_e) * TG * po;
                         auto req_res = [&](auto fq_tag) __attribute__((always_inline)) {
                             constexpr int fq = decltype(fq_tag)::value;
                             const uint32_t off = lane_bits + static_cast<uint32_t>(min(fq, g.C8out - 1 - oc_e * TG) * po);
@@ -1062,7 +1253,30 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                         for (int tw = 0; tw < TT; ++tw)
 #pragma unroll
                             for (int k = 0; k < 4; ++k) xq[tw][k] = acc[tw][(fq >> 2) % NF][4 * (fq & 3) + k];
-                        fast_quad(oc_e * TG + fq, xq, rb[fq], with_res);
+                        fast_quad(oc_e * TG + fq, xq, rb[fq], with_res, v0[fq]);
+                    };
+                    do_quad(std::integral_constant<int, 0>{});
+                    do_quad(std::integral_constant<int, 1>{});
+                    do_quad(std::integral_constant<int, 2>{});
+                    do_quad(std::integral_constant<int, 3>{});
+                    do_quad(std::integral_constant<int, 4>{});
+                    do_quad(std::integral_constant<int, 5>{});
+                    do_quad(std::integral_constant<int, 6>{});
+                    do_quad(std::integral_constant<int, 7>{});
+                } else if constexpr (DENSE) {
+                    DenseIn in[2] = {};
+                    dense_request(oc_e * TG, in[0]);
+                    auto do_quad = [&](auto fq_tag) __attribute__((always_inline)) {
+                        constexpr int fq = decltype(fq_tag)::value;
+                        if constexpr (fq < TG) {
+                            if constexpr (fq + 1 < TG) dense_request(oc_e * TG + fq + 1, in[(fq + 1) & 1]);
+                            float xq[TT][4];
+#pragma unroll
+                            for (int tw = 0; tw < TT; ++tw)
+#pragma unroll
+                                for (int k = 0; k < 4; ++k) xq[tw][k] = acc[tw][(fq >> 2) % NF][4 * (fq & 3) + k];
+                            dense_quad(oc_e * TG + fq, xq, in[fq & 1]);
+                        }
                     };
                     do_quad(std::integral_constant<int, 0>{});
                     do_quad(std::integral_constant<int, 1>{});
@@ -1075,7 +1289,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                 } else {
                     // A runtime loop over the wave's 8 quads keeps the code small; a quad's sums are copied out of the accumulators
                     // by a switch (constant register indices), so the accumulators stay in registers.
-                    for (int fq = 0; fq < 8; ++fq) {
+                    for (int fq = 0; fq < TG; ++fq) {
                         float xq[TT][4];
 #define SNNF_SPK_COPY_QUAD(F, Q)                                          \
     _Pragma("unroll") for (int tw = 0; tw < TT; ++tw)                     \
@@ -1114,9 +1328,13 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     if constexpr (FAST) {   // the residual bytes of the first quad travel while the workgroup meets
                         if (g.res_layout >= 0 && TT > 1) {
 #pragma unroll
-                            for (int tw = 0; tw < TT; ++tw) rb[tw] = fast_res(min(tw, t_count - 1), oc_e * TG + 4 * wk);
+                            for (int tw = 0; tw < TT; ++tw) rb[tw] = fast_res(tb + min(tw, t_count - 1), oc_e * TG + 4 * wk);
                         }
                     }
+                    float v0[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                    if constexpr (FAST) fast_v0(oc_e * TG + 4 * wk, v0);
+                    DenseIn in = {};
+                    if constexpr (DENSE) dense_request(oc_e * TG + 4 * wk, in);
                     __syncthreads();
                     const int partner = wave ^ 1;
                     int lane_x = lane;                   // opaque: the addresses below are computed here, not ahead of the matrix loop
@@ -1145,9 +1363,15 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                         if constexpr (FAST) {
                             if (e != 0 && g.res_layout >= 0 && TT > 1) {
 #pragma unroll
-                                for (int tw = 0; tw < TT; ++tw) rb[tw] = fast_res(min(tw, t_count - 1), j8);
+                                for (int tw = 0; tw < TT; ++tw) rb[tw] = fast_res(tb + min(tw, t_count - 1), j8);
                             }
-                            fast_quad(j8, xq, rb, g.res_layout >= 0);
+                            const float start[4] = {v0[0], v0[1], v0[2], v0[3]};
+                            if (e != 3) fast_v0(j8 + 1, v0);
+                            fast_quad(j8, xq, rb, g.res_layout >= 0, start);
+                        } else if constexpr (DENSE) {
+                            const DenseIn now = in;
+                            if (e != 3) dense_request(j8 + 1, in);
+                            dense_quad(j8, xq, now);
                         } else {
                             general_quad(j8, xq);
                         }
@@ -1172,8 +1396,16 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     if constexpr (FAST) {
                         if (e_first < 4 && g.res_layout >= 0 && TT > 1) {
 #pragma unroll
-                            for (int tw = 0; tw < TT; ++tw) rb[tw] = fast_res(min(tw, t_count - 1), oc_e * TG + 4 * r + e_first);
+                            for (int tw = 0; tw < TT; ++tw) rb[tw] = fast_res(tb + min(tw, t_count - 1), oc_e * TG + 4 * r + e_first);
                         }
+                    }
+                    float v0[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                    if constexpr (FAST) {
+                        if (e_first < 4) fast_v0(oc_e * TG + 4 * r + e_first, v0);
+                    }
+                    DenseIn in = {};
+                    if constexpr (DENSE) {
+                        if (e_first < 4) dense_request(oc_e * TG + 4 * r + e_first, in);
                     }
                     __syncthreads();
                     for (int e_own = e_first; e_own < 4; e_own += WK) {
@@ -1185,7 +1417,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                             sk_f32x4 sum[TT];
 #pragma unroll
                             for (int tw = 0; tw < TT; ++tw) sum[tw] = sk_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-                            if constexpr (FAST) {
+                            if constexpr (FAST || DENSE) {
                                 for (int k = 0; k < WK; k += 2) {
                                     sk_f32x4 p0[TT], p1[TT];
 #pragma unroll
@@ -1211,9 +1443,15 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                         if constexpr (FAST) {
                             if (e_own != e_first && g.res_layout >= 0 && TT > 1) {
 #pragma unroll
-                                for (int tw = 0; tw < TT; ++tw) rb[tw] = fast_res(min(tw, t_count - 1), j8);
+                                for (int tw = 0; tw < TT; ++tw) rb[tw] = fast_res(tb + min(tw, t_count - 1), j8);
                             }
-                            fast_quad(j8, xq, rb, g.res_layout >= 0);
+                            const float start[4] = {v0[0], v0[1], v0[2], v0[3]};
+                            if (e_own + WK < 4) fast_v0(j8 + WK, v0);
+                            fast_quad(j8, xq, rb, g.res_layout >= 0, start);
+                        } else if constexpr (DENSE) {
+                            const DenseIn now = in;
+                            if (e_own + WK < 4) dense_request(j8 + WK, in);
+                            dense_quad(j8, xq, now);
                         } else {
                             general_quad(j8, xq);
                         }
@@ -1230,13 +1468,39 @@ int launch_conv_spk_variant(const SpkLaunch& L) {
     auto run = [&](auto kernel) -> int {
         if (const int rc = reserve_lds(reinterpret_cast<const void*>(kernel), L.lds_bytes, "snnf_conv_lif_blocked"); rc != SNNF_OK) return rc;
         kernel<<<dim3(L.grid), kSpkWaves * 64, L.lds_bytes, L.stream>>>(L.xs, L.residuals, L.g, L.wpacked, L.bias, L.v_init,
-                                                                        static_cast<unsigned char*>(L.out), L.v_out, L.lif, L.wpacked2, L.bias2);
+                                                                        static_cast<unsigned char*>(L.out), L.v_out, L.lif, L.wpacked2, L.bias2, L.v_carry, L.lo_flags);
         return check_launch("snnf_conv_lif_blocked");
     };
+    if constexpr (IN == SNNF_LAYOUT_C8) {
+        if (L.dense_epilogue) {
+            if (L.g.narrow) return run(conv_spk_kernel<XT, TT, IN, true, false, false, false, true, true>);
+            return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, IN, true, false, false, false, false, true>) : run(conv_spk_kernel<XT, TT, IN, false, false, false, false, false, true>);
+        }
+    }
+    if constexpr (TT == 4) {
+        if (L.fast_epilogue && L.multi_window) {
+            if (L.g.narrow) return run(conv_spk_kernel<XT, TT, IN, true, true, false, false, true, false, true>);
+            return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, IN, true, true, false, false, false, false, true>) : run(conv_spk_kernel<XT, TT, IN, false, true, false, false, false, false, true>);
+        }
+    }
     if (L.g.narrow)
         return L.fast_epilogue ? run(conv_spk_kernel<XT, TT, IN, true, true, false, false, true>) : run(conv_spk_kernel<XT, TT, IN, true, false, false, false, true>);
     if (L.fast_epilogue) return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, IN, true, true>) : run(conv_spk_kernel<XT, TT, IN, false, true>);
     return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, IN, true, false>) : run(conv_spk_kernel<XT, TT, IN, false, false>);
+}
+
+// fp32 tensors as two bf16 terms each.
+template <int TT>
+int launch_conv_spk_split(const SpkLaunch& L) {
+    auto run = [&](auto kernel) -> int {
+        if (const int rc = reserve_lds(reinterpret_cast<const void*>(kernel), L.lds_bytes, "snnf_conv_lif"); rc != SNNF_OK) return rc;
+        kernel<<<dim3(L.grid), kSpkWaves * 64, L.lds_bytes, L.stream>>>(L.xs, L.residuals, L.g, L.wpacked, L.bias, L.v_init,
+                                                                        static_cast<unsigned char*>(L.out), L.v_out, L.lif, L.wpacked2, L.bias2, L.v_carry, L.lo_flags);
+        return check_launch("snnf_conv_lif");
+    };
+    constexpr int C = SNNF_LAYOUT_C8;
+    if (L.dense_epilogue) return L.g.wk_log2 > 0 ? run(conv_spk_kernel<float, TT, C, true, false, false, false, true, true>) : run(conv_spk_kernel<float, TT, C, false, false, false, false, true, true>);
+    return L.g.wk_log2 > 0 ? run(conv_spk_kernel<float, TT, C, true, false, false, false, true>) : run(conv_spk_kernel<float, TT, C, false, false, false, false, true>);
 }
 
 // The variants whose spikes leave as 2x2 average pools: straight-line epilogue, four steps (side by side, or of one frame).
@@ -1245,7 +1509,7 @@ int launch_conv_spk_pooled(const SpkLaunch& L, int tt) {
     auto run = [&](auto kernel) -> int {
         if (const int rc = reserve_lds(reinterpret_cast<const void*>(kernel), L.lds_bytes, "snnf_conv_lif_blocked_avgpool"); rc != SNNF_OK) return rc;
         kernel<<<dim3(L.grid), kSpkWaves * 64, L.lds_bytes, L.stream>>>(L.xs, L.residuals, L.g, L.wpacked, L.bias, L.v_init,
-                                                                        static_cast<unsigned char*>(L.out), L.v_out, L.lif, L.wpacked2, L.bias2);
+                                                                        static_cast<unsigned char*>(L.out), L.v_out, L.lif, L.wpacked2, L.bias2, L.v_carry, L.lo_flags);
         return check_launch("snnf_conv_lif_blocked_avgpool");
     };
     if (tt == 4 && L.g.narrow) return run(conv_spk_kernel<XT, 4, IN, true, true, false, true, true>);
@@ -1259,7 +1523,7 @@ int launch_conv_spk_frame(const SpkLaunch& L, bool pooled) {
     auto run = [&](auto kernel) -> int {
         if (const int rc = reserve_lds(reinterpret_cast<const void*>(kernel), L.lds_bytes, "snnf_conv_lif_blocked"); rc != SNNF_OK) return rc;
         kernel<<<dim3(L.grid), kSpkWaves * 64, L.lds_bytes, L.stream>>>(L.xs, L.residuals, L.g, L.wpacked, L.bias, L.v_init,
-                                                                        static_cast<unsigned char*>(L.out), L.v_out, L.lif, L.wpacked2, L.bias2);
+                                                                        static_cast<unsigned char*>(L.out), L.v_out, L.lif, L.wpacked2, L.bias2, L.v_carry, L.lo_flags);
         return check_launch("snnf_conv_lif_blocked");
     };
     constexpr int D = SNNF_LAYOUT_NCHW;
@@ -1274,10 +1538,14 @@ int launch_conv_spk_shortcut(const SpkLaunch& L) {
     auto run = [&](auto kernel) -> int {
         if (const int rc = reserve_lds(reinterpret_cast<const void*>(kernel), L.lds_bytes, "snnf_conv_lif_blocked_shortcut"); rc != SNNF_OK) return rc;
         kernel<<<dim3(L.grid), kSpkWaves * 64, L.lds_bytes, L.stream>>>(L.xs, L.residuals, L.g, L.wpacked, L.bias, L.v_init,
-                                                                        static_cast<unsigned char*>(L.out), L.v_out, L.lif, L.wpacked2, L.bias2);
+                                                                        static_cast<unsigned char*>(L.out), L.v_out, L.lif, L.wpacked2, L.bias2, L.v_carry, L.lo_flags);
         return check_launch("snnf_conv_lif_blocked_shortcut");
     };
     constexpr int B = SNNF_LAYOUT_BITS;
+    if (L.fast_epilogue && L.multi_window) {
+        if (L.g.narrow) return run(conv_spk_kernel<XT, 4, B, true, true, true, false, true, false, true>);
+        return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, 4, B, true, true, true, false, false, false, true>) : run(conv_spk_kernel<XT, 4, B, false, true, true, false, false, false, true>);
+    }
     if (L.g.narrow) return L.fast_epilogue ? run(conv_spk_kernel<XT, 4, B, true, true, true, false, true>) : run(conv_spk_kernel<XT, 4, B, true, false, true, false, true>);
     if (L.fast_epilogue) return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, 4, B, true, true, true>) : run(conv_spk_kernel<XT, 4, B, false, true, true>);
     return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, 4, B, true, false, true>) : run(conv_spk_kernel<XT, 4, B, false, false, true>);
@@ -1301,5 +1569,6 @@ int launch_conv_spk_bf16_pooled(const SpkLaunch& L, int tt);
 int launch_conv_spk_f16_pooled(const SpkLaunch& L, int tt);
 int launch_conv_spk_bf16_frame(const SpkLaunch& L, bool pooled);
 int launch_conv_spk_f16_frame(const SpkLaunch& L, bool pooled);
+int launch_conv_spk_f32(const SpkLaunch& L, int tt);
 
 }  // namespace snnf

@@ -98,6 +98,46 @@ __global__ __launch_bounds__(kThreads) void steps_to_c8_kernel(const StepPtrs xs
     }
 }
 
+// The T dense fp32 tensors of an operator call -> their high bf16 terms as one C8 tensor and, `lo_offset` bytes behind it, their low ones.
+// Bound by HBM. A thread owns one pixel of a channel group (8 loads of 4 bytes, 64 lanes side by side) and a wave 64 items: its byte of
+// `flags` says whether any of them has a low term, and only then are the low terms written - spikes, their averages and 8-bit pixels
+// have none, which saves a third of the traffic here and half of the matrix stages of the convolution behind it.
+__global__ __launch_bounds__(kThreads) void steps_to_c8_split_kernel(const StepPtrs xs, unsigned char* __restrict__ dst, unsigned char* __restrict__ flags,
+                                                                     uint32_t items, int C, int C8, uint32_t HW, FastDiv d_HW, FastDiv d_C8,
+                                                                     int64_t step_bytes, int64_t lo_offset, int64_t flag_stride) {
+    const uint32_t item = blockIdx.x * kThreads + threadIdx.x;
+    const bool have = item < items;
+    const uint32_t it = have ? item : 0u;
+    const uint32_t plane = static_cast<uint32_t>(fast_div(static_cast<int>(it), d_HW));
+    const uint32_t px = it - plane * HW;
+    const uint32_t n = static_cast<uint32_t>(fast_div(static_cast<int>(plane), d_C8));
+    const uint32_t c0 = (plane - n * C8) * 8;
+    const float* __restrict__ src = static_cast<const float*>(sk_kernarg_ptr(0, static_cast<int>(blockIdx.y))) + (static_cast<int64_t>(n) * C + c0) * HW + px;
+    unsigned char* __restrict__ out = dst + static_cast<int64_t>(blockIdx.y) * step_bytes + static_cast<int64_t>(it) * 16;
+    const int chans = min(8, C - static_cast<int>(c0));
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = have && j < chans ? src[j * HW] : 0.0f;
+    Pack<uint32_t, 4> hi, lo;
+    uint32_t any = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        hi.v[k] = split_bf16_bits(v[2 * k], false) | (split_bf16_bits(v[2 * k + 1], false) << 16);
+        lo.v[k] = split_bf16_bits(v[2 * k], true) | (split_bf16_bits(v[2 * k + 1], true) << 16);
+        any |= lo.v[k] & 0x7fff7fffu;
+    }
+    const bool wave_any = __ballot(any != 0u) != 0ull;
+    if (!have) return;
+    *reinterpret_cast<Pack<uint32_t, 4>*>(out) = hi;
+    if (wave_any) *reinterpret_cast<Pack<uint32_t, 4>*>(out + lo_offset) = lo;
+    if ((item & 63u) == 0u) {
+        unsigned char* __restrict__ mine = flags + static_cast<int64_t>(blockIdx.y) * flag_stride;
+        mine[item >> 6] = wave_any ? 1 : 0;
+        if (item + 64u >= items)     // the last wave fills the last dword of flags
+            for (uint32_t f = (item >> 6) + 1u; (f & 3u) != 0u; ++f) mine[f] = 0;
+    }
+}
+
 // Pooling of one group of 8 channels per thread: K x K window, stride 2, `pad` rows/columns of padding that never win a
 // maximum (average pooling takes no padding). Spikes are 0 / 1, so a maximum over bits is their OR.
 template <typename XT, int SRC, int DST, int K, bool IS_MAX>
@@ -247,6 +287,18 @@ int launch_steps_to_c8(const StepPtrs& xs, int T, void* dst, int N, int C, int H
     const dim3 grid(static_cast<unsigned>((items + kThreads - 1) / kThreads), static_cast<unsigned>(T));
     steps_to_c8_kernel<<<grid, kThreads, 0, stream>>>(xs, static_cast<uint16_t*>(dst), static_cast<uint32_t>(items), C, C8, static_cast<uint32_t>(HW),
                                                        make_fast_div(static_cast<int>(pairs)), make_fast_div(C8), static_cast<int64_t>(N) * C8 * HW * 8);
+    return check_launch("snnf_conv_lif");
+}
+
+int launch_steps_to_c8_split(const StepPtrs& xs, int T, void* dst, void* flags, int64_t lo_offset, int64_t flag_stride, int N, int C, int H, int W,
+                             hipStream_t stream) {
+    const int C8 = (C + 7) / 8;
+    const int64_t HW = static_cast<int64_t>(H) * W, items = HW * N * C8;
+    if (items >= (1LL << 30)) return fail(SNNF_ERR_UNSUPPORTED, "snnf_conv_lif: unsupported_shape: too many elements for the blocked copy");
+    const dim3 grid(static_cast<unsigned>((items + kThreads - 1) / kThreads), static_cast<unsigned>(T));
+    steps_to_c8_split_kernel<<<grid, kThreads, 0, stream>>>(xs, static_cast<unsigned char*>(dst), static_cast<unsigned char*>(flags), static_cast<uint32_t>(items), C,
+                                                             C8, static_cast<uint32_t>(HW), make_fast_div(static_cast<int>(HW)), make_fast_div(C8), items * 16,
+                                                             lo_offset, flag_stride);
     return check_launch("snnf_conv_lif");
 }
 

@@ -377,7 +377,7 @@ def _launch(kernel_key: str, steps: Sequence[torch.Tensor], residuals: Optional[
         # the caching allocator hands the block out again in the order of the stream the kernels run on.
         nbytes = 0
         if not _one_frame(xs):
-            nbytes = int(lib.snnf_conv_lif_workspace_bytes(T, n, cin, h, w, x_code, cout, kh, kw, sh, sw, ph, pw, v_code, 1 if rs is not None else 0))
+            nbytes = int(lib.snnf_conv_lif_scratch_bytes(T, n, cin, h, w, x_code, cout, kh, kw, sh, sw, ph, pw, v_code, 1 if rs is not None else 0))
         workspace = torch.empty(nbytes, dtype=torch.uint8, device=first.device) if nbytes else None
         _lib.check("snnf_conv_lif", lib.snnf_conv_lif_ws(
             xs, rs, T, n, cin, h, w, x_code, packed.data_ptr(), cout, kh, kw, sh, sw, ph, pw,
