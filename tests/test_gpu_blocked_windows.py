@@ -1,0 +1,35 @@
+"""Blocked convolutions of more timesteps than a window holds, bit-packed in and out: the straight-line epilogue passes the membrane from
+window to window. Against the CPU oracle for every way the waves of a workgroup share a tile, with last windows of one to four steps."""
+import pytest
+import torch
+
+from helpers import LIF, check, dev, gen, q, spikes
+from oracle import snn_oracle as O
+
+pytestmark = pytest.mark.gpu
+BF16, F16 = torch.bfloat16, torch.float16
+
+
+@pytest.mark.parametrize("Cin,Cout,H,W,N,T,dtype,residual,layout,waves,tile", [
+    (64, 64, 56, 56, 9, 5, BF16, True, "bits", "8x1x2", 64),      # two waves per tile, a last window of one step
+    (16, 64, 40, 40, 46, 6, BF16, True, "bits", "8x1x1", 64),     # a wave per tile, several rounds
+    (16, 72, 40, 40, 5, 8, F16, False, "c8", "8x1x1", 64),        # blocked inputs; eight channels in the last tile
+    (256, 128, 14, 14, 24, 7, BF16, True, "bits", "8x1x4", 64),   # four waves per tile
+    (512, 512, 7, 7, 9, 6, BF16, False, "bits", "8x1x8", 64),     # eight
+    (128, 40, 8, 8, 1, 16, BF16, True, "bits", "8x1x8", 32),      # tiles of 32 channels, four windows
+    (64, 96, 9, 11, 2, 9, F16, True, "c8", "8x1x4", 32),
+])
+def test_membrane_passes_from_window_to_window(snnf_lib, Cin, Cout, H, W, N, T, dtype, residual, layout, waves, tile):
+    from triton_snn_fusion_amd.runtime import hip_blocked_backend as B
+    g = gen(7000 + Cin + T)
+    x = torch.stack([spikes((N, Cin, H, W), 0.25, g) for _ in range(T)])
+    w, b = q(torch.randn(Cout, Cin, 3, 3, generator=g) * 2.0 * (2.0 / (Cin * 9)) ** 0.5, dtype), q(torch.randn(Cout, generator=g) * 0.1, dtype)
+    rs = torch.stack([spikes((N, Cout, H, W), 0.25, g) for _ in range(T)]) if residual else None
+    ref = O.temporal_conv_lif(list(x), w, b, torch.tensor(0.0), (1, 1), (1, 1), (1, 1), 1, *LIF, residuals=list(rs) if residual else None)
+    out, v = B.conv_lif_blocked(B.from_dense(dev(x, dtype), B.BITS if layout == "bits" else B.C8), dev(w, dtype), dev(b, dtype), [1, 1], [1, 1], LIF,
+                                residual=B.from_dense(dev(rs, dtype), B.BITS) if residual else None, out_layout=B.BITS, want_v=True)
+    plan = B.last_conv_plan()
+    assert int(plan["variant"]) >= 60 and int(plan["window"]) == 4, plan
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert (plan["waves"], int(plan["oc_tile"])) == (waves, tile), plan
+    check(B.to_dense(out), v, ref, what=f"{Cin}->{Cout} {H}x{W} T={T}")
