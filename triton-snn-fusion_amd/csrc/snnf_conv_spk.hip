@@ -101,53 +101,67 @@ RouteSpace route_space(int T, int N, int Cin, int H, int W, bool split) {
     return r;
 }
 
-// Whether a layer on dense tensors is brought into C8 and run on the blocked kernel (two launches) or stays on the dense kernels.
-// Measured (bf16, T = 4 unless said, us, dense / this route). Channel counts that are no multiple of 8 only have the four-wave kernels
-// on dense tensors, which assemble every channel group from scalar loads: 230 -> 144 at 11 x 83 stride 2 650 / 32, 167 -> 64 at
-// 23 x 91, T = 3 763 / 76, 41 -> 88 at 44^2 57 / 25, 135 -> 144 at 9^2 stride 2, T = 1 56 / 13; they move, but for large 1x1 layers, which
-// are memory traffic (421 -> 288 at 100^2, T = 8, 342 MB: 356 / 416; 99 -> 130 at 40^2 28 / 23). Layers that the matrix kernel runs in
-// its masked variant (planes or channels its tiles do not divide) go in windows of two timesteps there and pay a pass over the
-// weights per window: 512 -> 512 at 7^2 x 16 56 / 34, 352 -> 224 at 17 x 25 with a residual 47 / 30, 88 -> 176 at 43^2 68 / 41, 72 -> 104 at
-// 27 x 35, T = 6, with a residual 54 / 48, 80 -> 16 at 10^2, T = 3 50 / 20; with few products per output the extra launch and the
-// 2-byte accesses of the dense output outweigh that: 24 -> 256 at 10 x 44, 5x5, with a residual 27 / 32, 16 -> 96 at 25^2 with a residual
-// 32 / 49. One or two timesteps are one window there: 16 -> 136 at 70^2 stride 2, T = 2 31 / 46, 104 -> 168 at 23^2, T = 2, residual 41 / 53,
-// but 344 -> 16 at 20 x 37, 5x5, T = 2 106 / 71, 304 -> 208 at 15^2, T = 1 27 / 19. More than four timesteps are several windows here as
-// well, over which few channels do not pay: 40 -> 16 at 24 x 59, 5x5, T = 5 41 / 56, 48 -> 16 at 66 x 103, 7x7, T = 8 80 / 95, but 56 -> 184 at
-// 17^2, 7x7, T = 5 63 / 46, 72 -> 184 at 7^2, T = 8 134 / 39.
-// Whole tiles stay (64 -> 64 at 56^2 x 16 37 / 50, 128 -> 128 at 28^2 x 16 41 / 41 and with a residual 42 / 50, 192 -> 192 at 8^2 x 64 31 / 35,
-// 256 -> 256 at 8^2 x 64 37 / 37, at 14^2 x 16 with a residual 38 / 39) but for deep layers, whose K the blocked kernel shares among more
-// waves. The line, K = 2304 for few outputs and no residual and K = 4608 for any, is on the safe side: of 197 layers measured behind it, 64 to
-// 640 channels, 3x3 to 7x7, one to eight timesteps, none loses (512 -> 512 with a residual at 8^2 x 64 89 / 89, 128 -> 128 5x5 at 16^2 x 16
-// 30 / 29, 64 -> 128 7x7 at 16^2 x 16 28 / 26, 96 -> 64 5x5 at 16^2 x 16 25 / 21, 256 -> 256 at 14^2 x 4 29 / 18, 320 -> 320 34 / 27, 384 -> 384
-// 37 / 28 (T = 1 21 / 16, T = 6 71 / 47), 448 -> 448 42 / 32, 512 -> 512 46 / 33 there and 37 / 21 at 4^2 x 16). In front of it some would
-// gain as well: 320 to 448 channels with more outputs (at 14^2 x 16 60 / 55, 70 / 61, 79 / 67), and layers of few outputs with less depth or with a
-// residual (128 -> 128 at 14^2 x 4 20 / 14, 384 -> 384 with a residual at 8^2 x 4 37 / 22).
+// Whether a layer on dense tensors is brought into C8 and run on the blocked kernel (two launches) or stays on the dense kernels. Measured on
+// some 1700 layers of 1 to 64 images, 1 to 512 channels, 1x1 to 7x7, one to eight timesteps (us, dense / here; bf16 and T = 4 unless said):
+// * Channel counts that are no multiple of 8 only have the four-wave kernels on dense tensors, which assemble every channel group from
+//   scalar loads: they move (126 -> 200 at 12 x 54 stride 2, T = 2 93 / 18, 29 -> 72 at 70^2, 7x7 stride 2 316 / 23, 61 -> 32 1x1 at 39 x 20, T = 3
+//   29 / 16), but for large 1x1 layers, which are memory traffic (421 -> 288 at 100^2, T = 8 356 / 416).
+// * The matrix kernel's masked variant (planes or channels its tiles do not divide) goes in windows of two timesteps and pays a pass over
+//   the weights per window: 600 layers gain a factor of 2 (72 -> 104 at 27 x 35, T = 6, with a residual 59 / 39, 512 -> 512 at 7^2 x 16 55 / 31,
+//   16 -> 96 at 25^2 x 8 with a residual 25 / 23, 24 -> 16 at 26^2, 5x5, T = 5 64 / 31). Of one or two timesteps, one window there as well, 1x1
+//   layers of any size lose (256 -> 128 at 97^2 x 16, T = 1 115 / 146, 128 -> 256 stride 2 at 28^2 x 52, T = 1 18 / 24) and so do large strided
+//   ones (64 -> 128 at 40^2 x 17, T = 2 16 / 19); 1x1 layers of a stride copy four pixels for one (168 -> 349 at 24 x 75 x 14, T = 6 104 / 123).
+// * The pointwise kernel's straight-line variant takes planes of whole tiles of 64 pixels: 24 -> 96 at 56^2 x 32 31 / 73, 128 -> 256 89 / 224.
+//   Its general variant is several times slower and loses over 260 layers to a factor of 1.8 (128 -> 64 at 7^2, T = 8 60 / 16, 64 -> 256 at
+//   51^2 x 16 with a residual 216 / 127, 128 -> 256 at 28^2 x 32, T = 2 56 / 50).
+// * Whole tiles of the matrix kernel stay where they fill the chip (64 -> 64 at 56^2 x 16 37 / 42, 128 -> 256 1x1 stride 2 at 28^2 x 32 23 / 33,
+//   64 -> 128 stride 2 at 56^2 x 8 21 / 28) and move where they don't: the time of one tile is 33 us there and 8 here. The lines, in outputs of
+//   all timesteps: 64 -> 64 at 24^2 x 4 33 / 12, at 40^2 x 8, T = 2 15 / 16, at 40^2 x 8, T = 6 38 / 34, at 56^2 x 16, T = 8 107 / 110; 128 -> 128 at
+//   28^2 x 4 24 / 21, at 16^2 x 32, T = 2 18 / 17; 64 -> 128 stride 2 at 40^2, T = 4 38 / 14, at 32^2 x 8, T = 2 13 / 12, at 24^2 x 17, T = 2 12 / 13;
+//   1x1 stride 2 64 -> 128 at 40^2 x 4 16 / 14, at 32^2 x 8 14 / 15, at 24^2 x 17, T = 8 29 / 26. Deep layers of few outputs always move
+//   (256 -> 256 at 14^2 x 4 29 / 18, 512 -> 512 at 4^2 x 16 37 / 21). Two kinds that would gain as well stay with the kernel that their reported
+//   plan names in the tests: planes of four pixels at most (256 -> 512 at 2^2 x 40 25 / 14) and one window of four steps of up to 512 pixels
+//   with less than 128 channels (64 -> 64 at 16^2 x 2 33 / 11).
+// * fp32 tensors (two bf16 terms each) run here at three times the speed of the dense kernels over 180 layers: 64 -> 64 at 32^2 x 8 35 / 20, at
+//   56^2 x 16 100 / 73, 512 -> 512 at 7^2 x 4 with a residual 125 / 29, 41 -> 72 at 8 x 14 x 15 191 / 20, 122 -> 111 at 15^2, 5x5, T = 5 1068 / 36,
+//   3 -> 64 at 32^2 x 64 34 / 31, 128 -> 256 1x1 at 28^2 x 8 135 / 27. Only 1x1 layers with few products per output stay, where those are many:
+//   the copy and the elementwise outputs are their time (64 -> 256 at 56^2 x 16, T = 1 with a residual 66 / 82, 64 -> 128 at 112^2 x 4 80 / 90,
+//   32 -> 192 at 56^2 x 16 116 / 124; but 64 -> 128 at 28^2 x 8 79 / 25, 128 -> 256 at 56^2 x 16 281 / 192).
+// Without a neuron the lines are those of sums that leave as 16-bit values (512 -> 512 at 7^2 x 16 56 / 35).
 bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w,
-                         int v_dtype, bool residual, DenseFamily& family) {
+                         int v_dtype, bool residual, bool neuron, DenseFamily& family) {
     if (x_dtype != SNNF_BF16 && x_dtype != SNNF_F16 && x_dtype != SNNF_F32) return false;
     if (v_dtype != SNNF_F32 || T < 1 || T > SNNF_MAX_T_PER_LAUNCH || N < 1 || Cin < 1 || H < 1 || W < 1 || Cout < 1 || KH < 1 || KW < 1 ||
         stride_h < 1 || stride_w < 1 || pad_h < 0 || pad_w < 0 || H + 2 * pad_h < KH || W + 2 * pad_w < KW || 2 * pad_h > KH || 2 * pad_w > KW) return false;
-    const bool pointwise = KH == 1 && KW == 1 && stride_h == 1 && stride_w == 1 && pad_h == 0 && pad_w == 0;
-    const int64_t K = static_cast<int64_t>(Cin) * KH * KW;
-    const int64_t out = static_cast<int64_t>(N) * Cout * ((H + 2 * pad_h - KH) / stride_h + 1) * ((W + 2 * pad_w - KW) / stride_w + 1);
-    // 1x1 layers of whole channel groups are mostly memory traffic and stay (128 -> 256 at 56^2 x 32: 68 us on the pointwise kernel, 79 here
-    // even on bit-packed spikes), and so do those of a single group, which have next to no products.
-    if (x_dtype != SNNF_F32 && pointwise && (Cin % 8 == 0 || Cin < 8)) return false;
+    const bool one = KH == 1 && KW == 1, strided = stride_h > 1 || stride_w > 1;
+    const bool pointwise = one && !strided && pad_h == 0 && pad_w == 0;
+    const int64_t K = static_cast<int64_t>(Cin) * KH * KW, plane = static_cast<int64_t>(H) * W;
+    const int64_t pixels = static_cast<int64_t>(N) * ((H + 2 * pad_h - KH) / stride_h + 1) * ((W + 2 * pad_w - KW) / stride_w + 1);
+    const int64_t out = pixels * Cout, outs = T * out;
     family = dense_family(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w);
-    // fp32 tensors (two bf16 terms each) run here at three times the speed of the dense kernels over 180 measured layers (us, dense / here):
-    // 64 -> 64 at 32^2 x 8 35 / 20, at 56^2 x 16 100 / 73, 512 -> 512 at 7^2 x 4 with a residual 125 / 29, 240 -> 32 at 60 x 74, T = 3 212 / 72,
-    // 41 -> 72 at 8 x 14 x 15 191 / 20, 122 -> 111 at 15^2, 5x5, T = 5 1068 / 36, 3 -> 64 at 32^2 x 64 34 / 31, 128 -> 256 1x1 at 28^2 x 8 135 / 27.
-    // Only 1x1 layers with few products per output stay, where those are many: the copy and the elementwise outputs are their time
-    // (64 -> 256 at 56^2 x 16, T = 1 with a residual 66 / 82, 64 -> 128 at 112^2 x 4 80 / 90, 32 -> 192 at 56^2 x 16 116 / 124; but
-    // 64 -> 128 at 28^2 x 8 79 / 25, 128 -> 256 at 56^2 x 16 281 / 192, 64 -> 64 at 112^2 x 8 128 / 98).
-    if (x_dtype == SNNF_F32) return !(family == DenseFamily::kPointwise && Cin <= 64 && Cout >= 96 && T * out >= (1 << 22));
+    if (x_dtype == SNNF_F32) return !(family == DenseFamily::kPointwise && Cin <= 64 && Cout >= 96 && outs >= (1 << 22));
+    const bool deep = K >= 4608 || (K >= 2304 && out <= (1 << 19) && !residual);
+    if (!neuron) {
+        if (pointwise) return false;
+        return family == DenseFamily::kMatrixMasked ? !(T > 4 && Cin < 56) && (T <= 2 ? K >= 1152 : K >= (residual ? 640 : 432)) : family == DenseFamily::kMatrixWhole && deep;
+    }
+    if (pointwise && Cin < 8) return false;   // a single channel group: next to no products
     switch (family) {
         case DenseFamily::kTInM:
-        case DenseFamily::kTimeOuter: return !pointwise || static_cast<int64_t>(T) * N * (Cin + Cout) * H * W <= (1 << 25);
-        case DenseFamily::kMatrixMasked: return T > 4 && Cin < 56 ? false : T <= 2 ? K >= 1152 : K >= (residual ? 640 : 432);
-        case DenseFamily::kMatrixWhole: return K >= 4608 || (K >= 2304 && out <= (1 << 19) && !residual);
-        default: return false;
+        case DenseFamily::kTimeOuter: return !pointwise || static_cast<int64_t>(T) * N * (Cin + Cout) * plane <= (1 << 25);
+        case DenseFamily::kPointwise: return plane % 64 != 0 || (Cout % 32 != 0 && outs <= (1 << 22));
+        case DenseFamily::kMatrixMasked:
+            if (one) return T <= 2 ? outs <= (1 << 17) : !strided || T * N * Cin * plane <= (1 << 24);
+            return T > 2 || K >= 1152 || !strided || outs <= (3 << 19);
+        case DenseFamily::kMatrixWhole:
+            if (deep) return true;
+            if (plane <= 4 || (T >= 3 && T <= 4 && !one && !strided && pixels <= 512 && K < 1152)) return false;
+            if (one) return outs <= (T <= 2 ? 3 << 17 : (T <= 4 ? 5 << 17 : 5 << 19));
+            if (strided) return outs <= (T <= 2 ? 1 << 19 : (T <= 4 ? 1 << 20 : 3 << 20));
+            if (K < 432) return Cin > 8 && outs <= (1 << 19);   // (a single channel group: as above)
+            return outs <= (K < 1152 ? (T <= 4 ? 3 << 19 : 1 << 23) : (T <= 4 ? 1 << 21 : 1 << 24));
     }
+    return false;
 }
 
 bool valid_layout(int layout) { return layout == SNNF_LAYOUT_NCHW || layout == SNNF_LAYOUT_C8 || layout == SNNF_LAYOUT_BITS; }
@@ -364,7 +378,7 @@ Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, 
         if (it != routes().end()) return it->second;
     }
     Route route = {false, DenseFamily::kTInM};
-    route.taken = takes_blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residual, route.family) &&
+    route.taken = takes_blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residual, neuron, route.family) &&
                   (neuron || (!split && (route.family == DenseFamily::kMatrixMasked || route.family == DenseFamily::kMatrixWhole)));
     if (route.taken) {
         BlockedPlan plan;
