@@ -253,6 +253,7 @@ int snnf_conv_lif(const void* const* xs, const void* const* residuals, int T,
  *   snnf_conv_lif_workspace_bytes : the same for 16-bit activations beside an fp32 membrane, 0 for every other call.
  *   workspace : NULL (then this is snnf_conv_lif), or device memory, 16-byte aligned, contents undefined before and after.
  *               A smaller workspace than asked for is not used. Calls that share a workspace must not overlap in time.
+ *   v_dtype : a 16-bit membrane is held in fp32 (in the workspace, between the windows of a call) and rounded once at the end.
  */
 size_t snnf_conv_lif_scratch_bytes(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW,
                                    int stride_h, int stride_w, int pad_h, int pad_w, int v_dtype, int has_residual);

@@ -641,9 +641,17 @@ bool conv_call(const Call& c, Attempt& key, Op op, Pair* out) {
     const int N = static_cast<int>(x.size(0)), cin = static_cast<int>(x.size(1)), H = static_cast<int>(x.size(2)), W = static_cast<int>(x.size(3));
     const int64_t step = shape[0] * shape[1] * shape[2] * shape[3];
     Tensor spikes = op == kConvSingle ? empty(shape, x.scalar_type(), x) : empty({T, shape[0], shape[1], shape[2], shape[3]}, x.scalar_type(), x);
-    const bool wide = m.dtype != at::kFloat && T > (depthwise ? SNNF_MAX_T_PER_LAUNCH : 1);
-    WorkMembrane wm(x, m, shape, wide);
     const void* const* residuals = residual ? rs : nullptr;
+    const auto scratch_bytes = [&](int v_code) -> size_t {
+        if (depthwise || one_frame(steps, T)) return 0;
+        return snnf_conv_lif_scratch_bytes(static_cast<int>(T), N, cin, H, W, code_of(x.scalar_type()), static_cast<int>(shape[1]), static_cast<int>(kh),
+                                           static_cast<int>(kw), static_cast<int>(sh), static_cast<int>(sw), static_cast<int>(ph), static_cast<int>(pw),
+                                           v_code, residual ? 1 : 0);
+    };
+    // With scratch memory the library keeps a 16-bit membrane wide between its launches by itself.
+    size_t bytes = scratch_bytes(code_of(m.dtype));
+    const bool wide = bytes == 0 && m.dtype != at::kFloat && T > (depthwise ? SNNF_MAX_T_PER_LAUNCH : 1);
+    WorkMembrane wm(x, m, shape, wide);
     int status;
     if (depthwise) {
         status = snnf_dwconv3x3_lif(steps, residuals, static_cast<int>(T), N, cin, H, W, static_cast<int>(sh), code_of(x.scalar_type()), w.data_ptr(),
@@ -651,10 +659,7 @@ bool conv_call(const Call& c, Attempt& key, Op op, Pair* out) {
                                     static_cast<float>(lif.v_threshold), static_cast<float>(lif.v_reset), static_cast<float>(lif.tau), stream);
     } else {
         const Tensor packed = packed_weight(w, b, x.scalar_type());
-        const size_t bytes = one_frame(steps, T) ? 0
-            : snnf_conv_lif_scratch_bytes(static_cast<int>(T), N, cin, H, W, code_of(x.scalar_type()), static_cast<int>(shape[1]), static_cast<int>(kh),
-                                            static_cast<int>(kw), static_cast<int>(sh), static_cast<int>(sw), static_cast<int>(ph), static_cast<int>(pw),
-                                            wm.code(), residual ? 1 : 0);
+        if (wide) bytes = scratch_bytes(wm.code());
         Tensor workspace;
         if (bytes > 0) workspace = empty({static_cast<int64_t>(bytes)}, at::kByte, x);
         status = snnf_conv_lif_ws(steps, residuals, static_cast<int>(T), N, cin, H, W, code_of(x.scalar_type()), packed.data_ptr(),

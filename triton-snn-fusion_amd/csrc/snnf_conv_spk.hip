@@ -84,11 +84,12 @@ std::map<TunedKey, TunedPlan>& tuned_plans() {
 
 size_t c8_step_bytes(int N, int Cin, int H, int W) { return static_cast<size_t>(N) * ((Cin + 7) / 8) * H * W * 16; }
 
-// The workspace of a call on the blocked route: the C8 steps; of fp32 tensors the steps of their low terms and the flags behind them.
+// The workspace of a call on the blocked route: the C8 steps; of fp32 tensors the steps of their low terms and the flags behind them; the
+// fp32 membrane that a call of several windows with a 16-bit one passes from window to window (rounded once, at the end).
 struct RouteSpace {
-    size_t step, lo, flags, flag_stride, total;        // bytes; offsets of the low terms and of the flags
+    size_t step, lo, flags, flag_stride, carry, total; // bytes; offsets of the low terms, the flags and the membrane
 };
-RouteSpace route_space(int T, int N, int Cin, int H, int W, bool split) {
+RouteSpace route_space(int T, int N, int Cin, int H, int W, bool split, int64_t carried) {
     RouteSpace r = {};
     r.step = c8_step_bytes(N, Cin, H, W);
     r.total = r.step * T;
@@ -98,6 +99,8 @@ RouteSpace route_space(int T, int N, int Cin, int H, int W, bool split) {
         r.flag_stride = (r.step / 16 + 255) / 256 * 4;   // one byte per 64 items, in whole dwords
         r.total = r.flags + r.flag_stride * T;
     }
+    r.carry = r.total;                                   // (a multiple of 16: no call has both)
+    r.total += static_cast<size_t>(carried) * 4;
     return r;
 }
 
@@ -131,7 +134,7 @@ RouteSpace route_space(int T, int N, int Cin, int H, int W, bool split) {
 bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w,
                          int v_dtype, bool residual, bool neuron, DenseFamily& family) {
     if (x_dtype != SNNF_BF16 && x_dtype != SNNF_F16 && x_dtype != SNNF_F32) return false;
-    if (v_dtype != SNNF_F32 || T < 1 || T > SNNF_MAX_T_PER_LAUNCH || N < 1 || Cin < 1 || H < 1 || W < 1 || Cout < 1 || KH < 1 || KW < 1 ||
+    if ((v_dtype != SNNF_F32 && v_dtype != x_dtype) || T < 1 || T > SNNF_MAX_T_PER_LAUNCH || N < 1 || Cin < 1 || H < 1 || W < 1 || Cout < 1 || KH < 1 || KW < 1 ||
         stride_h < 1 || stride_w < 1 || pad_h < 0 || pad_w < 0 || H + 2 * pad_h < KH || W + 2 * pad_w < KW || 2 * pad_h > KH || 2 * pad_w > KW) return false;
     const bool one = KH == 1 && KW == 1, strided = stride_h > 1 || stride_w > 1;
     const bool pointwise = one && !strided && pad_h == 0 && pad_w == 0;
@@ -359,7 +362,7 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
 // matrix kernel only; what it refuses stays refused. The answer depends on the layer and the table of tuned plans alone and is
 // kept per layer: it is asked for twice per call.
 using RouteKey = std::array<int, 15>;
-struct Route { bool taken; DenseFamily family; };
+struct Route { bool taken; DenseFamily family; int windows; };
 std::mutex routes_mutex;
 std::map<RouteKey, Route>& routes() {
     static std::map<RouteKey, Route> known;
@@ -369,7 +372,7 @@ constexpr size_t kMaxRoutes = 4096;
 
 Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w,
                     int v_dtype, bool residual, bool neuron) {
-    if (!valid_dtype(x_dtype) || v_dtype != SNNF_F32) return {false, DenseFamily::kTInM};
+    if (!valid_dtype(x_dtype) || (v_dtype != SNNF_F32 && v_dtype != x_dtype)) return {false, DenseFamily::kTInM, 0};
     const bool split = x_dtype == SNNF_F32;
     const RouteKey key = {T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, residual ? 1 : 0, neuron ? 1 : 0, split ? 1 : 0};
     {
@@ -377,13 +380,14 @@ Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, 
         const auto it = routes().find(key);
         if (it != routes().end()) return it->second;
     }
-    Route route = {false, DenseFamily::kTInM};
+    Route route = {false, DenseFamily::kTInM, 0};
     route.taken = takes_blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residual, neuron, route.family) &&
                   (neuron || (!split && (route.family == DenseFamily::kMatrixMasked || route.family == DenseFamily::kMatrixWhole)));
     if (route.taken) {
         BlockedPlan plan;
         route.taken = plan_blocked("snnf_conv_lif_workspace_bytes", BlockedCall{T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, SNNF_LAYOUT_C8,
                                    residual ? SNNF_LAYOUT_NCHW : -1, SNNF_LAYOUT_NCHW, 0, false, neuron, false, neuron, false, nullptr, split}, plan) == SNNF_OK;
+        route.windows = plan.windows;
     }
     std::lock_guard<std::mutex> lock(routes_mutex);
     if (routes().size() >= kMaxRoutes) routes().clear();
@@ -391,11 +395,18 @@ Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, 
     return route;
 }
 
+// fp32 elements that pass from window to window beside a 16-bit membrane.
+int64_t carried_membrane(const Route& r, int v_dtype, int N, int H, int W, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w) {
+    if (v_dtype == SNNF_F32 || r.windows <= 1) return 0;
+    return static_cast<int64_t>(N) * Cout * ((H + 2 * pad_h - KH) / stride_h + 1) * ((W + 2 * pad_w - KW) / stride_w + 1);
+}
+
 // A call on dense tensors that runs here: its inputs, which are brought into C8 first, and the kernel family of the dense route.
 struct DenseRoute {
     const void* const* xs;
     DenseFamily family;
     RouteSpace space;
+    int v_dtype;
 };
 const char* family_name(DenseFamily f) {
     return f == DenseFamily::kTInM ? "t_in_m" : (f == DenseFamily::kTimeOuter ? "time_outer" : (f == DenseFamily::kPointwise ? "pointwise" : "matrix"));
@@ -472,22 +483,23 @@ extern "C" int snnf_conv_lif_blocked_avgpool(const void* const* xs, int x_layout
 
 extern "C" size_t snnf_conv_lif_workspace_bytes(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h,
                                                 int stride_w, int pad_h, int pad_w, int v_dtype, int residual) {
-    if (x_dtype != SNNF_BF16 && x_dtype != SNNF_F16) return 0;
+    if ((x_dtype != SNNF_BF16 && x_dtype != SNNF_F16) || v_dtype != SNNF_F32) return 0;
     return snnf_conv_lif_scratch_bytes(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residual);
 }
 
 extern "C" size_t snnf_conv_lif_scratch_bytes(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h,
                                               int stride_w, int pad_h, int pad_w, int v_dtype, int residual) {
     using namespace snnf;
-    if (!blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residual != 0, true).taken) return 0;
-    return route_space(T, N, Cin, H, W, x_dtype == SNNF_F32).total;
+    const Route route = blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residual != 0, true);
+    if (!route.taken) return 0;
+    return route_space(T, N, Cin, H, W, x_dtype == SNNF_F32, carried_membrane(route, v_dtype, N, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w)).total;
 }
 
 extern "C" size_t snnf_conv_bias_workspace_bytes(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h,
                                                  int stride_w, int pad_h, int pad_w, int residual) {
     using namespace snnf;
     if (!blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, SNNF_F32, residual != 0, false).taken) return 0;
-    return route_space(T, N, Cin, H, W, x_dtype == SNNF_F32).total;
+    return route_space(T, N, Cin, H, W, false, 0).total;
 }
 
 namespace snnf {
@@ -500,7 +512,8 @@ int run_blocked_route(const void* const* xs, const void* const* residuals, int T
     if (xs == nullptr || workspace == nullptr || (neuron && v_out == nullptr) || !aligned_to(workspace, 16) || out_step_stride < 0) return SNNF_ERR_UNSUPPORTED;
     const Route taken = blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residuals != nullptr, neuron != 0);
     if (!taken.taken) return SNNF_ERR_UNSUPPORTED;
-    const RouteSpace space = route_space(T, N, Cin, H, W, x_dtype == SNNF_F32);
+    const RouteSpace space = route_space(T, N, Cin, H, W, x_dtype == SNNF_F32,
+                                         neuron ? carried_membrane(taken, v_dtype, N, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w) : 0);
     if (workspace_bytes < space.total) return SNNF_ERR_UNSUPPORTED;
     bool shared = T > 1;
     const void* inner[SNNF_MAX_T_PER_LAUNCH];
@@ -510,7 +523,7 @@ int run_blocked_route(const void* const* xs, const void* const* residuals, int T
         inner[t] = static_cast<const char*>(workspace) + t * space.step;
     }
     if (shared) return SNNF_ERR_UNSUPPORTED;       // one frame for all timesteps is convolved once on the dense kernels too
-    const DenseRoute route = {xs, taken.family, space};
+    const DenseRoute route = {xs, taken.family, space, v_dtype};
     return conv_lif_blocked_impl(neuron ? "snnf_conv_lif" : "snnf_conv_bias", inner, SNNF_LAYOUT_C8, residuals, SNNF_LAYOUT_NCHW, T, N, Cin, H, W, x_dtype,
                                  packed_weight, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_init, out, SNNF_LAYOUT_NCHW, out_step_stride * dtype_size(x_dtype), v_out,
                                  neuron, v_threshold, v_reset, tau, stream, nullptr, false, &route);
@@ -569,8 +582,9 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     // Bytes a tensor in a layout is accessed by: bit-packed tensors by single bytes, blocked inputs by 16-byte groups, blocked
     // outputs and residuals by 4 channels (8 bytes), dense tensors by elements.
     auto need_align = [x_dtype](int layout, bool as_input) -> size_t { return layout == SNNF_LAYOUT_BITS ? 1 : (layout == SNNF_LAYOUT_C8 ? (as_input ? 16 : 8) : static_cast<size_t>(dtype_size(x_dtype))); };
+    const size_t v_align = dense != nullptr && dense->v_dtype != SNNF_F32 ? 2 : 4;
     if (!aligned_to(packed_weight, 16) || !aligned_to(out, need_align(out_layout, false)) || (out_step_stride % need_align(out_layout, false)) != 0 ||
-        (v_init != nullptr && !aligned_to(v_init, 4)) || (v_out != nullptr && !aligned_to(v_out, 4)))
+        (v_init != nullptr && !aligned_to(v_init, v_align)) || (v_out != nullptr && !aligned_to(v_out, v_align)))
         return fail(SNNF_ERR_INVALID_ARGUMENT, "%s: packed_weight, out (and its step stride) or a membrane pointer is misaligned", who);
     bool shared = T > 1;
     for (int t = 0; t < T; ++t) {
@@ -624,6 +638,10 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     L.out = out;
     L.v_out = neuron ? v_out : nullptr;
     L.v_carry = static_cast<float*>(L.v_out);
+    if (dense != nullptr && neuron && dense->v_dtype != SNNF_F32) {
+        L.g.v16 = 1;
+        L.v_carry = reinterpret_cast<float*>(static_cast<char*>(const_cast<void*>(xs[0])) + dense->space.carry);
+    }
     L.lif = make_lif_params(v_threshold, v_reset, tau);
     L.grid = p.grid;
     L.lds_bytes = p.lds_bytes;

@@ -347,6 +347,16 @@ def _one_frame(pointers) -> bool:
     return len(pointers) > 1 and len(set(pointers)) == 1
 
 
+def _scratch_bytes(pointers, first: torch.Tensor, weight, stride, padding, v_code: int, residual: bool) -> int:
+    """Scratch memory that snnf_conv_lif_ws runs the call with (one frame for all timesteps needs none)."""
+    if _one_frame(pointers):
+        return 0
+    n, cin, h, w = (int(d) for d in first.shape)
+    cout, _, kh, kw = (int(d) for d in weight.shape)
+    return int(_lib.lib().snnf_conv_lif_scratch_bytes(len(pointers), n, cin, h, w, _lib.dtype_code(first.dtype), cout, kh, kw, *_as_pair(stride),
+                                                      *_as_pair(padding), v_code, 1 if residual else 0))
+
+
 def _launch(kernel_key: str, steps: Sequence[torch.Tensor], residuals: Optional[Sequence[torch.Tensor]], weight, bias,
             v_init, stride, padding, v_threshold, v_reset, tau, spikes: torch.Tensor, v_out: torch.Tensor) -> None:
     """Enqueues the HIP kernel(s) for one fused conv+LIF call. `steps` are T contiguous [N, C, H, W] tensors."""
@@ -373,11 +383,9 @@ def _launch(kernel_key: str, steps: Sequence[torch.Tensor], residuals: Optional[
             float(v_threshold), float(v_reset), float(tau), stream))
     else:
         packed = _packed_weight(weight, bias, first.dtype)
-        # Scratch for the inputs in the channel-blocked layout where the library asks for it (one frame for all timesteps needs none);
-        # the caching allocator hands the block out again in the order of the stream the kernels run on.
-        nbytes = 0
-        if not _one_frame(xs):
-            nbytes = int(lib.snnf_conv_lif_scratch_bytes(T, n, cin, h, w, x_code, cout, kh, kw, sh, sw, ph, pw, v_code, 1 if rs is not None else 0))
+        # Scratch for the inputs in the channel-blocked layout where the library asks for it; the caching allocator hands the block out
+        # again in the order of the stream the kernels run on.
+        nbytes = _scratch_bytes(xs, first, weight, (sh, sw), (ph, pw), v_code, rs is not None)
         workspace = torch.empty(nbytes, dtype=torch.uint8, device=first.device) if nbytes else None
         _lib.check("snnf_conv_lif", lib.snnf_conv_lif_ws(
             xs, rs, T, n, cin, h, w, x_code, packed.data_ptr(), cout, kh, kw, sh, sw, ph, pw,
@@ -494,8 +502,11 @@ def _run_temporal(kind: str, xs, residuals, weight, bias, v_init, stride, paddin
     # membrane would be rounded at every hand-over, where the reference's kernel rounds once after the last step
     # (kernels/benchmark_conv_lif_temporal_general.py:707-716). How many launches the matrix kernels take depends on the
     # membrane dtype itself (their one-launch variant needs a float32 membrane), so every multi-step call with a 16-bit
-    # membrane computes with a float32 working membrane and rounds the result once: the same arithmetic on every call.
+    # membrane computes with a float32 working membrane and rounds the result once: the same arithmetic on every call. With scratch memory
+    # the library does so by itself.
     wide = v_dtype != torch.float32 and T > 1 and _takes_several_launches(kernel_key, T)
+    if wide and not kernel_key.startswith("depthwise_"):
+        wide = _scratch_bytes(_lib.step_pointers(steps), first, weight, stride, padding, _lib.dtype_code(v_dtype), res is not None) == 0
     v_work = torch.empty(out_shape, dtype=torch.float32, device=first.device) if wide else v_next
     if wide and isinstance(v_init, torch.Tensor) and v_init.dim() > 0:
         v_init = v_init.float()
