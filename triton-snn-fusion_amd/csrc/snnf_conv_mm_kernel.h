@@ -38,15 +38,23 @@ __host__ __device__ constexpr int mm_staging_slots(int load_mode, int tt, bool s
 }
 typedef float cv_f32x4 __attribute__((ext_vector_type(4)));
 
+// fast_div without a branch (the quotient of a divisor of 1 comes from a mask).
+__device__ __forceinline__ int mm_div(int n, const FastDiv& f) {
+    const uint32_t keep = f.d == 1u ? 0xffffffffu : 0u;
+    return static_cast<int>((__umulhi(static_cast<uint32_t>(n), f.mul) >> f.shift) | (static_cast<uint32_t>(n) & keep));
+}
+
 // NW waves per workgroup: 8 (one workgroup per CU) or 4 (two independent workgroups per CU, whose load, matrix and
 // epilogue phases overlap each other instead of running in lockstep across the whole CU).
-template <typename XT, int TT, int LM, bool FAST, bool SK, int NW>
+template <typename XT, int TT, int LM, bool FAST, bool SK, int NW, bool STAGED = false>
 __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void conv_mm_lif_kernel(
     const StepPtrs xs, const StepPtrs residuals, const int has_residual, const ConvGeom g,
     const uint16_t* __restrict__ wpacked, const float* __restrict__ bias, const void* __restrict__ v_init,
     XT* __restrict__ spikes, void* __restrict__ v_out, const LifParams lif) {
     extern __shared__ __align__(16) unsigned char lds[];
     constexpr bool F16 = dtype_of<XT>::value == SNNF_F16;
+    constexpr bool SPIKES = FAST && sizeof(XT) == 2 && !STAGED;   // the epilogue of 16-bit spikes
+    constexpr bool LATE = SPIKES && !SK && TT == 4;   // the next tile's loads go out when half of the accumulators have been used
     constexpr int RPE = LM == LOAD_PAIR32 ? 1 : 2;
     constexpr int SS = mm_staging_slots(LM, TT, SK);
     constexpr uint32_t ES = static_cast<uint32_t>(sizeof(XT));
@@ -294,26 +302,20 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu
     const bool m_inside = mpi < g.TI;                        // lanes beyond the tile read pixel (0, 0): finite, never stored
     const uint32_t b_base = static_cast<uint32_t>(m_inside ? ((mpi * g.NR + mpr * g.sh) * g.WT + mpc * g.sw) * g.pitch : 0);
 
-    // ---- kernel constants of the epilogue: lane = (channel row lane >> 2 of 16, pixels 8 (lane & 3) .. + 7 of the wave's 32).
-    const int row16 = lane >> 2;
-    const int pcx = lane & 3;
-    const int epix = wm * 32 + pcx * 8;
-    const int epi = fast_div(epix, g.d_tile_px);
-    const int erem = epix - epi * tile_px;
-    const int epr = fast_div(erem, g.d_TW);
-    const int epc = erem - epr * g.TW;
-    const bool lo_inside = epix + 4 <= g.TI * tile_px;       // FAST: planes and tiles are multiples of 4 (8 with 16-byte runs), so
-    const bool hi_inside = epix + 8 <= g.TI * tile_px;       // each half of a lane's run of 8 pixels is inside or outside as a whole
-    const uint32_t image_out = static_cast<uint32_t>(g.Cout) * static_cast<uint32_t>(g.Ho * g.Wo);
-    const uint32_t lane_px = static_cast<uint32_t>(epi) * image_out + static_cast<uint32_t>(epr * g.Wo + epc);
-    // The second half of the lane's run of 8 (pixels epix + 4 .. + 7): contiguous with the first half inside an image, but
-    // with tiles of several whole planes of 4 pixels (2x2 planes) it lies in the next image of the tile.
-    const int epi_hi = fast_div(epix + 4, g.d_tile_px);
-    const int erem_hi = epix + 4 - epi_hi * tile_px;
-    const int epr_hi = fast_div(erem_hi, g.d_TW);
-    const uint32_t lane_px_hi = static_cast<uint32_t>(epi_hi) * image_out + static_cast<uint32_t>(epr_hi * g.Wo + (erem_hi - epr_hi * g.TW));
-    float* __restrict__ stage_wr = stage + (half * 4) * kMmStagePitch + l32;
-    const float* __restrict__ stage_rd = stage + row16 * kMmStagePitch + pcx * 8;
+    // ---- pair table: slot 2 * pair + half of a packed chunk is (tap, channel group); where a pair's two slots lie in the staged halo,
+    // in units of 16 bytes (even slot | odd slot << 16). Lane i holds pair i, one v_readlane per matrix step: computed on the scalar
+    // unit instead, some 40 dependent instructions stood between two pairs (18 pairs in 14.4 k cycles, 9.2 k of them matrix
+    // instructions, at 64 -> 64). Pairs from 64 on (7x7 kernels) are still computed.
+    auto pair_offsets = [&](int pair) __attribute__((always_inline)) -> uint32_t {
+        const int s0 = 2 * pair, s1 = 2 * pair + 1;
+        // With a single channel group an odd tap count leaves the last k-slot empty (zero weights): it re-reads the last tap.
+        const int tap0 = min(s0 >> g.groups_log2, taps - 1), tap1 = min(s1 >> g.groups_log2, taps - 1);
+        const int kh0 = mm_div(tap0, g.d_KW), kh1 = mm_div(tap1, g.d_KW);
+        const uint32_t even = static_cast<uint32_t>((((kh0 * g.WT) + (tap0 - kh0 * g.KW)) * g.pitch + (s0 & (groups - 1)) * 16) >> 4);
+        const uint32_t odd = static_cast<uint32_t>((((kh1 * g.WT) + (tap1 - kh1 * g.KW)) * g.pitch + (s1 & (groups - 1)) * 16) >> 4);
+        return even | (odd << 16);
+    };
+    const uint32_t pair_table = pair_offsets(lane);
     const float c0f = lif.charge_mode == CHARGE_IF ? 0.0f : 1.0f;
     const float c1f = lif.charge_mode == CHARGE_IF ? 1.0f : lif.inv_tau;
     const bool divide = lif.charge_mode == CHARGE_DIVIDE;   // tau is not a power of two: a true division
@@ -340,8 +342,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu
         int next_work = work, next_oc_tile = oc_tile, next_img = img, next_oh0 = oh0, next_ow0 = ow0;
         bool next_tile = false;
         int stage_now = 0;       // the LDS stage the matrix steps are working on
-        // One pair of k-slots: slot 2 * pair + half -> (tap, channel group); both halves' LDS offsets are computed on the
-        // scalar unit, a lane picks its half's.
+        // One pair of k-slots: its LDS offsets come out of the pair table, a lane picks its half's.
         auto mma_pair = [&](int q, const unsigned char* __restrict__ bp0, const cv_u32x4& a0, const cv_u32x4& a1) __attribute__((always_inline)) {
             if constexpr (PARTS > 1) {   // q counts the stage's pairs three times over: part 2 reads the low terms
                 const int sp = min(g.stage_chunks, g.nchunks_r - stage_now * g.stage_chunks) * g.npairs;
@@ -349,16 +350,22 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu
                 q -= part * sp;
                 bp0 += part == 2 ? lo_off : 0;
             }
-            const int sub = fast_div(q, g.d_npairs);                 // chunk inside the stage
-            const int pair = q - sub * g.npairs;
-            const unsigned char* __restrict__ bp = bp0 + sub * (groups * 16);
-            const int s0 = 2 * pair, s1 = 2 * pair + 1;
-            // With a single channel group an odd tap count leaves the last k-slot empty (zero weights): it re-reads the last tap.
-            const int tap0 = s0 >> g.groups_log2, tap1 = min(s1 >> g.groups_log2, taps - 1);
-            const int kh0 = fast_div(tap0, g.d_KW), kh1 = fast_div(tap1, g.d_KW);
-            const int off_even = ((kh0 * g.WT) + (tap0 - kh0 * g.KW)) * g.pitch + (s0 & (groups - 1)) * 16;
-            const int off_odd = ((kh1 * g.WT) + (tap1 - kh1 * g.KW)) * g.pitch + (s1 & (groups - 1)) * 16;
-            const unsigned char* __restrict__ bq = bp + (half ? off_odd : off_even);
+            int sub, pair;                                           // chunk inside the stage, pair inside the chunk
+            if (g.stage_chunks == 1) {
+                sub = 0;
+                pair = q;
+            } else {
+                sub = fast_div(q, g.d_npairs);
+                pair = q - sub * g.npairs;
+            }
+            uint32_t both;
+            if (pair < 64) {
+                both = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(pair_table), pair));
+            } else {
+                both = pair_offsets(pair);
+            }
+            const uint32_t off_even = (both & 0xffffu) * 16u, off_odd = (both >> 16) * 16u;
+            const unsigned char* __restrict__ bq = bp0 + sub * (groups * 16) + (half ? off_odd : off_even);
 #pragma unroll
             for (int t = 0; t < TT; ++t) {
                 const cv_u32x4 b = *reinterpret_cast<const cv_u32x4*>(bq + t * tile_bytes);
@@ -407,7 +414,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu
                     nc = 0;
                     next_work = work + slots_per_xcd;
                     next_tile = decode(next_work, next_oc_tile, next_img, next_oh0, next_ow0);
-                    more = next_tile && !SK;   // split K: the next tile's loads go out after the epilogue (registers)
+                    more = next_tile && !SK && !LATE;   // split K: the next tile's loads go out after the epilogue (registers)
                     nimg = next_img;
                     halo_origin(next_oh0, next_ow0, nih, niw);
                 }
@@ -434,6 +441,37 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu
             }
         }
 
+        // ---- where this lane's results go: lane = (channel row lane >> 2 of 16, pixels 8 (lane & 3) .. + 7 of the wave's 32), and the one
+        // pixel of its accumulators. The lane is made opaque here, so that all of it is computed now: kept in registers across the
+        // matrix loop, which needs them all, it was spilled.
+        int lane_e = lane;
+        if constexpr (SPIKES) asm volatile("" : "+v"(lane_e));
+        const int half_e = lane_e >> 5, l32_e = lane_e & 31;
+        const int mpix_e = wm * 32 + l32_e;
+        const int mpi_e = mm_div(mpix_e, g.d_tile_px);
+        const int mrem_e = mpix_e - mpi_e * tile_px;
+        const int mpr_e = mm_div(mrem_e, g.d_TW);
+        const int mpc_e = mrem_e - mpr_e * g.TW;
+        const bool m_in = mpi_e < g.TI;
+        const int row16 = lane_e >> 2;
+        const int pcx = lane_e & 3;
+        const int epix = wm * 32 + pcx * 8;
+        const int epi = mm_div(epix, g.d_tile_px);
+        const int erem = epix - epi * tile_px;
+        const int epr = mm_div(erem, g.d_TW);
+        const int epc = erem - epr * g.TW;
+        const bool lo_inside = epix + 4 <= g.TI * tile_px;       // FAST: planes and tiles are multiples of 4 (8 with 16-byte runs), so
+        const bool hi_inside = epix + 8 <= g.TI * tile_px;       // each half of a lane's run of 8 pixels is inside or outside as a whole
+        const uint32_t image_out = static_cast<uint32_t>(g.Cout) * static_cast<uint32_t>(g.Ho * g.Wo);
+        const uint32_t lane_px = static_cast<uint32_t>(epi) * image_out + static_cast<uint32_t>(epr * g.Wo + epc);
+        // The second half of the lane's run of 8 (pixels epix + 4 .. + 7): contiguous with the first half inside an image, but
+        // with tiles of several whole planes of 4 pixels (2x2 planes) it lies in the next image of the tile.
+        const int epi_hi = mm_div(epix + 4, g.d_tile_px);
+        const int erem_hi = epix + 4 - epi_hi * tile_px;
+        const int epr_hi = mm_div(erem_hi, g.d_TW);
+        const uint32_t lane_px_hi = static_cast<uint32_t>(epi_hi) * image_out + static_cast<uint32_t>(epr_hi * g.Wo + (erem_hi - epr_hi * g.TW));
+        float* __restrict__ stage_wr = stage + (half_e * 4) * kMmStagePitch + l32_e;
+        const float* __restrict__ stage_rd = stage + row16 * kMmStagePitch + pcx * 8;
         // ---- epilogue. h = v + (x - v * c0) * c1 covers tau <= 1 and power-of-two tau exactly.
         // FAST: 16 channel rows x 32 pixels at a time go through the wave's LDS stage, so that a lane owns 8 consecutive pixels
         // of one channel row (16- or 8-byte accesses); the membrane of those 8 neurons lives in registers across the TT steps.
@@ -443,18 +481,18 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu
         const bool vf32 = FAST || g.v_is_f32;
         const bool wide = !FAST || g.run8 == 8;          // FAST: 16-byte spike accesses, or 8-byte ones when runs are only 8-byte aligned
         const uint32_t okmask = FAST ? ((lo_inside ? 0x0fu : 0u) | (hi_inside ? 0xf0u : 0u))
-                                     : ((m_inside && img + mpi < g.N && oh0 + mpr < g.Ho && ow0 + mpc < g.Wo) ? 0xffu : 0u);
+                                     : ((m_in && img + mpi_e < g.N && oh0 + mpr_e < g.Ho && ow0 + mpc_e < g.Wo) ? 0xffu : 0u);
         // Element offset of the lane's first pixel (FAST: of its run of 8) from the tile origin of its channel row.
-        const uint32_t px0 = FAST ? lane_px : static_cast<uint32_t>(mpi) * image_out + static_cast<uint32_t>(mpr * g.Wo + mpc);
+        const uint32_t px0 = FAST ? lane_px : static_cast<uint32_t>(mpi_e) * image_out + static_cast<uint32_t>(mpr_e * g.Wo + mpc_e);
         const uint32_t px4 = lane_px_hi;   // FAST: offset of the run's second half
         const int64_t tile_off = static_cast<int64_t>(img) * g.Cout * po + oh0 * g.Wo + ow0;   // uniform, elements
-        const bool analog = g.analog_out != 0;   // neuron-free output: conv + bias (+ residual) where the spikes would go
+        const bool analog = FAST ? STAGED && (sizeof(XT) == 4 || g.analog_out != 0) : g.analog_out != 0;   // neuron-free output: conv + bias (+ residual) where the spikes would go
 
         // One group = 8 accumulator registers of a 32-row fragment: FAST, after the transposition, this lane's channel row
         // row16 of the group's 16 rows; general variant, the lane's 8 rows first + {0..3, 8..11} with
         // first = 32 fragment + 16 (gidx & 1) + 4 half. `row_ok`: the lane has anything to load or store in the group.
         auto first_row = [&](int gidx) __attribute__((always_inline)) -> int {
-            return (ocf0 + (gidx >> 1)) * 32 + (gidx & 1) * 16 + (FAST ? row16 : 4 * half);
+            return (ocf0 + (gidx >> 1)) * 32 + (gidx & 1) * 16 + (FAST ? row16 : 4 * half_e);
         };
         auto row_delta = [&](int rr) __attribute__((always_inline)) -> int { return 8 * (rr >> 2) + (rr & 3); };
         // General variant: all 16 channel rows of the group exist (uniform; true for every group when Cout % 16 == 0), so
@@ -637,7 +675,159 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu
             }
         };
 
-        if constexpr (!SK) {
+        // SPIKES: the fast epilogue of 16-bit spikes. The neurons run where their sums are (a lane owns one pixel and 8 channel
+        // rows of a group) and leave one bit per step in a word of two per lane; the words go through the wave's LDS stage, from
+        // which a lane takes 8 neighbouring pixels of a channel row, one step of four, and expands them to a 16-byte store. The
+        // residual travels the other way: 16-byte loads of a group's rows, all steps at once and ahead of the spikes' way out, through
+        // the stage to the lanes. (Sums through the stage step by step, a chain of write, read, neuron and store for each of 16 steps and the
+        // residual waited for in every one, took 16.6 k cycles of a tile's 79 k at 64 -> 64 and 31.8 k with a residual.)
+        constexpr int CH = TT == 2 ? 2 : 4;                          // steps of a word
+        constexpr uint32_t ONE = F16 ? 0x3c00u : 0x3f80u;
+        const uint32_t px_lane = static_cast<uint32_t>(mpi_e) * image_out + static_cast<uint32_t>(mpr_e * g.Wo + mpc_e);   // this lane's pixel, from the tile origin
+        unsigned char* __restrict__ stage_b = reinterpret_cast<unsigned char*>(stage);
+        constexpr int kResPitch = 80;                                // bytes of a row of 32 residual values in the stage
+        // The residual of a group's 16 rows at the steps tc .. tc + CH - 1: lane = (row, run of 8 pixels).
+        auto res_request = [&](int gidx, int tc, cv_u32x4 (&raw)[CH]) __attribute__((always_inline)) {
+            if (!has_residual || !wave_has_work) return;
+            const uint32_t row = static_cast<uint32_t>((ocf0 + (gidx >> 1)) * 32 + (gidx & 1) * 16 + row16) * static_cast<uint32_t>(po);
+            const uint32_t at0 = row + (lo_inside ? px0 : 0u), at4 = row + (hi_inside ? px4 : 0u);   // (a lane outside reads the row's first run)
+#pragma unroll
+            for (int c = 0; c < CH; ++c) {
+                if (TT > 1 || tc + c < g.T) {
+                    const XT* __restrict__ res_t = static_cast<const XT*>(kernarg_table_entry(sizeof(StepPtrs), min(tc + c, g.T - 1))) + tile_off;
+                    const Pack<uint32_t, 2> a = *reinterpret_cast<const Pack<uint32_t, 2>*>(res_t + at0);
+                    const Pack<uint32_t, 2> b = *reinterpret_cast<const Pack<uint32_t, 2>*>(res_t + at4);
+                    raw[c] = cv_u32x4{a.v[0], a.v[1], b.v[0], b.v[1]};
+                }
+            }
+        };
+        // x += the residual of this lane's pixel and 8 rows, through half `buf` of the stage.
+        auto res_add = [&](const cv_u32x4& raw, int buf, float (&x)[8]) __attribute__((always_inline)) {
+            unsigned char* __restrict__ at = stage_b + buf * (16 * kResPitch);
+            __builtin_amdgcn_wave_barrier();
+            *reinterpret_cast<cv_u32x4*>(at + row16 * kResPitch + pcx * 16) = raw;
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int rr = 0; rr < 8; ++rr) {
+                const uint16_t bits = *reinterpret_cast<const uint16_t*>(at + ((rr >> 2) * 8 + half_e * 4 + (rr & 3)) * kResPitch + l32_e * 2);
+                if constexpr (SPIKES) x[rr] += to_float(XT{bits});
+            }
+        };
+        auto spikes_begin = [&](int gidx, float (&bvv)[8], float (&v)[8]) __attribute__((always_inline)) {
+            const int oc = (ocf0 + (gidx >> 1)) * 32 + (gidx & 1) * 16 + 4 * half_e;
+            const cv_f32x4 blo = *reinterpret_cast<const cv_f32x4*>(bias_lds + (oc - (oc_tile << g.wn_log2) * 64));
+            const cv_f32x4 bhi = *reinterpret_cast<const cv_f32x4*>(bias_lds + (oc + 8 - (oc_tile << g.wn_log2) * 64));
+#pragma unroll
+            for (int k = 0; k < 4; ++k) { bvv[k] = blo[k]; bvv[4 + k] = bhi[k]; v[k] = 0.0f; v[4 + k] = 0.0f; }
+            if (v_init != nullptr && m_in) {
+                const float* __restrict__ src = static_cast<const float*>(v_init) + tile_off + static_cast<int64_t>(oc) * po;
+#pragma unroll
+                for (int rr = 0; rr < 8; ++rr) v[rr] = src[static_cast<uint32_t>(row_delta(rr) * po) + px_lane];
+            }
+        };
+        auto spikes_step = [&](int c, const float (&x)[8], float (&v)[8], uint32_t (&word)[2]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int rr = 0; rr < 8; ++rr) {
+                const float h = v[rr] + (x[rr] - v[rr]) * lif.inv_tau;
+                const bool fired = h >= lif.v_threshold;
+                v[rr] = fired ? lif.v_reset : h;
+                word[rr >> 2] |= fired ? (1u << (4 * c + (rr & 3))) : 0u;
+            }
+        };
+        // Stores the spikes of the steps tc .. tc + cnt - 1 of a group from its words: lane = (step, quad, half, run of 8 pixels), 4 channel
+        // rows in turn; of one or two steps the lanes of the absent ones take a part of the rows.
+        auto spikes_store = [&](int gidx, int tc, int cnt, const uint32_t (&word)[2]) __attribute__((always_inline)) {
+            uint16_t* __restrict__ words = reinterpret_cast<uint16_t*>(stage_b);
+            __builtin_amdgcn_wave_barrier();
+            words[lane_e] = static_cast<uint16_t>(word[0]);
+            words[64 + lane_e] = static_cast<uint16_t>(word[1]);
+            __builtin_amdgcn_wave_barrier();
+            const int part = lane_e >> 4, four = (lane_e >> 2) & 3;      // four: (quad, half), a lane's 4 channel rows
+            const cv_u32x4 d = *reinterpret_cast<const cv_u32x4*>(words + (four >> 1) * 64 + (four & 1) * 32 + pcx * 8);
+            __builtin_amdgcn_wave_barrier();
+            const int rows = cnt == 1 ? 1 : (cnt == 2 ? 2 : 4);
+            const int step = cnt == 1 ? 0 : (cnt == 2 ? part >> 1 : part), first = cnt == 1 ? part : (cnt == 2 ? 2 * (part & 1) : 0);
+            if (step >= cnt || okmask == 0u) return;
+            const int64_t oc = (ocf0 + (gidx >> 1)) * 32 + (gidx & 1) * 16 + four * 4;
+            XT* __restrict__ out_t = spikes + (tc + step) * g.spike_step_stride + tile_off + oc * po;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                if (k >= rows) break;
+                cv_u32x4 o;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) o[j] = __umul24((d[j] >> (4 * step + first + k)) & 0x00010001u, ONE);
+                XT* __restrict__ row = out_t + static_cast<uint32_t>((first + k) * po);
+                if (wide) {
+                    *reinterpret_cast<cv_u32x4*>(row + px0) = o;
+                } else {
+                    const Pack<uint32_t, 2> a = {o[0], o[1]}, b = {o[2], o[3]};
+                    if (okmask & 0x0fu) *reinterpret_cast<Pack<uint32_t, 2>*>(row + px0) = a;
+                    if (okmask & 0xf0u) *reinterpret_cast<Pack<uint32_t, 2>*>(row + px4) = b;
+                }
+            }
+        };
+        auto spikes_end = [&](int gidx, const float (&v)[8]) __attribute__((always_inline)) {
+            if (!m_in) return;
+            const int oc = (ocf0 + (gidx >> 1)) * 32 + (gidx & 1) * 16 + 4 * half_e;
+            float* __restrict__ dst = static_cast<float*>(v_out) + tile_off + static_cast<int64_t>(oc) * po;
+#pragma unroll
+            for (int rr = 0; rr < 8; ++rr) dst[static_cast<uint32_t>(row_delta(rr) * po) + px_lane] = v[rr];
+        };
+
+        auto late_loads = [&]() __attribute__((always_inline)) {
+            // The registers of the loads begin here: idle slots would otherwise carry their old contents through the epilogue.
+#pragma unroll
+            for (int s = 0; s < SS; ++s)
+#pragma unroll
+                for (int t = 0; t < TT; ++t)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+#pragma unroll
+                        for (int r = 0; r < RPE; ++r) asm volatile("" : "=v"(pre[s][t][j][r]));
+            if (!next_tile) return;
+            int nih, niw;
+            halo_origin(next_oh0, next_ow0, nih, niw);
+            issue_loads(0, next_img, nih, niw);
+            fetch_bias(next_oc_tile);
+        };
+        if constexpr (SPIKES && !SK) {
+            if (wave_has_work) {
+                cv_u32x4 res[CH] = {};
+                res_request(0, 0, res);
+#pragma unroll
+                for (int gidx = 0; gidx < 4; ++gidx) {
+                    float bvv[8], v[8];
+                    spikes_begin(gidx, bvv, v);
+                    const int steps = TT == 1 ? g.T : min(TT, g.T);
+                    auto some_steps = [&](int tc) __attribute__((always_inline)) {
+                        uint32_t word[2] = {0u, 0u};
+#pragma unroll
+                        for (int c = 0; c < CH; ++c) {
+                            if (tc + c < steps) {
+                                float x[8];
+#pragma unroll
+                                for (int rr = 0; rr < 8; ++rr) x[rr] = acc[TT == 1 ? 0 : c][gidx >> 1][(gidx & 1) * 8 + rr] + bvv[rr];
+                                if (has_residual) res_add(res[c], c & 1, x);
+                                spikes_step(c, x, v, word);
+                            }
+                        }
+                        if (TT == 1 && tc + CH < steps) res_request(gidx, tc + CH, res);
+                        else if (gidx < 3) res_request(gidx + 1, 0, res);
+                        spikes_store(gidx, tc, min(CH, steps - tc), word);
+                    };
+                    if constexpr (TT == 1) {   // a single timestep, or one frame that feeds all of them
+                        for (int tc = 0; tc < steps; tc += CH) some_steps(tc);
+                    } else {
+                        some_steps(0);
+                    }
+                    spikes_end(gidx, v);
+                    __builtin_amdgcn_sched_barrier(0);   // one group at a time: hoisted loads and addresses of the next would be spilled
+                    if (LATE && gidx == 1) late_loads();
+                }
+            } else if constexpr (LATE) {
+                late_loads();
+            }
+        } else if constexpr (!SK) {
             if (wave_has_work) {
 #pragma unroll
                 for (int gidx = 0; gidx < 4; ++gidx) {
@@ -675,10 +865,15 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu
             bool row_ok[2];
             uint32_t row_off[2];
             float bvv[2][8], v[2][8];
+            uint32_t word[2][2] = {{0u, 0u}, {0u, 0u}};
+            cv_u32x4 res[2][CH] = {};
 #pragma unroll
             for (int gidx = 0; gidx < 4; ++gidx) {
                 const int owner = g.wk_log2 == 1 ? (gidx >> 1) : (gidx << (g.wk_log2 - 2));
-                if (owner == wk) {
+                if (SPIKES && owner == wk) {
+                    spikes_begin(gidx, bvv[gidx & 1], v[gidx & 1]);
+                    if constexpr (TT > 1) res_request(gidx, 0, res[gidx & 1]);
+                } else if (owner == wk) {
                     group_row(gidx, row_ok[gidx & 1], row_off[gidx & 1], bvv[gidx & 1]);
                     load_membrane(gidx, row_ok[gidx & 1], row_off[gidx & 1], v[gidx & 1]);
                 }
@@ -708,7 +903,33 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu
                             float xin[8];
 #pragma unroll
                             for (int k = 0; k < 4; ++k) { xin[k] = lo[k]; xin[4 + k] = hi[k]; }
-                            if constexpr (TT == 1) {   // one stage of input feeds all g.T timesteps
+                            if constexpr (SPIKES) {
+                                if (wave_has_work) {
+                                    if constexpr (TT == 1) {
+                                        for (int tc = 0; tc < g.T; tc += CH) {
+                                            cv_u32x4 now[CH] = {};
+                                            res_request(gidx, tc, now);
+                                            uint32_t w[2] = {0u, 0u};
+#pragma unroll
+                                            for (int c = 0; c < CH; ++c) {
+                                                if (tc + c < g.T) {
+                                                    float x[8];
+#pragma unroll
+                                                    for (int rr = 0; rr < 8; ++rr) x[rr] = xin[rr] + bvv[gidx & 1][rr];
+                                                    if (has_residual) res_add(now[c], c & 1, x);
+                                                    spikes_step(c, x, v[gidx & 1], w);
+                                                }
+                                            }
+                                            spikes_store(gidx, tc, min(CH, g.T - tc), w);
+                                        }
+                                    } else {
+#pragma unroll
+                                        for (int rr = 0; rr < 8; ++rr) xin[rr] += bvv[gidx & 1][rr];
+                                        if (has_residual) res_add(res[gidx & 1][t % CH], t & 1, xin);
+                                        spikes_step(t, xin, v[gidx & 1], word[gidx & 1]);
+                                    }
+                                }
+                            } else if constexpr (TT == 1) {   // one stage of input feeds all g.T timesteps
                                 for (int ts = 0; ts < g.T; ++ts)
                                     lif_step_group(ts, gidx, row_ok[gidx & 1], row_off[gidx & 1], bvv[gidx & 1], xin, v[gidx & 1]);
                             } else {
@@ -721,15 +942,17 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
             for (int gidx = 0; gidx < 4; ++gidx) {
                 const int owner = g.wk_log2 == 1 ? (gidx >> 1) : (gidx << (g.wk_log2 - 2));
-                if (owner == wk) store_membrane(gidx, row_ok[gidx & 1], row_off[gidx & 1], v[gidx & 1]);
+                if (SPIKES && owner == wk) {
+                    if (wave_has_work) {
+                        if constexpr (TT > 1) spikes_store(gidx, 0, min(TT, g.T), word[gidx & 1]);
+                        spikes_end(gidx, v[gidx & 1]);
+                    }
+                } else if (owner == wk) {
+                    store_membrane(gidx, row_ok[gidx & 1], row_off[gidx & 1], v[gidx & 1]);
+                }
             }
         }
-        if (SK && next_tile) {
-            int nih, niw;
-            halo_origin(next_oh0, next_ow0, nih, niw);
-            issue_loads(0, next_img, nih, niw);
-            fetch_bias(next_oc_tile);
-        }
+        if constexpr (SK) late_loads();
         work = next_work;
         oc_tile = next_oc_tile;
         img = next_img;
@@ -750,6 +973,10 @@ int launch_conv_mm_tt(const ConvLaunch& L, int load_mode, bool fast) {
     };
     auto pick = [&](auto lm) -> int {
         constexpr int LMV = decltype(lm)::value;
+        // STAGED: sums instead of spikes, and single 16-bit steps, for which the detour through words does not pay (64 -> 64 at 56^2 x 16,
+        // T = 1 22.7 us, 23.2 with it).
+        if (fast && (L.g.analog_out || (sizeof(XT) == 2 && L.g.T == 1)))
+            return split_k ? run(conv_mm_lif_kernel<XT, TT, LMV, true, true, NW, true>) : run(conv_mm_lif_kernel<XT, TT, LMV, true, false, NW, true>);
         if constexpr (NW == 8) {
             if (split_k)
                 return fast ? run(conv_mm_lif_kernel<XT, TT, LMV, true, true, 8>) : run(conv_mm_lif_kernel<XT, TT, LMV, false, true, 8>);
