@@ -1,6 +1,6 @@
 """Dense convolutions of whole tiles with 16-bit spikes on the matrix kernel: spikes leave as bits and the residual arrives through the
 wave's stage. Against the CPU oracle for runs of eight and of four pixels, one to four steps per word, several windows, one frame for all
-steps, shared tiles of waves, several images per tile and kernels of more than 64 pairs of k-slots."""
+steps, shared tiles of waves, several images per tile, waves without channels and kernels of more than 64 pairs of k-slots."""
 import pytest
 import torch
 
@@ -22,6 +22,7 @@ BF16, F16 = torch.bfloat16, torch.float16
     (256, 256, 14, 14, 3, 1, 4, 4, BF16, True, True, False),     # eight waves share a tile, runs of four
     (64, 128, 16, 16, 3, 1, 6, 2, F16, True, False, False),
     (256, 512, 2, 2, 3, 1, 4, 9, BF16, True, True, False),       # several images per tile
+    (128, 192, 12, 12, 3, 1, 6, 15, F16, True, True, False),     # waves share a tile, those of its last 64 channels of 256 have none
     (64, 64, 24, 24, 7, 1, 4, 2, BF16, False, False, False),     # 98 pairs
     (8, 64, 24, 24, 3, 1, 4, 2, F16, True, False, False),        # one channel group: the last slot of nine is empty
 ])

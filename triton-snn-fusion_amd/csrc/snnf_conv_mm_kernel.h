@@ -719,7 +719,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu
             const cv_f32x4 bhi = *reinterpret_cast<const cv_f32x4*>(bias_lds + (oc + 8 - (oc_tile << g.wn_log2) * 64));
 #pragma unroll
             for (int k = 0; k < 4; ++k) { bvv[k] = blo[k]; bvv[4 + k] = bhi[k]; v[k] = 0.0f; v[4 + k] = 0.0f; }
-            if (v_init != nullptr && m_in) {
+            if (v_init != nullptr && m_in && wave_has_work) {
                 const float* __restrict__ src = static_cast<const float*>(v_init) + tile_off + static_cast<int64_t>(oc) * po;
 #pragma unroll
                 for (int rr = 0; rr < 8; ++rr) v[rr] = src[static_cast<uint32_t>(row_delta(rr) * po) + px_lane];
