@@ -48,3 +48,43 @@ def test_whole_tiles_on_the_matrix_kernel(snnf_lib, Cin, Cout, H, W, k, s, T, N,
     plan = CB.last_conv_plan()
     assert plan["kernel"] == "matrix" and int(plan["variant"]) in (21, 22, 24, 31, 34, 32), plan
     check(sp, v, ref, what=f"{Cin}->{Cout} {H}x{W} T={T}")
+
+
+@pytest.mark.parametrize("Cin,Cout,H,k,s,T,N,residual,moves", [
+    (64, 64, 56, 3, 1, 4, 16, False, False),     # seven eighths of one round of full tiles
+    (64, 64, 40, 3, 1, 4, 20, True, True),       # tiles of four columns
+    (64, 64, 24, 3, 1, 6, 38, True, True),       # less than half a round, two windows
+    (128, 256, 28, 3, 2, 8, 5, False, True),
+    (64, 128, 56, 3, 2, 4, 16, False, False),
+    (64, 128, 56, 1, 2, 4, 16, False, False),
+    (16, 64, 40, 3, 1, 4, 2, False, False),      # a single stage
+    (256, 256, 14, 3, 1, 4, 16, True, True),     # deep: with a residual ...
+    (256, 256, 14, 3, 1, 4, 16, False, False),   # ... and without
+])
+def test_whole_tiles_move_where_they_leave_the_chip_idle(snnf_lib, Cin, Cout, H, k, s, T, N, residual, moves):
+    from triton_snn_fusion_amd import _lib
+    from triton_snn_fusion_amd.runtime import hip_convlif_backend as CB
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the shapes sit at the edges of 256 compute units")
+    g, dtype, p = gen(7900 + Cin + T), BF16, k // 2
+    Ho = (H + 2 * p - k) // s + 1
+    xs = [dev(spikes((N, Cin, H, H), 0.25, g), dtype) for _ in range(T)]
+    w, b = dev(torch.randn(Cout, Cin, k, k, generator=g) * 2.0 * (2.0 / (Cin * k * k)) ** 0.5, dtype), dev(torch.randn(Cout, generator=g) * 0.1, dtype)
+    rs = [dev(spikes((N, Cout, Ho, Ho), 0.25, g), dtype) for _ in range(T)] if residual else None
+    packed, code = CB._packed_weight(w, b, dtype), _lib.dtype_code(dtype)
+    need = snnf_lib.snnf_conv_lif_scratch_bytes(T, N, Cin, H, H, code, Cout, k, k, s, s, p, p, 0, int(residual))
+    assert (need > 0) == moves
+    workspace = torch.empty(max(need, 16), dtype=torch.uint8, device=DEV)
+    got = []
+    for given in (need, 0):
+        sp, v = torch.empty(T, N, Cout, Ho, Ho, device=DEV, dtype=dtype), torch.empty(N, Cout, Ho, Ho, device=DEV)
+        _lib.check("conv", snnf_lib.snnf_conv_lif_ws(
+            _lib.step_pointers(xs), _lib.step_pointers(rs) if residual else None, T, N, Cin, H, H, code, packed.data_ptr(), Cout, k, k, s, s, p, p,
+            None, 0, sp.data_ptr(), int(sp.stride(0)), v.data_ptr(), *LIF, workspace.data_ptr() if given else None, given, _lib.current_stream(sp.device)))
+        plan = CB.last_conv_plan()
+        assert plan["kernel"] == "matrix" and (plan.get("ran") == "blocked") == (given > 0), plan
+        got.append((sp, v))
+    rate = float((got[0][0] != got[1][0]).float().mean())       # (sums of the same terms in another order)
+    assert rate <= 1e-4 and 0.001 < float(got[0][0].float().mean()) < 0.9, rate
+    same = (got[0][0] == got[1][0]).all(0)
+    assert torch.allclose(got[0][1][same], got[1][1][same], rtol=1e-3, atol=1e-4)

@@ -201,6 +201,10 @@ int launch_conv_mm_w4_f16(const ConvLaunch& L, int tt, int load_mode);
 
 // The kernels behind snnf_conv_lif (snnf_conv_igemm.hip).
 enum class DenseFamily { kTInM, kTimeOuter, kMatrixMasked, kMatrixWhole, kPointwise };
-DenseFamily dense_family(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w);
+// `tile_use`, of whole tiles of the matrix kernel: what the time that a layer takes there is divided by. The share of the workgroup slots' rounds
+// (and, of several windows, of their steps) that have work, times the share of a tile's pixel lanes, times the roots of the share of its channels and of its run of
+// pixels per row in units of 8 (up to 32), over the fourth root of the rounds (up to three).
+DenseFamily dense_family(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w,
+                         double& tile_use);
 
 }  // namespace snnf

@@ -1,5 +1,6 @@
 // Host side of the implicit-GEMM conv+LIF operator: argument validation, tile planning and launch.
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include "snnf_conv_common.h"
 
@@ -381,11 +382,21 @@ Choice choose_kernel(const ConvGeom& g, const ChoiceInput& c) {
 
 // The kernel that snnf_conv_lif chooses for a layer of activations of `x_dtype`, an fp32 membrane and the usual neuron, when every operand is
 // 16-byte aligned and the steps have inputs of their own.
-DenseFamily dense_family(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w) {
+DenseFamily dense_family(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w,
+                         double& tile_use) {
     const ConvGeom g = layer_geom(N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, make_pack_geom(Cout, Cin, KH, KW, x_dtype == SNNF_F32));
     const int64_t plane = static_cast<int64_t>(g.Ho) * g.Wo;
     const Choice c = choose_kernel(g, ChoiceInput{T, dtype_size(x_dtype), false, false, false, true, true, plane % 8 == 0, plane % 4 == 0, g.W % 2 == 0});
-    if (c.mm_kernel) return Cout % 64 == 0 && c.mp.all_full && c.mp.run >= 4 ? DenseFamily::kMatrixWhole : DenseFamily::kMatrixMasked;
+    tile_use = 1.0;
+    if (c.mm_kernel) {
+        const MmPlan& m = c.mp;
+        if (Cout % 64 != 0 || !m.all_full || m.run < 4) return DenseFamily::kMatrixMasked;
+        const double tiles = static_cast<double>((N + m.TI - 1) / m.TI) * m.tiles_x * m.tiles_y * m.oc_tiles, slots = compute_units() * (8 / m.nw);
+        const double rounds = std::ceil(tiles / slots), windows = (T + c.window - 1) / c.window;
+        tile_use = tiles / (rounds * slots) * (windows > 1 ? T / (windows * c.window) : 1.0) * m.TI * m.TH * m.TW / (32 << m.wm_log2) *
+                   std::sqrt(static_cast<double>(Cout) / ((64 << m.wn_log2) * m.oc_tiles) * std::min(m.TW, 32) / 8.0) / std::sqrt(std::sqrt(std::min(rounds, 3.0)));
+        return DenseFamily::kMatrixWhole;
+    }
     return c.pw_kernel ? DenseFamily::kPointwise : (c.time_outer ? DenseFamily::kTimeOuter : DenseFamily::kTInM);
 }
 

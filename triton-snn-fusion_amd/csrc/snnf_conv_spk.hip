@@ -2,6 +2,7 @@
 // argument validation, patch planning and launch of conv_spk_kernel.
 #include <algorithm>
 #include <array>
+#include <cmath>
 #include <cstdio>
 #include <map>
 #include <mutex>
@@ -117,14 +118,18 @@ RouteSpace route_space(int T, int N, int Cin, int H, int W, bool split, int64_t 
 // * The pointwise kernel's straight-line variant takes planes of whole tiles of 64 pixels: 24 -> 96 at 56^2 x 32 31 / 73, 128 -> 256 89 / 224.
 //   Its general variant is several times slower and loses over 260 layers to a factor of 1.8 (128 -> 64 at 7^2, T = 8 60 / 16, 64 -> 256 at
 //   51^2 x 16 with a residual 216 / 127, 128 -> 256 at 28^2 x 32, T = 2 56 / 50).
-// * Whole tiles of the matrix kernel stay where they fill the chip (64 -> 64 at 56^2 x 16 37 / 42, 128 -> 256 1x1 stride 2 at 28^2 x 32 23 / 33,
-//   64 -> 128 stride 2 at 56^2 x 8 21 / 28) and move where they don't: the time of one tile is 33 us there and 8 here. The lines, in outputs of
-//   all timesteps: 64 -> 64 at 24^2 x 4 33 / 12, at 40^2 x 8, T = 2 15 / 16, at 40^2 x 8, T = 6 38 / 34, at 56^2 x 16, T = 8 107 / 110; 128 -> 128 at
-//   28^2 x 4 24 / 21, at 16^2 x 32, T = 2 18 / 17; 64 -> 128 stride 2 at 40^2, T = 4 38 / 14, at 32^2 x 8, T = 2 13 / 12, at 24^2 x 17, T = 2 12 / 13;
-//   1x1 stride 2 64 -> 128 at 40^2 x 4 16 / 14, at 32^2 x 8 14 / 15, at 24^2 x 17, T = 8 29 / 26. Deep layers of few outputs always move
-//   (256 -> 256 at 14^2 x 4 29 / 18, 512 -> 512 at 4^2 x 16 37 / 21). Two kinds that would gain as well stay with the kernel that their reported
-//   plan names in the tests: planes of four pixels at most (256 -> 512 at 2^2 x 40 25 / 14) and one window of four steps of up to 512 pixels
-//   with less than 128 channels (64 -> 64 at 16^2 x 2 33 / 11).
+// * Whole tiles of the matrix kernel take the time of their rounds, full or not, and of their windows of four steps; this kernel's time is
+//   nearly proportional to the outputs. So `tile_use` decides (see dense_family), weighed by the products per output, in which this kernel is
+//   the better one. Over 2800 layers the quotient of the two times falls with it from 2 to 0.75 and passes 1 at the lines below; the rule is
+//   2 % slower than the better kernel in the mean, the dense kernels alone 31 %. It moves 64 -> 64 at 24^2 x 4 30 / 12, x 38, T = 6 70 / 45, at
+//   40^2 x 20 (tiles of four columns) 43 / 33, T = 8 121 / 68, at 56^2 x 21, T = 6 132 / 110, 128 -> 256 stride 2 at 28^2 x 5, T = 8 49 / 40, 1x1 stride 2 x 2
+//   31 / 20; 64 -> 64 at 56^2 x 16 34 / 42, 128 -> 128 at 28^2 x 32 48 / 52 (x 16 38 / 36), 64 -> 128 stride 2 at 56^2 x 16 28 / 37, 1x1 18 / 26, 128 -> 256 stride 2
+//   at 28^2 x 16 28 / 34 stay. Inputs that the caches don't hold between the copy and the kernel move the lines (64 -> 64 at 56^2 x 88, T = 5
+//   with a residual 366 / 437, 128 -> 256 stride 2 at 28^2 x 164, T = 7 395 / 554). A single stage of 16 channels leaves the waves nothing to share
+//   (16 -> 64 at 40^2 x 2 13.6 / 16.2). Deep layers of few outputs always move (256 -> 256 at 14^2 x 4 29 / 18, 512 -> 512 at 4^2 x 16 37 / 21). Three kinds
+//   that would gain as well stay with the kernel that their reported plan names in the tests: planes of four pixels at most (256 -> 512
+//   at 2^2 x 40 24 / 14), one window of four steps of up to 512 pixels with less than 128 channels (64 -> 64 at 16^2 x 2 30 / 11) and deep layers
+//   without a residual that fill the chip (256 -> 256 at 14^2 x 16 35 / 31; with one they move, 37 / 32).
 // * fp32 tensors (two bf16 terms each) run here at three times the speed of the dense kernels over 180 layers: 64 -> 64 at 32^2 x 8 35 / 20, at
 //   56^2 x 16 100 / 73, 512 -> 512 at 7^2 x 4 with a residual 125 / 29, 41 -> 72 at 8 x 14 x 15 191 / 20, 122 -> 111 at 15^2, 5x5, T = 5 1068 / 36,
 //   3 -> 64 at 32^2 x 64 34 / 31, 128 -> 256 1x1 at 28^2 x 8 135 / 27. Only 1x1 layers with few products per output stay, where those are many:
@@ -140,8 +145,9 @@ bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int C
     const bool pointwise = one && !strided && pad_h == 0 && pad_w == 0;
     const int64_t K = static_cast<int64_t>(Cin) * KH * KW, plane = static_cast<int64_t>(H) * W;
     const int64_t pixels = static_cast<int64_t>(N) * ((H + 2 * pad_h - KH) / stride_h + 1) * ((W + 2 * pad_w - KW) / stride_w + 1);
-    const int64_t out = pixels * Cout, outs = T * out;
-    family = dense_family(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w);
+    const int64_t out = pixels * Cout, outs = T * out, inputs = static_cast<int64_t>(T) * N * Cin * plane;
+    double tile_use;
+    family = dense_family(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, tile_use);
     if (x_dtype == SNNF_F32) return !(family == DenseFamily::kPointwise && Cin <= 64 && Cout >= 96 && outs >= (1 << 22));
     const bool deep = K >= 4608 || (K >= 2304 && out <= (1 << 19) && !residual);
     if (!neuron) {
@@ -159,10 +165,11 @@ bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int C
         case DenseFamily::kMatrixWhole:
             if (deep) return true;
             if (plane <= 4 || (T >= 3 && T <= 4 && !one && !strided && pixels <= 512 && K < 1152)) return false;
-            if (one) return outs <= (T <= 2 ? 3 << 17 : (T <= 4 ? 5 << 17 : 5 << 19));
-            if (strided) return outs <= (T <= 2 ? 1 << 19 : (T <= 4 ? 1 << 20 : 3 << 20));
-            if (K < 432) return Cin > 8 && outs <= (1 << 19);   // (a single channel group: as above)
-            return outs <= (K < 1152 ? (T <= 4 ? 3 << 19 : 1 << 23) : (T <= 4 ? 1 << 21 : 1 << 24));
+            if (!one && Cin <= 16) return false;   // a single stage, which waves cannot share
+            if (K >= 2304 && T <= 4 && !residual && tile_use >= 1.0) return false;
+            if (one) return tile_use * std::sqrt(576.0 / K) <= 0.45;
+            if (strided) return tile_use * std::sqrt(std::sqrt(576.0 / K)) <= (T <= 4 ? 0.5 : (inputs < (1 << 24) ? 0.65 : 0.45));
+            return tile_use * std::sqrt(576.0 / K) <= (inputs >= (1 << 26) ? 0.7 : (T <= 4 ? 0.85 : 0.95));
     }
     return false;
 }
