@@ -660,13 +660,16 @@ bool conv_call(const Call& c, Attempt& key, Op op, Pair* out) {
     } else {
         const Tensor packed = packed_weight(w, b, x.scalar_type());
         if (wide) bytes = scratch_bytes(wm.code());
-        Tensor workspace;
-        if (bytes > 0) workspace = empty({static_cast<int64_t>(bytes)}, at::kByte, x);
+        c10::DataPtr workspace;            // (a tensor around it costs another microsecond)
+        if (bytes > 0) {
+            const c10::DeviceGuard guard(x.device());
+            workspace = c10::GetAllocator(c10::kCUDA)->allocate(bytes);
+        }
         status = snnf_conv_lif_ws(steps, residuals, static_cast<int>(T), N, cin, H, W, code_of(x.scalar_type()), packed.data_ptr(),
                                   static_cast<int>(shape[1]), static_cast<int>(kh), static_cast<int>(kw), static_cast<int>(sh), static_cast<int>(sw),
                                   static_cast<int>(ph), static_cast<int>(pw), wm.from, wm.code(), spikes.data_ptr(), step, wm.work.data_ptr(),
                                   static_cast<float>(lif.v_threshold), static_cast<float>(lif.v_reset), static_cast<float>(lif.tau),
-                                  bytes > 0 ? workspace.data_ptr() : nullptr, bytes, stream);
+                                  workspace.get(), bytes, stream);
     }
     if (status != 0) return false;
     wm.finish();

@@ -4,7 +4,9 @@
 #include <array>
 #include <cmath>
 #include <cstdio>
+#include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
 
 #include "snnf_conv_spk_kernel.h"
@@ -364,12 +366,30 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
     return SNNF_OK;
 }
 
+const char* family_name(DenseFamily f) {
+    return f == DenseFamily::kTInM ? "t_in_m" : (f == DenseFamily::kTimeOuter ? "time_outer" : (f == DenseFamily::kPointwise ? "pointwise" : "matrix"));
+}
+
+void plan_text(char* text, const BlockedPlan& p, const char* kernel, int epilogue, int window, bool from_dense) {
+    const SpkGeom& g = p.g;
+    snprintf(text, 256,
+             "kernel=%s variant=%d window=%d launches=%d tile=%dx%dx%d halo=%dx%d waves=8x1x%d oc_tiles=%d oc_tile=%d px_tiles=%d "
+             "stage_chunks=%d run=0 lds=%zu grid=%d tuned=%d shortcut_stages=%d%s",
+             kernel, (p.wk_log2 > 0 ? 50 : 40) + p.tt + epilogue, window, from_dense ? 2 : 1, g.PI, g.PR, g.PC, g.RR, g.RC, 1 << p.wk_log2, p.oc_tiles,
+             g.narrow ? 32 : 64, g.n_patches, g.G, p.lds_bytes, p.grid, (p.tuned_patch ? 1 : 0) + (p.tuned_split ? 2 : 0), g.sc_stages,
+             from_dense ? " route=c8 ran=blocked" : "");
+}
+
 // Whether a layer takes the blocked route: where the rule sends it there and the kernel then runs it. A layer that the planner refuses
 // (offsets, a kernel of too many steps, no patch that fits) gets no scratch memory asked for. Without a neuron the dense route has the
 // matrix kernel only; what it refuses stays refused. The answer depends on the layer and the table of tuned plans alone and is
-// kept per layer: it is asked for twice per call.
+// kept per layer with the plan and its text (made anew in each call they took 0.6 of its 11.5 us; it asks twice).
 using RouteKey = std::array<int, 15>;
-struct Route { bool taken; DenseFamily family; int windows; };
+struct KeptPlan {
+    BlockedPlan plan;
+    char text[2][256];                                 // with the general and with the dense epilogue
+};
+struct Route { bool taken; DenseFamily family; std::shared_ptr<const KeptPlan> kept; };
 std::mutex routes_mutex;
 std::map<RouteKey, Route>& routes() {
     static std::map<RouteKey, Route> known;
@@ -379,7 +399,7 @@ constexpr size_t kMaxRoutes = 4096;
 
 Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w,
                     int v_dtype, bool residual, bool neuron) {
-    if (!valid_dtype(x_dtype) || (v_dtype != SNNF_F32 && v_dtype != x_dtype)) return {false, DenseFamily::kTInM, 0};
+    if (!valid_dtype(x_dtype) || (v_dtype != SNNF_F32 && v_dtype != x_dtype)) return {false, DenseFamily::kTInM, nullptr};
     const bool split = x_dtype == SNNF_F32;
     const RouteKey key = {T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, residual ? 1 : 0, neuron ? 1 : 0, split ? 1 : 0};
     {
@@ -387,14 +407,18 @@ Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, 
         const auto it = routes().find(key);
         if (it != routes().end()) return it->second;
     }
-    Route route = {false, DenseFamily::kTInM, 0};
+    Route route = {false, DenseFamily::kTInM, nullptr};
     route.taken = takes_blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residual, neuron, route.family) &&
                   (neuron || (!split && (route.family == DenseFamily::kMatrixMasked || route.family == DenseFamily::kMatrixWhole)));
     if (route.taken) {
-        BlockedPlan plan;
+        const auto kept = std::make_shared<KeptPlan>();
+        BlockedPlan& plan = kept->plan;
         route.taken = plan_blocked("snnf_conv_lif_workspace_bytes", BlockedCall{T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, SNNF_LAYOUT_C8,
                                    residual ? SNNF_LAYOUT_NCHW : -1, SNNF_LAYOUT_NCHW, 0, false, neuron, false, neuron, false, nullptr, split}, plan) == SNNF_OK;
-        route.windows = plan.windows;
+        if (route.taken) {
+            for (int dense_epi = 0; dense_epi < 2; ++dense_epi) plan_text(kept->text[dense_epi], plan, family_name(route.family), dense_epi ? 40 : 0, plan.tt, true);
+            route.kept = kept;
+        }
     }
     std::lock_guard<std::mutex> lock(routes_mutex);
     if (routes().size() >= kMaxRoutes) routes().clear();
@@ -404,20 +428,17 @@ Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, 
 
 // fp32 elements that pass from window to window beside a 16-bit membrane.
 int64_t carried_membrane(const Route& r, int v_dtype, int N, int H, int W, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w) {
-    if (v_dtype == SNNF_F32 || r.windows <= 1) return 0;
+    if (v_dtype == SNNF_F32 || r.kept->plan.windows <= 1) return 0;
     return static_cast<int64_t>(N) * Cout * ((H + 2 * pad_h - KH) / stride_h + 1) * ((W + 2 * pad_w - KW) / stride_w + 1);
 }
 
 // A call on dense tensors that runs here: its inputs, which are brought into C8 first, and the kernel family of the dense route.
 struct DenseRoute {
     const void* const* xs;
-    DenseFamily family;
+    const KeptPlan* kept;
     RouteSpace space;
     int v_dtype;
 };
-const char* family_name(DenseFamily f) {
-    return f == DenseFamily::kTInM ? "t_in_m" : (f == DenseFamily::kTimeOuter ? "time_outer" : (f == DenseFamily::kPointwise ? "pointwise" : "matrix"));
-}
 
 }  // namespace
 
@@ -530,7 +551,7 @@ int run_blocked_route(const void* const* xs, const void* const* residuals, int T
         inner[t] = static_cast<const char*>(workspace) + t * space.step;
     }
     if (shared) return SNNF_ERR_UNSUPPORTED;       // one frame for all timesteps is convolved once on the dense kernels too
-    const DenseRoute route = {xs, taken.family, space, v_dtype};
+    const DenseRoute route = {xs, taken.kept.get(), space, v_dtype};
     return conv_lif_blocked_impl(neuron ? "snnf_conv_lif" : "snnf_conv_bias", inner, SNNF_LAYOUT_C8, residuals, SNNF_LAYOUT_NCHW, T, N, Cin, H, W, x_dtype,
                                  packed_weight, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_init, out, SNNF_LAYOUT_NCHW, out_step_stride * dtype_size(x_dtype), v_out,
                                  neuron, v_threshold, v_reset, tau, stream, nullptr, false, &route);
@@ -621,11 +642,14 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
             if (sc->xs[t] == nullptr) return fail(SNNF_ERR_INVALID_ARGUMENT, "%s: shortcut_xs[%d] is null", who, t);
     }
 
-    BlockedPlan p;
-    if (const int rc = plan_blocked(who, BlockedCall{T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, x_layout,
-                                                     residuals != nullptr ? res_layout : -1, out_layout, out_step_stride, shared, neuron != 0,
-                                                     v_init != nullptr, v_out != nullptr, pool2, sc, split}, p); rc != SNNF_OK)
-        return rc;
+    BlockedPlan made;
+    if (dense == nullptr) {
+        if (const int rc = plan_blocked(who, BlockedCall{T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, x_layout,
+                                                         residuals != nullptr ? res_layout : -1, out_layout, out_step_stride, shared, neuron != 0,
+                                                         v_init != nullptr, v_out != nullptr, pool2, sc, split}, made); rc != SNNF_OK)
+            return rc;
+    }
+    const BlockedPlan& p = dense != nullptr ? dense->kept->plan : made;
     const SpkGeom& g = p.g;
 
     SpkLaunch L = {};
@@ -639,6 +663,7 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
         L.bias2 = reinterpret_cast<const float*>(L.wpacked2 + packed_weight_elems(p.pg2));
     }
     L.g = g;
+    L.g.out_step_stride = out_step_stride;
     L.wpacked = static_cast<const uint16_t*>(packed_weight);
     L.bias = reinterpret_cast<const float*>(L.wpacked + packed_weight_elems(p.pg));
     L.v_init = neuron ? v_init : nullptr;
@@ -660,11 +685,8 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     // Dense tensors around the neuron: no range limit on the threshold, any reset potential, initial membrane, windows and channels.
     const bool dense_epi = neuron && x_layout == SNNF_LAYOUT_C8 && out_layout == SNNF_LAYOUT_NCHW && (residuals == nullptr || res_layout == SNNF_LAYOUT_NCHW) &&
                            L.lif.charge_mode == CHARGE_SCALE && L.lif.inv_tau == 0.5f && !L.lif.soft_reset && L.v_out != nullptr && !shared;
-    snprintf(snnf::conv_plan_buffer(), 256,
-             "kernel=%s variant=%d window=%d launches=%d tile=%dx%dx%d halo=%dx%d waves=8x1x%d oc_tiles=%d oc_tile=%d px_tiles=%d "
-             "stage_chunks=%d run=0 lds=%zu grid=%d tuned=%d shortcut_stages=%d%s",
-             dense != nullptr ? family_name(dense->family) : "blocked", (p.wk_log2 > 0 ? 50 : 40) + p.tt + (fast_epi ? 20 : (dense_epi ? 40 : 0)), shared ? T : p.tt, dense != nullptr ? 2 : 1, g.PI, g.PR, g.PC, g.RR, g.RC, 1 << p.wk_log2, p.oc_tiles, g.narrow ? 32 : 64, g.n_patches, g.G,
-             L.lds_bytes, p.grid, (p.tuned_patch ? 1 : 0) + (p.tuned_split ? 2 : 0), g.sc_stages, dense != nullptr ? " route=c8 ran=blocked" : "");
+    if (dense != nullptr) memcpy(snnf::conv_plan_buffer(), dense->kept->text[dense_epi ? 1 : 0], 256);
+    else plan_text(snnf::conv_plan_buffer(), p, "blocked", fast_epi ? 20 : (dense_epi ? 40 : 0), shared ? T : p.tt, false);
     L.fast_epilogue = fast_epi;
     L.multi_window = p.windows > 1;
     L.dense_epilogue = dense_epi;
