@@ -334,9 +334,11 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
         const uint32_t lane_b = lane_in_patch ? static_cast<uint32_t>(((pi * g.RR + prow * g.sh) * g.RC + pcol * g.sw) * 16) : 0u;
 
         const int ocf0 = oc_tile * NF;
-        // With K split over two waves the second one computes the tile's two 32-channel fragments in swapped places: each wave
-        // then finishes the fragment in its accumulators' first half (fragment wk) and hands over the second half.
-        const int swap_f = (SK && !NARROW && WK == 2) ? wk : 0;
+        // With K split over waves, every wave finishes a part of the tile's eight quads, which its accumulators hold in the same registers
+        // whatever the wave: the upper half of the waves computes the two 32-channel fragments in swapped places, and the lanes
+        // read the weight rows of a fragment with the quads exchanged (quad q of the accumulators is quad q ^ quad_x of the fragment).
+        const int swap_f = SK && !NARROW ? wk >> (g.wk_log2 - 1) : 0;
+        const int quad_x = SK && !NARROW ? (WK == 8 ? wk & 3 : (WK == 4 ? (wk & 1) * 2 : 0)) : 0;
         const int64_t w_frag0 = min(ocf0 + swap_f, g.nocf - 1);
         const int64_t w_frag1 = min(ocf0 + 1 - swap_f, g.nocf - 1);
 
@@ -569,7 +571,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                 else __builtin_amdgcn_s_setprio(1);
             }
             if (have) {
-                const uint32_t lane16 = static_cast<uint32_t>(lane) * 16u;
+                const uint32_t lane16 = static_cast<uint32_t>(lane ^ (quad_x * 8)) * 16u;
                 const unsigned char* __restrict__ bl = wlds + lane_b;
                 for (int stage = s_first; stage < nstages_all; stage += s_step) {
                     const bool second = SC && stage >= g.nstages;     // a stage of the shortcut
@@ -1312,40 +1314,59 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             } else {
                 // Split K: the WK waves of a tile add their partial sums through LDS (the staging regions are dead by then).
                 float* __restrict__ part = reinterpret_cast<float*>(lds + kSpkHeaderBytes);      // [wave][e 0..3][tw][lane][4]
-#define SNNF_SPK_PARK_QUAD(E, F)                                                                                                 \
+                // Quad Q of fragment F goes to place P of slot S (a slot per wave).
+#define SNNF_SPK_PARK_QUAD(S, P, F, Q)                                                                                           \
     _Pragma("unroll") for (int tw = 0; tw < TT; ++tw) {                                                                          \
-        const sk_f32x4 four = {acc[tw][(F) % NF][4 * (E)], acc[tw][(F) % NF][4 * (E) + 1], acc[tw][(F) % NF][4 * (E) + 2], acc[tw][(F) % NF][4 * (E) + 3]};  \
-        *reinterpret_cast<sk_f32x4*>(part + (((wave * 4 + (E)) * TT + tw) * 64 + lane) * 4) = four;                             \
+        const sk_f32x4 four = {acc[tw][(F) % NF][4 * (Q)], acc[tw][(F) % NF][4 * (Q) + 1], acc[tw][(F) % NF][4 * (Q) + 2], acc[tw][(F) % NF][4 * (Q) + 3]};  \
+        *reinterpret_cast<sk_f32x4*>(part + ((((S) * 4 + (P)) * TT + tw) * 64 + lane) * 4) = four;                              \
     }
-                if (!NARROW && WK == 2) {
-                    // Two waves per tile: wave wk finishes the four quads of fragment wk, which sit in the first half of its
-                    // accumulators (the second wave computes the fragments in swapped places). It hands its sums of the other
-                    // fragment to its partner and adds the partner's sums to its own, which never leave their registers: one exchange.
+                // The sums at place P of slot S are added to quad Q of the first fragment.
+#define SNNF_SPK_ADD_QUAD(S, P, Q)                                                                                               \
+    _Pragma("unroll") for (int tw = 0; tw < TT; ++tw) {                                                                          \
+        const sk_f32x4 four = *reinterpret_cast<const sk_f32x4*>(part + ((((S) * 4 + (P)) * TT + tw) * 64 + lane_x) * 4);        \
+        _Pragma("unroll") for (int k = 0; k < 4; ++k) acc[tw][0][4 * (Q) + k] += four[k];                                        \
+    }
+                if constexpr (!NARROW) {
+                    // Halves are exchanged until every wave owns 8 / WK quads: first the fragment that a wave does not finish, then two
+                    // quads of its own, then one. All waves add and finish at the same time; a slot that a wave has read takes what it
+                    // gives away next. (Quads parked by all waves and summed by one each, in two rounds of which half of eight waves
+                    // took no part, took 23.4 us at 512 -> 512, 7^2 x 16 against 22.4, 21.8 against 21.2 at 256 -> 256, 14^2 x 16, and in two windows 25.7
+                    // against 22.3 at 128 -> 256 stride 2, 40^2 x 3, T = 8; 1.04 over 60 such layers.)
                     __syncthreads();   // every wave is done with its staging region
-                    SNNF_SPK_PARK_QUAD(0, 1) SNNF_SPK_PARK_QUAD(1, 1) SNNF_SPK_PARK_QUAD(2, 1) SNNF_SPK_PARK_QUAD(3, 1)
+                    SNNF_SPK_PARK_QUAD(wave, 0, 1, 0) SNNF_SPK_PARK_QUAD(wave, 1, 1, 1) SNNF_SPK_PARK_QUAD(wave, 2, 1, 2) SNNF_SPK_PARK_QUAD(wave, 3, 1, 3)
+                    const int jq = oc_e * TG + 4 * swap_f;
                     uint32_t rb[TT];
 #pragma unroll
                     for (int tw = 0; tw < TT; ++tw) rb[tw] = 0u;
                     if constexpr (FAST) {   // the residual bytes of the first quad travel while the workgroup meets
                         if (g.res_layout >= 0 && TT > 1) {
 #pragma unroll
-                            for (int tw = 0; tw < TT; ++tw) rb[tw] = fast_res(tb + min(tw, t_count - 1), oc_e * TG + 4 * wk);
+                            for (int tw = 0; tw < TT; ++tw) rb[tw] = fast_res(tb + min(tw, t_count - 1), jq + quad_x);
                         }
                     }
                     float v0[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-                    if constexpr (FAST) fast_v0(oc_e * TG + 4 * wk, v0);
+                    if constexpr (FAST) fast_v0(jq + quad_x, v0);
                     DenseIn in = {};
-                    if constexpr (DENSE) dense_request(oc_e * TG + 4 * wk, in);
+                    if constexpr (DENSE) dense_request(jq + quad_x, in);
                     __syncthreads();
-                    const int partner = wave ^ 1;
                     int lane_x = lane;                   // opaque: the addresses below are computed here, not ahead of the matrix loop
                     asm volatile("" : "+v"(lane_x));
-                    for (int e = 0; e < 4; ++e) {
-                        const int j8 = oc_e * TG + 4 * wk + e;
-                        sk_f32x4 theirs[TT];
-#pragma unroll
-                        for (int tw = 0; tw < TT; ++tw)
-                            theirs[tw] = *reinterpret_cast<const sk_f32x4*>(part + (((partner * 4 + e) * TT + tw) * 64 + lane_x) * 4);
+                    const int across = wave ^ (WK >> 1);
+                    SNNF_SPK_ADD_QUAD(across, 0, 0) SNNF_SPK_ADD_QUAD(across, 1, 1) SNNF_SPK_ADD_QUAD(across, 2, 2) SNNF_SPK_ADD_QUAD(across, 3, 3)
+                    if (WK > 2) {
+                        const int from = across ^ (WK >> 2);
+                        SNNF_SPK_PARK_QUAD(across, 2, 0, 2) SNNF_SPK_PARK_QUAD(across, 3, 0, 3)
+                        __syncthreads();
+                        SNNF_SPK_ADD_QUAD(from, 2, 0) SNNF_SPK_ADD_QUAD(from, 3, 1)
+                        if (WK > 4) {
+                            SNNF_SPK_PARK_QUAD(from, 2, 0, 1)
+                            __syncthreads();
+                            SNNF_SPK_ADD_QUAD(from ^ 1, 2, 0)
+                        }
+                    }
+                    const int quads = 8 >> g.wk_log2;
+                    for (int e = 0; e < quads; ++e) {
+                        const int j8 = jq + (e ^ quad_x);
                         float xq[TT][4];
 #define SNNF_SPK_COPY_QUAD(F, Q)                                          \
     _Pragma("unroll") for (int tw = 0; tw < TT; ++tw)                     \
@@ -1357,39 +1378,29 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                             default: SNNF_SPK_COPY_QUAD(0, 3); break;
                         }
 #undef SNNF_SPK_COPY_QUAD
-#pragma unroll
-                        for (int tw = 0; tw < TT; ++tw)
-#pragma unroll
-                            for (int k = 0; k < 4; ++k) xq[tw][k] += theirs[tw][k];   // a sum of two terms: the same in either order
+                        const int j8_next = jq + ((e + 1) ^ quad_x);
                         if constexpr (FAST) {
                             if (e != 0 && g.res_layout >= 0 && TT > 1) {
 #pragma unroll
                                 for (int tw = 0; tw < TT; ++tw) rb[tw] = fast_res(tb + min(tw, t_count - 1), j8);
                             }
                             const float start[4] = {v0[0], v0[1], v0[2], v0[3]};
-                            if (e != 3) fast_v0(j8 + 1, v0);
+                            if (e + 1 < quads) fast_v0(j8_next, v0);
                             fast_quad(j8, xq, rb, g.res_layout >= 0, start);
                         } else if constexpr (DENSE) {
                             const DenseIn now = in;
-                            if (e != 3) dense_request(j8 + 1, in);
+                            if (e + 1 < quads) dense_request(j8_next, in);
                             dense_quad(j8, xq, now);
                         } else {
                             general_quad(j8, xq);
                         }
                     }
-                } else
-                // More waves per tile: four quads per round for all TT timesteps; quad 4 r + e of round r is finished by wave
-                // (4 r + e) mod WK of the tile, which adds the WK partial sums in a fixed order and then runs that quad's timesteps
-                // like the unsplit kernel.
-                for (int r = 0; r < NF; ++r) {
-                    __syncthreads();   // the previous round's sums are consumed (first round: every wave is done with its staging region)
-                    if (r == 0) {
-                        SNNF_SPK_PARK_QUAD(0, 0) SNNF_SPK_PARK_QUAD(1, 0) SNNF_SPK_PARK_QUAD(2, 0) SNNF_SPK_PARK_QUAD(3, 0)
-                    } else {
-                        SNNF_SPK_PARK_QUAD(0, 1) SNNF_SPK_PARK_QUAD(1, 1) SNNF_SPK_PARK_QUAD(2, 1) SNNF_SPK_PARK_QUAD(3, 1)
-                    }
-#undef SNNF_SPK_PARK_QUAD
-                    const int e_first = (wk - 4 * r) & (WK - 1);      // this wave finishes quads 4 r + e, e = e_first, e_first + WK, ... < 4
+                } else {
+                    // A narrow tile's four quads, all TT timesteps: quad e is finished by wave e mod WK of the tile, which adds the WK
+                    // partial sums in a fixed order and then runs that quad's timesteps like the unsplit kernel.
+                    __syncthreads();   // every wave is done with its staging region
+                    SNNF_SPK_PARK_QUAD(wave, 0, 0, 0) SNNF_SPK_PARK_QUAD(wave, 1, 0, 1) SNNF_SPK_PARK_QUAD(wave, 2, 0, 2) SNNF_SPK_PARK_QUAD(wave, 3, 0, 3)
+                    const int e_first = wk;      // this wave finishes quads e_first, e_first + WK, ... < 4
                     // The residual bytes of the wave's first quad travel while the workgroup meets.
                     uint32_t rb[TT];
 #pragma unroll
@@ -1397,20 +1408,20 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     if constexpr (FAST) {
                         if (e_first < 4 && g.res_layout >= 0 && TT > 1) {
 #pragma unroll
-                            for (int tw = 0; tw < TT; ++tw) rb[tw] = fast_res(tb + min(tw, t_count - 1), oc_e * TG + 4 * r + e_first);
+                            for (int tw = 0; tw < TT; ++tw) rb[tw] = fast_res(tb + min(tw, t_count - 1), oc_e * TG + e_first);
                         }
                     }
                     float v0[4] = {0.0f, 0.0f, 0.0f, 0.0f};
                     if constexpr (FAST) {
-                        if (e_first < 4) fast_v0(oc_e * TG + 4 * r + e_first, v0);
+                        if (e_first < 4) fast_v0(oc_e * TG + e_first, v0);
                     }
                     DenseIn in = {};
                     if constexpr (DENSE) {
-                        if (e_first < 4) dense_request(oc_e * TG + 4 * r + e_first, in);
+                        if (e_first < 4) dense_request(oc_e * TG + e_first, in);
                     }
                     __syncthreads();
                     for (int e_own = e_first; e_own < 4; e_own += WK) {
-                        const int j8 = oc_e * TG + 4 * r + e_own;
+                        const int j8 = oc_e * TG + e_own;
                         float xq[TT][4];
                         {
                             // The partial sums of the tile's waves, all timesteps of a wave (of two waves) in flight together (WK is a power
@@ -1459,6 +1470,8 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     }
                 }
             }
+#undef SNNF_SPK_PARK_QUAD
+#undef SNNF_SPK_ADD_QUAD
             if constexpr (SK) __syncthreads();   // the partial sums are read before the next window's staging overwrites them
         }
     }
