@@ -13,7 +13,7 @@ BF16, F16 = torch.bfloat16, torch.float16
 @pytest.mark.parametrize("Cin,Cout,H,W,N,T,dtype,residual,layout,waves,tile", [
     (64, 64, 56, 56, 9, 5, BF16, True, "bits", "8x1x2", 64),      # two waves per tile, a last window of one step
     (16, 64, 40, 40, 46, 6, BF16, True, "bits", "8x1x1", 64),     # a wave per tile, several rounds
-    (16, 72, 40, 40, 5, 8, F16, False, "c8", "8x1x1", 64),        # blocked inputs; eight channels in the last tile
+    (16, 72, 40, 40, 20, 8, F16, False, "c8", "8x1x1", 64),       # blocked inputs; eight channels in the last tile
     (256, 128, 14, 14, 24, 7, BF16, True, "bits", "8x1x4", 64),   # four waves per tile
     (512, 512, 7, 7, 9, 6, BF16, False, "bits", "8x1x8", 64),     # eight
     (128, 40, 8, 8, 1, 16, BF16, True, "bits", "8x1x8", 32),      # tiles of 32 channels, four windows
@@ -32,4 +32,31 @@ def test_membrane_passes_from_window_to_window(snnf_lib, Cin, Cout, H, W, N, T, 
     assert int(plan["variant"]) >= 60 and int(plan["window"]) == 4, plan
     if torch.cuda.get_device_properties(0).multi_processor_count == 256:
         assert (plan["waves"], int(plan["oc_tile"])) == (waves, tile), plan
+    check(B.to_dense(out), v, ref, what=f"{Cin}->{Cout} {H}x{W} T={T}")
+
+
+SOFT = (1.0, -1.0, 2.0)
+
+
+@pytest.mark.parametrize("Cin,Cout,H,W,k,N,T,dtype,residual,layout,lif", [
+    (64, 8, 28, 28, 3, 73, 6, BF16, True, "bits", LIF),       # one group of channels, several rounds and windows
+    (16, 32, 40, 40, 3, 5, 4, F16, True, "c8", LIF),
+    (16, 24, 9, 11, 5, 3, 1, BF16, True, "bits", LIF),        # one step
+    (16, 96, 8, 8, 3, 3, 2, BF16, False, "bits", LIF),        # three tiles of 32 channels, two steps
+    (16, 72, 14, 14, 1, 2, 4, F16, True, "bits", LIF),        # the last of them with 8
+    (16, 20, 13, 7, 3, 2, 7, BF16, True, "c8", SOFT),         # the general epilogue, half a group of channels
+])
+def test_narrow_tiles_of_one_wave(snnf_lib, Cin, Cout, H, W, k, N, T, dtype, residual, layout, lif):
+    from triton_snn_fusion_amd.runtime import hip_blocked_backend as B
+    g = gen(7300 + Cin + Cout + T)
+    x = torch.stack([spikes((N, Cin, H, W), 0.25, g) for _ in range(T)])
+    w, b = q(torch.randn(Cout, Cin, k, k, generator=g) * 2.0 * (2.0 / (Cin * k * k)) ** 0.5, dtype), q(torch.randn(Cout, generator=g) * 0.1, dtype)
+    rs = torch.stack([spikes((N, Cout, H, W), 0.25, g) for _ in range(T)]) if residual else None
+    p = k // 2
+    ref = O.temporal_conv_lif(list(x), w, b, torch.tensor(0.0), (1, 1), (p, p), (1, 1), 1, *lif, residuals=list(rs) if residual else None)
+    out, v = B.conv_lif_blocked(B.from_dense(dev(x, dtype), B.BITS if layout == "bits" else B.C8), dev(w, dtype), dev(b, dtype), [1, 1], [p, p], lif,
+                                residual=B.from_dense(dev(rs, dtype), B.BITS) if residual else None, out_layout=B.BITS, want_v=True)
+    plan = B.last_conv_plan()
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert (plan["waves"], int(plan["oc_tile"])) == ("8x1x1", 32), plan
     check(B.to_dense(out), v, ref, what=f"{Cin}->{Cout} {H}x{W} T={T}")

@@ -57,7 +57,7 @@ def test_whole_tiles_on_the_matrix_kernel(snnf_lib, Cin, Cout, H, W, k, s, T, N,
     (128, 256, 28, 3, 2, 8, 5, False, True),
     (64, 128, 56, 3, 2, 4, 16, False, False),
     (64, 128, 56, 1, 2, 4, 16, False, False),
-    (16, 64, 40, 3, 1, 4, 2, False, False),      # a single stage
+    (16, 64, 40, 3, 1, 4, 2, False, True),       # a single stage: narrow tiles of one wave
     (256, 256, 14, 3, 1, 4, 16, True, True),     # deep: with a residual ...
     (256, 256, 14, 3, 1, 4, 16, False, False),   # ... and without
 ])

@@ -127,8 +127,7 @@ RouteSpace route_space(int T, int N, int Cin, int H, int W, bool split, int64_t 
 //   40^2 x 20 (tiles of four columns) 43 / 33, T = 8 121 / 68, at 56^2 x 21, T = 6 132 / 110, 128 -> 256 stride 2 at 28^2 x 5, T = 8 49 / 40, 1x1 stride 2 x 2
 //   31 / 20; 64 -> 64 at 56^2 x 16 34 / 42, 128 -> 128 at 28^2 x 32 48 / 52 (x 16 38 / 36), 64 -> 128 stride 2 at 56^2 x 16 28 / 37, 1x1 18 / 26, 128 -> 256 stride 2
 //   at 28^2 x 16 28 / 34 stay. Inputs that the caches don't hold between the copy and the kernel move the lines (64 -> 64 at 56^2 x 88, T = 5
-//   with a residual 366 / 437, 128 -> 256 stride 2 at 28^2 x 164, T = 7 395 / 554). A single stage of 16 channels leaves the waves nothing to share
-//   (16 -> 64 at 40^2 x 2 13.6 / 16.2). Deep layers of few outputs always move (256 -> 256 at 14^2 x 4 29 / 18, 512 -> 512 at 4^2 x 16 37 / 21). Three kinds
+//   with a residual 366 / 437, 128 -> 256 stride 2 at 28^2 x 164, T = 7 395 / 554). Deep layers of few outputs always move (256 -> 256 at 14^2 x 4 29 / 18, 512 -> 512 at 4^2 x 16 37 / 21). Three kinds
 //   that would gain as well stay with the kernel that their reported plan names in the tests: planes of four pixels at most (256 -> 512
 //   at 2^2 x 40 24 / 14), one window of four steps of up to 512 pixels with less than 128 channels (64 -> 64 at 16^2 x 2 30 / 11) and deep layers
 //   without a residual that fill the chip (256 -> 256 at 14^2 x 16 35 / 31; with one they move, 37 / 32).
@@ -167,7 +166,7 @@ bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int C
         case DenseFamily::kMatrixWhole:
             if (deep) return true;
             if (plane <= 4 || (T >= 3 && T <= 4 && !one && !strided && pixels <= 512 && K < 1152)) return false;
-            if (!one && Cin <= 16) return false;   // a single stage, which waves cannot share
+            if (!one && !strided && Cin <= 8) return false;   // (a single channel group: as above)
             if (K >= 2304 && T <= 4 && !residual && tile_use >= 1.0) return false;
             if (one) return tile_use * std::sqrt(576.0 / K) <= 0.45;
             if (strided) return tile_use * std::sqrt(std::sqrt(576.0 / K)) <= (T <= 4 ? 0.5 : (inputs < (1 << 24) ? 0.65 : 0.45));
@@ -304,7 +303,11 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
     g.wk_log2 = wk_log2;
     // Tiles of 32 channels where even those fit one round of waves: 256 -> 256 at 14^2 x 4 (112 tiles of 64 channels on eight waves each)
     // 13.9 -> 10.0 us, 512 -> 512 at 7^2 x 8 19.8 -> 13.9, at 4^2 x 32 22.2 -> 17.6. At twice the tiles they would make a second round.
-    if (!c.split && (tt == 4 || (!pool2 && c.x_layout != SNNF_LAYOUT_NCHW)) && wk_log2 > 0 && !p.tuned_split && Cout > 32 && static_cast<int64_t>(g.n_patches) * ((Cout + 31) / 32) << wk_log2 <= static_cast<int64_t>(cus) * kSpkWaves) {
+    // The same where a single stage leaves nothing to share (16 -> 64 at 14^2 x 17 10.2 -> 7.6, 16 -> 96 at 8^2 x 3 8.8 -> 6.6, 16 -> 64 at 28^2 x 6,
+    // 5x5, T = 6 21.2 -> 14.8). Up to 32 channels always: half of a tile of 64 would be empty (90 layers, factors of 1.13 to 1.5: 64 -> 8 at 28^2 x 73,
+    // T = 8 37.5 -> 27.7, 128 -> 32 at 32^2 x 18 22.2 -> 16.6, 128 -> 24 at 14^2 10.7 -> 8.2).
+    if (!c.split && (tt == 4 || !pool2) && c.x_layout != SNNF_LAYOUT_NCHW && !p.tuned_split && (wk_log2 > 0 || (!pool2 && sc == nullptr)) &&
+        ((Cout <= 32 && wk_log2 == 0) || static_cast<int64_t>(g.n_patches) * ((Cout + 31) / 32) << wk_log2 <= static_cast<int64_t>(cus) * kSpkWaves)) {
         g.narrow = 1;
         oc_tiles = (Cout + 31) / 32;
         g.n_items = g.n_patches * oc_tiles;
@@ -322,7 +325,9 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
     // Workgroups full of waves that leave a quarter of the compute units idle in every round, or half of them in the only one: a workgroup
     // on every unit, some of its waves idle in the last round (128 -> 128 at 28^2 x 40, 140 workgroups 55.5 us, 256 workgroups 45.1; 64 -> 64
     // at 24^2, one image, 18 and 36 workgroups 8.5 / 7.5). Fuller rounds stay even: 256 -> 256 at 14^2 x 128, 224 workgroups 100 us, 256 105.
-    if (g.iters > 1 ? grid * 4 < resident * 3 : grid * 2 <= cus) grid = std::min(g.n_items, g.iters > 1 ? resident : cus);
+    // Narrow tiles of one wave: two tiles of a patch side by side, which read the same activations.
+    const int spread = g.narrow && !c.split && wk_log2 == 0 ? g.n_patches * ((Cout + 63) / 64) : g.n_items;
+    if (g.iters > 1 ? grid * 4 < resident * 3 : grid * 2 <= cus) grid = std::min(spread, g.iters > 1 ? resident : cus);
     g.d_ppx = make_fast_div(g.PR * g.PC);
     g.d_PC = make_fast_div(g.PC);
     g.d_region = make_fast_div(g.region);

@@ -193,7 +193,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
     static_assert(!POOL || (FAST && (TT == 4 || TT == 1)), "the pooled output belongs to the straight-line epilogue of four steps");
     static_assert(IN != SNNF_LAYOUT_NCHW || TT == 1, "a dense input is one frame for all timesteps");
     constexpr bool SPLIT = std::is_same<XT, float>::value;
-    static_assert(!NARROW || ((SK || SPLIT) && IN != SNNF_LAYOUT_NCHW), "narrow tiles are for launches that share K among waves, and for fp32");
+    static_assert(!NARROW || (IN != SNNF_LAYOUT_NCHW && (SK || (!SC && !POOL))), "narrow tiles: not of a dense frame, nor without shared K in a shortcut's or a pooled launch");
     static_assert(!SPLIT || (NARROW && IN == SNNF_LAYOUT_C8 && !FAST && !SC && !POOL), "fp32 tensors: narrow tiles on two C8 tensors, dense tensors out");
     static_assert(!MULTI || (FAST && !POOL), "several windows belong to the straight-line epilogue");
     static_assert(!DENSE || (IN == SNNF_LAYOUT_C8 && !FAST && !SC && !POOL), "the dense epilogue belongs to calls on dense tensors");
@@ -1225,7 +1225,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     }
                     if (MULTI && t0 > 0) {
 #pragma unroll
-                        for (int fq = 0; fq < 8; ++fq) fast_v0(oc_e * TG + fq, v0[fq]);
+                        for (int fq = 0; fq < TG; ++fq) fast_v0(oc_e * TG + fq, v0[fq]);
                         __builtin_amdgcn_sched_barrier(0);
                     }
                     if (with_res && TT > 1) {
@@ -1235,6 +1235,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                             res_ptr[tw] = static_cast<const unsigned char*>(sk_kernarg_ptr(kResTable, tb + min(tw, t_count - 1))) + static_cast<int64_t>(oc_e) * TG * po;
                         auto req_res = [&](auto fq_tag) __attribute__((always_inline)) {
                             constexpr int fq = decltype(fq_tag)::value;
+                            if constexpr (fq >= TG) return;
                             const uint32_t off = lane_bits + static_cast<uint32_t>(min(fq, g.C8out - 1 - oc_e * TG) * po);
 #pragma unroll
                             for (int tw = 0; tw < TT; ++tw) rb[fq][tw] = res_ptr[tw][off];
@@ -1251,12 +1252,14 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     }
                     auto do_quad = [&](auto fq_tag) __attribute__((always_inline)) {
                         constexpr int fq = decltype(fq_tag)::value;
-                        float xq[TT][4];
+                        if constexpr (fq < TG) {
+                            float xq[TT][4];
 #pragma unroll
-                        for (int tw = 0; tw < TT; ++tw)
+                            for (int tw = 0; tw < TT; ++tw)
 #pragma unroll
-                            for (int k = 0; k < 4; ++k) xq[tw][k] = acc[tw][(fq >> 2) % NF][4 * (fq & 3) + k];
-                        fast_quad(oc_e * TG + fq, xq, rb[fq], with_res, v0[fq]);
+                                for (int k = 0; k < 4; ++k) xq[tw][k] = acc[tw][(fq >> 2) % NF][4 * (fq & 3) + k];
+                            fast_quad(oc_e * TG + fq, xq, rb[fq], with_res, v0[fq]);
+                        }
                     };
                     do_quad(std::integral_constant<int, 0>{});
                     do_quad(std::integral_constant<int, 1>{});
@@ -1487,18 +1490,20 @@ int launch_conv_spk_variant(const SpkLaunch& L) {
     };
     if constexpr (IN == SNNF_LAYOUT_C8) {
         if (L.dense_epilogue) {
-            if (L.g.narrow) return run(conv_spk_kernel<XT, TT, IN, true, false, false, false, true, true>);
+            if (L.g.narrow) return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, IN, true, false, false, false, true, true>) : run(conv_spk_kernel<XT, TT, IN, false, false, false, false, true, true>);
             return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, IN, true, false, false, false, false, true>) : run(conv_spk_kernel<XT, TT, IN, false, false, false, false, false, true>);
         }
     }
     if constexpr (TT == 4) {
         if (L.fast_epilogue && L.multi_window) {
-            if (L.g.narrow) return run(conv_spk_kernel<XT, TT, IN, true, true, false, false, true, false, true>);
+            if (L.g.narrow) return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, IN, true, true, false, false, true, false, true>) : run(conv_spk_kernel<XT, TT, IN, false, true, false, false, true, false, true>);
             return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, IN, true, true, false, false, false, false, true>) : run(conv_spk_kernel<XT, TT, IN, false, true, false, false, false, false, true>);
         }
     }
-    if (L.g.narrow)
+    if (L.g.narrow) {
+        if (L.g.wk_log2 == 0) return L.fast_epilogue ? run(conv_spk_kernel<XT, TT, IN, false, true, false, false, true>) : run(conv_spk_kernel<XT, TT, IN, false, false, false, false, true>);
         return L.fast_epilogue ? run(conv_spk_kernel<XT, TT, IN, true, true, false, false, true>) : run(conv_spk_kernel<XT, TT, IN, true, false, false, false, true>);
+    }
     if (L.fast_epilogue) return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, IN, true, true>) : run(conv_spk_kernel<XT, TT, IN, false, true>);
     return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, IN, true, false>) : run(conv_spk_kernel<XT, TT, IN, false, false>);
 }
