@@ -60,3 +60,30 @@ def test_narrow_tiles_of_one_wave(snnf_lib, Cin, Cout, H, W, k, N, T, dtype, res
     if torch.cuda.get_device_properties(0).multi_processor_count == 256:
         assert (plan["waves"], int(plan["oc_tile"])) == ("8x1x1", 32), plan
     check(B.to_dense(out), v, ref, what=f"{Cin}->{Cout} {H}x{W} T={T}")
+
+
+@pytest.mark.parametrize("Cin,Cout,H,k,s,N,T,out,lif", [
+    (3, 64, 32, 3, 1, 2, 4, "bits", LIF),
+    (3, 96, 20, 7, 2, 1, 6, "bits", LIF),                     # three tiles of 32 channels, steps in a loop
+    (1, 8, 9, 3, 1, 3, 2, "c8", LIF),                         # the general epilogue
+    (3, 64, 32, 3, 1, 70, 8, "bits", LIF),                    # 2240 patches: tiles of 64 channels again
+    (2, 64, 16, 3, 1, 3, 4, "pooled", LIF),
+])
+def test_narrow_tiles_of_a_frame(snnf_lib, Cin, Cout, H, k, s, N, T, out, lif):
+    from triton_snn_fusion_amd.runtime import hip_blocked_backend as B
+    g = gen(7350 + Cout + T)
+    frame = q(torch.randn(N, Cin, H, H, generator=g), BF16)
+    w, b = q(torch.randn(Cout, Cin, k, k, generator=g) * 2.0 * (2.0 / (Cin * k * k)) ** 0.5, BF16), q(torch.randn(Cout, generator=g) * 0.1, BF16)
+    p = k // 2
+    ref = O.temporal_conv_lif([frame] * T, w, b, torch.tensor(0.0), (s, s), (p, p), (1, 1), 1, *lif)
+    x = B.input_frame(dev(frame, BF16), T)
+    if out == "pooled":
+        got = B.to_dense(B.conv_lif_blocked_avgpool(x, dev(w, BF16), dev(b, BF16), [s, s], [p, p], lif)[0]).float().cpu()
+        want = torch.stack([torch.nn.functional.avg_pool2d(t, 2) for t in ref[0]])
+        assert float((got != want).float().mean()) <= 1e-3
+    else:
+        o, v = B.conv_lif_blocked(x, dev(w, BF16), dev(b, BF16), [s, s], [p, p], lif, out_layout=B.BITS if out == "bits" else B.C8, want_v=True)
+        check(B.to_dense(o), v, ref, what=f"{Cin}->{Cout} {H}x{H} T={T}")
+    plan = B.last_conv_plan()
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert int(plan["oc_tile"]) == (64 if N == 70 else 32), plan

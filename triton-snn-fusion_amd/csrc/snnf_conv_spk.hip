@@ -304,10 +304,12 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
     // Tiles of 32 channels where even those fit one round of waves: 256 -> 256 at 14^2 x 4 (112 tiles of 64 channels on eight waves each)
     // 13.9 -> 10.0 us, 512 -> 512 at 7^2 x 8 19.8 -> 13.9, at 4^2 x 32 22.2 -> 17.6. At twice the tiles they would make a second round.
     // The same where a single stage leaves nothing to share (16 -> 64 at 14^2 x 17 10.2 -> 7.6, 16 -> 96 at 8^2 x 3 8.8 -> 6.6, 16 -> 64 at 28^2 x 6,
-    // 5x5, T = 6 21.2 -> 14.8). Up to 32 channels always: half of a tile of 64 would be empty (90 layers, factors of 1.13 to 1.5: 64 -> 8 at 28^2 x 73,
+    // 5x5, T = 6 21.2 -> 14.8; frames: 3 -> 64 at 32^2 x 8 8.5 -> 6.5, 7x7 at 224^2 10.0 -> 8.3, T = 8 16.6 -> 11.3); of one timestep
+    // two workgroups share a unit (3 -> 64 at 32^2 x 64, T = 8 15.6 -> 13.7, 16 -> 64 at 40^2 x 30 10.1 -> 8.7). Up to 32 channels always: half of a tile of 64 would be empty (90 layers, factors of 1.13 to 1.5: 64 -> 8 at 28^2 x 73,
     // T = 8 37.5 -> 27.7, 128 -> 32 at 32^2 x 18 22.2 -> 16.6, 128 -> 24 at 14^2 10.7 -> 8.2).
-    if (!c.split && (tt == 4 || !pool2) && c.x_layout != SNNF_LAYOUT_NCHW && !p.tuned_split && (wk_log2 > 0 || (!pool2 && sc == nullptr)) &&
-        ((Cout <= 32 && wk_log2 == 0) || static_cast<int64_t>(g.n_patches) * ((Cout + 31) / 32) << wk_log2 <= static_cast<int64_t>(cus) * kSpkWaves)) {
+    const bool frame = c.x_layout == SNNF_LAYOUT_NCHW;
+    if (!c.split && (tt == 4 || !pool2 || frame) && !p.tuned_split && (wk_log2 > 0 ? !frame : frame || (!pool2 && sc == nullptr)) &&
+        ((Cout <= 32 && wk_log2 == 0) || static_cast<int64_t>(g.n_patches) * ((Cout + 31) / 32) << wk_log2 <= static_cast<int64_t>(cus) * kSpkWaves * (tt == 1 && wk_log2 == 0 ? 2 : 1))) {
         g.narrow = 1;
         oc_tiles = (Cout + 31) / 32;
         g.n_items = g.n_patches * oc_tiles;

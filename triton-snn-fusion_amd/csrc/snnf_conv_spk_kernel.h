@@ -193,7 +193,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
     static_assert(!POOL || (FAST && (TT == 4 || TT == 1)), "the pooled output belongs to the straight-line epilogue of four steps");
     static_assert(IN != SNNF_LAYOUT_NCHW || TT == 1, "a dense input is one frame for all timesteps");
     constexpr bool SPLIT = std::is_same<XT, float>::value;
-    static_assert(!NARROW || (IN != SNNF_LAYOUT_NCHW && (SK || (!SC && !POOL))), "narrow tiles: not of a dense frame, nor without shared K in a shortcut's or a pooled launch");
+    static_assert(!NARROW || SK || (!SC && (!POOL || IN == SNNF_LAYOUT_NCHW)), "narrow tiles of one wave: not of a shortcut, and pooled only of a dense frame");
     static_assert(!SPLIT || (NARROW && IN == SNNF_LAYOUT_C8 && !FAST && !SC && !POOL), "fp32 tensors: narrow tiles on two C8 tensors, dense tensors out");
     static_assert(!MULTI || (FAST && !POOL), "several windows belong to the straight-line epilogue");
     static_assert(!DENSE || (IN == SNNF_LAYOUT_C8 && !FAST && !SC && !POOL), "the dense epilogue belongs to calls on dense tensors");
@@ -1546,6 +1546,10 @@ int launch_conv_spk_frame(const SpkLaunch& L, bool pooled) {
         return check_launch("snnf_conv_lif_blocked");
     };
     constexpr int D = SNNF_LAYOUT_NCHW;
+    if (L.g.narrow) {
+        if (pooled) return run(conv_spk_kernel<XT, 1, D, false, true, false, true, true>);
+        return L.fast_epilogue ? run(conv_spk_kernel<XT, 1, D, false, true, false, false, true>) : run(conv_spk_kernel<XT, 1, D, false, false, false, false, true>);
+    }
     if (pooled) return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, 1, D, true, true, false, true>) : run(conv_spk_kernel<XT, 1, D, false, true, false, true>);
     if (L.fast_epilogue) return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, 1, D, true, true>) : run(conv_spk_kernel<XT, 1, D, false, true>);
     return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, 1, D, true, false>) : run(conv_spk_kernel<XT, 1, D, false, false>);
