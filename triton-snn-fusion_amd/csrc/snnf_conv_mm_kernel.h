@@ -8,11 +8,11 @@
 //     tiles, 128 registers): a weight fragment feeds TT matrix instructions, an activation fragment two.
 //   * A tile is TH x TW output pixels of ONE image, so a lane's pixel, its LDS address and its output offset are kernel
 //     constants; a tile contributes uniform bases only. The halo tile in LDS holds explicit zeros for padding, so the
-//     matrix loop has no bounds logic: per pair of k-slots the (tap, channel group) offsets are walked on the scalar unit.
+//     matrix loop has no bounds logic: per pair of k-slots the (tap, channel group) offsets come out of a table in a register.
 //   * Staging loads are unconditional (out-of-image items read a valid address and are zeroed on their way into LDS)
-//     and issued from a single place one stage ahead; the LIF epilogue runs on a wave-private LDS stage, 16 channel rows
-//     x 32 pixels at a time, so that a lane owns 8 consecutive pixels: 16-byte spike stores, membrane in registers
-//     across the TT steps.
+//     and issued from a single place one stage ahead; the LIF epilogue goes through a wave-private LDS stage, 16 channel rows
+//     x 32 pixels at a time, so that a lane stores 8 consecutive pixels: 16 bytes of spikes. Whole tiles of 16-bit tensors send
+//     the spikes through it as bits (SPIKES below), single steps and sums without a neuron the sums themselves.
 //   * SK: layers with few pixels and many channels (deep stages) do not fill the machine with 64 x 32 wave tiles, so
 //     WK waves share an output tile, each taking every WK-th pair of k-slots, and add their sums through LDS.
 // FAST: every tile is full, runs of 8 pixels are contiguous and 16-byte aligned, Cout % 64 == 0, fp32 membrane, the

@@ -153,7 +153,7 @@ __device__ __forceinline__ sk_u32x4 sk_expand_bits(uint32_t byte) {
     return d;
 }
 
-// NARROW: tiles of 32 output channels (one weight fragment) for launches of few tiles that share K among waves: twice the workgroups,
+// NARROW: tiles of 32 output channels (one weight fragment) for layers of up to 32 channels and for launches of few tiles: twice the workgroups,
 // each with half the matrix instructions and half the weights in its chain of steps, which is what such a launch lasts (512 -> 512 at
 // 4^2, one image: 288 steps on eight waves, 19.1 -> 12.6 us; 64 -> 64 at 56^2 11.7 -> 8.7 us; of one timestep 512 -> 512 at 4^2 10.8 -> 7.5).
 // MULTI: the straight-line epilogue of calls of several windows, which pass the membrane on through memory (a variant of its own: the
