@@ -422,6 +422,13 @@ def test_scratch_is_asked_for_only_where_it_is_used(snnf_lib, shape, asked):
     assert snnf_lib.snnf_conv_bias_workspace_bytes(4, 16, 512, 7, 7, _lib.SNNF_BF16, 512, 3, 3, 1, 1, 1, 1, 0) == 4 * 16 * 64 * 49 * 16
 
 
+@pytest.mark.parametrize("T,N,Cin", [(16, 1 << 15, 4096), (16, 1 << 17, 1024), (8, 3 << 16, 1400), (4, 1 << 17, 4096)])
+def test_sizes_beyond_31_bits_do_not_wrap_in_the_rule(snnf_lib, T, N, Cin):
+    """Strided 1x1 layers move up to 2^24 inputs; these have 2^31 or more (their product as an int wraps to zero or below)."""
+    asks = lambda n: snnf_lib.snnf_conv_lif_scratch_bytes(T, n, Cin, 1, 1, _lib.SNNF_BF16, 64, 1, 1, 2, 2, 0, 0, _lib.SNNF_F32, 0)
+    assert T * N * Cin >= 1 << 31 and (asks(N), asks(1)) == (0, T * Cin // 8 * 16)
+
+
 def test_a_tuned_plan_is_seen_by_a_remembered_route(snnf_lib):
     """A 7x7 layer whose planned stages of four channel groups hold more steps than the table, and stages of two do not."""
     layer = (2, 2, 372, 5, 5, 384, 7, 7, 1, 1, 3, 3)

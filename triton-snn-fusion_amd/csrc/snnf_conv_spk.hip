@@ -161,7 +161,7 @@ bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int C
         case DenseFamily::kTimeOuter: return !pointwise || static_cast<int64_t>(T) * N * (Cin + Cout) * plane <= (1 << 25);
         case DenseFamily::kPointwise: return plane % 64 != 0 || (Cout % 32 != 0 && outs <= (1 << 22));
         case DenseFamily::kMatrixMasked:
-            if (one) return T <= 2 ? outs <= (1 << 17) : !strided || T * N * Cin * plane <= (1 << 24);
+            if (one) return T <= 2 ? outs <= (1 << 17) : !strided || inputs <= (1 << 24);
             return T > 2 || K >= 1152 || !strided || outs <= (3 << 19);
         case DenseFamily::kMatrixWhole:
             if (deep) return true;
