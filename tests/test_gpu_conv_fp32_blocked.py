@@ -106,3 +106,29 @@ def test_infinities_and_nan_reach_the_same_neurons(snnf_lib):
     want = run(snnf_lib, xs, w, b, rs, v0, 3, 1, LIF, 255, 0)
     assert torch.equal(got[1].isnan(), want[1].isnan()) and got[1].isnan().any()
     assert torch.equal(got[0], want[0]) and torch.allclose(got[1], want[1], rtol=1e-5, atol=1e-6, equal_nan=True)
+
+
+@pytest.mark.parametrize("Cin,Cout,H,W,k,s,T,N,groups", [
+    (16, 32, 40, 24, 3, 1, 4, 2, None),         # tiles of part of an image
+    (40, 24, 23, 31, 3, 1, 3, 2, (0, 3, 4)),    # flags of 64 items across rows and channel groups; a stage with a single group
+    (24, 24, 64, 8, 5, 2, 5, 1, (1, 2)),        # two windows, the last of one timestep
+    (600, 16, 9, 14, 1, 1, 2, 2, (0, 10, 63, 64, 73, 74)),    # more than 64 channel groups
+    (6, 16, 33, 33, 3, 1, 4, 1, None),          # pairs of taps
+    (64, 16, 4, 4, 3, 1, 4, 5, (0, 7)),         # several images per tile
+])
+def test_a_low_term_counts_wherever_it_is(snnf_lib, Cin, Cout, H, W, k, s, T, N, groups):
+    """One input per call, 1 + 2^-9 (terms 1 and 2^-9), between zeros: an output that it reaches is one product, whose dropped part, the
+    product of the two low terms, is 2^-16 of it or less. The sums of the silent neuron are scaled by powers of two."""
+    g = gen(6300 + Cin)
+    Ho, Wo = (H + 2 * (k // 2) - k) // s + 1, (W + 2 * (k // 2) - k) // s + 1
+    w = torch.randn(Cout, Cin, k, k, generator=g).sign() * (torch.rand(Cout, Cin, k, k, generator=g) + 0.5)
+    places = [(h, x) for h in sorted({0, 1, H // 2, H - 2, H - 1}) for x in (0, W // 2, W - 1)]
+    for i, (h, x) in enumerate(places):
+        xs = [torch.zeros(N, Cin, H, W) for _ in range(T)]
+        group = (groups or range(-(-Cin // 8)))[i % len(groups or range(-(-Cin // 8)))]
+        xs[i % T][i % N, min(group * 8 + i % 8, Cin - 1), h, x] = 1.0 + 2.0 ** -9
+        got = run(snnf_lib, xs, w, torch.zeros(Cout), None, torch.tensor(0.0), k, s, (1e9, 0.0, 2.0), 255)[1].double().cpu()
+        v64 = torch.zeros(N, Cout, Ho, Wo, dtype=torch.float64)
+        for step in xs:
+            v64 = (v64 + torch.nn.functional.conv2d(step.double(), w.double(), None, s, k // 2)) / 2
+        assert torch.all((got - v64).abs() <= v64.abs() * 2.0 ** -15), (h, x, group)

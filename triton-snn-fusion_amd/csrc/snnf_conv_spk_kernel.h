@@ -536,16 +536,35 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             const int s_first = SK ? wk : 0;
             const int s_step = SK ? WK : 1;
             int nstages_all = SC ? g.nstages + g.sc_stages : g.nstages;
+            // SPLIT: stages of low terms only where the tile's halo has any in this window: bit c8 & 63 of `low_groups` says that channel group
+            // c8 has one in the rows of the halo. A lane reads the flags of one group, RR W / 64 of them and one more; the groups of whole
+            // images (tiles of several, at most 32 pixels a group) are one short range of flags and run all their low stages or none.
+            // Reading whole images for every tile, and running all low stages of an image for one low term in it, took 64 -> 64 at 224^2 114 us
+            // without low terms (here 69) and 147 with a single one (76), 512 -> 512 at 112^2 722 (575) and 1231 (579), 64 -> 8 as 1x1 at
+            // 640^2, one timestep, 156 (54); 64 -> 64 at 32^2 x 8 is the same, 20 us.
+            uint64_t low_groups = 0;
             if constexpr (SPLIT) {
-                // Stages of low terms only where the tile's images have any in this window (their flags are one range of bytes per step).
-                const int image_items = g.C8in * g.H * g.W;
-                const int w0 = (n0 * image_items) >> 8, w1 = (min(n0 + g.PI, g.N) * image_items - 1) >> 8;   // dwords of four flags
-                uint32_t any = 0;
-                for (int t = t0; t < min(t0 + TT, nsteps_t); ++t) {
-                    const uint32_t* __restrict__ flags_t = reinterpret_cast<const uint32_t*>(lo_flags + static_cast<int64_t>(t) * g.flag_stride);
-                    for (int w = w0 + lane; w <= w1; w += 64) any |= flags_t[w];
+                const int plane = g.H * g.W;
+                const bool images = g.PI > 1;
+                const int r0 = images ? 0 : max(ih_lo, 0);
+                const int items = images ? min(g.PI, g.N - n0) * g.C8in * plane : (min(ih_lo + g.RR, g.H) - r0) * g.W;
+                const int dwords = ((items - 1) >> 8) + 2;                       // of four flags, 256 items; that many at most
+                for (int c0 = 0; c0 < (images ? 1 : g.C8in); c0 += 64) {
+                    const bool mine = images || c0 + lane < g.C8in;
+                    const int first = ((n0 * g.C8in + (!images && mine ? c0 + lane : 0)) * g.H + r0) * g.W, last = first + items - 1;
+                    const int w0 = first >> 8, w1 = last >> 8;
+                    uint32_t any = 0;
+                    for (int d = images ? lane : 0; d < dwords; d += images ? 64 : 1) {
+                        const int w = min(w0 + d, w1);
+                        const uint32_t mask = (w == w0 ? ~0u << ((first >> 6 & 3) * 8) : ~0u) & (w == w1 ? ~0u >> ((3 - (last >> 6 & 3)) * 8) : ~0u);
+#pragma unroll
+                        for (int t = 0; t < TT; ++t)
+                            any |= reinterpret_cast<const uint32_t*>(lo_flags + static_cast<int64_t>(min(t0 + t, nsteps_t - 1)) * g.flag_stride)[w] & mask;
+                    }
+                    low_groups |= __ballot(mine && any != 0u);
                 }
-                if (__ballot(any != 0u) != 0ull) nstages_all = 2 * g.nstages;
+                if (images && low_groups != 0) low_groups = ~0ull;
+                if (low_groups != 0) nstages_all = 2 * g.nstages;
             }
             if constexpr (PRE) {
                 if (have && s_first < nstages_all) stage_req(s_first);
@@ -577,6 +596,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     const bool second = SC && stage >= g.nstages;     // a stage of the shortcut
                     const bool low = SPLIT && stage >= g.nstages;     // a stage of low activation terms: against the high weight terms alone
                     const int gg0 = (second || low ? stage - g.nstages : stage) * g.G;
+                    if (SPLIT && low && (low_groups >> (gg0 & 63) & ((1ull << g.G) - 1)) == 0) continue;
                     const int gpc_l2 = second ? g.sc_gpc_log2 : g.gpc_log2;
                     const int chunk = gg0 >> gpc_l2;
                     const int pbase = chunk * (second ? g.sc_npairs : g.npairs) + ((gg0 - (chunk << gpc_l2)) >> 1);   // pair of (tap 0, the stage's first two groups)
