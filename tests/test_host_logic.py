@@ -429,6 +429,23 @@ def test_sizes_beyond_31_bits_do_not_wrap_in_the_rule(snnf_lib, T, N, Cin):
     assert T * N * Cin >= 1 << 31 and (asks(N), asks(1)) == (0, T * Cin // 8 * 16)
 
 
+@pytest.mark.parametrize("layer,moves", [  # (T, N, Cin, H, W, Cout, stride), 1x1 on float32 tensors
+    ((2, 36, 96, 112, 112, 192, 2), False),     # whole tiles of the matrix kernel, one window, a full chip
+    ((2, 36, 96, 4, 4, 192, 2), True),          # ... most of the chip idle
+    ((4, 3, 64, 80, 80, 512, 2), False),        # ... many outputs
+    ((4, 1, 32, 56, 56, 192, 2), True),         # ... few
+    ((12, 5, 256, 24, 24, 512, 2), True),       # ... several windows
+    ((2, 4, 48, 125, 125, 248, 2), False),      # its masked tiles, one window, many outputs
+    ((1, 12, 192, 20, 20, 128, 2), True),       # ... few
+    ((4, 49, 3, 88, 64, 120, 2), True),         # ... two windows
+    ((2, 12, 192, 28, 28, 256, 1), False),      # no stride: one window, many outputs
+    ((4, 5, 192, 48, 48, 128, 1), True),
+])
+def test_which_1x1_layers_of_float32_tensors_move(snnf_lib, layer, moves):
+    T, N, Cin, H, W, Cout, s = layer
+    assert (snnf_lib.snnf_conv_lif_scratch_bytes(T, N, Cin, H, W, _lib.SNNF_F32, Cout, 1, 1, s, s, 0, 0, _lib.SNNF_F32, 0) > 0) == moves
+
+
 def test_a_tuned_plan_is_seen_by_a_remembered_route(snnf_lib):
     """A 7x7 layer whose planned stages of four channel groups hold more steps than the table, and stages of two do not."""
     layer = (2, 2, 372, 5, 5, 384, 7, 7, 1, 1, 3, 3)

@@ -131,11 +131,16 @@ RouteSpace route_space(int T, int N, int Cin, int H, int W, bool split, int64_t 
 //   that would gain as well stay with the kernel that their reported plan names in the tests: planes of four pixels at most (256 -> 512
 //   at 2^2 x 40 24 / 14), one window of four steps of up to 512 pixels with less than 128 channels (64 -> 64 at 16^2 x 2 30 / 11) and deep layers
 //   without a residual that fill the chip (256 -> 256 at 14^2 x 16 35 / 31; with one they move, 37 / 32).
-// * fp32 tensors (two bf16 terms each) run here at three times the speed of the dense kernels over 180 layers: 64 -> 64 at 32^2 x 8 35 / 20, at
-//   56^2 x 16 100 / 73, 512 -> 512 at 7^2 x 4 with a residual 125 / 29, 41 -> 72 at 8 x 14 x 15 191 / 20, 122 -> 111 at 15^2, 5x5, T = 5 1068 / 36,
-//   3 -> 64 at 32^2 x 64 34 / 31, 128 -> 256 1x1 at 28^2 x 8 135 / 27. Only 1x1 layers with few products per output stay, where those are many:
-//   the copy and the elementwise outputs are their time (64 -> 256 at 56^2 x 16, T = 1 with a residual 66 / 82, 64 -> 128 at 112^2 x 4 80 / 90,
-//   32 -> 192 at 56^2 x 16 116 / 124; but 64 -> 128 at 28^2 x 8 79 / 25, 128 -> 256 at 56^2 x 16 281 / 192).
+// * fp32 tensors (two bf16 terms each) run here at two and a half times the speed of the dense kernels over 1500 layers without low terms, and at
+//   1.85 times where every input has one: 64 -> 64 at 32^2 x 8 35 / 20, at 56^2 x 16 100 / 73, 512 -> 512 at 7^2 x 4 with a residual 125 / 29, 41 -> 72
+//   at 8 x 14 x 15 191 / 20, 122 -> 111 at 15^2, 5x5, T = 5 1068 / 36, 3 -> 64 at 32^2 x 64 34 / 31, 128 -> 256 1x1 at 28^2 x 8 135 / 27. 1x1 layers
+//   stay where the copy and the elementwise outputs are their time: on the pointwise kernel those with few products per output and many outputs
+//   (64 -> 256 at 56^2 x 16, T = 1 with a residual 66 / 82, 64 -> 128 at 112^2 x 4 80 / 90, 32 -> 192 at 56^2 x 16 116 / 124; but 64 -> 128 at 28^2 x 8
+//   79 / 25, 128 -> 256 at 56^2 x 16 281 / 192); on the matrix kernel, which takes up to four steps in one window, those of a stride, of
+//   whose copy a quarter is read, unless that kernel would leave the chip idle or they have few outputs or several windows (without low
+//   terms / with them everywhere: 96 -> 192 at 112^2 x 36, T = 2 0.54 / 0.34 of its speed, 64 -> 512 at 80^2 x 3 0.80 / 0.54, 48 -> 248 at 125^2 x 4, T = 2
+//   0.80 / 0.65; 32 -> 192 at 56^2 1.90 / 1.55, 256 -> 512 at 24^2 x 5, T = 12 4.46 / 2.73), and others of one or two steps and many outputs (192 -> 256
+//   at 28^2 x 12, T = 2 0.89 / 0.69; 192 -> 128 x 3 1.37 / 1.12).
 // Without a neuron the lines are those of sums that leave as 16-bit values (512 -> 512 at 7^2 x 16 56 / 35).
 bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w,
                          int v_dtype, bool residual, bool neuron, DenseFamily& family) {
@@ -149,7 +154,12 @@ bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int C
     const int64_t out = pixels * Cout, outs = T * out, inputs = static_cast<int64_t>(T) * N * Cin * plane;
     double tile_use;
     family = dense_family(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, tile_use);
-    if (x_dtype == SNNF_F32) return !(family == DenseFamily::kPointwise && Cin <= 64 && Cout >= 96 && outs >= (1 << 22));
+    if (x_dtype == SNNF_F32) {
+        if (one && family == DenseFamily::kMatrixWhole)
+            return strided ? (T <= 2 ? tile_use <= 0.4 : T > 4 || outs <= (3 << 21)) : T > 2 || outs <= (3 << 20);
+        if (one && strided && family == DenseFamily::kMatrixMasked) return T > 2 || outs <= (1 << 20);
+        return !(family == DenseFamily::kPointwise && Cin <= 64 && Cout >= 96 && outs >= (1 << 22));
+    }
     const bool deep = K >= 4608 || (K >= 2304 && out <= (1 << 19) && !residual);
     if (!neuron) {
         if (pointwise) return false;
