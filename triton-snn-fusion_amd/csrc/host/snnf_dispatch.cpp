@@ -336,12 +336,13 @@ struct WorkMembrane {
     const void* from;
     WorkMembrane(const Tensor& x, const Membrane& m, at::IntArrayRef shape, bool wide) : out(empty(shape, m.dtype, x)), from(data_or_null(m.from)) {
         work = out;
-        if (wide) {
-            work = empty(shape, at::kFloat, x);
-            if (m.from) {
-                start = m.from->to(at::kFloat);
-                from = start.data_ptr();
-            }
+        if (wide) widen(x, m, shape);
+    }
+    void widen(const Tensor& x, const Membrane& m, at::IntArrayRef shape) {
+        work = empty(shape, at::kFloat, x);
+        if (m.from) {
+            start = m.from->to(at::kFloat);
+            from = start.data_ptr();
         }
     }
     int code() const { return code_of(work.scalar_type()); }
@@ -443,6 +444,18 @@ bool one_frame(const void* const* steps, int64_t T) {
     for (int64_t t = 1; t < T; ++t)
         if (steps[t] != steps[0]) return false;
     return T > 1;
+}
+
+// Scratch memory of a convolution from the pool of the current stream; none where the allocator has none left: such a call runs on the dense
+// kernels. (A DataPtr, not a tensor: that costs another microsecond.)
+c10::DataPtr scratch_memory(const Tensor& like, size_t bytes) {
+    if (bytes == 0) return {};
+    const c10::DeviceGuard guard(like.device());
+    try {
+        return c10::GetAllocator(c10::kCUDA)->allocate(bytes);
+    } catch (const c10::OutOfMemoryError&) {
+        return {};
+    }
 }
 
 bool scan_call(const Call& c, Attempt& key, Pair* out) {
@@ -649,9 +662,9 @@ bool conv_call(const Call& c, Attempt& key, Op op, Pair* out) {
                                            v_code, residual ? 1 : 0);
     };
     // With scratch memory the library keeps a 16-bit membrane wide between its launches by itself.
+    const bool narrow = m.dtype != at::kFloat && T > (depthwise ? SNNF_MAX_T_PER_LAUNCH : 1);
     size_t bytes = scratch_bytes(code_of(m.dtype));
-    const bool wide = bytes == 0 && m.dtype != at::kFloat && T > (depthwise ? SNNF_MAX_T_PER_LAUNCH : 1);
-    WorkMembrane wm(x, m, shape, wide);
+    WorkMembrane wm(x, m, shape, narrow && bytes == 0);
     int status;
     if (depthwise) {
         status = snnf_dwconv3x3_lif(steps, residuals, static_cast<int>(T), N, cin, H, W, static_cast<int>(sh), code_of(x.scalar_type()), w.data_ptr(),
@@ -659,11 +672,10 @@ bool conv_call(const Call& c, Attempt& key, Op op, Pair* out) {
                                     static_cast<float>(lif.v_threshold), static_cast<float>(lif.v_reset), static_cast<float>(lif.tau), stream);
     } else {
         const Tensor packed = packed_weight(w, b, x.scalar_type());
-        if (wide) bytes = scratch_bytes(wm.code());
-        c10::DataPtr workspace;            // (a tensor around it costs another microsecond)
-        if (bytes > 0) {
-            const c10::DeviceGuard guard(x.device());
-            workspace = c10::GetAllocator(c10::kCUDA)->allocate(bytes);
+        const c10::DataPtr workspace = scratch_memory(x, bytes);
+        if (bytes > 0 && !workspace) {
+            bytes = 0;
+            if (narrow) wm.widen(x, m, shape);
         }
         status = snnf_conv_lif_ws(steps, residuals, static_cast<int>(T), N, cin, H, W, code_of(x.scalar_type()), packed.data_ptr(),
                                   static_cast<int>(shape[1]), static_cast<int>(kh), static_cast<int>(kw), static_cast<int>(sh), static_cast<int>(sw),
@@ -1119,16 +1131,16 @@ PyObject* dense_conv_bias(Args& a) {
     const bool ran = unlocked([&] {
         const Tensor packed = packed_weight(*w, *b, x->scalar_type());
         out = empty({T, N, cout, ho, wo}, x->scalar_type(), *x);
-        const size_t bytes = snnf_conv_bias_workspace_bytes(static_cast<int>(T), static_cast<int>(N), static_cast<int>(x->size(2)), static_cast<int>(H),
-                                                            static_cast<int>(W), code_of(x->scalar_type()), static_cast<int>(cout), static_cast<int>(kh),
-                                                            static_cast<int>(kw), static_cast<int>(sh), static_cast<int>(sw), static_cast<int>(ph),
-                                                            static_cast<int>(pw), 0);
-        Tensor workspace;
-        if (bytes > 0) workspace = empty({static_cast<int64_t>(bytes)}, at::kByte, *x);
+        size_t bytes = snnf_conv_bias_workspace_bytes(static_cast<int>(T), static_cast<int>(N), static_cast<int>(x->size(2)), static_cast<int>(H),
+                                                      static_cast<int>(W), code_of(x->scalar_type()), static_cast<int>(cout), static_cast<int>(kh),
+                                                      static_cast<int>(kw), static_cast<int>(sh), static_cast<int>(sw), static_cast<int>(ph),
+                                                      static_cast<int>(pw), 0);
+        const c10::DataPtr workspace = scratch_memory(*x, bytes);
+        if (!workspace) bytes = 0;
         return snnf_conv_bias_ws(steps, nullptr, static_cast<int>(T), static_cast<int>(N), static_cast<int>(x->size(2)), static_cast<int>(H), static_cast<int>(W),
                                  code_of(x->scalar_type()), packed.data_ptr(), static_cast<int>(cout), static_cast<int>(kh), static_cast<int>(kw),
                                  static_cast<int>(sh), static_cast<int>(sw), static_cast<int>(ph), static_cast<int>(pw), out.data_ptr(), out.stride(0),
-                                 bytes > 0 ? workspace.data_ptr() : nullptr, bytes, stream_of(*x)) == 0;
+                                 workspace.get(), bytes, stream_of(*x)) == 0;
     });
     return ran ? THPVariable_Wrap(out) : none();
 }

@@ -357,9 +357,22 @@ def _scratch_bytes(pointers, first: torch.Tensor, weight, stride, padding, v_cod
                                                       *_as_pair(padding), v_code, 1 if residual else 0))
 
 
+def _scratch_memory(nbytes: int, device) -> Optional[torch.Tensor]:
+    """Scratch memory of a convolution (the caching allocator hands the block out again in the order of the stream the kernels run on), or
+    None where there is none left: such a call runs on the dense kernels, which need none."""
+    if not nbytes:
+        return None
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
+
+
 def _launch(kernel_key: str, steps: Sequence[torch.Tensor], residuals: Optional[Sequence[torch.Tensor]], weight, bias,
-            v_init, stride, padding, v_threshold, v_reset, tau, spikes: torch.Tensor, v_out: torch.Tensor) -> None:
-    """Enqueues the HIP kernel(s) for one fused conv+LIF call. `steps` are T contiguous [N, C, H, W] tensors."""
+            v_init, stride, padding, v_threshold, v_reset, tau, spikes: torch.Tensor, v_out: torch.Tensor,
+            workspace: Optional[torch.Tensor]) -> None:
+    """Enqueues the HIP kernel(s) for one fused conv+LIF call. `steps` are T contiguous [N, C, H, W] tensors. `workspace`: scratch memory for
+    the inputs in the channel-blocked layout, where the library asks for it."""
     lib = _lib.lib()
     first = steps[0]
     T = len(steps)
@@ -383,14 +396,10 @@ def _launch(kernel_key: str, steps: Sequence[torch.Tensor], residuals: Optional[
             float(v_threshold), float(v_reset), float(tau), stream))
     else:
         packed = _packed_weight(weight, bias, first.dtype)
-        # Scratch for the inputs in the channel-blocked layout where the library asks for it; the caching allocator hands the block out
-        # again in the order of the stream the kernels run on.
-        nbytes = _scratch_bytes(xs, first, weight, (sh, sw), (ph, pw), v_code, rs is not None)
-        workspace = torch.empty(nbytes, dtype=torch.uint8, device=first.device) if nbytes else None
         _lib.check("snnf_conv_lif", lib.snnf_conv_lif_ws(
             xs, rs, T, n, cin, h, w, x_code, packed.data_ptr(), cout, kh, kw, sh, sw, ph, pw,
             _lib.ptr(vi), v_code, spikes.data_ptr(), step_stride, v_out.data_ptr(),
-            float(v_threshold), float(v_reset), float(tau), _lib.ptr(workspace), nbytes, stream))
+            float(v_threshold), float(v_reset), float(tau), _lib.ptr(workspace), 0 if workspace is None else workspace.numel(), stream))
 
 
 def run_hip_temporal_conv_bias(xs: Sequence[torch.Tensor], weight, bias, stride, padding,
@@ -426,11 +435,11 @@ def run_hip_temporal_conv_bias(xs: Sequence[torch.Tensor], weight, bias, stride,
     nbytes = 0
     if not _one_frame(pointers):
         nbytes = int(lib.snnf_conv_bias_workspace_bytes(T, n, cin, h, w, x_code, cout, kh, kw, sh, sw, ph, pw, 1 if res is not None else 0))
-    workspace = torch.empty(nbytes, dtype=torch.uint8, device=first.device) if nbytes else None
+    workspace = _scratch_memory(nbytes, first.device)
     _lib.check("snnf_conv_bias", lib.snnf_conv_bias_ws(
         pointers, _lib.step_pointers(res) if res is not None else None, T, n, cin, h, w,
         x_code, packed.data_ptr(), cout, kh, kw, sh, sw, ph, pw,
-        out.data_ptr(), int(out.stride(0)), _lib.ptr(workspace), nbytes, _lib.current_stream(first.device)))
+        out.data_ptr(), int(out.stride(0)), _lib.ptr(workspace), 0 if workspace is None else workspace.numel(), _lib.current_stream(first.device)))
     return out
 
 
@@ -504,13 +513,15 @@ def _run_temporal(kind: str, xs, residuals, weight, bias, v_init, stride, paddin
     # membrane dtype itself (their one-launch variant needs a float32 membrane), so every multi-step call with a 16-bit
     # membrane computes with a float32 working membrane and rounds the result once: the same arithmetic on every call. With scratch memory
     # the library does so by itself.
-    wide = v_dtype != torch.float32 and T > 1 and _takes_several_launches(kernel_key, T)
-    if wide and not kernel_key.startswith("depthwise_"):
-        wide = _scratch_bytes(_lib.step_pointers(steps), first, weight, stride, padding, _lib.dtype_code(v_dtype), res is not None) == 0
+    workspace = None
+    if not kernel_key.startswith("depthwise_"):
+        workspace = _scratch_memory(_scratch_bytes(_lib.step_pointers(steps), first, weight, stride, padding, _lib.dtype_code(v_dtype), res is not None),
+                                    first.device)
+    wide = v_dtype != torch.float32 and T > 1 and _takes_several_launches(kernel_key, T) and workspace is None
     v_work = torch.empty(out_shape, dtype=torch.float32, device=first.device) if wide else v_next
     if wide and isinstance(v_init, torch.Tensor) and v_init.dim() > 0:
         v_init = v_init.float()
-    _launch(kernel_key, steps, res, weight, bias, v_init, stride, padding, v_threshold, v_reset, tau, spikes, v_work)
+    _launch(kernel_key, steps, res, weight, bias, v_init, stride, padding, v_threshold, v_reset, tau, spikes, v_work, workspace)
     if wide:
         v_next.copy_(v_work)
     diagnostics = kernel_dtype_diagnostics(first.dtype)
