@@ -150,7 +150,7 @@ int snnf_pwconv_lif_rowbits(const void* const* xs_bits, int T, int N, int Cin, i
  * C * H * W % 8 == 0, 16-byte aligned operands) run as ONE launch: a workgroup owns a sample and a range of classes, counts the
  * sample's spikes per channel in LDS and multiplies its weight rows with them; the workspace is then not touched.
  * snnf_lif_pool_linear_launches() says which of the two forms a shape takes (1 or 2; 0 for invalid extents), assuming
- * aligned operands.
+ * aligned operands and a v_out that is not v_init (in place, a sample whose classes take several workgroups takes two launches).
  */
 size_t snnf_lif_pool_linear_workspace_bytes(int N, int C);
 int snnf_lif_pool_linear_launches(int T, int N, int C, int H, int W, int K);

@@ -705,7 +705,9 @@ int lif_pool_linear_impl(const char* who, const void* const* xs, int T, int N, i
     {
         bool aligned = aligned_to(v_out, 16) && (v_init == nullptr || aligned_to(v_init, 16)) && aligned_to(fc_weight, 16);
         for (int t = 0; t < T; ++t) aligned = aligned && aligned_to(xs[t], 16);
-        const int class_blocks = aligned ? one_launch_class_blocks(T, N, C, HW, K) : 0;
+        int class_blocks = aligned ? one_launch_class_blocks(T, N, C, HW, K) : 0;
+        // All class ranges of a sample read its initial membrane and the first one stores the final one: not in the same memory.
+        if (class_blocks > 1 && v_init == v_out) class_blocks = 0;
         if (class_blocks > 0) {
             const dim3 grid(class_blocks, N);
             const int per_block = (K + class_blocks - 1) / class_blocks;
