@@ -422,6 +422,16 @@ def test_scratch_is_asked_for_only_where_it_is_used(snnf_lib, shape, asked):
     assert snnf_lib.snnf_conv_bias_workspace_bytes(4, 16, 512, 7, 7, _lib.SNNF_BF16, 512, 3, 3, 1, 1, 1, 1, 0) == 4 * 16 * 64 * 49 * 16
 
 
+def test_kernels_make_no_promise_that_membranes_are_apart():
+    """The header lets v_out be v_init, and a call of several windows reads what it stored in v_out: a kernel that declares such a pointer
+    __restrict__ allows the compiler to move the one's loads across the other's stores."""
+    csrc = os.path.join(ROOT, "triton-snn-fusion_amd", "csrc")
+    sources = {name: open(os.path.join(csrc, name)).read() for name in sorted(os.listdir(csrc)) if name.endswith((".h", ".hip"))}
+    assert sum(len(re.findall(r"\*\s*v_out\w*[,)]", text)) for text in sources.values()) > 10
+    for name, text in sources.items():
+        assert not re.search(r"__restrict__\s+v_(init|out|carry)\w*", text), name
+
+
 @pytest.mark.parametrize("T,N,Cin", [(16, 1 << 15, 4096), (16, 1 << 17, 1024), (8, 3 << 16, 1400), (4, 1 << 17, 4096)])
 def test_sizes_beyond_31_bits_do_not_wrap_in_the_rule(snnf_lib, T, N, Cin):
     """Strided 1x1 layers move up to 2^24 inputs; these have 2^31 or more (their product as an int wraps to zero or below)."""

@@ -45,8 +45,8 @@ __global__ __launch_bounds__(kConvThreads) void conv_lif_kernel(const StepPtrs x
                                                                 const int has_residual, const ConvGeom g,
                                                                 const uint16_t* __restrict__ wpacked,
                                                                 const float* __restrict__ bias,
-                                                                const void* __restrict__ v_init,
-                                                                XT* __restrict__ spikes, void* __restrict__ v_out,
+                                                                const void* v_init,
+                                                                XT* __restrict__ spikes, void* v_out,
                                                                 const LifParams lif) {
     extern __shared__ __align__(16) unsigned char lds[];
     constexpr bool F16 = dtype_of<XT>::value == SNNF_F16;

@@ -49,8 +49,8 @@ __device__ __forceinline__ int mm_div(int n, const FastDiv& f) {
 template <typename XT, int TT, int LM, bool FAST, bool SK, int NW, bool STAGED = false>
 __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void conv_mm_lif_kernel(
     const StepPtrs xs, const StepPtrs residuals, const int has_residual, const ConvGeom g,
-    const uint16_t* __restrict__ wpacked, const float* __restrict__ bias, const void* __restrict__ v_init,
-    XT* __restrict__ spikes, void* __restrict__ v_out, const LifParams lif) {
+    const uint16_t* __restrict__ wpacked, const float* __restrict__ bias, const void* v_init,
+    XT* __restrict__ spikes, void* v_out, const LifParams lif) {
     extern __shared__ __align__(16) unsigned char lds[];
     constexpr bool F16 = dtype_of<XT>::value == SNNF_F16;
     constexpr bool SPIKES = FAST && sizeof(XT) == 2 && !STAGED;   // the epilogue of 16-bit spikes

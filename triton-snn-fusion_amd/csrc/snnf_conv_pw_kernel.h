@@ -80,8 +80,8 @@ __global__ __launch_bounds__(kConvThreads, 2) __attribute__((amdgpu_waves_per_eu
                                                                       const int has_residual, const ConvGeom g,
                                                                       const uint16_t* __restrict__ wpacked,
                                                                       const float* __restrict__ bias,
-                                                                      const void* __restrict__ v_init,
-                                                                      XT* __restrict__ spikes, void* __restrict__ v_out,
+                                                                      const void* v_init,
+                                                                      XT* __restrict__ spikes, void* v_out,
                                                                       const LifParams lif) {
     extern __shared__ __align__(16) unsigned char lds[];
     static_assert(!DIRECT || (FAST && STD && sizeof(XT) == 2), "the accumulator-layout LIF step is for the fast variant on 16-bit activations");

@@ -430,7 +430,7 @@ Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, 
     if (route.taken) {
         const auto kept = std::make_shared<KeptPlan>();
         BlockedPlan& plan = kept->plan;
-        route.taken = plan_blocked("snnf_conv_lif_workspace_bytes", BlockedCall{T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, SNNF_LAYOUT_C8,
+        route.taken = plan_blocked("snnf_conv_lif_scratch_bytes", BlockedCall{T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, SNNF_LAYOUT_C8,
                                    residual ? SNNF_LAYOUT_NCHW : -1, SNNF_LAYOUT_NCHW, 0, false, neuron, false, neuron, false, nullptr, split}, plan) == SNNF_OK;
         if (route.taken) {
             for (int dense_epi = 0; dense_epi < 2; ++dense_epi) plan_text(kept->text[dense_epi], plan, family_name(route.family), dense_epi ? 40 : 0, plan.tt, true);
@@ -683,13 +683,13 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     L.g.out_step_stride = out_step_stride;
     L.wpacked = static_cast<const uint16_t*>(packed_weight);
     L.bias = reinterpret_cast<const float*>(L.wpacked + packed_weight_elems(p.pg));
-    L.v_init = neuron ? v_init : nullptr;
+    L.g.v_in_place = neuron && v_init != nullptr && v_init == v_out ? 1 : 0;
+    L.v_start = neuron && L.g.v_in_place == 0 ? v_init : nullptr;
     L.out = out;
-    L.v_out = neuron ? v_out : nullptr;
-    L.v_carry = static_cast<float*>(L.v_out);
+    L.v_store = neuron ? v_out : nullptr;
     if (dense != nullptr && neuron && dense->v_dtype != SNNF_F32) {
         L.g.v16 = 1;
-        L.v_carry = reinterpret_cast<float*>(static_cast<char*>(const_cast<void*>(xs[0])) + dense->space.carry);
+        L.v_scratch = reinterpret_cast<float*>(static_cast<char*>(const_cast<void*>(xs[0])) + dense->space.carry);
     }
     L.lif = make_lif_params(v_threshold, v_reset, tau);
     L.grid = p.grid;
@@ -701,7 +701,7 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
                           v_init == nullptr && (p.windows == 1 || p.tt == 4) && Cout % 8 == 0;
     // Dense tensors around the neuron: no range limit on the threshold, any reset potential, initial membrane, windows and channels.
     const bool dense_epi = neuron && x_layout == SNNF_LAYOUT_C8 && out_layout == SNNF_LAYOUT_NCHW && (residuals == nullptr || res_layout == SNNF_LAYOUT_NCHW) &&
-                           L.lif.charge_mode == CHARGE_SCALE && L.lif.inv_tau == 0.5f && !L.lif.soft_reset && L.v_out != nullptr && !shared;
+                           L.lif.charge_mode == CHARGE_SCALE && L.lif.inv_tau == 0.5f && !L.lif.soft_reset && L.v_store != nullptr && !shared;
     if (dense != nullptr) memcpy(snnf::conv_plan_buffer(), dense->kept->text[dense_epi ? 1 : 0], 256);
     else plan_text(snnf::conv_plan_buffer(), p, "blocked", fast_epi ? 20 : (dense_epi ? 40 : 0), shared ? T : p.tt, false);
     L.fast_epilogue = fast_epi;

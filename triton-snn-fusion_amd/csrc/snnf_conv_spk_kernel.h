@@ -86,7 +86,8 @@ struct SpkGeom {
     // `w_lo_offset` elements behind. One byte per 64 items of the C8 tensor tells whether any of them has a low term; only those are written.
     int64_t lo_offset, w_lo_offset;
     int64_t flag_stride;         // bytes of the flags of one timestep (a multiple of 4)
-    int v16;                     // v_init and v_out hold the activation dtype; the windows in between pass v_carry on
+    int v16;                     // v_start and v_store hold the activation dtype; the windows in between pass v_scratch on
+    int v_in_place;              // the initial membrane lies in v_store
     FastDiv d_ppx, d_PC, d_region, d_rrrc, d_RC, d_n_patches, d_patches_img, d_patches_x, d_gpc, d_hg, d_nst, d_KW;
 };
 
@@ -96,10 +97,10 @@ struct SpkLaunch {
     SpkGeom g;
     const uint16_t* wpacked;
     const float* bias;
-    const void* v_init;
+    const void* v_start;        // initial membrane (null: zero, or in v_store: see SpkGeom::v_in_place)
     void* out;
-    void* v_out;
-    float* v_carry;             // the membrane between the windows of a call (v_out itself where that is fp32)
+    void* v_store;              // final membrane, and fp32 ones between the windows of a call
+    float* v_scratch;           // those of a call with a 16-bit membrane, else null
     LifParams lif;
     const uint16_t* wpacked2;   // packed weight and bias of the shortcut (sc_stages > 0), else null
     const float* bias2;
@@ -165,16 +166,16 @@ __device__ __forceinline__ sk_u32x4 sk_expand_bits(uint32_t byte) {
 template <typename XT, int TT, int IN, bool SK, bool FAST, bool SC = false, bool POOL = false, bool NARROW = false, bool DENSE = false, bool MULTI = false>
 __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_eu(TT == 1 ? 4 : 2, TT == 1 ? 4 : 2))) void conv_spk_kernel(
     const StepPtrs xs, const StepPtrs residuals, const SpkGeom g, const uint16_t* __restrict__ wpacked,
-    const float* __restrict__ bias, const void* __restrict__ v_init, unsigned char* __restrict__ out,
-    void* __restrict__ v_out_any, const LifParams lif, const uint16_t* __restrict__ wpacked2, const float* __restrict__ bias2,
-    float* v_carry, const unsigned char* __restrict__ lo_flags) {
+    const float* __restrict__ bias, const void* __restrict__ v_start, unsigned char* __restrict__ out,
+    void* __restrict__ v_store, const LifParams lif, const uint16_t* __restrict__ wpacked2, const float* __restrict__ bias2,
+    float* __restrict__ v_scratch, const unsigned char* __restrict__ lo_flags) {
     extern __shared__ __align__(16) unsigned char lds[];
     // ---- every cache line of the kernel arguments is touched once, in one round trip: the compiler loads the arguments
     // where they are used, all over the prologue, and each of those loads then hits the scalar cache instead of waiting
     // for memory in turn.
     {
         auto ka = __builtin_amdgcn_kernarg_segment_ptr();
-        // The explicit arguments are two step tables, the geometry, five pointers and the neuron: the last dword that is
+        // The explicit arguments are two step tables, the geometry, nine pointers and the neuron: the last dword that is
         // touched must lie inside them (what follows is the hidden-argument area, which the compiler may leave out).
         constexpr size_t kExplicitArgBytes = 2 * sizeof(StepPtrs) + sizeof(SpkGeom) + 9 * sizeof(void*) + sizeof(LifParams);
         static_assert(0x2c0 + 4 <= kExplicitArgBytes, "argument prefetch reads past the explicit kernel arguments");
@@ -197,7 +198,11 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
     static_assert(!SPLIT || (NARROW && IN == SNNF_LAYOUT_C8 && !FAST && !SC && !POOL), "fp32 tensors: narrow tiles on two C8 tensors, dense tensors out");
     static_assert(!MULTI || (FAST && !POOL), "several windows belong to the straight-line epilogue");
     static_assert(!DENSE || (IN == SNNF_LAYOUT_C8 && !FAST && !SC && !POOL), "the dense epilogue belongs to calls on dense tensors");
-    float* const v_out = static_cast<float*>(v_out_any);
+    // No two of the membrane arguments are the same memory: a call in place passes no v_start, and only one with a 16-bit membrane has a
+    // v_scratch. (Promising nothing here instead cost the straight-line epilogue 2 %: ResNet-18, 16 images of 224x224 361 -> 369 us.)
+    float* const v_out = static_cast<float*>(v_store);
+    const void* const v_init = g.v_in_place ? v_store : v_start;
+    float* const v_carry = g.v16 ? v_scratch : v_out;
     constexpr int NF = NARROW ? 1 : 2;         // 32-channel weight fragments of a tile
     constexpr int TG = 4 * NF;                 // channel groups of 8 of a tile
     constexpr bool F16 = dtype_of<XT>::value == SNNF_F16;
@@ -738,7 +743,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             }
             const bool first_window = t0 == 0, last_window = t0 + TT >= nsteps_t;
             const void* v_src = first_window ? v_init : v_carry;          // later windows continue from the stored membrane
-            void* const v_dst = last_window ? v_out_any : v_carry;
+            void* const v_dst = last_window ? v_store : v_carry;
             const bool v_src16 = !SPLIT && g.v16 && first_window, v_dst16 = !SPLIT && g.v16 && last_window;
             const int t_count = g.shared_x ? g.T : min(TT, g.T - t0);      // LIF steps of this window
             // (Made opaque here: everything derived from the lane's pixel offset is then computed after the matrix loop instead of
@@ -1504,8 +1509,8 @@ template <typename XT, int TT, int IN>
 int launch_conv_spk_variant(const SpkLaunch& L) {
     auto run = [&](auto kernel) -> int {
         if (const int rc = reserve_lds(reinterpret_cast<const void*>(kernel), L.lds_bytes, "snnf_conv_lif_blocked"); rc != SNNF_OK) return rc;
-        kernel<<<dim3(L.grid), kSpkWaves * 64, L.lds_bytes, L.stream>>>(L.xs, L.residuals, L.g, L.wpacked, L.bias, L.v_init,
-                                                                        static_cast<unsigned char*>(L.out), L.v_out, L.lif, L.wpacked2, L.bias2, L.v_carry, L.lo_flags);
+        kernel<<<dim3(L.grid), kSpkWaves * 64, L.lds_bytes, L.stream>>>(L.xs, L.residuals, L.g, L.wpacked, L.bias, L.v_start,
+                                                                        static_cast<unsigned char*>(L.out), L.v_store, L.lif, L.wpacked2, L.bias2, L.v_scratch, L.lo_flags);
         return check_launch("snnf_conv_lif_blocked");
     };
     if constexpr (IN == SNNF_LAYOUT_C8) {
@@ -1533,8 +1538,8 @@ template <int TT>
 int launch_conv_spk_split(const SpkLaunch& L) {
     auto run = [&](auto kernel) -> int {
         if (const int rc = reserve_lds(reinterpret_cast<const void*>(kernel), L.lds_bytes, "snnf_conv_lif"); rc != SNNF_OK) return rc;
-        kernel<<<dim3(L.grid), kSpkWaves * 64, L.lds_bytes, L.stream>>>(L.xs, L.residuals, L.g, L.wpacked, L.bias, L.v_init,
-                                                                        static_cast<unsigned char*>(L.out), L.v_out, L.lif, L.wpacked2, L.bias2, L.v_carry, L.lo_flags);
+        kernel<<<dim3(L.grid), kSpkWaves * 64, L.lds_bytes, L.stream>>>(L.xs, L.residuals, L.g, L.wpacked, L.bias, L.v_start,
+                                                                        static_cast<unsigned char*>(L.out), L.v_store, L.lif, L.wpacked2, L.bias2, L.v_scratch, L.lo_flags);
         return check_launch("snnf_conv_lif");
     };
     constexpr int C = SNNF_LAYOUT_C8;
@@ -1547,8 +1552,8 @@ template <typename XT, int IN>
 int launch_conv_spk_pooled(const SpkLaunch& L, int tt) {
     auto run = [&](auto kernel) -> int {
         if (const int rc = reserve_lds(reinterpret_cast<const void*>(kernel), L.lds_bytes, "snnf_conv_lif_blocked_avgpool"); rc != SNNF_OK) return rc;
-        kernel<<<dim3(L.grid), kSpkWaves * 64, L.lds_bytes, L.stream>>>(L.xs, L.residuals, L.g, L.wpacked, L.bias, L.v_init,
-                                                                        static_cast<unsigned char*>(L.out), L.v_out, L.lif, L.wpacked2, L.bias2, L.v_carry, L.lo_flags);
+        kernel<<<dim3(L.grid), kSpkWaves * 64, L.lds_bytes, L.stream>>>(L.xs, L.residuals, L.g, L.wpacked, L.bias, L.v_start,
+                                                                        static_cast<unsigned char*>(L.out), L.v_store, L.lif, L.wpacked2, L.bias2, L.v_scratch, L.lo_flags);
         return check_launch("snnf_conv_lif_blocked_avgpool");
     };
     if (tt == 4 && L.g.narrow) return run(conv_spk_kernel<XT, 4, IN, true, true, false, true, true>);
@@ -1561,8 +1566,8 @@ template <typename XT>
 int launch_conv_spk_frame(const SpkLaunch& L, bool pooled) {
     auto run = [&](auto kernel) -> int {
         if (const int rc = reserve_lds(reinterpret_cast<const void*>(kernel), L.lds_bytes, "snnf_conv_lif_blocked"); rc != SNNF_OK) return rc;
-        kernel<<<dim3(L.grid), kSpkWaves * 64, L.lds_bytes, L.stream>>>(L.xs, L.residuals, L.g, L.wpacked, L.bias, L.v_init,
-                                                                        static_cast<unsigned char*>(L.out), L.v_out, L.lif, L.wpacked2, L.bias2, L.v_carry, L.lo_flags);
+        kernel<<<dim3(L.grid), kSpkWaves * 64, L.lds_bytes, L.stream>>>(L.xs, L.residuals, L.g, L.wpacked, L.bias, L.v_start,
+                                                                        static_cast<unsigned char*>(L.out), L.v_store, L.lif, L.wpacked2, L.bias2, L.v_scratch, L.lo_flags);
         return check_launch("snnf_conv_lif_blocked");
     };
     constexpr int D = SNNF_LAYOUT_NCHW;
@@ -1580,8 +1585,8 @@ template <typename XT>
 int launch_conv_spk_shortcut(const SpkLaunch& L) {
     auto run = [&](auto kernel) -> int {
         if (const int rc = reserve_lds(reinterpret_cast<const void*>(kernel), L.lds_bytes, "snnf_conv_lif_blocked_shortcut"); rc != SNNF_OK) return rc;
-        kernel<<<dim3(L.grid), kSpkWaves * 64, L.lds_bytes, L.stream>>>(L.xs, L.residuals, L.g, L.wpacked, L.bias, L.v_init,
-                                                                        static_cast<unsigned char*>(L.out), L.v_out, L.lif, L.wpacked2, L.bias2, L.v_carry, L.lo_flags);
+        kernel<<<dim3(L.grid), kSpkWaves * 64, L.lds_bytes, L.stream>>>(L.xs, L.residuals, L.g, L.wpacked, L.bias, L.v_start,
+                                                                        static_cast<unsigned char*>(L.out), L.v_store, L.lif, L.wpacked2, L.bias2, L.v_scratch, L.lo_flags);
         return check_launch("snnf_conv_lif_blocked_shortcut");
     };
     constexpr int B = SNNF_LAYOUT_BITS;

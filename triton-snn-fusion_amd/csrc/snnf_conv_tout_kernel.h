@@ -35,9 +35,9 @@ __global__ __launch_bounds__(kConvThreads, 2) void conv_lif_tout_kernel(const St
                                                                         const int has_residual, const ConvGeom g,
                                                                         const uint16_t* __restrict__ wpacked,
                                                                         const float* __restrict__ bias,
-                                                                        const void* __restrict__ v_init,
+                                                                        const void* v_init,
                                                                         XT* __restrict__ spikes,
-                                                                        void* __restrict__ v_out, const LifParams lif) {
+                                                                        void* v_out, const LifParams lif) {
     extern __shared__ __align__(16) unsigned char lds[];
     constexpr bool F16 = dtype_of<XT>::value == SNNF_F16;
     constexpr int RPE = LM == LOAD_PAIR32 ? 1 : 2;

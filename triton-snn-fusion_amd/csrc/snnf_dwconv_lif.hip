@@ -58,9 +58,9 @@ template <typename XT, typename VT, int STRIDE, int PX, bool STD>
 __global__ __launch_bounds__(kThreads) void dwconv3x3_lif_kernel(StepPtrs xs, StepPtrs residuals, int has_residual,
                                                                  int T, DwGeom g, const XT* __restrict__ weight,
                                                                  const XT* __restrict__ bias,
-                                                                 const VT* __restrict__ v_init,
+                                                                 const VT* v_init,
                                                                  XT* __restrict__ spikes, int64_t spike_step_stride,
-                                                                 VT* __restrict__ v_out, LifParams lif) {
+                                                                 VT* v_out, LifParams lif) {
     extern __shared__ __align__(16) float tile[];
     constexpr bool BITS = false;                       // dense 0 / 1 spikes only (the packed output is the dot-product kernel's)
     constexpr int IN_COLS = (PX - 1) * STRIDE + 3;
@@ -332,9 +332,9 @@ template <typename XT, typename VT, bool STD, bool BITS = false, bool BITS_IN = 
 __global__ __launch_bounds__(kThreads) void dwconv3x3_lif_dot_kernel(StepPtrs xs, StepPtrs residuals, int has_residual,
                                                                      int T, DwGeom g, const XT* __restrict__ weight,
                                                                      const XT* __restrict__ bias,
-                                                                     const VT* __restrict__ v_init,
+                                                                     const VT* v_init,
                                                                      XT* __restrict__ spikes, int64_t spike_step_stride,
-                                                                     VT* __restrict__ v_out, LifParams lif) {
+                                                                     VT* v_out, LifParams lif) {
     extern __shared__ __align__(16) unsigned char dot_tile_bytes[];
     uint16_t* __restrict__ tile = reinterpret_cast<uint16_t*>(dot_tile_bytes);
     constexpr int PX = 8;

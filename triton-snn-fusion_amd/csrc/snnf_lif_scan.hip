@@ -11,8 +11,8 @@ constexpr int kThreads = 256;
 // transaction, so a 64-lane wave moves 1 KiB per instruction.
 template <typename XT, typename VT, int VEC, int TC>
 __global__ __launch_bounds__(kThreads) void lif_scan_kernel(StepPtrs xs, int T, int64_t numel,
-                                                            const VT* __restrict__ v_init, XT* __restrict__ spikes,
-                                                            int64_t spike_step_stride, VT* __restrict__ v_out,
+                                                            const VT* v_init, XT* __restrict__ spikes,
+                                                            int64_t spike_step_stride, VT* v_out,
                                                             LifParams lif) {
     const int64_t first = (static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x) * VEC;
     if (first >= numel) return;

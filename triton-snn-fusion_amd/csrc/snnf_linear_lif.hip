@@ -146,8 +146,8 @@ template <int TT> struct LinWaves { static constexpr int value = TT <= 8 ? 8 : 4
 template <typename XT, typename VT, int TT, bool FAST, int OCF>
 __global__ __launch_bounds__(LinWaves<TT>::value * 64) void linear_lif_kernel(StepPtrs xs, LinGeom g, const XT* __restrict__ W,
                                                                               const XT* __restrict__ bias,
-                                                                              const VT* __restrict__ v_init, XT* __restrict__ spikes,
-                                                                              VT* __restrict__ v_out, LifParams lif) {
+                                                                              const VT* v_init, XT* __restrict__ spikes,
+                                                                              VT* v_out, LifParams lif) {
     constexpr int NW = LinWaves<TT>::value;
     constexpr int TILE_OC = OCF * kTileOC;
     constexpr int OUTS = TILE_OC * kTileM;                    // outputs per workgroup and timestep
@@ -302,8 +302,8 @@ template <int TT, int OCF, int SLABK, int TM> struct StagedShape {
 template <typename XT, typename VT, int TT, int OCF, bool DB, int SLABK, int TM, bool XBITS = false, bool SBITS = false>
 __global__ __launch_bounds__(kStagedWaves * 64) void linear_lif_staged_kernel(StepPtrs xs, LinGeom g, const XT* __restrict__ W,
                                                                               const XT* __restrict__ bias,
-                                                                              const VT* __restrict__ v_init, XT* __restrict__ spikes,
-                                                                              VT* __restrict__ v_out, LifParams lif,
+                                                                              const VT* v_init, XT* __restrict__ spikes,
+                                                                              VT* v_out, LifParams lif,
                                                                               float* __restrict__ ws_partial, int* __restrict__ ws_count,
                                                                               int slabs_per_part) {
     using SH = StagedShape<TT, OCF, SLABK, TM>;

@@ -21,7 +21,7 @@ constexpr int kMaxPlanes = 1024;  // planes per workgroup (HW == 1 gives kThread
 
 template <typename XT, typename VT>
 __global__ __launch_bounds__(kThreads) void lif_pool_kernel(StepPtrs xs, int T, int planes, int HW, int planes_per_block,
-                                                            const VT* __restrict__ v_init, VT* __restrict__ v_out,
+                                                            const VT* v_init, VT* v_out,
                                                             int* __restrict__ counts, LifParams lif) {
     __shared__ int plane_count[kMaxPlanes];
     const int plane0 = blockIdx.x * planes_per_block;
@@ -80,7 +80,7 @@ constexpr int kVec = 8;
 
 template <typename XT, typename VT, int TC>
 __global__ __launch_bounds__(kThreads) void lif_pool_vec_kernel(StepPtrs xs, int T, int planes, int HW, int planes_per_block,
-                                                                const VT* __restrict__ v_init, VT* __restrict__ v_out,
+                                                                const VT* v_init, VT* v_out,
                                                                 int* __restrict__ counts, LifParams lif, int stream_out) {
     __shared__ int plane_count[kMaxPlanes];
     const int plane0 = blockIdx.x * planes_per_block;
@@ -431,7 +431,7 @@ __device__ __forceinline__ void classify_counts(const int* plane_count, int n, i
 
 template <typename XT, typename VT>
 __global__ __launch_bounds__(kThreads) void lif_pool_linear_one_kernel(StepPtrs xs, int T, int C, int HW, int K, int classes_per_block,
-                                                                       const VT* __restrict__ v_init, VT* __restrict__ v_out,
+                                                                       const VT* v_init, VT* v_out,
                                                                        const XT* __restrict__ Wt, const XT* __restrict__ bias,
                                                                        XT* __restrict__ out, LifParams lif, float inv_hw, float steps) {
     __shared__ __align__(16) int plane_count[kOneMaxC];
