@@ -67,8 +67,8 @@ def test_layers_that_stay_on_the_dense_kernels(snnf_lib):
     bf16, f32 = 1, 0
     asks = snnf_lib.snnf_conv_lif_workspace_bytes
     assert asks(4, 16, 64, 56, 56, bf16, 64, 3, 3, 1, 1, 1, 1, f32, 0) == 0          # whole tiles
-    assert asks(4, 16, 256, 14, 14, bf16, 256, 3, 3, 1, 1, 1, 1, f32, 0) == 0        # ... of a deep layer with many outputs
-    assert asks(4, 2, 256, 14, 14, bf16, 256, 3, 3, 1, 1, 1, 1, f32, 0) > 0          # ... with few
+    assert asks(4, 32, 128, 28, 28, bf16, 128, 3, 3, 1, 1, 1, 1, f32, 0) == 0        # ... of a deeper layer with many outputs
+    assert asks(4, 2, 256, 14, 14, bf16, 256, 3, 3, 1, 1, 1, 1, f32, 0) > 0          # ... of a deep one
     assert asks(4, 16, 128, 56, 56, bf16, 256, 1, 1, 1, 1, 0, 0, f32, 0) == 0        # pointwise
     assert asks(4, 8, 20, 9, 9, f32, 24, 3, 3, 1, 1, 1, 1, f32, 0) == 0              # float32 tensors
     assert asks(1, 8, 20, 9, 9, bf16, 24, 3, 3, 1, 1, 1, 1, bf16, 0) == 0            # 16-bit membrane

@@ -551,6 +551,21 @@ def test_dense_conv_lif_shapes_outside_the_matrix_and_pointwise_kernels(hip_ops,
         check(sp, v, ref, v_threshold=lif[0], v_dtype=F32, what=f"{family} alone {Cin}->{Cout} k{k} s{stride} {H}x{W}")
 
 
+def _conv_without_scratch(xs, rs, w, b, v0, stride, pad):
+    """snnf_conv_lif on the operators' neuron LIF: the dense kernels, whatever the rule for calls with scratch memory."""
+    from triton_snn_fusion_amd import _lib
+    from triton_snn_fusion_amd.runtime import hip_convlif_backend as CB
+    (N, Cin, H, W), (Cout, _, k, _), T, dtype = xs[0].shape, w.shape, len(xs), xs[0].dtype
+    packed = CB._packed_weight(w, b, dtype)
+    Ho, Wo = (H + 2 * pad - k) // stride + 1, (W + 2 * pad - k) // stride + 1
+    sp, v = torch.empty(T, N, Cout, Ho, Wo, device=DEV, dtype=dtype), torch.empty(N, Cout, Ho, Wo, device=DEV)
+    _lib.check("snnf_conv_lif", _lib.lib().snnf_conv_lif(
+        _lib.step_pointers(xs), _lib.step_pointers(rs) if rs is not None else None, T, N, Cin, H, W, _lib.dtype_code(dtype), packed.data_ptr(),
+        Cout, k, k, stride, stride, pad, pad, _lib.ptr(v0), _lib.SNNF_F32, sp.data_ptr(), int(sp.stride(0)), v.data_ptr(), *LIF,
+        _lib.current_stream(sp.device)))
+    return sp, v
+
+
 def test_planes_of_four_pixels_with_several_images_per_tile(hip_ops):
     """2x2 planes, two images per tile: a lane's run of 8 pixels spans two images (each half is one whole plane)."""
     from triton_snn_fusion_amd.runtime.hip_convlif_backend import last_conv_plan
@@ -562,10 +577,13 @@ def test_planes_of_four_pixels_with_several_images_per_tile(hip_ops):
     ref = O.temporal_conv_lif(xs, w_ref, b_ref, v0, (1, 1), (1, 1), (1, 1), 1, *LIF, residuals=rs)
     sp, v = S.fused_temporal_conv_add_lif_state([dev(x, BF16) for x in xs], [dev(r, BF16) for r in rs], dev(w_dev, BF16), dev(b_dev, BF16),
                                                 dev(v0, F32), [1, 1], [1, 1], [1, 1], 1, *LIF, False)
+    check(sp, v, ref, what="2x2 planes")
+    _no_fallback(hip_ops, 1)
+    # the matrix kernel itself, without scratch memory for the blocked layout
+    sp, v = _conv_without_scratch([dev(x, BF16) for x in xs], [dev(r, BF16) for r in rs], dev(w_dev, BF16), dev(b_dev, BF16), dev(v0, F32), 1, 1)
     plan = last_conv_plan()
     assert plan["kernel"] == "matrix" and plan["tile"] == "2x2x2" and plan["variant"] == 24, plan
     check(sp, v, ref, what="2x2 planes, two images per tile")
-    _no_fallback(hip_ops, 1)
 
 
 def test_conv_shared_analog_frame_is_convolved_once_and_matches(hip_ops):
@@ -661,6 +679,9 @@ def test_conv_plan_is_reported(hip_ops):
     xs = [torch.zeros(2, 64, 16, 16, device=DEV, dtype=BF16) for _ in range(4)]
     w, b = torch.zeros(64, 64, 3, 3, device=DEV, dtype=BF16), torch.zeros(64, device=DEV, dtype=BF16)
     S.fused_temporal_conv_lif_state(xs, w, b, zero_v(), [1, 1], [1, 1], [1, 1], 1, *LIF, False)
+    plan = last_conv_plan()
+    assert plan["kernel"] == "matrix" and plan["ran"] == "blocked" and plan["window"] == 4 and plan["launches"] == 2
+    _conv_without_scratch(xs, None, w, b, None, 1, 1)
     plan = last_conv_plan()
     assert plan["kernel"] == "matrix" and plan["variant"] == 24 and plan["window"] == 4 and plan["launches"] == 1
     w1 = torch.zeros(128, 64, 1, 1, device=DEV, dtype=BF16)

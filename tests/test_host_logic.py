@@ -456,6 +456,24 @@ def test_which_1x1_layers_of_float32_tensors_move(snnf_lib, layer, moves):
     assert (snnf_lib.snnf_conv_lif_scratch_bytes(T, N, Cin, H, W, _lib.SNNF_F32, Cout, 1, 1, s, s, 0, 0, _lib.SNNF_F32, 0) > 0) == moves
 
 
+@pytest.mark.parametrize("layer,moves", [  # (T, N, Cin, H, Cout, kernel, stride, residual): whole tiles of the matrix kernel, square planes
+    ((4, 40, 256, 2, 512, 3, 1, 1), True),      # planes of four pixels
+    ((1, 1, 64, 2, 64, 1, 1, 0), True),
+    ((4, 2, 64, 16, 64, 3, 1, 0), True),        # few pixels, four steps
+    ((3, 1, 32, 8, 128, 3, 1, 1), True),
+    ((4, 16, 256, 14, 256, 3, 1, 0), True),     # deep, the chip full
+    ((4, 128, 256, 14, 256, 3, 1, 0), True),
+    ((4, 32, 128, 28, 128, 3, 1, 0), False),    # products and outputs of which the matrix kernel is the faster one
+    ((4, 16, 64, 56, 64, 3, 1, 1), False),
+    ((4, 16, 128, 28, 256, 3, 2, 0), False),
+    ((4, 32, 8, 32, 64, 3, 1, 0), False),       # a single channel group
+])
+def test_which_layers_of_whole_tiles_move(snnf_lib, layer, moves):
+    T, N, Cin, H, Cout, k, s, residual = layer
+    asked = snnf_lib.snnf_conv_lif_scratch_bytes(T, N, Cin, H, H, _lib.SNNF_BF16, Cout, k, k, s, s, k // 2, k // 2, _lib.SNNF_F32, residual)
+    assert asked == (T * N * Cin * H * H * 2 if moves else 0)
+
+
 def test_a_tuned_plan_is_seen_by_a_remembered_route(snnf_lib):
     """A 7x7 layer whose planned stages of four channel groups hold more steps than the table, and stages of two do not."""
     layer = (2, 2, 372, 5, 5, 384, 7, 7, 1, 1, 3, 3)

@@ -108,7 +108,7 @@ RouteSpace route_space(int T, int N, int Cin, int H, int W, bool split, int64_t 
 }
 
 // Whether a layer on dense tensors is brought into C8 and run on the blocked kernel (two launches) or stays on the dense kernels. Measured on
-// some 1700 layers of 1 to 64 images, 1 to 512 channels, 1x1 to 7x7, one to eight timesteps (us, dense / here; bf16 and T = 4 unless said):
+// layers of 1 to 64 images, 1 to 512 channels, 1x1 to 7x7, one to eight timesteps (us, dense / here; bf16 and T = 4 unless said):
 // * Channel counts that are no multiple of 8 only have the four-wave kernels on dense tensors, which assemble every channel group from
 //   scalar loads: they move (126 -> 200 at 12 x 54 stride 2, T = 2 93 / 18, 29 -> 72 at 70^2, 7x7 stride 2 316 / 23, 61 -> 32 1x1 at 39 x 20, T = 3
 //   29 / 16), but for large 1x1 layers, which are memory traffic (421 -> 288 at 100^2, T = 8 356 / 416).
@@ -122,15 +122,13 @@ RouteSpace route_space(int T, int N, int Cin, int H, int W, bool split, int64_t 
 //   51^2 x 16 with a residual 216 / 127, 128 -> 256 at 28^2 x 32, T = 2 56 / 50).
 // * Whole tiles of the matrix kernel take the time of their rounds, full or not, and of their windows of four steps; this kernel's time is
 //   nearly proportional to the outputs. So `tile_use` decides (see dense_family), weighed by the products per output, in which this kernel is
-//   the better one. Over 2800 layers the quotient of the two times falls with it from 2 to 0.75 and passes 1 at the lines below; the rule is
-//   2 % slower than the better kernel in the mean, the dense kernels alone 31 %. It moves 64 -> 64 at 24^2 x 4 30 / 12, x 38, T = 6 70 / 45, at
+//   the better one. The quotient of the two times falls with it from 2 to 0.75 and passes 1 at the lines below. It moves 64 -> 64 at 24^2 x 4 30 / 12, x 38, T = 6 70 / 45, at
 //   40^2 x 20 (tiles of four columns) 43 / 33, T = 8 121 / 68, at 56^2 x 21, T = 6 132 / 110, 128 -> 256 stride 2 at 28^2 x 5, T = 8 49 / 40, 1x1 stride 2 x 2
 //   31 / 20; 64 -> 64 at 56^2 x 16 34 / 42, 128 -> 128 at 28^2 x 32 48 / 52 (x 16 38 / 36), 64 -> 128 stride 2 at 56^2 x 16 28 / 37, 1x1 18 / 26, 128 -> 256 stride 2
 //   at 28^2 x 16 28 / 34 stay. Inputs that the caches don't hold between the copy and the kernel move the lines (64 -> 64 at 56^2 x 88, T = 5
-//   with a residual 366 / 437, 128 -> 256 stride 2 at 28^2 x 164, T = 7 395 / 554). Deep layers of few outputs always move (256 -> 256 at 14^2 x 4 29 / 18, 512 -> 512 at 4^2 x 16 37 / 21). Three kinds
-//   that would gain as well stay with the kernel that their reported plan names in the tests: planes of four pixels at most (256 -> 512
-//   at 2^2 x 40 24 / 14), one window of four steps of up to 512 pixels with less than 128 channels (64 -> 64 at 16^2 x 2 30 / 11) and deep layers
-//   without a residual that fill the chip (256 -> 256 at 14^2 x 16 35 / 31; with one they move, 37 / 32).
+//   with a residual 366 / 437, 128 -> 256 stride 2 at 28^2 x 164, T = 7 395 / 554). Deep layers of few outputs always move (256 -> 256 at 14^2 x 4 29 / 18, 512 -> 512 at 4^2 x 16 37 / 21). Over 22300 layers of
+//   whole tiles, planes of four pixels, few pixels and deep layers among them, the rule is 1 % slower than the better kernel in the mean, the dense kernels
+//   alone 54 % (256 -> 512 at 2^2 x 40 24 / 14, 64 -> 64 at 16^2 x 2 30 / 11, 256 -> 256 at 14^2 x 16 35 / 31, with a residual 37 / 32).
 // * fp32 tensors (two bf16 terms each) run here at two and a half times the speed of the dense kernels over 1500 layers without low terms, and at
 //   1.85 times where every input has one: 64 -> 64 at 32^2 x 8 35 / 20, at 56^2 x 16 100 / 73, 512 -> 512 at 7^2 x 4 with a residual 125 / 29, 41 -> 72
 //   at 8 x 14 x 15 191 / 20, 122 -> 111 at 15^2, 5x5, T = 5 1068 / 36, 3 -> 64 at 32^2 x 64 34 / 31, 128 -> 256 1x1 at 28^2 x 8 135 / 27. 1x1 layers
@@ -175,9 +173,7 @@ bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int C
             return T > 2 || K >= 1152 || !strided || outs <= (3 << 19);
         case DenseFamily::kMatrixWhole:
             if (deep) return true;
-            if (plane <= 4 || (T >= 3 && T <= 4 && !one && !strided && pixels <= 512 && K < 1152)) return false;
             if (!one && !strided && Cin <= 8) return false;   // (a single channel group: as above)
-            if (K >= 2304 && T <= 4 && !residual && tile_use >= 1.0) return false;
             if (one) return tile_use * std::sqrt(576.0 / K) <= 0.45;
             if (strided) return tile_use * std::sqrt(std::sqrt(576.0 / K)) <= (T <= 4 ? 0.5 : (inputs < (1 << 24) ? 0.65 : 0.45));
             return tile_use * std::sqrt(576.0 / K) <= (inputs >= (1 << 26) ? 0.7 : (T <= 4 ? 0.85 : 0.95));
