@@ -134,6 +134,42 @@ def test_tiles_spread_over_compute_units(snnf_lib, Cin, Cout, H, W, N, grid):
     check(B.to_dense(out), v, ref, what=f"{Cin}->{Cout} {H}x{W} x {N}")
 
 
+@pytest.mark.parametrize("Cin,Cout,H,W,k,s,N,dtype,layout,tile", [
+    (32, 512, 2, 2, 5, 1, 123, BF16, "bits", "4x2x2"),      # the halos of eight planes of 6 x 6 don't fit, those of four do
+    (32, 512, 4, 4, 3, 2, 125, BF16, "bits", "4x2x2"),      # ... of 5 x 5
+    (64, 512, 8, 8, 3, 2, 66, F16, "c8", "1x4x4"),          # two planes of 9 x 9
+    (32, 64, 2, 2, 5, 1, 257, F16, "nchw", "4x2x2"),        # ... and dense tensors around, as a call of two launches
+    (32, 64, 4, 4, 5, 2, 64, BF16, "bits", "1x2x1"),        # 256 pixels: parts of planes
+    (32, 64, 4, 4, 5, 2, 65, BF16, "bits", "2x2x2"),        # 260: whole ones
+])
+def test_whole_planes_whose_halos_do_not_fit(snnf_lib, Cin, Cout, H, W, k, s, N, dtype, layout, tile):
+    from triton_snn_fusion_amd.runtime import hip_blocked_backend as B
+    from triton_snn_fusion_amd.runtime import hip_convlif_backend as CB
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the shapes sit at the edges of 256 compute units")
+    g = gen(5000 + N)
+    p = k // 2
+    x = torch.stack([spikes((N, Cin, H, W), 0.25, g) for _ in range(4)])
+    w, b = q(torch.randn(Cout, Cin, k, k, generator=g) * 2.0 * (2.0 / (Cin * k * k)) ** 0.5, dtype), q(torch.randn(Cout, generator=g) * 0.1, dtype)
+    ref = O.temporal_conv_lif(list(x), w, b, torch.tensor(0.0), (s, s), (p, p), (1, 1), 1, *LIF)
+    if layout == "nchw":
+        dx, Ho, Wo = [dev(t, dtype) for t in x], (H + 2 * p - k) // s + 1, (W + 2 * p - k) // s + 1
+        from triton_snn_fusion_amd import _lib
+        need = snnf_lib.snnf_conv_lif_scratch_bytes(4, N, Cin, H, W, _lib.dtype_code(dtype), Cout, k, k, s, s, p, p, 0, 0)
+        assert need > 0
+        workspace, packed = torch.empty(need, dtype=torch.uint8, device=DEV), CB._packed_weight(dev(w, dtype), dev(b, dtype), dtype)
+        sp, v = torch.empty(4, N, Cout, Ho, Wo, device=DEV, dtype=dtype), torch.empty(N, Cout, Ho, Wo, device=DEV)
+        _lib.check("snnf_conv_lif_ws", snnf_lib.snnf_conv_lif_ws(
+            _lib.step_pointers(dx), None, 4, N, Cin, H, W, _lib.dtype_code(dtype), packed.data_ptr(), Cout, k, k, s, s, p, p, None, 0,
+            sp.data_ptr(), int(sp.stride(0)), v.data_ptr(), *LIF, workspace.data_ptr(), need, _lib.current_stream(sp.device)))
+    else:
+        layout = {"bits": B.BITS, "c8": B.C8}[layout]
+        out, v = B.conv_lif_blocked(B.from_dense(dev(x, dtype), layout), dev(w, dtype), dev(b, dtype), [s, s], [p, p], LIF, out_layout=layout, want_v=True)
+        sp = B.to_dense(out)
+    assert CB.last_conv_plan()["tile"] == tile, CB.last_conv_plan()
+    check(sp, v, ref, what=f"{Cin}->{Cout} {k}x{k}/{s} {H}x{W} x {N}")
+
+
 @pytest.mark.parametrize("T,out", [(1, "bits"), (2, "bits"), (1, "c8"), (2, "nchw")])
 def test_narrow_tiles_of_short_windows(snnf_lib, T, out):
     """One and two timesteps on tiles of 32 channels, straight-line and general epilogue, a last tile of 8 channels."""

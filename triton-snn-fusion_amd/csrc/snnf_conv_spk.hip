@@ -42,18 +42,26 @@ bool plan_spk(const SpkGeom& g0, int tt, SpkPlan& best, int only_pc = 0, int onl
         const int rr = (pr - 1) * g0.sh + g0.KH;
         const int rc = (pc - 1) * g0.sw + g0.KW;
         if (rr > 255 || rc > 255) continue;
-        const int region = pi * rr * rc;
-        int G = 0;
-        if (g0.tap_pairs) {
-            if (region <= 64 * kSpkSlots && tt * (region + 1) * 16 <= kWaveLds) G = 1;
-        } else {
-            for (int cand = g0.gpc; cand >= 2; cand >>= 1) {
-                if (only_g > 0 && cand > only_g) continue;
-                if (cand * region <= 64 * kSpkSlots && tt * (cand * region + 1) * 16 <= kWaveLds) {   // + the dummy item of a timestep
-                    G = cand;
-                    break;
+        // Where the halos of so many planes don't fit (5x5 on 2x2 planes, strided 3x3 onto 2x2 and 4x4) half as many, and again, before a part
+        // of one plane: 512 -> 512 stride 2 from 4x4 x 155 in tiles of 2 x 1 pixels 170 us, of four planes 48, 256 -> 512, 5x5 on 2x2 x 122,
+        // T = 8 252 / 55. Up to 256 pixels times tiles of channels parts are faster, as more workgroups (384 -> 64, 5x5 stride 2 from 4x4 x 15
+        // 21.0 / 24.1; the quotient passes 1 there over 770 layers).
+        const bool fewer = static_cast<int64_t>(g0.N) * pr * pc * oc_tiles > cus;
+        int region, G = 0;
+        for (;; pi >>= 1) {
+            region = pi * rr * rc;
+            if (g0.tap_pairs) {
+                if (region <= 64 * kSpkSlots && tt * (region + 1) * 16 <= kWaveLds) G = 1;
+            } else {
+                for (int cand = g0.gpc; cand >= 2; cand >>= 1) {
+                    if (only_g > 0 && cand > only_g) continue;
+                    if (cand * region <= 64 * kSpkSlots && tt * (cand * region + 1) * 16 <= kWaveLds) {   // + the dummy item of a timestep
+                        G = cand;
+                        break;
+                    }
                 }
             }
+            if (G > 0 || pi == 1 || !fewer) break;
         }
         if (G == 0) continue;
         const int patches_x = (g0.Wo + pc - 1) / pc;
