@@ -59,7 +59,7 @@ def test_whole_tiles_on_the_matrix_kernel(snnf_lib, Cin, Cout, H, W, k, s, T, N,
     (64, 128, 56, 1, 2, 4, 16, False, False),
     (16, 64, 40, 3, 1, 4, 2, False, True),       # a single stage: narrow tiles of one wave
     (256, 256, 14, 3, 1, 4, 16, True, True),     # deep: with a residual ...
-    (256, 256, 14, 3, 1, 4, 16, False, False),   # ... and without
+    (256, 256, 14, 3, 1, 4, 16, False, True),    # ... and without
 ])
 def test_whole_tiles_move_where_they_leave_the_chip_idle(snnf_lib, Cin, Cout, H, k, s, T, N, residual, moves):
     from triton_snn_fusion_amd import _lib
