@@ -250,7 +250,8 @@ int snnf_conv_lif(const void* const* xs, const void* const* residuals, int T,
  * additions.
  *   snnf_conv_lif_scratch_bytes : bytes with which this call takes that route (0: the call is snnf_conv_lif). A call whose
  *               timesteps all read one frame never takes it and needs none.
- *   snnf_conv_lif_workspace_bytes : the same for 16-bit activations beside an fp32 membrane, 0 for every other call.
+ *   snnf_conv_lif_workspace_bytes : the older question, which knows 16-bit activations beside an fp32 membrane only and answers 0 for every other
+ *               call (that call then runs as snnf_conv_lif). Ask snnf_conv_lif_scratch_bytes instead.
  *   workspace : NULL (then this is snnf_conv_lif), or device memory, 16-byte aligned, contents undefined before and after.
  *               A smaller workspace than asked for is not used. Calls that share a workspace must not overlap in time.
  *   v_dtype : a 16-bit membrane is held in fp32 (in the workspace, between the windows of a call) and rounded once at the end.
