@@ -144,7 +144,8 @@ __device__ __forceinline__ void store_streaming(T* dst, const Pack<T, N>& value)
 // ---------------------------------------------------------------------------------------------------------------
 // LIF neuron (runtime/snn_custom_ops.py:384-409). The charge rule is chosen on the host once per launch.
 // Kernels take the membrane pointers without __restrict__: a caller may pass one buffer as v_init and v_out, and later windows of a
-// call read what the one before them stored there. Each element is read and stored by the same lane. (The blocked kernel's are apart.)
+// call read what the one before them stored there. Each element is read and stored by the same lane.
+// (Those of the blocked and of the staged linear kernel are apart: a call in place passes its buffer once.)
 // ---------------------------------------------------------------------------------------------------------------
 enum ChargeMode : int {
     CHARGE_IF = 0,        // tau <= 1:            h = v + x

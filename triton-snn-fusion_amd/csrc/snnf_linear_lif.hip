@@ -32,6 +32,7 @@ struct LinGeom {
     int64_t spike_step_stride; // elements
     int ksteps;                // ceil(Fin / 32)
     int kparts;                // 1, or 3 for fp32 tensors
+    int v_in_place = 0;        // staged kernel: the initial membrane lies in v_store
 };
 
 // Eight consecutive K elements of one row as a matrix-core operand (bf16 for fp32/bf16 storage, fp16 for fp16 storage).
@@ -302,8 +303,8 @@ template <int TT, int OCF, int SLABK, int TM> struct StagedShape {
 template <typename XT, typename VT, int TT, int OCF, bool DB, int SLABK, int TM, bool XBITS = false, bool SBITS = false>
 __global__ __launch_bounds__(kStagedWaves * 64) void linear_lif_staged_kernel(StepPtrs xs, LinGeom g, const XT* __restrict__ W,
                                                                               const XT* __restrict__ bias,
-                                                                              const VT* v_init, XT* __restrict__ spikes,
-                                                                              VT* v_out, LifParams lif,
+                                                                              const VT* __restrict__ v_start, XT* __restrict__ spikes,
+                                                                              VT* __restrict__ v_store, LifParams lif,
                                                                               float* __restrict__ ws_partial, int* __restrict__ ws_count,
                                                                               int slabs_per_part) {
     using SH = StagedShape<TT, OCF, SLABK, TM>;
@@ -326,6 +327,9 @@ __global__ __launch_bounds__(kStagedWaves * 64) void linear_lif_staged_kernel(St
     const bool out_live = tid < OUTS && out_m < g.M && out_oc < g.Fout;
     const int64_t out_index = static_cast<int64_t>(out_live ? out_m : 0) * g.Fout + (out_live ? out_oc : 0);
     const float bv = bias != nullptr ? to_float(bias[out_live ? out_oc : 0]) : 0.0f;
+    // A call in place passes no v_start, so the two membrane arguments are never the same memory. (Promising nothing to the compiler instead cost
+    // 1.5 %: 8 x 64, 2048 -> 1024 10.04 -> 10.20 us.)
+    const VT* const v_init = g.v_in_place ? v_store : v_start;
     const float v_first = v_init != nullptr ? to_float(v_init[out_index]) : 0.0f;
 
     // Staging items of this thread: item i = tid + j * NT is octet i % 16 of operand row i / 16 (NT is a multiple of 16, so
@@ -542,7 +546,7 @@ __global__ __launch_bounds__(kStagedWaves * 64) void linear_lif_staged_kernel(St
                 }
             }
         }
-        if (v_out != nullptr && out_live) v_out[out_index] = from_float<VT>(v);
+        if (v_store != nullptr && out_live) v_store[out_index] = from_float<VT>(v);
     }
 }
 
@@ -566,8 +570,10 @@ int launch_staged_db(dim3 grid, int slabs_per_part, const LinWorkspace& ws, cons
                                                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
         if (raised != hipSuccess) return fail(SNNF_ERR_LAUNCH, "snnf_linear_lif: cannot reserve %zu bytes of LDS", lds);
     }
-    kernel<<<grid, kStagedWaves * 64, lds, stream>>>(xs, g, static_cast<const XT*>(W), static_cast<const XT*>(bias),
-                                                     static_cast<const VT*>(v_init), static_cast<XT*>(spikes),
+    LinGeom placed = g;
+    placed.v_in_place = v_init != nullptr && v_init == v_out ? 1 : 0;
+    kernel<<<grid, kStagedWaves * 64, lds, stream>>>(xs, placed, static_cast<const XT*>(W), static_cast<const XT*>(bias),
+                                                     placed.v_in_place ? nullptr : static_cast<const VT*>(v_init), static_cast<XT*>(spikes),
                                                      static_cast<VT*>(v_out), lif,
                                                      reinterpret_cast<float*>(static_cast<char*>(ws.base) + kLinCounterBytes),
                                                      static_cast<int*>(ws.base), slabs_per_part);
