@@ -297,7 +297,7 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
     g.nstages = (g.C8in + g.G - 1) / g.G;
     g.IT = g.G * g.region;
     g.JT = (g.IT + 63) / 64;
-    g.lds_wave_bytes = tt * (g.IT + 1) * 16;
+    g.lds_wave_bytes = std::max(tt * (g.IT + 1) * 16, 256);   // (a tile's bias passes through it)
     int& oc_tiles = p.oc_tiles;
     oc_tiles = g.narrow ? (Cout + 31) / 32 : (Cout + 63) / 64;
     g.n_items = g.n_patches * oc_tiles;
@@ -344,15 +344,15 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
     // Narrow tiles of one wave: two tiles of a patch side by side, which read the same activations.
     const int spread = g.narrow && !c.split && wk_log2 == 0 ? g.n_patches * ((Cout + 63) / 64) : g.n_items;
     if (g.iters > 1 ? grid * 4 < resident * 3 : grid * 2 <= cus) grid = std::min(spread, g.iters > 1 ? resident : cus);
-    g.d_ppx = make_fast_div(g.PR * g.PC);
-    g.d_PC = make_fast_div(g.PC);
-    g.d_region = make_fast_div(g.region);
-    g.d_rrrc = make_fast_div(g.RR * g.RC);
-    g.d_RC = make_fast_div(g.RC);
-    g.d_n_patches = make_fast_div(g.n_patches);
-    g.d_patches_img = make_fast_div(g.patches_img);
-    g.d_patches_x = make_fast_div(g.patches_x);
-    g.d_gpc = make_fast_div(g.gpc);
+    g.grid = grid;
+    g.d_ppx = make_spk_div(g.PR * g.PC);
+    g.d_PC = make_spk_div(g.PC);
+    g.d_region = make_spk_div(g.region);
+    g.d_rrrc = make_spk_div(g.RR * g.RC);
+    g.d_RC = make_spk_div(g.RC);
+    g.d_n_patches = make_spk_div(g.n_patches);
+    g.d_patches_img = make_spk_div(g.patches_img);
+    g.d_patches_x = make_spk_div(g.patches_x);
     const int hg = g.tap_pairs ? 1 : g.G / 2;
     const int nst = g.tap_pairs ? g.npairs : g.taps * hg;
     g.kw_mul = (KW & (KW - 1)) == 0 ? 65536 / KW : 65536 / KW + 1;
@@ -381,9 +381,6 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
         g.sc_npairs = pg2.npairs;
         g.sc_frag_stride = static_cast<int64_t>(pg2.nchunks) * pg2.npairs * (kFragBytes / 2);
     }
-    g.d_hg = make_fast_div(hg);
-    g.d_nst = make_fast_div(nst);
-    g.d_KW = make_fast_div(KW);
     return SNNF_OK;
 }
 
@@ -728,7 +725,6 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     if (pool2) {
         if (!fast_epi || p.windows != 1 || (p.tt != 4 && !shared))
             return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_pool: the pooled output needs the usual neuron (tau 2, hard reset to 0) and the four steps in one window", who);
-        L.g.pool2 = 1;
         if (x_layout == SNNF_LAYOUT_NCHW) return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_frame(L, true) : launch_conv_spk_f16_frame(L, true);
         return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_pooled(L, p.tt) : launch_conv_spk_f16_pooled(L, p.tt);
     }

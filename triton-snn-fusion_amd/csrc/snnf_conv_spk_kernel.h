@@ -41,8 +41,21 @@ constexpr int kSpkMaxSteps = 60;                  // matrix steps per stage, at 
 constexpr size_t kSpkTableBytes = (kSpkMaxSteps + 4) * 16;      // the workgroup's step table at the start of LDS
 constexpr int kSpkDescs = 64 * kSpkSlots;                       // staging items of one timestep, at most
 constexpr size_t kSpkDescBytes = kSpkDescs * 8;                 // the workgroup's staging descriptors behind the step table
-constexpr size_t kSpkPosBytes = 32 * 4;            // where each of the 32 pixels of a tile sits inside the patch
+constexpr size_t kSpkPosBytes = 32 * 8;            // where each of the 32 pixels of a tile sits inside the patch, and its top-left input in the staged halo
 constexpr size_t kSpkHeaderBytes = kSpkTableBytes + kSpkDescBytes + kSpkPosBytes;   // what precedes the waves' staging regions in LDS
+
+// n / d for 0 <= n < 2^31 as one multiply-high and a shift, for every d from 1: with s = ceil(log2 d) and mul = ceil(2^(31+s) / d), 2 n mul / 2^32 / 2^s
+// exceeds n / d by less than 1 / d. (fast_div's general form takes another multiply or a select for a divisor of 1.)
+struct SpkDiv {
+    uint32_t mul;
+    int shift;
+};
+inline SpkDiv make_spk_div(int d) {
+    int s = 0;
+    while ((1LL << s) < d) ++s;
+    return {static_cast<uint32_t>(((1ULL << (31 + s)) + static_cast<uint64_t>(d) - 1) / static_cast<uint64_t>(d)), s};
+}
+__device__ __forceinline__ int sk_div(int n, const SpkDiv& f) { return static_cast<int>(__umulhi(static_cast<uint32_t>(n) * 2u, f.mul) >> f.shift); }
 
 struct SpkGeom {
     int N, Cin, H, W, Cout, KH, KW, sh, sw, ph, pw, Ho, Wo;
@@ -71,7 +84,7 @@ struct SpkGeom {
     int narrow;                  // tiles of 32 output channels instead of 64
     int in_layout, res_layout, out_layout;   // snnf_layout codes; res_layout < 0: no residual
     int analog_out;              // no neuron: the sums themselves are written (C8 or NCHW)
-    int pool2;                   // the POOL variants: the spikes leave as their 2x2 averages (quarters, C8, half the plane)
+    int grid;                    // workgroups of the launch (read from here: the hidden arguments lie in a cache line of their own)
     int64_t out_step_stride;     // bytes between timesteps of `out`
     int lds_wave_bytes;          // private staging region of a wave (a multiple of 16)
     int64_t frag_stride;         // 16-bit elements between consecutive 32-row fragments of the packed weight
@@ -88,7 +101,7 @@ struct SpkGeom {
     int64_t flag_stride;         // bytes of the flags of one timestep (a multiple of 4)
     int v16;                     // v_start and v_store hold the activation dtype; the windows in between pass v_scratch on
     int v_in_place;              // the initial membrane lies in v_store
-    FastDiv d_ppx, d_PC, d_region, d_rrrc, d_RC, d_n_patches, d_patches_img, d_patches_x, d_gpc, d_hg, d_nst, d_KW;
+    SpkDiv d_ppx, d_PC, d_region, d_rrrc, d_RC, d_n_patches, d_patches_img, d_patches_x;
 };
 
 struct SpkLaunch {
@@ -123,10 +136,22 @@ __device__ __forceinline__ sk_f32x16 sk_mfma(sk_u32x4 a, sk_u32x4 b, sk_f32x16 c
     }
 }
 
+// The way from a kernel's start to its first requests is bound by the number of instructions and the round trips it waits for: at 512 -> 512, 7^2 x 16 it took
+// 8.6 k of a launch's 43 k cycles, with a condition and a wait per quad of biases, branches around each comparison of a descriptor, divisions by 1 as a
+// special case and 90 scalars of the epilogue worked out and spilled in front, and takes 5.9 k as it stands (20.6 -> 20.1 us at 64 -> 64, 56^2 x 16,
+// 21.4 -> 20.1 at 512 -> 512, 7^2 x 16, 12.4 -> 11.7 at 4^2, one image, 18.5 -> 17.1 at 64 -> 128 stride 2).
+// A uniform value that is computed where it stands: the compiler otherwise works out everything that depends on the kernel arguments alone ahead
+// of all loops, and keeps it in (and reads it back from) lanes of vector registers.
+__device__ __forceinline__ int sk_here(int x) {
+    asm volatile("" : "+s"(x));
+    return x;
+}
+
 // Entry i of a table of pointers passed by value as a kernel argument, read from the kernel-argument segment (arguments
 // start at offset 0 of that segment, in declaration order and naturally aligned): indexing the by-value struct with a
 // runtime index would copy it to scratch memory.
 typedef const void* sk_cvp;
+typedef const __attribute__((address_space(1))) unsigned char* sk_global_bytes;
 __device__ __forceinline__ const void* sk_kernarg_ptr(int table_offset_bytes, int i) {
     typedef const __attribute__((address_space(4))) unsigned char* ka_bytes;
     typedef const __attribute__((address_space(4))) sk_cvp* ka_entry;
@@ -134,23 +159,34 @@ __device__ __forceinline__ const void* sk_kernarg_ptr(int table_offset_bytes, in
     return *(ka_entry)(ka + table_offset_bytes + i * 8);
 }
 
-// Eight spike bits -> eight 16-bit ones or zeros (ONE = the dtype's 1.0), channel j in element j.
-// fast_div without a branch: the multiply-high runs for a divisor of 1 as well (its multiplier is 0, the quotient then
-// comes from the mask). The staging decode divides three times per item; a uniform branch around each of them costs more
-// than the multiply and keeps the compiler from overlapping the items.
-__device__ __forceinline__ int sk_div(int n, const FastDiv& f) {
-    const uint32_t keep = f.d == 1u ? 0xffffffffu : 0u;
-    return static_cast<int>((__umulhi(static_cast<uint32_t>(n), f.mul) >> f.shift) | (static_cast<uint32_t>(n) & keep));
+// The kernel's arguments as they lie in the kernel-argument segment (the order of its parameters).
+struct SpkArgs {
+    StepPtrs xs, residuals;
+    SpkGeom g;
+    const void *wpacked, *bias, *v_start, *out, *v_store;
+    LifParams lif;
+    const void *wpacked2, *bias2, *v_scratch, *lo_flags;
+};
+__device__ __forceinline__ const __attribute__((address_space(4))) SpkArgs& sk_kernarg_spk() {
+    auto ka = __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(ka));       // (opaque: what is derived from it is computed where it is used)
+    return *(const __attribute__((address_space(4))) SpkArgs*)ka;
 }
 
+// Eight spike bits -> eight 16-bit ones or zeros (ONE = the dtype's 1.0), channel j in element j. `twice` holds the byte in both halves
+// (bit j at bits j and 16 + j, from one byte permutation that also drops the bytes of padding): per pair of channels one mask and one
+// packed multiplication, by the 1.0 shifted down by the bit's place (both dtypes' 1.0 end in seven zero bits or more).
+typedef uint16_t sk_u16x2 __attribute__((ext_vector_type(2)));
 template <uint32_t ONE>
-__device__ __forceinline__ sk_u32x4 sk_expand_bits(uint32_t byte) {
-    const uint32_t m = __umul24(byte, 0x8001u);   // bit i of the byte at bits i and 15 + i
+__device__ __forceinline__ sk_u32x4 sk_expand_bits(uint32_t twice) {
+    static_assert((ONE & 0x7fu) == 0, "the dtype's 1.0 is shifted down by up to seven bits");
     sk_u32x4 d;
-    d[0] = __umul24(m & 0x10001u, ONE);
-    d[1] = __umul24((m >> 2) & 0x10001u, ONE);
-    d[2] = __umul24((m >> 4) & 0x10001u, ONE);
-    d[3] = __umul24((m >> 6) & 0x10001u, ONE);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const sk_u16x2 bits = __builtin_bit_cast(sk_u16x2, twice & ((1u << (2 * k)) | (0x20000u << (2 * k))));
+        const sk_u16x2 one = {static_cast<uint16_t>(ONE >> (2 * k)), static_cast<uint16_t>(ONE >> (2 * k + 1))};
+        d[k] = __builtin_bit_cast(uint32_t, static_cast<sk_u16x2>(bits * one));
+    }
     return d;
 }
 
@@ -177,15 +213,14 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
         auto ka = __builtin_amdgcn_kernarg_segment_ptr();
         // The explicit arguments are two step tables, the geometry, nine pointers and the neuron: the last dword that is
         // touched must lie inside them (what follows is the hidden-argument area, which the compiler may leave out).
-        constexpr size_t kExplicitArgBytes = 2 * sizeof(StepPtrs) + sizeof(SpkGeom) + 9 * sizeof(void*) + sizeof(LifParams);
-        static_assert(0x2c0 + 4 <= kExplicitArgBytes, "argument prefetch reads past the explicit kernel arguments");
-        static_assert(0x300 + 4 <= kExplicitArgBytes && kExplicitArgBytes <= 0x340, "argument prefetch does not end in the last cache line of the arguments");
-        uint32_t d0, d1, d2, d3, d4, d5, d6, d7, d8, d9, d10, d11;
+        constexpr size_t kExplicitArgBytes = sizeof(SpkArgs);
+        static_assert(0x280 + 4 <= kExplicitArgBytes && kExplicitArgBytes <= 0x2c0, "argument prefetch does not end in the last cache line of the explicit arguments");
+        uint32_t d0, d1, d2, d3, d4, d5, d6, d7, d8, d9;
         asm volatile(
-            "s_load_dword %0, %12, 0x40\n\ts_load_dword %1, %12, 0x80\n\ts_load_dword %2, %12, 0xc0\n\ts_load_dword %3, %12, 0x100\n\t"
-            "s_load_dword %4, %12, 0x140\n\ts_load_dword %5, %12, 0x180\n\ts_load_dword %6, %12, 0x1c0\n\ts_load_dword %7, %12, 0x200\n\t"
-            "s_load_dword %8, %12, 0x240\n\ts_load_dword %9, %12, 0x280\n\ts_load_dword %10, %12, 0x2c0\n\ts_load_dword %11, %12, 0x300\n\ts_waitcnt lgkmcnt(0)"
-            : "=&s"(d0), "=&s"(d1), "=&s"(d2), "=&s"(d3), "=&s"(d4), "=&s"(d5), "=&s"(d6), "=&s"(d7), "=&s"(d8), "=&s"(d9), "=&s"(d10), "=&s"(d11)
+            "s_load_dword %0, %10, 0x40\n\ts_load_dword %1, %10, 0x80\n\ts_load_dword %2, %10, 0xc0\n\ts_load_dword %3, %10, 0x100\n\t"
+            "s_load_dword %4, %10, 0x140\n\ts_load_dword %5, %10, 0x180\n\ts_load_dword %6, %10, 0x1c0\n\ts_load_dword %7, %10, 0x200\n\t"
+            "s_load_dword %8, %10, 0x240\n\ts_load_dword %9, %10, 0x280\n\ts_waitcnt lgkmcnt(0)"
+            : "=&s"(d0), "=&s"(d1), "=&s"(d2), "=&s"(d3), "=&s"(d4), "=&s"(d5), "=&s"(d6), "=&s"(d7), "=&s"(d8), "=&s"(d9)
             : "s"(ka));
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -221,12 +256,9 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
     const int wk = SK ? (wave & (WK - 1)) : 0;
     const int tile_in_block = SK ? (wave >> g.wk_log2) : wave;
     const int tiles_per_block = SK ? (kSpkWaves >> g.wk_log2) : kSpkWaves;
-    const int po = g.Ho * g.Wo;
     const int nsteps_t = g.shared_x ? 1 : g.T;          // timesteps with a convolution of their own
     const int hg = g.tap_pairs ? 1 : (g.G >> 1);        // k-slot pairs per tap and stage
     const int nst = g.tap_pairs ? g.npairs : g.taps * hg;   // matrix steps per stage
-    const bool common_lif = lif.charge_mode == CHARGE_SCALE && !lif.soft_reset;
-    const bool half_tau = lif.inv_tau == 0.5f;
 
     // ---- step table of the workgroup: for step i of a stage, the byte offset of its weight fragments from the stage's
     // first pair and the LDS offset of its activations (tap and channel group of the half's k-slot), once for the lower and
@@ -234,31 +266,32 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
     // arithmetic. Steps beyond the last repeat it (prefetch only).
     {
         sk_u32x4* __restrict__ table = reinterpret_cast<sk_u32x4*>(lds);
-        if (tid < nst + 4) {
-            const int i = min(tid, nst - 1);
+        const int tid_t = tid - 7 * 64;          // (at most 64 entries)
+        if (tid_t >= 0 && tid_t < nst + 4) {
+            const int i = min(tid_t, nst - 1);
             sk_u32x4 e;
             if (g.tap_pairs) {
                 const int tap0 = 2 * i, tap1 = min(2 * i + 1, g.taps - 1);   // an odd tap count leaves the last k-slot empty (zero weights)
-                const int kh0 = tap0 / g.KW, kh1 = tap1 / g.KW;
+                const int kh0 = (tap0 * g.kw_mul) >> 16, kh1 = (tap1 * g.kw_mul) >> 16;
                 e[0] = static_cast<uint32_t>(i * kFragBytes);
                 e[1] = static_cast<uint32_t>((kh0 * g.RC + (tap0 - kh0 * g.KW)) * 16);
                 e[3] = static_cast<uint32_t>((kh1 * g.RC + (tap1 - kh1 * g.KW)) * 16);
             } else {
                 const int tap = i >> g.hg_log2;
                 const int gp = i & (hg - 1);
-                const int kh = tap / g.KW;
+                const int kh = (tap * g.kw_mul) >> 16;
                 const int tapoff = (kh * g.RC + (tap - kh * g.KW)) * 16;
                 e[0] = static_cast<uint32_t>((tap * g.pair_tap_stride + gp) * kFragBytes);
                 e[1] = static_cast<uint32_t>(tapoff + (2 * gp) * region16);
                 e[3] = static_cast<uint32_t>(tapoff + (2 * gp + 1) * region16);
             }
             e[2] = e[0];
-            table[tid] = e;
+            table[tid_t] = e;
         }
         if constexpr (SC) {
             // The shortcut's stages: one tap, the centre of the main kernel (the lane's own pixel), on the same halo; entries
             // behind the main table's.
-            const int i2 = tid - (nst + 4);
+            const int i2 = tid_t - (nst + 4);
             if (i2 >= 0 && i2 < hg + 4) {
                 const int gp = min(i2, hg - 1);
                 const int tapoff = (g.ph * g.RC + g.pw) * 16;
@@ -267,7 +300,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                 e[1] = static_cast<uint32_t>(tapoff + (2 * gp) * region16);
                 e[2] = e[0];
                 e[3] = static_cast<uint32_t>(tapoff + (2 * gp + 1) * region16);
-                table[tid] = e;
+                table[tid_t] = e;
             }
         }
         // ---- staging descriptors of the workgroup: item e of a timestep's stage = (channel group gq, image ii, halo row r, halo
@@ -294,14 +327,18 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
         }
         // ---- where pixel p of a tile sits inside the patch: image, row and column, packed. Every item reads its lane's entry
         // back: kept in registers these values would live (or be spilled) across the matrix loop of every variant.
-        if (tid < 32) {
+        // (Built by the sixth wave and the step table by the eighth: the first ones have the descriptors of a usual stage.)
+        if (tid >= 5 * 64 && tid < 5 * 64 + 32) {
+            const int p32 = tid - 5 * 64;
             const int ppx = g.PR * g.PC;
-            const int pi = sk_div(tid, g.d_ppx);
-            const int prem = tid - pi * ppx;
+            const int pi = sk_div(p32, g.d_ppx);
+            const int prem = p32 - pi * ppx;
             const int prow = sk_div(prem, g.d_PC);
             const int pcol = prem - prow * g.PC;
-            reinterpret_cast<uint32_t*>(lds + kSpkTableBytes + kSpkDescBytes)[tid] =
-                static_cast<uint32_t>(pi) | (static_cast<uint32_t>(prow) << 8) | (static_cast<uint32_t>(pcol) << 16);
+            Pack<uint32_t, 2> e;
+            e.v[0] = static_cast<uint32_t>(pi) | (static_cast<uint32_t>(prow) << 8) | (static_cast<uint32_t>(pcol) << 16);
+            e.v[1] = pi < g.PI ? static_cast<uint32_t>(((pi * g.RR + prow * g.sh) * g.RC + pcol * g.sw) * 16) : 0u;
+            reinterpret_cast<Pack<uint32_t, 2>*>(lds + kSpkTableBytes + kSpkDescBytes)[p32] = e;
         }
         __syncthreads();
     }
@@ -311,7 +348,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
     // Workgroups are handed to the eight XCDs in turn (workgroup b runs on XCD b % 8) and every XCD has an L2 of its own.
     // Items are ordered output-channel tile first, so the workgroups of one XCD take a contiguous range of them: an XCD then
     // reads the weights of few output-channel tiles (one, for a 512-channel layer) instead of the whole tensor.
-    const int nb = static_cast<int>(gridDim.x);
+    const int nb = g.grid;
     const int xcd = static_cast<int>(blockIdx.x) & 7;
     const int block_l = xcd * (nb >> 3) + min(xcd, nb & 7) + (static_cast<int>(blockIdx.x) >> 3);
     for (int it = 0; it < g.iters; ++it) {
@@ -330,64 +367,17 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
         const int ih_lo = oh0 * g.sh - g.ph;
         const int iw_lo = ow0 * g.sw - g.pw;
 
-        // ---- this lane's output pixel inside the patch, and where its top-left input sits in the staged halo.
-        const uint32_t lane_pos = reinterpret_cast<const uint32_t*>(lds + kSpkTableBytes + kSpkDescBytes)[l32];
-        const int pi = static_cast<int>(lane_pos & 255u);
-        const int prow = static_cast<int>((lane_pos >> 8) & 255u);
-        const int pcol = static_cast<int>(lane_pos >> 16);
-        const bool lane_in_patch = pi < g.PI;
-        const uint32_t lane_b = lane_in_patch ? static_cast<uint32_t>(((pi * g.RR + prow * g.sh) * g.RC + pcol * g.sw) * 16) : 0u;
-
         const int ocf0 = oc_tile * NF;
         // With K split over waves, every wave finishes a part of the tile's eight quads, which its accumulators hold in the same registers
         // whatever the wave: the upper half of the waves computes the two 32-channel fragments in swapped places, and the lanes
         // read the weight rows of a fragment with the quads exchanged (quad q of the accumulators is quad q ^ quad_x of the fragment).
         const int swap_f = SK && !NARROW ? wk >> (g.wk_log2 - 1) : 0;
-        const int quad_x = SK && !NARROW ? (WK == 8 ? wk & 3 : (WK == 4 ? (wk & 1) * 2 : 0)) : 0;
+        const int quad_x = SK && !NARROW ? (wk << (3 - g.wk_log2)) & 3 : 0;      // (eight waves: wk & 3, four: 2 (wk & 1), two: 0)
         const int64_t w_frag0 = min(ocf0 + swap_f, g.nocf - 1);
         const int64_t w_frag1 = min(ocf0 + 1 - swap_f, g.nocf - 1);
 
-        // ---- this lane's output pixel.
-        const int n = n0 + pi;
-        const int oh = oh0 + prow;
-        const int ow = ow0 + pcol;
-        const bool px_ok = have && lane_in_patch && n < g.N && oh < g.Ho && ow < g.Wo;
-        const int pxo = px_ok ? oh * g.Wo + ow : 0;
-        const int n_c = px_ok ? n : 0;
-
         for (int t0 = 0; t0 < nsteps_t; t0 += TT) {
-            // The accumulators start from the bias: register 4 q + k of fragment f is channel 64 oc_tile + 32 f + 8 q + 4 half + k.
-            // With K split over waves only the first one adds it. The bias is requested here and copied into the accumulators
-            // after the first stage's activations have been requested, so that both round trips to memory overlap.
             sk_f32x16 acc[TT][NF];
-            sk_f32x4 bias4[NF][4];
-            {
-                const int nbias = g.nocf * 32;               // bias values behind the packed weight (zero beyond Cout)
-#pragma unroll
-                for (int f = 0; f < NF; ++f)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const int ch0 = oc_tile * (32 * NF) + f * 32 + q * 8 + 4 * half;
-                        bias4[f][q] = sk_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-                        if (ch0 < nbias && (!SK || wk == 0)) bias4[f][q] = *reinterpret_cast<const sk_f32x4*>(bias + ch0);
-                    }
-                if constexpr (SC) {
-                    sk_f32x4 more[NF][4];
-#pragma unroll
-                    for (int f = 0; f < NF; ++f)
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            const int ch0 = oc_tile * (32 * NF) + f * 32 + q * 8 + 4 * half;
-                            more[f][q] = sk_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-                            if (ch0 < nbias && (!SK || wk == 0)) more[f][q] = *reinterpret_cast<const sk_f32x4*>(bias2 + ch0);
-                        }
-#pragma unroll
-                    for (int f = 0; f < NF; ++f)
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) bias4[f][q] += more[f][q];
-                }
-            }
-
             // One LDS stage: G channel groups of the patch's halo for TT timesteps, from global memory into this wave's region.
             // Item e = slot * 64 + lane of a timestep = (group, image, row, column) of the halo; its LDS address is 16 e. Items
             // are decoded on the fly (nothing about them is kept in registers across the matrix loop) and move in batches of 4
@@ -401,7 +391,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             // padding) and a flag nibble (bit j: real data).
             // A stage at or beyond g.nstages (SC only) is one of the shortcut's: same halo items, taken from the second input at
             // the sampled positions.
-            auto batch_decode = [&](int s, int jb, int lane_s, int (&idx)[4]) __attribute__((always_inline)) -> uint32_t {
+            auto batch_decode = [&](int s, int jb, int lane_s, uint32_t (&idx)[4]) __attribute__((always_inline)) -> uint32_t {
                 const bool second = SC && s >= g.nstages;
                 const int gg0 = ((SC || SPLIT) && s >= g.nstages ? s - g.nstages : s) * g.G;
                 const int c8 = second ? g.sc_C8 : g.C8in;
@@ -414,42 +404,44 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     const Pack<uint32_t, 2> d = desc[(jb + j) * 64 + lane_s];
                     const int r = static_cast<int>(d.v[1] & 255u), c = static_cast<int>((d.v[1] >> 8) & 255u);
                     const int ii = static_cast<int>((d.v[1] >> 16) & 255u), gq = static_cast<int>(d.v[1] >> 24);
-                    const bool ok = n0 + ii < g.N && gg0 + gq < c8 && static_cast<unsigned>(ih_lo + r) < static_cast<unsigned>(g.H) &&
-                                    static_cast<unsigned>(iw_lo + c) < static_cast<unsigned>(g.W);
+                    // (& and not &&: a branch around each comparison waits for each descriptor in turn)
+                    const bool ok = static_cast<bool>(static_cast<int>(n0 + ii < g.N) & static_cast<int>(gg0 + gq < c8) &
+                                                      static_cast<int>(static_cast<unsigned>(ih_lo + r) < static_cast<unsigned>(g.H)) &
+                                                      static_cast<int>(static_cast<unsigned>(iw_lo + c) < static_cast<unsigned>(g.W)));
                     int off = static_cast<int>(d.v[0]);
                     if constexpr (SC) {
                         if (second) off = ((ii * g.sc_C8 + gq) * g.sc_H + r * g.sc_sh) * g.sc_W + c * g.sc_sw;
                     }
-                    idx[j] = ok ? base_u + off : 0;
+                    idx[j] = ok ? static_cast<uint32_t>(base_u + off) : 0u;
                     ok_bits |= ok ? (1u << j) : 0u;
                 }
                 return ok_bits;
             };
-            auto batch_load_bits = [&](int s, const int (&idx)[4], uint32_t (&raw)[TT][4]) __attribute__((always_inline)) {
+            auto batch_load_bits = [&](int s, const uint32_t (&idx)[4], uint32_t (&raw)[TT][4]) __attribute__((always_inline)) {
                 const int ptr_table = SC && s >= g.nstages ? kResTable : 0;
 #pragma unroll
                 for (int t = 0; t < TT; ++t) {
                     const int ts = t0 + t < nsteps_t ? t0 + t : t0;   // steps beyond T repeat the window's first and are never stored
-                    const unsigned char* __restrict__ src = static_cast<const unsigned char*>(sk_kernarg_ptr(ptr_table, ts));
+                    const sk_global_bytes src = (sk_global_bytes)sk_kernarg_ptr(ptr_table, ts);
 #pragma unroll
                     for (int j = 0; j < 4; ++j) raw[t][j] = src[idx[j]];
                 }
             };
             auto batch_put_bits = [&](int jb, int lane_s, uint32_t ok_bits, const uint32_t (&raw)[TT][4]) __attribute__((always_inline)) {
 #pragma unroll
-                for (int t = 0; t < TT; ++t)
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t keep = ((ok_bits >> j) & 1u) ? 0x0c000c00u : 0x0c0c0c0cu;   // v_perm: byte 0 at bytes 0 and 2, or zeros
+                    // every slot writes: an item beyond the stage goes to the timestep's dummy item
+                    unsigned char* const item = wlds + min((jb + j) * 64 + lane_s, g.IT) * 16;
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const sk_u32x4 d = sk_expand_bits<ONE>(((ok_bits >> j) & 1u) ? raw[t][j] : 0u);
-                        // every slot writes: an item beyond the stage goes to the timestep's dummy item
-                        *reinterpret_cast<sk_u32x4*>(wlds + t * tile_t + min((jb + j) * 64 + lane_s, g.IT) * 16) = d;
-                    }
+                    for (int t = 0; t < TT; ++t) *reinterpret_cast<sk_u32x4*>(item + t * tile_t) = sk_expand_bits<ONE>(__builtin_amdgcn_perm(raw[t][j], raw[t][j], keep));
+                }
             };
             // Requests the first batch of stage s (PRE only).
             auto stage_req = [&](int s) __attribute__((always_inline)) {
                 int lane_s = lane;
                 asm volatile("" : "+v"(lane_s));
-                int idx[4];
+                uint32_t idx[4];
                 pre_ok = batch_decode(s, 0, lane_s, idx);
                 batch_load_bits(s, idx, pre_raw);
             };
@@ -463,14 +455,14 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                 asm volatile("" : "+v"(lane_s));   // (its results would sit in registers, or in scratch memory, across the matrix loop)
 #pragma unroll
                 for (int jb = 0; jb < kSpkSlots; jb += 4) {
-                    if (jb < g.JT) {
+                    if (jb < sk_here(g.JT)) {
                         if constexpr (PRE) {
                             if (jb == 0) {
                                 batch_put_bits(0, lane_s, pre_ok, pre_raw);
                                 continue;
                             }
                         }
-                        int idx[4];
+                        uint32_t idx[4];
                         const uint32_t ok_bits = batch_decode(s, jb, lane_s, idx);
                         if constexpr (IN == SNNF_LAYOUT_BITS) {
                             uint32_t raw[TT][4];
@@ -488,7 +480,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                                 for (int k = 0; k < 8; ++k) {
                                     if (k < g.Cin) {
 #pragma unroll
-                                        for (int j = 0; j < 4; ++j) h[j][k] = src[idx[j] + k * plane];
+                                        for (int j = 0; j < 4; ++j) h[j][k] = src[idx[j] + static_cast<uint32_t>(k * plane)];
                                     } else {
 #pragma unroll
                                         for (int j = 0; j < 4; ++j) h[j][k] = 0u;
@@ -519,7 +511,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                                 }
                                 sk_u32x4 raw[4];
 #pragma unroll
-                                for (int j = 0; j < 4; ++j) raw[j] = *reinterpret_cast<const sk_u32x4*>(src + static_cast<int64_t>(idx[j]) * 16);
+                                for (int j = 0; j < 4; ++j) raw[j] = *reinterpret_cast<const sk_u32x4*>(src + idx[j] * 16u);
 #pragma unroll
                                 for (int j = 0; j < 4; ++j) {
                                     sk_u32x4 d;
@@ -574,20 +566,43 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             if constexpr (PRE) {
                 if (have && s_first < nstages_all) stage_req(s_first);
             }
+            // The accumulators start from the bias: register 4 q + k of fragment f is channel 64 oc_tile + 32 f + 8 q + 4 half + k. With K
+            // split over waves only the first one adds it; the others read the zeros behind it. One value per lane is requested here, right
+            // behind the first stage's activations, and goes through the wave's region of LDS ahead of that stage.
+            const int first_bias = ((!SK || wk == 0) ? oc_tile * (32 * NF) : ((g.nocf + 1) >> 1) * 64) + (NARROW ? l32 : lane);
+            float bias_lane = bias[first_bias];
+            float bias2_lane = 0.0f;
+            if constexpr (SC) bias2_lane = bias2[first_bias];
+            // ---- this lane's output pixel, and where its top-left input sits in the staged halo.
+            int lane_l = l32;
+            asm volatile("" : "+v"(lane_l));
+            const Pack<uint32_t, 2> lane_pos = reinterpret_cast<const Pack<uint32_t, 2>*>(lds + kSpkTableBytes + kSpkDescBytes)[lane_l];
+            const uint32_t lane_b = lane_pos.v[1];
             // The epilogue's view of the tile's channel block, opaque from here on: the scalar arithmetic that depends on it
             // (per-quad base addresses and store predicates, several hundred scalar instructions that the compiler computes
             // ahead of time) then runs after the tile's first loads have been requested, under their latency, instead of in
             // front of them.
             int oc_e = oc_tile;
             asm volatile("" : "+s"(oc_e));
+            auto park_bias = [&]() __attribute__((always_inline)) {
+                if constexpr (SC) bias_lane += bias2_lane;
+                reinterpret_cast<float*>(wlds)[lane] = bias_lane;
+                __builtin_amdgcn_wave_barrier();
 #pragma unroll
-            for (int f = 0; f < NF; ++f)
+                for (int f = 0; f < NF; ++f)
 #pragma unroll
-                for (int q = 0; q < 4; ++q)
+                    for (int q = 0; q < 4; ++q) {
+                        const sk_f32x4 b4 = *reinterpret_cast<const sk_f32x4*>(wlds + (f * 32 + q * 8 + 4 * half) * 4);
 #pragma unroll
-                    for (int t = 0; t < TT; ++t)
+                        for (int k = 0; k < 4; ++k) acc[0][f][4 * q + k] = b4[k];
+                    }
+            };
+            auto start_sums = [&]() __attribute__((always_inline)) {
 #pragma unroll
-                        for (int k = 0; k < 4; ++k) acc[t][f][4 * q + k] = bias4[f][q][k];
+                for (int t = 1; t < TT; ++t)
+#pragma unroll
+                    for (int f = 0; f < NF; ++f) acc[t][f] = acc[0][f];
+            };
             if constexpr (!SK) {
                 // The two waves of a SIMD unit (waves w and w + 4 of the workgroup) run out of phase: the first has the matrix
                 // cores to itself and then runs its epilogue, on the vector unit, under the second one's matrix instructions.
@@ -597,6 +612,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             if (have) {
                 const uint32_t lane16 = static_cast<uint32_t>(lane ^ (quad_x * 8)) * 16u;
                 const unsigned char* __restrict__ bl = wlds + lane_b;
+#pragma clang loop unroll(disable)
                 for (int stage = s_first; stage < nstages_all; stage += s_step) {
                     const bool second = SC && stage >= g.nstages;     // a stage of the shortcut
                     const bool low = SPLIT && stage >= g.nstages;     // a stage of low activation terms: against the high weight terms alone
@@ -643,7 +659,9 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     req_a(1, tb[2]);
                     req_a(2, tb[4]);
                     Pack<uint32_t, 2> ent = tb[6];       // entry of the step whose weights are requested next
+                    if (stage == s_first) park_bias();
                     stage_in(stage);
+                    if (stage == s_first) start_sums();
                     if constexpr (PRE) {
                         if (stage + s_step < nstages_all) stage_req(stage + s_step);
                     }
@@ -735,6 +753,26 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                 }
             }
 
+            else {   // (a wave without a tile: never stored)
+                park_bias();
+                start_sums();
+            }
+
+            // The epilogue reads the geometry and the neuron again, from the (cached) kernel arguments: see sk_here.
+            const auto& args = sk_kernarg_spk();
+            const auto& g = args.g;
+            const LifParams lif = {args.lif.v_threshold, args.lif.v_reset, args.lif.tau, args.lif.inv_tau, args.lif.charge_mode, args.lif.soft_reset};
+            const int po = g.Ho * g.Wo;
+            const int wave_all = wave;
+            const int wave = sk_here(wave_all);
+            const int WK = SK ? (1 << g.wk_log2) : 1;
+            const int wk = SK ? (wave & (WK - 1)) : 0;
+            const int tile_in_block = SK ? (wave >> g.wk_log2) : wave;
+            const int swap_f = SK && !NARROW ? wk >> (g.wk_log2 - 1) : 0;
+            const int quad_x = SK && !NARROW ? (wk << (3 - g.wk_log2)) & 3 : 0;
+            const bool common_lif = lif.charge_mode == CHARGE_SCALE && !lif.soft_reset;
+            const bool half_tau = lif.inv_tau == 0.5f;
+
             // ---- epilogue. Accumulator register 4 q + k of fragment f holds channel 32 f + 8 q + 4 half + k of the lane's
             // pixel: a "quad" (f, q) is the lane's half of channel group j8 = TG oc_tile + 4 f + q. One quad at a time: its bias
             // and membrane (4 + 4 registers) live across its timesteps; a lane's addresses are 32-bit offsets from uniform bases.
@@ -746,10 +784,19 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             void* const v_dst = last_window ? v_store : v_carry;
             const bool v_src16 = !SPLIT && g.v16 && first_window, v_dst16 = !SPLIT && g.v16 && last_window;
             const int t_count = g.shared_x ? g.T : min(TT, g.T - t0);      // LIF steps of this window
-            // (Made opaque here: everything derived from the lane's pixel offset is then computed after the matrix loop instead of
+            // (Made opaque here: everything derived from the lane's pixel is then computed after the matrix loop instead of
             // before it, where the compiler would otherwise park two dozen store addresses in registers or scratch memory.)
-            int pxo_e = pxo, n_e = n_c, half_e = half;
-            asm volatile("" : "+v"(pxo_e), "+v"(n_e), "+v"(half_e));
+            int half_e = half;
+            uint32_t pos_e = lane_pos.v[0];
+            asm volatile("" : "+v"(pos_e), "+v"(half_e));
+            const int pi = static_cast<int>(pos_e & 255u);
+            const int n = n0 + pi;
+            const int oh = oh0 + static_cast<int>((pos_e >> 8) & 255u);
+            const int ow = ow0 + static_cast<int>(pos_e >> 16);
+            const bool px_ok = static_cast<bool>(static_cast<int>(have) & static_cast<int>(pi < g.PI) & static_cast<int>(n < g.N) & static_cast<int>(oh < g.Ho) &
+                                                 static_cast<int>(ow < g.Wo));
+            const int pxo_e = px_ok ? oh * g.Wo + ow : 0;
+            const int n_e = px_ok ? n : 0;
             const uint32_t lane_nchw = static_cast<uint32_t>((n_e * g.Cout + 4 * half_e) * po + pxo_e);        // elements
             const uint32_t lane_c8 = static_cast<uint32_t>(((n_e * g.C8out) * po + pxo_e) * 8 + 4 * half_e);   // elements
             const uint32_t lane_bits = static_cast<uint32_t>((n_e * g.C8out) * po + pxo_e);                  // bytes
@@ -1006,7 +1053,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                 for (int t = 0; t < 4; ++t) w[t] = __umul24((fired >> (4 * (3 - t))) & 15u, 0x00204081u) & 0x01010101u;
                 int lane_e = lane;
                 asm volatile("" : "+v"(lane_e));
-                const uint32_t pos = reinterpret_cast<const uint32_t*>(lds + kSpkTableBytes + kSpkDescBytes)[lane_e & 31];
+                const uint32_t pos = reinterpret_cast<const uint32_t*>(lds + kSpkTableBytes + kSpkDescBytes)[2 * (lane_e & 31)];
                 const int pi_e = static_cast<int>(pos & 255u), prow_e = static_cast<int>((pos >> 8) & 255u), pcol_e = static_cast<int>(pos >> 16);
                 const bool odd_col = (pcol_e & 1) != 0, odd_row = (prow_e & 1) != 0;
                 uint32_t keep0 = odd_col ? w[2] : w[0], keep1 = odd_col ? w[3] : w[1];
