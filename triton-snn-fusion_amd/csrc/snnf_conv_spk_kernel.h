@@ -147,6 +147,11 @@ __device__ __forceinline__ int sk_here(int x) {
     return x;
 }
 
+// Which part of a tile's K a wave has. Waves w and w + 4 share a SIMD: the first parts, which have a stage more where the stages don't divide evenly, go
+// to different SIMDs (72 -> 104 at 28^2 x 5 with a residual, five stages on four waves, 13.2 -> 11.9 us: four stages on the first SIMD and two on each of
+// the others; 80 -> 128 at 20^2 x 6 9.6 -> 9.1; even splits are the same).
+__device__ __forceinline__ int sk_share(int wave, int WK) { return (wave & (WK - 1)) ^ (WK < 8 && wave >= 4 ? WK >> 1 : 0); }
+
 // Entry i of a table of pointers passed by value as a kernel argument, read from the kernel-argument segment (arguments
 // start at offset 0 of that segment, in declaration order and naturally aligned): indexing the by-value struct with a
 // runtime index would copy it to scratch memory.
@@ -253,7 +258,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
     const int tile_t = g.G * region16 + 16;    // bytes of one timestep's stage: its items and one dummy item that absorbs the writes of idle staging slots
 
     const int WK = SK ? (1 << g.wk_log2) : 1;
-    const int wk = SK ? (wave & (WK - 1)) : 0;
+    const int wk = SK ? sk_share(wave, WK) : 0;
     const int tile_in_block = SK ? (wave >> g.wk_log2) : wave;
     const int tiles_per_block = SK ? (kSpkWaves >> g.wk_log2) : kSpkWaves;
     const int nsteps_t = g.shared_x ? 1 : g.T;          // timesteps with a convolution of their own
@@ -766,7 +771,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             const int wave_all = wave;
             const int wave = sk_here(wave_all);
             const int WK = SK ? (1 << g.wk_log2) : 1;
-            const int wk = SK ? (wave & (WK - 1)) : 0;
+            const int wk = SK ? sk_share(wave, WK) : 0;
             const int tile_in_block = SK ? (wave >> g.wk_log2) : wave;
             const int swap_f = SK && !NARROW ? wk >> (g.wk_log2 - 1) : 0;
             const int quad_x = SK && !NARROW ? (wk << (3 - g.wk_log2)) & 3 : 0;
@@ -1474,7 +1479,8 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     // A narrow tile's four quads, all TT timesteps: quad e is finished by wave e mod WK of the tile, which adds the WK
                     // partial sums in a fixed order and then runs that quad's timesteps like the unsplit kernel.
                     __syncthreads();   // every wave is done with its staging region
-                    SNNF_SPK_PARK_QUAD(wave, 0, 0, 0) SNNF_SPK_PARK_QUAD(wave, 1, 0, 1) SNNF_SPK_PARK_QUAD(wave, 2, 0, 2) SNNF_SPK_PARK_QUAD(wave, 3, 0, 3)
+                    const int slot = tile_in_block * WK + wk;      // (in the order of the parts)
+                    SNNF_SPK_PARK_QUAD(slot, 0, 0, 0) SNNF_SPK_PARK_QUAD(slot, 1, 0, 1) SNNF_SPK_PARK_QUAD(slot, 2, 0, 2) SNNF_SPK_PARK_QUAD(slot, 3, 0, 3)
                     const int e_first = wk;      // this wave finishes quads e_first, e_first + WK, ... < 4
                     // The residual bytes of the wave's first quad travel while the workgroup meets.
                     uint32_t rb[TT];
