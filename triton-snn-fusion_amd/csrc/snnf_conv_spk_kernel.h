@@ -608,11 +608,13 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
 #pragma unroll
                     for (int f = 0; f < NF; ++f) acc[t][f] = acc[0][f];
             };
-            if constexpr (!SK) {
-                // The two waves of a SIMD unit (waves w and w + 4 of the workgroup) run out of phase: the first has the matrix
-                // cores to itself and then runs its epilogue, on the vector unit, under the second one's matrix instructions.
-                if (wave < 4) __builtin_amdgcn_s_setprio(2);
-                else __builtin_amdgcn_s_setprio(1);
+            // Waves of several tiles take turns of one tile each: half a tile out of step, one's epilogue runs under the other's matrix instructions, and
+            // both end together (the older wave ahead all the way, the other one's last tile ran alone: 256 -> 256 at 14^2 x 128 105.3 -> 102.9 us,
+            // 128 -> 128 at 28^2 x 128 110.4 -> 104.3; turns of a stage each kept the two in step, 64 -> 64 at 56^2 x 128 99.9 -> 102.4).
+            if (!SK && g.iters > 1) {
+                if (wave >= 4) __builtin_amdgcn_s_setprio(2);
+                else if (it & 1) __builtin_amdgcn_s_setprio(1);
+                else __builtin_amdgcn_s_setprio(3);
             }
             if (have) {
                 const uint32_t lane16 = static_cast<uint32_t>(lane ^ (quad_x * 8)) * 16u;
@@ -671,6 +673,19 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                         if (stage + s_step < nstages_all) stage_req(stage + s_step);
                     }
                     read_b(0, bo[0]);
+                    // The two waves of a SIMD (w and w + 4) share its matrix cores, and the older one wins every instruction at equal priority: it then
+                    // ran through its stages alone, and the other one through its own, with nothing under either's staging. So the wave with more
+                    // stages left goes first (parts of a tile: 128 -> 128 at 28^2 x 16 20.9 -> 20.0 us, 512 -> 512 at 7^2 x 16 19.8 -> 18.9), and where waves have
+                    // several tiles, each in turn for the length of one (half a tile out of step, so that one's epilogue runs under the other's matrix
+                    // instructions, and both end together: 256 -> 256 at 14^2 x 128 98.9 -> 97.0, 128 -> 128 at 28^2 x 128 104.9 -> 100.4). Staging gives way to
+                    // them, unless it takes a second batch of items (64 -> 128 stride 2 at 56^2 x 16 17.3 -> 16.9).
+                    // The two waves of a SIMD (w and w + 4) share its matrix cores, and at equal priority the older one wins every instruction: it ran
+                    // through all its stages, and then the other one through its own, with nothing under either's staging. So a wave on its last stage
+                    // gives way to one that is not (128 -> 128 at 28^2 x 16, two stages per wave, 20.9 -> 20.4 us, 72 -> 104 at 28^2 x 5 12.4 -> 12.1).
+                    if (SK || g.iters == 1) {
+                        if (stage + s_step < nstages_all) __builtin_amdgcn_s_setprio(2);
+                        else __builtin_amdgcn_s_setprio(1);
+                    }
                     int st = 0;
                     // Four steps per trip, no branch inside: weights three steps ahead (4 register sets), activations one step
                     // ahead (2 sets). A wave issues in order and a matrix instruction occupies the matrix pipe for 32 cycles: the
@@ -781,9 +796,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             // ---- epilogue. Accumulator register 4 q + k of fragment f holds channel 32 f + 8 q + 4 half + k of the lane's
             // pixel: a "quad" (f, q) is the lane's half of channel group j8 = TG oc_tile + 4 f + q. One quad at a time: its bias
             // and membrane (4 + 4 registers) live across its timesteps; a lane's addresses are 32-bit offsets from uniform bases.
-            if constexpr (!SK) {
-                if (wave < 4) __builtin_amdgcn_s_setprio(0);
-            }
+            if constexpr (!SK) __builtin_amdgcn_s_setprio(0);
             const bool first_window = t0 == 0, last_window = t0 + TT >= nsteps_t;
             const void* v_src = first_window ? v_init : v_carry;          // later windows continue from the stored membrane
             void* const v_dst = last_window ? v_store : v_carry;
