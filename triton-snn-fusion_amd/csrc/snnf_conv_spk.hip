@@ -332,7 +332,8 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
     // Workgroups that are resident together: one per compute unit, or two where a wave needs at most a quarter of a SIMD's
     // registers (one timestep's accumulators) and two staging areas fit the LDS. The tiles are dealt evenly over as many
     // rounds as that takes.
-    p.lds_bytes = std::max(kSpkHeaderBytes + static_cast<size_t>(kSpkWaves) * g.lds_wave_bytes, wk_log2 > 0 ? kSpkHeaderBytes + kSpkPartialBytes : size_t{0});
+    if (wk_log2 > 0) g.lds_wave_bytes = std::max(g.lds_wave_bytes, kSpkPartialBytes);
+    p.lds_bytes = kSpkHeaderBytes + static_cast<size_t>(kSpkWaves) * g.lds_wave_bytes;
     const int resident = cus * ((tt == 1 && 2 * (p.lds_bytes + 1024) <= kMaxLds) ? 2 : 1);
     const int blocks = (g.n_items + tiles_per_block - 1) / tiles_per_block;
     g.iters = (blocks + resident - 1) / resident;

@@ -36,7 +36,7 @@ constexpr int kSpkWaves = 8;                      // waves per workgroup, one wo
 #define SPK_SLOTS 8
 #endif
 constexpr int kSpkSlots = SPK_SLOTS;                      // staging items per lane and timestep, at most
-constexpr size_t kSpkPartialBytes = kSpkWaves * 16 * 64 * 16;  // split-K: every wave parks 4 quads x up to 4 timesteps of partial sums per round
+constexpr int kSpkPartialBytes = 16 * 64 * 16;     // split-K: a wave parks 4 quads x up to 4 timesteps of partial sums in its region
 constexpr int kSpkMaxSteps = 60;                  // matrix steps per stage, at most (the step table holds 4 more)
 constexpr size_t kSpkTableBytes = (kSpkMaxSteps + 4) * 16;      // the workgroup's step table at the start of LDS
 constexpr int kSpkDescs = 64 * kSpkSlots;                       // staging items of one timestep, at most
@@ -382,7 +382,13 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
         const int64_t w_frag1 = min(ocf0 + 1 - swap_f, g.nocf - 1);
 
         for (int t0 = 0; t0 < nsteps_t; t0 += TT) {
+            // (Defined here, as anything: what is first written under a condition inside a loop is otherwise carried around all loops by the compiler,
+            // 128 registers that are never read again through the whole epilogue.)
             sk_f32x16 acc[TT][NF];
+#pragma unroll
+            for (int t = 0; t < TT; ++t)
+#pragma unroll
+                for (int f = 0; f < NF; ++f) asm("" : "=v"(acc[t][f]));
             // One LDS stage: G channel groups of the patch's halo for TT timesteps, from global memory into this wave's region.
             // Item e = slot * 64 + lane of a timestep = (group, image, row, column) of the halo; its LDS address is 16 e. Items
             // are decoded on the fly (nothing about them is kept in registers across the matrix loop) and move in batches of 4
@@ -569,7 +575,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                 if (low_groups != 0) nstages_all = 2 * g.nstages;
             }
             if constexpr (PRE) {
-                if (have && s_first < nstages_all) stage_req(s_first);
+                stage_req(s_first);      // (there is one for every wave; one without a tile reads the first tile's)
             }
             // The accumulators start from the bias: register 4 q + k of fragment f is channel 64 oc_tile + 32 f + 8 q + 4 half + k. With K
             // split over waves only the first one adds it; the others read the zeros behind it. One value per lane is requested here, right
@@ -787,7 +793,6 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             const int wave = sk_here(wave_all);
             const int WK = SK ? (1 << g.wk_log2) : 1;
             const int wk = SK ? sk_share(wave, WK) : 0;
-            const int tile_in_block = SK ? (wave >> g.wk_log2) : wave;
             const int swap_f = SK && !NARROW ? wk >> (g.wk_log2 - 1) : 0;
             const int quad_x = SK && !NARROW ? (wk << (3 - g.wk_log2)) & 3 : 0;
             const bool common_lif = lif.charge_mode == CHARGE_SCALE && !lif.soft_reset;
@@ -1045,18 +1050,28 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     }
                 }
             };
-            // The same for exactly the four steps of a whole window, without a condition per step: the lower half
-            // stores steps 0 and 2, the upper half steps 1 and 3.
-            auto fast_store4 = [&](int j8, uint32_t quiet) __attribute__((always_inline)) {
-                const uint32_t fired = ~quiet;
-                const auto both = __builtin_amdgcn_permlane32_swap(fired, fired, false, false);
-                if (j8 < g.C8out && px_ok) {
-                    unsigned char* __restrict__ ob = out + static_cast<int64_t>(j8) * po + static_cast<int64_t>(tb) * g.out_step_stride;
-                    const uint32_t first = lane_bits + (half_e ? static_cast<uint32_t>(g.out_step_stride) : 0u);
-                    const uint32_t sh = half_e ? 8u : 12u;
-                    ob[first] = static_cast<unsigned char>(((both[0] >> sh) & 15u) | (((both[1] >> sh) & 15u) << 4));
-                    ob[first + 2u * static_cast<uint32_t>(g.out_step_stride)] =
-                        static_cast<unsigned char>(((both[0] >> (sh - 8u)) & 15u) | (((both[1] >> (sh - 8u)) & 15u) << 4));
+            // The same for exactly the four steps of a whole window, of two quads (or of one, with j8b < 0) at once: step i of a word is its nibble
+            // 3 - i, so that masked nibbles of both halves' words are whole bytes. The lower half stores steps 0 and 2, the upper half steps 1 and 3.
+            const uint32_t step_stride = static_cast<uint32_t>(g.out_step_stride);
+            const uint32_t store_first = lane_bits + (half_e ? step_stride : 0u), store_second = store_first + 2u * step_stride;
+            const uint32_t nib_down = half_e ? 0u : 4u;
+            unsigned char* __restrict__ const out_w = out + static_cast<int64_t>(tb) * g.out_step_stride;
+            auto fast_store4 = [&](int j8a, uint32_t quiet_a, int j8b, uint32_t quiet_b) __attribute__((always_inline)) {
+                const uint32_t word = quiet_a | (quiet_b << 16);
+                const auto both = __builtin_amdgcn_permlane32_swap(word, word, false, false);
+                const uint32_t lo = (both[0] >> nib_down) & 0x0f0f0f0fu, hi = (both[1] << (4u - nib_down)) & 0xf0f0f0f0u;
+                const uint32_t bytes = ~(lo | hi);               // quad a: steps 2 / 3 and 0 / 1 of this half, then quad b's
+                if (px_ok) {
+                    if (j8a < g.C8out) {
+                        unsigned char* __restrict__ ob = out_w + static_cast<int64_t>(j8a) * po;
+                        ob[store_first] = static_cast<unsigned char>(bytes >> 8);
+                        ob[store_second] = static_cast<unsigned char>(bytes);
+                    }
+                    if (j8b >= 0 && j8b < g.C8out) {
+                        unsigned char* __restrict__ ob = out_w + static_cast<int64_t>(j8b) * po;
+                        ob[store_first] = static_cast<unsigned char>(bytes >> 24);
+                        ob[store_second] = static_cast<unsigned char>(bytes >> 16);
+                    }
                 }
             };
             // The four steps 0..3 as 2x2 average pools of the spikes (POOL): the four lanes of a window (patches have even
@@ -1064,32 +1079,36 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             // reduce-scatter of two exchanges (first with the horizontal neighbour, two steps each way; then with the vertical
             // one, one step each way), and the lane at window position (row r, column c) ends up with step 2 c + r, whose
             // four quarters it stores as 16-bit values of the pooled, channel-blocked tensor.
+            bool odd_col = false, odd_row = false;
+            int side = 0, along = 0;
+            uint32_t pool_off = 0;
+            if constexpr (POOL) {
+                const int prow_e = static_cast<int>((pos_e >> 8) & 255u), pcol_e = static_cast<int>(pos_e >> 16);
+                odd_col = (pcol_e & 1) != 0;
+                odd_row = (prow_e & 1) != 0;
+                side = (lane ^ 1) * 4;
+                along = (lane + (odd_row ? -g.PC : g.PC)) * 4;
+                const int hp = g.Ho >> 1, wp = g.Wo >> 1;
+                const uint32_t step = (odd_col ? 2u : 0u) + (odd_row ? 1u : 0u);
+                pool_off = static_cast<uint32_t>(((n * g.C8out * hp + (oh >> 1)) * wp + (ow >> 1)) * 8 + 4 * half_e) * 2u + step * static_cast<uint32_t>(g.out_step_stride);
+            }
             auto fast_store4_pooled = [&](int j8, uint32_t quiet) __attribute__((always_inline)) {
                 const uint32_t fired = ~quiet;
                 uint32_t w[4];
 #pragma unroll
                 for (int t = 0; t < 4; ++t) w[t] = __umul24((fired >> (4 * (3 - t))) & 15u, 0x00204081u) & 0x01010101u;
-                int lane_e = lane;
-                asm volatile("" : "+v"(lane_e));
-                const uint32_t pos = reinterpret_cast<const uint32_t*>(lds + kSpkTableBytes + kSpkDescBytes)[2 * (lane_e & 31)];
-                const int pi_e = static_cast<int>(pos & 255u), prow_e = static_cast<int>((pos >> 8) & 255u), pcol_e = static_cast<int>(pos >> 16);
-                const bool odd_col = (pcol_e & 1) != 0, odd_row = (prow_e & 1) != 0;
                 uint32_t keep0 = odd_col ? w[2] : w[0], keep1 = odd_col ? w[3] : w[1];
                 const uint32_t give0 = odd_col ? w[0] : w[2], give1 = odd_col ? w[1] : w[3];
-                const int side = (lane_e ^ 1) * 4;
                 keep0 += static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(side, static_cast<int>(give0)));
                 keep1 += static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(side, static_cast<int>(give1)));
                 uint32_t keep = odd_row ? keep1 : keep0;
                 const uint32_t give = odd_row ? keep0 : keep1;
-                keep += static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute((lane_e + (odd_row ? -g.PC : g.PC)) * 4, static_cast<int>(give)));
+                keep += static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(along, static_cast<int>(give)));
                 if (j8 < g.C8out && px_ok) {
-                    const int step = (odd_col ? 2 : 0) + (odd_row ? 1 : 0);
-                    const int hp = g.Ho >> 1, wp = g.Wo >> 1;
-                    const uint32_t off = static_cast<uint32_t>(((((n0 + pi_e) * g.C8out + j8) * hp + ((oh0 + prow_e) >> 1)) * wp + ((ow0 + pcol_e) >> 1)) * 8 + 4 * half_e);
                     Pack<XT, 4> q4;
 #pragma unroll
                     for (int k = 0; k < 4; ++k) q4.v[k] = from_float<XT>(static_cast<float>((keep >> (8 * k)) & 255u) * 0.25f);
-                    *reinterpret_cast<Pack<XT, 4>*>(out + static_cast<int64_t>(step) * g.out_step_stride + static_cast<int64_t>(off) * 2) = q4;
+                    *reinterpret_cast<Pack<XT, 4>*>(out + static_cast<int64_t>(j8) * ((g.Ho >> 1) * (g.Wo >> 1)) * 16 + pool_off) = q4;
                 }
             };
             // A quad's membrane from the window before.
@@ -1111,7 +1130,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
 #pragma unroll
                         for (int i = 0; i < 4; ++i) fast_step4(xq[0], i, S, quiet);
                         if constexpr (POOL) fast_store4_pooled(j8, quiet);
-                        else fast_store4(j8, quiet);
+                        else fast_store4(j8, quiet, -1, 0u);
                     } else {
                         for (int ta0 = 0; ta0 < t_count; ta0 += 8) {
                             const int cnt = min(8, t_count - ta0);
@@ -1145,7 +1164,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                         }
                         if constexpr (TT == 4) {
                             if constexpr (POOL) fast_store4_pooled(j8, quiet);
-                            else fast_store4(j8, quiet);
+                            else fast_store4(j8, quiet, -1, 0u);
                         } else {
                             fast_store(tb, TT, j8, quiet);
                         }
@@ -1169,6 +1188,48 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
 #pragma unroll
                     for (int k = 0; k < 4; ++k) vp[lane_nchw + static_cast<uint32_t>(k * po)] = S[k] * unscale;
                 }
+            };
+            // The quads of a usual tile - four steps from a zero membrane that is not asked for - two at a time, without a condition per quad: 8.4 k -> 5.2 k
+            // cycles for a wave's eight quads, 11.5 k -> 7.9 k with a residual (64 -> 64 at 56^2 x 16 19.5 -> 18.4 us and 20.7 -> 19.8).
+            const bool lean = (TT == 4 || TT == 1) && !MULTI && t_count == 4 && v_out == nullptr;
+            auto lean_quad = [&](const float (&xq)[TT][4], const uint32_t (&rb)[TT], auto res_tag) __attribute__((always_inline)) -> uint32_t {
+                float S[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                uint32_t quiet = 0;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if constexpr (decltype(res_tag)::value) {
+                        float x[4];
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) x[k] = xq[i % TT][k];
+                        fast_add_res(rb[i % TT], x);
+                        fast_step4(x, i, S, quiet);
+                    } else {
+                        fast_step4(xq[i % TT], i, S, quiet);
+                    }
+                }
+                return quiet;
+            };
+            // Quad FQ, and FQ + 1 with TWO, of the sums `sum(timestep, quad, k)`, as the channel groups j8a and j8b.
+            auto lean_pair = [&](const auto& sum, auto fq_tag, auto two_tag, auto res_tag, int j8a, int j8b, const uint32_t (&ra)[TT], const uint32_t (&rb)[TT]) __attribute__((always_inline)) {
+                constexpr int FQ = decltype(fq_tag)::value;
+                constexpr bool TWO = decltype(two_tag)::value;
+                uint32_t qa, qb = 0;
+                float xq[TT][4];
+#pragma unroll
+                for (int tw = 0; tw < TT; ++tw)
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) xq[tw][k] = sum(tw, FQ, k);
+                qa = lean_quad(xq, ra, res_tag);
+                if constexpr (POOL) fast_store4_pooled(j8a, qa);
+                if constexpr (TWO) {
+#pragma unroll
+                    for (int tw = 0; tw < TT; ++tw)
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) xq[tw][k] = sum(tw, FQ + 1, k);
+                    qb = lean_quad(xq, rb, res_tag);
+                    if constexpr (POOL) fast_store4_pooled(j8b, qb);
+                }
+                if constexpr (!POOL) fast_store4(j8a, qa, TWO ? j8b : -1, qb);
             };
             // DENSE: dense spikes (and residual) around the usual neuron (tau 2, hard reset), any number of windows and channels. A lane's
             // pixel is one element of a channel plane, so spikes, residual and membrane move as single elements, 32 lanes side by side.
@@ -1340,25 +1401,65 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                         req_res(std::integral_constant<int, 7>{});
                         __builtin_amdgcn_sched_barrier(0);
                     }
-                    auto do_quad = [&](auto fq_tag) __attribute__((always_inline)) {
-                        constexpr int fq = decltype(fq_tag)::value;
-                        if constexpr (fq < TG) {
-                            float xq[TT][4];
-#pragma unroll
-                            for (int tw = 0; tw < TT; ++tw)
-#pragma unroll
-                                for (int k = 0; k < 4; ++k) xq[tw][k] = acc[tw][(fq >> 2) % NF][4 * (fq & 3) + k];
-                            fast_quad(oc_e * TG + fq, xq, rb[fq], with_res, v0[fq]);
+                    auto lean_all = [&](auto res_tag) __attribute__((always_inline)) {
+                        const int j0 = oc_e * TG;
+                        const std::true_type two;
+                        const auto sum = [&](int tw, int fq, int k) __attribute__((always_inline)) { return acc[tw][(fq >> 2) % NF][4 * (fq & 3) + k]; };
+                        lean_pair(sum, std::integral_constant<int, 0>{}, two, res_tag, j0, j0 + 1, rb[0], rb[1]);
+                        lean_pair(sum, std::integral_constant<int, 2>{}, two, res_tag, j0 + 2, j0 + 3, rb[2], rb[3]);
+                        if constexpr (TG == 8) {
+                            lean_pair(sum, std::integral_constant<int, 4>{}, two, res_tag, j0 + 4, j0 + 5, rb[4], rb[5]);
+                            lean_pair(sum, std::integral_constant<int, 6>{}, two, res_tag, j0 + 6, j0 + 7, rb[6], rb[7]);
                         }
                     };
-                    do_quad(std::integral_constant<int, 0>{});
-                    do_quad(std::integral_constant<int, 1>{});
-                    do_quad(std::integral_constant<int, 2>{});
-                    do_quad(std::integral_constant<int, 3>{});
-                    do_quad(std::integral_constant<int, 4>{});
-                    do_quad(std::integral_constant<int, 5>{});
-                    do_quad(std::integral_constant<int, 6>{});
-                    do_quad(std::integral_constant<int, 7>{});
+                    if constexpr (MULTI) {
+                        auto do_quad = [&](auto fq_tag) __attribute__((always_inline)) {
+                            constexpr int fq = decltype(fq_tag)::value;
+                            if constexpr (fq < TG) {
+                                float xq[TT][4];
+#pragma unroll
+                                for (int tw = 0; tw < TT; ++tw)
+#pragma unroll
+                                    for (int k = 0; k < 4; ++k) xq[tw][k] = acc[tw][(fq >> 2) % NF][4 * (fq & 3) + k];
+                                fast_quad(oc_e * TG + fq, xq, rb[fq], with_res, v0[fq]);
+                            }
+                        };
+                        do_quad(std::integral_constant<int, 0>{});
+                        do_quad(std::integral_constant<int, 1>{});
+                        do_quad(std::integral_constant<int, 2>{});
+                        do_quad(std::integral_constant<int, 3>{});
+                        do_quad(std::integral_constant<int, 4>{});
+                        do_quad(std::integral_constant<int, 5>{});
+                        do_quad(std::integral_constant<int, 6>{});
+                        do_quad(std::integral_constant<int, 7>{});
+                    } else if (lean && !with_res) {
+                        lean_all(std::false_type{});
+                    } else if (lean && TT == 4) {
+                        lean_all(std::true_type{});
+                    } else {
+                        // A loop: a quad's sums are copied out of the accumulators by a switch (constant register indices).
+                        for (int fq = 0; fq < TG; ++fq) {
+                            float xq[TT][4];
+                            uint32_t rq[TT];
+#define SNNF_SPK_COPY_QUAD(F, Q)                                                                                          \
+    _Pragma("unroll") for (int tw = 0; tw < TT; ++tw) {                                                                   \
+        _Pragma("unroll") for (int k = 0; k < 4; ++k) xq[tw][k] = acc[tw][(F) % NF][4 * (Q) + k];                         \
+        rq[tw] = rb[4 * (F) + (Q)][tw];                                                                                   \
+    }
+                            switch (fq) {
+                                case 0: SNNF_SPK_COPY_QUAD(0, 0); break;
+                                case 1: SNNF_SPK_COPY_QUAD(0, 1); break;
+                                case 2: SNNF_SPK_COPY_QUAD(0, 2); break;
+                                case 3: SNNF_SPK_COPY_QUAD(0, 3); break;
+                                case 4: SNNF_SPK_COPY_QUAD(1, 0); break;
+                                case 5: SNNF_SPK_COPY_QUAD(1, 1); break;
+                                case 6: SNNF_SPK_COPY_QUAD(1, 2); break;
+                                default: SNNF_SPK_COPY_QUAD(1, 3); break;
+                            }
+#undef SNNF_SPK_COPY_QUAD
+                            fast_quad(oc_e * TG + fq, xq, rq, with_res, v0[0]);
+                        }
+                    }
                 } else if constexpr (DENSE) {
                     DenseIn in[2] = {};
                     dense_request(oc_e * TG, in[0]);
@@ -1405,95 +1506,186 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     }
                 }
             } else {
-                // Split K: the WK waves of a tile add their partial sums through LDS (the staging regions are dead by then).
-                float* __restrict__ part = reinterpret_cast<float*>(lds + kSpkHeaderBytes);      // [wave][e 0..3][tw][lane][4]
-                // Quad Q of fragment F goes to place P of slot S (a slot per wave).
+                // Split K: the WK waves of a tile add their partial sums through LDS. A wave's slot is its own staging region, which it has read when it
+                // parks its sums there: the waves that are done first park while the others still multiply, and the workgroup meets once before the first
+                // sums are read. With that, reads that are all requested before the first is waited for (in turn, 16 latencies of 130 cycles), one round
+                // instead of two between the last four waves, the residual bytes of all quads under way from the start, and the lean quads above, a wave
+                // of 128 -> 128 at 28^2 x 16 has its sums 3.4 k cycles after its last product instead of 4.4 k and is done 2.3 k later instead of 4.5 k, at
+                // 512 -> 512, 7^2 x 16 5.1 k instead of 7.0 k (20.2 -> 19.3 us, 18.9 -> 18.5; 64 -> 128 stride 2 16.9 -> 16.1, 72 -> 104 at 28^2 x 5 with a residual 11.9 -> 11.1).
+                unsigned char* __restrict__ part = lds + kSpkHeaderBytes;      // [wave][place 0..3][tw][lane][4 floats]
+                const int slot_bytes = g.lds_wave_bytes;
+                int lane_p = lane;                       // opaque: the addresses below are computed here, not ahead of the matrix loop
+                asm volatile("" : "+v"(lane_p));
+                // Quad Q of fragment F goes to place P of slot S.
 #define SNNF_SPK_PARK_QUAD(S, P, F, Q)                                                                                           \
     _Pragma("unroll") for (int tw = 0; tw < TT; ++tw) {                                                                          \
         const sk_f32x4 four = {acc[tw][(F) % NF][4 * (Q)], acc[tw][(F) % NF][4 * (Q) + 1], acc[tw][(F) % NF][4 * (Q) + 2], acc[tw][(F) % NF][4 * (Q) + 3]};  \
-        *reinterpret_cast<sk_f32x4*>(part + ((((S) * 4 + (P)) * TT + tw) * 64 + lane) * 4) = four;                              \
-    }
-                // The sums at place P of slot S are added to quad Q of the first fragment.
-#define SNNF_SPK_ADD_QUAD(S, P, Q)                                                                                               \
-    _Pragma("unroll") for (int tw = 0; tw < TT; ++tw) {                                                                          \
-        const sk_f32x4 four = *reinterpret_cast<const sk_f32x4*>(part + ((((S) * 4 + (P)) * TT + tw) * 64 + lane_x) * 4);        \
-        _Pragma("unroll") for (int k = 0; k < 4; ++k) acc[tw][0][4 * (Q) + k] += four[k];                                        \
+        *reinterpret_cast<sk_f32x4*>(part + (S) * slot_bytes + (((P) * TT + tw) * 64 + lane_p) * 16) = four;                      \
     }
                 if constexpr (!NARROW) {
                     // Halves are exchanged until every wave owns 8 / WK quads: first the fragment that a wave does not finish, then two
-                    // quads of its own, then one. All waves add and finish at the same time; a slot that a wave has read takes what it
+                    // quads of its own (three of eight waves). All waves add and finish at the same time; a slot that a wave has read takes what it
                     // gives away next. (Quads parked by all waves and summed by one each, in two rounds of which half of eight waves
                     // took no part, took 23.4 us at 512 -> 512, 7^2 x 16 against 22.4, 21.8 against 21.2 at 256 -> 256, 14^2 x 16, and in two windows 25.7
                     // against 22.3 at 128 -> 256 stride 2, 40^2 x 3, T = 8; 1.04 over 60 such layers.)
-                    __syncthreads();   // every wave is done with its staging region
                     SNNF_SPK_PARK_QUAD(wave, 0, 1, 0) SNNF_SPK_PARK_QUAD(wave, 1, 1, 1) SNNF_SPK_PARK_QUAD(wave, 2, 1, 2) SNNF_SPK_PARK_QUAD(wave, 3, 1, 3)
                     const int jq = oc_e * TG + 4 * swap_f;
-                    uint32_t rb[TT];
+                    const int quads = 8 >> g.wk_log2;
+                    // The residual bytes (and membranes of the window before) of all of the wave's quads travel while the workgroup meets: a second round
+                    // trip for the second quad and on, after the sums had met, was 0.8 k cycles each.
+                    uint32_t rb[4][TT];
+                    float v0[4][4];
+                    DenseIn in = {};
 #pragma unroll
-                    for (int tw = 0; tw < TT; ++tw) rb[tw] = 0u;
-                    if constexpr (FAST) {   // the residual bytes of the first quad travel while the workgroup meets
+                    for (int e = 0; e < 4; ++e) {
+#pragma unroll
+                        for (int tw = 0; tw < TT; ++tw) rb[e][tw] = 0u;
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) v0[e][k] = 0.0f;
+                    }
+                    if constexpr (FAST) {
                         if (g.res_layout >= 0 && TT > 1) {
+                            const unsigned char* res_t[TT];
 #pragma unroll
-                            for (int tw = 0; tw < TT; ++tw) rb[tw] = fast_res(tb + min(tw, t_count - 1), jq + quad_x);
+                            for (int tw = 0; tw < TT; ++tw) res_t[tw] = static_cast<const unsigned char*>(sk_kernarg_ptr(kResTable, tb + min(tw, t_count - 1)));
+#pragma unroll
+                            for (int e = 0; e < 4; ++e)
+                                if (e < quads) {
+                                    const uint32_t off = lane_bits + static_cast<uint32_t>(min(jq + (e ^ quad_x), g.C8out - 1) * po);
+#pragma unroll
+                                    for (int tw = 0; tw < TT; ++tw) rb[e][tw] = res_t[tw][off];
+                                }
+                        }
+                        if constexpr (MULTI) {
+#pragma unroll
+                            for (int e = 0; e < 4; ++e)
+                                if (e < quads) fast_v0(jq + (e ^ quad_x), v0[e]);
                         }
                     }
-                    float v0[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-                    if constexpr (FAST) fast_v0(jq + quad_x, v0);
-                    DenseIn in = {};
                     if constexpr (DENSE) dense_request(jq + quad_x, in);
                     __syncthreads();
-                    int lane_x = lane;                   // opaque: the addresses below are computed here, not ahead of the matrix loop
-                    asm volatile("" : "+v"(lane_x));
                     const int across = wave ^ (WK >> 1);
-                    SNNF_SPK_ADD_QUAD(across, 0, 0) SNNF_SPK_ADD_QUAD(across, 1, 1) SNNF_SPK_ADD_QUAD(across, 2, 2) SNNF_SPK_ADD_QUAD(across, 3, 3)
-                    if (WK > 2) {
-                        const int from = across ^ (WK >> 2);
-                        SNNF_SPK_PARK_QUAD(across, 2, 0, 2) SNNF_SPK_PARK_QUAD(across, 3, 0, 3)
-                        __syncthreads();
-                        SNNF_SPK_ADD_QUAD(from, 2, 0) SNNF_SPK_ADD_QUAD(from, 3, 1)
-                        if (WK > 4) {
-                            SNNF_SPK_PARK_QUAD(from, 2, 0, 1)
-                            __syncthreads();
-                            SNNF_SPK_ADD_QUAD(from ^ 1, 2, 0)
+                    unsigned char* const mine = part + across * slot_bytes + lane_p * 16;      // the slot that this wave reads, and takes for its own from then on
+                    // Place `place` of slot `slot`: a quad of all timesteps.
+                    auto take = [&](int slot, int place, sk_f32x4 (&four)[TT]) __attribute__((always_inline)) {
+#pragma unroll
+                        for (int tw = 0; tw < TT; ++tw) four[tw] = *reinterpret_cast<const sk_f32x4*>(part + slot * slot_bytes + ((place * TT + tw) * 64 + lane_p) * 16);
+                    };
+                    auto give = [&](int place, const sk_f32x4 (&four)[TT]) __attribute__((always_inline)) {
+#pragma unroll
+                        for (int tw = 0; tw < TT; ++tw) *reinterpret_cast<sk_f32x4*>(mine + (place * TT + tw) * 1024) = four[tw];
+                    };
+                    auto add = [&](sk_f32x4 (&to)[TT], const sk_f32x4 (&four)[TT]) __attribute__((always_inline)) {
+#pragma unroll
+                        for (int tw = 0; tw < TT; ++tw)
+#pragma unroll
+                            for (int k = 0; k < 4; ++k) to[tw][k] += four[tw][k];
+                    };
+                    sk_f32x4 own[4][TT];
+                    {
+                        sk_f32x4 sums[4][TT];            // (all requested before the first is waited for: one latency instead of sixteen)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) take(across, q, sums[q]);
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+#pragma unroll
+                            for (int tw = 0; tw < TT; ++tw)
+#pragma unroll
+                                for (int k = 0; k < 4; ++k) own[q][tw][k] = acc[tw][0][4 * q + k];
+                            add(own[q], sums[q]);
                         }
                     }
-                    const int quads = 8 >> g.wk_log2;
-                    for (int e = 0; e < quads; ++e) {
-                        const int j8 = jq + (e ^ quad_x);
-                        float xq[TT][4];
-#define SNNF_SPK_COPY_QUAD(F, Q)                                          \
-    _Pragma("unroll") for (int tw = 0; tw < TT; ++tw)                     \
-        _Pragma("unroll") for (int k = 0; k < 4; ++k) xq[tw][k] = acc[tw][(F) % NF][4 * (Q) + k]
-                        switch (e) {
-                            case 0: SNNF_SPK_COPY_QUAD(0, 0); break;
-                            case 1: SNNF_SPK_COPY_QUAD(0, 1); break;
-                            case 2: SNNF_SPK_COPY_QUAD(0, 2); break;
-                            default: SNNF_SPK_COPY_QUAD(0, 3); break;
-                        }
-#undef SNNF_SPK_COPY_QUAD
-                        const int j8_next = jq + ((e + 1) ^ quad_x);
-                        if constexpr (FAST) {
-                            if (e != 0 && g.res_layout >= 0 && TT > 1) {
-#pragma unroll
-                                for (int tw = 0; tw < TT; ++tw) rb[tw] = fast_res(tb + min(tw, t_count - 1), j8);
+                    // The wave's finished quads: run at once (FAST, usual tiles), or left in LDS for the loop below.
+                    auto finish = [&](auto quads_tag) __attribute__((always_inline)) {
+                        constexpr int QUADS = decltype(quads_tag)::value;
+                        if constexpr (FAST && (TT == 4 || TT == 1)) {
+                            const auto sum = [&](int tw, int q, int k) __attribute__((always_inline)) { return own[q][tw][k]; };
+                            auto lean_all = [&](auto res_tag) __attribute__((always_inline)) {
+                                lean_pair(sum, std::integral_constant<int, 0>{}, std::integral_constant<bool, (QUADS > 1)>{}, res_tag, jq + quad_x, jq + (1 ^ quad_x), rb[0], rb[1]);
+                                if constexpr (QUADS == 4) lean_pair(sum, std::integral_constant<int, 2>{}, std::true_type{}, res_tag, jq + 2, jq + 3, rb[2], rb[3]);
+                            };
+                            if (lean && g.res_layout < 0) {
+                                lean_all(std::false_type{});
+                                return;
                             }
-                            const float start[4] = {v0[0], v0[1], v0[2], v0[3]};
-                            if (e + 1 < quads) fast_v0(j8_next, v0);
-                            fast_quad(j8, xq, rb, g.res_layout >= 0, start);
-                        } else if constexpr (DENSE) {
-                            const DenseIn now = in;
-                            if (e + 1 < quads) dense_request(j8_next, in);
-                            dense_quad(j8, xq, now);
-                        } else {
-                            general_quad(j8, xq);
+                            if (lean && TT == 4) {
+                                lean_all(std::true_type{});
+                                return;
+                            }
+                        }
+#pragma unroll
+                        for (int q = 0; q < QUADS; ++q) give(q, own[q]);
+                    };
+                    if (WK == 2) {
+                        finish(std::integral_constant<int, 4>{});
+                    } else if (WK == 4) {
+                        give(2, own[2]);
+                        give(3, own[3]);
+                        __syncthreads();
+                        sk_f32x4 sums[2][TT];
+                        take(across ^ 1, 2, sums[0]);
+                        take(across ^ 1, 3, sums[1]);
+                        __builtin_amdgcn_sched_barrier(0);
+                        add(own[0], sums[0]);
+                        add(own[1], sums[1]);
+                        finish(std::integral_constant<int, 2>{});
+                    } else {
+                        // Of four waves each keeps one quad and gives the others theirs, added as (own + second) + (first + third).
+                        give(1, own[1]);
+                        give(2, own[2]);
+                        give(3, own[3]);
+                        __syncthreads();
+                        sk_f32x4 first[TT], second[TT], third[TT];
+                        take(across ^ 2, 2, second);
+                        take(across ^ 1, 1, first);
+                        take(across ^ 3, 3, third);
+                        __builtin_amdgcn_sched_barrier(0);
+                        add(own[0], second);
+                        add(first, third);
+                        add(own[0], first);
+                        finish(std::integral_constant<int, 1>{});
+                    }
+                    if (!(FAST && lean && (TT == 4 || (TT == 1 && g.res_layout < 0)))) {
+                        for (int e = 0; e < quads; ++e) {
+                            const int j8 = jq + (e ^ quad_x);
+                            float xq[TT][4];
+#pragma unroll
+                            for (int tw = 0; tw < TT; ++tw) {
+                                const sk_f32x4 four = *reinterpret_cast<const sk_f32x4*>(mine + (e * TT + tw) * 1024);
+#pragma unroll
+                                for (int k = 0; k < 4; ++k) xq[tw][k] = four[k];
+                            }
+                            if constexpr (FAST) {
+                                float start[4] = {v0[0][0], v0[0][1], v0[0][2], v0[0][3]};
+                                uint32_t rq[TT];
+#pragma unroll
+                                for (int tw = 0; tw < TT; ++tw) rq[tw] = rb[0][tw];
+                                if (e > 0) {     // (constant register indices)
+#pragma unroll
+                                    for (int q = 1; q < 4; ++q)
+                                        if (e == q) {
+#pragma unroll
+                                            for (int tw = 0; tw < TT; ++tw) rq[tw] = rb[q][tw];
+#pragma unroll
+                                            for (int k = 0; k < 4; ++k) start[k] = v0[q][k];
+                                        }
+                                }
+                                fast_quad(j8, xq, rq, g.res_layout >= 0, start);
+                            } else if constexpr (DENSE) {
+                                const DenseIn now = in;
+                                if (e + 1 < quads) dense_request(jq + ((e + 1) ^ quad_x), in);
+                                dense_quad(j8, xq, now);
+                            } else {
+                                general_quad(j8, xq);
+                            }
                         }
                     }
                 } else {
                     // A narrow tile's four quads, all TT timesteps: quad e is finished by wave e mod WK of the tile, which adds the WK
                     // partial sums in a fixed order and then runs that quad's timesteps like the unsplit kernel.
-                    __syncthreads();   // every wave is done with its staging region
-                    const int slot = tile_in_block * WK + wk;      // (in the order of the parts)
-                    SNNF_SPK_PARK_QUAD(slot, 0, 0, 0) SNNF_SPK_PARK_QUAD(slot, 1, 0, 1) SNNF_SPK_PARK_QUAD(slot, 2, 0, 2) SNNF_SPK_PARK_QUAD(slot, 3, 0, 3)
+                    SNNF_SPK_PARK_QUAD(wave, 0, 0, 0) SNNF_SPK_PARK_QUAD(wave, 1, 0, 1) SNNF_SPK_PARK_QUAD(wave, 2, 0, 2) SNNF_SPK_PARK_QUAD(wave, 3, 0, 3)
+                    const int part0 = wave ^ wk;         // the slot of part k is part0 ^ k
                     const int e_first = wk;      // this wave finishes quads e_first, e_first + WK, ... < 4
                     // The residual bytes of the wave's first quad travel while the workgroup meets.
                     uint32_t rb[TT];
@@ -1518,27 +1710,35 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                         const int j8 = oc_e * TG + e_own;
                         float xq[TT][4];
                         {
-                            // The partial sums of the tile's waves, all timesteps of a wave (of two waves) in flight together (WK is a power
-                            // of two >= 2); added in the order of the waves.
+                            // The partial sums of the tile's waves, all timesteps of two or four waves in flight together (WK is a power of two >= 2); added
+                            // in the order of the parts.
                             sk_f32x4 sum[TT];
 #pragma unroll
                             for (int tw = 0; tw < TT; ++tw) sum[tw] = sk_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                            auto add_parts = [&](auto n_tag, int k) __attribute__((always_inline)) {
+                                constexpr int PARTS = decltype(n_tag)::value;
+                                sk_f32x4 p[PARTS][TT];
+#pragma unroll
+                                for (int i = 0; i < PARTS; ++i)
+#pragma unroll
+                                    for (int tw = 0; tw < TT; ++tw) p[i][tw] = *reinterpret_cast<const sk_f32x4*>(part + (part0 ^ (k + i)) * slot_bytes + ((e_own * TT + tw) * 64 + lane_p) * 16);
+                                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                                for (int i = 0; i < PARTS; ++i)
+#pragma unroll
+                                    for (int tw = 0; tw < TT; ++tw)
+#pragma unroll
+                                        for (int c = 0; c < 4; ++c) sum[tw][c] += p[i][tw][c];
+                            };
                             if constexpr (FAST || DENSE) {
-                                for (int k = 0; k < WK; k += 2) {
-                                    sk_f32x4 p0[TT], p1[TT];
-#pragma unroll
-                                    for (int tw = 0; tw < TT; ++tw) {
-                                        p0[tw] = *reinterpret_cast<const sk_f32x4*>(part + ((((tile_in_block * WK + k) * 4 + e_own) * TT + tw) * 64 + lane) * 4);
-                                        p1[tw] = *reinterpret_cast<const sk_f32x4*>(part + ((((tile_in_block * WK + k + 1) * 4 + e_own) * TT + tw) * 64 + lane) * 4);
-                                    }
-#pragma unroll
-                                    for (int tw = 0; tw < TT; ++tw) sum[tw] = (sum[tw] + p0[tw]) + p1[tw];
-                                }
+                                if (WK == 2) add_parts(std::integral_constant<int, 2>{}, 0);
+                                else
+                                    for (int k = 0; k < WK; k += 4) add_parts(std::integral_constant<int, 4>{}, k);
                             } else {   // the general epilogue has no registers to spare: one wave's sums at a time
                                 for (int k = 0; k < WK; ++k) {
 #pragma unroll
                                     for (int tw = 0; tw < TT; ++tw)
-                                        sum[tw] += *reinterpret_cast<const sk_f32x4*>(part + ((((tile_in_block * WK + k) * 4 + e_own) * TT + tw) * 64 + lane) * 4);
+                                        sum[tw] += *reinterpret_cast<const sk_f32x4*>(part + (part0 ^ k) * slot_bytes + ((e_own * TT + tw) * 64 + lane_p) * 16);
                                 }
                             }
 #pragma unroll
@@ -1553,7 +1753,13 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                             }
                             const float start[4] = {v0[0], v0[1], v0[2], v0[3]};
                             if (e_own + WK < 4) fast_v0(j8 + WK, v0);
-                            fast_quad(j8, xq, rb, g.res_layout >= 0, start);
+                            if (lean && (g.res_layout < 0 || TT == 4)) {
+                                const uint32_t quiet = g.res_layout < 0 ? lean_quad(xq, rb, std::false_type{}) : lean_quad(xq, rb, std::true_type{});
+                                if constexpr (POOL) fast_store4_pooled(j8, quiet);
+                                else fast_store4(j8, quiet, -1, 0u);
+                            } else {
+                                fast_quad(j8, xq, rb, g.res_layout >= 0, start);
+                            }
                         } else if constexpr (DENSE) {
                             const DenseIn now = in;
                             if (e_own + WK < 4) dense_request(j8 + WK, in);
@@ -1565,7 +1771,6 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                 }
             }
 #undef SNNF_SPK_PARK_QUAD
-#undef SNNF_SPK_ADD_QUAD
             if constexpr (SK) __syncthreads();   // the partial sums are read before the next window's staging overwrites them
         }
     }
