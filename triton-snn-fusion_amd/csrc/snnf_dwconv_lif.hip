@@ -4,7 +4,7 @@
 // LDS. A workgroup owns PB consecutive (n, c) planes (or a band of TH output rows of one plane), keeps an fp32 copy of
 // the input band with a zero halo in LDS, and every thread keeps the fp32 membrane of its PX-wide output strips in
 // registers for the whole time loop.
-#include "snnf_common.h"
+#include "snnf_conv_common.h"
 
 namespace snnf {
 namespace {
@@ -303,6 +303,153 @@ int launch(const StepPtrs& xs, const StepPtrs& res, int has_res, int T, DwGeom g
 }
 
 // ---------------------------------------------------------------------------------------------------------------
+// Stride 2, 16-bit activations in rows of whole 16-byte vectors, without LDS: a lane reads the three input rows of its strip of 4 outputs
+// straight from memory, 16 bytes and the dword in front of them per row. Half of the rows belong to two strips and come from the vector cache
+// the second time, so a step costs a lane six loads, no barrier, no transposition and no tile to zero; lanes of a wave read
+// contiguous rows. (On the tile of `dwconv3x3_lif_kernel` a lane takes 17 floats of a row one by one, 16 floats from its neighbour's: the reads
+// of a wave fall into a few of the LDS banks.) Padding comes from the range check of buffer loads, which answers zero beyond the frame.
+// What bounds it: HBM. 64 channels at 64x64 x 32, T = 4 (84 MB and 8 MB of membrane) 42.4 -> 19.0 us, 128 at 32x32 x 32 25.3 -> 10.0,
+// one image
+// 11.1 -> 5.2 (48x48) and 9.8 -> 5.0 (24x24). The same without LDS at stride 1, where every row is read three times and a strip takes nine loads, lost: 128 channels
+// at 56x56 x 32 and the pointwise layer behind them 126 -> 145 us.
+// ---------------------------------------------------------------------------------------------------------------
+typedef uint32_t dw_u32x4 __attribute__((ext_vector_type(4)));
+
+// The lower and the upper element of a dword of two 16-bit values.
+template <typename XT> __device__ __forceinline__ float low_element(uint32_t d) { return to_float(XT{static_cast<uint16_t>(d)}); }
+template <typename XT> __device__ __forceinline__ float high_element(uint32_t d) { return to_float(XT{static_cast<uint16_t>(d >> 16)}); }
+template <> __device__ __forceinline__ float high_element<bf16_t>(uint32_t d) { return __uint_as_float(d & 0xffff0000u); }
+
+constexpr int64_t kDirectMaxFrame = 0x7fffff00ll;     // bytes of one timestep's input: offsets from 2^31 on lie outside
+constexpr uint32_t kDirectOutside = 0x80000000u;
+constexpr int kDirectPx = 4;                          // outputs of a strip
+
+struct DwDirect {
+    int strips;              // output strips in all: N * C * Ho * (Wo / 4)
+    int C, H, W, Ho, SW;     // SW: strips per output row
+    uint32_t frame_bytes;
+    FastDiv d_SW, d_Ho, d_C;
+};
+
+// The two pointer tables MUST be the first two kernel parameters.
+template <typename XT, typename VT, bool STD>
+__global__ __launch_bounds__(kThreads) void dwconv3x3_s2_lif_direct_kernel(StepPtrs xs, StepPtrs residuals, int has_residual, int T, DwDirect g,
+                                                                           const XT* __restrict__ weight, const XT* __restrict__ bias,
+                                                                           const VT* v_init, XT* __restrict__ spikes, int64_t spike_step_stride,
+                                                                           VT* v_out, LifParams lif) {
+    constexpr int PX = kDirectPx;
+    static_assert(sizeof(XT) == 2, "strips of one 16-byte vector per input row");
+    const int i = static_cast<int>(blockIdx.x) * kThreads + static_cast<int>(threadIdx.x);
+    if (i >= g.strips) return;
+    const int orow = fast_div(i, g.d_SW);
+    const int strip = i - orow * g.SW;
+    const int plane = fast_div(orow, g.d_Ho);
+    const int oh = orow - plane * g.Ho;
+    const int c = plane - fast_div(plane, g.d_C) * g.C;
+    const int64_t out = static_cast<int64_t>(i) * PX;       // elements
+
+    uint32_t mid[3], left[3];
+#pragma unroll
+    for (int kh = 0; kh < 3; ++kh) {
+        const int ih = oh * 2 - 1 + kh;
+        const bool in = ih >= 0 && ih < g.H;
+        const uint32_t off = static_cast<uint32_t>((plane * g.H + ih) * g.W + strip * 8) * 2u;
+        mid[kh] = in ? off : kDirectOutside;
+        left[kh] = in && strip > 0 ? off - 4u : kDirectOutside;
+    }
+    dw_u32x4 x[3];
+    uint32_t xl[3];
+    Pack<XT, PX> res = {};
+    auto issue_loads = [&](int t) __attribute__((always_inline)) {
+        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(dw_table_entry(0, t)), 0, g.frame_bytes, 0x00027000);
+#pragma unroll
+        for (int kh = 0; kh < 3; ++kh) {
+            x[kh] = __builtin_bit_cast(dw_u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, mid[kh], 0, 0));
+            xl[kh] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, left[kh], 0, 0);
+        }
+        if (has_residual) res = *reinterpret_cast<const Pack<XT, PX>*>(static_cast<const XT*>(dw_table_entry(sizeof(StepPtrs), t)) + out);
+    };
+    issue_loads(0);
+
+    float w[9];
+#pragma unroll
+    for (int j = 0; j < 9; ++j) w[j] = to_float(weight[c * 9 + j]);
+    const float b = to_float(bias[c]);
+    float v[PX];
+    if (v_init != nullptr) {
+        load_strip_as_float<VT, PX>(v_init + out, v);
+    } else {
+#pragma unroll
+        for (int j = 0; j < PX; ++j) v[j] = 0.0f;
+    }
+
+    for (int t = 0; t < T; ++t) {
+        float acc[PX];
+#pragma unroll
+        for (int j = 0; j < PX; ++j) acc[j] = b;
+#pragma unroll
+        for (int kh = 0; kh < 3; ++kh) {
+            float in[9];                  // input columns -1 .. 7 of the strip
+            in[0] = high_element<XT>(xl[kh]);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                in[1 + 2 * k] = low_element<XT>(x[kh][k]);
+                in[2 + 2 * k] = high_element<XT>(x[kh][k]);
+            }
+#pragma unroll
+            for (int j = 0; j < PX; ++j)
+#pragma unroll
+                for (int kw = 0; kw < 3; ++kw) acc[j] = fmaf(in[j * 2 + kw], w[kh * 3 + kw], acc[j]);
+        }
+        if (has_residual) {
+#pragma unroll
+            for (int j = 0; j < PX; ++j) acc[j] += to_float(res.v[j]);
+        }
+        if (t + 1 < T) issue_loads(t + 1);
+        Pack<XT, PX> s;
+#pragma unroll
+        for (int j = 0; j < PX; ++j) {
+            bool fired;
+            if constexpr (STD) {
+                const float h = v[j] + (acc[j] - v[j]) * lif.inv_tau;
+                fired = h >= lif.v_threshold;
+                v[j] = fired ? lif.v_reset : h;
+            } else {
+                fired = lif_step(acc[j], v[j], lif);
+            }
+            s.v[j] = spike_value<XT>(fired);
+        }
+        *reinterpret_cast<Pack<XT, PX>*>(spikes + t * spike_step_stride + out) = s;
+    }
+    Pack<VT, PX> vo;
+#pragma unroll
+    for (int j = 0; j < PX; ++j) vo.v[j] = from_float<VT>(v[j]);
+    *reinterpret_cast<Pack<VT, PX>*>(v_out + out) = vo;
+}
+
+template <typename XT, typename VT>
+int launch_direct(const StepPtrs& xs, const StepPtrs& res, int has_res, int T, const DwGeom& g, const void* weight, const void* bias, const void* v_init,
+                  void* spikes, int64_t spike_step_stride, void* v_out, const LifParams& lif, hipStream_t stream) {
+    DwDirect d = {};
+    d.C = g.C;
+    d.H = g.H;
+    d.W = g.W;
+    d.Ho = g.Ho;
+    d.SW = g.W / 8;
+    d.strips = g.planes * g.Ho * d.SW;
+    d.frame_bytes = static_cast<uint32_t>(static_cast<int64_t>(g.planes) * g.H * g.W * 2);
+    d.d_SW = make_fast_div(d.SW);
+    d.d_Ho = make_fast_div(d.Ho);
+    d.d_C = make_fast_div(d.C);
+    const dim3 grid((static_cast<unsigned>(d.strips) + kThreads - 1) / kThreads);
+    auto kernel = lif.charge_mode == CHARGE_SCALE && !lif.soft_reset ? dwconv3x3_s2_lif_direct_kernel<XT, VT, true>
+                                                                     : dwconv3x3_s2_lif_direct_kernel<XT, VT, false>;
+    kernel<<<grid, kThreads, 0, stream>>>(xs, res, has_res, T, d, static_cast<const XT*>(weight), static_cast<const XT*>(bias),
+                                          static_cast<const VT*>(v_init), static_cast<XT*>(spikes), spike_step_stride, static_cast<VT*>(v_out), lif);
+    return check_launch("snnf_dwconv3x3_lif");
+}
+
+// ---------------------------------------------------------------------------------------------------------------
 // Stride 1, strips of 8 pixels, 16-bit activations: the LDS tile keeps the activations in their 16-bit form (a prefetched
 // vector goes in with one 16-byte write and no conversion) and the taps run on the packed dot-product instruction
 // (two 16-bit products added to an fp32 accumulator): the products are exact in fp32, as with an fp32 multiply-add, and an
@@ -312,7 +459,6 @@ int launch(const StepPtrs& xs, const StepPtrs& res, int has_res, int T, DwGeom g
 // the strip at elements e0 .. e0 + 7 (e0 a multiple of 8) a row costs one 16-byte read and the two dwords around it.
 // ---------------------------------------------------------------------------------------------------------------
 constexpr int kDotColOffset = 8;
-typedef uint32_t dw_u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 dw_bf16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 dw_f16x2 __attribute__((ext_vector_type(2)));
 
@@ -592,23 +738,27 @@ int launch_dot(const StepPtrs& xs, const StepPtrs& res, int has_res, int T, DwGe
 
 
 template <typename XT, typename VT, int STRIDE>
-int dispatch_px(int px, const StepPtrs& xs, const StepPtrs& res, int has_res, int T, const DwGeom& g,
+int dispatch_px(int px, bool direct, const StepPtrs& xs, const StepPtrs& res, int has_res, int T, const DwGeom& g,
                 const void* weight, const void* bias, const void* v_init, void* spikes, int64_t sss, void* v_out,
                 const LifParams& lif, hipStream_t stream) {
-    if constexpr (STRIDE == 1 && sizeof(XT) == 2) {
-        if (px == 8) return launch_dot<XT, VT>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
+    if constexpr (sizeof(XT) == 2) {
+        if (direct) {
+            if constexpr (STRIDE == 1) return launch_dot<XT, VT>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
+            else return launch_direct<XT, VT>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
+        }
+    } else if (px == 8) {
+        return launch<XT, VT, STRIDE, 8>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
     }
-    if (px == 8) return launch<XT, VT, STRIDE, 8>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
-    if (px == 4) return launch<XT, VT, STRIDE, 4>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
+    if (px >= 4) return launch<XT, VT, STRIDE, 4>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
     return launch<XT, VT, STRIDE, 1>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
 }
 
 template <typename XT, typename VT>
-int dispatch_stride(int stride, int px, const StepPtrs& xs, const StepPtrs& res, int has_res, int T, const DwGeom& g,
+int dispatch_stride(int stride, int px, bool direct, const StepPtrs& xs, const StepPtrs& res, int has_res, int T, const DwGeom& g,
                     const void* weight, const void* bias, const void* v_init, void* spikes, int64_t sss, void* v_out,
                     const LifParams& lif, hipStream_t stream) {
-    if (stride == 1) return dispatch_px<XT, VT, 1>(px, xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
-    return dispatch_px<XT, VT, 2>(px, xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
+    if (stride == 1) return dispatch_px<XT, VT, 1>(px, direct, xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
+    return dispatch_px<XT, VT, 2>(px, direct, xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
 }
 
 // One byte of row-packed spikes -> eight 0 / 1 elements (16 bytes).
@@ -792,18 +942,24 @@ extern "C" int snnf_dwconv3x3_lif(const void* const* xs, const void* const* resi
             xp.p[t] = xs[t0 + t];
             if (residuals != nullptr) rp.p[t] = residuals[t0 + t];
         }
+        // 16-bit activations in strips of 8 input columns (`direct`): the dot-product kernel at stride 1, the kernel without LDS at stride 2, whose strips
+        // are 4 outputs wide (a plane of whole vectors and 16-byte aligned steps; frames within its 32-bit offsets). What is left of
+        // 16-bit calls takes at most 4 outputs a strip.
+        bool direct = x_dtype != SNNF_F32 && W % 8 == 0 && px >= 8 / stride &&
+                      (stride == 1 || static_cast<int64_t>(g.planes) * H * W * xsize <= kDirectMaxFrame);
+        for (int t = 0; t < tw && direct; ++t) direct = aligned_to(xs[t0 + t], 16);
         const int has_res = residuals != nullptr ? 1 : 0;
         int rc;
         if (x_dtype == SNNF_F32) {
-            rc = dispatch_stride<float, float>(stride, px, xp, rp, has_res, tw, g, weight, bias, vi, sp, spike_step_stride, v_out, lif, hs);
+            rc = dispatch_stride<float, float>(stride, px, direct, xp, rp, has_res, tw, g, weight, bias, vi, sp, spike_step_stride, v_out, lif, hs);
         } else if (x_dtype == SNNF_BF16) {
             rc = v_dtype == SNNF_F32
-                     ? dispatch_stride<bf16_t, float>(stride, px, xp, rp, has_res, tw, g, weight, bias, vi, sp, spike_step_stride, v_out, lif, hs)
-                     : dispatch_stride<bf16_t, bf16_t>(stride, px, xp, rp, has_res, tw, g, weight, bias, vi, sp, spike_step_stride, v_out, lif, hs);
+                     ? dispatch_stride<bf16_t, float>(stride, px, direct, xp, rp, has_res, tw, g, weight, bias, vi, sp, spike_step_stride, v_out, lif, hs)
+                     : dispatch_stride<bf16_t, bf16_t>(stride, px, direct, xp, rp, has_res, tw, g, weight, bias, vi, sp, spike_step_stride, v_out, lif, hs);
         } else {
             rc = v_dtype == SNNF_F32
-                     ? dispatch_stride<f16_t, float>(stride, px, xp, rp, has_res, tw, g, weight, bias, vi, sp, spike_step_stride, v_out, lif, hs)
-                     : dispatch_stride<f16_t, f16_t>(stride, px, xp, rp, has_res, tw, g, weight, bias, vi, sp, spike_step_stride, v_out, lif, hs);
+                     ? dispatch_stride<f16_t, float>(stride, px, direct, xp, rp, has_res, tw, g, weight, bias, vi, sp, spike_step_stride, v_out, lif, hs)
+                     : dispatch_stride<f16_t, f16_t>(stride, px, direct, xp, rp, has_res, tw, g, weight, bias, vi, sp, spike_step_stride, v_out, lif, hs);
         }
         if (rc != SNNF_OK) return rc;
     }
