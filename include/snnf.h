@@ -439,7 +439,8 @@ int snnf_conv_blocked_tune(int T, int N, int Cin, int H, int W, int Cout, int KH
 /* Describes what the most recent snnf_conv_lif / snnf_conv_bias call on this thread selected: kernel family, timesteps per launch, tile
  * and wave decomposition, LDS bytes, grid ("key=value" pairs, empty before the first call). A layer that snnf_conv_lif_ws brought
  * into the channel-blocked layout says route=c8 and ran=blocked: "kernel" is then the family that snnf_conv_lif would have run it
- * on, the rest describes the launch of the blocked kernel (whose tiles hold "oc_tile" = 32 or 64 output channels). Plays the role of the
+ * on, the rest describes the launch of the blocked kernel (whose tiles hold "oc_tile" = 32 or 64 output channels).
+ * few=IxRxCx16xG: a layer of few output pixels, which G workgroups of 16 channels and I images x R x C pixels run instead of those tiles. Plays the role of the
  * reference's get_autotune_best_config (kernels/benchmark_conv_lif_temporal_general.py:1332-1369), whose result the
  * operator layer publishes as kernel_temporal_config (runtime/snn_custom_ops.py:341-353): selection here is a
  * deterministic planner, and this is how a host reads its decision. The pointer stays valid for the thread's lifetime. */

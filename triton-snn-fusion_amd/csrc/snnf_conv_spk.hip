@@ -9,6 +9,7 @@
 #include <memory>
 #include <mutex>
 
+#include "snnf_conv_few.h"
 #include "snnf_conv_spk_kernel.h"
 
 namespace snnf {
@@ -216,6 +217,9 @@ struct BlockedPlan {
     int tt = 0, windows = 0, wk_log2 = 0, oc_tiles = 0, grid = 0;
     size_t lds_bytes = 0;
     bool tuned_patch = false, tuned_split = false;
+    bool few = false;                                  // the kernel for few output pixels runs instead
+    FewGeom few_g = {};
+    size_t few_lds = 0;
 };
 
 // Everything that decides whether and how the kernel runs a call; nothing is enqueued.
@@ -382,6 +386,24 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
         g.sc_npairs = pg2.npairs;
         g.sc_frag_stride = static_cast<int64_t>(pg2.nchunks) * pg2.npairs * (kFragBytes / 2);
     }
+    // Layers whose K several waves share, in few tiles: the kernel for few pixels. One that could be pooled takes it with and without its pool or not at
+    // all, so that the pooled launch has the sums of the unpooled one.
+    if (neuron && !c.split && !shared && sc == nullptr && wk_log2 > 0 && !p.tuned_patch && !p.tuned_split && (c.out_layout != SNNF_LAYOUT_C8 || pool2) && c.res_layout != SNNF_LAYOUT_C8) {
+        FewGeom& f = p.few_g;
+        f.N = N; f.C8in = g.C8in; f.H = H; f.W = W; f.Cout = Cout; f.C8out = g.C8out; f.KH = KH; f.KW = KW;
+        f.sh = stride_h; f.sw = stride_w; f.ph = pad_h; f.pw = pad_w; f.Ho = g.Ho; f.Wo = g.Wo; f.T = T;
+        f.taps = g.taps; f.kw_mul = g.kw_mul;
+        f.res_layout = c.res_layout; f.out_layout = c.out_layout; f.pool = pool2 ? 1 : 0;
+        const FewGeom blank = f;
+        const bool poolable = T == 4 && (g.Ho & 1) == 0 && (g.Wo & 1) == 0 && Cout % 8 == 0 && c.res_layout < 0 && c.out_layout != SNNF_LAYOUT_NCHW;
+        p.few = plan_few(f, pg, p.few_lds);
+        if (p.few && poolable) {
+            FewGeom other = blank;
+            size_t other_lds;
+            other.pool = pool2 ? 0 : 1;
+            p.few = plan_few(other, pg, other_lds);
+        }
+    }
     return SNNF_OK;
 }
 
@@ -397,6 +419,11 @@ void plan_text(char* text, const BlockedPlan& p, const char* kernel, int epilogu
              kernel, (p.wk_log2 > 0 ? 50 : 40) + p.tt + epilogue, window, from_dense ? 2 : 1, g.PI, g.PR, g.PC, g.RR, g.RC, 1 << p.wk_log2, p.oc_tiles,
              g.narrow ? 32 : 64, g.n_patches, g.G, p.lds_bytes, p.grid, (p.tuned_patch ? 1 : 0) + (p.tuned_split ? 2 : 0), g.sc_stages,
              from_dense ? " route=c8 ran=blocked" : "");
+    // A launch of few pixels: the workgroups (images x rows x columns x channels x their number) that run instead of the tiles above.
+    if (p.few) {
+        const size_t n = strlen(text);
+        snprintf(text + n, 256 - n, " few=%dx%dx%dx16x%d", p.few_g.PI, p.few_g.PR, p.few_g.PC, p.few_g.grid);
+    }
 }
 
 // Whether a layer takes the blocked route: where the rule sends it there and the kernel then runs it. A layer that the planner refuses
@@ -726,6 +753,15 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     if (pool2) {
         if (!fast_epi || p.windows != 1 || (p.tt != 4 && !shared))
             return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_pool: the pooled output needs the usual neuron (tau 2, hard reset to 0) and the four steps in one window", who);
+    }
+    if (p.few) {
+        FewLaunch F = {L.xs, L.residuals, p.few_g, L.wpacked, L.bias, L.v_start, L.out, L.v_store, L.lif, p.few_lds, L.stream};
+        F.g.out_step_stride = out_step_stride;
+        F.g.v16 = L.g.v16;
+        F.g.v_in_place = L.g.v_in_place;
+        return launch_conv_few(F, x_dtype == SNNF_F16, x_layout);
+    }
+    if (pool2) {
         if (x_layout == SNNF_LAYOUT_NCHW) return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_frame(L, true) : launch_conv_spk_f16_frame(L, true);
         return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_pooled(L, p.tt) : launch_conv_spk_f16_pooled(L, p.tt);
     }
