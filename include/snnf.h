@@ -438,7 +438,7 @@ int snnf_conv_blocked_tune(int T, int N, int Cin, int H, int W, int Cout, int KH
 
 /* Describes what the most recent snnf_conv_lif / snnf_conv_bias call on this thread selected: kernel family, timesteps per launch, tile
  * and wave decomposition, LDS bytes, grid ("key=value" pairs, empty before the first call). A layer that snnf_conv_lif_ws brought
- * into the channel-blocked layout says route=c8 and ran=blocked: "kernel" is then the family that snnf_conv_lif would have run it
+ * into the channel-blocked layout says route=c8 and ran=blocked, a frame for all timesteps that it read as it is route=frame: "kernel" is then the family that snnf_conv_lif would have run it
  * on, the rest describes the launch of the blocked kernel (whose tiles hold "oc_tile" = 32 or 64 output channels).
  * few=IxRxCx16xG: a layer of few output pixels, which G workgroups of 16 channels and I images x R x C pixels run instead of those tiles. Plays the role of the
  * reference's get_autotune_best_config (kernels/benchmark_conv_lif_temporal_general.py:1332-1369), whose result the

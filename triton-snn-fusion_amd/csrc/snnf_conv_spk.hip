@@ -74,11 +74,17 @@ bool plan_spk(const SpkGeom& g0, int tt, SpkPlan& best, int only_pc = 0, int onl
         // Wide patches store longer runs of a row; stages of 4 slots move in one batch.
         double score = eff / (1.0 + 0.08 * (halo - 1.0)) * (1.0 + 0.004 * std::min(pc, 16));
         if (G * region > 256) score *= 0.97;
+        // A frame whose spikes leave as dense tensors is bound by its stores, 2-byte elements side by side along a row: what a pixel costs goes with the 64-byte
+        // lines that a patch row touches (of row starts anywhere), and runs that are no multiple of 32 bytes share more of them. us in patches of
+        // 8, 14, 16, 28 and 32 columns: 3 -> 64 7x7 stride 2 at 224^2 x 16 62.6, 56.8, 48.5, 51.8, 49.6, at 112^2 x 28 32.1, 32.6, 27.8, 25.1, 24.7, 3x3 at
+        // 32^2 x 64 21.4, 22.8, 15.3, 18.1, 14.2, 3 -> 100 at 33^2 x 9 11.2, 9.5, 9.4, 10.8, 10.9.
+        const bool dense_frame = g0.in_layout == SNNF_LAYOUT_NCHW && g0.out_layout == SNNF_LAYOUT_NCHW;
+        if (dense_frame) score = eff / ((0.85 + 4.8 * (1.0 + (pc - 1) / 32.0) / pc) * (pc % 16 == 0 ? 1.0 : 1.12));
         // Waves own whole tiles: a launch of a little more than one round of waves takes as long as one of two. 88 -> 176 channels at
         // 43^2 x 5 is 1980 tiles of 4 x 8 pixels (31 us) or 2205 of 4 x 7 (53 us) on 2048 waves. Among patches of several rounds the fewer
         // tiles win (256 -> 256 at 14^2 x 128: 3584 of 2 x 14 99 us, 4096 of 4 x 8 103 us).
         const int64_t tiles = static_cast<int64_t>(img_groups) * patches_x * patches_y * oc_tiles, slots = static_cast<int64_t>(cus) * kSpkWaves;
-        if (tiles > slots) score *= 0.6;
+        if (tiles > slots && !dense_frame) score *= 0.6;
         if (score > best.score) best = SpkPlan{pr, pc, pi, rr, rc, region, G, patches_x, patches_y, img_groups, score};
     }
     return best.score > 0.0;
@@ -411,14 +417,15 @@ const char* family_name(DenseFamily f) {
     return f == DenseFamily::kTInM ? "t_in_m" : (f == DenseFamily::kTimeOuter ? "time_outer" : (f == DenseFamily::kPointwise ? "pointwise" : "matrix"));
 }
 
-void plan_text(char* text, const BlockedPlan& p, const char* kernel, int epilogue, int window, bool from_dense) {
+enum DenseRouteKind { kNoRoute, kCopyRoute, kFrameRoute };
+void plan_text(char* text, const BlockedPlan& p, const char* kernel, int epilogue, int window, DenseRouteKind route) {
     const SpkGeom& g = p.g;
     snprintf(text, 256,
              "kernel=%s variant=%d window=%d launches=%d tile=%dx%dx%d halo=%dx%d waves=8x1x%d oc_tiles=%d oc_tile=%d px_tiles=%d "
              "stage_chunks=%d run=0 lds=%zu grid=%d tuned=%d shortcut_stages=%d%s",
-             kernel, (p.wk_log2 > 0 ? 50 : 40) + p.tt + epilogue, window, from_dense ? 2 : 1, g.PI, g.PR, g.PC, g.RR, g.RC, 1 << p.wk_log2, p.oc_tiles,
+             kernel, (p.wk_log2 > 0 ? 50 : 40) + p.tt + epilogue, window, route == kCopyRoute ? 2 : 1, g.PI, g.PR, g.PC, g.RR, g.RC, 1 << p.wk_log2, p.oc_tiles,
              g.narrow ? 32 : 64, g.n_patches, g.G, p.lds_bytes, p.grid, (p.tuned_patch ? 1 : 0) + (p.tuned_split ? 2 : 0), g.sc_stages,
-             from_dense ? " route=c8 ran=blocked" : "");
+             route == kCopyRoute ? " route=c8 ran=blocked" : (route == kFrameRoute ? " route=frame ran=blocked" : ""));
     // A launch of few pixels: the workgroups (images x rows x columns x channels x their number) that run instead of the tiles above.
     if (p.few) {
         const size_t n = strlen(text);
@@ -430,7 +437,7 @@ void plan_text(char* text, const BlockedPlan& p, const char* kernel, int epilogu
 // (offsets, a kernel of too many steps, no patch that fits) gets no scratch memory asked for. Without a neuron the dense route has the
 // matrix kernel only; what it refuses stays refused. The answer depends on the layer and the table of tuned plans alone and is
 // kept per layer with the plan and its text (made anew in each call they took 0.6 of its 11.5 us; it asks twice).
-using RouteKey = std::array<int, 15>;
+using RouteKey = std::array<int, 16>;
 struct KeptPlan {
     BlockedPlan plan;
     char text[2][256];                                 // with the general and with the dense epilogue
@@ -442,12 +449,14 @@ std::map<RouteKey, Route>& routes() {
     return known;
 }
 constexpr size_t kMaxRoutes = 4096;
+constexpr int64_t kMostFrameOutputs = 3ll << 25;      // elements, of a frame's layer on the blocked kernel (see takes_frame)
 
+// `frame`: one input of at most eight channels for all timesteps, which the kernel reads as it is.
 Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w,
-                    int v_dtype, bool residual, bool neuron) {
+                    int v_dtype, bool residual, bool neuron, bool frame = false) {
     if (!valid_dtype(x_dtype) || (v_dtype != SNNF_F32 && v_dtype != x_dtype)) return {false, DenseFamily::kTInM, nullptr};
     const bool split = x_dtype == SNNF_F32;
-    const RouteKey key = {T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, residual ? 1 : 0, neuron ? 1 : 0, split ? 1 : 0};
+    const RouteKey key = {T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, residual ? 1 : 0, neuron ? 1 : 0, split ? 1 : 0, frame ? 1 : 0};
     {
         std::lock_guard<std::mutex> lock(routes_mutex);
         const auto it = routes().find(key);
@@ -456,13 +465,17 @@ Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, 
     Route route = {false, DenseFamily::kTInM, nullptr};
     route.taken = takes_blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residual, neuron, route.family) &&
                   (neuron || (!split && (route.family == DenseFamily::kMatrixMasked || route.family == DenseFamily::kMatrixWhole)));
+    if (frame)                                         // (see takes_frame)
+        route.taken = route.family != DenseFamily::kPointwise &&
+                      static_cast<int64_t>(T) * N * Cout * ((H + 2 * pad_h - KH) / stride_h + 1) * ((W + 2 * pad_w - KW) / stride_w + 1) <= kMostFrameOutputs;
     if (route.taken) {
         const auto kept = std::make_shared<KeptPlan>();
         BlockedPlan& plan = kept->plan;
-        route.taken = plan_blocked("snnf_conv_lif_scratch_bytes", BlockedCall{T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, SNNF_LAYOUT_C8,
-                                   residual ? SNNF_LAYOUT_NCHW : -1, SNNF_LAYOUT_NCHW, 0, false, neuron, false, neuron, false, nullptr, split}, plan) == SNNF_OK;
+        route.taken = plan_blocked("snnf_conv_lif_scratch_bytes", BlockedCall{T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w,
+                                   frame ? SNNF_LAYOUT_NCHW : SNNF_LAYOUT_C8, residual ? SNNF_LAYOUT_NCHW : -1, SNNF_LAYOUT_NCHW, 0, frame, neuron, false, neuron, false,
+                                   nullptr, split}, plan) == SNNF_OK;
         if (route.taken) {
-            for (int dense_epi = 0; dense_epi < 2; ++dense_epi) plan_text(kept->text[dense_epi], plan, family_name(route.family), dense_epi ? 40 : 0, plan.tt, true);
+            for (int dense_epi = 0; dense_epi < 2; ++dense_epi) plan_text(kept->text[dense_epi], plan, family_name(route.family), dense_epi ? 40 : 0, frame ? T : plan.tt, frame ? kFrameRoute : kCopyRoute);
             route.kept = kept;
         }
     }
@@ -478,7 +491,7 @@ int64_t carried_membrane(const Route& r, int v_dtype, int N, int H, int W, int C
     return static_cast<int64_t>(N) * Cout * ((H + 2 * pad_h - KH) / stride_h + 1) * ((W + 2 * pad_w - KW) / stride_w + 1);
 }
 
-// A call on dense tensors that runs here: its inputs, which are brought into C8 first, and the kernel family of the dense route.
+// A call on dense tensors that runs here: its inputs, which are brought into C8 first (null: a frame, which is read as it is), and its plan.
 struct DenseRoute {
     const void* const* xs;
     const KeptPlan* kept;
@@ -578,25 +591,46 @@ extern "C" size_t snnf_conv_bias_workspace_bytes(int T, int N, int Cin, int H, i
 
 namespace snnf {
 namespace {
+// One dense 16-bit frame of at most eight channels for all timesteps (the first layer of a network) around the usual neuron (tau 2, hard reset) goes to the
+// blocked kernel, which reads the frame as it is and needs no scratch memory (us, matrix kernel / here, T = 4, bf16): 3 -> 64 7x7 stride 2 at 224^2 x 16 62.8 / 48.5, one
+// image 14.6 / 9.9, 3x3 at 32^2 x 64 19.7 / 14.2, one image 11.5 / 6.9, 3 -> 32 stride 2 at 128^2 x 32 33.3 / 14.6, 1 -> 64 5x5 at 28^2 x 50 18.6 / 14.6, 4 -> 96 at 50^2 x 20
+// 40.3 / 20.3, 8 -> 128 at 56^2 x 16 35.5 / 25.4; T = 8 3 -> 64 3x3 at 32^2 x 64 25.8 / 18.7, 4 -> 96 60.3 / 31.2. What the pointwise kernel takes stays there (8 -> 256 1x1 at
+// 56^2 x 16 33.4 / 50.9), and outputs beyond 100 million elements, of which the matrix kernel writes whole lines (7x7 at 224^2 x 16, T = 8, 103 million, 112 / 117). Other neurons take its general epilogue, which is slower than the matrix kernel's
+// (77.5 at 224^2 x 16), and stay.
+bool takes_frame(bool shared, int T, int Cin, int x_dtype, int v_dtype, bool residual, const LifParams& lif) {
+    return shared && T <= SNNF_MAX_T_PER_LAUNCH && Cin <= 8 && (x_dtype == SNNF_BF16 || x_dtype == SNNF_F16) && v_dtype == SNNF_F32 && !residual &&
+           lif.charge_mode == CHARGE_SCALE && lif.inv_tau == 0.5f && !lif.soft_reset;
+}
+
 // The blocked route of a call on dense tensors: SNNF_ERR_UNSUPPORTED (nothing enqueued) when it does not apply.
 int run_blocked_route(const void* const* xs, const void* const* residuals, int T, int N, int Cin, int H, int W, int x_dtype, const void* packed_weight,
                       int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w, const void* v_init, int v_dtype, void* out,
                       int64_t out_step_stride, void* v_out, int neuron, float v_threshold, float v_reset, float tau, void* workspace,
                       size_t workspace_bytes, void* stream) {
-    if (xs == nullptr || workspace == nullptr || (neuron && v_out == nullptr) || !aligned_to(workspace, 16) || out_step_stride < 0) return SNNF_ERR_UNSUPPORTED;
+    if (xs == nullptr || (neuron && v_out == nullptr) || out_step_stride < 0 || T < 1 || T > SNNF_MAX_T_PER_LAUNCH || N < 1 || Cin < 1 || H < 1 || W < 1 || Cout < 1 ||
+        KH < 1 || KW < 1 || stride_h < 1 || stride_w < 1 || pad_h < 0 || pad_w < 0 || H + 2 * pad_h < KH || W + 2 * pad_w < KW || 2 * pad_h > KH || 2 * pad_w > KW || tau == 0.0f)
+        return SNNF_ERR_UNSUPPORTED;
+    bool shared = T > 1;
+    for (int t = 0; t < T; ++t) {
+        if (xs[t] == nullptr) return SNNF_ERR_UNSUPPORTED;
+        shared = shared && xs[t] == xs[0];
+    }
+    if (neuron && takes_frame(shared, T, Cin, x_dtype, v_dtype, residuals != nullptr, make_lif_params(v_threshold, v_reset, tau))) {
+        const Route frame = blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, false, true, true);
+        if (!frame.taken) return SNNF_ERR_UNSUPPORTED;
+        const DenseRoute route = {nullptr, frame.kept.get(), RouteSpace{}, v_dtype};
+        return conv_lif_blocked_impl("snnf_conv_lif", xs, SNNF_LAYOUT_NCHW, nullptr, SNNF_LAYOUT_NCHW, T, N, Cin, H, W, x_dtype, packed_weight, Cout, KH, KW, stride_h, stride_w,
+                                     pad_h, pad_w, v_init, out, SNNF_LAYOUT_NCHW, out_step_stride * dtype_size(x_dtype), v_out, 1, v_threshold, v_reset, tau, stream, nullptr,
+                                     false, &route);
+    }
+    if (workspace == nullptr || !aligned_to(workspace, 16) || shared) return SNNF_ERR_UNSUPPORTED;   // one frame for all timesteps is convolved once on the dense kernels too
     const Route taken = blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residuals != nullptr, neuron != 0);
     if (!taken.taken) return SNNF_ERR_UNSUPPORTED;
     const RouteSpace space = route_space(T, N, Cin, H, W, x_dtype == SNNF_F32,
                                          neuron ? carried_membrane(taken, v_dtype, N, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w) : 0);
     if (workspace_bytes < space.total) return SNNF_ERR_UNSUPPORTED;
-    bool shared = T > 1;
     const void* inner[SNNF_MAX_T_PER_LAUNCH];
-    for (int t = 0; t < T; ++t) {
-        if (xs[t] == nullptr) return SNNF_ERR_UNSUPPORTED;
-        shared = shared && xs[t] == xs[0];
-        inner[t] = static_cast<const char*>(workspace) + t * space.step;
-    }
-    if (shared) return SNNF_ERR_UNSUPPORTED;       // one frame for all timesteps is convolved once on the dense kernels too
+    for (int t = 0; t < T; ++t) inner[t] = static_cast<const char*>(workspace) + t * space.step;
     const DenseRoute route = {xs, taken.kept.get(), space, v_dtype};
     return conv_lif_blocked_impl(neuron ? "snnf_conv_lif" : "snnf_conv_bias", inner, SNNF_LAYOUT_C8, residuals, SNNF_LAYOUT_NCHW, T, N, Cin, H, W, x_dtype,
                                  packed_weight, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_init, out, SNNF_LAYOUT_NCHW, out_step_stride * dtype_size(x_dtype), v_out,
@@ -729,14 +763,16 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
                           L.lif.v_threshold >= 1e-30f && L.lif.v_threshold <= 1e30f &&   // its multiples by 2^t stay normal numbers
                           v_init == nullptr && (p.windows == 1 || p.tt == 4) && Cout % 8 == 0;
     // Dense tensors around the neuron: no range limit on the threshold, any reset potential, initial membrane, windows and channels.
-    const bool dense_epi = neuron && x_layout == SNNF_LAYOUT_C8 && out_layout == SNNF_LAYOUT_NCHW && (residuals == nullptr || res_layout == SNNF_LAYOUT_NCHW) &&
-                           L.lif.charge_mode == CHARGE_SCALE && L.lif.inv_tau == 0.5f && !L.lif.soft_reset && L.v_store != nullptr && !shared;
+    // (A frame for all timesteps: without a residual, with or without a membrane.)
+    const bool frame_epi = x_layout == SNNF_LAYOUT_NCHW && shared && residuals == nullptr;
+    const bool dense_epi = neuron && (frame_epi || (x_layout == SNNF_LAYOUT_C8 && !shared && L.v_store != nullptr)) && out_layout == SNNF_LAYOUT_NCHW &&
+                           (residuals == nullptr || res_layout == SNNF_LAYOUT_NCHW) && L.lif.charge_mode == CHARGE_SCALE && L.lif.inv_tau == 0.5f && !L.lif.soft_reset;
     if (dense != nullptr) memcpy(snnf::conv_plan_buffer(), dense->kept->text[dense_epi ? 1 : 0], 256);
-    else plan_text(snnf::conv_plan_buffer(), p, "blocked", fast_epi ? 20 : (dense_epi ? 40 : 0), shared ? T : p.tt, false);
+    else plan_text(snnf::conv_plan_buffer(), p, "blocked", fast_epi ? 20 : (dense_epi ? 40 : 0), shared ? T : p.tt, kNoRoute);
     L.fast_epilogue = fast_epi;
     L.multi_window = p.windows > 1;
     L.dense_epilogue = dense_epi;
-    if (dense != nullptr) {   // the plan stands: bring the dense inputs into the C8 buffers behind `xs`
+    if (dense != nullptr && dense->xs != nullptr) {   // the plan stands: bring the dense inputs into the C8 buffers behind `xs`
         StepPtrs from = {};
         for (int t = 0; t < T; ++t) from.p[t] = dense->xs[t];
         char* const base = static_cast<char*>(const_cast<void*>(xs[0]));

@@ -237,7 +237,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
     static_assert(!NARROW || SK || (!SC && (!POOL || IN == SNNF_LAYOUT_NCHW)), "narrow tiles of one wave: not of a shortcut, and pooled only of a dense frame");
     static_assert(!SPLIT || (NARROW && IN == SNNF_LAYOUT_C8 && !FAST && !SC && !POOL), "fp32 tensors: narrow tiles on two C8 tensors, dense tensors out");
     static_assert(!MULTI || (FAST && !POOL), "several windows belong to the straight-line epilogue");
-    static_assert(!DENSE || (IN == SNNF_LAYOUT_C8 && !FAST && !SC && !POOL), "the dense epilogue belongs to calls on dense tensors");
+    static_assert(!DENSE || (IN != SNNF_LAYOUT_BITS && !FAST && !SC && !POOL), "the dense epilogue belongs to calls on dense tensors");
     // No two of the membrane arguments are the same memory: a call in place passes no v_start, and only one with a 16-bit membrane has a
     // v_scratch. (Promising nothing here instead cost the straight-line epilogue 2 %: ResNet-18, 16 images of 224x224 361 -> 369 us.)
     float* const v_out = static_cast<float*>(v_store);
@@ -245,6 +245,9 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
     float* const v_carry = g.v16 ? v_scratch : v_out;
     constexpr int NF = NARROW ? 1 : 2;         // 32-channel weight fragments of a tile
     constexpr int TG = 4 * NF;                 // channel groups of 8 of a tile
+    // A dense frame with dense spikes is computed as the matrix kernel computes it (which takes frames per timestep, and other neurons): the bias
+    // behind the sums, the charge as v + (x - v) / 2. One frame T times and T equal frames have the same results, bit for bit.
+    constexpr bool LATE_BIAS = DENSE && IN == SNNF_LAYOUT_NCHW;
     constexpr bool F16 = dtype_of<XT>::value == SNNF_F16;
     constexpr uint32_t ONE = F16 ? 0x3c00u : 0x3f80u;
     constexpr int kResTable = static_cast<int>(sizeof(StepPtrs));
@@ -596,6 +599,13 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             int oc_e = oc_tile;
             asm volatile("" : "+s"(oc_e));
             auto park_bias = [&]() __attribute__((always_inline)) {
+                if constexpr (LATE_BIAS) {
+#pragma unroll
+                    for (int f = 0; f < NF; ++f)
+#pragma unroll
+                        for (int k = 0; k < 16; ++k) acc[0][f][k] = 0.0f;
+                    return;
+                }
                 if constexpr (SC) bias_lane += bias2_lane;
                 reinterpret_cast<float*>(wlds)[lane] = bias_lane;
                 __builtin_amdgcn_wave_barrier();
@@ -1237,10 +1247,12 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             // 12 us in single elements and in runs of 16 bytes alike. The residual (and the membrane of a previous window) of a
             // quad is requested one quad ahead: waited for in turn it cost 28 us on 64 -> 64 at 56^2 x 16 (67 -> 39 us without).
             using DT = typename std::conditional<SPLIT, uint32_t, uint16_t>::type;     // an element's bits
-            struct DenseIn { uint32_t res[TT][4]; uint32_t v[4]; };
+            constexpr bool FRAME = LATE_BIAS;                   // one sum for all steps, no residual
+            struct DenseIn { uint32_t res[TT][4]; uint32_t v[4]; sk_f32x4 bias; };
             auto dense_request = [&](int j8_any, DenseIn& in) __attribute__((always_inline)) {
                 const int j8 = min(j8_any, g.C8out - 1);
                 const int left = g.Cout - (j8 * 8 + 4 * half_e);     // channels of this lane's quad, and beyond
+                if constexpr (FRAME) in.bias = *reinterpret_cast<const sk_f32x4*>(bias + j8 * 8 + 4 * half_e);     // (zeros beyond the last)
                 auto get = [&](auto ragged_tag) __attribute__((always_inline)) {
                     constexpr bool RAGGED = decltype(ragged_tag)::value;
                     // Lanes without a pixel read pixel 0 of image 0; channels beyond the last are not read.
@@ -1290,24 +1302,29 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                 auto run = [&](auto ragged_tag) __attribute__((always_inline)) {
                     constexpr bool RAGGED = decltype(ragged_tag)::value;
                     if (px_ok && left > 0) {
+                        auto step = [&](int t, int tw) __attribute__((always_inline)) {
+                            DT* __restrict__ op = reinterpret_cast<DT*>(out + static_cast<int64_t>(t) * g.out_step_stride) + static_cast<int64_t>(j8) * 8 * po;
 #pragma unroll
-                        for (int tw = 0; tw < TT; ++tw) {
-                            if (tw < t_count) {
-                                DT* __restrict__ op = reinterpret_cast<DT*>(out + static_cast<int64_t>(t0 + tw) * g.out_step_stride) + static_cast<int64_t>(j8) * 8 * po;
-#pragma unroll
-                                for (int k = 0; k < 4; ++k) {
-                                    float x = xq[tw][k];
-                                    if (g.res_layout >= 0) {
-                                        if constexpr (SPLIT) x += __uint_as_float(in.res[tw][k]);
-                                        else x += to_float(XT{static_cast<uint16_t>(in.res[tw][k])});
-                                    }
-                                    const float h = (v[k] + x) * 0.5f;
-                                    const bool fired = h >= lif.v_threshold;
-                                    v[k] = fired ? lif.v_reset : h;
-                                    const DT spike = fired ? static_cast<DT>(SPLIT ? 0x3f800000u : ONE) : DT{0};
-                                    if (!RAGGED || k < left) op[lane_nchw + static_cast<uint32_t>(k * po)] = spike;
+                            for (int k = 0; k < 4; ++k) {
+                                float x = xq[tw][k];
+                                if constexpr (FRAME) x += in.bias[k];
+                                if (!FRAME && g.res_layout >= 0) {
+                                    if constexpr (SPLIT) x += __uint_as_float(in.res[tw][k]);
+                                    else x += to_float(XT{static_cast<uint16_t>(in.res[tw][k])});
                                 }
+                                const float h = FRAME ? v[k] + (x - v[k]) * 0.5f : (v[k] + x) * 0.5f;
+                                const bool fired = h >= lif.v_threshold;
+                                v[k] = fired ? lif.v_reset : h;
+                                const DT spike = fired ? static_cast<DT>(SPLIT ? 0x3f800000u : ONE) : DT{0};
+                                if (!RAGGED || k < left) op[lane_nchw + static_cast<uint32_t>(k * po)] = spike;
                             }
+                        };
+                        if constexpr (FRAME) {
+                            for (int t = 0; t < t_count; ++t) step(t, 0);
+                        } else {
+#pragma unroll
+                            for (int tw = 0; tw < TT; ++tw)
+                                if (tw < t_count) step(t0 + tw, tw);
                         }
                         if (v_dst16) {
                             if constexpr (!SPLIT) {
@@ -1316,7 +1333,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                                 for (int k = 0; k < 4; ++k)
                                     if (!RAGGED || k < left) vp[lane_nchw + static_cast<uint32_t>(k * po)] = from_float<XT>(v[k]);
                             }
-                        } else {
+                        } else if (!FRAME || v_dst != nullptr) {      // (a network's own layers keep no membrane)
                             float* vp = static_cast<float*>(v_dst) + static_cast<int64_t>(j8) * 8 * po;
 #pragma unroll
                             for (int k = 0; k < 4; ++k)
@@ -1842,6 +1859,10 @@ int launch_conv_spk_frame(const SpkLaunch& L, bool pooled) {
         return check_launch("snnf_conv_lif_blocked");
     };
     constexpr int D = SNNF_LAYOUT_NCHW;
+    if (L.dense_epilogue) {
+        if (L.g.narrow) return run(conv_spk_kernel<XT, 1, D, false, false, false, false, true, true>);
+        return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, 1, D, true, false, false, false, false, true>) : run(conv_spk_kernel<XT, 1, D, false, false, false, false, false, true>);
+    }
     if (L.g.narrow) {
         if (pooled) return run(conv_spk_kernel<XT, 1, D, false, true, false, true, true>);
         return L.fast_epilogue ? run(conv_spk_kernel<XT, 1, D, false, true, false, false, true>) : run(conv_spk_kernel<XT, 1, D, false, false, false, false, true>);

@@ -343,7 +343,7 @@ def _v_init_pointer(v_init, out_shape, v_dtype, device):
 
 
 def _one_frame(pointers) -> bool:
-    """Whether all of several timesteps read the same tensor (convolved once, on the dense kernels)."""
+    """Whether all of several timesteps read the same tensor (convolved once, without scratch memory)."""
     return len(pointers) > 1 and len(set(pointers)) == 1
 
 
