@@ -1,4 +1,4 @@
-"""Depthwise 3x3 of stride 2 on 16-bit activations in rows of whole 16-byte vectors (the kernel without LDS) against the oracle.
+"""Depthwise 3x3 on 16-bit activations in rows of whole 16-byte vectors on the kernel without LDS (stride 2, small launches of stride 1) against the oracle.
 
 Weights, biases and inputs are fixed-point numbers whose sums of nine are exact in float32: spikes and membranes are the oracle's bit for bit."""
 import pytest
@@ -62,3 +62,25 @@ def test_an_output_sees_its_nine_inputs_only(hip_ops, value):
     got = v.cpu()
     assert torch.equal(torch.where(torch.arange(64).view(1, 2, 4, 8) == 9, clean, got), clean)
     assert s[0, 0, 0, 1, 1].item() == (1.0 if value == float("inf") else 0.0)
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16])
+@pytest.mark.parametrize("N,C,H,W,T,residual", [(1, 2, 1, 8, 1, False), (2, 5, 7, 16, 4, True), (1, 16, 15, 40, 3, False), (1, 24, 48, 48, 17, True), (8, 64, 32, 64, 2, False),
+                                                (8, 65, 32, 64, 2, False)])
+def test_stride_1_without_lds(hip_ops, dtype, N, C, H, W, T, residual):
+    """Launches of up to 131072 strips (the last but one) and the first on the tile in LDS: the same dot products in the same order as on row-packed spikes."""
+    from triton_snn_fusion_amd.runtime import hip_blocked_backend as B
+    g = gen(7 * H + C)
+    xs = [spikes((N, C, H, W), 0.4, g) for _ in range(T)]
+    rs = [spikes((N, C, H, W), 0.3, g) for _ in range(T)] if residual else None
+    w, b = _layer(C, g)
+    ref = O.temporal_conv_lif(xs, w, b, torch.tensor(0.0), (1, 1), (1, 1), (1, 1), C, *LIF, residuals=rs)
+    dx, dr = [dev(x, dtype) for x in xs], None if rs is None else [dev(r, dtype) for r in rs]
+    args = (dev(w, dtype), dev(b, dtype), zero_v(F32), [1, 1], [1, 1], [1, 1], C, *LIF, False)
+    s, v = S.fused_temporal_depthwise_conv_lif_state(dx, *args) if rs is None else S.fused_temporal_conv_add_lif_state_depthwise(dx, dr, *args)
+    assert torch.equal(s.float().cpu(), ref[0]) and torch.equal(v.cpu(), ref[1])
+    noisy = [(x * 0.83).to(dtype) for x in dx]                  # (sums that round)
+    args = (dev(w * 0.77, dtype), dev(b, dtype), zero_v(F32), [1, 1], [1, 1], [1, 1], C, *LIF, False)
+    s1, v1 = S.fused_temporal_depthwise_conv_lif_state(noisy, *args)
+    bits, v2 = B.depthwise_conv_lif_rowbits(noisy, args[0], args[1], LIF)
+    assert torch.equal(B.unpack_rowbits(bits, dtype), s1) and torch.equal(v1, v2)

@@ -303,17 +303,30 @@ int launch(const StepPtrs& xs, const StepPtrs& res, int has_res, int T, DwGeom g
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// Stride 2, 16-bit activations in rows of whole 16-byte vectors, without LDS: a lane reads the three input rows of its strip of 4 outputs
+// Stride 2, and small launches of stride 1, 16-bit activations in rows of whole 16-byte vectors, without LDS: a lane reads the three input rows of its strip of 4 outputs
 // straight from memory, 16 bytes and the dword in front of them per row. Half of the rows belong to two strips and come from the vector cache
 // the second time, so a step costs a lane six loads, no barrier, no transposition and no tile to zero; lanes of a wave read
 // contiguous rows. (On the tile of `dwconv3x3_lif_kernel` a lane takes 17 floats of a row one by one, 16 floats from its neighbour's: the reads
 // of a wave fall into a few of the LDS banks.) Padding comes from the range check of buffer loads, which answers zero beyond the frame.
 // What bounds it: HBM. 64 channels at 64x64 x 32, T = 4 (84 MB and 8 MB of membrane) 42.4 -> 19.0 us, 128 at 32x32 x 32 25.3 -> 10.0,
 // one image
-// 11.1 -> 5.2 (48x48) and 9.8 -> 5.0 (24x24). The same without LDS at stride 1, where every row is read three times and a strip takes nine loads, lost: 128 channels
-// at 56x56 x 32 and the pointwise layer behind them 126 -> 145 us.
+// 11.1 -> 5.2 (48x48) and 9.8 -> 5.0 (24x24).
+// Stride 1 (8 outputs a strip, the dword behind them as well, the dot products of the kernel below in its order): nine loads a strip and every row three times lose
+// where the vector caches are busy (128 channels at 56x56 x 32 and the pointwise layer behind them 126 -> 145 us), but a launch of up to two workgroups per
+// compute unit is its set-up, which is shorter here: 32 channels at 48x48,
+// one image 7.2 -> 6.0 us, 128 at 24x24 8.0 -> 6.0 (at 32x32 x 16, two rounds of it, 23.6 with the pointwise layer, 24.1 without LDS).
 // ---------------------------------------------------------------------------------------------------------------
 typedef uint32_t dw_u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 dw_bf16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 dw_f16x2 __attribute__((ext_vector_type(2)));
+
+template <typename XT>
+__device__ __forceinline__ float dot2_acc(uint32_t a, uint32_t b, float c) {
+    if constexpr (dtype_of<XT>::value == SNNF_BF16)
+        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(dw_bf16x2, a), __builtin_bit_cast(dw_bf16x2, b), c, false);
+    else
+        return __builtin_amdgcn_fdot2(__builtin_bit_cast(dw_f16x2, a), __builtin_bit_cast(dw_f16x2, b), c, false);
+}
 
 // The lower and the upper element of a dword of two 16-bit values.
 template <typename XT> __device__ __forceinline__ float low_element(uint32_t d) { return to_float(XT{static_cast<uint16_t>(d)}); }
@@ -322,22 +335,22 @@ template <> __device__ __forceinline__ float high_element<bf16_t>(uint32_t d) { 
 
 constexpr int64_t kDirectMaxFrame = 0x7fffff00ll;     // bytes of one timestep's input: offsets from 2^31 on lie outside
 constexpr uint32_t kDirectOutside = 0x80000000u;
-constexpr int kDirectPx = 4;                          // outputs of a strip
+constexpr int64_t kDirectStrips = 1 << 17;            // stride 1: strips up to which a launch takes this kernel
 
 struct DwDirect {
-    int strips;              // output strips in all: N * C * Ho * (Wo / 4)
+    int strips;              // output strips of 8 input columns in all
     int C, H, W, Ho, SW;     // SW: strips per output row
     uint32_t frame_bytes;
     FastDiv d_SW, d_Ho, d_C;
 };
 
 // The two pointer tables MUST be the first two kernel parameters.
-template <typename XT, typename VT, bool STD>
-__global__ __launch_bounds__(kThreads) void dwconv3x3_s2_lif_direct_kernel(StepPtrs xs, StepPtrs residuals, int has_residual, int T, DwDirect g,
-                                                                           const XT* __restrict__ weight, const XT* __restrict__ bias,
-                                                                           const VT* v_init, XT* __restrict__ spikes, int64_t spike_step_stride,
-                                                                           VT* v_out, LifParams lif) {
-    constexpr int PX = kDirectPx;
+template <typename XT, typename VT, int STRIDE, bool STD>
+__global__ __launch_bounds__(kThreads) void dwconv3x3_lif_direct_kernel(StepPtrs xs, StepPtrs residuals, int has_residual, int T, DwDirect g,
+                                                                        const XT* __restrict__ weight, const XT* __restrict__ bias,
+                                                                        const VT* v_init, XT* __restrict__ spikes, int64_t spike_step_stride,
+                                                                        VT* v_out, LifParams lif) {
+    constexpr int PX = 8 / STRIDE;                        // outputs of a strip
     static_assert(sizeof(XT) == 2, "strips of one 16-byte vector per input row");
     const int i = static_cast<int>(blockIdx.x) * kThreads + static_cast<int>(threadIdx.x);
     if (i >= g.strips) return;
@@ -348,17 +361,18 @@ __global__ __launch_bounds__(kThreads) void dwconv3x3_s2_lif_direct_kernel(StepP
     const int c = plane - fast_div(plane, g.d_C) * g.C;
     const int64_t out = static_cast<int64_t>(i) * PX;       // elements
 
-    uint32_t mid[3], left[3];
+    uint32_t mid[3], left[3], right[3];
 #pragma unroll
     for (int kh = 0; kh < 3; ++kh) {
-        const int ih = oh * 2 - 1 + kh;
+        const int ih = oh * STRIDE - 1 + kh;
         const bool in = ih >= 0 && ih < g.H;
         const uint32_t off = static_cast<uint32_t>((plane * g.H + ih) * g.W + strip * 8) * 2u;
         mid[kh] = in ? off : kDirectOutside;
         left[kh] = in && strip > 0 ? off - 4u : kDirectOutside;
+        right[kh] = in && strip + 1 < g.SW ? off + 16u : kDirectOutside;
     }
     dw_u32x4 x[3];
-    uint32_t xl[3];
+    uint32_t xl[3], xr[3];
     Pack<XT, PX> res = {};
     auto issue_loads = [&](int t) __attribute__((always_inline)) {
         const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(dw_table_entry(0, t)), 0, g.frame_bytes, 0x00027000);
@@ -366,14 +380,29 @@ __global__ __launch_bounds__(kThreads) void dwconv3x3_s2_lif_direct_kernel(StepP
         for (int kh = 0; kh < 3; ++kh) {
             x[kh] = __builtin_bit_cast(dw_u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, mid[kh], 0, 0));
             xl[kh] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, left[kh], 0, 0);
+            if constexpr (STRIDE == 1) xr[kh] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, right[kh], 0, 0);
         }
         if (has_residual) res = *reinterpret_cast<const Pack<XT, PX>*>(static_cast<const XT*>(dw_table_entry(sizeof(StepPtrs), t)) + out);
     };
     issue_loads(0);
 
     float w[9];
+    uint32_t wp[3][4];                                     // stride 1: the operand pairs of dwconv3x3_lif_dot_kernel
+    const uint16_t* __restrict__ wbits = reinterpret_cast<const uint16_t*>(weight) + c * 9;
 #pragma unroll
-    for (int j = 0; j < 9; ++j) w[j] = to_float(weight[c * 9 + j]);
+    for (int kh = 0; kh < 3; ++kh) {
+        const uint32_t w0 = wbits[kh * 3], w1 = wbits[kh * 3 + 1], w2 = wbits[kh * 3 + 2];
+        if constexpr (STRIDE == 1) {
+            wp[kh][0] = w1 | (w2 << 16);
+            wp[kh][1] = w0 << 16;
+            wp[kh][2] = w0 | (w1 << 16);
+            wp[kh][3] = w2;
+        } else {
+            w[kh * 3] = to_float(XT{static_cast<uint16_t>(w0)});
+            w[kh * 3 + 1] = to_float(XT{static_cast<uint16_t>(w1)});
+            w[kh * 3 + 2] = to_float(XT{static_cast<uint16_t>(w2)});
+        }
+    }
     const float b = to_float(bias[c]);
     float v[PX];
     if (v_init != nullptr) {
@@ -389,17 +418,30 @@ __global__ __launch_bounds__(kThreads) void dwconv3x3_s2_lif_direct_kernel(StepP
         for (int j = 0; j < PX; ++j) acc[j] = b;
 #pragma unroll
         for (int kh = 0; kh < 3; ++kh) {
-            float in[9];                  // input columns -1 .. 7 of the strip
-            in[0] = high_element<XT>(xl[kh]);
+            if constexpr (STRIDE == 1) {
+                const dw_u32x4 d = x[kh];
+                const uint32_t A = wp[kh][0], B = wp[kh][1], C = wp[kh][2], D = wp[kh][3];
+                acc[0] = dot2_acc<XT>(d[0], A, dot2_acc<XT>(xl[kh], B, acc[0]));
+                acc[1] = dot2_acc<XT>(d[0], C, dot2_acc<XT>(d[1], D, acc[1]));
+                acc[2] = dot2_acc<XT>(d[1], A, dot2_acc<XT>(d[0], B, acc[2]));
+                acc[3] = dot2_acc<XT>(d[1], C, dot2_acc<XT>(d[2], D, acc[3]));
+                acc[4] = dot2_acc<XT>(d[2], A, dot2_acc<XT>(d[1], B, acc[4]));
+                acc[5] = dot2_acc<XT>(d[2], C, dot2_acc<XT>(d[3], D, acc[5]));
+                acc[6] = dot2_acc<XT>(d[3], A, dot2_acc<XT>(d[2], B, acc[6]));
+                acc[7] = dot2_acc<XT>(d[3], C, dot2_acc<XT>(xr[kh], D, acc[7]));
+            } else {
+                float in[9];                  // input columns -1 .. 7 of the strip
+                in[0] = high_element<XT>(xl[kh]);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                in[1 + 2 * k] = low_element<XT>(x[kh][k]);
-                in[2 + 2 * k] = high_element<XT>(x[kh][k]);
+                for (int k = 0; k < 4; ++k) {
+                    in[1 + 2 * k] = low_element<XT>(x[kh][k]);
+                    in[2 + 2 * k] = high_element<XT>(x[kh][k]);
+                }
+#pragma unroll
+                for (int j = 0; j < PX; ++j)
+#pragma unroll
+                    for (int kw = 0; kw < 3; ++kw) acc[j] = fmaf(in[j * STRIDE + kw], w[kh * 3 + kw], acc[j]);
             }
-#pragma unroll
-            for (int j = 0; j < PX; ++j)
-#pragma unroll
-                for (int kw = 0; kw < 3; ++kw) acc[j] = fmaf(in[j * 2 + kw], w[kh * 3 + kw], acc[j]);
         }
         if (has_residual) {
 #pragma unroll
@@ -427,7 +469,7 @@ __global__ __launch_bounds__(kThreads) void dwconv3x3_s2_lif_direct_kernel(StepP
     *reinterpret_cast<Pack<VT, PX>*>(v_out + out) = vo;
 }
 
-template <typename XT, typename VT>
+template <typename XT, typename VT, int STRIDE>
 int launch_direct(const StepPtrs& xs, const StepPtrs& res, int has_res, int T, const DwGeom& g, const void* weight, const void* bias, const void* v_init,
                   void* spikes, int64_t spike_step_stride, void* v_out, const LifParams& lif, hipStream_t stream) {
     DwDirect d = {};
@@ -442,8 +484,8 @@ int launch_direct(const StepPtrs& xs, const StepPtrs& res, int has_res, int T, c
     d.d_Ho = make_fast_div(d.Ho);
     d.d_C = make_fast_div(d.C);
     const dim3 grid((static_cast<unsigned>(d.strips) + kThreads - 1) / kThreads);
-    auto kernel = lif.charge_mode == CHARGE_SCALE && !lif.soft_reset ? dwconv3x3_s2_lif_direct_kernel<XT, VT, true>
-                                                                     : dwconv3x3_s2_lif_direct_kernel<XT, VT, false>;
+    auto kernel = lif.charge_mode == CHARGE_SCALE && !lif.soft_reset ? dwconv3x3_lif_direct_kernel<XT, VT, STRIDE, true>
+                                                                     : dwconv3x3_lif_direct_kernel<XT, VT, STRIDE, false>;
     kernel<<<grid, kThreads, 0, stream>>>(xs, res, has_res, T, d, static_cast<const XT*>(weight), static_cast<const XT*>(bias),
                                           static_cast<const VT*>(v_init), static_cast<XT*>(spikes), spike_step_stride, static_cast<VT*>(v_out), lif);
     return check_launch("snnf_dwconv3x3_lif");
@@ -459,16 +501,6 @@ int launch_direct(const StepPtrs& xs, const StepPtrs& res, int has_res, int T, c
 // the strip at elements e0 .. e0 + 7 (e0 a multiple of 8) a row costs one 16-byte read and the two dwords around it.
 // ---------------------------------------------------------------------------------------------------------------
 constexpr int kDotColOffset = 8;
-typedef __bf16 dw_bf16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 dw_f16x2 __attribute__((ext_vector_type(2)));
-
-template <typename XT>
-__device__ __forceinline__ float dot2_acc(uint32_t a, uint32_t b, float c) {
-    if constexpr (dtype_of<XT>::value == SNNF_BF16)
-        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(dw_bf16x2, a), __builtin_bit_cast(dw_bf16x2, b), c, false);
-    else
-        return __builtin_amdgcn_fdot2(__builtin_bit_cast(dw_f16x2, a), __builtin_bit_cast(dw_f16x2, b), c, false);
-}
 
 // BITS: the spikes of a strip and timestep leave as one byte (bit j = pixel 8 x + j of the row) instead of eight 16-bit
 // values: [T][N][C][Ho][Wo / 8] bytes, `spike_step_stride` then counts bytes; the final membrane is optional.
@@ -743,8 +775,10 @@ int dispatch_px(int px, bool direct, const StepPtrs& xs, const StepPtrs& res, in
                 const LifParams& lif, hipStream_t stream) {
     if constexpr (sizeof(XT) == 2) {
         if (direct) {
-            if constexpr (STRIDE == 1) return launch_dot<XT, VT>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
-            else return launch_direct<XT, VT>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
+            if constexpr (STRIDE == 1) {
+                if (static_cast<int64_t>(g.planes) * g.H * (g.W / 8) > kDirectStrips) return launch_dot<XT, VT>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
+            }
+            return launch_direct<XT, VT, STRIDE>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
         }
     } else if (px == 8) {
         return launch<XT, VT, STRIDE, 8>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
@@ -942,7 +976,7 @@ extern "C" int snnf_dwconv3x3_lif(const void* const* xs, const void* const* resi
             xp.p[t] = xs[t0 + t];
             if (residuals != nullptr) rp.p[t] = residuals[t0 + t];
         }
-        // 16-bit activations in strips of 8 input columns (`direct`): the dot-product kernel at stride 1, the kernel without LDS at stride 2, whose strips
+        // 16-bit activations in strips of 8 input columns (`direct`): the dot-product kernel at stride 1 (small launches: without LDS), the kernel without LDS at stride 2, whose strips
         // are 4 outputs wide (a plane of whole vectors and 16-byte aligned steps; frames within its 32-bit offsets). What is left of
         // 16-bit calls takes at most 4 outputs a strip.
         bool direct = x_dtype != SNNF_F32 && W % 8 == 0 && px >= 8 / stride &&
