@@ -139,8 +139,10 @@ RouteSpace route_space(int T, int N, int Cin, int H, int W, bool split, int64_t 
 //   nearly proportional to the outputs. So `tile_use` decides (see dense_family), weighed by the products per output, in which this kernel is
 //   the better one. The quotient of the two times falls with it from 2 to 0.75 and passes 1 at the lines below. It moves 64 -> 64 at 24^2 x 4 30 / 12, x 38, T = 6 70 / 45, at
 //   40^2 x 20 (tiles of four columns) 43 / 33, T = 8 121 / 68, at 56^2 x 21, T = 6 132 / 110, 128 -> 256 stride 2 at 28^2 x 5, T = 8 49 / 40, 1x1 stride 2 x 2
-//   31 / 20; 64 -> 64 at 56^2 x 16 34 / 42, 128 -> 128 at 28^2 x 32 48 / 52 (x 16 38 / 36), 64 -> 128 stride 2 at 56^2 x 16 28 / 37, 1x1 18 / 26, 128 -> 256 stride 2
-//   at 28^2 x 16 28 / 34 stay. Inputs that the caches don't hold between the copy and the kernel move the lines (64 -> 64 at 56^2 x 88, T = 5
+//   31 / 20; 64 -> 64 at 56^2 x 16 34 / 42, 128 -> 128 at 28^2 x 32 52 / 55, 64 -> 128 stride 2 at 56^2 x 16 28 / 37, 1x1 18 / 26, 128 -> 256 stride 2
+//   at 28^2 x 16 28 / 34 stay. Where a step's copy takes up to 5 MB, so that the L2 caches hold all of it for the kernel, the line lies higher: 128 -> 128 at 28^2 x 4 20.8 / 17.7,
+//   x 16 with a residual 40.8 / 36.5, T = 8 80 / 65, 64 -> 64 at 32^2 x 8 17.0 / 15.2, 64 -> 192 at 28^2 x 48 82 / 70; over 140 drawn layers beyond the other lines the quotient is
+//   1.21 there, 10 lose up to 11 %, most of them with 24 inputs; beyond 4 M elements a step 0.97. Inputs that the caches don't hold between the copy and the kernel move the lines (64 -> 64 at 56^2 x 88, T = 5
 //   with a residual 366 / 437, 128 -> 256 stride 2 at 28^2 x 164, T = 7 395 / 554). Deep layers of few outputs always move (256 -> 256 at 14^2 x 4 29 / 18, 512 -> 512 at 4^2 x 16 37 / 21). Over 22300 layers of
 //   whole tiles, planes of four pixels, few pixels and deep layers among them, the rule is 1 % slower than the better kernel in the mean, the dense kernels
 //   alone 54 % (256 -> 512 at 2^2 x 40 24 / 14, 64 -> 64 at 16^2 x 2 30 / 11, 256 -> 256 at 14^2 x 16 35 / 31, with a residual 37 / 32).
@@ -191,7 +193,7 @@ bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int C
             if (!one && !strided && Cin <= 8) return false;   // (a single channel group: as above)
             if (one) return tile_use * std::sqrt(576.0 / K) <= 0.45;
             if (strided) return tile_use * std::sqrt(std::sqrt(576.0 / K)) <= (T <= 4 ? 0.5 : (inputs < (1 << 24) ? 0.65 : 0.45));
-            return tile_use * std::sqrt(576.0 / K) <= (inputs >= (1 << 26) ? 0.7 : (T <= 4 ? 0.85 : 0.95));
+            return tile_use * std::sqrt(576.0 / K) <= (inputs / T <= (5 << 19) ? 1.1 : (inputs >= (1 << 26) ? 0.7 : (T <= 4 ? 0.85 : 0.95)));
     }
     return false;
 }
