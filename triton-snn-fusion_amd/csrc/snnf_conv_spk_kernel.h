@@ -1088,10 +1088,11 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             // extents, so a window lies inside one wave half) hold one byte-wide count per channel and step, add them in a
             // reduce-scatter of two exchanges (first with the horizontal neighbour, two steps each way; then with the vertical
             // one, one step each way), and the lane at window position (row r, column c) ends up with step 2 c + r, whose
-            // four quarters it stores as 16-bit values of the pooled, channel-blocked tensor.
+            // four quarters it stores as 16-bit values of the pooled, channel-blocked tensor. (The caller's steps may lie any distance apart, in
+            // either direction: the step's base has 64 bits, the place inside its frame 32.)
             bool odd_col = false, odd_row = false;
             int side = 0, along = 0;
-            uint32_t pool_off = 0;
+            unsigned char* pool_out = nullptr;
             if constexpr (POOL) {
                 const int prow_e = static_cast<int>((pos_e >> 8) & 255u), pcol_e = static_cast<int>(pos_e >> 16);
                 odd_col = (pcol_e & 1) != 0;
@@ -1099,8 +1100,8 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                 side = (lane ^ 1) * 4;
                 along = (lane + (odd_row ? -g.PC : g.PC)) * 4;
                 const int hp = g.Ho >> 1, wp = g.Wo >> 1;
-                const uint32_t step = (odd_col ? 2u : 0u) + (odd_row ? 1u : 0u);
-                pool_off = static_cast<uint32_t>(((n * g.C8out * hp + (oh >> 1)) * wp + (ow >> 1)) * 8 + 4 * half_e) * 2u + step * static_cast<uint32_t>(g.out_step_stride);
+                const int step = (odd_col ? 2 : 0) + (odd_row ? 1 : 0);
+                pool_out = out + static_cast<int64_t>(step) * g.out_step_stride + static_cast<uint32_t>(((n_e * g.C8out * hp + (oh >> 1)) * wp + (ow >> 1)) * 8 + 4 * half_e) * 2u;
             }
             auto fast_store4_pooled = [&](int j8, uint32_t quiet) __attribute__((always_inline)) {
                 const uint32_t fired = ~quiet;
@@ -1118,7 +1119,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     Pack<XT, 4> q4;
 #pragma unroll
                     for (int k = 0; k < 4; ++k) q4.v[k] = from_float<XT>(static_cast<float>((keep >> (8 * k)) & 255u) * 0.25f);
-                    *reinterpret_cast<Pack<XT, 4>*>(out + static_cast<int64_t>(j8) * ((g.Ho >> 1) * (g.Wo >> 1)) * 16 + pool_off) = q4;
+                    *reinterpret_cast<Pack<XT, 4>*>(pool_out + static_cast<int64_t>(j8) * ((g.Ho >> 1) * (g.Wo >> 1)) * 16) = q4;
                 }
             };
             // A quad's membrane from the window before.
