@@ -105,3 +105,36 @@ def test_dense_tensors_of_few_pixels(hip_ops, dtype, vdtype):
                                                dev(v0, vdtype), [1, 1], [1, 1], [1, 1], 1, *LIF, False)
     assert "few" in CB.last_conv_plan(), CB.last_conv_plan()
     assert torch.equal(s.float().cpu(), ref[0]) and torch.equal(v.cpu(), ref[1].to(vdtype))
+
+
+@pytest.mark.parametrize("lif", [(1.0, -1.0, 2.0), LIF, (1.0, 0.25, 2.0)])
+@pytest.mark.parametrize("T", [4, 5])
+def test_rounding_of_the_charge(B, lif, T):
+    """Membranes of 24 bits, on which (v + x) / 2 and v + (x - v) / 2 round differently: the charge of the tiles of conv_spk_kernel for either reset, with a soft
+    reset the oracle's own."""
+    g = gen(17)
+    Cin, Cout, H = 128, 64, 6
+    x, w, b, _ = _operands(T, 1, Cin, Cout, H, H, 3, 1, False, "bits", g)
+    v0 = torch.randn((1, Cout, H, H), generator=g) * 0.7
+    ref = O.temporal_conv_lif([x[t] for t in range(T)], w, b, v0, (1, 1), (1, 1), (1, 1), 1, *lif)
+    first = torch.nn.functional.conv2d(x[0], w, b, padding=1)
+    differ = float(((v0 + first) * 0.5 != v0 + (first - v0) * 0.5).float().mean())
+    assert differ > 0.02, differ                                           # the two forms are told apart
+    xb = B.from_dense(dev(x, BF16), B.BITS)
+
+    def call():
+        out, v = B.conv_lif_blocked(xb, dev(w, BF16), dev(b, BF16), [1, 1], [1, 1], lif, v_init=dev(v0, torch.float32), want_v=True)
+        return B.to_dense(out).float().cpu(), v.cpu(), B.last_conv_plan()
+
+    sp, v, plan = call()
+    assert "few" in plan, plan
+    key = (T, 1, Cin, H, H, Cout, 3, 3, 1, 1, 1, 1, 0)
+    B.register_tuned_plan(key, int(plan["tile"].split("x")[2]), 0, 0)
+    try:
+        sp2, v2, plan2 = call()
+    finally:
+        B.register_tuned_plan(key, 0, 0, 0)
+    assert "few" not in plan2, plan2
+    assert torch.equal(sp, sp2) and torch.equal(v, v2)
+    if lif[1] < 0:
+        assert torch.equal(sp, ref[0]) and torch.equal(v, ref[1])

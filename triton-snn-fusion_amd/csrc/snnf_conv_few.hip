@@ -116,7 +116,7 @@ __global__ __launch_bounds__(kFewThreads, 2) void conv_few_kernel(const StepPtrs
     const bool neuron = cq < 4 && np_live && ch < g.Cout && nn < g.N && noh < g.Ho && now < g.Wo;
     const uint32_t at_nchw = neuron ? static_cast<uint32_t>(((nn * g.Cout + ch) * g.Ho + noh) * g.Wo + now) : 0u;
     const uint32_t at_bits = neuron ? static_cast<uint32_t>(((nn * g.C8out + (ch >> 3)) * g.Ho + noh) * g.Wo + now) : 0u;
-    const bool half_tau = lif.charge_mode == CHARGE_SCALE && lif.inv_tau == 0.5f;
+    const bool half_tau = lif.charge_mode == CHARGE_SCALE && lif.inv_tau == 0.5f && !lif.soft_reset;
     float v = 0.0f, b = 0.0f;
     if (neuron) {
         b = bias[ch];
@@ -293,10 +293,10 @@ __global__ __launch_bounds__(kFewThreads, 2) void conv_few_kernel(const StepPtrs
                     if (g.res_layout == SNNF_LAYOUT_BITS) x[i] += static_cast<float>((res[i] >> (ch & 7)) & 1u);
                     else if (g.res_layout >= 0) x[i] += to_float(XT{static_cast<uint16_t>(res[i])});
                     bool fired;
-                    if (half_tau) {                                   // (as in conv_spk_kernel: one rounding)
+                    if (half_tau) {                                   // (as in conv_spk_kernel: one rounding, with a hard reset)
                         const float h = (v + x[i]) * 0.5f;
                         fired = h >= lif.v_threshold;
-                        v = fired ? (lif.soft_reset ? h - lif.v_threshold : lif.v_reset) : h;
+                        v = fired ? lif.v_reset : h;
                     } else {
                         fired = lif_step(x[i], v, lif);
                     }
