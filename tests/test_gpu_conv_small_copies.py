@@ -32,3 +32,17 @@ def test_moved_layer(hip_ops, residual):
     s, v = S.fused_temporal_conv_lif_state(dx, *args) if r is None else S.fused_temporal_conv_add_lif_state(dx, [dev(t, BF16) for t in r], *args)
     assert CB.last_conv_plan()["ran"] == "blocked", CB.last_conv_plan()
     assert torch.equal(s.float().cpu(), ref[0]) and torch.allclose(v.cpu(), ref[1], rtol=1e-6, atol=1e-6)
+
+
+@pytest.mark.parametrize("T,N,Cin,Cout,H,W,residual,moves", [
+    (4, 16, 128, 128, 28, 28, 1, True),        # 1792 waves of 2048
+    (4, 11, 64, 64, 56, 56, 1, False),         # 1078
+    (2, 58, 32, 512, 32, 32, 1, False),        # more than two rounds
+    (4, 20, 64, 64, 48, 28, 0, False),         # patches of four columns
+    (4, 16, 128, 64, 28, 28, 1, False),        # few output channels for the copy
+    (1, 8, 64, 128, 80, 28, 1, True),          # one timestep
+    (4, 8, 64, 64, 32, 32, 0, True),           # narrow tiles
+])
+def test_layers_that_fill_the_waves(snnf_lib, T, N, Cin, Cout, H, W, residual, moves):
+    """Beyond the usual line only layers move whose plan on the blocked kernel is a good one."""
+    assert (snnf_lib.snnf_conv_lif_scratch_bytes(T, N, Cin, H, W, 1, Cout, 3, 3, 1, 1, 1, 1, 0, residual) > 0) == moves

@@ -140,9 +140,8 @@ RouteSpace route_space(int T, int N, int Cin, int H, int W, bool split, int64_t 
 //   the better one. The quotient of the two times falls with it from 2 to 0.75 and passes 1 at the lines below. It moves 64 -> 64 at 24^2 x 4 30 / 12, x 38, T = 6 70 / 45, at
 //   40^2 x 20 (tiles of four columns) 43 / 33, T = 8 121 / 68, at 56^2 x 21, T = 6 132 / 110, 128 -> 256 stride 2 at 28^2 x 5, T = 8 49 / 40, 1x1 stride 2 x 2
 //   31 / 20; 64 -> 64 at 56^2 x 16 34 / 42, 128 -> 128 at 28^2 x 32 52 / 55, 64 -> 128 stride 2 at 56^2 x 16 28 / 37, 1x1 18 / 26, 128 -> 256 stride 2
-//   at 28^2 x 16 28 / 34 stay. Where a step's copy takes up to 5 MB, so that the L2 caches hold all of it for the kernel, the line lies higher: 128 -> 128 at 28^2 x 4 20.8 / 17.7,
-//   x 16 with a residual 40.8 / 36.5, T = 8 80 / 65, 64 -> 64 at 32^2 x 8 17.0 / 15.2, 64 -> 192 at 28^2 x 48 82 / 70; over 140 drawn layers beyond the other lines the quotient is
-//   1.21 there, 10 lose up to 11 %, most of them with 24 inputs; beyond 4 M elements a step 0.97. Inputs that the caches don't hold between the copy and the kernel move the lines (64 -> 64 at 56^2 x 88, T = 5
+//   at 28^2 x 16 28 / 34 stay. Where a step's copy takes up to 5 MB, so that the L2 caches hold all of it for the kernel, the line lies higher for layers that fill this kernel's
+//   waves (see `fills_waves`); beyond 4 M elements a step the quotient is 0.97. Inputs that the caches don't hold between the copy and the kernel move the lines (64 -> 64 at 56^2 x 88, T = 5
 //   with a residual 366 / 437, 128 -> 256 stride 2 at 28^2 x 164, T = 7 395 / 554). Deep layers of few outputs always move (256 -> 256 at 14^2 x 4 29 / 18, 512 -> 512 at 4^2 x 16 37 / 21). Over 22300 layers of
 //   whole tiles, planes of four pixels, few pixels and deep layers among them, the rule is 1 % slower than the better kernel in the mean, the dense kernels
 //   alone 54 % (256 -> 512 at 2^2 x 40 24 / 14, 64 -> 64 at 16^2 x 2 30 / 11, 256 -> 256 at 14^2 x 16 35 / 31, with a residual 37 / 32).
@@ -158,7 +157,8 @@ RouteSpace route_space(int T, int N, int Cin, int H, int W, bool split, int64_t 
 //   at 28^2 x 12, T = 2 0.89 / 0.69; 192 -> 128 x 3 1.37 / 1.12).
 // Without a neuron the lines are those of sums that leave as 16-bit values (512 -> 512 at 7^2 x 16 56 / 35).
 bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w,
-                         int v_dtype, bool residual, bool neuron, DenseFamily& family) {
+                         int v_dtype, bool residual, bool neuron, DenseFamily& family, double& weigh) {
+    weigh = 0.0;
     if (x_dtype != SNNF_BF16 && x_dtype != SNNF_F16 && x_dtype != SNNF_F32) return false;
     if ((v_dtype != SNNF_F32 && v_dtype != x_dtype) || T < 1 || T > SNNF_MAX_T_PER_LAUNCH || N < 1 || Cin < 1 || H < 1 || W < 1 || Cout < 1 || KH < 1 || KW < 1 ||
         stride_h < 1 || stride_w < 1 || pad_h < 0 || pad_w < 0 || H + 2 * pad_h < KH || W + 2 * pad_w < KW || 2 * pad_h > KH || 2 * pad_w > KW) return false;
@@ -193,7 +193,11 @@ bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int C
             if (!one && !strided && Cin <= 8) return false;   // (a single channel group: as above)
             if (one) return tile_use * std::sqrt(576.0 / K) <= 0.45;
             if (strided) return tile_use * std::sqrt(std::sqrt(576.0 / K)) <= (T <= 4 ? 0.5 : (inputs < (1 << 24) ? 0.65 : 0.45));
-            return tile_use * std::sqrt(576.0 / K) <= (inputs / T <= (5 << 19) ? 1.1 : (inputs >= (1 << 26) ? 0.7 : (T <= 4 ? 0.85 : 0.95)));
+            const double weighed = tile_use * std::sqrt(576.0 / K);
+            if (weighed <= (inputs >= (1 << 26) ? 0.7 : (T <= 4 ? 0.85 : 0.95))) return true;
+            if (inputs / T > (5 << 19) || weighed > 1.1) return false;
+            weigh = weighed;
+            return true;
     }
     return false;
 }
@@ -415,6 +419,22 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
     return SNNF_OK;
 }
 
+// Whether a layer of whole tiles beyond the usual line, whose copy is small, moves (see takes_blocked_route): `weigh` is its `tile_use` weighed by the products per output, up
+// to 1.1. Of 842 drawn layers there 134 lose, up to a quarter, and what they lose by stands in this kernel's plan: waves without a tile (64 -> 64 at 56^2 x 11 with a residual, 1078 tiles
+// on 2048 waves, 37.5 / 43.7), more than two rounds of waves (32 -> 512 at 32^2 x 58, T = 2, with a residual 168 / 190), patches of four columns (64 -> 64 at 48 x 28 x 20 28 / 36), and few
+// output channels for a copy (128 -> 64 at 28^2 x 16 with a residual 26 / 28; 24 inputs lose no more often than others). Narrow tiles lose little by idle waves, one
+// timestep nothing (116 layers, 1.23). The line takes 471 of the 842 at 1.16 in the mean, 13 of which lose, up to 8 % (40 -> 64 at 16^2 x 25, T = 3 13.8 / 15.0); the others are at 1.03, a third of them below 1.
+// 128 -> 128 at 28^2 x 4 20.8 / 17.7, x 16 with a residual 40.8 / 36.5, T = 8 80 / 65, 64 -> 64 at 32^2 x 8 17.0 / 15.2, 64 -> 192 at 28^2 x 48 82 / 70.
+bool fills_waves(const BlockedPlan& p, double weigh, int T, int Cout) {
+    if (T == 1 || p.few) return true;
+    const SpkGeom& g = p.g;
+    const double line = weigh * (1.0 + 40.0 / Cout);
+    if (g.PC < 8) return false;
+    if (g.narrow) return line <= 1.65;
+    const double waves = static_cast<double>(g.iters) * compute_units() * kSpkWaves;
+    return g.iters <= 2 && line <= 1.55 * std::min(1.0, static_cast<double>(static_cast<int64_t>(g.n_items) << p.wk_log2) / waves);
+}
+
 const char* family_name(DenseFamily f) {
     return f == DenseFamily::kTInM ? "t_in_m" : (f == DenseFamily::kTimeOuter ? "time_outer" : (f == DenseFamily::kPointwise ? "pointwise" : "matrix"));
 }
@@ -465,7 +485,8 @@ Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, 
         if (it != routes().end()) return it->second;
     }
     Route route = {false, DenseFamily::kTInM, nullptr};
-    route.taken = takes_blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residual, neuron, route.family) &&
+    double weigh;
+    route.taken = takes_blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residual, neuron, route.family, weigh) &&
                   (neuron || (!split && (route.family == DenseFamily::kMatrixMasked || route.family == DenseFamily::kMatrixWhole)));
     if (frame)                                         // (see takes_frame)
         route.taken = route.family != DenseFamily::kPointwise &&
@@ -475,7 +496,8 @@ Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, 
         BlockedPlan& plan = kept->plan;
         route.taken = plan_blocked("snnf_conv_lif_scratch_bytes", BlockedCall{T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w,
                                    frame ? SNNF_LAYOUT_NCHW : SNNF_LAYOUT_C8, residual ? SNNF_LAYOUT_NCHW : -1, SNNF_LAYOUT_NCHW, 0, frame, neuron, false, neuron, false,
-                                   nullptr, split}, plan) == SNNF_OK;
+                                   nullptr, split}, plan) == SNNF_OK &&
+                      (frame || weigh == 0.0 || fills_waves(plan, weigh, T, Cout));
         if (route.taken) {
             for (int dense_epi = 0; dense_epi < 2; ++dense_epi) plan_text(kept->text[dense_epi], plan, family_name(route.family), dense_epi ? 40 : 0, frame ? T : plan.tt, frame ? kFrameRoute : kCopyRoute);
             route.kept = kept;
