@@ -58,3 +58,25 @@ def test_frames_that_stay_on_the_dense_kernels(hip_ops, lif, residual, dtype, Ci
     else:
         S.fused_temporal_conv_lif_state([dx] * 4, *args)
     assert CB.last_conv_plan().get("route") != "frame", CB.last_conv_plan()
+
+
+@pytest.mark.parametrize("T,N,Cin,Cout,H,W,k,s,frame", [
+    (4, 19, 3, 64, 224, 224, 7, 2, True),      # a stem of 61 million outputs
+    (4, 20, 3, 64, 224, 224, 7, 2, False),     # of 64
+    (8, 45, 4, 96, 96, 25, 1, 1, True),        # 1x1 on the time-outer kernel, 83 million
+    (8, 50, 4, 96, 96, 25, 1, 1, False),       # 92
+    (4, 30, 3, 64, 112, 112, 3, 1, True),      # whole tiles of stride 1, 96 million
+])
+def test_line_of_large_outputs(hip_ops, T, N, Cin, Cout, H, W, k, s, frame):
+    """Large first layers stay on the dense kernel where that is the faster one; either way an image has the spikes that it has alone."""
+    from triton_snn_fusion_amd.runtime import hip_convlif_backend as CB
+    S = torch.ops.snn_custom
+    x = torch.randint(-32, 33, (N, Cin, H, W), device=DEV, dtype=torch.int8).to(BF16) / 16
+    w = (torch.randint(-16, 17, (Cout, Cin, k, k), device=DEV, dtype=torch.int8).to(BF16) / 64)
+    b = torch.zeros(Cout, device=DEV, dtype=BF16)
+    args = (w, b, torch.zeros((), device=DEV), [s, s], [k // 2, k // 2], [1, 1], 1, *LIF, False)
+    sp, _ = S.fused_temporal_conv_lif_state([x] * T, *args)
+    assert (CB.last_conv_plan().get("route") == "frame") == frame, CB.last_conv_plan()
+    alone, _ = S.fused_temporal_conv_lif_state([x[-1:]] * T, *args)          # (one image: always the blocked kernel)
+    assert CB.last_conv_plan().get("route") == "frame"
+    assert torch.equal(sp[:, -1:], alone) and 0.0 < float(alone.float().mean()) < 1.0

@@ -471,7 +471,17 @@ std::map<RouteKey, Route>& routes() {
     return known;
 }
 constexpr size_t kMaxRoutes = 4096;
-constexpr int64_t kMostFrameOutputs = 3ll << 25;      // elements, of a frame's layer on the blocked kernel (see takes_frame)
+
+// Outputs (elements, all steps) up to which the blocked kernel takes a frame's layer. It is bound by its stores, 2-byte elements in runs of a patch row, which share lines with the next
+// patch's, and falls behind where many are under way (that the caches then no longer hold them until they are whole is a guess). Quotients of the dense kernel's time and this one's, over 200 layers, by millions of outputs:
+// * strided whole tiles of the matrix kernel (stems): 1.18 from 40 to 63 (the smallest 1.05), 0.98 to 84, 1.05 to 101 (8 of these 13 up to 1.00, down to 0.90), 0.93 beyond: 3 -> 64 7x7
+//   stride 2 at 224^2 x 18 66 / 60 us, x 20 75 / 82, x 24 96 / 96, x 28 113 / 122, T = 8, x 10 53 / 59;
+// * 1x1 on the time-outer kernel: 2.2 to 84 (the smallest 1.6), 0.64 to 5 at 84 to 100, half of them below 1 beyond (4 -> 96 at 96 x 25 x 50, T = 8 81 / 126);
+// * whole tiles of stride 1 1.14 to 63, 1.4 to 84, 1.07 to 101, 0.94 to 1.45 beyond; layers that tiles do not divide 2.2, 1.8 (one of 7 loses, 0.95), 1.6 and, beyond, 1.36 (29 layers, two of which lose: 0.80, 0.90).
+int64_t most_frame_outputs(DenseFamily family, bool strided) {
+    if (family == DenseFamily::kTInM || family == DenseFamily::kTimeOuter) return 5ll << 24;
+    return family == DenseFamily::kMatrixWhole && strided ? 15ll << 22 : 3ll << 25;
+}
 
 // `frame`: one input of at most eight channels for all timesteps, which the kernel reads as it is.
 Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w,
@@ -490,7 +500,8 @@ Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, 
                   (neuron || (!split && (route.family == DenseFamily::kMatrixMasked || route.family == DenseFamily::kMatrixWhole)));
     if (frame)                                         // (see takes_frame)
         route.taken = route.family != DenseFamily::kPointwise &&
-                      static_cast<int64_t>(T) * N * Cout * ((H + 2 * pad_h - KH) / stride_h + 1) * ((W + 2 * pad_w - KW) / stride_w + 1) <= kMostFrameOutputs;
+                      static_cast<int64_t>(T) * N * Cout * ((H + 2 * pad_h - KH) / stride_h + 1) * ((W + 2 * pad_w - KW) / stride_w + 1) <=
+                          most_frame_outputs(route.family, stride_h > 1 || stride_w > 1);
     if (route.taken) {
         const auto kept = std::make_shared<KeptPlan>();
         BlockedPlan& plan = kept->plan;
@@ -619,7 +630,7 @@ namespace {
 // blocked kernel, which reads the frame as it is and needs no scratch memory (us, matrix kernel / here, T = 4, bf16): 3 -> 64 7x7 stride 2 at 224^2 x 16 62.8 / 48.5, one
 // image 14.6 / 9.9, 3x3 at 32^2 x 64 19.7 / 14.2, one image 11.5 / 6.9, 3 -> 32 stride 2 at 128^2 x 32 33.3 / 14.6, 1 -> 64 5x5 at 28^2 x 50 18.6 / 14.6, 4 -> 96 at 50^2 x 20
 // 40.3 / 20.3, 8 -> 128 at 56^2 x 16 35.5 / 25.4; T = 8 3 -> 64 3x3 at 32^2 x 64 25.8 / 18.7, 4 -> 96 60.3 / 31.2. What the pointwise kernel takes stays there (8 -> 256 1x1 at
-// 56^2 x 16 33.4 / 50.9), and outputs beyond 100 million elements, of which the matrix kernel writes whole lines (7x7 at 224^2 x 16, T = 8, 103 million, 112 / 117). Other neurons take its general epilogue, which is slower than the matrix kernel's
+// 56^2 x 16 33.4 / 50.9), and more outputs than `most_frame_outputs`. Other neurons take its general epilogue, which is slower than the matrix kernel's
 // (77.5 at 224^2 x 16), and stay.
 bool takes_frame(bool shared, int T, int Cin, int x_dtype, int v_dtype, bool residual, const LifParams& lif) {
     return shared && T <= SNNF_MAX_T_PER_LAUNCH && Cin <= 8 && (x_dtype == SNNF_BF16 || x_dtype == SNNF_F16) && v_dtype == SNNF_F32 && !residual &&
