@@ -38,7 +38,7 @@ def test_dense_frame(hip_ops, Cin, Cout, H, W, k, s, N, T, dtype, vdtype, membra
     plan = CB.last_conv_plan()
     assert plan["route"] == "frame" and plan["ran"] == "blocked" and int(plan["window"]) == T, plan
     assert torch.equal(sp.float().cpu(), ref[0]) and 0.01 < float(ref[0].mean()) < 0.9
-    # a neuron that keeps charging ends with more bits than float32 has; both charge it as v + (x - v) / 2
+    # (a neuron that keeps charging ends with more bits than float32 has: charged as v + (x - v) / 2, as by the oracle)
     assert torch.equal(v.cpu(), ref[1].to(vdtype))
     sp2, v2 = S.fused_temporal_conv_lif_state([dx.clone() for _ in range(T)], *args)
     assert torch.equal(sp, sp2) and torch.allclose(v.float(), v2.float(), rtol=1e-6 if vdtype == F32 else 2.0 ** -7, atol=1e-6)
@@ -80,3 +80,34 @@ def test_line_of_large_outputs(hip_ops, T, N, Cin, Cout, H, W, k, s, frame):
     alone, _ = S.fused_temporal_conv_lif_state([x[-1:]] * T, *args)          # (one image: always the blocked kernel)
     assert CB.last_conv_plan().get("route") == "frame"
     assert torch.equal(sp[:, -1:], alone) and 0.0 < float(alone.float().mean()) < 1.0
+
+
+@pytest.mark.parametrize("Cin,Cout,H,k,s,N,T,dtype,same_bits", [
+    (3, 64, 32, 3, 1, 2, 4, BF16, True),       # whole tiles of the matrix kernel, the same order of products
+    (3, 64, 32, 3, 1, 2, 8, F16, True),
+    (3, 64, 224, 7, 2, 2, 4, BF16, False),     # (a small batch of strided layers takes the copy route per timestep)
+    (8, 64, 56, 3, 1, 4, 4, F16, False),       # whole tiles, another order
+    (3, 64, 33, 3, 1, 2, 4, BF16, False),      # planes that tiles do not divide: the copy route per timestep
+])
+def test_equal_frames_with_sums_that_round(hip_ops, Cin, Cout, H, k, s, N, T, dtype, same_bits):
+    """One frame T times against T equal frames on operands whose sums round: the same bits where both add in the same order, else within what the order of additions
+    can change - n products of magnitude sum A differ by up to 2 n 2^-24 A between two orders, and a neuron's halvings sum such differences to less than one of them."""
+    from triton_snn_fusion_amd.runtime import hip_convlif_backend as CB
+    S = torch.ops.snn_custom
+    g = gen(7 * Cin + H)
+    x = dev(torch.randn((N, Cin, H, H), generator=g), dtype)
+    w = dev(torch.randn((Cout, Cin, k, k), generator=g) * 3 * (2 / (Cin * k * k)) ** 0.5, dtype)
+    b = dev(torch.randn(Cout, generator=g) * 0.1, dtype)
+    args = (w, b, torch.zeros((), device=DEV), [s, s], [k // 2, k // 2], [1, 1], 1, *LIF, False)
+    sp, v = S.fused_temporal_conv_lif_state([x] * T, *args)
+    assert CB.last_conv_plan().get("route") == "frame", CB.last_conv_plan()
+    sp2, v2 = S.fused_temporal_conv_lif_state([x.clone() for _ in range(T)], *args)
+    assert CB.last_conv_plan().get("route") != "frame", CB.last_conv_plan()
+    if same_bits:
+        assert "route" not in CB.last_conv_plan(), CB.last_conv_plan()
+        assert torch.equal(sp, sp2) and torch.equal(v, v2)
+    total = torch.nn.functional.conv2d(x.float().cpu().abs(), w.float().cpu().abs(), b.float().cpu().abs(), s, k // 2)
+    bound = (2 * (Cin * k * k + 1) + 4 * T) * 2.0 ** -24 * (total + 1.0)     # (four roundings of a charge per step, of values up to A + 1)
+    same = (sp == sp2).all(0).cpu()
+    assert float((~same).float().mean()) < 1e-4                              # neurons at the threshold
+    assert bool(((v - v2).cpu().abs() <= bound)[same].all())

@@ -245,8 +245,10 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
     float* const v_carry = g.v16 ? v_scratch : v_out;
     constexpr int NF = NARROW ? 1 : 2;         // 32-channel weight fragments of a tile
     constexpr int TG = 4 * NF;                 // channel groups of 8 of a tile
-    // A dense frame with dense spikes is computed as the matrix kernel computes it (which takes frames per timestep, and other neurons): the bias
-    // behind the sums, the charge as v + (x - v) / 2. One frame T times and T equal frames have the same results, bit for bit.
+    // A dense frame with dense spikes is computed in the form of the matrix kernel (which takes other neurons, and frames per timestep of whole tiles): the bias
+    // behind the sums, the charge as v + (x - v) / 2. One frame T times and T equal frames then have the same bits where that kernel also adds a sum's products in this
+    // order (3 -> 64 3x3 at 32^2, 7x7 stride 2 at 224^2 x 16). On other channels and kernels (8 -> 64, 1 -> 64 5x5), and where equal frames take the copy route, whose sums
+    // start from the bias (3 -> 64 at 33^2), they differ in a membrane's last bits where sums round.
     constexpr bool LATE_BIAS = DENSE && IN == SNNF_LAYOUT_NCHW;
     constexpr bool F16 = dtype_of<XT>::value == SNNF_F16;
     constexpr uint32_t ONE = F16 ? 0x3c00u : 0x3f80u;
