@@ -232,7 +232,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
 
     static_assert(!SC || (IN == SNNF_LAYOUT_BITS && TT == 4), "the shortcut variants take bit-packed inputs, four timesteps at a time");
     static_assert(!POOL || (FAST && (TT == 4 || TT == 1)), "the pooled output belongs to the straight-line epilogue of four steps");
-    static_assert(IN != SNNF_LAYOUT_NCHW || TT == 1, "a dense input is one frame for all timesteps");
+    static_assert(IN != SNNF_LAYOUT_NCHW || (TT == 1 && !SK), "a dense input is one frame for all timesteps, of one channel group");
     constexpr bool SPLIT = std::is_same<XT, float>::value;
     static_assert(!NARROW || SK || (!SC && (!POOL || IN == SNNF_LAYOUT_NCHW)), "narrow tiles of one wave: not of a shortcut, and pooled only of a dense frame");
     static_assert(!SPLIT || (NARROW && IN == SNNF_LAYOUT_C8 && !FAST && !SC && !POOL), "fp32 tensors: narrow tiles on two C8 tensors, dense tensors out");
@@ -817,7 +817,8 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             const bool first_window = t0 == 0, last_window = t0 + TT >= nsteps_t;
             const void* v_src = first_window ? v_init : v_carry;          // later windows continue from the stored membrane
             void* const v_dst = last_window ? v_store : v_carry;
-            const bool v_src16 = !SPLIT && g.v16 && first_window, v_dst16 = !SPLIT && g.v16 && last_window;
+            constexpr bool V16 = !SPLIT && IN != SNNF_LAYOUT_NCHW;     // a frame's membrane is fp32 (takes_frame; the internal layouts know no other)
+            const bool v_src16 = V16 && g.v16 && first_window, v_dst16 = V16 && g.v16 && last_window;
             const int t_count = g.shared_x ? g.T : min(TT, g.T - t0);      // LIF steps of this window
             // (Made opaque here: everything derived from the lane's pixel is then computed after the matrix loop instead of
             // before it, where the compiler would otherwise park two dozen store addresses in registers or scratch memory.)
@@ -1852,7 +1853,8 @@ int launch_conv_spk_pooled(const SpkLaunch& L, int tt) {
     return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, 1, IN, true, true, false, true>) : run(conv_spk_kernel<XT, 1, IN, false, true, false, true>);
 }
 
-// The variants that read the network's input as it is: one dense frame of at most 8 channels for all timesteps.
+// The variants that read the network's input as it is: one dense frame of at most 8 channels for all timesteps, hence one channel group in one stage, which
+// waves can't share.
 template <typename XT>
 int launch_conv_spk_frame(const SpkLaunch& L, bool pooled) {
     auto run = [&](auto kernel) -> int {
@@ -1864,15 +1866,14 @@ int launch_conv_spk_frame(const SpkLaunch& L, bool pooled) {
     constexpr int D = SNNF_LAYOUT_NCHW;
     if (L.dense_epilogue) {
         if (L.g.narrow) return run(conv_spk_kernel<XT, 1, D, false, false, false, false, true, true>);
-        return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, 1, D, true, false, false, false, false, true>) : run(conv_spk_kernel<XT, 1, D, false, false, false, false, false, true>);
+        return run(conv_spk_kernel<XT, 1, D, false, false, false, false, false, true>);
     }
     if (L.g.narrow) {
         if (pooled) return run(conv_spk_kernel<XT, 1, D, false, true, false, true, true>);
         return L.fast_epilogue ? run(conv_spk_kernel<XT, 1, D, false, true, false, false, true>) : run(conv_spk_kernel<XT, 1, D, false, false, false, false, true>);
     }
-    if (pooled) return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, 1, D, true, true, false, true>) : run(conv_spk_kernel<XT, 1, D, false, true, false, true>);
-    if (L.fast_epilogue) return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, 1, D, true, true>) : run(conv_spk_kernel<XT, 1, D, false, true>);
-    return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, 1, D, true, false>) : run(conv_spk_kernel<XT, 1, D, false, false>);
+    if (pooled) return run(conv_spk_kernel<XT, 1, D, false, true, false, true>);
+    return L.fast_epilogue ? run(conv_spk_kernel<XT, 1, D, false, true>) : run(conv_spk_kernel<XT, 1, D, false, false>);
 }
 
 // The variants with a projection shortcut in the accumulators: bit-packed inputs, four timesteps side by side.
