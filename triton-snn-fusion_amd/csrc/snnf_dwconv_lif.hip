@@ -308,13 +308,12 @@ int launch(const StepPtrs& xs, const StepPtrs& res, int has_res, int T, DwGeom g
 // the second time, so a step costs a lane six loads, no barrier, no transposition and no tile to zero; lanes of a wave read
 // contiguous rows. (On the tile of `dwconv3x3_lif_kernel` a lane takes 17 floats of a row one by one, 16 floats from its neighbour's: the reads
 // of a wave fall into a few of the LDS banks.) Padding comes from the range check of buffer loads, which answers zero beyond the frame.
-// What bounds it: HBM. 64 channels at 64x64 x 32, T = 4 (84 MB and 8 MB of membrane) 42.4 -> 19.0 us, 128 at 32x32 x 32 25.3 -> 10.0,
-// one image
+// What bounds it: HBM. 64 channels at 64x64 x 32, T = 4 (84 MB and 8 MB of membrane) 42.4 -> 19.0 us, 128 at 32x32 x 32 25.3 -> 10.0, one image
 // 11.1 -> 5.2 (48x48) and 9.8 -> 5.0 (24x24).
 // Stride 1 (8 outputs a strip, the dword behind them as well, the dot products of the kernel below in its order): nine loads a strip and every row three times lose
 // where the vector caches are busy (128 channels at 56x56 x 32 and the pointwise layer behind them 126 -> 145 us), but a launch of up to two workgroups per
-// compute unit is its set-up, which is shorter here: 32 channels at 48x48,
-// one image 7.2 -> 6.0 us, 128 at 24x24 8.0 -> 6.0 (at 32x32 x 16, two rounds of it, 23.6 with the pointwise layer, 24.1 without LDS).
+// compute unit is its set-up, which is shorter here: 32 channels at 48x48, one image 7.2 -> 6.0 us, 128 at 24x24 8.0 -> 6.0 (at 32x32 x 16, two rounds of it, 23.6
+// with the pointwise layer, 24.1 without LDS).
 // ---------------------------------------------------------------------------------------------------------------
 typedef uint32_t dw_u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 dw_bf16x2 __attribute__((ext_vector_type(2)));
@@ -335,7 +334,8 @@ template <> __device__ __forceinline__ float high_element<bf16_t>(uint32_t d) { 
 
 constexpr int64_t kDirectMaxFrame = 0x7fffff00ll;     // bytes of one timestep's input: offsets from 2^31 on lie outside
 constexpr uint32_t kDirectOutside = 0x80000000u;
-constexpr int64_t kDirectStrips = 1 << 17;            // stride 1: strips up to which a launch takes this kernel
+// Stride 1: strips up to which a launch takes this kernel, a strip a thread on two workgroups per compute unit.
+int64_t direct_strips() { return 2ll * compute_units() * kThreads; }
 
 struct DwDirect {
     int strips;              // output strips of 8 input columns in all
@@ -776,7 +776,7 @@ int dispatch_px(int px, bool direct, const StepPtrs& xs, const StepPtrs& res, in
     if constexpr (sizeof(XT) == 2) {
         if (direct) {
             if constexpr (STRIDE == 1) {
-                if (static_cast<int64_t>(g.planes) * g.H * (g.W / 8) > kDirectStrips) return launch_dot<XT, VT>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
+                if (static_cast<int64_t>(g.planes) * g.H * (g.W / 8) > direct_strips()) return launch_dot<XT, VT>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
             }
             return launch_direct<XT, VT, STRIDE>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
         }
