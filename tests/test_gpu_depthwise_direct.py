@@ -84,3 +84,31 @@ def test_stride_1_without_lds(hip_ops, dtype, N, C, H, W, T, residual):
     s1, v1 = S.fused_temporal_depthwise_conv_lif_state(noisy, *args)
     bits, v2 = B.depthwise_conv_lif_rowbits(noisy, args[0], args[1], LIF)
     assert torch.equal(B.unpack_rowbits(bits, dtype), s1) and torch.equal(v1, v2)
+
+
+@pytest.mark.parametrize("dtype,vdtype,T,residual,membrane,lif", [
+    (BF16, F32, 2, True, True, LIF),
+    (F16, F32, 2, True, False, (1.0, 0.25, 2.0)),
+    (BF16, BF16, 3, False, True, LIF),               # 16-bit membranes
+    (F16, F16, 2, True, True, LIF),
+    (BF16, F32, 2, True, True, (1.0, -1.0, 3.0)),    # the general neuron: soft reset, a tau that is no power of two
+    (F16, F16, 2, False, False, (1.0, -1.0, 2.0)),
+    (F16, F32, 2, False, True, (1.0, 0.0, 1.0)),     # integrate and fire
+    (BF16, F32, 18, True, True, LIF),                # two windows of steps
+])
+def test_stride_1_tile_in_lds(hip_ops, dtype, vdtype, T, residual, membrane, lif):
+    """Dense spikes from the tile in LDS, at the fewest strips that it takes (on 256 compute units): residuals, membranes of either dtype, every neuron, several windows."""
+    N, C, H, W = 8, 65, 32, 64
+    assert N * C * H * W // 8 > 2 * 256 * 256
+    g = gen(T + 3 * int(residual))
+    xs = [spikes((N, C, H, W), 0.4, g) for _ in range(T)]
+    rs = [spikes((N, C, H, W), 0.3, g) for _ in range(T)] if residual else None
+    w, b = _layer(C, g)
+    v0 = torch.randint(-16, 16, (N, C, H, W), generator=g) / 32.0 if membrane else None
+    ref = O.temporal_conv_lif(xs, w, b, torch.tensor(0.0) if v0 is None else v0, (1, 1), (1, 1), (1, 1), C, *lif, residuals=rs)
+    vi = zero_v(vdtype) if v0 is None else dev(v0, vdtype)
+    args = (dev(w, dtype), dev(b, dtype), vi, [1, 1], [1, 1], [1, 1], C, *lif, False)
+    dx = [dev(x, dtype) for x in xs]
+    s, v = S.fused_temporal_depthwise_conv_lif_state(dx, *args) if rs is None else S.fused_temporal_conv_add_lif_state_depthwise(dx, [dev(r, dtype) for r in rs], *args)
+    assert torch.equal(s.float().cpu(), ref[0]) and torch.equal(v.cpu(), ref[1].to(vdtype))
+    assert 0.01 < float(ref[0].mean()) < 0.99

@@ -187,8 +187,9 @@ def test_random_linear_scan_and_tail_cases(hip_ops, seed, cases):
 
 @pytest.mark.parametrize("seed,cases", [(17, 150)])
 def test_random_row_packed_depthwise_and_pointwise_cases(hip_ops, seed, cases):
-    """The entry points on row-packed spikes against the dense operators (themselves gated on the oracle above): the same
-    kernels with another fetch or store, so spikes and membranes are compared bit for bit."""
+    """The entry points on row-packed spikes against the dense operators (themselves gated on the oracle above), bit for bit: the
+    same pointwise kernel with another fetch or store, and the depthwise tile in LDS against the kernel without LDS that dense
+    launches of these sizes take (rows of whole vectors; the same products in the same order)."""
     from triton_snn_fusion_amd.runtime import hip_blocked_backend as B
     from triton_snn_fusion_amd.runtime.hip_convlif_backend import last_conv_plan
     rnd = random.Random(seed)

@@ -485,7 +485,7 @@ def test_internal_layouts_track_the_dense_executor(hip_ops, name):
     print(f"{name}: internal layouts vs dense executor, cosine similarity of the logits {cos:.5f}")
     assert cos > 0.8, cos
     if name == "mobilenet":
-        # The row-packed entry points are the dense kernels with another fetch / store: every spike tensor up to the last
+        # The row-packed entry points add what the dense kernels add, in the same order: every spike tensor up to the last
         # convolution is the same, bit for bit (the last convolution and the tail differ: its sums meet the tail's neuron
         # unrounded on the internal layouts).
         same = [(d["name"], torch.equal(d["spikes"], i["spikes"])) for d, i in zip(dense.record, internal.record)
