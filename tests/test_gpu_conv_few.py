@@ -138,3 +138,26 @@ def test_rounding_of_the_charge(B, lif, T):
     assert torch.equal(sp, sp2) and torch.equal(v, v2)
     if lif[1] < 0:
         assert torch.equal(sp, ref[0]) and torch.equal(v, ref[1])
+
+
+@pytest.mark.parametrize("Cin,k,value", [(72, 3, float("inf")), (72, 3, float("nan")), (200, 1, float("inf")), (200, 1, float("nan")), (64, 5, float("inf"))])
+def test_an_output_sees_its_own_inputs_only(B, Cin, k, value):
+    """An infinity or NaN reaches the outputs whose window holds it and no other: neither through the entry that an odd number leaves without a partner, nor through
+    padding, an odd number of channel groups or pixels beyond the plane."""
+    g = gen(Cin + k)
+    T, Cout, H, W = 4, 48, 5, 7
+    x, w, b, _ = _operands(T, 1, Cin, Cout, H, W, k, 1, False, "c8", g)
+    w = torch.where(w == 0, torch.full_like(w, w.abs().max().item()), w).abs()       # (no product is 0 x infinity, all have one sign)
+    xb = B.from_dense(dev(x, BF16), B.C8)
+    args = (dev(w, BF16), dev(b, BF16), [1, 1], [k // 2, k // 2], LIF)
+    sp, v = B.conv_lif_blocked(xb, *args, want_v=True)
+    assert "few" in B.last_conv_plan(), B.last_conv_plan()
+    bad = x.clone()
+    bad[1, 0, Cin - 1, 4, 6] = value                                                 # the last channel of the last pixel
+    sp2, v2 = B.conv_lif_blocked(B.from_dense(dev(bad, BF16), B.C8), *args, want_v=True)
+    seen = torch.zeros((H, W), dtype=torch.bool)
+    seen[max(0, 4 - k // 2):, max(0, 6 - k // 2):] = True
+    one, two = B.to_dense(sp).float().cpu(), B.to_dense(sp2).float().cpu()
+    assert torch.equal(v.cpu()[:, :, ~seen], v2.cpu()[:, :, ~seen]) and torch.equal(one[..., ~seen], two[..., ~seen]) and torch.equal(one[0], two[0])
+    fired = two[1, 0][:, seen]
+    assert bool((fired == (1.0 if value == float("inf") else 0.0)).all()), fired
