@@ -6,14 +6,14 @@
 // channel groups of 8, v_mfma_f32_32x32x16, fp32 accumulate, TT timesteps side by side against one weight fragment), but:
 //   * a group of 8 channels of one pixel is 16 contiguous bytes in C8 and one byte in BITS, i.e. already the matrix
 //     operand of a lane: staging is one load and one 16-byte LDS write per item, no transposition; a spike byte is
-//     expanded to eight 16-bit ones with 13 integer instructions on its way into LDS;
+//     expanded to eight 16-bit ones with 9 integer instructions on its way into LDS;
 //   * every wave is its own pipeline: it owns a patch of 32 output pixels x 64 output channels x TT timesteps, stages
 //     the halo of its patch into a private LDS region and never meets a workgroup barrier in the matrix loop, so the
 //     eight waves of a compute unit drift apart and one wave's staging and epilogue overlap another's matrix work;
 //   * spikes leave as bits: the accumulator layout gives a lane 4 consecutive channels of its pixel, the two halves of
 //     a wave exchange their nibbles with one cross-lane move and store bytes; the membrane is fp32 NCHW and optional;
 //   * deep layers with few pixels split K over WK waves of a workgroup (whole LDS stages each) and add their partial
-//     sums through LDS in a fixed order, one timestep per round;
+//     sums through LDS in a fixed order;
 //   * neighbours of a convolution that fit its tile join its launch: the 1x1 projection shortcut of a residual block as
 //     further K steps on a second input (SC), the 2x2 average pool of the spikes as a reduce-scatter between the four
 //     lanes of a window (POOL), and a network's dense input frame of at most 8 channels read as it is (IN = NCHW).
@@ -627,8 +627,8 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     for (int f = 0; f < NF; ++f) acc[t][f] = acc[0][f];
             };
             // Waves of several tiles take turns of one tile each: half a tile out of step, one's epilogue runs under the other's matrix instructions, and
-            // both end together (the older wave ahead all the way, the other one's last tile ran alone: 256 -> 256 at 14^2 x 128 105.3 -> 102.9 us,
-            // 128 -> 128 at 28^2 x 128 110.4 -> 104.3; turns of a stage each kept the two in step, 64 -> 64 at 56^2 x 128 99.9 -> 102.4).
+            // both end together (the older wave ahead all the way, the other one's last tile ran alone: 256 -> 256 at 14^2 x 128 97.1 -> 95.9 us,
+            // 128 -> 128 at 28^2 x 128 101.1 -> 98.0, 64 -> 64 at 56^2 x 128 96.0 -> 95.7; turns of a stage each kept the two in step and lost 2 % there).
             if (!SK && g.iters > 1) {
                 if (wave >= 4) __builtin_amdgcn_s_setprio(2);
                 else if (it & 1) __builtin_amdgcn_s_setprio(1);
@@ -691,15 +691,10 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                         if (stage + s_step < nstages_all) stage_req(stage + s_step);
                     }
                     read_b(0, bo[0]);
-                    // The two waves of a SIMD (w and w + 4) share its matrix cores, and the older one wins every instruction at equal priority: it then
-                    // ran through its stages alone, and the other one through its own, with nothing under either's staging. So the wave with more
-                    // stages left goes first (parts of a tile: 128 -> 128 at 28^2 x 16 20.9 -> 20.0 us, 512 -> 512 at 7^2 x 16 19.8 -> 18.9), and where waves have
-                    // several tiles, each in turn for the length of one (half a tile out of step, so that one's epilogue runs under the other's matrix
-                    // instructions, and both end together: 256 -> 256 at 14^2 x 128 98.9 -> 97.0, 128 -> 128 at 28^2 x 128 104.9 -> 100.4). Staging gives way to
-                    // them, unless it takes a second batch of items (64 -> 128 stride 2 at 56^2 x 16 17.3 -> 16.9).
                     // The two waves of a SIMD (w and w + 4) share its matrix cores, and at equal priority the older one wins every instruction: it ran
                     // through all its stages, and then the other one through its own, with nothing under either's staging. So a wave on its last stage
-                    // gives way to one that is not (128 -> 128 at 28^2 x 16, two stages per wave, 20.9 -> 20.4 us, 72 -> 104 at 28^2 x 5 12.4 -> 12.1).
+                    // gives way to one that is not (128 -> 128 at 28^2 x 16, two stages per wave, 18.1 -> 17.6 us, 512 -> 512 at 7^2 x 16 18.7 -> 18.3, 64 -> 128 stride 2 at
+                    // 56^2 x 16 16.1 -> 15.5; 72 -> 104 at 28^2 x 5 with a residual, one or two stages, 11.0 either way).
                     if (SK || g.iters == 1) {
                         if (stage + s_step < nstages_all) __builtin_amdgcn_s_setprio(2);
                         else __builtin_amdgcn_s_setprio(1);
