@@ -497,6 +497,8 @@ int launch_direct(const StepPtrs& xs, const StepPtrs& res, int has_res, int T, c
 // (two 16-bit products added to an fp32 accumulator): the products are exact in fp32, as with an fp32 multiply-add, and an
 // output takes two instructions per kernel row instead of three. This kernel is bound by its vector and LDS instructions
 // (with a third of the taps it runs at 6.5 TB/s), so the count is what matters.
+// An instruction's unused element is multiplied by zero: inputs are finite (an infinity also makes the outputs two columns beside it NaN, here and at
+// stride 1 without LDS).
 // Row layout: input column c at element kDotColOffset + c; the elements before and after the row are the zero halo. For
 // the strip at elements e0 .. e0 + 7 (e0 a multiple of 8) a row costs one 16-byte read and the two dwords around it.
 // ---------------------------------------------------------------------------------------------------------------
