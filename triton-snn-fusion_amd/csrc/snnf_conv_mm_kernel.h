@@ -207,10 +207,13 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) __attribute__((amdgpu_waves_per_eu
                         for (int k = 0; k < 4; ++k) {
                             const float a0 = __uint_as_float(pre[s][t][2 * k][0]), a1 = __uint_as_float(pre[s][t][2 * k + 1][0]);
                             const float b0 = __uint_as_float(pre[s][t][2 * k][1]), b1 = __uint_as_float(pre[s][t][2 * k + 1][1]);
-                            lo[k] = split_bf16_bits(a0, false) | (split_bf16_bits(a1, false) << 16);
-                            hi[k] = split_bf16_bits(b0, false) | (split_bf16_bits(b1, false) << 16);
-                            lo2[k] = zero0 ? 0u : (split_bf16_bits(a0, true) | (split_bf16_bits(a1, true) << 16));
-                            hi2[k] = zero1 ? 0u : (split_bf16_bits(b0, true) | (split_bf16_bits(b1, true) << 16));
+                            uint32_t a_high, a_low, b_high, b_low;
+                            split_bf16_pair(a0, a1, a_high, a_low);
+                            split_bf16_pair(b0, b1, b_high, b_low);
+                            lo[k] = a_high;
+                            hi[k] = b_high;
+                            lo2[k] = zero0 ? 0u : a_low;
+                            hi2[k] = zero1 ? 0u : b_low;
                         }
                         unsigned char* dst2 = lds + t * tile_bytes + item_dst[s] + lo_off;
                         *reinterpret_cast<cv_u32x4*>(dst2) = lo2;

@@ -122,8 +122,7 @@ __global__ __launch_bounds__(kThreads) void steps_to_c8_split_kernel(const StepP
     uint32_t any = 0;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        hi.v[k] = split_bf16_bits(v[2 * k], false) | (split_bf16_bits(v[2 * k + 1], false) << 16);
-        lo.v[k] = split_bf16_bits(v[2 * k], true) | (split_bf16_bits(v[2 * k + 1], true) << 16);
+        split_bf16_pair(v[2 * k], v[2 * k + 1], hi.v[k], lo.v[k]);
         any |= lo.v[k] & 0x7fff7fffu;
     }
     const bool wave_any = __ballot(any != 0u) != 0ull;
