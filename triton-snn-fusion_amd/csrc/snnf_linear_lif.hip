@@ -3,11 +3,10 @@
 // Both operands are K-contiguous in memory (x rows and W rows), which is the per-lane operand order of
 // v_mfma_f32_16x16x32 (8 consecutive k per lane). All T timesteps of a row tile share one weight fragment (the weight is
 // streamed once per workgroup, not once per timestep), and each thread runs the LIF recurrence over T for its (row,
-// output feature) pair with the membrane in a register. Two kernels: the staged one (4 timesteps or more, aligned rows)
-// moves K slabs of all operand rows through LDS with coalesced loads; the direct one (everything else) loads fragments
-// straight from global memory, its 8 (beyond 8 timesteps, 4) waves splitting K in pairs of K steps with partial sums
-// meeting in LDS.
+// output feature) pair with the membrane in a register. The staged kernel moves K slabs of all operand rows through LDS with
+// coalesced loads; the direct one (short K of one or two timesteps) loads fragments straight from global memory.
 #include <algorithm>
+#include <type_traits>
 
 #include "snnf_common.h"
 
@@ -24,14 +23,13 @@ constexpr int kTileM = 16;    // rows per workgroup (per timestep)
 
 // fp32 tensors: both operands enter the matrix cores as two bf16 terms (value rounded to bf16, and the rounded remainder),
 // and three of the four products are accumulated: w_hi x_hi + w_lo x_hi + w_hi x_lo (the fourth is below 2^-16 of the
-// result). The three products are three passes over K ("K parts"): part 0 multiplies the high terms, part 1 the weights' low
-// terms with the activations' high terms, part 2 the other way round. 16-bit tensors have one part.
+// result). A slab of both terms lies in LDS; the products of a K step follow each other in the order above.
 struct LinGeom {
     int T, M, Fin, Fout;
     int64_t x_row_stride;      // elements
     int64_t spike_step_stride; // elements
-    int ksteps;                // ceil(Fin / 32)
-    int kparts;                // 1, or 3 for fp32 tensors
+    int x_even = 0;            // staged kernel: whether the timesteps' activations lie at equal distances,
+    int64_t x_step_stride = 0; // ... and the bytes between them
     int v_in_place = 0;        // staged kernel: the initial membrane lies in v_store
 };
 
@@ -41,81 +39,49 @@ template <> struct Frag<bf16_t> { using type = bf16x8; };
 template <> struct Frag<float> { using type = bf16x8; };
 template <> struct Frag<f16_t> { using type = f16x8; };
 
-// Two fp32 values as a pair of bf16 terms: their roundings to bf16, or (low_term) what those roundings left over.
-__device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi, bool low_term) {
-    return split_bf16_bits(lo, low_term) | (split_bf16_bits(hi, low_term) << 16);
-}
-
-// Loads k .. k+7 of `row`; elements at or beyond `kmax` read as zero. FAST requires 16-byte aligned rows and kmax % 8 == 0
-// and is branch-free (an octet beyond kmax re-reads the row's first one and is zeroed): a branch around a load would make
-// the compiler wait for every load before it issues the next.
-template <typename XT, bool FAST>
-__device__ __forceinline__ u32x4 load_octet(const XT* __restrict__ row, int k, int kmax, bool low_term = false) {
-    u32x4 out = {0u, 0u, 0u, 0u};
-    if constexpr (FAST) {
-        const bool inside = k < kmax;
-        const XT* __restrict__ src = row + (inside ? k : 0);
-        if constexpr (sizeof(XT) == 2) {
-            out = *reinterpret_cast<const u32x4*>(src);
-        } else {
-            const f32x4 a = *reinterpret_cast<const f32x4*>(src);
-            const f32x4 b = *reinterpret_cast<const f32x4*>(src + 4);
-            out[0] = pack_bf16x2(a[0], a[1], low_term);
-            out[1] = pack_bf16x2(a[2], a[3], low_term);
-            out[2] = pack_bf16x2(b[0], b[1], low_term);
-            out[3] = pack_bf16x2(b[2], b[3], low_term);
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) out[j] = inside ? out[j] : 0u;
-    } else if constexpr (sizeof(XT) == 2) {
-        const uint16_t* p = reinterpret_cast<const uint16_t*>(row);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t lo = (k + 2 * j) < kmax ? p[k + 2 * j] : 0u;
-            const uint32_t hi = (k + 2 * j + 1) < kmax ? p[k + 2 * j + 1] : 0u;
-            out[j] = lo | (hi << 16);
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const float lo = (k + 2 * j) < kmax ? to_float(row[k + 2 * j]) : 0.0f;
-            const float hi = (k + 2 * j + 1) < kmax ? to_float(row[k + 2 * j + 1]) : 0.0f;
-            out[j] = pack_bf16x2(lo, hi, low_term);
-        }
-    }
-    return out;
-}
-
-// The same octet in two steps, for loads that stay in flight over other work: the raw 16 (fp32 storage: 32) bytes as
+// Eight K elements of a row in two steps, for loads that stay in flight over other work: the raw 16 (fp32 storage: 32) bytes as
 // loaded, and their conversion to a matrix operand (zero when the octet lies beyond K) at the point of use. Converting
-// where the load is issued would make the wave wait for it there.
+// where the load is issued would make the wave wait for it there. A row may start at any element: the loads are of 16 bytes
+// at the alignment of an element, which the hardware takes at any address (measured the same as aligned ones on aligned rows).
 template <typename XT> struct RawOctet { u32x4 lo; };
-template <> struct RawOctet<float> { f32x4 lo, hi; };
+template <> struct RawOctet<float> { u32x4 lo, hi; };
 template <typename XT>
 __device__ __forceinline__ RawOctet<XT> load_raw_octet(const XT* __restrict__ src) {
     RawOctet<XT> r;
-    if constexpr (sizeof(XT) == 2) {
-        r.lo = *reinterpret_cast<const u32x4*>(src);
-    } else {
-        r.lo = *reinterpret_cast<const f32x4*>(src);
-        r.hi = *reinterpret_cast<const f32x4*>(src + 4);
-    }
+    __builtin_memcpy(&r.lo, src, 16);
+    if constexpr (sizeof(XT) == 4) __builtin_memcpy(&r.hi, src + 4, 16);
     return r;
 }
-template <typename XT>
-__device__ __forceinline__ u32x4 finish_octet(const RawOctet<XT>& r, bool inside, bool low_term) {
-    u32x4 out;
-    if constexpr (sizeof(XT) == 2) {
-        out = r.lo;
-    } else {
-        out[0] = pack_bf16x2(r.lo[0], r.lo[1], low_term);
-        out[1] = pack_bf16x2(r.lo[2], r.lo[3], low_term);
-        out[2] = pack_bf16x2(r.hi[0], r.hi[1], low_term);
-        out[3] = pack_bf16x2(r.hi[2], r.hi[3], low_term);
-    }
+// The octet in which a row ends inside was loaded from the row's last eight elements: its first element is element `drop` of what was
+// loaded, and what comes behind the row's last one is zero.
+__device__ __forceinline__ void drop_elements(RawOctet<bf16_t>& r, int drop) {
+    uint64_t a = r.lo[0] | static_cast<uint64_t>(r.lo[1]) << 32, b = r.lo[2] | static_cast<uint64_t>(r.lo[3]) << 32;
+    if (drop & 4) { a = b; b = 0; }
+    const int bits = 16 * (drop & 3);
+    if (bits != 0) { a = a >> bits | b << (64 - bits); b >>= bits; }
+    r.lo = u32x4{static_cast<uint32_t>(a), static_cast<uint32_t>(a >> 32), static_cast<uint32_t>(b), static_cast<uint32_t>(b >> 32)};
+}
+__device__ __forceinline__ void drop_elements(RawOctet<f16_t>& r, int drop) {
+    RawOctet<bf16_t> same = {r.lo};
+    drop_elements(same, drop);
+    r.lo = same.lo;
+}
+__device__ __forceinline__ void drop_elements(RawOctet<float>& r, int drop) {
+    uint32_t e[8] = {r.lo[0], r.lo[1], r.lo[2], r.lo[3], r.hi[0], r.hi[1], r.hi[2], r.hi[3]};
 #pragma unroll
-    for (int j = 0; j < 4; ++j) out[j] = inside ? out[j] : 0u;
-    return out;
+    for (int step = 4; step >= 1; step >>= 1)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const uint32_t moved = i + step < 8 ? e[i + step < 8 ? i + step : 0] : 0u;
+            e[i] = (drop & step) ? moved : e[i];
+        }
+    r.lo = u32x4{e[0], e[1], e[2], e[3]};
+    r.hi = u32x4{e[4], e[5], e[6], e[7]};
+}
+__device__ __forceinline__ u32x4 keep_octet(u32x4 v, bool inside) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = inside ? v[j] : 0u;
+    return v;
 }
 
 // Eight features at one bit each (bit j = feature j) as a matrix operand of zeros and ones.
@@ -139,91 +105,68 @@ __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
     }
 }
 
-// Waves per workgroup: they split K, so more waves mean more loads in flight per CU.
-template <int TT> struct LinWaves { static constexpr int value = TT <= 8 ? 8 : 4; };
-
-// OCF: fragments of 16 output features per workgroup. Two fragments share every activation fragment (half the activation
-// traffic per output) at the price of half as many workgroups.
-template <typename XT, typename VT, int TT, bool FAST, int OCF>
-__global__ __launch_bounds__(LinWaves<TT>::value * 64) void linear_lif_kernel(StepPtrs xs, LinGeom g, const XT* __restrict__ W,
-                                                                              const XT* __restrict__ bias,
-                                                                              const VT* v_init, XT* __restrict__ spikes,
-                                                                              VT* v_out, LifParams lif) {
-    constexpr int NW = LinWaves<TT>::value;
-    constexpr int TILE_OC = OCF * kTileOC;
-    constexpr int OUTS = TILE_OC * kTileM;                    // outputs per workgroup and timestep
-    constexpr int PITCH = TILE_OC + 4;                        // floats per row of a partial tile: the 16-byte writes of
-                                                              // 8 consecutive lanes (8 rows) then fall into distinct banks
-    constexpr int SLAB = kTileM * PITCH;                      // floats per (wave, timestep)
-    extern __shared__ __align__(16) float partial[];          // [NW][TT][kTileM][PITCH]
+// One or two timesteps of 16-bit rows of whole octets and a short K: the fragments come straight from memory, eight waves split K in pairs of steps, and their
+// partial sums meet in LDS. There is one trip to memory and one meeting, where a slab in LDS takes two (see launch_tt).
+constexpr int kDirectWaves = 8;
+template <typename XT, typename VT, int TT>
+__global__ __launch_bounds__(kDirectWaves * 64) void linear_lif_direct_kernel(StepPtrs xs, LinGeom g, const XT* __restrict__ W, const XT* __restrict__ bias,
+                                                                              const VT* v_init, XT* __restrict__ spikes, VT* v_out, LifParams lif) {
+    static_assert(sizeof(XT) == 2, "16-bit tensors");
+    constexpr int PITCH = kTileOC + 4;      // floats per row of a partial tile: the 16-byte writes of 8 consecutive lanes (8 rows) then fall into distinct banks
+    constexpr int SLAB = kTileM * PITCH;    // floats per (wave, timestep)
+    __shared__ __align__(16) float partial[kDirectWaves * TT * SLAB];
     const int wave = threadIdx.x >> 6;
     const int lane = threadIdx.x & 63;
-    const int oc0 = blockIdx.x * TILE_OC;
+    const int oc0 = blockIdx.x * kTileOC;
     const int m0 = blockIdx.y * kTileM;
 
     // Operand rows of this lane (clamped: out-of-range rows compute garbage that is never stored).
-    const int b_row = min(m0 + (lane & 15), g.M - 1);
     const int koff = (lane >> 4) * 8;
-    const XT* wrow[OCF];
-#pragma unroll
-    for (int f = 0; f < OCF; ++f) wrow[f] = W + static_cast<int64_t>(min(oc0 + f * kTileOC + (lane & 15), g.Fout - 1)) * g.Fin;
+    const XT* const wrow = W + static_cast<int64_t>(min(oc0 + (lane & 15), g.Fout - 1)) * g.Fin;
     const XT* xrow[TT];
 #pragma unroll
-    for (int t = 0; t < TT; ++t) xrow[t] = static_cast<const XT*>(xs.p[t]) + static_cast<int64_t>(b_row) * g.x_row_stride;
+    for (int t = 0; t < TT; ++t) xrow[t] = static_cast<const XT*>(xs.p[t]) + static_cast<int64_t>(min(m0 + (lane & 15), g.M - 1)) * g.x_row_stride;
 
-    f32x4 acc[OCF][TT];
+    f32x4 acc[TT];
 #pragma unroll
-    for (int f = 0; f < OCF; ++f)
-#pragma unroll
-        for (int t = 0; t < TT; ++t) acc[f][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-
+    for (int t = 0; t < TT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     // K steps (32 elements of K each) are dealt to the waves in pairs: the two steps of a pair read the two halves of the
     // same 128-byte lines of every operand row back to back. The loads of both steps are issued before the first
-    // matrix instruction; the other wave of the SIMD covers the wait.
-    u32x4 a0[OCF], a1[OCF], b0[TT], b1[TT];
-    auto fetch = [&](int s, u32x4 (&a)[OCF], u32x4 (&b)[TT]) __attribute__((always_inline)) {
-        int part = 0;        // fp32 tensors: step s of K part `part` (see LinGeom)
-        if constexpr (sizeof(XT) == 4) {
-            part = s >= 2 * g.ksteps ? 2 : (s >= g.ksteps ? 1 : 0);
-            s -= part * g.ksteps;
-        }
+    // matrix instruction; the other wave of the SIMD covers the wait. (No branch around a load: an octet beyond K re-reads the row's first one and is zeroed.)
+    u32x4 a0, a1, b0[TT], b1[TT];
+    auto fetch = [&](int s, u32x4& a, u32x4 (&b)[TT]) __attribute__((always_inline)) {
         const int k = s * 32 + koff;
+        const bool inside = k < g.Fin;
+        const int ks = inside ? k : 0;
+        a = keep_octet(*reinterpret_cast<const u32x4*>(wrow + ks), inside);
 #pragma unroll
-        for (int f = 0; f < OCF; ++f) a[f] = load_octet<XT, FAST>(wrow[f], k, g.Fin, part == 1);
-#pragma unroll
-        for (int t = 0; t < TT; ++t) b[t] = load_octet<XT, FAST>(xrow[t], k, g.Fin, part == 2);
+        for (int t = 0; t < TT; ++t) b[t] = keep_octet(*reinterpret_cast<const u32x4*>(xrow[t] + ks), inside);
     };
-    auto multiply = [&](const u32x4 (&a)[OCF], const u32x4 (&b)[TT]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int t = 0; t < TT; ++t)
-#pragma unroll
-            for (int f = 0; f < OCF; ++f) acc[f][t] = mfma16<XT>(a[f], b[t], acc[f][t]);
-    };
-    const int all_steps = g.kparts * g.ksteps;
-    for (int s = 2 * wave; s < all_steps; s += 2 * NW) {
+    const int all_steps = (g.Fin + 31) / 32;
+    for (int s = 2 * wave; s < all_steps; s += 2 * kDirectWaves) {
         const bool second = s + 1 < all_steps;
         fetch(s, a0, b0);
         if (second) fetch(s + 1, a1, b1);
-        multiply(a0, b0);
-        if (second) multiply(a1, b1);
+#pragma unroll
+        for (int t = 0; t < TT; ++t) acc[t] = mfma16<XT>(a0, b0[t], acc[t]);
+        if (second) {
+#pragma unroll
+            for (int t = 0; t < TT; ++t) acc[t] = mfma16<XT>(a1, b1[t], acc[t]);
+        }
     }
 
     // D[i = oc][j = m]: lane holds column j = lane % 16, rows i = 4 * (lane / 16) + r.
 #pragma unroll
     for (int t = 0; t < TT; ++t)
 #pragma unroll
-        for (int f = 0; f < OCF; ++f)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                partial[(wave * TT + t) * SLAB + (lane & 15) * PITCH + f * kTileOC + (lane >> 4) * 4 + r] = acc[f][t][r];
+        for (int r = 0; r < 4; ++r) partial[(wave * TT + t) * SLAB + (lane & 15) * PITCH + (lane >> 4) * 4 + r] = acc[t][r];
     __syncthreads();
 
-    // Output e of the tile = (row e / TILE_OC, feature e % TILE_OC): consecutive threads write consecutive features. The
-    // partial sums are added in a fixed order.
-    for (int e = threadIdx.x; e < OUTS; e += NW * 64) {
-        const int slot = (e / TILE_OC) * PITCH + e % TILE_OC;
-        const int m = m0 + e / TILE_OC;
-        const int oc = oc0 + e % TILE_OC;
+    // Output e of the tile = (row e / 16, feature e % 16): consecutive threads write consecutive features. The partial sums are added in a fixed order.
+    for (int e = threadIdx.x; e < kTileOC * kTileM; e += kDirectWaves * 64) {
+        const int slot = (e / kTileOC) * PITCH + e % kTileOC;
+        const int m = m0 + e / kTileOC;
+        const int oc = oc0 + e % kTileOC;
         if (m >= g.M || oc >= g.Fout) continue;
         const float bv = bias != nullptr ? to_float(bias[oc]) : 0.0f;
         const int64_t o = static_cast<int64_t>(m) * g.Fout + oc;
@@ -233,36 +176,61 @@ __global__ __launch_bounds__(LinWaves<TT>::value * 64) void linear_lif_kernel(St
             if (t < g.T) {      // a guard, not a break: a second loop exit keeps the compiler from unrolling over t
                 float sum = 0.0f;
 #pragma unroll
-                for (int w = 0; w < NW; w += 2) sum += partial[(w * TT + t) * SLAB + slot] + partial[((w + 1) * TT + t) * SLAB + slot];
-                const float cur = sum + bv;
-                spikes[t * g.spike_step_stride + o] = spike_value<XT>(lif_step(cur, v, lif));
+                for (int w = 0; w < kDirectWaves; w += 2) sum += partial[(w * TT + t) * SLAB + slot] + partial[((w + 1) * TT + t) * SLAB + slot];
+                spikes[t * g.spike_step_stride + o] = spike_value<XT>(lif_step(sum + bv, v, lif));
             }
         }
         v_out[o] = from_float<VT>(v);
     }
 }
 
-template <typename XT, typename VT, int TT, bool FAST, int OCF>
-int launch_one(const StepPtrs& xs, const LinGeom& g, const void* W, const void* bias, const void* v_init, void* spikes,
-               void* v_out, const LifParams& lif, hipStream_t stream) {
-    constexpr int NW = LinWaves<TT>::value;
-    constexpr size_t lds = static_cast<size_t>(NW) * TT * kTileM * (OCF * kTileOC + 4) * sizeof(float);
-    static_assert(lds <= 160 * 1024, "partial sums exceed LDS");
-    const dim3 grid((g.Fout + OCF * kTileOC - 1) / (OCF * kTileOC), (g.M + kTileM - 1) / kTileM);
+template <typename XT, typename VT, int TT>
+int launch_direct(const StepPtrs& xs, const LinGeom& g, const void* W, const void* bias, const void* v_init, void* spikes, void* v_out, const LifParams& lif,
+                  hipStream_t stream) {
+    const dim3 grid((g.Fout + kTileOC - 1) / kTileOC, (g.M + kTileM - 1) / kTileM);
     if (grid.y > 65535) return fail(SNNF_ERR_UNSUPPORTED, "snnf_linear_lif: M=%d too large", g.M);
-    auto kernel = linear_lif_kernel<XT, VT, TT, FAST, OCF>;
-    if (lds > 64 * 1024) {
-        static const hipError_t raised =
-            hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-        if (raised != hipSuccess) return fail(SNNF_ERR_LAUNCH, "snnf_linear_lif: cannot reserve %zu bytes of LDS", lds);
+    linear_lif_direct_kernel<XT, VT, TT><<<grid, kDirectWaves * 64, 0, stream>>>(xs, g, static_cast<const XT*>(W), static_cast<const XT*>(bias), static_cast<const VT*>(v_init),
+                                                                                 static_cast<XT*>(spikes), static_cast<VT*>(v_out), lif);
+    return check_launch("snnf_linear_lif");
+}
+
+// Rows of less than eight features, which have no octet to load: a thread per output, fp32 products.
+constexpr int kShortThreads = 256;
+template <typename XT, typename VT>
+__global__ __launch_bounds__(kShortThreads) void linear_lif_short_kernel(StepPtrs xs, LinGeom g, const XT* __restrict__ W, const XT* __restrict__ bias,
+                                                                         const VT* v_init, XT* __restrict__ spikes, VT* v_out, LifParams lif) {
+    const int64_t o = static_cast<int64_t>(blockIdx.x) * kShortThreads + threadIdx.x;
+    if (o >= static_cast<int64_t>(g.M) * g.Fout) return;
+    const int64_t m = o / g.Fout;
+    const int oc = static_cast<int>(o - m * g.Fout);
+    float w[7];
+#pragma unroll
+    for (int k = 0; k < 7; ++k) w[k] = k < g.Fin ? to_float(W[static_cast<int64_t>(oc) * g.Fin + k]) : 0.0f;
+    const float bv = bias != nullptr ? to_float(bias[oc]) : 0.0f;
+    float v = v_init != nullptr ? to_float(v_init[o]) : 0.0f;
+    for (int t = 0; t < g.T; ++t) {
+        const XT* __restrict__ x = static_cast<const XT*>(xs.p[t]) + m * g.x_row_stride;
+        float sum = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 7; ++k)
+            if (k < g.Fin) sum = fmaf(w[k], to_float(x[k]), sum);
+        spikes[t * g.spike_step_stride + o] = spike_value<XT>(lif_step(sum + bv, v, lif));
     }
-    kernel<<<grid, NW * 64, lds, stream>>>(xs, g, static_cast<const XT*>(W), static_cast<const XT*>(bias),
-                                           static_cast<const VT*>(v_init), static_cast<XT*>(spikes), static_cast<VT*>(v_out), lif);
+    v_out[o] = from_float<VT>(v);
+}
+
+template <typename XT, typename VT>
+int launch_short(const StepPtrs& xs, const LinGeom& g, const void* W, const void* bias, const void* v_init, void* spikes, void* v_out, const LifParams& lif,
+                 hipStream_t stream) {
+    const int64_t blocks = (static_cast<int64_t>(g.M) * g.Fout + kShortThreads - 1) / kShortThreads;
+    if ((g.M + kTileM - 1) / kTileM > 65535 || blocks > 0x7fffffffLL) return fail(SNNF_ERR_UNSUPPORTED, "snnf_linear_lif: M=%d too large", g.M);
+    linear_lif_short_kernel<XT, VT><<<dim3(static_cast<unsigned>(blocks)), kShortThreads, 0, stream>>>(
+        xs, g, static_cast<const XT*>(W), static_cast<const XT*>(bias), static_cast<const VT*>(v_init), static_cast<XT*>(spikes), static_cast<VT*>(v_out), lif);
     return check_launch("snnf_linear_lif");
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// Staged variant (4 timesteps or more, 16-byte aligned rows, Fin % 8 == 0). Operand fragments fetched straight from
+// Staged variant. Operand fragments fetched straight from
 // global memory put the 16 rows of a fragment in 16 adjacent lanes, i.e. 16 different cache lines per 256 bytes
 // fetched, and the texture path then delivers about 16 bytes per clock and CU. Here a K slab of 128 elements of every
 // operand row (the TM x TT activation rows and the 16 x OCF weight rows of the tile) is fetched with adjacent lanes on
@@ -278,10 +246,10 @@ constexpr int kSlabK = 128;                       // K elements per slab = 4 mat
 
 // TM rows of the batch per workgroup: 16, or 8 where 16-row tiles would leave half of the compute units idle (a fragment
 // of 16 activation rows then holds two timesteps of the 8 rows; the tile stages half the activations per weight row).
-template <int TT, int OCF, int SLABK, int TM> struct StagedShape {
-    static_assert(TM == 8 || TM == 16, "8 or 16 batch rows per tile");
+template <int TT, int OCF, int SLABK, int TM, int PLANES> struct StagedShape {
+    static_assert(TM == 8 || TM == 16 || TM == 32, "8, 16 or 32 batch rows per tile");
     static constexpr int FRAGS = TT * TM / 16;                   // activation fragments (16 rows: TM rows of 16 / TM timesteps) per K step
-    static constexpr int TPW = FRAGS >= 8 ? 4 : 2;               // fragments per wave: its weight fragments serve all of them (LDS reads per
+    static constexpr int TPW = FRAGS >= 8 ? 4 : (FRAGS >= 2 ? 2 : 1);   // fragments per wave: its weight fragments serve all of them (LDS reads per
                                                                  // matrix instruction fall with the size of a wave's register tile)
     static constexpr int TG = FRAGS / TPW;                       // wave groups along time
     static constexpr int KSPLIT = kStagedWaves / TG;             // waves sharing the K steps of a slab
@@ -291,23 +259,26 @@ template <int TT, int OCF, int SLABK, int TM> struct StagedShape {
     static constexpr int ITEMS = (ROWS * (SLABK / 8) + kStagedWaves * 64 - 1) / (kStagedWaves * 64);   // octets per thread
     static constexpr int RING = ITEMS <= 3 ? 4 : 2;              // slabs in flight per thread (even; ITEMS x 4 registers each, 8 for fp32 storage)
     static constexpr int PITCH = OCF * kTileOC + 4;              // floats per row of an accumulator tile in LDS
-    static constexpr size_t slab_bytes = static_cast<size_t>(ROWS) * PITCH_B;
+    static constexpr size_t plane_bytes = static_cast<size_t>(ROWS) * PITCH_B;
+    static constexpr size_t slab_bytes = PLANES * plane_bytes;   // fp32 tensors: the high terms of all rows, then the low ones
     static constexpr size_t acc_bytes = static_cast<size_t>(KSPLIT) * TT * TM * PITCH * sizeof(float);
     static constexpr size_t lds_bytes = slab_bytes > acc_bytes ? slab_bytes : acc_bytes;
 };
 
+// SPECIAL: K that ends inside an octet, or that fits the ring of slabs (a variant of its own: with the branches for both the loop took 4 % longer, 8 x 64, 2048 -> 1024
+// 11.4 -> 12.0 us).
 // XBITS: the activation rows are rows of bits (byte b of a row = features 8 b ... 8 b + 7, bit j = feature 8 b + j; the row
 // stride is in bytes), expanded to 0 / 1 operands where a slab is parked. SBITS: the spikes leave as bits in the same form
 // ([T][M][Fout / 8] bytes, the step stride in bytes) instead of elements. Both are the internal layouts of a network executor
 // (a convolution on a plane of a few pixels is this matrix product, see snnf_linear_lif_bits).
-template <typename XT, typename VT, int TT, int OCF, bool DB, int SLABK, int TM, bool XBITS = false, bool SBITS = false>
+template <typename XT, typename VT, int TT, int OCF, bool DB, int SLABK, int TM, bool SPECIAL, bool XBITS = false, bool SBITS = false>
 __global__ __launch_bounds__(kStagedWaves * 64) void linear_lif_staged_kernel(StepPtrs xs, LinGeom g, const XT* __restrict__ W,
                                                                               const XT* __restrict__ bias,
                                                                               const VT* __restrict__ v_start, XT* __restrict__ spikes,
                                                                               VT* __restrict__ v_store, LifParams lif,
                                                                               float* __restrict__ ws_partial, int* __restrict__ ws_count,
                                                                               int slabs_per_part) {
-    using SH = StagedShape<TT, OCF, SLABK, TM>;
+    using SH = StagedShape<TT, OCF, SLABK, TM, sizeof(XT) == 4 ? 2 : 1>;
     constexpr int kSlabOctets = SLABK / 8;            // 16-byte staging items per operand row
     constexpr int kSlabPitch = SH::PITCH_B;
     constexpr int NT = kStagedWaves * 64;
@@ -341,7 +312,6 @@ __global__ __launch_bounds__(kStagedWaves * 64) void linear_lif_staged_kernel(St
     const XT* item_row[SH::ITEMS];
     uint32_t item_dst[SH::ITEMS];
     bool item_live[SH::ITEMS];
-    bool item_is_w[SH::ITEMS];
 #pragma unroll
     for (int j = 0; j < SH::ITEMS; ++j) {
         const int row = tid / kSlabOctets + j * (NT / kSlabOctets);
@@ -351,8 +321,12 @@ __global__ __launch_bounds__(kStagedWaves * 64) void linear_lif_staged_kernel(St
         if (r < TT * TM) {
             const int t = r / TM;
             const void* base = xs.p[0];
+            if (g.x_even) {      // (a packed tensor's steps: one product instead of a select per step)
+                base = static_cast<const unsigned char*>(base) + min(t, g.T - 1) * g.x_step_stride;
+            } else {
 #pragma unroll
-            for (int u = 1; u < TT; ++u) base = t == u ? xs.p[u] : base;
+                for (int u = 1; u < TT; ++u) base = t == u ? xs.p[u] : base;
+            }
             if constexpr (XBITS)       // a byte pointer kept in the array of element pointers
                 ptr = reinterpret_cast<const XT*>(static_cast<const unsigned char*>(base) + static_cast<int64_t>(min(m0 + r % TM, g.M - 1)) * g.x_row_stride);
             else
@@ -361,7 +335,6 @@ __global__ __launch_bounds__(kStagedWaves * 64) void linear_lif_staged_kernel(St
             ptr = W + static_cast<int64_t>(min(oc0 + r - TT * TM, g.Fout - 1)) * g.Fin;
         }
         item_row[j] = ptr;
-        item_is_w[j] = r >= TT * TM;
         item_dst[j] = static_cast<uint32_t>(r * kSlabPitch + octet * 16);
     }
 
@@ -381,24 +354,16 @@ __global__ __launch_bounds__(kStagedWaves * 64) void linear_lif_staged_kernel(St
     // slab s + 1 cannot overtake the reads of slab s - 1, which every wave finished before the barrier of slab s).
     constexpr int RING = SH::RING;
     RawOctet<XT> pre[RING][SH::ITEMS];
-    bool pre_inside[RING];
-    int pre_part[RING];       // fp32 tensors: the K part a slab belongs to (see LinGeom)
-    // K split over workgroups: workgroup z of a tile takes slabs [z * slabs_per_part, ...) (all of them without a split). The
-    // slabs of an fp32 tensor's three K parts follow each other: slab s is slab s % unit of part s / unit.
+    int pre_left[RING];       // elements of the octet that lie inside K (0 or below: none); where K holds whole octets, whether it does
+    // K split over workgroups: workgroup z of a tile takes slabs [z * slabs_per_part, ...) (all of them without a split).
     const int slab0 = static_cast<int>(blockIdx.z) * slabs_per_part;
-    const int unit = (g.Fin + SLABK - 1) / SLABK;                        // slabs of one pass over K
-    const int slab_end = min(g.kparts * unit, slab0 + slabs_per_part);   // this workgroup's slabs end here: beyond it, zeros
+    const int slab_end = min((g.Fin + SLABK - 1) / SLABK, slab0 + slabs_per_part);   // this workgroup's slabs end here: beyond it, zeros
     const int rounds = (slabs_per_part + RING - 1) / RING;
     auto fetch = [&](int slab, int r) __attribute__((always_inline)) {
-        int part = 0, real = slab;
-        if constexpr (sizeof(XT) == 4) {
-            part = slab >= 2 * unit ? 2 : (slab >= unit ? 1 : 0);
-            real = slab - part * unit;
-        }
-        pre_part[r] = part;
-        const int k = real * SLABK + octet * 8;
-        pre_inside[r] = slab < slab_end && k < g.Fin;
-        const int ks = pre_inside[r] ? k : 0;
+        const int k = slab * SLABK + octet * 8;
+        if constexpr (SPECIAL) pre_left[r] = slab < slab_end ? g.Fin - k : 0;
+        else pre_left[r] = slab < slab_end && k < g.Fin ? 1 : 0;
+        const int ks = pre_left[r] > 0 ? (SPECIAL ? min(k, g.Fin - 8) : k) : 0;      // (Fin >= 8: the host)
 #pragma unroll
         for (int j = 0; j < SH::ITEMS; ++j) {
             if (XBITS && j * kRowsPerPass < TT * TM)       // one byte = the octet's eight features
@@ -409,10 +374,18 @@ __global__ __launch_bounds__(kStagedWaves * 64) void linear_lif_staged_kernel(St
     };
     // Fragment addresses in the slab: lane = 16 q + r reads K elements 8 q .. 8 q + 7 of row r of its fragment.
     const uint32_t frag_off = static_cast<uint32_t>((lane & 15) * kSlabPitch + (lane >> 4) * 16);
+    // A part of K that fits the ring is fetched at once and walked without further loads (rounded up to the ring, 1 x 256, 256 -> 256 takes 5.0 us instead of 3.8).
+    const bool short_k = SPECIAL && slab_end - slab0 < RING;
+    if (!short_k) {
 #pragma unroll
-    for (int r = 0; r < RING; ++r) {
-        fetch(slab0 + r, r);
-        __builtin_amdgcn_sched_barrier(0);      // oldest slab first, as in the loop: its wait then leaves the others in flight
+        for (int r = 0; r < RING; ++r) {
+            fetch(slab0 + r, r);
+            __builtin_amdgcn_sched_barrier(0);      // oldest slab first, as in the loop: its wait then leaves the others in flight
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < RING - 1; ++r)
+            if (slab0 + r < slab_end) fetch(slab0 + r, r);
     }
     // A slab parked in LDS from the ring, and this wave's K steps of a parked slab (every KSPLIT-th), four at a time: their
     // operand reads go out together.
@@ -420,35 +393,61 @@ __global__ __launch_bounds__(kStagedWaves * 64) void linear_lif_staged_kernel(St
 #pragma unroll
         for (int j = 0; j < SH::ITEMS; ++j)
             if (item_live[j]) {
-                if (XBITS && j * kRowsPerPass < TT * TM)
-                    *reinterpret_cast<u32x4*>(buf + item_dst[j]) = expand_bit_octet<XT>(pre[r][j].lo[0], pre_inside[r]);
-                else
-                    *reinterpret_cast<u32x4*>(buf + item_dst[j]) = finish_octet<XT>(pre[r][j], pre_inside[r], pre_part[r] == (item_is_w[j] ? 1 : 2));
+                if (XBITS && j * kRowsPerPass < TT * TM) {
+                    *reinterpret_cast<u32x4*>(buf + item_dst[j]) = expand_bit_octet<XT>(pre[r][j].lo[0], pre_left[r] > 0);
+                } else {
+                    if constexpr (SPECIAL) {      // K may end inside an octet
+                        if (pre_left[r] < 8) drop_elements(pre[r][j], 8 - max(pre_left[r], 1));
+                    }
+                    if constexpr (sizeof(XT) == 4) {
+                        u32x4 hi, lo;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const u32x4& from = i < 2 ? pre[r][j].lo : pre[r][j].hi;
+                            uint32_t high, low;
+                            split_bf16_pair(__uint_as_float(from[2 * (i & 1)]), __uint_as_float(from[2 * (i & 1) + 1]), high, low);
+                            hi[i] = high;
+                            lo[i] = low;
+                        }
+                        *reinterpret_cast<u32x4*>(buf + item_dst[j]) = keep_octet(hi, pre_left[r] > 0);
+                        *reinterpret_cast<u32x4*>(buf + SH::plane_bytes + item_dst[j]) = keep_octet(lo, pre_left[r] > 0);
+                    } else {
+                        *reinterpret_cast<u32x4*>(buf + item_dst[j]) = keep_octet(pre[r][j].lo, pre_left[r] > 0);
+                    }
+                }
             }
     };
     auto multiply = [&](const unsigned char* buf) __attribute__((always_inline)) {
         constexpr int OWN = SLABK / 32 / SH::KSPLIT;
+        constexpr int P = sizeof(XT) == 4 ? 2 : 1;
+        constexpr int TOGETHER = P == 1 ? 4 : (SH::ITEMS > 5 ? 1 : 2);      // (registers)
         const unsigned char* own = buf + frag_off + (kp % SH::KSPLIT) * 64;
 #pragma unroll
-        for (int i0 = 0; i0 < OWN; i0 += 4) {
-            u32x4 a[4][OCF], b[4][SH::TPW];
+        for (int i0 = 0; i0 < OWN; i0 += TOGETHER) {
+            u32x4 a[TOGETHER][P][OCF], b[TOGETHER][P][SH::TPW];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
+            for (int i = 0; i < TOGETHER; ++i) {
                 if (i0 + i < OWN) {
                     const int off = (i0 + i) * SH::KSPLIT * 64;
 #pragma unroll
-                    for (int f = 0; f < OCF; ++f) a[i][f] = *reinterpret_cast<const u32x4*>(own + (TT * TM + f * kTileOC) * kSlabPitch + off);
+                    for (int p = 0; p < P; ++p) {
 #pragma unroll
-                    for (int u = 0; u < SH::TPW; ++u) b[i][u] = *reinterpret_cast<const u32x4*>(own + (tg * SH::TPW + u) * 16 * kSlabPitch + off);
+                        for (int f = 0; f < OCF; ++f) a[i][p][f] = *reinterpret_cast<const u32x4*>(own + p * SH::plane_bytes + (TT * TM + f * kTileOC) * kSlabPitch + off);
+#pragma unroll
+                        for (int u = 0; u < SH::TPW; ++u) b[i][p][u] = *reinterpret_cast<const u32x4*>(own + p * SH::plane_bytes + (tg * SH::TPW + u) * 16 * kSlabPitch + off);
+                    }
                 }
             }
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
+            for (int i = 0; i < TOGETHER; ++i) {
                 if (i0 + i < OWN) {
+                    // fp32 tensors: w_hi x_hi, w_lo x_hi, w_hi x_lo (see LinGeom)
 #pragma unroll
-                    for (int u = 0; u < SH::TPW; ++u)
+                    for (int term = 0; term < (P == 2 ? 3 : 1); ++term)
 #pragma unroll
-                        for (int f = 0; f < OCF; ++f) acc[f][u] = mfma16<XT>(a[i][f], b[i][u], acc[f][u]);
+                        for (int u = 0; u < SH::TPW; ++u)
+#pragma unroll
+                            for (int f = 0; f < OCF; ++f) acc[f][u] = mfma16<XT>(a[i][term == 1 ? 1 : 0][f], b[i][term == 2 ? 1 : 0][u], acc[f][u]);
                 }
             }
         }
@@ -456,7 +455,18 @@ __global__ __launch_bounds__(kStagedWaves * 64) void linear_lif_staged_kernel(St
     // Parking slab s + 1 (in the other buffer) ahead of the multiplication of slab s, so that a slab's barrier does not wait
     // for its writes, measured slower (64 rows x 8 timesteps 2048 -> 1024: 10.0 -> 10.4 us, 16 rows 25088 -> 4096: 63 -> 76):
     // the wait for the loads of s + 1 then stands before the work on s.
-    for (int round = 0; round < rounds; ++round) {
+    if (short_k) {
+#pragma unroll
+        for (int r = 0; r < RING - 1; ++r) {
+            if (slab0 + r < slab_end) {
+                unsigned char* buf = staged_lds + (DB ? (r & 1) * SH::slab_bytes : 0);
+                park(r, buf);
+                __syncthreads();
+                multiply(buf);
+                if (!DB) __syncthreads();
+            }
+        }
+    } else for (int round = 0; round < rounds; ++round) {
 #pragma unroll
         for (int r = 0; r < RING; ++r) {
             const int slab = slab0 + round * RING + r;
@@ -558,19 +568,24 @@ struct LinWorkspace {
 constexpr size_t kLinCounterBytes = 64 * 1024;     // 16384 tiles
 constexpr int kLinLongK = 96;                      // K slabs from which two K parts of 16-row tiles beat 8-row tiles (see linear_half_row_tiles)
 
-template <typename XT, typename VT, int TT, int OCF, bool DB, int SLABK, int TM, bool XBITS = false, bool SBITS = false>
-int launch_staged_db(dim3 grid, int slabs_per_part, const LinWorkspace& ws, const StepPtrs& xs, const LinGeom& g, const void* W, const void* bias,
+template <typename XT, typename VT, int TT, int OCF, bool DB, int SLABK, int TM, bool SPECIAL, bool XBITS = false, bool SBITS = false>
+int launch_staged_form(dim3 grid, int slabs_per_part, const LinWorkspace& ws, const StepPtrs& xs, const LinGeom& g, const void* W, const void* bias,
                      const void* v_init, void* spikes, void* v_out, const LifParams& lif, hipStream_t stream) {
-    using SH = StagedShape<TT, OCF, SLABK, TM>;
+    using SH = StagedShape<TT, OCF, SLABK, TM, sizeof(XT) == 4 ? 2 : 1>;
     constexpr size_t lds = DB ? 2 * SH::slab_bytes : SH::lds_bytes;
     static_assert(lds <= 160 * 1024 && SH::acc_bytes <= lds, "slabs exceed LDS");
-    auto kernel = linear_lif_staged_kernel<XT, VT, TT, OCF, DB, SLABK, TM, XBITS, SBITS>;
+    auto kernel = linear_lif_staged_kernel<XT, VT, TT, OCF, DB, SLABK, TM, SPECIAL, XBITS, SBITS>;
     if (lds > 64 * 1024) {
         static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
         if (raised != hipSuccess) return fail(SNNF_ERR_LAUNCH, "snnf_linear_lif: cannot reserve %zu bytes of LDS", lds);
     }
     LinGeom placed = g;
+    const auto at = [&](int t) { return static_cast<const char*>(xs.p[t]); };
+    placed.x_step_stride = g.T > 1 ? at(1) - at(0) : 0;
+    placed.x_even = 1;
+    for (int t = 2; t < g.T; ++t)
+        if (at(t) - at(t - 1) != placed.x_step_stride) placed.x_even = 0;
     placed.v_in_place = v_init != nullptr && v_init == v_out ? 1 : 0;
     kernel<<<grid, kStagedWaves * 64, lds, stream>>>(xs, placed, static_cast<const XT*>(W), static_cast<const XT*>(bias),
                                                      placed.v_in_place ? nullptr : static_cast<const VT*>(v_init), static_cast<XT*>(spikes),
@@ -578,6 +593,16 @@ int launch_staged_db(dim3 grid, int slabs_per_part, const LinWorkspace& ws, cons
                                                      reinterpret_cast<float*>(static_cast<char*>(ws.base) + kLinCounterBytes),
                                                      static_cast<int*>(ws.base), slabs_per_part);
     return check_launch("snnf_linear_lif");
+}
+
+template <typename XT, typename VT, int TT, int OCF, bool DB, int SLABK, int TM, bool XBITS, bool SBITS>
+int launch_staged_db(dim3 grid, int slabs_per_part, const LinWorkspace& ws, const StepPtrs& xs, const LinGeom& g, const void* W, const void* bias,
+                     const void* v_init, void* spikes, void* v_out, const LifParams& lif, hipStream_t stream) {
+    if constexpr (!XBITS && !SBITS) {
+        if ((g.Fin & 7) != 0 || slabs_per_part < StagedShape<TT, OCF, SLABK, TM, sizeof(XT) == 4 ? 2 : 1>::RING)
+            return launch_staged_form<XT, VT, TT, OCF, DB, SLABK, TM, true>(grid, slabs_per_part, ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
+    }
+    return launch_staged_form<XT, VT, TT, OCF, DB, SLABK, TM, false, XBITS, SBITS>(grid, slabs_per_part, ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
 }
 
 // Parts the K dimension of a tile is split into: two, for a layer with a long K whose tiles leave half of the compute
@@ -595,12 +620,12 @@ int launch_staged(const LinWorkspace& ws, const StepPtrs& xs, const LinGeom& g, 
                   void* v_out, const LifParams& lif, hipStream_t stream) {
     dim3 grid((g.Fout + OCF * kTileOC - 1) / (OCF * kTileOC), (g.M + TM - 1) / TM);
     if (grid.y > 65535) return fail(SNNF_ERR_UNSUPPORTED, "snnf_linear_lif: M=%d too large", g.M);
-    const int unit_slabs = g.kparts * ((g.Fin + SLABK - 1) / SLABK);          // all K parts of an fp32 tensor
+    const int unit_slabs = (g.Fin + SLABK - 1) / SLABK;
     const int64_t tiles = static_cast<int64_t>(grid.x) * grid.y;
     const size_t part_bytes = static_cast<size_t>(TT) * OCF * kTileOC * TM * sizeof(float);
     int parts = ws.base != nullptr ? linear_split_parts(tiles, unit_slabs * (SLABK / kSlabK), part_bytes, ws.bytes) : 1;
     const int unit_slabs_per_part = (unit_slabs + parts - 1) / parts;
-    using SH = StagedShape<TT, OCF, SLABK, TM>;
+    using SH = StagedShape<TT, OCF, SLABK, TM, sizeof(XT) == 4 ? 2 : 1>;
     parts = (unit_slabs + unit_slabs_per_part - 1) / unit_slabs_per_part;      // no empty part
     grid.z = parts;
     // Two slab buffers where a CU gets one workgroup anyway (they would cost occupancy otherwise) and both fit LDS.
@@ -623,7 +648,7 @@ inline bool linear_half_row_tiles(const LinWorkspace& ws, const LinGeom& g) {
     if (g.M <= 8) return true;
     const int64_t oc_tiles = g.Fout % (2 * kTileOC) == 0 ? g.Fout / (2 * kTileOC) : (g.Fout + kTileOC - 1) / kTileOC;
     if (oc_tiles * ((g.M + kTileM - 1) / kTileM) * 2 > compute_units()) return false;
-    const int unit_slabs = g.kparts * ((g.Fin + kSlabK - 1) / kSlabK);
+    const int unit_slabs = (g.Fin + kSlabK - 1) / kSlabK;
     if (ws.base == nullptr || unit_slabs < 32) return true;                  // K is not split either way
     if (oc_tiles * ((g.M + 7) / 8) * 2 <= compute_units()) return true;      // tiles of 8 rows split K as well
     // 16-row tiles in two K parts or 8-row tiles unsplit: up to 4 timesteps the split wins (16 rows 4096 -> 4096: 13.6
@@ -639,33 +664,46 @@ int launch_staged_tt(const LinWorkspace& ws, const StepPtrs& xs, const LinGeom& 
     // 16 rows, 2048 -> 1024: 8.9 -> 7.9 us; 8 rows 25088 -> 1000: 39.5 -> 33.6); wide tiles are slower that way (64 rows
     // 2048 -> 1024: 10.1 -> 11.0 us).
     constexpr int kWide = (TM == 8 && OCF == 1) ? 2 * kSlabK : kSlabK;
+    if constexpr (OCF == 1 && TM == kTileM) {
+        if (g.T == 1) return g.M <= kTileM ? launch_staged<XT, VT, 1, 1, kTileM, 2 * kSlabK>(ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream)
+                                           : launch_staged<XT, VT, 1, 1, 2 * kTileM, 2 * kSlabK>(ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
+        if (g.T == 2) return launch_staged<XT, VT, 2, 1, kTileM, 2 * kSlabK>(ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
+    }
     if (g.T <= 4) return launch_staged<XT, VT, 4, OCF, TM, TM == 8 ? 2 * kSlabK : kSlabK>(ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
     if (g.T <= 8) return launch_staged<XT, VT, 8, OCF, TM, kWide>(ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
     return launch_staged<XT, VT, 16, OCF, TM, kWide>(ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
 }
 
-template <typename XT, typename VT, bool FAST>
-int launch_tt(const LinWorkspace& ws, const StepPtrs& xs, const LinGeom& g, const void* W, const void* bias, const void* v_init, void* spikes,
+// Which kernel runs a layer (us; `aligned`: rows of whole octets at 16-byte addresses):
+// * The staged kernel takes rows that start and end anywhere, and any number of timesteps: its loads are of 16 bytes at any element's address, and the octet in which
+//   a row ends is fetched from the row's last eight elements and shifted. Elementwise loads of such rows took 46 us at 4 x 64, 2047 -> 1024 (here 11.0), 94 at 5 x 206,
+//   555 -> 858 in fp16 (24), 1206 at 8 x 16, 25085 -> 4096 (116). fp32 rows are fetched and split once for the three products, not once for each: 8 x 64, 2048 -> 1024
+//   48 -> 21, 1 x 5, 3001 -> 77 71 -> 10, 6 x 120, 2640 -> 96 55 -> 26.
+// * One or two timesteps of 16-bit rows: against fragments straight from memory (aligned rows) it gains from K = 1024 on (1 x 64, 2048 -> 1024 6.6 / 6.0, x 2 8.9 / 6.9, 1 x 256, 1024 -> 4096 33 / 21,
+//   2 x 16, 25088 -> 1000 67 / 33) and loses below (1 x 100, 200 -> 3000 5.1 / 8.0, 2 x 200, 512 -> 512 5.8 / 6.4, 2 x 128, 768 -> 3072 16.6 / 19.0), and up to 4096 where few tiles
+//   leave the loads of each workgroup alone (2 x 3, 2400 -> 64 5.6 / 6.8; one step up to 2048, 1 x 32, 1536 -> 512 5.4 / 5.7). In fp32 it gains everywhere (1 x 32, 512 -> 10 7.3 / 4.5).
+template <typename XT, typename VT>
+int launch_tt(bool aligned, const LinWorkspace& ws, const StepPtrs& xs, const LinGeom& g, const void* W, const void* bias, const void* v_init, void* spikes,
               void* v_out, const LifParams& lif, hipStream_t stream) {
-    if constexpr (FAST) {
-        if (g.T > 2) {
-            // Two feature fragments per workgroup (half the activation traffic) when that still leaves at least 128 workgroups.
-            const bool half_rows = linear_half_row_tiles(ws, g);
-            const int tm = half_rows ? 8 : kTileM;
-            const bool wide = g.Fout % (2 * kTileOC) == 0 && static_cast<int64_t>(g.Fout / (2 * kTileOC)) * ((g.M + tm - 1) / tm) >= 128;
-            if (half_rows) {
-                if (wide) return launch_staged_tt<XT, VT, 2, 8>(ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
-                return launch_staged_tt<XT, VT, 1, 8>(ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
-            }
-            if (wide) return launch_staged_tt<XT, VT, 2, kTileM>(ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
-            return launch_staged_tt<XT, VT, 1, kTileM>(ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
+    if (g.Fin >= 8) {
+        if constexpr (sizeof(XT) == 2) {
+            const int64_t tiles = static_cast<int64_t>((g.Fout + kTileOC - 1) / kTileOC) * ((g.M + kTileM - 1) / kTileM);
+            if (aligned && g.T <= 2 && (g.Fin < 1024 || (g.Fin < 4096 && tiles <= 16) || (g.Fin < 2048 && g.T == 1 && tiles <= 64)))
+                return g.T == 1 ? launch_direct<XT, VT, 1>(xs, g, W, bias, v_init, spikes, v_out, lif, stream) : launch_direct<XT, VT, 2>(xs, g, W, bias, v_init, spikes, v_out, lif, stream);
         }
+        if (g.T <= 2) return launch_staged_tt<XT, VT, 1, kTileM>(ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
+        // Two feature fragments per workgroup (half the activation traffic) when that still leaves at least 128 workgroups.
+        const bool half_rows = linear_half_row_tiles(ws, g);
+        const int tm = half_rows ? 8 : kTileM;
+        const bool wide = g.Fout % (2 * kTileOC) == 0 && static_cast<int64_t>(g.Fout / (2 * kTileOC)) * ((g.M + tm - 1) / tm) >= 128;
+        if (half_rows) {
+            if (wide) return launch_staged_tt<XT, VT, 2, 8>(ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
+            return launch_staged_tt<XT, VT, 1, 8>(ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
+        }
+        if (wide) return launch_staged_tt<XT, VT, 2, kTileM>(ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
+        return launch_staged_tt<XT, VT, 1, kTileM>(ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
     }
-    if (g.T <= 1) return launch_one<XT, VT, 1, FAST, 1>(xs, g, W, bias, v_init, spikes, v_out, lif, stream);
-    if (g.T <= 2) return launch_one<XT, VT, 2, FAST, 1>(xs, g, W, bias, v_init, spikes, v_out, lif, stream);
-    if (g.T <= 4) return launch_one<XT, VT, 4, FAST, 1>(xs, g, W, bias, v_init, spikes, v_out, lif, stream);
-    if (g.T <= 8) return launch_one<XT, VT, 8, FAST, 1>(xs, g, W, bias, v_init, spikes, v_out, lif, stream);
-    return launch_one<XT, VT, 16, FAST, 1>(xs, g, W, bias, v_init, spikes, v_out, lif, stream);
+    return launch_short<XT, VT>(xs, g, W, bias, v_init, spikes, v_out, lif, stream);
 }
 
 // The internal-layout forms: spikes out as bits, activation rows as elements or as bits; wide tiles (Fout % 32 == 0), 3 to 8
@@ -679,13 +717,6 @@ int launch_bits(const LinWorkspace& ws, const StepPtrs& xs, const LinGeom& g, co
     }
     if (g.T <= 4) return launch_staged<XT, float, 4, 2, kTileM, kSlabK, XBITS, true>(ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
     return launch_staged<XT, float, 8, 2, kTileM, kSlabK, XBITS, true>(ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
-}
-
-template <typename XT, typename VT>
-int launch(bool fast, const LinWorkspace& ws, const StepPtrs& xs, const LinGeom& g, const void* W, const void* bias, const void* v_init,
-           void* spikes, void* v_out, const LifParams& lif, hipStream_t stream) {
-    return fast ? launch_tt<XT, VT, true>(ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream)
-                : launch_tt<XT, VT, false>(ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
 }
 
 }  // namespace
@@ -755,17 +786,16 @@ static int linear_lif_impl(const char* who, const void* const* xs, int T, int M,
     const LifParams lif = make_lif_params(v_threshold, v_reset, tau);
     const int xsize = dtype_size(x_dtype);
     hipStream_t hs = as_stream(stream);
-    const int per16 = 16 / xsize;
 
     for (int t0 = 0; t0 < T; t0 += SNNF_MAX_T_PER_LAUNCH) {
         const int tw = (T - t0) < SNNF_MAX_T_PER_LAUNCH ? (T - t0) : SNNF_MAX_T_PER_LAUNCH;
         int tt = 1;
         while (tt < tw) tt *= 2;
         StepPtrs ptrs = {};
-        bool fast = Fin % 8 == 0 && x_row_stride % per16 == 0 && aligned_to(weight, 16);
+        bool aligned = Fin % 8 == 0 && x_row_stride % (16 / xsize) == 0 && aligned_to(weight, 16);
         for (int t = 0; t < tt; ++t) {
             ptrs.p[t] = xs[t0 + (t < tw ? t : 0)];  // padded steps re-read step 0 and are never stored
-            fast = fast && aligned_to(ptrs.p[t], 16);
+            aligned = aligned && aligned_to(ptrs.p[t], 16);
         }
         LinGeom g;
         g.T = tw;
@@ -774,18 +804,16 @@ static int linear_lif_impl(const char* who, const void* const* xs, int T, int M,
         g.Fout = Fout;
         g.x_row_stride = x_row_stride;
         g.spike_step_stride = spike_step_stride;
-        g.ksteps = (Fin + 31) / 32;
-        g.kparts = x_dtype == SNNF_F32 ? 3 : 1;
         const void* vi = t0 == 0 ? v_init : v_out;
         void* sp = static_cast<char*>(spikes) + static_cast<int64_t>(t0) * spike_step_stride * xsize;
         int rc;
-        if (x_dtype == SNNF_F32) rc = launch<float, float>(fast, ws, ptrs, g, weight, bias, vi, sp, v_out, lif, hs);
+        if (x_dtype == SNNF_F32) rc = launch_tt<float, float>(aligned, ws, ptrs, g, weight, bias, vi, sp, v_out, lif, hs);
         else if (x_dtype == SNNF_BF16)
-            rc = v_dtype == SNNF_F32 ? launch<bf16_t, float>(fast, ws, ptrs, g, weight, bias, vi, sp, v_out, lif, hs)
-                                     : launch<bf16_t, bf16_t>(fast, ws, ptrs, g, weight, bias, vi, sp, v_out, lif, hs);
+            rc = v_dtype == SNNF_F32 ? launch_tt<bf16_t, float>(aligned, ws, ptrs, g, weight, bias, vi, sp, v_out, lif, hs)
+                                     : launch_tt<bf16_t, bf16_t>(aligned, ws, ptrs, g, weight, bias, vi, sp, v_out, lif, hs);
         else
-            rc = v_dtype == SNNF_F32 ? launch<f16_t, float>(fast, ws, ptrs, g, weight, bias, vi, sp, v_out, lif, hs)
-                                     : launch<f16_t, f16_t>(fast, ws, ptrs, g, weight, bias, vi, sp, v_out, lif, hs);
+            rc = v_dtype == SNNF_F32 ? launch_tt<f16_t, float>(aligned, ws, ptrs, g, weight, bias, vi, sp, v_out, lif, hs)
+                                     : launch_tt<f16_t, f16_t>(aligned, ws, ptrs, g, weight, bias, vi, sp, v_out, lif, hs);
         if (rc != SNNF_OK) return rc;
     }
     return SNNF_OK;
@@ -829,8 +857,6 @@ extern "C" int snnf_linear_lif_bits(const void* const* xs, int x_bits, int T, in
     g.Fout = Fout;
     g.x_row_stride = x_row_stride;
     g.spike_step_stride = spike_step_stride;
-    g.ksteps = (Fin + 31) / 32;
-    g.kparts = 1;
     const LinWorkspace ws = {workspace, workspace != nullptr ? workspace_bytes : 0};
     const LifParams lif = make_lif_params(v_threshold, v_reset, tau);
     hipStream_t hs = as_stream(stream);
