@@ -2,6 +2,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
+#include "snnf_conv_columns.h"
 #include "snnf_conv_common.h"
 
 #include <cstdlib>
@@ -478,6 +479,20 @@ int conv_lif_impl(const void* const* xs, const void* const* residuals, int T, in
     if (analog_out && !mm_kernel)
         return fail(SNNF_ERR_UNSUPPORTED, "snnf_conv_bias: unsupported_shape: only layers the 8-wave matrix kernel takes "
                     "(Cin %% 8 == 0 or Cin < 8, tiles that fit LDS)");
+    // 1x1 layers without a neuron that leave the matrix kernel (see takes_columns).
+    if (analog_out && KH == 1 && KW == 1 && pad_h == 0 && pad_w == 0 && residuals == nullptr && xsize == 2 && T <= SNNF_MAX_T_PER_LAUNCH &&
+        takes_columns(T, N, Cin, H, W, Cout, stride_h, stride_w)) {
+        ColumnsLaunch L = {};
+        for (int t = 0; t < T; ++t) L.xs.p[t] = xs[t];
+        L.T = T;
+        L.g.out_step_stride = spike_step_stride;
+        L.wpacked = static_cast<const uint16_t*>(packed_weight);
+        L.bias = reinterpret_cast<const float*>(L.wpacked + packed_weight_elems(pg));
+        L.out = spikes;
+        L.stream = hs;
+        snprintf(snnf::conv_plan_buffer(), 256, "kernel=matrix variant=0 window=%d launches=1 ran=columns", T);
+        return launch_conv_columns(L, N, Cin, H, W, Cout, stride_h, stride_w, pg, x_dtype == SNNF_F16);
+    }
     // Pointwise kernel: where the weight fragments live (registers only in the fast variant) and the LDS that takes.
     auto pw_config = [&](bool allow_regs, ConvGeom& gg) -> size_t {
         const size_t xb = static_cast<size_t>(64) * gg.pitch;
