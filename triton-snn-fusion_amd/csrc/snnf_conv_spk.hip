@@ -360,7 +360,14 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
     // at 24^2, one image, 18 and 36 workgroups 8.5 / 7.5). Fuller rounds stay even: 256 -> 256 at 14^2 x 128, 224 workgroups 100 us, 256 105.
     // Narrow tiles of one wave: two tiles of a patch side by side, which read the same activations.
     const int spread = g.narrow && !c.split && wk_log2 == 0 ? g.n_patches * ((Cout + 63) / 64) : g.n_items;
-    if (g.iters > 1 ? grid * 4 < resident * 3 : grid * 2 <= cus) grid = std::min(spread, g.iters > 1 ? resident : cus);
+    // The same where the last of three or more rounds is at most half full (of one timestep, whose workgroups run two to a unit, seven tenths of any round): every
+    // unit, and a few waves with a tile more, against fewer units with full rounds. us, full rounds / every unit, by the rounds that all units would take, 64 -> 64 at 56^2: 2.49 (52 images)
+    // 45.2 / 41.7, 3.45 56.8 / 53.8, 5.36 83.8 / 81.2, 6.13 (128) 111 / 105; 128 -> 128 at 28^2: 2.30 72.7 / 70.3, 3.50 98.2 / 94.8; 64 -> 128 stride 2 3.06 81.1 / 76.3; stem at 224^2: 1.53
+    // (16 images) 32.5 / 31.7, 2.30 42.8 / 38.9, 3.06 55.3 / 51.6, 12.25 175 / 171. Fuller rounds gain nothing (64 -> 64 at 4.98 74.2 / 75.0, 6.89 102.2 / 102.1, stem 6.89 94.1 / 95.4), and of two
+    // rounds the second one takes as long for a single tile of a SIMD as for two (256 -> 256 at 14^2, 1.53 90.3 / 95.1, 64 -> 64 at 56^2 x 32 30.8 / 32.1).
+    const double rounds = static_cast<double>(g.n_items) / (static_cast<double>(resident) * tiles_per_block), over = rounds - std::floor(rounds);
+    const bool part = resident > cus ? rounds > 1.0 && over <= 0.7 : rounds > 2.0 && over <= 0.5;
+    if (g.iters > 1 ? grid * 4 < resident * 3 || part : grid * 2 <= cus) grid = std::min(spread, g.iters > 1 ? resident : cus);
     g.grid = grid;
     g.d_ppx = make_spk_div(g.PR * g.PC);
     g.d_PC = make_spk_div(g.PC);
