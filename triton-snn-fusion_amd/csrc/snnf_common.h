@@ -207,6 +207,22 @@ __device__ __forceinline__ bool lif_step(float x, float& v, const LifParams& p) 
     return fired;
 }
 
+// The usual neuron: a power-of-two tau and a hard reset. Kernels that unroll many steps take it on a path of its own (`lif_step` is a chain of
+// uniform branches with a division in it, some 40 instructions a step that a wave fetches even where it does not run them).
+__host__ __device__ __forceinline__ bool usual_neuron(const LifParams& p) { return p.charge_mode == CHARGE_SCALE && !p.soft_reset; }
+
+template <bool USUAL>
+__device__ __forceinline__ bool lif_step_as(float x, float& v, const LifParams& p) {
+    if constexpr (!USUAL) {
+        return lif_step(x, v, p);
+    } else {
+        const float h = v + (x - v) * p.inv_tau;
+        const bool fired = h >= p.v_threshold;
+        v = fired ? p.v_reset : h;
+        return fired;
+    }
+}
+
 // Up to SNNF_MAX_T_PER_LAUNCH per-timestep base pointers, passed to kernels by value.
 struct StepPtrs {
     const void* p[SNNF_MAX_T_PER_LAUNCH];

@@ -1,15 +1,21 @@
 // Temporal LIF scan: streams x[t] once, keeps the membrane in registers for all T steps, writes dense 0/1 spikes
 // once and the final membrane once. Bound by HBM bandwidth: (2*T + 1) * numel elements of traffic, ~6 flops each.
+#include <type_traits>
+
 #include "snnf_common.h"
 
 namespace snnf {
 namespace {
 
 constexpr int kThreads = 256;
+// Timesteps in flight where their number is no constant: four of them, or (TC < 0) each stored before the next is loaded, which fp32 tensors that stream from memory prefer: they have
+// enough waves to overlap (2 M neurons, T = 3 10.1 us, four in flight 10.8; T = 16 51.4 / 53.0; but 200 k neurons, T = 16 12.6 -> 5.8, bf16 13.4 -> 6.1, 2 M neurons in bf16 30.0 -> 25.0).
+constexpr int kInFlight = 4;
+constexpr int64_t kStreamNeurons = 1 << 20;
 
 // One thread owns VEC consecutive neurons; every load/store of a thread is one 16-byte (or narrower, VEC == 1)
 // transaction, so a 64-lane wave moves 1 KiB per instruction.
-template <typename XT, typename VT, int VEC, int TC>
+template <typename XT, typename VT, int VEC, int TC, bool USUAL>
 __global__ __launch_bounds__(kThreads) void lif_scan_kernel(StepPtrs xs, int T, int64_t numel,
                                                             const VT* v_init, XT* __restrict__ spikes,
                                                             int64_t spike_step_stride, VT* v_out,
@@ -29,7 +35,6 @@ __global__ __launch_bounds__(kThreads) void lif_scan_kernel(StepPtrs xs, int T, 
         for (int i = 0; i < VEC; ++i) v[i] = 0.0f;
     }
 
-    const int steps = TC > 0 ? TC : T;
     if constexpr (TC > 0) {
         // Issue every timestep's load before the recurrence so that T independent 16-byte loads are in flight.
         XV xin[TC];
@@ -39,16 +44,25 @@ __global__ __launch_bounds__(kThreads) void lif_scan_kernel(StepPtrs xs, int T, 
         for (int t = 0; t < TC; ++t) {
             XV out;
 #pragma unroll
-            for (int i = 0; i < VEC; ++i) out.v[i] = spike_value<XT>(lif_step(to_float(xin[t].v[i]), v[i], lif));
+            for (int i = 0; i < VEC; ++i) out.v[i] = spike_value<XT>(lif_step_as<USUAL>(to_float(xin[t].v[i]), v[i], lif));
             *reinterpret_cast<XV*>(spikes + t * spike_step_stride + first) = out;
         }
     } else {
-        for (int t = 0; t < steps; ++t) {
-            const XV xin = *reinterpret_cast<const XV*>(static_cast<const XT*>(xs.p[t]) + first);
-            XV out;
+        constexpr int CHUNK = TC < 0 ? 1 : kInFlight;
+        for (int t0 = 0; t0 < T; t0 += CHUNK) {
+            XV xin[CHUNK];
 #pragma unroll
-            for (int i = 0; i < VEC; ++i) out.v[i] = spike_value<XT>(lif_step(to_float(xin.v[i]), v[i], lif));
-            *reinterpret_cast<XV*>(spikes + t * spike_step_stride + first) = out;
+            for (int u = 0; u < CHUNK; ++u)
+                if (t0 + u < T) xin[u] = *reinterpret_cast<const XV*>(static_cast<const XT*>(xs.p[t0 + u]) + first);
+#pragma unroll
+            for (int u = 0; u < CHUNK; ++u) {
+                if (t0 + u < T) {
+                    XV out;
+#pragma unroll
+                    for (int i = 0; i < VEC; ++i) out.v[i] = spike_value<XT>(lif_step_as<USUAL>(to_float(xin[u].v[i]), v[i], lif));
+                    *reinterpret_cast<XV*>(spikes + (t0 + u) * spike_step_stride + first) = out;
+                }
+            }
         }
     }
 
@@ -68,12 +82,19 @@ int launch_lif_scan(const StepPtrs& xs, int T, int64_t numel, const void* v_init
     const VT* vi = static_cast<const VT*>(v_init);
     XT* sp = static_cast<XT*>(spikes);
     VT* vo = static_cast<VT*>(v_out);
+    auto go = [&](auto steps) {
+        constexpr int TC = decltype(steps)::value;
+        if (usual_neuron(lif)) lif_scan_kernel<XT, VT, VEC, TC, true><<<grid, kThreads, 0, stream>>>(xs, T, numel, vi, sp, spike_step_stride, vo, lif);
+        else lif_scan_kernel<XT, VT, VEC, TC, false><<<grid, kThreads, 0, stream>>>(xs, T, numel, vi, sp, spike_step_stride, vo, lif);
+    };
     switch (T) {
-        case 1: lif_scan_kernel<XT, VT, VEC, 1><<<grid, kThreads, 0, stream>>>(xs, T, numel, vi, sp, spike_step_stride, vo, lif); break;
-        case 2: lif_scan_kernel<XT, VT, VEC, 2><<<grid, kThreads, 0, stream>>>(xs, T, numel, vi, sp, spike_step_stride, vo, lif); break;
-        case 4: lif_scan_kernel<XT, VT, VEC, 4><<<grid, kThreads, 0, stream>>>(xs, T, numel, vi, sp, spike_step_stride, vo, lif); break;
-        case 8: lif_scan_kernel<XT, VT, VEC, 8><<<grid, kThreads, 0, stream>>>(xs, T, numel, vi, sp, spike_step_stride, vo, lif); break;
-        default: lif_scan_kernel<XT, VT, VEC, 0><<<grid, kThreads, 0, stream>>>(xs, T, numel, vi, sp, spike_step_stride, vo, lif); break;
+        case 1: go(std::integral_constant<int, 1>{}); break;
+        case 2: go(std::integral_constant<int, 2>{}); break;
+        case 4: go(std::integral_constant<int, 4>{}); break;
+        case 8: go(std::integral_constant<int, 8>{}); break;
+        default:
+            if (sizeof(XT) == 4 && numel >= kStreamNeurons) go(std::integral_constant<int, -1>{});
+            else go(std::integral_constant<int, 0>{});
     }
     return check_launch("snnf_lif_scan");
 }

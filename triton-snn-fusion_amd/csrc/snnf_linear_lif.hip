@@ -533,29 +533,41 @@ __global__ __launch_bounds__(kStagedWaves * 64) void linear_lif_staged_kernel(St
         const int slot = (e / TILE_OC) * SH::PITCH + e % TILE_OC;
         float v = v_first;
         const float* __restrict__ all = ws_partial + static_cast<int64_t>(tile) * parts * (TT * OUTS) + e;
+        // The sums of all timesteps first, a part's together (every part holds TT of them): their loads overlap.
+        float sum[TT];
 #pragma unroll
-        for (int t = 0; t < TT; ++t) {
-            if (t < g.T) {      // a guard, not a break: a second loop exit keeps the compiler from unrolling over t
-                float sum = 0.0f;
-                if (parts > 1) {
-                    for (int z = 0; z < parts; ++z) sum += __hip_atomic_load(all + (static_cast<int64_t>(z) * TT + t) * OUTS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                } else {
+        for (int t = 0; t < TT; ++t) sum[t] = 0.0f;
+        if (parts > 1) {
+            for (int z = 0; z < parts; ++z) {
 #pragma unroll
-                    for (int w = 0; w < SH::KSPLIT; ++w) sum += partial[(w * TT + t) * SLAB_F + slot];
-                }
-                const float cur = sum + bv;
-                const bool fired = lif_step(cur, v, lif);
-                if constexpr (SBITS) {
-                    // Lane l of the wave holds feature oc0 + l % TILE_OC (a multiple of 8 apart from l % 8): byte l / 8 of the ballot.
-                    const uint64_t fired_lanes = __ballot(fired && out_live);
-                    if ((lane & 7) == 0 && out_live)
-                        reinterpret_cast<unsigned char*>(spikes)[t * g.spike_step_stride + static_cast<int64_t>(out_m) * (g.Fout >> 3) + (out_oc >> 3)] =
-                            static_cast<unsigned char>(fired_lanes >> lane);
-                } else {
-                    spikes[t * g.spike_step_stride + out_index] = spike_value<XT>(fired);
-                }
+                for (int t = 0; t < TT; ++t) sum[t] += __hip_atomic_load(all + (static_cast<int64_t>(z) * TT + t) * OUTS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        } else {
+#pragma unroll
+            for (int t = 0; t < TT; ++t) {
+#pragma unroll
+                for (int w = 0; w < SH::KSPLIT; ++w) sum[t] += partial[(w * TT + t) * SLAB_F + slot];
             }
         }
+        auto recurrence = [&](auto usual) __attribute__((always_inline)) {
+#pragma unroll
+            for (int t = 0; t < TT; ++t) {
+                if (t < g.T) {      // a guard, not a break: a second loop exit keeps the compiler from unrolling over t
+                    const bool fired = lif_step_as<decltype(usual)::value>(sum[t] + bv, v, lif);
+                    if constexpr (SBITS) {
+                        // Lane l of the wave holds feature oc0 + l % TILE_OC (a multiple of 8 apart from l % 8): byte l / 8 of the ballot.
+                        const uint64_t fired_lanes = __ballot(fired && out_live);
+                        if ((lane & 7) == 0 && out_live)
+                            reinterpret_cast<unsigned char*>(spikes)[t * g.spike_step_stride + static_cast<int64_t>(out_m) * (g.Fout >> 3) + (out_oc >> 3)] =
+                                static_cast<unsigned char>(fired_lanes >> lane);
+                    } else {
+                        spikes[t * g.spike_step_stride + out_index] = spike_value<XT>(fired);
+                    }
+                }
+            }
+        };
+        if (usual_neuron(lif)) recurrence(std::true_type{});
+        else recurrence(std::false_type{});
         if (v_store != nullptr && out_live) v_store[out_index] = from_float<VT>(v);
     }
 }

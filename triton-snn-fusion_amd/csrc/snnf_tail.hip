@@ -92,8 +92,8 @@ __global__ __launch_bounds__(kThreads) void lif_pool_vec_kernel(StepPtrs xs, int
 
     // A workgroup whose neuron count is a multiple of 8 (all but, at most, the last one) moves whole vectors only; its
     // loop body has no branch around a load, so all loads of a pass are in flight together.
-    auto pass = [&](int i0, auto whole_tag) __attribute__((always_inline)) {
-        constexpr bool whole = decltype(whole_tag)::value;
+    auto pass = [&](int i0, auto whole_tag, auto usual_tag) __attribute__((always_inline)) {
+        constexpr bool whole = decltype(whole_tag)::value, usual = decltype(usual_tag)::value;
         float v[kVec];
         int fired[kVec];
 #pragma unroll
@@ -121,7 +121,7 @@ __global__ __launch_bounds__(kThreads) void lif_pool_vec_kernel(StepPtrs xs, int
 #pragma unroll
             for (int t = 0; t < TC; ++t)
 #pragma unroll
-                for (int j = 0; j < kVec; ++j) fired[j] += lif_step(to_float(px[t].v[j]), v[j], lif) ? 1 : 0;
+                for (int j = 0; j < kVec; ++j) fired[j] += lif_step_as<usual>(to_float(px[t].v[j]), v[j], lif) ? 1 : 0;
         } else {
             for (int t0 = 0; t0 < T; t0 += 4) {
                 Pack<XT, kVec> px[4];
@@ -141,7 +141,7 @@ __global__ __launch_bounds__(kThreads) void lif_pool_vec_kernel(StepPtrs xs, int
                 for (int u = 0; u < 4; ++u) {
                     if (t0 + u < T) {
 #pragma unroll
-                        for (int j = 0; j < kVec; ++j) fired[j] += lif_step(to_float(px[u].v[j]), v[j], lif) ? 1 : 0;
+                        for (int j = 0; j < kVec; ++j) fired[j] += lif_step_as<usual>(to_float(px[u].v[j]), v[j], lif) ? 1 : 0;
                     }
                 }
             }
@@ -189,11 +189,12 @@ __global__ __launch_bounds__(kThreads) void lif_pool_vec_kernel(StepPtrs xs, int
             if (run != 0) atomicAdd(&plane_count[p], run);
         }
     };
-    if (elems % kVec == 0) {
-        for (int i0 = threadIdx.x * kVec; i0 < elems; i0 += kThreads * kVec) pass(i0, std::true_type{});
-    } else {
-        for (int i0 = threadIdx.x * kVec; i0 < elems; i0 += kThreads * kVec) pass(i0, std::false_type{});
-    }
+    auto passes = [&](auto whole_tag, auto usual_tag) __attribute__((always_inline)) {
+        for (int i0 = threadIdx.x * kVec; i0 < elems; i0 += kThreads * kVec) pass(i0, whole_tag, usual_tag);
+    };
+    if (elems % kVec != 0) passes(std::false_type{}, std::false_type{});
+    else if (usual_neuron(lif)) passes(std::true_type{}, std::true_type{});
+    else passes(std::true_type{}, std::false_type{});
     __syncthreads();
     for (int i = threadIdx.x; i < planes_here; i += kThreads) counts[plane0 + i] = plane_count[i];
 }
@@ -375,28 +376,29 @@ __global__ __launch_bounds__(kThreads) void count_linear_mm_kernel(const int* __
 }
 
 // The whole tail in one launch, for tails as small as those at the end of a network: a workgroup owns one sample and a range
-// of classes. It runs the sample's LIF recurrence (a thread owns 8 consecutive neurons per pass, 16-byte loads, four timesteps
-// in flight), counts the spikes per channel in LDS and multiplies its classes' weight rows with the counts right away: no
+// of classes. It runs the sample's LIF recurrence (a thread owns 8 consecutive neurons, 16-byte loads, all timesteps of T <= 4
+// and eight of more in flight), counts the spikes per channel in LDS and multiplies its classes' weight rows with the counts right away: no
 // counts in memory, no second launch. The workgroups of a sample that differ in their class range repeat the recurrence (the
 // sample's activations come from L2 then); the first of them writes the membrane. The products run like
 // count_linear_vec_kernel's (a wave owns kRowsPerWave rows, a lane 8 consecutive channels per trip, shuffle reduction), so the
 // two paths give the same sums bit for bit.
+// Such a launch is one chain of latencies: launch, loads, recurrence, counters, weights. A workgroup has 256, 512 or 1024 threads, so that one pass takes all neurons (passes of 256
+// threads follow each other: 512 channels of 3x3, 16 samples, T = 4 14.1 us -> 5.7, 4x4 18.5 -> 5.9), and the usual neuron runs without lif_step's branches (1x1 6.3 -> 5.0).
 constexpr int kOneMaxC = 2048;                    // channels of a sample whose counters fit the workgroup's LDS array
-constexpr int64_t kOneMaxSampleWork = 32 * 1024;  // T * C * HW of one sample, at most: 128 LIF steps per thread. Larger samples are better spread
-// over many workgroups by the pooling kernel of the two-launch path, and so are the larger ones of these (us, one launch / two, bf16, T = 4, 512 channels x 16 samples: 1x1
-// 10 classes 5.9 / 7.7, 2x2 6.1 / 7.6, 2x2 1000 classes 7.9 / 8.6, 3x3 14.1 / 8.8, 4x4 18.5 / 8.7, and without this limit 7x7 48.7 / 9.1): the passes of a workgroup follow each
-// other, and every class range repeats them.
+constexpr int kOneMaxNeurons = 1024 * kVec;       // of a sample: one pass
+constexpr int64_t kOneMaxSampleWork = 32 * 1024;  // T * C * HW of one sample, at most: the pooling kernel of the two-launch path spreads more over many workgroups
+                                                  // (512 channels of 4x4 x 16, T = 8, 100 classes, one launch / two 8.3 / 8.2 us, 1000 classes 10.6 / 8.3)
 
 // out[n, k] = (Wt[k, :] . counts / HW + steps * bias[k]) * out_scale for the classes of this workgroup's range, from the
 // per-channel spike counts of sample n in LDS: kRowsPerWave rows per wave and pass, a lane takes 8 channels at a time.
-template <typename XT>
+template <typename XT, int THREADS>
 __device__ __forceinline__ void classify_counts(const int* plane_count, int n, int C, int K, int classes_per_block, const XT* __restrict__ Wt,
                                                 const XT* __restrict__ bias, XT* __restrict__ out, float inv_hw, float steps, float out_scale) {
     const int wave = threadIdx.x >> 6;
     const int lane = threadIdx.x & 63;
     const int k_begin = blockIdx.x * classes_per_block;
     const int k_end = min(K, k_begin + classes_per_block);
-    for (int k0 = k_begin + wave * kRowsPerWave; k0 < k_end; k0 += (kThreads / 64) * kRowsPerWave) {
+    for (int k0 = k_begin + wave * kRowsPerWave; k0 < k_end; k0 += (THREADS / 64) * kRowsPerWave) {
         float acc[kRowsPerWave];
 #pragma unroll
         for (int r = 0; r < kRowsPerWave; ++r) acc[r] = 0.0f;
@@ -431,8 +433,8 @@ __device__ __forceinline__ void classify_counts(const int* plane_count, int n, i
     }
 }
 
-template <typename XT, typename VT>
-__global__ __launch_bounds__(kThreads) void lif_pool_linear_one_kernel(StepPtrs xs, int T, int C, int HW, int K, int classes_per_block,
+template <typename XT, typename VT, int THREADS, int TC>
+__global__ __launch_bounds__(THREADS) void lif_pool_linear_one_kernel(StepPtrs xs, int T, int C, int HW, int K, int classes_per_block,
                                                                        const VT* v_init, VT* v_out,
                                                                        const XT* __restrict__ Wt, const XT* __restrict__ bias,
                                                                        XT* __restrict__ out, LifParams lif, float inv_hw, float steps) {
@@ -441,9 +443,10 @@ __global__ __launch_bounds__(kThreads) void lif_pool_linear_one_kernel(StepPtrs 
     const int elems = C * HW;                                    // a multiple of 8 (host)
     const int64_t base = static_cast<int64_t>(n) * elems;
     const bool writes_v = blockIdx.x == 0;
-    for (int i = threadIdx.x; i < C; i += kThreads) plane_count[i] = 0;
+    for (int i = threadIdx.x; i < C; i += THREADS) plane_count[i] = 0;
     __syncthreads();
-    for (int i0 = threadIdx.x * kVec; i0 < elems; i0 += kThreads * kVec) {
+    auto pass = [&](int i0, auto usual_tag) __attribute__((always_inline)) {
+        constexpr bool usual = decltype(usual_tag)::value;
         float v[kVec];
         int fired[kVec];
 #pragma unroll
@@ -456,16 +459,16 @@ __global__ __launch_bounds__(kThreads) void lif_pool_linear_one_kernel(StepPtrs 
 #pragma unroll
             for (int j = 0; j < kVec; ++j) v[j] = to_float(pv.v[j]);
         }
-        for (int t0 = 0; t0 < T; t0 += 4) {
-            Pack<XT, kVec> px[4];
+        for (int t0 = 0; t0 < T; t0 += TC) {
+            Pack<XT, kVec> px[TC];
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
+            for (int u = 0; u < TC; ++u)
                 if (t0 + u < T) px[u] = *reinterpret_cast<const Pack<XT, kVec>*>(static_cast<const XT*>(xs.p[t0 + u]) + base + i0);
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
+            for (int u = 0; u < TC; ++u) {
                 if (t0 + u < T) {
 #pragma unroll
-                    for (int j = 0; j < kVec; ++j) fired[j] += lif_step(to_float(px[u].v[j]), v[j], lif) ? 1 : 0;
+                    for (int j = 0; j < kVec; ++j) fired[j] += lif_step_as<usual>(to_float(px[u].v[j]), v[j], lif) ? 1 : 0;
                 }
             }
         }
@@ -490,9 +493,13 @@ __global__ __launch_bounds__(kThreads) void lif_pool_linear_one_kernel(StepPtrs 
             }
         }
         if (run != 0) atomicAdd(&plane_count[p], run);
-    }
+    };
+    if (usual_neuron(lif))
+        for (int i0 = threadIdx.x * kVec; i0 < elems; i0 += THREADS * kVec) pass(i0, std::true_type{});
+    else
+        for (int i0 = threadIdx.x * kVec; i0 < elems; i0 += THREADS * kVec) pass(i0, std::false_type{});
     __syncthreads();
-    classify_counts<XT>(plane_count, n, C, K, classes_per_block, Wt, bias, out, inv_hw, steps, 1.0f);
+    classify_counts<XT, THREADS>(plane_count, n, C, K, classes_per_block, Wt, bias, out, inv_hw, steps, 1.0f);
 }
 
 // Average pool and classifier on bit-packed spikes (one byte = 8 channels of a pixel), summed over T: the workgroup of a
@@ -573,16 +580,27 @@ __global__ __launch_bounds__(kThreads) void spike_pool_linear_kernel(const unsig
         flush();
     }
     __syncthreads();
-    classify_counts<XT>(plane_count, n, C, K, classes_per_block, Wt, bias, out, inv_hw, steps, out_scale);
+    classify_counts<XT, kThreads>(plane_count, n, C, K, classes_per_block, Wt, bias, out, inv_hw, steps, out_scale);
 }
 
-// Class ranges per sample of the one-launch tail: at least 16 classes each (one pass of the workgroup's four waves), no more
-// workgroups than two per compute unit. 0: the shape takes the two launches.
+// Threads of a workgroup of the one-launch tail: one pass over the sample's neurons.
+int one_launch_threads(int C, int HW) {
+    const int64_t neurons = static_cast<int64_t>(C) * HW;
+    return neurons <= 256 * kVec ? 256 : (neurons <= 512 * kVec ? 512 : 1024);
+}
+
+// Class ranges per sample of the one-launch tail: at least as many classes each as the workgroup's waves take at a time, no more
+// workgroups than two per compute unit (of 256 threads; as many threads of the larger ones). 0: the shape takes the two launches, where a workgroup would take its classes in
+// many rounds: a round is 1.3 us, the second launch 2 to 3. us, one launch / two, bf16, T = 4: 512 channels, 1000 classes, 16 samples (two rounds) 6.9 / 7.9, 64 (eight) 14.6 / 8.1, fp32 15.3 / 14.4; 480
+// channels of 3x3 in workgroups of 512, 16 samples (one round) 7.0 / 7.7, 64 (four) 13.9 / 8.0.
 int one_launch_class_blocks(int T, int N, int C, int HW, int K) {
-    const int64_t work = static_cast<int64_t>(T) * C * HW;
-    if (C > kOneMaxC || C % kVec != 0 || (static_cast<int64_t>(C) * HW) % kVec != 0 || work > kOneMaxSampleWork) return 0;
-    const int rows_per_pass = (kThreads / 64) * kRowsPerWave;
-    return std::max(1, std::min((K + rows_per_pass - 1) / rows_per_pass, 512 / std::max(1, N)));
+    const int64_t neurons = static_cast<int64_t>(C) * HW;
+    if (C > kOneMaxC || C % kVec != 0 || neurons > kOneMaxNeurons || T * neurons > kOneMaxSampleWork) return 0;
+    const int threads = one_launch_threads(C, HW);
+    const int rows = (threads / 64) * kRowsPerWave;
+    const int blocks = std::max(1, std::min((K + rows - 1) / rows, 512 * 256 / threads / std::max(1, N)));
+    const int rounds = ((K + blocks - 1) / blocks + rows - 1) / rows;
+    return rounds <= (threads == 256 ? 3 : 1) ? blocks : 0;
 }
 
 template <typename XT, typename VT>
@@ -671,6 +689,24 @@ extern "C" size_t snnf_lif_pool_linear_workspace_bytes(int N, int C) {
 namespace snnf {
 namespace {
 
+template <typename XT, typename VT>
+void launch_one(int threads, dim3 grid, hipStream_t hs, const StepPtrs& xs, int T, int C, int HW, int K, int per_block, const void* v_init, void* v_out,
+                const void* fc_weight, const void* fc_bias, void* out, const LifParams& lif, float inv_hw, float steps) {
+    auto go = [&](auto threads_tag, auto tc_tag) {
+        constexpr int THREADS = decltype(threads_tag)::value;
+        lif_pool_linear_one_kernel<XT, VT, THREADS, decltype(tc_tag)::value><<<grid, THREADS, 0, hs>>>(
+            xs, T, C, HW, K, per_block, static_cast<const VT*>(v_init), static_cast<VT*>(v_out), static_cast<const XT*>(fc_weight), static_cast<const XT*>(fc_bias),
+            static_cast<XT*>(out), lif, inv_hw, steps);
+    };
+    auto steps_in_flight = [&](auto threads_tag) {
+        if (T <= 4) go(threads_tag, std::integral_constant<int, 4>{});
+        else go(threads_tag, std::integral_constant<int, 8>{});
+    };
+    if (threads == 256) steps_in_flight(std::integral_constant<int, 256>{});
+    else if (threads == 512) steps_in_flight(std::integral_constant<int, 512>{});
+    else steps_in_flight(std::integral_constant<int, 1024>{});
+}
+
 // Shared body of the two entry points: `counts` is N * C ints of device memory (the caller's workspace or the library's
 // own static array).
 int lif_pool_linear_impl(const char* who, const void* const* xs, int T, int N, int C, int H, int W, int x_dtype,
@@ -715,10 +751,9 @@ int lif_pool_linear_impl(const char* who, const void* const* xs, int T, int N, i
             const int per_block = (K + class_blocks - 1) / class_blocks;
             const float inv_hw = 1.0f / static_cast<float>(HW);
             const float steps = static_cast<float>(T);
+            const int threads = one_launch_threads(C, HW);
 #define SNNF_TAIL_ONE(XT, VT)                                                                                               \
-    lif_pool_linear_one_kernel<XT, VT><<<grid, kThreads, 0, hs>>>(ptrs, T, C, HW, K, per_block, static_cast<const VT*>(v_init), \
-                                                                  static_cast<VT*>(v_out), static_cast<const XT*>(fc_weight),   \
-                                                                  static_cast<const XT*>(fc_bias), static_cast<XT*>(out_sum), lif, inv_hw, steps)
+    launch_one<XT, VT>(threads, grid, hs, ptrs, T, C, HW, K, per_block, v_init, v_out, fc_weight, fc_bias, out_sum, lif, inv_hw, steps)
             if (x_dtype == SNNF_F32) SNNF_TAIL_ONE(float, float);
             else if (x_dtype == SNNF_BF16) {
                 if (v_dtype == SNNF_F32) SNNF_TAIL_ONE(bf16_t, float);
