@@ -122,6 +122,11 @@ RouteSpace route_space(int T, int N, int Cin, int H, int W, bool split, int64_t 
     return r;
 }
 
+// Timesteps in windows of three: no more windows than of four, and a matrix step then multiplies nothing for steps beyond T (3, 5, 6 and 9 timesteps; the rest would take more windows). us, windows of
+// four / three, T = 3: 64 -> 64 at 56^2 x 16 on bits 20.6 / 15.8, x 40 35.6 / 26.1, 128 -> 128 at 28^2 x 16 with a residual 19.0 / 15.1, dense 30.9 / 27.3, 512 -> 512 at 7^2 x 7 12.8 / 10.7; T = 6
+// 36.1 / 32.9, 69.3 / 61.8, 36.6 / 30.4, 53.3 / 47.6, 23.4 / 19.5; fp32 104 -> 328 at 16^2 x 23, T = 5 78.7 / 66.7. 121 layers: 1.13 in the mean, none slower; the same bits.
+bool threes(int T) { return T != 1 && (T + 2) / 3 == (T + 3) / 4; }
+
 // Whether a layer on dense tensors is brought into C8 and run on the blocked kernel (two launches) or stays on the dense kernels. Measured on
 // layers of 1 to 64 images, 1 to 512 channels, 1x1 to 7x7, one to eight timesteps (us, dense / here; bf16 and T = 4 unless said):
 // * Channel counts that are no multiple of 8 only have the four-wave kernels on dense tensors, which assemble every channel group from
@@ -192,9 +197,14 @@ bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int C
             if (deep) return true;
             if (!one && !strided && Cin <= 8) return false;   // (a single channel group: as above)
             if (one) return tile_use * std::sqrt(576.0 / K) <= 0.45;
-            if (strided) return tile_use * std::sqrt(std::sqrt(576.0 / K)) <= (T <= 4 ? 0.5 : (inputs < (1 << 24) ? 0.65 : 0.45));
+            // (In windows of three this kernel gains an eighth and the lines lie further up. us, dense / here, with the weighed use: T = 3 64 -> 64 at 56^2 x 9 (0.86) 30.0 / 25.7, x 28 (1.13) 57.0 / 48.7,
+            // 32 -> 64 at 32^2 x 90 (1.18) 41.0 / 38.7, x 48 (1.5) 23.2 / 27.2; T = 5 64 -> 64 at 56^2 x 16 (0.96) 63.2 / 53.6, T = 6 (1.15) 63.4 / 58.9, with a residual 69.6 / 73.4; strided T = 3
+            // 128 -> 256 at 28^2 x 5 (0.53) 21.1 / 16.0, x 90 (0.61) 91.4 / 96.3, x 48 (0.65) 65.0 / 54.6, x 28 (0.75) 34.4 / 36.3; T = 6 64 -> 128 at 56^2 x 28 (0.56) 94.0 / 78.3, x 48 (0.58) 137.9 / 142.9,
+            // 128 -> 256 at 28^2 x 9 (0.72) 43.0 / 32.4, 64 -> 128 at 56^2 x 9 (1.21) 36.1 / 34.0.)
+            const bool three = threes(T);
+            if (strided) return tile_use * std::sqrt(std::sqrt(576.0 / K)) <= (T <= 4 ? (three ? 0.66 : 0.5) : (inputs < (1 << 24) ? (three ? 1.25 : 0.65) : (three ? 0.57 : 0.45)));
             const double weighed = tile_use * std::sqrt(576.0 / K);
-            if (weighed <= (inputs >= (1 << 26) ? 0.7 : (T <= 4 ? 0.85 : 0.95))) return true;
+            if (weighed <= (inputs >= (1 << 26) ? 0.7 : (T <= 4 ? (three ? 1.2 : 0.85) : (three ? 1.1 : 0.95)))) return true;
             if (inputs / T > (5 << 19) || weighed > 1.1) return false;
             weigh = weighed;
             return true;
@@ -234,8 +244,8 @@ struct BlockedPlan {
     size_t few_lds = 0;
 };
 
-// Everything that decides whether and how the kernel runs a call; nothing is enqueued.
-int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
+// Everything that decides whether and how the kernel runs a call; nothing is enqueued. `window`: all timesteps in one window of so many (0: windows of up to four).
+int plan_window(const char* who, const BlockedCall& c, BlockedPlan& p, int window) {
     const int T = c.T, N = c.N, Cin = c.Cin, H = c.H, W = c.W, Cout = c.Cout, KH = c.KH, KW = c.KW;
     const int stride_h = c.stride_h, stride_w = c.stride_w, pad_h = c.pad_h, pad_w = c.pad_w;
     const bool shared = c.shared, neuron = c.neuron, pool2 = c.pool2;
@@ -261,7 +271,7 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
     g.taps = KH * KW;
     g.frag_stride = static_cast<int64_t>(pg.nchunks) * pg.npairs * (kFragBytes / 2);
     g.w_lo_offset = static_cast<int64_t>(pg.nchunks_r) * pg.npairs * (kFragBytes / 2);   // part 1 of the weight (kSplitParts)
-    g.narrow = c.split ? 1 : 0;
+    g.narrow = c.split || window > 0 ? 1 : 0;
     g.T = T;
     g.shared_x = shared ? 1 : 0;
     g.in_layout = c.x_layout;
@@ -270,9 +280,9 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
     g.analog_out = neuron ? 0 : 1;
     g.out_step_stride = c.out_step_stride;
 
-    // Timesteps side by side: 4 (2 for T == 2, 1 for a single step or a shared frame), fewer when the halo does not fit.
+    // Timesteps side by side: 4 (2 for T == 2, 1 for a single step or a shared frame, 3 where that takes no more windows), fewer when the halo does not fit.
     int& tt = p.tt;
-    tt = shared || T == 1 ? 1 : (T == 2 ? 2 : 4);
+    tt = window > 0 ? window : (shared || T == 1 ? 1 : (T == 2 ? 2 : (!pool2 && threes(T) ? 3 : 4)));
     TunedPlan tuned = {0, 0, 0};
     if (!c.split) {   // (measured on 16-bit activations)
         const TunedKey key = {T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, shared ? 1 : 0};
@@ -286,10 +296,10 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
                     who, g.Ho, g.Wo);
     bool planned = (tuned.patch_cols > 0 || tuned.stage_groups > 0) && plan_spk(g, tt, pl, tuned.patch_cols, tuned.stage_groups, pool2);
     p.tuned_patch = planned;
-    for (; !planned && tt >= 1; tt >>= 1) {
+    for (; !planned && tt >= 1; tt = tt == 3 ? 2 : tt >> 1) {
         planned = plan_spk(g, tt, pl, 0, 0, pool2);
         if (planned) break;
-        if (pool2) break;   // the pooled store covers the four steps of one window
+        if (pool2 || window > 0) break;   // the pooled store covers the four steps of one window
     }
     if (!planned)
         return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_shape: no patch of this layer fits a wave's LDS region (kernel %dx%d, stride %dx%d)",
@@ -303,7 +313,7 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
         while (pl.G > 2 && (g.C8in + pl.G - 1) / pl.G < share) pl.G >>= 1;
     }
     p.windows = shared ? 1 : (T + tt - 1) / tt;
-    if (neuron && p.windows > 1 && !c.has_v_out)
+    if (neuron && !shared && T > std::min(tt, 4) && !c.has_v_out)
         return fail(SNNF_ERR_INVALID_ARGUMENT, "%s: v_out is required when the timesteps take %d windows of %d (it carries the membrane between them)",
                     who, p.windows, tt);
     g.PR = pl.PR; g.PC = pl.PC; g.PI = pl.PI; g.RR = pl.RR; g.RC = pl.RC; g.region = pl.region; g.G = pl.G;
@@ -394,7 +404,7 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
         PackGeom& pg2 = p.pg2;
         pg2 = make_pack_geom(Cout, sc->Cin, 1, 1, false);
         const int gpc2 = pg2.CK / 8;
-        if (tt != 4 || g.tap_pairs || gpc2 % g.G != 0 || nst + 4 + hg + 4 > kSpkMaxSteps + 4)
+        if (tt < 3 || g.tap_pairs || gpc2 % g.G != 0 || nst + 4 + hg + 4 > kSpkMaxSteps + 4)
             return fail(SNNF_ERR_UNSUPPORTED, "%s: unsupported_shortcut: this layer's plan (window %d, %d channel groups per stage, %d steps) has no room for a shortcut",
                         who, tt, g.G, nst);
         g.sc_C8 = sc->Cin / 8;
@@ -426,6 +436,23 @@ int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
     return SNNF_OK;
 }
 
+// Five and six timesteps take one window where two windows of three would be short: narrow tiles whose K several waves share, with up to 16 matrix steps to each.
+// Such a launch lasts as long as one tile's chain of set-up, stages, exchange of sums and epilogue, which it then has once instead of twice. us, two windows / one, T = 6:
+// 64 -> 64 at 24^2 x 8 11.9 / 10.1 (bits), 17.2 / 15.9 (dense), 72 -> 240 at 10^2 x 9 19.2 / 17.2, T = 5: 32 -> 296 at 15^2 x 6 with a residual 17.3 / 15.7, 24 -> 27 at 10 x 28 x 11 15.6 / 13.5;
+// 11 layers, the smallest gain 1.08. Longer shares lose to the six steps' smaller stages and narrow tiles to wide ones (256 -> 256 at 8^2 x 10 with a
+// residual, dense, 18 steps 19.8 / 20.8, 512 -> 512 at 7^2 x 7 25.4 / 28.0, 128 -> 128 at 28^2 x 16 30.4 / 35.5). Eight steps in one window lose there too (512 -> 512
+// at 7^2 x 7, T = 8 23.2 / 26.8): nothing is multiplied for steps beyond T, and the activations of a narrow tile come from LDS at its full rate.
+int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
+    if (const int rc = plan_window(who, c, p, 0); rc != SNNF_OK) return rc;
+    if ((c.T != 5 && c.T != 6) || c.shared || c.split || c.shortcut != nullptr || p.tt != 3 || p.few || p.tuned_patch || p.tuned_split || p.g.tap_pairs || !p.g.narrow ||
+        p.wk_log2 == 0 || ((p.g.taps * p.g.C8in / 2) >> p.wk_log2) > 16) return SNNF_OK;
+    BlockedPlan one;
+    if (plan_window(who, c, one, 6) != SNNF_OK || one.wk_log2 == 0) return SNNF_OK;   // (a wave alone has no variant)
+    one.few = false;                                   // (the plan above has answered that)
+    p = one;
+    return SNNF_OK;
+}
+
 // Whether a layer of whole tiles beyond the usual line, whose copy is small, moves (see takes_blocked_route): `weigh` is its `tile_use` weighed by the products per output, up
 // to 1.1. Of 842 drawn layers there 134 lose, up to a quarter, and what they lose by stands in this kernel's plan: waves without a tile (64 -> 64 at 56^2 x 11 with a residual, 1078 tiles
 // on 2048 waves, 37.5 / 43.7), more than two rounds of waves (32 -> 512 at 32^2 x 58, T = 2, with a residual 168 / 190), patches of four columns (64 -> 64 at 48 x 28 x 20 28 / 36), and few
@@ -449,6 +476,8 @@ const char* family_name(DenseFamily f) {
 enum DenseRouteKind { kNoRoute, kCopyRoute, kFrameRoute };
 void plan_text(char* text, const BlockedPlan& p, const char* kernel, int epilogue, int window, DenseRouteKind route) {
     const SpkGeom& g = p.g;
+    // (window: the timesteps that a window of the layer holds. Of `threes` it runs three, as the variant's last digit says.)
+    if (p.tt == 3) window = 4;
     snprintf(text, 256,
              "kernel=%s variant=%d window=%d launches=%d tile=%dx%dx%d halo=%dx%d waves=8x1x%d oc_tiles=%d oc_tile=%d px_tiles=%d "
              "stage_chunks=%d run=0 lds=%zu grid=%d tuned=%d shortcut_stages=%d%s",
@@ -527,9 +556,9 @@ Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, 
     return route;
 }
 
-// fp32 elements that pass from window to window beside a 16-bit membrane.
+// fp32 elements that pass from window to window beside a 16-bit membrane, and room for them in calls of more than four timesteps.
 int64_t carried_membrane(const Route& r, int v_dtype, int N, int H, int W, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w) {
-    if (v_dtype == SNNF_F32 || r.kept->plan.windows <= 1) return 0;
+    if (v_dtype == SNNF_F32 || (r.kept->plan.windows <= 1 && r.kept->plan.tt <= 4)) return 0;   // (one window of six keeps the answer that two had)
     return static_cast<int64_t>(N) * Cout * ((H + 2 * pad_h - KH) / stride_h + 1) * ((W + 2 * pad_w - KW) / stride_w + 1);
 }
 
@@ -803,7 +832,7 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     const bool fast_epi = neuron && (out_layout == SNNF_LAYOUT_BITS || pool2) && (residuals == nullptr || res_layout == SNNF_LAYOUT_BITS) &&
                           L.lif.charge_mode == CHARGE_SCALE && L.lif.inv_tau == 0.5f && L.lif.v_reset == 0.0f &&
                           L.lif.v_threshold >= 1e-30f && L.lif.v_threshold <= 1e30f &&   // its multiples by 2^t stay normal numbers
-                          v_init == nullptr && (p.windows == 1 || p.tt == 4) && Cout % 8 == 0;
+                          v_init == nullptr && (p.windows == 1 || p.tt >= 3) && Cout % 8 == 0;
     // Dense tensors around the neuron: no range limit on the threshold, any reset potential, initial membrane, windows and channels.
     // (A frame for all timesteps: without a residual, with or without a membrane.)
     const bool frame_epi = x_layout == SNNF_LAYOUT_NCHW && shared && residuals == nullptr;
@@ -843,8 +872,11 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
         if (x_layout == SNNF_LAYOUT_NCHW) return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_frame(L, true) : launch_conv_spk_f16_frame(L, true);
         return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_pooled(L, p.tt) : launch_conv_spk_f16_pooled(L, p.tt);
     }
+    if (sc != nullptr && p.tt == 3) return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_three_shortcut(L) : launch_conv_spk_f16_three_shortcut(L);
     if (sc != nullptr) return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_shortcut(L) : launch_conv_spk_f16_shortcut(L);
     if (x_layout == SNNF_LAYOUT_NCHW) return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_frame(L, false) : launch_conv_spk_f16_frame(L, false);
+    if (p.tt == 6) return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_long(L) : launch_conv_spk_f16_long(L);
+    if (p.tt == 3) return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_three(L) : launch_conv_spk_f16_three(L);
     if (x_layout == SNNF_LAYOUT_BITS) return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_bits(L, p.tt) : launch_conv_spk_f16_bits(L, p.tt);
     return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_c8(L, p.tt) : launch_conv_spk_f16_c8(L, p.tt);
 }

@@ -2,5 +2,5 @@
 #include "snnf_conv_spk_kernel.h"
 
 namespace snnf {
-int launch_conv_spk_f16_shortcut(const SpkLaunch& L) { return launch_conv_spk_shortcut<f16_t>(L); }
+int launch_conv_spk_f16_shortcut(const SpkLaunch& L) { return launch_conv_spk_shortcut<f16_t, 4>(L); }
 }  // namespace snnf

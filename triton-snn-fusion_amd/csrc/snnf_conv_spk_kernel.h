@@ -230,13 +230,14 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
     }
     __builtin_amdgcn_sched_barrier(0);
 
-    static_assert(!SC || (IN == SNNF_LAYOUT_BITS && TT == 4), "the shortcut variants take bit-packed inputs, four timesteps at a time");
+    static_assert(!SC || (IN == SNNF_LAYOUT_BITS && (TT == 3 || TT == 4)), "the shortcut variants take bit-packed inputs, three or four timesteps at a time");
     static_assert(!POOL || (FAST && (TT == 4 || TT == 1)), "the pooled output belongs to the straight-line epilogue of four steps");
     static_assert(IN != SNNF_LAYOUT_NCHW || (TT == 1 && !SK), "a dense input is one frame for all timesteps, of one channel group");
     constexpr bool SPLIT = std::is_same<XT, float>::value;
     static_assert(!NARROW || SK || (!SC && (!POOL || IN == SNNF_LAYOUT_NCHW)), "narrow tiles of one wave: not of a shortcut, and pooled only of a dense frame");
     static_assert(!SPLIT || (NARROW && IN == SNNF_LAYOUT_C8 && !FAST && !SC && !POOL), "fp32 tensors: narrow tiles on two C8 tensors, dense tensors out");
     static_assert(!MULTI || (FAST && !POOL), "several windows belong to the straight-line epilogue");
+    static_assert(TT <= 4 || (NARROW && SK && !SPLIT && !SC && !POOL && !MULTI), "more than four timesteps side by side: narrow tiles of 16-bit tensors whose K waves share, one window");
     static_assert(!DENSE || (IN != SNNF_LAYOUT_BITS && !FAST && !SC && !POOL), "the dense epilogue belongs to calls on dense tensors");
     // No two of the membrane arguments are the same memory: a call in place passes no v_start, and only one with a 16-bit membrane has a
     // v_scratch. (Promising nothing here instead cost the straight-line epilogue 2 %: ResNet-18, 16 images of 224x224 361 -> 369 us.)
@@ -245,6 +246,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
     float* const v_carry = g.v16 ? v_scratch : v_out;
     constexpr int NF = NARROW ? 1 : 2;         // 32-channel weight fragments of a tile
     constexpr int TG = 4 * NF;                 // channel groups of 8 of a tile
+    constexpr int TL = TT > 4 ? 4 : TT;        // timesteps whose activations a matrix step holds at a time
     // A dense frame with dense spikes is computed in the form of the matrix kernel (which takes other neurons, and frames per timestep of whole tiles): the bias
     // behind the sums, the charge as v + (x - v) / 2. One frame T times and T equal frames then have the same bits where that kernel also adds a sum's products in this
     // order (3 -> 64 3x3 at 32^2, 7x7 stride 2 at 224^2 x 16). On other channels and kernels (8 -> 64, 1 -> 64 5x5), and where equal frames take the copy route, whose sums
@@ -654,7 +656,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     const int nst_s = second ? hg : nst;
                     constexpr int WF = SPLIT ? 2 : NF;    // weight fragments of a step: two of 32 channels, or the two terms of one
                     sk_u32x4 wa[4][WF];
-                    sk_u32x4 wb[2][TT];
+                    sk_u32x4 wb[2][TL];
                     uint32_t bo[4];
                     // Requests the weight fragments of the step described by table entry `e` and notes where its activations are.
                     auto req_a = [&](int slot, const Pack<uint32_t, 2>& e) __attribute__((always_inline)) {
@@ -665,11 +667,11 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     };
                     auto read_b = [&](int slot, uint32_t boff) __attribute__((always_inline)) {
 #pragma unroll
-                        for (int t = 0; t < TT; ++t) wb[slot][t] = *reinterpret_cast<const sk_u32x4*>(bl + boff + t * tile_t);
+                        for (int t = 0; t < TL; ++t) wb[slot][t] = *reinterpret_cast<const sk_u32x4*>(bl + boff + t * tile_t);
                     };
                     auto mma = [&](int sa, int sb) __attribute__((always_inline)) {
 #pragma unroll
-                        for (int t = 0; t < TT; ++t) {
+                        for (int t = 0; t < TL; ++t) {
                             acc[t][0] = sk_mfma<F16>(wa[sa][0], wb[sb][t], acc[t][0]);
                             if constexpr (!NARROW) acc[t][1] = sk_mfma<F16>(wa[sa][1], wb[sb][t], acc[t][1]);
                         }
@@ -679,6 +681,15 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                                 for (int t = 0; t < TT; ++t) acc[t][0] = sk_mfma<F16>(wa[sa][1], wb[sb][t], acc[t][0]);
                             }
                         }
+                    };
+                    // The timesteps from the fifth on (TT > 4): a matrix step's second half, against the same weights.
+                    auto read_b_late = [&](int slot, uint32_t boff) __attribute__((always_inline)) {
+#pragma unroll
+                        for (int t = TL; t < TT; ++t) wb[slot][t - TL] = *reinterpret_cast<const sk_u32x4*>(bl + boff + t * tile_t);
+                    };
+                    auto mma_late = [&](int sa, int sb) __attribute__((always_inline)) {
+#pragma unroll
+                        for (int t = TL; t < TT; ++t) acc[t][0] = sk_mfma<F16>(wa[sa][0], wb[sb][t - TL], acc[t][0]);
                     };
                     req_a(0, tb[0]);
                     req_a(1, tb[2]);
@@ -708,6 +719,20 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     auto step_order = [&]() __attribute__((always_inline)) {
                         constexpr int kMfma = 0x008, kValu = 0x002, kVmemRead = 0x020, kDsRead = 0x100;
                         if constexpr (SPLIT) return;
+                        if constexpr (TT > 4) {      // (the first half of a step: four matrix instructions, the second half's activations)
+                            __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(kValu, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(kVmemRead, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(kDsRead, 2, 0);
+                            __builtin_amdgcn_sched_group_barrier(kValu, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(kDsRead, 3, 0);
+                            __builtin_amdgcn_sched_group_barrier(kValu, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+                            __builtin_amdgcn_sched_barrier(0);
+                            return;
+                        }
                         if constexpr (NARROW) {
                             __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
                             __builtin_amdgcn_sched_group_barrier(kValu, 1, 0);
@@ -716,6 +741,10 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                                 __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
                                 __builtin_amdgcn_sched_group_barrier(kDsRead, 2, 0);
                                 __builtin_amdgcn_sched_group_barrier(kValu, 1, 0);
+                            }
+                            if constexpr (TT == 3) {
+                                __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+                                __builtin_amdgcn_sched_group_barrier(kDsRead, 2, 0);
                             }
                             if constexpr (TT >= 4) {
                                 __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
@@ -740,6 +769,12 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                             __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 0);
                             __builtin_amdgcn_sched_group_barrier(kValu, 1, 0);
                         }
+                        if constexpr (TT == 3) {
+                            __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(kValu, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+                        }
                         if constexpr (TT >= 4) {
                             __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
                             __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 0);
@@ -751,6 +786,52 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                         }
                         __builtin_amdgcn_sched_barrier(0);
                     };
+                    auto late_order = [&]() __attribute__((always_inline)) {   // the second half: TT - 4 matrix instructions, the next step's first activations
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+                        if constexpr (TT > 6) __builtin_amdgcn_sched_group_barrier(0x008, TT - 6, 0);
+                        __builtin_amdgcn_sched_barrier(0);
+                    };
+                    if constexpr (TT > 4) {
+                        // Weights as below; the activations one half step ahead.
+                        auto step = [&](int cur, int next, int far, int i) __attribute__((always_inline)) {
+                            req_a(far, ent);
+                            ent = tb[2 * (st + i)];
+                            read_b_late(1, bo[cur]);
+                            mma(cur, 0);
+                            step_order();
+                            read_b(0, bo[next]);
+                            mma_late(cur, 1);
+                            late_order();
+                        };
+                        for (; st + 4 <= nst_s; st += 4) {
+                            step(0, 1, 3, 4);
+                            step(1, 2, 0, 5);
+                            step(2, 3, 1, 6);
+                            step(3, 0, 2, 7);
+                        }
+                        if (st < nst_s) {
+                            read_b_late(1, bo[0]);
+                            mma(0, 0);
+                            if (st + 1 < nst_s) read_b(0, bo[1]);
+                            mma_late(0, 1);
+                            if (st + 1 < nst_s) {
+                                read_b_late(1, bo[1]);
+                                mma(1, 0);
+                                if (st + 2 < nst_s) read_b(0, bo[2]);
+                                mma_late(1, 1);
+                                if (st + 2 < nst_s) {
+                                    read_b_late(1, bo[2]);
+                                    mma(2, 0);
+                                    mma_late(2, 1);
+                                }
+                            }
+                        }
+                        continue;
+                    }
                     for (; st + 4 <= nst_s; st += 4) {
                         req_a(3, ent);
                         ent = tb[2 * (st + 4)];
@@ -1200,12 +1281,14 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             };
             // The quads of a usual tile - four steps from a zero membrane that is not asked for - two at a time, without a condition per quad: 8.4 k -> 5.2 k
             // cycles for a wave's eight quads, 11.5 k -> 7.9 k with a residual (64 -> 64 at 56^2 x 16 19.5 -> 18.4 us and 20.7 -> 19.8).
-            const bool lean = (TT == 4 || TT == 1) && !MULTI && t_count == 4 && v_out == nullptr;
+            constexpr bool LEAN = TT == 4 || TT == 3 || TT == 1;
+            constexpr int LT = TT == 3 ? 3 : 4;      // (of three steps where the window has three)
+            const bool lean = LEAN && !MULTI && t_count == LT && v_out == nullptr;
             auto lean_quad = [&](const float (&xq)[TT][4], const uint32_t (&rb)[TT], auto res_tag) __attribute__((always_inline)) -> uint32_t {
                 float S[4] = {0.0f, 0.0f, 0.0f, 0.0f};
                 uint32_t quiet = 0;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
+                for (int i = 0; i < LT; ++i) {
                     if constexpr (decltype(res_tag)::value) {
                         float x[4];
 #pragma unroll
@@ -1238,7 +1321,12 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     qb = lean_quad(xq, rb, res_tag);
                     if constexpr (POOL) fast_store4_pooled(j8b, qb);
                 }
-                if constexpr (!POOL) fast_store4(j8a, qa, TWO ? j8b : -1, qb);
+                if constexpr (TT == 3) {
+                    fast_store(tb, 3, j8a, qa);
+                    if constexpr (TWO) fast_store(tb, 3, j8b, qb);
+                } else if constexpr (!POOL) {
+                    fast_store4(j8a, qa, TWO ? j8b : -1, qb);
+                }
             };
             // DENSE: dense spikes (and residual) around the usual neuron (tau 2, hard reset), any number of windows and channels. A lane's
             // pixel is one element of a channel plane, so spikes, residual and membrane move as single elements, 32 lanes side by side.
@@ -1450,7 +1538,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                         do_quad(std::integral_constant<int, 7>{});
                     } else if (lean && !with_res) {
                         lean_all(std::false_type{});
-                    } else if (lean && TT == 4) {
+                    } else if (lean && TT >= 3) {
                         lean_all(std::true_type{});
                     } else {
                         // A loop: a quad's sums are copied out of the accumulators by a switch (constant register indices).
@@ -1615,7 +1703,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                     // The wave's finished quads: run at once (FAST, usual tiles), or left in LDS for the loop below.
                     auto finish = [&](auto quads_tag) __attribute__((always_inline)) {
                         constexpr int QUADS = decltype(quads_tag)::value;
-                        if constexpr (FAST && (TT == 4 || TT == 1)) {
+                        if constexpr (FAST && LEAN) {
                             const auto sum = [&](int tw, int q, int k) __attribute__((always_inline)) { return own[q][tw][k]; };
                             auto lean_all = [&](auto res_tag) __attribute__((always_inline)) {
                                 lean_pair(sum, std::integral_constant<int, 0>{}, std::integral_constant<bool, (QUADS > 1)>{}, res_tag, jq + quad_x, jq + (1 ^ quad_x), rb[0], rb[1]);
@@ -1625,7 +1713,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                                 lean_all(std::false_type{});
                                 return;
                             }
-                            if (lean && TT == 4) {
+                            if (lean && TT >= 3) {
                                 lean_all(std::true_type{});
                                 return;
                             }
@@ -1662,7 +1750,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                         add(own[0], first);
                         finish(std::integral_constant<int, 1>{});
                     }
-                    if (!(FAST && lean && (TT == 4 || (TT == 1 && g.res_layout < 0)))) {
+                    if (!(FAST && lean && (TT >= 3 || (TT == 1 && g.res_layout < 0)))) {
                         for (int e = 0; e < quads; ++e) {
                             const int j8 = jq + (e ^ quad_x);
                             float xq[TT][4];
@@ -1700,7 +1788,18 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                 } else {
                     // A narrow tile's four quads, all TT timesteps: quad e is finished by wave e mod WK of the tile, which adds the WK
                     // partial sums in a fixed order and then runs that quad's timesteps like the unsplit kernel.
-                    SNNF_SPK_PARK_QUAD(wave, 0, 0, 0) SNNF_SPK_PARK_QUAD(wave, 1, 0, 1) SNNF_SPK_PARK_QUAD(wave, 2, 0, 2) SNNF_SPK_PARK_QUAD(wave, 3, 0, 3)
+                    // (Of more than four timesteps a slot holds four at a time: the first four of all quads, then the others.)
+                    auto park = [&](auto from_tag, auto to_tag) __attribute__((always_inline)) {
+                        constexpr int FROM = decltype(from_tag)::value, TO = decltype(to_tag)::value;
+#pragma unroll
+                        for (int q = 0; q < 4; ++q)
+#pragma unroll
+                            for (int tw = FROM; tw < TO; ++tw) {
+                                const sk_f32x4 four = {acc[tw][0][4 * q], acc[tw][0][4 * q + 1], acc[tw][0][4 * q + 2], acc[tw][0][4 * q + 3]};
+                                *reinterpret_cast<sk_f32x4*>(part + wave * slot_bytes + ((q * TL + tw - FROM) * 64 + lane_p) * 16) = four;
+                            }
+                    };
+                    park(std::integral_constant<int, 0>{}, std::integral_constant<int, TL>{});
                     const int part0 = wave ^ wk;         // the slot of part k is part0 ^ k
                     const int e_first = wk;      // this wave finishes quads e_first, e_first + WK, ... < 4
                     // The residual bytes of the wave's first quad travel while the workgroup meets.
@@ -1722,46 +1821,47 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                         if (e_first < 4) dense_request(oc_e * TG + e_first, in);
                     }
                     __syncthreads();
-                    for (int e_own = e_first; e_own < 4; e_own += WK) {
+                    // The partial sums of the tile's waves for the N timesteps that are parked, of two or four waves in flight together (WK is a power of two
+                    // >= 2); added in the order of the parts.
+                    auto gather = [&](auto n_tag, int e_own, sk_f32x4* __restrict__ sum) __attribute__((always_inline)) {
+                        constexpr int N = decltype(n_tag)::value;
+#pragma unroll
+                        for (int tw = 0; tw < N; ++tw) sum[tw] = sk_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                        auto add_parts = [&](auto parts_tag, int k) __attribute__((always_inline)) {
+                            constexpr int PARTS = decltype(parts_tag)::value;
+                            sk_f32x4 p[PARTS][N];
+#pragma unroll
+                            for (int i = 0; i < PARTS; ++i)
+#pragma unroll
+                                for (int tw = 0; tw < N; ++tw) p[i][tw] = *reinterpret_cast<const sk_f32x4*>(part + (part0 ^ (k + i)) * slot_bytes + ((e_own * TL + tw) * 64 + lane_p) * 16);
+                            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                            for (int i = 0; i < PARTS; ++i)
+#pragma unroll
+                                for (int tw = 0; tw < N; ++tw)
+#pragma unroll
+                                    for (int c = 0; c < 4; ++c) sum[tw][c] += p[i][tw][c];
+                        };
+                        if constexpr (FAST || DENSE) {
+                            if (WK == 2) add_parts(std::integral_constant<int, 2>{}, 0);
+                            else
+                                for (int k = 0; k < WK; k += 4) add_parts(std::integral_constant<int, 4>{}, k);
+                        } else {   // the general epilogue has no registers to spare: one wave's sums at a time
+                            for (int k = 0; k < WK; ++k) {
+#pragma unroll
+                                for (int tw = 0; tw < N; ++tw)
+                                    sum[tw] += *reinterpret_cast<const sk_f32x4*>(part + (part0 ^ k) * slot_bytes + ((e_own * TL + tw) * 64 + lane_p) * 16);
+                            }
+                        }
+                    };
+                    // One of the wave's quads, with its sums.
+                    auto run_quad = [&](int e_own, const sk_f32x4 (&sum)[TT]) __attribute__((always_inline)) {
                         const int j8 = oc_e * TG + e_own;
                         float xq[TT][4];
-                        {
-                            // The partial sums of the tile's waves, all timesteps of two or four waves in flight together (WK is a power of two >= 2); added
-                            // in the order of the parts.
-                            sk_f32x4 sum[TT];
 #pragma unroll
-                            for (int tw = 0; tw < TT; ++tw) sum[tw] = sk_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-                            auto add_parts = [&](auto n_tag, int k) __attribute__((always_inline)) {
-                                constexpr int PARTS = decltype(n_tag)::value;
-                                sk_f32x4 p[PARTS][TT];
+                        for (int tw = 0; tw < TT; ++tw)
 #pragma unroll
-                                for (int i = 0; i < PARTS; ++i)
-#pragma unroll
-                                    for (int tw = 0; tw < TT; ++tw) p[i][tw] = *reinterpret_cast<const sk_f32x4*>(part + (part0 ^ (k + i)) * slot_bytes + ((e_own * TT + tw) * 64 + lane_p) * 16);
-                                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                                for (int i = 0; i < PARTS; ++i)
-#pragma unroll
-                                    for (int tw = 0; tw < TT; ++tw)
-#pragma unroll
-                                        for (int c = 0; c < 4; ++c) sum[tw][c] += p[i][tw][c];
-                            };
-                            if constexpr (FAST || DENSE) {
-                                if (WK == 2) add_parts(std::integral_constant<int, 2>{}, 0);
-                                else
-                                    for (int k = 0; k < WK; k += 4) add_parts(std::integral_constant<int, 4>{}, k);
-                            } else {   // the general epilogue has no registers to spare: one wave's sums at a time
-                                for (int k = 0; k < WK; ++k) {
-#pragma unroll
-                                    for (int tw = 0; tw < TT; ++tw)
-                                        sum[tw] += *reinterpret_cast<const sk_f32x4*>(part + (part0 ^ k) * slot_bytes + ((e_own * TT + tw) * 64 + lane_p) * 16);
-                                }
-                            }
-#pragma unroll
-                            for (int tw = 0; tw < TT; ++tw)
-#pragma unroll
-                                for (int k = 0; k < 4; ++k) xq[tw][k] = sum[tw][k];
-                        }
+                            for (int k = 0; k < 4; ++k) xq[tw][k] = sum[tw][k];
                         if constexpr (FAST) {
                             if (e_own != e_first && g.res_layout >= 0 && TT > 1) {
 #pragma unroll
@@ -1769,9 +1869,10 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                             }
                             const float start[4] = {v0[0], v0[1], v0[2], v0[3]};
                             if (e_own + WK < 4) fast_v0(j8 + WK, v0);
-                            if (lean && (g.res_layout < 0 || TT == 4)) {
+                            if (lean && (g.res_layout < 0 || TT >= 3)) {
                                 const uint32_t quiet = g.res_layout < 0 ? lean_quad(xq, rb, std::false_type{}) : lean_quad(xq, rb, std::true_type{});
                                 if constexpr (POOL) fast_store4_pooled(j8, quiet);
+                                else if constexpr (TT == 3) fast_store(tb, 3, j8, quiet);
                                 else fast_store4(j8, quiet, -1, 0u);
                             } else {
                                 fast_quad(j8, xq, rb, g.res_layout >= 0, start);
@@ -1782,6 +1883,28 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                             dense_quad(j8, xq, now);
                         } else {
                             general_quad(j8, xq);
+                        }
+                    };
+                    if constexpr (TT > 4) {
+                        sk_f32x4 sums[2][TT];    // (a wave of two finishes two quads, one of four or eight at most one)
+                        if (e_first < 4) gather(std::integral_constant<int, TL>{}, e_first, sums[0]);
+                        if (WK == 2) gather(std::integral_constant<int, TL>{}, e_first + 2, sums[1]);
+                        __syncthreads();
+                        park(std::integral_constant<int, TL>{}, std::integral_constant<int, TT>{});
+                        __syncthreads();
+                        if (e_first < 4) {
+                            gather(std::integral_constant<int, TT - TL>{}, e_first, sums[0] + TL);
+                            run_quad(e_first, sums[0]);
+                        }
+                        if (WK == 2) {
+                            gather(std::integral_constant<int, TT - TL>{}, e_first + 2, sums[1] + TL);
+                            run_quad(e_first + 2, sums[1]);
+                        }
+                    } else {
+                        for (int e_own = e_first; e_own < 4; e_own += WK) {
+                            sk_f32x4 sum[TT];
+                            gather(std::integral_constant<int, TT>{}, e_own, sum);
+                            run_quad(e_own, sum);
                         }
                     }
                 }
@@ -1806,7 +1929,7 @@ int launch_conv_spk_variant(const SpkLaunch& L) {
             return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, IN, true, false, false, false, false, true>) : run(conv_spk_kernel<XT, TT, IN, false, false, false, false, false, true>);
         }
     }
-    if constexpr (TT == 4) {
+    if constexpr (TT >= 3) {
         if (L.fast_epilogue && L.multi_window) {
             if (L.g.narrow) return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, IN, true, true, false, false, true, false, true>) : run(conv_spk_kernel<XT, TT, IN, false, true, false, false, true, false, true>);
             return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, IN, true, true, false, false, false, false, true>) : run(conv_spk_kernel<XT, TT, IN, false, true, false, false, false, false, true>);
@@ -1871,8 +1994,8 @@ int launch_conv_spk_frame(const SpkLaunch& L, bool pooled) {
     return L.fast_epilogue ? run(conv_spk_kernel<XT, 1, D, false, true>) : run(conv_spk_kernel<XT, 1, D, false, false>);
 }
 
-// The variants with a projection shortcut in the accumulators: bit-packed inputs, four timesteps side by side.
-template <typename XT>
+// The variants with a projection shortcut in the accumulators: bit-packed inputs, three or four timesteps side by side.
+template <typename XT, int TT>
 int launch_conv_spk_shortcut(const SpkLaunch& L) {
     auto run = [&](auto kernel) -> int {
         if (const int rc = reserve_lds(reinterpret_cast<const void*>(kernel), L.lds_bytes, "snnf_conv_lif_blocked_shortcut"); rc != SNNF_OK) return rc;
@@ -1882,12 +2005,27 @@ int launch_conv_spk_shortcut(const SpkLaunch& L) {
     };
     constexpr int B = SNNF_LAYOUT_BITS;
     if (L.fast_epilogue && L.multi_window) {
-        if (L.g.narrow) return run(conv_spk_kernel<XT, 4, B, true, true, true, false, true, false, true>);
-        return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, 4, B, true, true, true, false, false, false, true>) : run(conv_spk_kernel<XT, 4, B, false, true, true, false, false, false, true>);
+        if (L.g.narrow) return run(conv_spk_kernel<XT, TT, B, true, true, true, false, true, false, true>);
+        return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, B, true, true, true, false, false, false, true>) : run(conv_spk_kernel<XT, TT, B, false, true, true, false, false, false, true>);
     }
-    if (L.g.narrow) return L.fast_epilogue ? run(conv_spk_kernel<XT, 4, B, true, true, true, false, true>) : run(conv_spk_kernel<XT, 4, B, true, false, true, false, true>);
-    if (L.fast_epilogue) return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, 4, B, true, true, true>) : run(conv_spk_kernel<XT, 4, B, false, true, true>);
-    return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, 4, B, true, false, true>) : run(conv_spk_kernel<XT, 4, B, false, false, true>);
+    if (L.g.narrow) return L.fast_epilogue ? run(conv_spk_kernel<XT, TT, B, true, true, true, false, true>) : run(conv_spk_kernel<XT, TT, B, true, false, true, false, true>);
+    if (L.fast_epilogue) return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, B, true, true, true>) : run(conv_spk_kernel<XT, TT, B, false, true, true>);
+    return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, B, true, false, true>) : run(conv_spk_kernel<XT, TT, B, false, false, true>);
+}
+
+// Five or six timesteps in one window: narrow tiles whose K several waves share.
+template <typename XT, int TT, int IN>
+int launch_conv_spk_long(const SpkLaunch& L) {
+    auto run = [&](auto kernel) -> int {
+        if (const int rc = reserve_lds(reinterpret_cast<const void*>(kernel), L.lds_bytes, "snnf_conv_lif_blocked"); rc != SNNF_OK) return rc;
+        kernel<<<dim3(L.grid), kSpkWaves * 64, L.lds_bytes, L.stream>>>(L.xs, L.residuals, L.g, L.wpacked, L.bias, L.v_start,
+                                                                        static_cast<unsigned char*>(L.out), L.v_store, L.lif, L.wpacked2, L.bias2, L.v_scratch, L.lo_flags);
+        return check_launch("snnf_conv_lif_blocked");
+    };
+    if constexpr (IN == SNNF_LAYOUT_C8) {
+        if (L.dense_epilogue) return run(conv_spk_kernel<XT, TT, IN, true, false, false, false, true, true>);
+    }
+    return L.fast_epilogue ? run(conv_spk_kernel<XT, TT, IN, true, true, false, false, true>) : run(conv_spk_kernel<XT, TT, IN, true, false, false, false, true>);
 }
 
 template <typename XT, int IN>
@@ -1899,8 +2037,14 @@ int launch_conv_spk_tt(const SpkLaunch& L, int tt) {
 
 // One launcher per activation dtype and input layout (each in its own translation unit, so that they compile in parallel).
 int launch_conv_spk_bf16_bits(const SpkLaunch& L, int tt);
+int launch_conv_spk_bf16_long(const SpkLaunch& L);
+int launch_conv_spk_bf16_three(const SpkLaunch& L);
+int launch_conv_spk_bf16_three_shortcut(const SpkLaunch& L);
 int launch_conv_spk_bf16_c8(const SpkLaunch& L, int tt);
 int launch_conv_spk_f16_bits(const SpkLaunch& L, int tt);
+int launch_conv_spk_f16_long(const SpkLaunch& L);
+int launch_conv_spk_f16_three(const SpkLaunch& L);
+int launch_conv_spk_f16_three_shortcut(const SpkLaunch& L);
 int launch_conv_spk_f16_c8(const SpkLaunch& L, int tt);
 int launch_conv_spk_bf16_shortcut(const SpkLaunch& L);
 int launch_conv_spk_f16_shortcut(const SpkLaunch& L);
