@@ -125,7 +125,7 @@ RouteSpace route_space(int T, int N, int Cin, int H, int W, bool split, int64_t 
 // Timesteps in windows of three: no more windows than of four, and a matrix step then multiplies nothing for steps beyond T (3, 5, 6 and 9 timesteps; the rest would take more windows). us, windows of
 // four / three, T = 3: 64 -> 64 at 56^2 x 16 on bits 20.6 / 15.8, x 40 35.6 / 26.1, 128 -> 128 at 28^2 x 16 with a residual 19.0 / 15.1, dense 30.9 / 27.3, 512 -> 512 at 7^2 x 7 12.8 / 10.7; T = 6
 // 36.1 / 32.9, 69.3 / 61.8, 36.6 / 30.4, 53.3 / 47.6, 23.4 / 19.5; fp32 104 -> 328 at 16^2 x 23, T = 5 78.7 / 66.7. 121 layers: 1.13 in the mean, none slower; the same bits.
-bool threes(int T) { return T != 1 && (T + 2) / 3 == (T + 3) / 4; }
+bool threes(int T) { return T > 2 && (T + 2) / 3 == (T + 3) / 4; }
 
 // Whether a layer on dense tensors is brought into C8 and run on the blocked kernel (two launches) or stays on the dense kernels. Measured on
 // layers of 1 to 64 images, 1 to 512 channels, 1x1 to 7x7, one to eight timesteps (us, dense / here; bf16 and T = 4 unless said):
