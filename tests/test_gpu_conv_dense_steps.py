@@ -1,0 +1,68 @@
+"""Dense 16-bit convolutions whose kernel reads the frames of the timesteps itself, without a copy in another layout: against the CPU oracle at the edges of pairs of pixels,
+rows and channel groups, where an infinity or NaN beside the image, the channels or the batch must not be met, and the general path for other neurons."""
+import pytest
+import torch
+
+from helpers import DEV, LIF, check, dev, gen, q, spikes
+from oracle import snn_oracle as O
+
+pytestmark = pytest.mark.gpu
+BF16, F16 = torch.bfloat16, torch.float16
+SOFT = (1.0, -1.0, 2.0)
+
+
+def _run(xs, rs, w, b, zero, s, p, lif):
+    S = torch.ops.snn_custom
+    args = (w, b, zero, [s, s], [p, p], [1, 1], 1, *lif, False)
+    return S.fused_temporal_conv_lif_state(xs, *args) if rs is None else S.fused_temporal_conv_add_lif_state(xs, rs, *args)
+
+
+@pytest.mark.parametrize("Cin,Cout,H,W,k,s,N,T,dtype,residual,lif,route", [
+    (64, 64, 32, 32, 3, 1, 8, 4, BF16, False, LIF, "frames"),     # whole groups, four waves a tile
+    (20, 33, 13, 17, 3, 1, 12, 4, F16, True, LIF, "frames"),       # odd rows and single channels, in and out
+    (72, 104, 27, 35, 3, 1, 2, 6, F16, True, LIF, "frames"),       # windows of three
+    (64, 64, 24, 24, 3, 1, 4, 5, BF16, True, LIF, "frames"),       # one window
+    (40, 48, 9, 9, 5, 1, 20, 2, BF16, False, LIF, "frames"),
+    (48, 24, 23, 21, 3, 2, 16, 3, BF16, False, LIF, "frames"),     # stride 2: pairs half of which no window reads
+    (30, 18, 5, 31, 1, 1, 40, 8, BF16, True, LIF, "frames"),       # 1x1, odd rows, two windows
+    (128, 96, 3, 64, 3, 1, 14, 1, F16, False, LIF, "frames"),      # one timestep
+    (24, 40, 64, 2, 3, 1, 30, 4, BF16, False, LIF, "frames"),      # rows of two pixels
+    (24, 40, 64, 1, 3, 1, 40, 4, BF16, False, LIF, "c8"),         # of one: no pairs
+    (16, 64, 40, 40, 3, 1, 12, 4, BF16, True, LIF, None),         # a wave a tile
+    (64, 64, 32, 32, 3, 1, 8, 4, BF16, False, SOFT, "c8"),        # another neuron: the copy
+])
+def test_against_the_oracle(hip_ops, snnf_lib, Cin, Cout, H, W, k, s, N, T, dtype, residual, lif, route):
+    from triton_snn_fusion_amd.runtime import hip_convlif_backend as CB
+    g = gen(9300 + Cin + Cout + T)
+    p = k // 2
+    Ho, Wo = (H + 2 * p - k) // s + 1, (W + 2 * p - k) // s + 1
+    x = q(torch.randn(T, N, Cin, H, W, generator=g), dtype)      # any values
+    w, b = q(torch.randn(Cout, Cin, k, k, generator=g) * (2.0 / (Cin * k * k)) ** 0.5, dtype), q(torch.randn(Cout, generator=g) * 0.1, dtype)
+    rs = torch.stack([spikes((N, Cout, Ho, Wo), 0.25, g) for _ in range(T)]) if residual else None
+    ref = O.temporal_conv_lif(list(x), w, b, torch.tensor(0.0), (s, s), (p, p), (1, 1), 1, *lif, residuals=list(rs) if residual else None)
+    # Every frame lies between infinities, one element off an address of four bytes.
+    frame = N * Cin * H * W
+    room = torch.full((T, frame + 2 + frame % 2), float("inf"), dtype=dtype, device=DEV)
+    xs = [room[t, 1:1 + frame].view(N, Cin, H, W) for t in range(T)]
+    for t in range(T):
+        xs[t].copy_(x[t])
+    sp, v = _run(xs, None if rs is None else [dev(t, dtype) for t in rs], dev(w, dtype), dev(b, dtype), torch.zeros((), device=DEV), s, p, lif)
+    plan = CB.last_conv_plan()
+    if route is not None and torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert plan.get("reads", plan.get("route")) == route, plan
+    check(sp, v, ref, what=f"{Cin}->{Cout} {H}x{W} T={T}", max_rate=1e-3)
+
+
+def test_infinities_stay_in_their_windows(hip_ops, snnf_lib):
+    """An infinity in the last channel of an image reaches its own windows and no neighbour's: pixels outside the image and channels beyond the last are zeros."""
+    g = gen(9390)
+    T, N, C, H, W = 4, 10, 20, 11, 13
+    x = spikes((T, N, C, H, W), 0.3, g)
+    w, b = q(torch.randn(24, C, 3, 3, generator=g) * 0.2, BF16), q(torch.randn(24, generator=g) * 0.1, BF16)
+    clean, _ = _run([dev(t, BF16) for t in x], None, dev(w, BF16), dev(b, BF16), torch.zeros((), device=DEV), 1, 1, LIF)
+    bad = x.clone()
+    bad[:, 4, C - 1, H - 1, W - 1] = float("nan")
+    got, _ = _run([dev(t, BF16) for t in bad], None, dev(w, BF16), dev(b, BF16), torch.zeros((), device=DEV), 1, 1, LIF)
+    met = torch.zeros(T, N, 24, H, W, dtype=torch.bool)
+    met[:, 4, :, H - 2:, W - 2:] = True
+    assert torch.equal(got.cpu()[~met], clean.cpu()[~met])

@@ -41,7 +41,8 @@ bool plan_spk(const SpkGeom& g0, int tt, SpkPlan& best, int only_pc = 0, int onl
         const int oc_tiles = g0.narrow ? (g0.Cout + 31) / 32 : (g0.Cout + 63) / 64;
         if (pi > 1 && ((g0.N + pi - 1) / pi) * oc_tiles * 2 < cus) pi >>= 1;
         const int rr = (pr - 1) * g0.sh + g0.KH;
-        const int rc = (pc - 1) * g0.sw + g0.KW;
+        const int pair = g0.in_layout == kSpkSteps ? 2 : 1;    // items that a lane stages at a time
+        const int rc = ((pc - 1) * g0.sw + g0.KW + pair - 1) / pair * pair;
         if (rr > 255 || rc > 255) continue;
         // Where the halos of so many planes don't fit (5x5 on 2x2 planes, strided 3x3 onto 2x2 and 4x4) half as many, and again, before a part
         // of one plane: 512 -> 512 stride 2 from 4x4 x 155 in tiles of 2 x 1 pixels 170 us, of four planes 48, 256 -> 512, 5x5 on 2x2 x 122,
@@ -52,11 +53,11 @@ bool plan_spk(const SpkGeom& g0, int tt, SpkPlan& best, int only_pc = 0, int onl
         for (;; pi >>= 1) {
             region = pi * rr * rc;
             if (g0.tap_pairs) {
-                if (region <= 64 * kSpkSlots && tt * (region + 1) * 16 <= kWaveLds) G = 1;
+                if (region <= 64 * kSpkSlots && tt * (region + pair) * 16 <= kWaveLds) G = 1;
             } else {
                 for (int cand = g0.gpc; cand >= 2; cand >>= 1) {
                     if (only_g > 0 && cand > only_g) continue;
-                    if (cand * region <= 64 * kSpkSlots && tt * (cand * region + 1) * 16 <= kWaveLds) {   // + the dummy item of a timestep
+                    if (cand * region <= 64 * kSpkSlots && tt * (cand * region + pair) * 16 <= kWaveLds) {   // + the dummy items of a timestep
                         G = cand;
                         break;
                     }
@@ -322,8 +323,9 @@ int plan_window(const char* who, const BlockedCall& c, BlockedPlan& p, int windo
     g.n_patches = pl.img_groups * g.patches_img;
     g.nstages = (g.C8in + g.G - 1) / g.G;
     g.IT = g.G * g.region;
-    g.JT = (g.IT + 63) / 64;
-    g.lds_wave_bytes = std::max(tt * (g.IT + 1) * 16, 256);   // (a tile's bias passes through it)
+    const int pair = g.in_layout == kSpkSteps ? 2 : 1;
+    g.JT = (g.IT / pair + 63) / 64;
+    g.lds_wave_bytes = std::max(tt * (g.IT + pair) * 16, 256);   // (a tile's bias passes through it)
     int& oc_tiles = p.oc_tiles;
     oc_tiles = g.narrow ? (Cout + 31) / 32 : (Cout + 63) / 64;
     g.n_items = g.n_patches * oc_tiles;
@@ -417,7 +419,7 @@ int plan_window(const char* who, const BlockedCall& c, BlockedPlan& p, int windo
     }
     // Layers whose K several waves share, in few tiles: the kernel for few pixels. One that could be pooled takes it with and without its pool or not at
     // all, so that the pooled launch has the sums of the unpooled one.
-    if (neuron && !c.split && !shared && sc == nullptr && wk_log2 > 0 && !p.tuned_patch && !p.tuned_split && (c.out_layout != SNNF_LAYOUT_C8 || pool2) && c.res_layout != SNNF_LAYOUT_C8) {
+    if (neuron && !c.split && !shared && sc == nullptr && c.x_layout != kSpkSteps && wk_log2 > 0 && !p.tuned_patch && !p.tuned_split && (c.out_layout != SNNF_LAYOUT_C8 || pool2) && c.res_layout != SNNF_LAYOUT_C8) {
         FewGeom& f = p.few_g;
         f.N = N; f.C8in = g.C8in; f.H = H; f.W = W; f.Cout = Cout; f.C8out = g.C8out; f.KH = KH; f.KW = KW;
         f.sh = stride_h; f.sw = stride_w; f.ph = pad_h; f.pw = pad_w; f.Ho = g.Ho; f.Wo = g.Wo; f.T = T;
@@ -469,11 +471,27 @@ bool fills_waves(const BlockedPlan& p, double weigh, int T, int Cout) {
     return g.iters <= 2 && line <= 1.55 * std::min(1.0, static_cast<double>(static_cast<int64_t>(g.n_items) << p.wk_log2) / waves);
 }
 
+// Whether the kernel reads the dense frames of a call itself instead of a launch that brings them into C8 first. That launch takes 3 to 4 us and the time of the bytes it moves; without it every tile
+// assembles its halo from loads of two pixels of one channel, and `loads` of them for a compute unit take 3.6 ns each, half as much again from patches of short rows, and
+// more than twice where a wave has a tile of its own, all of whose stages then wait for them in turn. Fitted to 107 drawn layers, of which this takes 78, at 1.24 in the mean (four lose 2 to 22 %); the others
+// would be at 0.98. us, copy / here: T = 4 64 -> 64 at 32^2 x 8 14.6 / 11.5, 128 -> 128 at 20^2 x 7 16.0 / 12.1, 168 -> 56 1x1 at 36^2 x 4 17.0 / 9.8, 256 -> 256 at 14^2 x 16 with a residual
+// 30.1 / 26.5, 256 -> 512 stride 2 27.9 / 22.5, 72 -> 104 at 27 x 35 x 5 with a residual, T = 6 28.4 / 25.0, 48 -> 18 1x1 at 9^2 x 9, T = 3 10.7 / 7.1; not taken: 88 -> 96 at 104^2 x 2 38.9 / 43.8,
+// 229 -> 80 at 24 x 108 x 23, T = 2 109 / 166. Strided layers of up to two channel groups are not among them and keep the copy, as do rows of one pixel, which have no pairs.
+bool reads_steps(const BlockedPlan& p, int T) {
+    const SpkGeom& g = p.g;
+    if (g.W < 2 || (g.C8in <= 2 && (g.sh > 1 || g.sw > 1))) return false;
+    const double units = std::min(p.grid, compute_units());
+    const double loads = static_cast<double>(g.n_items) / units * g.C8in * g.region * T / 16.0;
+    const double megabytes = static_cast<double>(g.N) * g.C8in * g.H * g.W * T * 16e-6;
+    return 2.7 + 0.28 * megabytes > loads * (0.0036 + (p.wk_log2 == 0 ? 0.0052 : 0.0) + (g.PC < 8 ? 0.0018 : 0.0));
+}
+
 const char* family_name(DenseFamily f) {
     return f == DenseFamily::kTInM ? "t_in_m" : (f == DenseFamily::kTimeOuter ? "time_outer" : (f == DenseFamily::kPointwise ? "pointwise" : "matrix"));
 }
 
-enum DenseRouteKind { kNoRoute, kCopyRoute, kFrameRoute };
+// (kStepsRoute: the blocked route, whose kernel reads the dense frames itself; one launch.)
+enum DenseRouteKind { kNoRoute, kCopyRoute, kFrameRoute, kStepsRoute };
 void plan_text(char* text, const BlockedPlan& p, const char* kernel, int epilogue, int window, DenseRouteKind route) {
     const SpkGeom& g = p.g;
     // (window: the timesteps that a window of the layer holds. Of `threes` it runs three, as the variant's last digit says.)
@@ -483,7 +501,7 @@ void plan_text(char* text, const BlockedPlan& p, const char* kernel, int epilogu
              "stage_chunks=%d run=0 lds=%zu grid=%d tuned=%d shortcut_stages=%d%s",
              kernel, (p.wk_log2 > 0 ? 50 : 40) + p.tt + epilogue, window, route == kCopyRoute ? 2 : 1, g.PI, g.PR, g.PC, g.RR, g.RC, 1 << p.wk_log2, p.oc_tiles,
              g.narrow ? 32 : 64, g.n_patches, g.G, p.lds_bytes, p.grid, (p.tuned_patch ? 1 : 0) + (p.tuned_split ? 2 : 0), g.sc_stages,
-             route == kCopyRoute ? " route=c8 ran=blocked" : (route == kFrameRoute ? " route=frame ran=blocked" : ""));
+             route == kCopyRoute ? " route=c8 ran=blocked" : (route == kFrameRoute ? " route=frame ran=blocked" : (route == kStepsRoute ? " route=c8 ran=blocked reads=frames" : "")));
     // A launch of few pixels: the workgroups (images x rows x columns x channels x their number) that run instead of the tiles above.
     if (p.few) {
         const size_t n = strlen(text);
@@ -499,6 +517,8 @@ using RouteKey = std::array<int, 16>;
 struct KeptPlan {
     BlockedPlan plan;
     char text[2][256];                                 // with the general and with the dense epilogue
+    BlockedPlan steps;                                 // of the kernel on the dense frames themselves, where the dense epilogue applies (see `reads_steps`; grid 0: never)
+    char steps_text[256];
 };
 struct Route { bool taken; DenseFamily family; std::shared_ptr<const KeptPlan> kept; };
 std::mutex routes_mutex;
@@ -547,6 +567,14 @@ Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, 
                       (frame || weigh == 0.0 || fills_waves(plan, weigh, T, Cout));
         if (route.taken) {
             for (int dense_epi = 0; dense_epi < 2; ++dense_epi) plan_text(kept->text[dense_epi], plan, family_name(route.family), dense_epi ? 40 : 0, frame ? T : plan.tt, frame ? kFrameRoute : kCopyRoute);
+            if (!frame && neuron && !split && !plan.few) {
+                BlockedPlan direct;
+                if (plan_blocked("snnf_conv_lif", BlockedCall{T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, kSpkSteps, residual ? SNNF_LAYOUT_NCHW : -1,
+                                 SNNF_LAYOUT_NCHW, 0, false, true, false, true, false, nullptr, false}, direct) == SNNF_OK && reads_steps(direct, T)) {
+                    kept->steps = direct;
+                    plan_text(kept->steps_text, direct, family_name(route.family), 40, direct.tt, kStepsRoute);
+                }
+            }
             route.kept = kept;
         }
     }
@@ -800,12 +828,17 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
                                                          v_init != nullptr, v_out != nullptr, pool2, sc, split}, made); rc != SNNF_OK)
             return rc;
     }
-    const BlockedPlan& p = dense != nullptr ? dense->kept->plan : made;
+    // (Of a dense call xs are the C8 buffers; a wave's K, stages and sums don't depend on which of the two it reads.)
+    const LifParams lif_params = make_lif_params(v_threshold, v_reset, tau);
+    const bool usual = lif_params.charge_mode == CHARGE_SCALE && lif_params.inv_tau == 0.5f && !lif_params.soft_reset;
+    const bool steps = dense != nullptr && dense->xs != nullptr && dense->kept->steps.grid > 0 && usual && v_out != nullptr &&
+                       std::all_of(dense->xs, dense->xs + T, [](const void* x) { return aligned_to(x, 2); });
+    const BlockedPlan& p = dense == nullptr ? made : (steps ? dense->kept->steps : dense->kept->plan);
     const SpkGeom& g = p.g;
 
     SpkLaunch L = {};
     for (int t = 0; t < T; ++t) {
-        L.xs.p[t] = xs[t];
+        L.xs.p[t] = steps ? dense->xs[t] : xs[t];
         if (residuals != nullptr) L.residuals.p[t] = residuals[t];
         if (sc != nullptr) L.residuals.p[t] = sc->xs[t];   // the second input travels in the residual's place (a shortcut launch has no residual)
     }
@@ -825,7 +858,7 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
         L.g.v16 = 1;
         L.v_scratch = reinterpret_cast<float*>(static_cast<char*>(const_cast<void*>(xs[0])) + dense->space.carry);
     }
-    L.lif = make_lif_params(v_threshold, v_reset, tau);
+    L.lif = lif_params;
     L.grid = p.grid;
     L.lds_bytes = p.lds_bytes;
     L.stream = as_stream(stream);
@@ -837,12 +870,14 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     // (A frame for all timesteps: without a residual, with or without a membrane.)
     const bool frame_epi = x_layout == SNNF_LAYOUT_NCHW && shared && residuals == nullptr;
     const bool dense_epi = neuron && (frame_epi || (x_layout == SNNF_LAYOUT_C8 && !shared && L.v_store != nullptr)) && out_layout == SNNF_LAYOUT_NCHW &&
-                           (residuals == nullptr || res_layout == SNNF_LAYOUT_NCHW) && L.lif.charge_mode == CHARGE_SCALE && L.lif.inv_tau == 0.5f && !L.lif.soft_reset;
-    if (dense != nullptr) memcpy(snnf::conv_plan_buffer(), dense->kept->text[dense_epi ? 1 : 0], 256);
+                           (residuals == nullptr || res_layout == SNNF_LAYOUT_NCHW) && usual;
+    if (steps) memcpy(snnf::conv_plan_buffer(), dense->kept->steps_text, 256);
+    else if (dense != nullptr) memcpy(snnf::conv_plan_buffer(), dense->kept->text[dense_epi ? 1 : 0], 256);
     else plan_text(snnf::conv_plan_buffer(), p, "blocked", fast_epi ? 20 : (dense_epi ? 40 : 0), shared ? T : p.tt, kNoRoute);
     L.fast_epilogue = fast_epi;
     L.multi_window = p.windows > 1;
     L.dense_epilogue = dense_epi;
+    if (steps) return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_steps(L, p.tt) : launch_conv_spk_f16_steps(L, p.tt);
     if (dense != nullptr && dense->xs != nullptr) {   // the plan stands: bring the dense inputs into the C8 buffers behind `xs`
         StepPtrs from = {};
         for (int t = 0; t < T; ++t) from.p[t] = dense->xs[t];

@@ -37,6 +37,7 @@ constexpr int kSpkWaves = 8;                      // waves per workgroup, one wo
 #endif
 constexpr int kSpkSlots = SPK_SLOTS;                      // staging items per lane and timestep, at most
 constexpr int kSpkPartialBytes = 16 * 64 * 16;     // split-K: a wave parks 4 quads x up to 4 timesteps of partial sums in its region
+constexpr int kSpkSteps = 16;                     // an input layout of this kernel alone (no code of the library's): dense frames, one per timestep
 constexpr int kSpkMaxSteps = 60;                  // matrix steps per stage, at most (the step table holds 4 more)
 constexpr size_t kSpkTableBytes = (kSpkMaxSteps + 4) * 16;      // the workgroup's step table at the start of LDS
 constexpr int kSpkDescs = 64 * kSpkSlots;                       // staging items of one timestep, at most
@@ -201,6 +202,8 @@ __device__ __forceinline__ sk_u32x4 sk_expand_bits(uint32_t twice) {
 // MULTI: the straight-line epilogue of calls of several windows, which pass the membrane on through memory (a variant of its own: the
 // loads of that membrane cost the calls of one window 3 to 5 %). 64 -> 64 at 56^2 x 16, T = 8, with a residual 70.2 -> 39.6 us against the
 // general epilogue, 128 -> 128 at 20^2 x 3, T = 6 18.4 -> 14.9, 512 -> 512 at 7^2 x 7, T = 8 29.0 -> 25.0.
+// IN = kSpkSteps: dense frames, one per timestep, as they are: a lane brings two neighbouring pixels of 8 channels into LDS, from eight loads of 4 bytes that hold
+// one channel each (at any even address). Which calls take it instead of a launch that brings them into C8 first: see `reads_steps`.
 // SPLIT (XT = float): fp32 tensors as two bf16 terms. The tile is a narrow one whose two weight fragments are the high and the low terms
 // of the same 32 channels, both multiplied with the high terms of the activations; stages of the low activation terms follow where the
 // tile's halo has any (spikes, averages of spikes and 8-bit pixels have none).
@@ -234,6 +237,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
     static_assert(!POOL || (FAST && (TT == 4 || TT == 1)), "the pooled output belongs to the straight-line epilogue of four steps");
     static_assert(IN != SNNF_LAYOUT_NCHW || (TT == 1 && !SK), "a dense input is one frame for all timesteps, of one channel group");
     constexpr bool SPLIT = std::is_same<XT, float>::value;
+    static_assert(IN != kSpkSteps || (DENSE && !SPLIT), "dense frames per timestep belong to the dense epilogue of 16-bit tensors");
     static_assert(!NARROW || SK || (!SC && (!POOL || IN == SNNF_LAYOUT_NCHW)), "narrow tiles of one wave: not of a shortcut, and pooled only of a dense frame");
     static_assert(!SPLIT || (NARROW && IN == SNNF_LAYOUT_C8 && !FAST && !SC && !POOL), "fp32 tensors: narrow tiles on two C8 tensors, dense tensors out");
     static_assert(!MULTI || (FAST && !POOL), "several windows belong to the straight-line epilogue");
@@ -262,7 +266,8 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
     const int l32 = lane & 31;
     unsigned char* const wlds = lds + kSpkHeaderBytes + wave * g.lds_wave_bytes;
     const int region16 = g.region * 16;        // bytes of one channel group of the halo
-    const int tile_t = g.G * region16 + 16;    // bytes of one timestep's stage: its items and one dummy item that absorbs the writes of idle staging slots
+    constexpr int PAIR = IN == kSpkSteps ? 2 : 1;          // items that a lane stages at a time: neighbours in a halo row (whose length is even)
+    const int tile_t = g.G * region16 + 16 * PAIR;    // bytes of one timestep's stage: its items and dummy ones that absorb the writes of idle staging slots
 
     const int WK = SK ? (1 << g.wk_log2) : 1;
     const int wk = SK ? sk_share(wave, WK) : 0;
@@ -324,14 +329,14 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             Pack<uint32_t, 2> d;
             d.v[0] = 0u;
             d.v[1] = 0xff000000u;
-            if (e < g.IT) {
-                const int gq = sk_div(e, g.d_region);
-                const int rem = e - gq * g.region;
+            if (e * PAIR < g.IT) {
+                const int gq = sk_div(e * PAIR, g.d_region);
+                const int rem = e * PAIR - gq * g.region;
                 const int ii = sk_div(rem, g.d_rrrc);
                 const int rem2 = rem - ii * (g.RR * g.RC);
                 const int r = sk_div(rem2, g.d_RC);
                 const int c = rem2 - r * g.RC;
-                if constexpr (IN == SNNF_LAYOUT_NCHW) d.v[0] = static_cast<uint32_t>(((ii * g.Cin + gq * 8) * g.H + r) * g.W + c);   // elements of a dense frame
+                if constexpr (IN == SNNF_LAYOUT_NCHW || IN == kSpkSteps) d.v[0] = static_cast<uint32_t>(((ii * g.Cin + gq * 8) * g.H + r) * g.W + c);   // elements of a dense frame
                 else d.v[0] = static_cast<uint32_t>(((ii * g.C8in + gq) * g.H + r) * g.W + c);
                 d.v[1] = static_cast<uint32_t>(r) | (static_cast<uint32_t>(c) << 8) | (static_cast<uint32_t>(ii) << 16) | (static_cast<uint32_t>(gq) << 24);
             }
@@ -467,10 +472,67 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             // Item e = slot * 64 + lane of a timestep = (group, image, row, column) of the halo; its LDS address is 16 e. Items
             // are decoded on the fly (nothing about them is kept in registers across the matrix loop) and move in batches of 4
             // slots x TT timesteps: all loads of a batch are in flight together.
+            // ... of dense frames: all timesteps of 64 pairs of items together.
+            auto stage_pairs = [&](int s, int lane_s) __attribute__((always_inline)) {
+                const int plane = g.H * g.W, gg0 = s * g.G;
+                const int base_u = ((n0 * g.Cin + gg0 * 8) * g.H + ih_lo) * g.W + iw_lo;
+#pragma unroll
+                for (int jb = 0; jb < kSpkSlots / 2; ++jb) {
+                    if (jb < sk_here(g.JT)) {
+                        const Pack<uint32_t, 2> d = desc[jb * 64 + lane_s];
+                        const int r = static_cast<int>(d.v[1] & 255u), c = iw_lo + static_cast<int>((d.v[1] >> 8) & 255u);
+                        const int ii = static_cast<int>((d.v[1] >> 16) & 255u), gq = static_cast<int>(d.v[1] >> 24);
+                        const bool ok = static_cast<bool>(static_cast<int>(n0 + ii < g.N) & static_cast<int>(gg0 + gq < g.C8in) &
+                                                          static_cast<int>(static_cast<unsigned>(ih_lo + r) < static_cast<unsigned>(g.H)));
+                        const bool in0 = ok & (static_cast<unsigned>(c) < static_cast<unsigned>(g.W)), in1 = ok & (static_cast<unsigned>(c + 1) < static_cast<unsigned>(g.W));
+                        // A pair of which one pixel lies in the image is read with that pixel's other neighbour (rows have at least two).
+                        const uint32_t off = in0 || in1 ? static_cast<uint32_t>(base_u + static_cast<int>(d.v[0]) + (in0 ? (in1 ? 0 : -1) : 1)) : 0u;
+                        constexpr uint32_t kLow = 0x05040100u, kHigh = 0x07060302u, kNone = 0x0c0c0c0cu;     // v_perm: the low or the high halves of two words
+                        const uint32_t sel0 = in0 ? (in1 ? kLow : kHigh) : kNone, sel1 = in1 ? (in0 ? kHigh : kLow) : kNone;
+                        const int left = in0 || in1 ? g.Cin - (gg0 + gq) * 8 : g.Cin;    // channels of this group, and beyond (of the first one where there is no pixel)
+                        struct __attribute__((packed, aligned(2))) Word { uint32_t v; };
+                        uint32_t raw[TT][8];
+                        if (g.Cin & 7) {
+#pragma unroll
+                            for (int t = 0; t < TT; ++t) {
+                                const uint16_t* __restrict__ src = static_cast<const uint16_t*>(sk_kernarg_ptr(0, t0 + t < nsteps_t ? t0 + t : t0));
+#pragma unroll
+                                for (int k = 0; k < 8; ++k) raw[t][k] = reinterpret_cast<const Word*>(src + (off + static_cast<uint32_t>(min(k, left - 1) * plane)))->v;
+                            }
+#pragma unroll
+                            for (int t = 0; t < TT; ++t)
+#pragma unroll
+                                for (int k = 0; k < 8; ++k) raw[t][k] = k < left ? raw[t][k] : 0u;
+                        } else {
+#pragma unroll
+                            for (int t = 0; t < TT; ++t) {
+                                const uint16_t* __restrict__ src = static_cast<const uint16_t*>(sk_kernarg_ptr(0, t0 + t < nsteps_t ? t0 + t : t0));
+#pragma unroll
+                                for (int k = 0; k < 8; ++k) raw[t][k] = reinterpret_cast<const Word*>(src + (off + static_cast<uint32_t>(k * plane)))->v;
+                            }
+                        }
+                        unsigned char* const item = wlds + min((jb * 64 + lane_s) * 2, g.IT) * 16;
+#pragma unroll
+                        for (int t = 0; t < TT; ++t) {
+                            sk_u32x4 a, b;
+#pragma unroll
+                            for (int k = 0; k < 4; ++k) {
+                                a[k] = __builtin_amdgcn_perm(raw[t][2 * k + 1], raw[t][2 * k], sel0);
+                                b[k] = __builtin_amdgcn_perm(raw[t][2 * k + 1], raw[t][2 * k], sel1);
+                            }
+                            *reinterpret_cast<sk_u32x4*>(item + t * tile_t) = a;
+                            *reinterpret_cast<sk_u32x4*>(item + t * tile_t + 16) = b;
+                        }
+                    }
+                }
+            };
             auto stage_in = [&](int s) __attribute__((always_inline)) {
                 __builtin_amdgcn_wave_barrier();   // the matrix steps of the previous stage have read their operands
                 int lane_s = lane;                 // opaque: the decode below stays here instead of being hoisted out of every loop
                 asm volatile("" : "+v"(lane_s));   // (its results would sit in registers, or in scratch memory, across the matrix loop)
+                if constexpr (IN == kSpkSteps) {
+                    stage_pairs(s, lane_s);
+                } else {
 #pragma unroll
                 for (int jb = 0; jb < kSpkSlots; jb += 4) {
                     if (jb < sk_here(g.JT)) {
@@ -540,6 +602,7 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                             }
                         }
                     }
+                }
                 }
                 __builtin_amdgcn_wave_barrier();   // LDS serves a wave's accesses in order: the reads below see these writes
             };
@@ -2028,6 +2091,23 @@ int launch_conv_spk_long(const SpkLaunch& L) {
     return L.fast_epilogue ? run(conv_spk_kernel<XT, TT, IN, true, true, false, false, true>) : run(conv_spk_kernel<XT, TT, IN, true, false, false, false, true>);
 }
 
+// Dense frames per timestep around the dense epilogue.
+template <typename XT, int TT>
+int launch_conv_spk_steps(const SpkLaunch& L) {
+    auto run = [&](auto kernel) -> int {
+        if (const int rc = reserve_lds(reinterpret_cast<const void*>(kernel), L.lds_bytes, "snnf_conv_lif"); rc != SNNF_OK) return rc;
+        kernel<<<dim3(L.grid), kSpkWaves * 64, L.lds_bytes, L.stream>>>(L.xs, L.residuals, L.g, L.wpacked, L.bias, L.v_start,
+                                                                        static_cast<unsigned char*>(L.out), L.v_store, L.lif, L.wpacked2, L.bias2, L.v_scratch, L.lo_flags);
+        return check_launch("snnf_conv_lif");
+    };
+    if constexpr (TT > 4) {
+        return run(conv_spk_kernel<XT, TT, kSpkSteps, true, false, false, false, true, true>);
+    } else {
+        if (L.g.narrow) return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, kSpkSteps, true, false, false, false, true, true>) : run(conv_spk_kernel<XT, TT, kSpkSteps, false, false, false, false, true, true>);
+        return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, kSpkSteps, true, false, false, false, false, true>) : run(conv_spk_kernel<XT, TT, kSpkSteps, false, false, false, false, false, true>);
+    }
+}
+
 template <typename XT, int IN>
 int launch_conv_spk_tt(const SpkLaunch& L, int tt) {
     if (tt == 4) return launch_conv_spk_variant<XT, 4, IN>(L);
@@ -2038,11 +2118,13 @@ int launch_conv_spk_tt(const SpkLaunch& L, int tt) {
 // One launcher per activation dtype and input layout (each in its own translation unit, so that they compile in parallel).
 int launch_conv_spk_bf16_bits(const SpkLaunch& L, int tt);
 int launch_conv_spk_bf16_long(const SpkLaunch& L);
+int launch_conv_spk_bf16_steps(const SpkLaunch& L, int tt);
 int launch_conv_spk_bf16_three(const SpkLaunch& L);
 int launch_conv_spk_bf16_three_shortcut(const SpkLaunch& L);
 int launch_conv_spk_bf16_c8(const SpkLaunch& L, int tt);
 int launch_conv_spk_f16_bits(const SpkLaunch& L, int tt);
 int launch_conv_spk_f16_long(const SpkLaunch& L);
+int launch_conv_spk_f16_steps(const SpkLaunch& L, int tt);
 int launch_conv_spk_f16_three(const SpkLaunch& L);
 int launch_conv_spk_f16_three_shortcut(const SpkLaunch& L);
 int launch_conv_spk_f16_c8(const SpkLaunch& L, int tt);
