@@ -1,4 +1,4 @@
-"""Dense 16-bit convolutions whose kernel reads the frames of the timesteps itself, without a copy in another layout: against the CPU oracle at the edges of pairs of pixels,
+"""Dense convolutions whose kernel reads the frames of the timesteps itself, without a copy in another layout: against the CPU oracle at the edges of pairs of pixels,
 rows and channel groups, where an infinity or NaN beside the image, the channels or the batch must not be met, and the general path for other neurons."""
 import pytest
 import torch
@@ -7,7 +7,7 @@ from helpers import DEV, LIF, check, dev, gen, q, spikes
 from oracle import snn_oracle as O
 
 pytestmark = pytest.mark.gpu
-BF16, F16 = torch.bfloat16, torch.float16
+BF16, F16, F32 = torch.bfloat16, torch.float16, torch.float32
 SOFT = (1.0, -1.0, 2.0)
 
 
@@ -51,6 +51,45 @@ def test_against_the_oracle(hip_ops, snnf_lib, Cin, Cout, H, W, k, s, N, T, dtyp
     if route is not None and torch.cuda.get_device_properties(0).multi_processor_count == 256:
         assert plan.get("reads", plan.get("route")) == route, plan
     check(sp, v, ref, what=f"{Cin}->{Cout} {H}x{W} T={T}", max_rate=1e-3)
+
+
+@pytest.mark.parametrize("Cin,Cout,H,W,k,s,N,T,residual,low", [
+    (64, 64, 32, 32, 3, 1, 8, 4, False, "none"),          # spikes: no low terms
+    (64, 64, 32, 32, 3, 1, 8, 4, False, "all"),
+    (72, 24, 14, 14, 3, 1, 3, 4, True, "one"),            # five stages on four waves, a low term in the last one alone
+    (88, 40, 20, 19, 3, 1, 4, 3, False, "one"),           # six on four, odd rows
+    (20, 33, 13, 17, 3, 1, 6, 6, True, "all"),            # single channels, windows of three
+    (168, 24, 9, 9, 3, 2, 6, 2, False, "all"),            # eight waves, stride 2
+    (30, 18, 5, 31, 1, 1, 20, 1, True, "one"),            # 1x1, one timestep
+    (16, 24, 30, 31, 3, 1, 20, 5, False, "all"),          # one stage: a wave a tile
+])
+def test_fp32_terms_against_the_oracle(hip_ops, snnf_lib, Cin, Cout, H, W, k, s, N, T, residual, low):
+    from triton_snn_fusion_amd.runtime import hip_convlif_backend as CB
+    g = gen(9350 + Cin + Cout + T)
+    p = k // 2
+    Ho, Wo = (H + 2 * p - k) // s + 1, (W + 2 * p - k) // s + 1
+    x = torch.randn(T, N, Cin, H, W, generator=g) if low == "all" else spikes((T, N, Cin, H, W), 0.3, g)
+    if low == "one":
+        x[T - 1, N - 1, Cin - 1, H // 2, W - 1] = 1.0 + 2.0 ** -10       # (a low term that a bf16 sum over the window shows)
+    w, b = torch.randn(Cout, Cin, k, k, generator=g) * (2.0 / (Cin * k * k)) ** 0.5, torch.randn(Cout, generator=g) * 0.1
+    rs = torch.stack([spikes((N, Cout, Ho, Wo), 0.25, g) for _ in range(T)]) if residual else None
+    ref = O.temporal_conv_lif(list(x), w, b, torch.tensor(0.0), (s, s), (p, p), (1, 1), 1, *LIF, residuals=list(rs) if residual else None)
+    frame = N * Cin * H * W
+    room = torch.full((T, frame + 2), float("inf"), device=DEV)
+    xs = [room[t, 1:1 + frame].view(N, Cin, H, W) for t in range(T)]
+    for t in range(T):
+        xs[t].copy_(x[t])
+    sp, v = _run(xs, None if rs is None else [dev(t, F32) for t in rs], dev(w, F32), dev(b, F32), torch.zeros((), device=DEV), s, p, LIF)
+    plan = CB.last_conv_plan()
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert plan.get("reads") == "frames", plan
+    check(sp, v, ref, what=f"{Cin}->{Cout} {H}x{W} T={T}", max_rate=1e-3)
+    if low == "one":      # the low term's own share: the call without it, on the neurons that have the same spikes
+        xs[T - 1][N - 1, Cin - 1, H // 2, W - 1] = 1.0
+        sp1, v1 = _run(xs, None if rs is None else [dev(t, F32) for t in rs], dev(w, F32), dev(b, F32), torch.zeros((), device=DEV), s, p, LIF)
+        same = (sp == sp1).all(0) & (sp[-1] == 0)
+        changed = ((v - v1) != 0) & same
+        assert int(changed.sum()) > 0 and int(changed[:N - 1].sum()) == 0
 
 
 def test_infinities_stay_in_their_windows(hip_ops, snnf_lib):

@@ -476,13 +476,16 @@ bool fills_waves(const BlockedPlan& p, double weigh, int T, int Cout) {
 // more than twice where a wave has a tile of its own, all of whose stages then wait for them in turn. Fitted to 107 drawn layers, of which this takes 78, at 1.24 in the mean (four lose 2 to 22 %); the others
 // would be at 0.98. us, copy / here: T = 4 64 -> 64 at 32^2 x 8 14.6 / 11.5, 128 -> 128 at 20^2 x 7 16.0 / 12.1, 168 -> 56 1x1 at 36^2 x 4 17.0 / 9.8, 256 -> 256 at 14^2 x 16 with a residual
 // 30.1 / 26.5, 256 -> 512 stride 2 27.9 / 22.5, 72 -> 104 at 27 x 35 x 5 with a residual, T = 6 28.4 / 25.0, 48 -> 18 1x1 at 9^2 x 9, T = 3 10.7 / 7.1; not taken: 88 -> 96 at 104^2 x 2 38.9 / 43.8,
-// 229 -> 80 at 24 x 108 x 23, T = 2 109 / 166. Strided layers of up to two channel groups are not among them and keep the copy, as do rows of one pixel, which have no pairs.
-bool reads_steps(const BlockedPlan& p, int T) {
+// 229 -> 80 at 24 x 108 x 23, T = 2 109 / 166. fp32 tensors, whose pairs take loads of 8 bytes and twice the rounding to two terms: of 77 drawn layers 39, at 1.19 in the mean (five lose
+// 2 to 12 %), the others would be at 0.83: 64 -> 64 at 32^2 x 8 16.1 / 14.7, 88 -> 88 at 20^2 x 9, T = 3 16.2 / 11.7, 256 -> 88 1x1 at 8^2 x 16 with a residual 13.3 / 9.4; 128 -> 128 at 28^2 x 16 50.4 / 65.7.
+// Strided layers of up to two channel groups are not among the measured and keep the copy, as do rows of one pixel, which have no pairs.
+bool reads_steps(const BlockedPlan& p, int T, bool split) {
     const SpkGeom& g = p.g;
     if (g.W < 2 || (g.C8in <= 2 && (g.sh > 1 || g.sw > 1))) return false;
     const double units = std::min(p.grid, compute_units());
     const double loads = static_cast<double>(g.n_items) / units * g.C8in * g.region * T / 16.0;
-    const double megabytes = static_cast<double>(g.N) * g.C8in * g.H * g.W * T * 16e-6;
+    const double megabytes = static_cast<double>(g.N) * g.C8in * g.H * g.W * T * 16e-6;      // of one term
+    if (split) return 3.1 + 0.3 * megabytes > loads * (0.0083 + (p.wk_log2 == 0 ? 0.0022 : 0.0));
     return 2.7 + 0.28 * megabytes > loads * (0.0036 + (p.wk_log2 == 0 ? 0.0052 : 0.0) + (g.PC < 8 ? 0.0018 : 0.0));
 }
 
@@ -567,10 +570,10 @@ Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, 
                       (frame || weigh == 0.0 || fills_waves(plan, weigh, T, Cout));
         if (route.taken) {
             for (int dense_epi = 0; dense_epi < 2; ++dense_epi) plan_text(kept->text[dense_epi], plan, family_name(route.family), dense_epi ? 40 : 0, frame ? T : plan.tt, frame ? kFrameRoute : kCopyRoute);
-            if (!frame && neuron && !split && !plan.few) {
+            if (!frame && neuron && !plan.few) {
                 BlockedPlan direct;
                 if (plan_blocked("snnf_conv_lif", BlockedCall{T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, kSpkSteps, residual ? SNNF_LAYOUT_NCHW : -1,
-                                 SNNF_LAYOUT_NCHW, 0, false, true, false, true, false, nullptr, false}, direct) == SNNF_OK && reads_steps(direct, T)) {
+                                 SNNF_LAYOUT_NCHW, 0, false, true, false, true, false, nullptr, split}, direct) == SNNF_OK && reads_steps(direct, T, split)) {
                     kept->steps = direct;
                     plan_text(kept->steps_text, direct, family_name(route.family), 40, direct.tt, kStepsRoute);
                 }
@@ -832,7 +835,7 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     const LifParams lif_params = make_lif_params(v_threshold, v_reset, tau);
     const bool usual = lif_params.charge_mode == CHARGE_SCALE && lif_params.inv_tau == 0.5f && !lif_params.soft_reset;
     const bool steps = dense != nullptr && dense->xs != nullptr && dense->kept->steps.grid > 0 && usual && v_out != nullptr &&
-                       std::all_of(dense->xs, dense->xs + T, [](const void* x) { return aligned_to(x, 2); });
+                       std::all_of(dense->xs, dense->xs + T, [x_dtype](const void* x) { return aligned_to(x, dtype_size(x_dtype)); });
     const BlockedPlan& p = dense == nullptr ? made : (steps ? dense->kept->steps : dense->kept->plan);
     const SpkGeom& g = p.g;
 
@@ -877,6 +880,7 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     L.fast_epilogue = fast_epi;
     L.multi_window = p.windows > 1;
     L.dense_epilogue = dense_epi;
+    if (steps && split) return launch_conv_spk_f32_steps(L, p.tt);
     if (steps) return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_steps(L, p.tt) : launch_conv_spk_f16_steps(L, p.tt);
     if (dense != nullptr && dense->xs != nullptr) {   // the plan stands: bring the dense inputs into the C8 buffers behind `xs`
         StepPtrs from = {};

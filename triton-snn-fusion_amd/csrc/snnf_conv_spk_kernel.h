@@ -237,9 +237,9 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
     static_assert(!POOL || (FAST && (TT == 4 || TT == 1)), "the pooled output belongs to the straight-line epilogue of four steps");
     static_assert(IN != SNNF_LAYOUT_NCHW || (TT == 1 && !SK), "a dense input is one frame for all timesteps, of one channel group");
     constexpr bool SPLIT = std::is_same<XT, float>::value;
-    static_assert(IN != kSpkSteps || (DENSE && !SPLIT), "dense frames per timestep belong to the dense epilogue of 16-bit tensors");
+    static_assert(IN != kSpkSteps || DENSE, "dense frames per timestep belong to the dense epilogue");
     static_assert(!NARROW || SK || (!SC && (!POOL || IN == SNNF_LAYOUT_NCHW)), "narrow tiles of one wave: not of a shortcut, and pooled only of a dense frame");
-    static_assert(!SPLIT || (NARROW && IN == SNNF_LAYOUT_C8 && !FAST && !SC && !POOL), "fp32 tensors: narrow tiles on two C8 tensors, dense tensors out");
+    static_assert(!SPLIT || (NARROW && (IN == SNNF_LAYOUT_C8 || IN == kSpkSteps) && !FAST && !SC && !POOL), "fp32 tensors: narrow tiles on two C8 tensors or dense frames, dense tensors out");
     static_assert(!MULTI || (FAST && !POOL), "several windows belong to the straight-line epilogue");
     static_assert(TT <= 4 || (NARROW && SK && !SPLIT && !SC && !POOL && !MULTI), "more than four timesteps side by side: narrow tiles of 16-bit tensors whose K waves share, one window");
     static_assert(!DENSE || (IN != SNNF_LAYOUT_BITS && !FAST && !SC && !POOL), "the dense epilogue belongs to calls on dense tensors");
@@ -408,6 +408,10 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             // PRE (bit-packed inputs, lean epilogue): the first batch of the NEXT stage is requested before the matrix steps of the
             // current one and sits in registers meanwhile, so that its latency hides behind them.
             constexpr bool PRE = FAST && IN == SNNF_LAYOUT_BITS;
+            int nstages_all = SC ? g.nstages + g.sc_stages : g.nstages;
+            uint64_t low_groups = 0;             // SPLIT: which stages of low terms run (below)
+            // The first stage of low terms; of dense frames a wave's own follow its own, so that what it found decides.
+            const int low_first = SPLIT && IN == kSpkSteps && SK ? ((g.nstages + (1 << g.wk_log2) - 1) >> g.wk_log2) << g.wk_log2 : g.nstages;
             uint32_t pre_raw[TT][4];
             uint32_t pre_ok = 0;
             // Decodes the 4 items of batch jb of stage s from the workgroup's descriptors: their global index (0 when they are
@@ -473,8 +477,10 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             // are decoded on the fly (nothing about them is kept in registers across the matrix loop) and move in batches of 4
             // slots x TT timesteps: all loads of a batch are in flight together.
             // ... of dense frames: all timesteps of 64 pairs of items together.
-            auto stage_pairs = [&](int s, int lane_s) __attribute__((always_inline)) {
-                const int plane = g.H * g.W, gg0 = s * g.G;
+            // (fp32: the high bf16 terms, or the low ones; whether any item has one is the answer.)
+            auto stage_pairs = [&](int gg0, bool low_terms, int lane_s) __attribute__((always_inline)) -> bool {
+                const int plane = g.H * g.W;
+                uint32_t any = 0;
                 const int base_u = ((n0 * g.Cin + gg0 * 8) * g.H + ih_lo) * g.W + iw_lo;
 #pragma unroll
                 for (int jb = 0; jb < kSpkSlots / 2; ++jb) {
@@ -490,6 +496,42 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                         constexpr uint32_t kLow = 0x05040100u, kHigh = 0x07060302u, kNone = 0x0c0c0c0cu;     // v_perm: the low or the high halves of two words
                         const uint32_t sel0 = in0 ? (in1 ? kLow : kHigh) : kNone, sel1 = in1 ? (in0 ? kHigh : kLow) : kNone;
                         const int left = in0 || in1 ? g.Cin - (gg0 + gq) * 8 : g.Cin;    // channels of this group, and beyond (of the first one where there is no pixel)
+                        unsigned char* const item = wlds + min((jb * 64 + lane_s) * 2, g.IT) * 16;
+                        if constexpr (SPLIT) {
+                            struct __attribute__((packed, aligned(4))) Two { float v[2]; };
+                            const bool take0 = in0 && !in1, take1 = in0 && in1;      // which of the two values is the first pixel's second, and the second one's
+                            Two raw[TT][8];
+#pragma unroll
+                            for (int t = 0; t < TT; ++t) {
+                                const float* __restrict__ src = static_cast<const float*>(sk_kernarg_ptr(0, t0 + t < nsteps_t ? t0 + t : t0));
+#pragma unroll
+                                for (int k = 0; k < 8; ++k) raw[t][k] = *reinterpret_cast<const Two*>(src + (off + static_cast<uint32_t>(min(k, left - 1) * plane)));
+                            }
+#pragma unroll
+                            for (int t = 0; t < TT; ++t) {
+                                sk_u32x4 a, b;
+#pragma unroll
+                                for (int k = 0; k < 4; ++k) {
+                                    float f0[2], f1[2];
+#pragma unroll
+                                    for (int i = 0; i < 2; ++i) {
+                                        const Two& two = raw[t][2 * k + i];
+                                        const bool here = 2 * k + i < left;
+                                        f0[i] = in0 && here ? (take0 ? two.v[1] : two.v[0]) : 0.0f;
+                                        f1[i] = in1 && here ? (take1 ? two.v[1] : two.v[0]) : 0.0f;
+                                    }
+                                    uint32_t hi0, lo0, hi1, lo1;
+                                    split_bf16_pair(f0[0], f0[1], hi0, lo0);
+                                    split_bf16_pair(f1[0], f1[1], hi1, lo1);
+                                    any |= (lo0 | lo1) & 0x7fff7fffu;
+                                    a[k] = low_terms ? lo0 : hi0;
+                                    b[k] = low_terms ? lo1 : hi1;
+                                }
+                                *reinterpret_cast<sk_u32x4*>(item + t * tile_t) = a;
+                                *reinterpret_cast<sk_u32x4*>(item + t * tile_t + 16) = b;
+                            }
+                            continue;
+                        }
                         struct __attribute__((packed, aligned(2))) Word { uint32_t v; };
                         uint32_t raw[TT][8];
                         if (g.Cin & 7) {
@@ -511,7 +553,6 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                                 for (int k = 0; k < 8; ++k) raw[t][k] = reinterpret_cast<const Word*>(src + (off + static_cast<uint32_t>(k * plane)))->v;
                             }
                         }
-                        unsigned char* const item = wlds + min((jb * 64 + lane_s) * 2, g.IT) * 16;
 #pragma unroll
                         for (int t = 0; t < TT; ++t) {
                             sk_u32x4 a, b;
@@ -525,13 +566,19 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
                         }
                     }
                 }
+                return __ballot(any != 0u) != 0ull;
             };
             auto stage_in = [&](int s) __attribute__((always_inline)) {
                 __builtin_amdgcn_wave_barrier();   // the matrix steps of the previous stage have read their operands
                 int lane_s = lane;                 // opaque: the decode below stays here instead of being hoisted out of every loop
                 asm volatile("" : "+v"(lane_s));   // (its results would sit in registers, or in scratch memory, across the matrix loop)
                 if constexpr (IN == kSpkSteps) {
-                    stage_pairs(s, lane_s);
+                    const bool low_terms = SPLIT && s >= low_first;
+                    const int at = low_terms ? s - low_first : s;
+                    if (stage_pairs(at * g.G, low_terms, lane_s) && !low_terms) {
+                        low_groups |= 1ull << (at & 63);
+                        nstages_all = 2 * low_first;
+                    }
                 } else {
 #pragma unroll
                 for (int jb = 0; jb < kSpkSlots; jb += 4) {
@@ -613,15 +660,14 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
             // sets, activation fragments one step ahead through two.
             const int s_first = SK ? wk : 0;
             const int s_step = SK ? WK : 1;
-            int nstages_all = SC ? g.nstages + g.sc_stages : g.nstages;
             // SPLIT: stages of low terms only where the tile's halo has any in this window: bit c8 & 63 of `low_groups` says that channel group
             // c8 has one in the rows of the halo. A lane reads the flags of one group, RR W / 64 of them and one more; the groups of whole
             // images (tiles of several, at most 32 pixels a group) are one short range of flags and run all their low stages or none.
             // Reading whole images for every tile, and running all low stages of an image for one low term in it, took 64 -> 64 at 224^2 114 us
             // without low terms (here 69) and 147 with a single one (76), 512 -> 512 at 112^2 722 (575) and 1231 (579), 64 -> 8 as 1x1 at
             // 640^2, one timestep, 156 (54); 64 -> 64 at 32^2 x 8 is the same, 20 us.
-            uint64_t low_groups = 0;
-            if constexpr (SPLIT) {
+            // Of dense frames a wave finds the low terms of a stage as it brings in the high ones, and runs those of its own stages behind them: bit s & 63 is stage s.
+            if constexpr (SPLIT && IN != kSpkSteps) {
                 const int plane = g.H * g.W;
                 const bool images = g.PI > 1;
                 const int r0 = images ? 0 : max(ih_lo, 0);
@@ -705,9 +751,14 @@ __global__ __launch_bounds__(kSpkWaves * 64, 1) __attribute__((amdgpu_waves_per_
 #pragma clang loop unroll(disable)
                 for (int stage = s_first; stage < nstages_all; stage += s_step) {
                     const bool second = SC && stage >= g.nstages;     // a stage of the shortcut
-                    const bool low = SPLIT && stage >= g.nstages;     // a stage of low activation terms: against the high weight terms alone
-                    const int gg0 = (second || low ? stage - g.nstages : stage) * g.G;
-                    if (SPLIT && low && (low_groups >> (gg0 & 63) & ((1ull << g.G) - 1)) == 0) continue;
+                    const bool low = SPLIT && stage >= low_first;     // a stage of low activation terms: against the high weight terms alone
+                    const int gg0 = (second ? stage - g.nstages : low ? stage - low_first : stage) * g.G;
+                    if constexpr (SPLIT && IN == kSpkSteps) {
+                        // (The waves' shares are of one length here: the last round of stages may have none for a wave.)
+                        if (gg0 >= g.nstages * g.G || (low && (low_groups >> ((stage - low_first) & 63) & 1ull) == 0)) continue;
+                    } else if (SPLIT && low && (low_groups >> (gg0 & 63) & ((1ull << g.G) - 1)) == 0) {
+                        continue;
+                    }
                     const int gpc_l2 = second ? g.sc_gpc_log2 : g.gpc_log2;
                     const int chunk = gg0 >> gpc_l2;
                     const int pbase = chunk * (second ? g.sc_npairs : g.npairs) + ((gg0 - (chunk << gpc_l2)) >> 1);   // pair of (tap 0, the stage's first two groups)
@@ -2091,7 +2142,7 @@ int launch_conv_spk_long(const SpkLaunch& L) {
     return L.fast_epilogue ? run(conv_spk_kernel<XT, TT, IN, true, true, false, false, true>) : run(conv_spk_kernel<XT, TT, IN, true, false, false, false, true>);
 }
 
-// Dense frames per timestep around the dense epilogue.
+// Dense frames per timestep around the dense epilogue (fp32: narrow tiles alone).
 template <typename XT, int TT>
 int launch_conv_spk_steps(const SpkLaunch& L) {
     auto run = [&](auto kernel) -> int {
@@ -2103,8 +2154,9 @@ int launch_conv_spk_steps(const SpkLaunch& L) {
     if constexpr (TT > 4) {
         return run(conv_spk_kernel<XT, TT, kSpkSteps, true, false, false, false, true, true>);
     } else {
-        if (L.g.narrow) return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, kSpkSteps, true, false, false, false, true, true>) : run(conv_spk_kernel<XT, TT, kSpkSteps, false, false, false, false, true, true>);
-        return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, kSpkSteps, true, false, false, false, false, true>) : run(conv_spk_kernel<XT, TT, kSpkSteps, false, false, false, false, false, true>);
+        if (std::is_same<XT, float>::value || L.g.narrow) return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, kSpkSteps, true, false, false, false, true, true>) : run(conv_spk_kernel<XT, TT, kSpkSteps, false, false, false, false, true, true>);
+        if constexpr (!std::is_same<XT, float>::value)
+            return L.g.wk_log2 > 0 ? run(conv_spk_kernel<XT, TT, kSpkSteps, true, false, false, false, false, true>) : run(conv_spk_kernel<XT, TT, kSpkSteps, false, false, false, false, false, true>);
     }
 }
 
@@ -2135,5 +2187,6 @@ int launch_conv_spk_f16_pooled(const SpkLaunch& L, int tt);
 int launch_conv_spk_bf16_frame(const SpkLaunch& L, bool pooled);
 int launch_conv_spk_f16_frame(const SpkLaunch& L, bool pooled);
 int launch_conv_spk_f32(const SpkLaunch& L, int tt);
+int launch_conv_spk_f32_steps(const SpkLaunch& L, int tt);
 
 }  // namespace snnf
