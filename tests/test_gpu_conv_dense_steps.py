@@ -29,6 +29,11 @@ def _run(xs, rs, w, b, zero, s, p, lif):
     (24, 40, 64, 2, 3, 1, 30, 4, BF16, False, LIF, "frames"),      # rows of two pixels
     (24, 40, 64, 1, 3, 1, 40, 4, BF16, False, LIF, "c8"),         # of one: no pairs
     (16, 64, 40, 40, 3, 1, 12, 4, BF16, True, LIF, None),         # a wave a tile
+    (32, 64, 12, 12, 3, 1, 1, 4, BF16, False, SOFT, "frames"),    # few pixels, any neuron
+    (20, 30, 9, 7, 3, 1, 2, 8, F16, True, LIF, "frames"),         # two windows, single channels
+    (40, 64, 14, 13, 5, 1, 1, 2, BF16, False, LIF, "frames"),
+    (72, 40, 11, 1, 3, 1, 3, 4, BF16, True, LIF, "frames"),       # rows of one pixel
+    (512, 64, 7, 7, 3, 1, 1, 4, BF16, False, LIF, "c8"),          # too many channels for a workgroup's loads
     (64, 64, 32, 32, 3, 1, 8, 4, BF16, False, SOFT, "c8"),        # another neuron: the copy
 ])
 def test_against_the_oracle(hip_ops, snnf_lib, Cin, Cout, H, W, k, s, N, T, dtype, residual, lif, route):

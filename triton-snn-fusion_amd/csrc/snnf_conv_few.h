@@ -7,6 +7,7 @@ namespace snnf {
 
 struct FewGeom {
     int N, C8in, H, W, Cout, C8out, KH, KW, sh, sw, ph, pw, Ho, Wo, T;
+    int Cin;
     int taps, kw_mul;            // tap / KW == (tap * kw_mul) >> 16
     int res_layout, out_layout;  // snnf_layout codes; res_layout < 0: no residual
     int pool;                    // 2x2 averages of the spikes leave, in C8

@@ -173,9 +173,12 @@ __global__ __launch_bounds__(kFewThreads, 2) void conv_few_kernel(const StepPtrs
         // ---- the halo of the patch: all channel groups x all steps of the window, four items of a thread in flight. The first ones are requested in front
         // of the weights, so that nothing is waited for behind those.
         const int items = g.Gs * g.region;
-        constexpr int BATCH = IN == SNNF_LAYOUT_BITS ? 4 : 2;
+        // (Of dense frames one item, from eight loads of a channel each.)
+        constexpr int BATCH = IN == SNNF_LAYOUT_BITS ? 4 : (IN == kSpkSteps ? 1 : 2);
         uint32_t okb = 0;
-        typename std::conditional<IN == SNNF_LAYOUT_BITS, uint32_t, sk_u32x4>::type raw[4][BATCH];
+        typename std::conditional<IN == SNNF_LAYOUT_C8, sk_u32x4, uint32_t>::type raw[4][IN == kSpkSteps ? 8 : BATCH];
+        const int in_stride = IN == kSpkSteps ? g.Cin : g.C8in, in_group = IN == kSpkSteps ? 8 : 1;
+        int left = 8;                                  // channels of a dense item's group, and beyond
         auto request = [&](int e0) __attribute__((always_inline)) {
             uint32_t idx[BATCH];
             okb = 0;
@@ -190,8 +193,9 @@ __global__ __launch_bounds__(kFewThreads, 2) void conv_few_kernel(const StepPtrs
                 const int ih = ih_lo + r, iw = iw_lo + rem2 - r * g.RC;
                 const bool ok = static_cast<bool>(static_cast<int>(n0 + ii < g.N) & static_cast<int>(gq < g.C8in) & static_cast<int>(static_cast<unsigned>(ih) < static_cast<unsigned>(g.H)) &
                                                   static_cast<int>(static_cast<unsigned>(iw) < static_cast<unsigned>(g.W)));
-                idx[j] = ok ? static_cast<uint32_t>((((n0 + ii) * g.C8in + gq) * g.H + ih) * g.W + iw) : 0u;
+                idx[j] = ok ? static_cast<uint32_t>((((n0 + ii) * in_stride + gq * in_group) * g.H + ih) * g.W + iw) : 0u;
                 okb |= ok ? 1u << j : 0u;
+                if constexpr (IN == kSpkSteps) left = g.Cin - (ok ? gq * 8 : 0);
             }
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
@@ -200,6 +204,10 @@ __global__ __launch_bounds__(kFewThreads, 2) void conv_few_kernel(const StepPtrs
                         const sk_global_bytes src = (sk_global_bytes)sk_kernarg_ptr(0, t0 + t);
 #pragma unroll
                         for (int j = 0; j < BATCH; ++j) raw[t][j] = src[idx[j]];
+                    } else if constexpr (IN == kSpkSteps) {
+                        const uint16_t* const src = static_cast<const uint16_t*>(sk_kernarg_ptr(0, t0 + t));
+#pragma unroll
+                        for (int k = 0; k < 8; ++k) raw[t][k] = src[idx[0] + static_cast<uint32_t>(min(k, left - 1) * (g.H * g.W))];
                     } else {
                         const sk_u32x4* const src = static_cast<const sk_u32x4*>(sk_kernarg_ptr(0, t0 + t));
 #pragma unroll
@@ -219,6 +227,10 @@ __global__ __launch_bounds__(kFewThreads, 2) void conv_few_kernel(const StepPtrs
                         if constexpr (IN == SNNF_LAYOUT_BITS) {
                             const uint32_t keep = ok ? 0x0c000c00u : 0x0c0c0c0cu;   // byte 0 at bytes 0 and 2, or zeros
                             d = sk_expand_bits<ONE>(__builtin_amdgcn_perm(raw[t][j], raw[t][j], keep));
+                        } else if constexpr (IN == kSpkSteps) {
+#pragma unroll
+                            for (int k = 0; k < 4; ++k)
+                                d[k] = (ok && 2 * k < left ? raw[t][2 * k] : 0u) | (ok && 2 * k + 1 < left ? raw[t][2 * k + 1] << 16 : 0u);
                         } else {
 #pragma unroll
                             for (int k = 0; k < 4; ++k) d[k] = ok ? raw[t][j][k] : 0u;
@@ -432,6 +444,7 @@ bool plan_few(FewGeom& g, const PackGeom& pg, size_t& lds_bytes) {
 }
 
 int launch_conv_few(const FewLaunch& L, bool f16, int in_layout) {
+    if (in_layout == kSpkSteps) return f16 ? launch<f16_t, kSpkSteps>(L) : launch<bf16_t, kSpkSteps>(L);
     if (in_layout == SNNF_LAYOUT_BITS) return f16 ? launch<f16_t, SNNF_LAYOUT_BITS>(L) : launch<bf16_t, SNNF_LAYOUT_BITS>(L);
     return f16 ? launch<f16_t, SNNF_LAYOUT_C8>(L) : launch<bf16_t, SNNF_LAYOUT_C8>(L);
 }

@@ -421,7 +421,7 @@ int plan_window(const char* who, const BlockedCall& c, BlockedPlan& p, int windo
     // all, so that the pooled launch has the sums of the unpooled one.
     if (neuron && !c.split && !shared && sc == nullptr && c.x_layout != kSpkSteps && wk_log2 > 0 && !p.tuned_patch && !p.tuned_split && (c.out_layout != SNNF_LAYOUT_C8 || pool2) && c.res_layout != SNNF_LAYOUT_C8) {
         FewGeom& f = p.few_g;
-        f.N = N; f.C8in = g.C8in; f.H = H; f.W = W; f.Cout = Cout; f.C8out = g.C8out; f.KH = KH; f.KW = KW;
+        f.N = N; f.Cin = Cin; f.C8in = g.C8in; f.H = H; f.W = W; f.Cout = Cout; f.C8out = g.C8out; f.KH = KH; f.KW = KW;
         f.sh = stride_h; f.sw = stride_w; f.ph = pad_h; f.pw = pad_w; f.Ho = g.Ho; f.Wo = g.Wo; f.T = T;
         f.taps = g.taps; f.kw_mul = g.kw_mul;
         f.res_layout = c.res_layout; f.out_layout = c.out_layout; f.pool = pool2 ? 1 : 0;
@@ -489,6 +489,11 @@ bool reads_steps(const BlockedPlan& p, int T, bool split) {
     return 2.7 + 0.28 * megabytes > loads * (0.0036 + (p.wk_log2 == 0 ? 0.0052 : 0.0) + (g.PC < 8 ? 0.0018 : 0.0));
 }
 
+// The same for the kernel of few pixels: a workgroup's threads bring in its halo item by item, eight loads each, which takes what the copy does at some 2300 items of all timesteps.
+// Workgroups of one column fragment, the smallest launches: the others keep the copy.
+// us, copy / here, 47 layers: 32 -> 64 at 12^2, T = 4 7.7 / 5.9 (256 items), 128 -> 256 at 8^2 8.1 / 6.9 (1024), 128 -> 256 at 8^2, T = 8 10.4 / 10.0 (2048); 512 -> 512 at 2^2 10.9 / 12.7 (4096), at 7^2 12.2 / 16.6 (6912).
+bool few_reads_steps(const BlockedPlan& p, bool split) { return p.few && !split && p.few_g.frags == 1 && static_cast<int64_t>(p.few_g.Gs) * p.few_g.region * p.few_g.T <= 2304; }
+
 const char* family_name(DenseFamily f) {
     return f == DenseFamily::kTInM ? "t_in_m" : (f == DenseFamily::kTimeOuter ? "time_outer" : (f == DenseFamily::kPointwise ? "pointwise" : "matrix"));
 }
@@ -520,6 +525,7 @@ using RouteKey = std::array<int, 16>;
 struct KeptPlan {
     BlockedPlan plan;
     char text[2][256];                                 // with the general and with the dense epilogue
+    bool few_steps;                                    // the kernel for few pixels reads the dense frames itself (`few_reads_steps`)
     BlockedPlan steps;                                 // of the kernel on the dense frames themselves, where the dense epilogue applies (see `reads_steps`; grid 0: never)
     char steps_text[256];
 };
@@ -569,7 +575,9 @@ Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, 
                                    nullptr, split}, plan) == SNNF_OK &&
                       (frame || weigh == 0.0 || fills_waves(plan, weigh, T, Cout));
         if (route.taken) {
-            for (int dense_epi = 0; dense_epi < 2; ++dense_epi) plan_text(kept->text[dense_epi], plan, family_name(route.family), dense_epi ? 40 : 0, frame ? T : plan.tt, frame ? kFrameRoute : kCopyRoute);
+            for (int dense_epi = 0; dense_epi < 2; ++dense_epi) plan_text(kept->text[dense_epi], plan, family_name(route.family), dense_epi ? 40 : 0, frame ? T : plan.tt,
+                                                                                  frame ? kFrameRoute : (few_reads_steps(plan, split) ? kStepsRoute : kCopyRoute));
+            kept->few_steps = !frame && few_reads_steps(plan, split);
             if (!frame && neuron && !plan.few) {
                 BlockedPlan direct;
                 if (plan_blocked("snnf_conv_lif", BlockedCall{T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, kSpkSteps, residual ? SNNF_LAYOUT_NCHW : -1,
@@ -834,14 +842,15 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     // (Of a dense call xs are the C8 buffers; a wave's K, stages and sums don't depend on which of the two it reads.)
     const LifParams lif_params = make_lif_params(v_threshold, v_reset, tau);
     const bool usual = lif_params.charge_mode == CHARGE_SCALE && lif_params.inv_tau == 0.5f && !lif_params.soft_reset;
-    const bool steps = dense != nullptr && dense->xs != nullptr && dense->kept->steps.grid > 0 && usual && v_out != nullptr &&
-                       std::all_of(dense->xs, dense->xs + T, [x_dtype](const void* x) { return aligned_to(x, dtype_size(x_dtype)); });
+    const bool frames = dense != nullptr && dense->xs != nullptr && std::all_of(dense->xs, dense->xs + T, [x_dtype](const void* x) { return aligned_to(x, dtype_size(x_dtype)); });
+    const bool steps = frames && dense->kept->steps.grid > 0 && usual && v_out != nullptr;
+    const bool few_steps = frames && dense->kept->few_steps;
     const BlockedPlan& p = dense == nullptr ? made : (steps ? dense->kept->steps : dense->kept->plan);
     const SpkGeom& g = p.g;
 
     SpkLaunch L = {};
     for (int t = 0; t < T; ++t) {
-        L.xs.p[t] = steps ? dense->xs[t] : xs[t];
+        L.xs.p[t] = steps || few_steps ? dense->xs[t] : xs[t];
         if (residuals != nullptr) L.residuals.p[t] = residuals[t];
         if (sc != nullptr) L.residuals.p[t] = sc->xs[t];   // the second input travels in the residual's place (a shortcut launch has no residual)
     }
@@ -882,7 +891,7 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     L.dense_epilogue = dense_epi;
     if (steps && split) return launch_conv_spk_f32_steps(L, p.tt);
     if (steps) return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_steps(L, p.tt) : launch_conv_spk_f16_steps(L, p.tt);
-    if (dense != nullptr && dense->xs != nullptr) {   // the plan stands: bring the dense inputs into the C8 buffers behind `xs`
+    if (dense != nullptr && dense->xs != nullptr && !few_steps) {   // the plan stands: bring the dense inputs into the C8 buffers behind `xs`
         StepPtrs from = {};
         for (int t = 0; t < T; ++t) from.p[t] = dense->xs[t];
         char* const base = static_cast<char*>(const_cast<void*>(xs[0]));
@@ -905,7 +914,7 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
         F.g.out_step_stride = out_step_stride;
         F.g.v16 = L.g.v16;
         F.g.v_in_place = L.g.v_in_place;
-        return launch_conv_few(F, x_dtype == SNNF_F16, x_layout);
+        return launch_conv_few(F, x_dtype == SNNF_F16, few_steps ? kSpkSteps : x_layout);
     }
     if (pool2) {
         if (x_layout == SNNF_LAYOUT_NCHW) return x_dtype == SNNF_BF16 ? launch_conv_spk_bf16_frame(L, true) : launch_conv_spk_f16_frame(L, true);
