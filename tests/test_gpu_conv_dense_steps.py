@@ -97,6 +97,33 @@ def test_fp32_terms_against_the_oracle(hip_ops, snnf_lib, Cin, Cout, H, W, k, s,
         assert int(changed.sum()) > 0 and int(changed[:N - 1].sum()) == 0
 
 
+@pytest.mark.parametrize("Cin,Cout,H,k,s,N,T", [
+    (27, 328, 15, 7, 2, 5, 4),       # whose frames would take two windows where the copy takes one
+    (72, 104, 27, 3, 1, 2, 6),       # two of each
+    (64, 64, 24, 3, 1, 4, 5),        # one of six
+    (48, 40, 20, 5, 1, 6, 3),
+])
+def test_scratch_memory_is_not_left(hip_ops, snnf_lib, Cin, Cout, H, k, s, N, T):
+    """A 16-bit membrane passes from window to window in the scratch memory that the query asks for: what lies behind it stays as it was."""
+    from triton_snn_fusion_amd import _lib
+    from triton_snn_fusion_amd.runtime import hip_convlif_backend as CB
+    g = gen(9380 + Cin)
+    p, code = k // 2, _lib.dtype_code(F16)
+    Ho = (H + 2 * p - k) // s + 1
+    x = [spikes((N, Cin, H, H), 0.25, g) for _ in range(T)]
+    xs = [dev(t, F16) for t in x]
+    w, b = q(torch.randn(Cout, Cin, k, k, generator=g) * 2.0 * (2.0 / (Cin * k * k)) ** 0.5, F16), q(torch.randn(Cout, generator=g) * 0.1, F16)
+    packed = CB._packed_weight(dev(w, F16), dev(b, F16), F16)
+    need = snnf_lib.snnf_conv_lif_scratch_bytes(T, N, Cin, H, H, code, Cout, k, k, s, s, p, p, code, 0)
+    room = torch.full((need + N * Cout * Ho * Ho * 4 + 4096,), 171, dtype=torch.uint8, device=DEV)      # (a whole fp32 membrane behind it)
+    sp, v = torch.empty(T, N, Cout, Ho, Ho, device=DEV, dtype=F16), torch.empty(N, Cout, Ho, Ho, device=DEV, dtype=F16)
+    _lib.check("ws", snnf_lib.snnf_conv_lif_ws(_lib.step_pointers(xs), None, T, N, Cin, H, H, code, packed.data_ptr(), Cout, k, k, s, s, p, p, None, code,
+                                               sp.data_ptr(), int(sp.stride(0)), v.data_ptr(), *LIF, room.data_ptr(), need, _lib.current_stream(sp.device)))
+    assert CB.last_conv_plan().get("ran") == "blocked"
+    assert int((room[need:] != 171).sum()) == 0
+    check(sp, v, O.temporal_conv_lif(x, w, b, torch.tensor(0.0), (s, s), (p, p), (1, 1), 1, *LIF), v_dtype=F16)
+
+
 def test_infinities_stay_in_their_windows(hip_ops, snnf_lib):
     """An infinity in the last channel of an image reaches its own windows and no neighbour's: pixels outside the image and channels beyond the last are zeros."""
     g = gen(9390)

@@ -581,7 +581,8 @@ Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, 
             if (!frame && neuron && !plan.few) {
                 BlockedPlan direct;
                 if (plan_blocked("snnf_conv_lif", BlockedCall{T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, kSpkSteps, residual ? SNNF_LAYOUT_NCHW : -1,
-                                 SNNF_LAYOUT_NCHW, 0, false, true, false, true, false, nullptr, split}, direct) == SNNF_OK && reads_steps(direct, T, split)) {
+                                 SNNF_LAYOUT_NCHW, 0, false, true, false, true, false, nullptr, split}, direct) == SNNF_OK && reads_steps(direct, T, split) &&
+                    direct.windows <= std::max(plan.windows, plan.tt > 4 ? 2 : 1)) {   // (the scratch memory holds what passes from window to window of `plan`)
                     kept->steps = direct;
                     plan_text(kept->steps_text, direct, family_name(route.family), 40, direct.tt, kStepsRoute);
                 }
@@ -843,7 +844,8 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     const LifParams lif_params = make_lif_params(v_threshold, v_reset, tau);
     const bool usual = lif_params.charge_mode == CHARGE_SCALE && lif_params.inv_tau == 0.5f && !lif_params.soft_reset;
     const bool frames = dense != nullptr && dense->xs != nullptr && std::all_of(dense->xs, dense->xs + T, [x_dtype](const void* x) { return aligned_to(x, dtype_size(x_dtype)); });
-    const bool steps = frames && dense->kept->steps.grid > 0 && usual && v_out != nullptr;
+    const bool steps = frames && dense->kept->steps.grid > 0 && usual && v_out != nullptr &&
+                       (dense->kept->steps.windows == 1 || dense->v_dtype == SNNF_F32 || x_dtype == SNNF_F32 || dense->space.total > dense->space.carry);
     const bool few_steps = frames && dense->kept->few_steps;
     const BlockedPlan& p = dense == nullptr ? made : (steps ? dense->kept->steps : dense->kept->plan);
     const SpkGeom& g = p.g;
