@@ -282,8 +282,11 @@ int plan_window(const char* who, const BlockedCall& c, BlockedPlan& p, int windo
     g.out_step_stride = c.out_step_stride;
 
     // Timesteps side by side: 4 (2 for T == 2, 1 for a single step or a shared frame, 3 where that takes no more windows), fewer when the halo does not fit.
+    // Where four don't fit, three only do with few pixels a tile, and two it is (160 -> 40 7x7 stride 2 at 21^2 x 29, T = 6 in patches of 11 x 1 77 us, of 2 x 11 55).
     int& tt = p.tt;
-    tt = window > 0 ? window : (shared || T == 1 ? 1 : (T == 2 ? 2 : (!pool2 && threes(T) ? 3 : 4)));
+    SpkPlan fours;
+    const bool three = !shared && !pool2 && threes(T) && plan_spk(g, 4, fours);
+    tt = window > 0 ? window : (shared || T == 1 ? 1 : (T == 2 ? 2 : (three ? 3 : 4)));
     TunedPlan tuned = {0, 0, 0};
     if (!c.split) {   // (measured on 16-bit activations)
         const TunedKey key = {T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, shared ? 1 : 0};
