@@ -492,6 +492,136 @@ int launch_direct(const StepPtrs& xs, const StepPtrs& res, int has_res, int T, c
 }
 
 // ---------------------------------------------------------------------------------------------------------------
+// Stride 1, 16-bit rows of any length from 8 on that start anywhere, without LDS: a lane has 8 outputs of a row and reads 16 bytes (at any even address) and the element on
+// either side of each of the three input rows, no matter where these lie against whole vectors. The last strip of a row ends with it: it computes outputs of the strip before
+// as well, from the same operands in the same order, and both write the same bits (so the initial membrane may not lie where the final one goes). The taps are
+// the fp32 multiply-adds of `dwconv3x3_lif_kernel`, whose strips of one pixel (of four where rows are a multiple of that) take these rows otherwise: an element at a time into LDS and back.
+// What bounds it: HBM from some 100 MB on, below that the chain of a lane's loads. 50 drawn layers of such rows: 1.39 times in the mean, the smallest 0.88 (295 channels at 100 x 13 x 7, T = 8 34.6 -> 39.5 us,
+// whose rows of 13 take two strips); 264 channels at 23^2 x 27, T = 3 45.8 -> 20.8, 88 at 78^2 x 8, T = 1 26.8 -> 10.1 (floor 6.6), 88 at 65^2 x 31, T = 4 91.5 -> 59.5 (44.6),
+// 56 at 66^2 x 23 46.4 -> 22.6, 272 at 100^2 x 3 49.0 -> 33.9 (31.6), 64 at 17^2 x 16 7.0 -> 5.6, 88 at 17^2 x 2, T = 5 5.3 -> 5.8.
+// The two pointer tables MUST be the first two kernel parameters.
+// ---------------------------------------------------------------------------------------------------------------
+template <typename XT, typename VT, bool STD>
+__global__ __launch_bounds__(kThreads) void dwconv3x3_lif_rows_kernel(StepPtrs xs, StepPtrs residuals, int has_residual, int T, DwDirect g,
+                                                                      const XT* __restrict__ weight, const XT* __restrict__ bias,
+                                                                      const VT* v_init, XT* spikes, int64_t spike_step_stride, VT* v_out, LifParams lif) {
+    constexpr int PX = 8;
+    struct __attribute__((packed, aligned(2))) Row { uint32_t d[4]; };
+    struct __attribute__((packed, aligned(2))) Out { XT v[PX]; };
+    struct __attribute__((packed, aligned(sizeof(VT)))) Membrane { VT v[PX]; };
+    const int i = static_cast<int>(blockIdx.x) * kThreads + static_cast<int>(threadIdx.x);
+    if (i >= g.strips) return;
+    const int row = fast_div(i, g.d_SW);
+    const int strip = i - row * g.SW;
+    const int plane = fast_div(row, g.d_Ho);
+    const int oh = row - plane * g.Ho;
+    const int c = plane - fast_div(plane, g.d_C) * g.C;
+    const int c0 = min(strip * PX, g.W - PX);
+    const uint32_t out = static_cast<uint32_t>(row) * static_cast<uint32_t>(g.W) + static_cast<uint32_t>(c0);       // elements
+    const bool has_left = c0 > 0, has_right = c0 + PX < g.W;
+    // Rows above and below the plane are read from the row itself and dropped.
+    const bool up = oh > 0, down = oh + 1 < g.H;
+    const uint32_t at[3] = {up ? out - static_cast<uint32_t>(g.W) : out, out, down ? out + static_cast<uint32_t>(g.W) : out};
+    Row x[3];
+    uint16_t xl[3], xr[3];
+    Out res = {};
+    auto issue_loads = [&](int t) __attribute__((always_inline)) {
+        const uint16_t* __restrict__ src = static_cast<const uint16_t*>(dw_table_entry(0, t));
+#pragma unroll
+        for (int kh = 0; kh < 3; ++kh) {
+            x[kh] = *reinterpret_cast<const Row*>(src + at[kh]);
+            xl[kh] = src[has_left ? at[kh] - 1u : at[kh]];
+            xr[kh] = src[has_right ? at[kh] + static_cast<uint32_t>(PX) : at[kh]];
+        }
+        if (has_residual) res = *reinterpret_cast<const Out*>(static_cast<const XT*>(dw_table_entry(sizeof(StepPtrs), t)) + out);
+    };
+    issue_loads(0);
+    float w[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) w[k] = to_float(weight[c * 9 + k]);
+    const float b = to_float(bias[c]);
+    float v[PX];
+    if (v_init != nullptr) {
+        const Membrane start = *reinterpret_cast<const Membrane*>(v_init + out);
+#pragma unroll
+        for (int j = 0; j < PX; ++j) v[j] = to_float(start.v[j]);
+    } else {
+#pragma unroll
+        for (int j = 0; j < PX; ++j) v[j] = 0.0f;
+    }
+    for (int t = 0; t < T; ++t) {
+        float acc[PX];
+#pragma unroll
+        for (int j = 0; j < PX; ++j) acc[j] = b;
+#pragma unroll
+        for (int kh = 0; kh < 3; ++kh) {
+            const bool there = kh == 0 ? up : (kh == 2 ? down : true);
+            float in[PX + 2];                     // input columns c0 - 1 .. c0 + 8
+            in[0] = there && has_left ? to_float(XT{xl[kh]}) : 0.0f;
+            in[PX + 1] = there && has_right ? to_float(XT{xr[kh]}) : 0.0f;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const uint32_t d = there ? x[kh].d[k] : 0u;
+                in[1 + 2 * k] = low_element<XT>(d);
+                in[2 + 2 * k] = high_element<XT>(d);
+            }
+#pragma unroll
+            for (int j = 0; j < PX; ++j)
+#pragma unroll
+                for (int kw = 0; kw < 3; ++kw) acc[j] = fmaf(in[j + kw], w[kh * 3 + kw], acc[j]);
+        }
+        if (has_residual) {
+#pragma unroll
+            for (int j = 0; j < PX; ++j) acc[j] += to_float(res.v[j]);
+        }
+        if (t + 1 < T) issue_loads(t + 1);
+        Out o;
+#pragma unroll
+        for (int j = 0; j < PX; ++j) {
+            bool fired;
+            if constexpr (STD) {
+                const float h = v[j] + (acc[j] - v[j]) * lif.inv_tau;
+                fired = h >= lif.v_threshold;
+                v[j] = fired ? lif.v_reset : h;
+            } else {
+                fired = lif_step(acc[j], v[j], lif);
+            }
+            o.v[j] = spike_value<XT>(fired);
+        }
+        *reinterpret_cast<Out*>(spikes + t * spike_step_stride + out) = o;
+    }
+    Membrane end;
+#pragma unroll
+    for (int j = 0; j < PX; ++j) end.v[j] = from_float<VT>(v[j]);
+    *reinterpret_cast<Membrane*>(v_out + out) = end;
+}
+
+template <typename XT, typename VT>
+int launch_rows(const StepPtrs& xs, const StepPtrs& res, int has_res, int T, const DwGeom& g, const void* weight, const void* bias, const void* v_init,
+                void* spikes, int64_t spike_step_stride, void* v_out, const LifParams& lif, hipStream_t stream) {
+    DwDirect d = {};
+    d.C = g.C;
+    d.H = g.H;
+    d.W = g.W;
+    d.Ho = g.Ho;
+    d.SW = (g.W + 7) / 8;
+    d.strips = g.planes * g.Ho * d.SW;
+    d.d_SW = make_fast_div(d.SW);
+    d.d_Ho = make_fast_div(d.Ho);
+    d.d_C = make_fast_div(d.C);
+    const dim3 grid((static_cast<unsigned>(d.strips) + kThreads - 1) / kThreads);
+    auto kernel = lif.charge_mode == CHARGE_SCALE && !lif.soft_reset ? dwconv3x3_lif_rows_kernel<XT, VT, true> : dwconv3x3_lif_rows_kernel<XT, VT, false>;
+    kernel<<<grid, kThreads, 0, stream>>>(xs, res, has_res, T, d, static_cast<const XT*>(weight), static_cast<const XT*>(bias),
+                                          static_cast<const VT*>(v_init), static_cast<XT*>(spikes), spike_step_stride, static_cast<VT*>(v_out), lif);
+    return check_launch("snnf_dwconv3x3_lif");
+}
+
+// Which calls the kernel of any rows takes (see there).
+bool takes_rows(const DwGeom& g, const void* v_init, const void* v_out) {
+    return g.W >= 8 && v_init != v_out && static_cast<int64_t>(g.planes) * g.H * g.W * 2 <= kDirectMaxFrame;
+}
+
+// ---------------------------------------------------------------------------------------------------------------
 // Stride 1, strips of 8 pixels, 16-bit activations: the LDS tile keeps the activations in their 16-bit form (a prefetched
 // vector goes in with one 16-byte write and no conversion) and the taps run on the packed dot-product instruction
 // (two 16-bit products added to an fp32 accumulator): the products are exact in fp32, as with an fp32 multiply-add, and an
@@ -781,6 +911,9 @@ int dispatch_px(int px, bool direct, const StepPtrs& xs, const StepPtrs& res, in
                 if (static_cast<int64_t>(g.planes) * g.H * (g.W / 8) > direct_strips()) return launch_dot<XT, VT>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
             }
             return launch_direct<XT, VT, STRIDE>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
+        }
+        if constexpr (STRIDE == 1) {
+            if (takes_rows(g, v_init, v_out)) return launch_rows<XT, VT>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
         }
     } else if (px == 8) {
         return launch<XT, VT, STRIDE, 8>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
