@@ -33,6 +33,9 @@ def _run(xs, rs, w, b, zero, s, p, lif):
     (20, 30, 9, 7, 3, 1, 2, 8, F16, True, LIF, "frames"),         # two windows, single channels
     (40, 64, 14, 13, 5, 1, 1, 2, BF16, False, LIF, "frames"),
     (72, 40, 11, 1, 3, 1, 3, 4, BF16, True, LIF, "frames"),       # rows of one pixel
+    (96, 104, 33, 31, 1, 1, 4, 2, BF16, True, LIF, "frames"),     # 1x1 of two timesteps
+    (96, 104, 33, 31, 1, 1, 4, 2, BF16, True, SOFT, None),        # and on the dense kernels for another neuron
+    (136, 32, 68, 11, 1, 1, 9, 1, F16, False, LIF, "frames"),
     (512, 64, 7, 7, 3, 1, 1, 4, BF16, False, LIF, "c8"),          # too many channels for a workgroup's loads
     (64, 64, 32, 32, 3, 1, 8, 4, BF16, False, SOFT, "c8"),        # another neuron: the copy
 ])

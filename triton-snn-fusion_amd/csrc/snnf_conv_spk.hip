@@ -136,7 +136,7 @@ bool threes(int T) { return T > 2 && (T + 2) / 3 == (T + 3) / 4; }
 // * The matrix kernel's masked variant (planes or channels its tiles do not divide) goes in windows of two timesteps and pays a pass over
 //   the weights per window: 600 layers gain a factor of 2 (72 -> 104 at 27 x 35, T = 6, with a residual 59 / 39, 512 -> 512 at 7^2 x 16 55 / 31,
 //   16 -> 96 at 25^2 x 8 with a residual 25 / 23, 24 -> 16 at 26^2, 5x5, T = 5 64 / 31). Of one or two timesteps, one window there as well, 1x1
-//   layers of any size lose (256 -> 128 at 97^2 x 16, T = 1 115 / 146, 128 -> 256 stride 2 at 28^2 x 52, T = 1 18 / 24) and so do large strided
+//   layers of any size lose with the copy (256 -> 128 at 97^2 x 16, T = 1 115 / 146, 128 -> 256 stride 2 at 28^2 x 52, T = 1 18 / 24) and so do large strided
 //   ones (64 -> 128 at 40^2 x 17, T = 2 16 / 19); 1x1 layers of a stride copy four pixels for one (168 -> 349 at 24 x 75 x 14, T = 6 104 / 123).
 // * The pointwise kernel's straight-line variant takes planes of whole tiles of 64 pixels: 24 -> 96 at 56^2 x 32 31 / 73, 128 -> 256 89 / 224.
 //   Its general variant is several times slower and loses over 260 layers to a factor of 1.8 (128 -> 64 at 7^2, T = 8 60 / 16, 64 -> 256 at
@@ -162,6 +162,7 @@ bool threes(int T) { return T > 2 && (T + 2) / 3 == (T + 3) / 4; }
 //   0.80 / 0.65; 32 -> 192 at 56^2 1.90 / 1.55, 256 -> 512 at 24^2 x 5, T = 12 4.46 / 2.73), and others of one or two steps and many outputs (192 -> 256
 //   at 28^2 x 12, T = 2 0.89 / 0.69; 192 -> 128 x 3 1.37 / 1.12).
 // Without a neuron the lines are those of sums that leave as 16-bit values (512 -> 512 at 7^2 x 16 56 / 35).
+// `weigh`: above zero a layer only moves where `fills_waves` says so, below only where the kernel reads the dense frames itself.
 bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w,
                          int v_dtype, bool residual, bool neuron, DenseFamily& family, double& weigh) {
     weigh = 0.0;
@@ -192,6 +193,11 @@ bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int C
         case DenseFamily::kTimeOuter: return !pointwise || static_cast<int64_t>(T) * N * (Cin + Cout) * plane <= (1 << 25);
         case DenseFamily::kPointwise: return plane % 64 != 0 || (Cout % 32 != 0 && outs <= (1 << 22));
         case DenseFamily::kMatrixMasked:
+            // One or two timesteps of a 1x1 layer of stride 1 move where the kernel reads the frames itself: 17 layers, 1.82 in the mean, one loses 10 % (us, dense / here, 360 -> 24 at 13 x 48 x 17, T = 2
+            // 26.2 / 8.1, 136 -> 16 at 68 x 11 x 20, T = 1 13.1 / 7.2, 144 -> 205 at 12 x 54 x 28, T = 1 28.7 / 20.6, 216 -> 88 at 52^2 x 28, T = 2 55.4 / 61.8; of five that
+            // keep the copy 464 -> 164 at 34 x 33 x 9, T = 1 21.3 / 34.1).
+            if (pointwise && T <= 2 && outs > (1 << 17)) weigh = -1.0;
+            if (pointwise && T <= 2) return true;
             if (one) return T <= 2 ? outs <= (1 << 17) : !strided || inputs <= (1 << 24);
             return T > 2 || K >= 1152 || !strided || outs <= (3 << 19);
         case DenseFamily::kMatrixWhole:
@@ -531,6 +537,7 @@ struct KeptPlan {
     bool few_steps;                                    // the kernel for few pixels reads the dense frames itself (`few_reads_steps`)
     BlockedPlan steps;                                 // of the kernel on the dense frames themselves, where the dense epilogue applies (see `reads_steps`; grid 0: never)
     char steps_text[256];
+    bool steps_only;                                   // a call that doesn't read its frames stays on the dense kernels
 };
 struct Route { bool taken; DenseFamily family; std::shared_ptr<const KeptPlan> kept; };
 std::mutex routes_mutex;
@@ -576,7 +583,7 @@ Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, 
         route.taken = plan_blocked("snnf_conv_lif_scratch_bytes", BlockedCall{T, N, Cin, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w,
                                    frame ? SNNF_LAYOUT_NCHW : SNNF_LAYOUT_C8, residual ? SNNF_LAYOUT_NCHW : -1, SNNF_LAYOUT_NCHW, 0, frame, neuron, false, neuron, false,
                                    nullptr, split}, plan) == SNNF_OK &&
-                      (frame || weigh == 0.0 || fills_waves(plan, weigh, T, Cout));
+                      (frame || weigh <= 0.0 || fills_waves(plan, weigh, T, Cout));
         if (route.taken) {
             for (int dense_epi = 0; dense_epi < 2; ++dense_epi) plan_text(kept->text[dense_epi], plan, family_name(route.family), dense_epi ? 40 : 0, frame ? T : plan.tt,
                                                                                   frame ? kFrameRoute : (few_reads_steps(plan, split) ? kStepsRoute : kCopyRoute));
@@ -590,7 +597,9 @@ Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, 
                     plan_text(kept->steps_text, direct, family_name(route.family), 40, direct.tt, kStepsRoute);
                 }
             }
-            route.kept = kept;
+            kept->steps_only = weigh < 0.0;
+            if (kept->steps_only && kept->steps.grid == 0) route.taken = false;
+            else route.kept = kept;
         }
     }
     std::lock_guard<std::mutex> lock(routes_mutex);
@@ -705,6 +714,9 @@ extern "C" size_t snnf_conv_bias_workspace_bytes(int T, int N, int Cin, int H, i
 
 namespace snnf {
 namespace {
+// The neuron of the dense epilogue.
+bool usual_neuron(const LifParams& lif) { return lif.charge_mode == CHARGE_SCALE && lif.inv_tau == 0.5f && !lif.soft_reset; }
+
 // One dense 16-bit frame of at most eight channels for all timesteps (the first layer of a network) around the usual neuron (tau 2, hard reset) goes to the
 // blocked kernel, which reads the frame as it is and needs no scratch memory (us, matrix kernel / here, T = 4, bf16): 3 -> 64 7x7 stride 2 at 224^2 x 16 62.8 / 48.5, one
 // image 14.6 / 9.9, 3x3 at 32^2 x 64 19.7 / 14.2, one image 11.5 / 6.9, 3 -> 32 stride 2 at 128^2 x 32 33.3 / 14.6, 1 -> 64 5x5 at 28^2 x 50 18.6 / 14.6, 4 -> 96 at 50^2 x 20
@@ -713,7 +725,7 @@ namespace {
 // (77.5 at 224^2 x 16), and stay.
 bool takes_frame(bool shared, int T, int Cin, int x_dtype, int v_dtype, bool residual, const LifParams& lif) {
     return shared && T <= SNNF_MAX_T_PER_LAUNCH && Cin <= 8 && (x_dtype == SNNF_BF16 || x_dtype == SNNF_F16) && v_dtype == SNNF_F32 && !residual &&
-           lif.charge_mode == CHARGE_SCALE && lif.inv_tau == 0.5f && !lif.soft_reset;
+           usual_neuron(lif);
 }
 
 // The blocked route of a call on dense tensors: SNNF_ERR_UNSUPPORTED (nothing enqueued) when it does not apply.
@@ -740,6 +752,7 @@ int run_blocked_route(const void* const* xs, const void* const* residuals, int T
     if (workspace == nullptr || !aligned_to(workspace, 16) || shared) return SNNF_ERR_UNSUPPORTED;   // one frame for all timesteps is convolved once on the dense kernels too
     const Route taken = blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residuals != nullptr, neuron != 0);
     if (!taken.taken) return SNNF_ERR_UNSUPPORTED;
+    if (taken.kept->steps_only && !usual_neuron(make_lif_params(v_threshold, v_reset, tau))) return SNNF_ERR_UNSUPPORTED;
     const RouteSpace space = route_space(T, N, Cin, H, W, x_dtype == SNNF_F32,
                                          neuron ? carried_membrane(taken, v_dtype, N, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w) : 0);
     if (workspace_bytes < space.total) return SNNF_ERR_UNSUPPORTED;
@@ -845,7 +858,7 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     }
     // (Of a dense call xs are the C8 buffers; a wave's K, stages and sums don't depend on which of the two it reads.)
     const LifParams lif_params = make_lif_params(v_threshold, v_reset, tau);
-    const bool usual = lif_params.charge_mode == CHARGE_SCALE && lif_params.inv_tau == 0.5f && !lif_params.soft_reset;
+    const bool usual = usual_neuron(lif_params);
     const bool frames = dense != nullptr && dense->xs != nullptr && std::all_of(dense->xs, dense->xs + T, [x_dtype](const void* x) { return aligned_to(x, dtype_size(x_dtype)); });
     const bool steps = frames && dense->kept->steps.grid > 0 && usual && v_out != nullptr &&
                        (dense->kept->steps.windows == 1 || dense->v_dtype == SNNF_F32 || x_dtype == SNNF_F32 || dense->space.total > dense->space.carry);
