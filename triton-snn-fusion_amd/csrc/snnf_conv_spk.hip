@@ -715,7 +715,7 @@ extern "C" size_t snnf_conv_bias_workspace_bytes(int T, int N, int Cin, int H, i
 namespace snnf {
 namespace {
 // The neuron of the dense epilogue.
-bool usual_neuron(const LifParams& lif) { return lif.charge_mode == CHARGE_SCALE && lif.inv_tau == 0.5f && !lif.soft_reset; }
+bool dense_epilogue_neuron(const LifParams& lif) { return lif.charge_mode == CHARGE_SCALE && lif.inv_tau == 0.5f && !lif.soft_reset; }
 
 // One dense 16-bit frame of at most eight channels for all timesteps (the first layer of a network) around the usual neuron (tau 2, hard reset) goes to the
 // blocked kernel, which reads the frame as it is and needs no scratch memory (us, matrix kernel / here, T = 4, bf16): 3 -> 64 7x7 stride 2 at 224^2 x 16 62.8 / 48.5, one
@@ -725,7 +725,7 @@ bool usual_neuron(const LifParams& lif) { return lif.charge_mode == CHARGE_SCALE
 // (77.5 at 224^2 x 16), and stay.
 bool takes_frame(bool shared, int T, int Cin, int x_dtype, int v_dtype, bool residual, const LifParams& lif) {
     return shared && T <= SNNF_MAX_T_PER_LAUNCH && Cin <= 8 && (x_dtype == SNNF_BF16 || x_dtype == SNNF_F16) && v_dtype == SNNF_F32 && !residual &&
-           usual_neuron(lif);
+           dense_epilogue_neuron(lif);
 }
 
 // The blocked route of a call on dense tensors: SNNF_ERR_UNSUPPORTED (nothing enqueued) when it does not apply.
@@ -752,7 +752,7 @@ int run_blocked_route(const void* const* xs, const void* const* residuals, int T
     if (workspace == nullptr || !aligned_to(workspace, 16) || shared) return SNNF_ERR_UNSUPPORTED;   // one frame for all timesteps is convolved once on the dense kernels too
     const Route taken = blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residuals != nullptr, neuron != 0);
     if (!taken.taken) return SNNF_ERR_UNSUPPORTED;
-    if (taken.kept->steps_only && !usual_neuron(make_lif_params(v_threshold, v_reset, tau))) return SNNF_ERR_UNSUPPORTED;
+    if (taken.kept->steps_only && !dense_epilogue_neuron(make_lif_params(v_threshold, v_reset, tau))) return SNNF_ERR_UNSUPPORTED;
     const RouteSpace space = route_space(T, N, Cin, H, W, x_dtype == SNNF_F32,
                                          neuron ? carried_membrane(taken, v_dtype, N, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w) : 0);
     if (workspace_bytes < space.total) return SNNF_ERR_UNSUPPORTED;
@@ -858,7 +858,7 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     }
     // (Of a dense call xs are the C8 buffers; a wave's K, stages and sums don't depend on which of the two it reads.)
     const LifParams lif_params = make_lif_params(v_threshold, v_reset, tau);
-    const bool usual = usual_neuron(lif_params);
+    const bool usual = dense_epilogue_neuron(lif_params);
     const bool frames = dense != nullptr && dense->xs != nullptr && std::all_of(dense->xs, dense->xs + T, [x_dtype](const void* x) { return aligned_to(x, dtype_size(x_dtype)); });
     const bool steps = frames && dense->kept->steps.grid > 0 && usual && v_out != nullptr &&
                        (dense->kept->steps.windows == 1 || dense->v_dtype == SNNF_F32 || x_dtype == SNNF_F32 || dense->space.total > dense->space.carry);

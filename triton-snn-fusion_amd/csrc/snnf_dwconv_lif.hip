@@ -1112,8 +1112,8 @@ extern "C" int snnf_dwconv3x3_lif(const void* const* xs, const void* const* resi
             if (residuals != nullptr) rp.p[t] = residuals[t0 + t];
         }
         // 16-bit activations in strips of 8 input columns (`direct`): the dot-product kernel at stride 1 (small launches: without LDS), the kernel without LDS at stride 2, whose strips
-        // are 4 outputs wide (a plane of whole vectors and 16-byte aligned steps; frames within its 32-bit offsets). What is left of
-        // 16-bit calls takes at most 4 outputs a strip.
+        // are 4 outputs wide (a plane of whole vectors and 16-byte aligned steps; frames within its 32-bit offsets). Other
+        // 16-bit rows of stride 1 take the kernel of any rows (`takes_rows`), and what is left at most 4 outputs a strip.
         bool direct = x_dtype != SNNF_F32 && W % 8 == 0 && px >= 8 / stride &&
                       (stride == 1 || static_cast<int64_t>(g.planes) * H * W * xsize <= kDirectMaxFrame);
         for (int t = 0; t < tw && direct; ++t) direct = aligned_to(xs[t0 + t], 16);
