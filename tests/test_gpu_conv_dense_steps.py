@@ -127,6 +127,27 @@ def test_scratch_memory_is_not_left(hip_ops, snnf_lib, Cin, Cout, H, k, s, N, T)
     check(sp, v, O.temporal_conv_lif(x, w, b, torch.tensor(0.0), (s, s), (p, p), (1, 1), 1, *LIF), v_dtype=F16)
 
 
+@pytest.mark.parametrize("N,H", [(8, 32), (1, 12)])      # tiles, few pixels
+def test_spikes_over_the_inputs(hip_ops, snnf_lib, N, H):
+    """Inputs that the spikes are written over are copied first."""
+    from triton_snn_fusion_amd import _lib
+    from triton_snn_fusion_amd.runtime import hip_convlif_backend as CB
+    g = gen(9395)
+    T, C, code = 4, 32, _lib.dtype_code(BF16)
+    x = torch.stack([spikes((N, C, H, H), 0.25, g) for _ in range(T)])
+    w, b = dev(torch.randn(C, C, 3, 3, generator=g) * 0.2, BF16), dev(torch.randn(C, generator=g) * 0.1, BF16)
+    packed = CB._packed_weight(w, b, BF16)
+    need = snnf_lib.snnf_conv_lif_scratch_bytes(T, N, C, H, H, code, C, 3, 3, 1, 1, 1, 1, 0, 0)
+    room, got = torch.empty(need, dtype=torch.uint8, device=DEV), []
+    for over in (False, True):
+        xs = dev(x, BF16)
+        sp, v = xs if over else torch.empty_like(xs), torch.empty(N, C, H, H, device=DEV)
+        _lib.check("ws", snnf_lib.snnf_conv_lif_ws(_lib.step_pointers(list(xs)), None, T, N, C, H, H, code, packed.data_ptr(), C, 3, 3, 1, 1, 1, 1, None, 0, sp.data_ptr(),
+                                                   int(sp.stride(0)), v.data_ptr(), *LIF, room.data_ptr(), need, _lib.current_stream(sp.device)))
+        got.append((sp.clone(), v))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and 0 < float(got[0][0].float().mean()) < 1
+
+
 def test_infinities_stay_in_their_windows(hip_ops, snnf_lib):
     """An infinity in the last channel of an image reaches its own windows and no neighbour's: pixels outside the image and channels beyond the last are zeros."""
     g = gen(9390)

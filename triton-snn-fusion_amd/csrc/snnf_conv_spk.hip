@@ -859,7 +859,15 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
     // (Of a dense call xs are the C8 buffers; a wave's K, stages and sums don't depend on which of the two it reads.)
     const LifParams lif_params = make_lif_params(v_threshold, v_reset, tau);
     const bool usual = dense_epilogue_neuron(lif_params);
-    const bool frames = dense != nullptr && dense->xs != nullptr && std::all_of(dense->xs, dense->xs + T, [x_dtype](const void* x) { return aligned_to(x, dtype_size(x_dtype)); });
+    // (Frames that the call writes to, spikes or membrane, are copied first.)
+    const auto apart = [&](const void* x) {
+        const auto in = reinterpret_cast<uintptr_t>(x), to = reinterpret_cast<uintptr_t>(out), v = reinterpret_cast<uintptr_t>(v_out);
+        const uintptr_t in_end = in + static_cast<uintptr_t>(N) * Cin * H * W * dtype_size(x_dtype);
+        const uintptr_t neurons = static_cast<uintptr_t>(N) * Cout * ((H + 2 * pad_h - KH) / stride_h + 1) * ((W + 2 * pad_w - KW) / stride_w + 1);
+        const uintptr_t to_end = to + static_cast<uintptr_t>(T - 1) * static_cast<uintptr_t>(out_step_stride) + neurons * dtype_size(x_dtype);
+        return aligned_to(x, dtype_size(x_dtype)) && (in >= to_end || to >= in_end) && (v_out == nullptr || in >= v + neurons * 4 || v >= in_end);
+    };
+    const bool frames = dense != nullptr && dense->xs != nullptr && std::all_of(dense->xs, dense->xs + T, apart);
     const bool steps = frames && dense->kept->steps.grid > 0 && usual && v_out != nullptr &&
                        (dense->kept->steps.windows == 1 || dense->v_dtype == SNNF_F32 || x_dtype == SNNF_F32 || dense->space.total > dense->space.carry);
     const bool few_steps = frames && dense->kept->few_steps;
