@@ -17,14 +17,16 @@ SOFT = (1.0, -1.0, 3.0)
 @pytest.mark.parametrize("dtype", [BF16, F16])
 @pytest.mark.parametrize("N,C,H,W,T,residual,v_dtype,start,lif", [
     (1, 2, 1, 9, 1, False, F32, False, LIF),          # one row; the second strip is one pixel
-    (2, 3, 2, 15, 4, True, F32, False, LIF),
+    (2, 3, 2, 15, 2, True, F32, False, LIF),
     (3, 5, 7, 8, 3, False, F32, True, LIF),           # whole vectors that start between them
-    (2, 3, 11, 13, 4, True, None, True, LIF),         # a membrane of the activations' type
-    (1, 70, 17, 17, 5, False, F32, False, LIF),       # several workgroups
+    (2, 3, 11, 13, 2, True, None, True, LIF),         # a membrane of the activations' type
+    (2, 70, 40, 31, 5, False, F32, False, LIF),       # odd rows of several steps, in many strips
+    (1, 230, 30, 17, 4, True, None, True, LIF),
+    (1, 70, 17, 17, 5, False, F32, False, LIF),       # and in few: in LDS
     (2, 6, 20, 20, 2, True, F32, False, LIF),         # rows of a multiple of four
-    (1, 4, 9, 31, 20, False, F32, False, LIF),        # a second launch, which goes on in place
+    (1, 9, 9, 30, 20, False, F32, False, LIF),        # a second launch, which goes on in place
     (2, 3, 5, 7, 3, True, F32, False, LIF),           # shorter than a strip
-    (1, 4, 9, 31, 3, True, F32, True, SOFT),
+    (1, 4, 9, 31, 2, True, F32, True, SOFT),
 ])
 def test_rows_that_start_and_end_anywhere(hip_ops, snnf_lib, N, C, H, W, T, residual, v_dtype, start, lif, dtype):
     from triton_snn_fusion_amd import _lib
