@@ -90,6 +90,7 @@ int snnf_lif_scan(const void* const* xs, int T, int64_t numel, int x_dtype,
  *   xs[t]        : [N, C, H, W] x_dtype          weight : [C, 1, 3, 3] w_dtype        bias : [C] w_dtype
  *   residuals[t] : [N, C, Ho, Wo] x_dtype or residuals == NULL
  *   spikes       : [T, N, C, Ho, Wo] x_dtype (timestep stride `spike_step_stride` elements), v_out : [N, C, Ho, Wo] v_dtype
+ * v_out may be v_init, and the spikes may be written over the residuals of their timestep; no other output may lie over an input.
  */
 int snnf_dwconv3x3_lif(const void* const* xs, const void* const* residuals, int T,
                        int N, int C, int H, int W, int stride, int x_dtype,

@@ -64,3 +64,27 @@ def test_rows_that_start_and_end_anywhere(hip_ops, snnf_lib, N, C, H, W, T, resi
             assert torch.equal(got[in_place][1], q(ref[1], v_dtype))
     if start:
         assert torch.equal(got[True][1], got[False][1])
+
+
+@pytest.mark.parametrize("C,H,W,T", [
+    (200, 40, 18, 4),        # strips of two workgroups share a row's outputs
+    (120, 60, 17, 2),
+    (300, 60, 31, 3),
+])
+@pytest.mark.parametrize("over", ["spikes", "membrane"])
+def test_outputs_over_what_is_read(hip_ops, snnf_lib, C, H, W, T, over):
+    """Spikes that are written over the residuals, and a final membrane over the last residual: every output is added to once."""
+    from triton_snn_fusion_amd import _lib
+    g = gen(5290 + C)
+    w, b = torch.randint(-64, 65, (C, 1, 3, 3), generator=g) / 64.0, torch.randint(-16, 17, (C,), generator=g) / 64.0
+    x = torch.randint(-8, 9, (T, 1, C, H, W), generator=g) / 4.0
+    rs = torch.randint(0, 2, (T, 1, C, H, W), generator=g) * 0.75
+    ref = O.temporal_conv_lif(list(x), w, b, torch.tensor(0.0), (1, 1), (1, 1), (1, 1), C, *LIF, residuals=list(rs))
+    dx, dr, dw, db, code = dev(x, BF16), dev(rs, BF16), dev(w, BF16), dev(b, BF16), _lib.dtype_code(BF16)
+    sp = dr if over == "spikes" else torch.empty_like(dx)
+    v = dr[T - 1] if over == "membrane" else torch.empty(1, C, H, W, dtype=BF16, device=DEV)
+    _lib.check("dw", snnf_lib.snnf_dwconv3x3_lif(
+        _lib.step_pointers(list(dx)), _lib.step_pointers(list(dr)), T, 1, C, H, W, 1, code, dw.data_ptr(), db.data_ptr(), code, None, code, sp.data_ptr(), int(sp.stride(0)),
+        v.data_ptr(), *LIF, _lib.current_stream(sp.device)))
+    assert torch.equal(sp.float().cpu(), ref[0]) and torch.equal(v.float().cpu(), q(ref[1], BF16))
+    assert 0.0 < float(ref[0].mean()) < 1.0

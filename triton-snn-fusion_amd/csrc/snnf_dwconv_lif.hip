@@ -494,7 +494,7 @@ int launch_direct(const StepPtrs& xs, const StepPtrs& res, int has_res, int T, c
 // ---------------------------------------------------------------------------------------------------------------
 // Stride 1, 16-bit rows of any length from 8 on that start anywhere, without LDS: a lane has 8 outputs of a row and reads 16 bytes (at any even address) and the element on
 // either side of each of the three input rows, no matter where these lie against whole vectors. The last strip of a row ends with it: it computes outputs of the strip before
-// as well, from the same operands in the same order, and both write the same bits (so the initial membrane may not lie where the final one goes). The taps are
+// as well, from the same operands in the same order, and both write the same bits (so nothing that a call reads may lie where it writes: `takes_rows`). The taps are
 // the fp32 multiply-adds of `dwconv3x3_lif_kernel`, whose strips of one pixel (of four where rows are a multiple of that) take these rows otherwise: an element at a time into LDS and back.
 // What bounds it: HBM from some 100 MB on, below that the chain of a lane's loads. Of 50 drawn layers of such rows, 1.39 times in the mean, those that lose stay (`takes_rows`); 264 channels at 23^2 x 27, T = 3 45.8 -> 20.8, 88 at 78^2 x 8, T = 1 26.8 -> 10.1 (floor 6.6), 88 at 65^2 x 31, T = 4 91.5 -> 59.5 (44.6),
 // 56 at 66^2 x 23 46.4 -> 22.6, 272 at 100^2 x 3 49.0 -> 33.9 (31.6), 64 at 17^2 x 16 7.0 -> 5.6.
@@ -618,8 +618,21 @@ int launch_rows(const StepPtrs& xs, const StepPtrs& res, int has_res, int T, con
 // Which calls the kernel of any rows takes (see there). Odd rows start between dwords, where a 16-byte access takes longer than on even ones, and the time per step counts for more the more
 // there are: us, in LDS / here, 224 channels at 49 x W x 25, T = 1, 4, 8: W = 9 17.1 / 10.6, 22.4 / 27.2, 31.5 / 48.6, 13 30.5 / 11.3, 40.6 / 27.7, 59.6 / 49.3, 17 30.6 / 14.5, 40.6 / 37.5, 59.7 / 68.7,
 // 21 42.8 / 14.9, 54.8 / 37.9, 74.5 / 69.6; 10 17.2 / 8.4, 23.1 / 16.9, 33.1 / 26.8, 18 30.6 / 11.6, 40.5 / 22.7, 59.6 / 37.2. Small launches of odd rows gain up to two steps (64 at 17^2 x 4 3.6 / 3.3, 4.9 / 5.2, 6.5 / 7.6).
-bool takes_rows(int T, const DwGeom& g, const void* v_init, const void* v_out) {
-    if (g.W < 8 || v_init == v_out || static_cast<int64_t>(g.planes) * g.H * g.W * 2 > kDirectMaxFrame) return false;
+// Calls that write over what they read (a membrane in place, spikes over the residuals) stay in LDS, where every output has one owner.
+bool takes_rows(const StepPtrs& xs, const StepPtrs& res, int has_res, int T, const DwGeom& g, const void* v_init, int vsize, const void* spikes, int64_t spike_step_stride,
+                const void* v_out) {
+    const int64_t neurons = static_cast<int64_t>(g.planes) * g.H * g.W;
+    if (g.W < 8 || neurons * 2 > kDirectMaxFrame) return false;
+    const int64_t last = (T - 1) * spike_step_stride * 2;         // (the step stride may descend)
+    const intptr_t out = reinterpret_cast<intptr_t>(spikes), out_from = out + std::min<int64_t>(last, 0), out_to = out + std::max<int64_t>(last, 0) + neurons * 2;
+    const intptr_t end = reinterpret_cast<intptr_t>(v_out), end_to = end + neurons * vsize;
+    const auto written = [&](const void* p, int size) {
+        const intptr_t from = reinterpret_cast<intptr_t>(p), to = from + neurons * size;
+        return (from < out_to && out_from < to) || (from < end_to && end < to);
+    };
+    if (v_init != nullptr && written(v_init, vsize)) return false;
+    for (int t = 0; t < T; ++t)
+        if (written(xs.p[t], 2) || (has_res && written(res.p[t], 2))) return false;
     if (g.W % 2 == 0 || T <= 2) return true;
     return static_cast<int64_t>(g.planes) * g.H * ((g.W + 7) / 8) >= 20000 && g.W >= (T <= 4 ? 11 : 21);
 }
@@ -916,7 +929,8 @@ int dispatch_px(int px, bool direct, const StepPtrs& xs, const StepPtrs& res, in
             return launch_direct<XT, VT, STRIDE>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
         }
         if constexpr (STRIDE == 1) {
-            if (takes_rows(T, g, v_init, v_out)) return launch_rows<XT, VT>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
+            if (takes_rows(xs, res, has_res, T, g, v_init, static_cast<int>(sizeof(VT)), spikes, sss, v_out))
+                return launch_rows<XT, VT>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
         }
     } else if (px == 8) {
         return launch<XT, VT, STRIDE, 8>(xs, res, has_res, T, g, weight, bias, v_init, spikes, sss, v_out, lif, stream);
