@@ -1,5 +1,6 @@
 """Blocked convolutions of more timesteps than a window holds, bit-packed in and out: the straight-line epilogue passes the membrane from
-window to window. Against the CPU oracle for every way the waves of a workgroup share a tile, with last windows of one to four steps."""
+window to window. Against the CPU oracle for every way the waves of a workgroup share a tile, with windows of four timesteps (the last one of one to
+four) and of three (five, six and nine timesteps)."""
 import pytest
 import torch
 
@@ -10,16 +11,22 @@ pytestmark = pytest.mark.gpu
 BF16, F16 = torch.bfloat16, torch.float16
 
 
-@pytest.mark.parametrize("Cin,Cout,H,W,N,T,dtype,residual,layout,waves,tile", [
-    (64, 64, 56, 56, 9, 5, BF16, True, "bits", "8x1x2", 64),      # two waves per tile, a last window of one step
-    (16, 64, 40, 40, 46, 6, BF16, True, "bits", "8x1x1", 64),     # a wave per tile, several rounds
-    (16, 72, 40, 40, 20, 8, F16, False, "c8", "8x1x1", 64),       # blocked inputs; eight channels in the last tile
-    (256, 128, 14, 14, 24, 7, BF16, True, "bits", "8x1x4", 64),   # four waves per tile
-    (512, 512, 7, 7, 9, 6, BF16, False, "bits", "8x1x8", 64),     # eight
-    (128, 40, 8, 8, 1, 16, BF16, True, "bits", "8x1x8", 32),      # tiles of 32 channels, four windows
-    (64, 96, 9, 11, 2, 9, F16, True, "c8", "8x1x4", 32),
+@pytest.mark.parametrize("Cin,Cout,H,W,N,T,window,dtype,residual,layout,waves,tile", [
+    (64, 64, 56, 56, 9, 5, 3, BF16, True, "bits", "8x1x2", 64),       # two waves per tile; windows of three, the last one of two steps
+    (64, 64, 56, 56, 9, 13, 4, BF16, True, "bits", "8x1x2", 64),      # windows of four, the last one of one step
+    (16, 64, 40, 40, 46, 6, 3, BF16, True, "bits", "8x1x1", 64),      # a wave per tile, several rounds
+    (16, 64, 40, 40, 46, 10, 4, BF16, True, "bits", "8x1x1", 64),     # windows of four, the last one of two steps
+    (16, 72, 40, 40, 20, 8, 4, F16, False, "c8", "8x1x1", 64),        # blocked inputs; eight channels in the last tile
+    (256, 128, 14, 14, 24, 7, 4, BF16, True, "bits", "8x1x4", 64),    # four waves per tile; a last window of three steps
+    (256, 128, 14, 14, 24, 13, 4, BF16, True, "bits", "8x1x4", 64),
+    (512, 512, 7, 7, 9, 6, 3, BF16, False, "bits", "8x1x8", 64),      # eight
+    (512, 512, 7, 7, 9, 10, 4, BF16, False, "bits", "8x1x8", 64),
+    (128, 40, 8, 8, 1, 16, 4, BF16, True, "bits", "8x1x8", 32),       # tiles of 32 channels, four windows
+    (128, 40, 8, 8, 1, 13, 4, BF16, True, "bits", "8x1x8", 32),
+    (64, 96, 9, 11, 2, 9, 3, F16, True, "c8", "8x1x4", 32),
+    (64, 96, 9, 11, 2, 10, 4, F16, True, "c8", "8x1x4", 32),
 ])
-def test_membrane_passes_from_window_to_window(snnf_lib, Cin, Cout, H, W, N, T, dtype, residual, layout, waves, tile):
+def test_membrane_passes_from_window_to_window(snnf_lib, Cin, Cout, H, W, N, T, window, dtype, residual, layout, waves, tile):
     from triton_snn_fusion_amd.runtime import hip_blocked_backend as B
     g = gen(7000 + Cin + T)
     x = torch.stack([spikes((N, Cin, H, W), 0.25, g) for _ in range(T)])
@@ -29,7 +36,7 @@ def test_membrane_passes_from_window_to_window(snnf_lib, Cin, Cout, H, W, N, T, 
     out, v = B.conv_lif_blocked(B.from_dense(dev(x, dtype), B.BITS if layout == "bits" else B.C8), dev(w, dtype), dev(b, dtype), [1, 1], [1, 1], LIF,
                                 residual=B.from_dense(dev(rs, dtype), B.BITS) if residual else None, out_layout=B.BITS, want_v=True)
     plan = B.last_conv_plan()
-    assert int(plan["variant"]) >= 60 and int(plan["window"]) == 4, plan
+    assert int(plan["variant"]) >= 60 and int(plan["window"]) == window, plan
     if torch.cuda.get_device_properties(0).multi_processor_count == 256:
         assert (plan["waves"], int(plan["oc_tile"])) == (waves, tile), plan
     check(B.to_dense(out), v, ref, what=f"{Cin}->{Cout} {H}x{W} T={T}")

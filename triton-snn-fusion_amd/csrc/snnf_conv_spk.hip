@@ -511,8 +511,6 @@ const char* family_name(DenseFamily f) {
 enum DenseRouteKind { kNoRoute, kCopyRoute, kFrameRoute, kStepsRoute };
 void plan_text(char* text, const BlockedPlan& p, const char* kernel, int epilogue, int window, DenseRouteKind route) {
     const SpkGeom& g = p.g;
-    // (window: the timesteps that a window of the layer holds. Of `threes` it runs three, as the variant's last digit says.)
-    if (p.tt == 3) window = 4;
     snprintf(text, 256,
              "kernel=%s variant=%d window=%d launches=%d tile=%dx%dx%d halo=%dx%d waves=8x1x%d oc_tiles=%d oc_tile=%d px_tiles=%d "
              "stage_chunks=%d run=0 lds=%zu grid=%d tuned=%d shortcut_stages=%d%s",
