@@ -49,3 +49,12 @@ def test_rows_of_any_length(snnf_lib, T, M, Fin, Fout, pad, dtype, shift):
         s.data_ptr(), M * Fout, v.data_ptr(), *LIF, _lib.current_stream(s.device)))
     assert torch.equal(s.float().cpu(), torch.stack(ref))
     assert torch.allclose(v.cpu(), v_ref, rtol=1e-6, atol=1e-6)            # (a neuron that keeps charging ends with more bits than float32 has)
+
+
+@pytest.mark.parametrize("T,M,Fin,Fout", [
+    (1, 80, 1040, 704), (1, 69, 1424, 1361), (1, 80, 2048, 704), (1, 300, 1088, 1200),       # straight from memory, and staged from 2048 on
+    (2, 3, 1048, 2505), (2, 65, 1080, 500), (2, 20, 3776, 188), (2, 5, 5456, 10),
+])
+def test_one_and_two_steps_on_either_side_of_the_line(snnf_lib, T, M, Fin, Fout):
+    """K just above multiples of 1024 and of 512, which the two kernels for one and two timesteps of aligned rows go over in rounds and in passes."""
+    test_rows_of_any_length(snnf_lib, T, M, Fin, Fout, 0, BF16, 0)

@@ -6,6 +6,7 @@
 // output feature) pair with the membrane in a register. The staged kernel moves K slabs of all operand rows through LDS with
 // coalesced loads; the direct one (short K of one or two timesteps) loads fragments straight from global memory.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "snnf_common.h"
@@ -686,21 +687,45 @@ int launch_staged_tt(const LinWorkspace& ws, const StepPtrs& xs, const LinGeom& 
     return launch_staged<XT, VT, 16, OCF, TM, kWide>(ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
 }
 
+// Whether one or two timesteps of aligned 16-bit rows run on fragments straight from memory. Its eight waves go over K in passes of 512 elements, the staged kernel in rounds of its ring, 1024 elements,
+// whose last one counts in full: a K just above a multiple of 1024 is the worst case of the one and next to none of the other. Both times are estimated from what was measured on 970 layers of
+// K from 1024 to 11200 (to 8 % either way): a constant, passes or rounds at so much each, more of it the more of the compute units have a tile and for each further tile of a unit; passes also by the
+// batch rows that are there, and half as much again where all rows start in the same place of a 128-byte line. us, direct / staged, one step: 5 x 16 rows and 1040 -> 2540 5.1 / 8.7, 69 rows 1424 -> 1361 6.5 / 8.7,
+// 64 rows 2048 -> 1024 6.6 / 6.0, 256 rows 1024 -> 4096 33 / 21; two: 65 rows 1080 -> 1693 8.1 / 12.1, 1 row 1048 -> 2505 4.3 / 6.1, 5456 -> 10 7.5 / 10.0, 23 rows 3776 -> 188 12.7 / 8.3, 15 rows 10624 -> 153 29 / 16,
+// 16 rows 25088 -> 1000 67 / 33. With a line of K = 1024 alone 367 of 1500 drawn layers were slower than straight from memory, up to 1.7 times; with this one 12 of 2000, one by more than a tenth. Short K and few tiles are below the line without an estimate (1 x 100, 200 -> 3000 5.1 / 8.0,
+// 2 x 200, 512 -> 512 5.8 / 6.4, 2 x 128, 768 -> 3072 16.6 / 19.0, 2 x 3, 2400 -> 64 5.6 / 6.8, 1 x 32, 1536 -> 512 5.4 / 5.7).
+inline bool takes_direct(const LinGeom& g) {
+    const int64_t oc_tiles = (g.Fout + kTileOC - 1) / kTileOC, tiles = oc_tiles * ((g.M + kTileM - 1) / kTileM);
+    if (g.Fin < 1024 || (g.Fin < 4096 && tiles <= 16) || (g.Fin < 2048 && g.T == 1 && tiles <= 64)) return true;
+    const bool tall = g.T == 1 && g.M > kTileM;       // (staged tiles of 32 rows)
+    const double units = compute_units(), direct_load = tiles / units, staged_load = tall ? oc_tiles * ((g.M + 2 * kTileM - 1) / (2 * kTileM)) / units : direct_load;
+    const double passes = ((g.Fin + 31) / 32 + 15) / 16, rounds = ((g.Fin + 2 * kSlabK - 1) / (2 * kSlabK) + 3) / 4;
+    const double rows = std::min(g.M, kTileM) / static_cast<double>(kTileM);
+    const auto first = [](double load) { return std::min(load, 1.0); };
+    const auto more = [](double load) { return std::max(load - 1.0, 0.0); };
+    const bool in_step = g.Fin % 64 == 0;
+    if (g.T == 1) {
+        const double direct = 2.6 + passes * (0.53 + rows * (in_step ? 0.31 : 0.07) + 0.27 * first(direct_load) + 0.83 * more(direct_load));
+        const double staged = 3.4 + rounds * (0.82 + (tall ? 0.33 : 0.0) + 0.29 * first(staged_load) + 1.63 * more(std::ceil(staged_load))) + 1.17 * more(std::ceil(staged_load));      // (whole rounds of workgroups)
+        return direct <= 1.03 * staged;
+    }
+    const double direct = 2.7 + passes * (0.49 + rows * (in_step ? 0.79 : 0.39) + 0.22 * first(direct_load) + 1.17 * more(direct_load));
+    const double staged = 3.6 + rounds * (1.09 + 0.43 * first(staged_load) + 1.52 * more(staged_load)) + 0.79 * more(staged_load);
+    return direct <= staged;
+}
+
 // Which kernel runs a layer (us; `aligned`: rows of whole octets at 16-byte addresses):
 // * The staged kernel takes rows that start and end anywhere, and any number of timesteps: its loads are of 16 bytes at any element's address, and the octet in which
 //   a row ends is fetched from the row's last eight elements and shifted. Elementwise loads of such rows took 46 us at 4 x 64, 2047 -> 1024 (here 11.0), 94 at 5 x 206,
 //   555 -> 858 in fp16 (24), 1206 at 8 x 16, 25085 -> 4096 (116). fp32 rows are fetched and split once for the three products, not once for each: 8 x 64, 2048 -> 1024
 //   48 -> 21, 1 x 5, 3001 -> 77 71 -> 10, 6 x 120, 2640 -> 96 55 -> 26.
-// * One or two timesteps of 16-bit rows: against fragments straight from memory (aligned rows) it gains from K = 1024 on (1 x 64, 2048 -> 1024 6.6 / 6.0, x 2 8.9 / 6.9, 1 x 256, 1024 -> 4096 33 / 21,
-//   2 x 16, 25088 -> 1000 67 / 33) and loses below (1 x 100, 200 -> 3000 5.1 / 8.0, 2 x 200, 512 -> 512 5.8 / 6.4, 2 x 128, 768 -> 3072 16.6 / 19.0), and up to 4096 where few tiles
-//   leave the loads of each workgroup alone (2 x 3, 2400 -> 64 5.6 / 6.8; one step up to 2048, 1 x 32, 1536 -> 512 5.4 / 5.7). In fp32 it gains everywhere (1 x 32, 512 -> 10 7.3 / 4.5).
+// * One or two timesteps of 16-bit rows run on fragments straight from memory where `takes_direct` says so (aligned rows). In fp32 the staged kernel gains everywhere (1 x 32, 512 -> 10 7.3 / 4.5).
 template <typename XT, typename VT>
 int launch_tt(bool aligned, const LinWorkspace& ws, const StepPtrs& xs, const LinGeom& g, const void* W, const void* bias, const void* v_init, void* spikes,
               void* v_out, const LifParams& lif, hipStream_t stream) {
     if (g.Fin >= 8) {
         if constexpr (sizeof(XT) == 2) {
-            const int64_t tiles = static_cast<int64_t>((g.Fout + kTileOC - 1) / kTileOC) * ((g.M + kTileM - 1) / kTileM);
-            if (aligned && g.T <= 2 && (g.Fin < 1024 || (g.Fin < 4096 && tiles <= 16) || (g.Fin < 2048 && g.T == 1 && tiles <= 64)))
+            if (aligned && g.T <= 2 && takes_direct(g))
                 return g.T == 1 ? launch_direct<XT, VT, 1>(xs, g, W, bias, v_init, spikes, v_out, lif, stream) : launch_direct<XT, VT, 2>(xs, g, W, bias, v_init, spikes, v_out, lif, stream);
         }
         if (g.T <= 2) return launch_staged_tt<XT, VT, 1, kTileM>(ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
