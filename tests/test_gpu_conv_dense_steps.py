@@ -100,6 +100,27 @@ def test_fp32_terms_against_the_oracle(hip_ops, snnf_lib, Cin, Cout, H, W, k, s,
         assert int(changed.sum()) > 0 and int(changed[:N - 1].sum()) == 0
 
 
+@pytest.mark.parametrize("Cin,Cout,H,W,k,s,N,T,dtype", [
+    (264, 101, 67, 67, 3, 1, 1, 4, BF16),         # many loads to a tile
+    (456, 32, 16, 17, 1, 1, 8, 8, BF16),          # 1x1 in columns of two pixels
+    (116, 72, 34, 27, 7, 2, 25, 1, BF16),         # two waves a tile instead of four, for its wider halo
+    (328, 40, 10, 53, 1, 1, 11, 6, F32),
+])
+def test_layers_that_the_copy_is_faster_for(hip_ops, snnf_lib, Cin, Cout, H, W, k, s, N, T, dtype):
+    from triton_snn_fusion_amd.runtime import hip_convlif_backend as CB
+    g = gen(9370 + Cin)
+    p = k // 2
+    x, b = [spikes((N, Cin, H, W), 0.2, g) for _ in range(T)], torch.randint(-16, 17, (Cout,), generator=g) / 64.0
+    w = torch.randint(-64, 65, (Cout, Cin, k, k), generator=g) / 512.0      # (sums that are exact in any order)
+    sp, v = _run([dev(t, dtype) for t in x], None, dev(w, dtype), dev(b, dtype), torch.zeros((), device=DEV), s, p, LIF)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        plan = CB.last_conv_plan()
+        assert plan.get("reads") is None and plan.get("route") == "c8", plan
+    ref = O.temporal_conv_lif(x, w, b, torch.tensor(0.0), (s, s), (p, p), (1, 1), 1, *LIF)
+    assert torch.equal(sp.float().cpu(), ref[0]) and 0.0 < float(ref[0].mean()) < 1.0
+    check(sp, v, ref, what=f"{Cin}->{Cout} {H}x{W} T={T}")
+
+
 @pytest.mark.parametrize("Cin,Cout,H,k,s,N,T", [
     (27, 328, 15, 7, 2, 5, 4),       # whose frames would take two windows where the copy takes one
     (72, 104, 27, 3, 1, 2, 6),       # two of each
