@@ -148,6 +148,30 @@ def test_scratch_memory_is_not_left(hip_ops, snnf_lib, Cin, Cout, H, k, s, N, T)
     check(sp, v, O.temporal_conv_lif(x, w, b, torch.tensor(0.0), (s, s), (p, p), (1, 1), 1, *LIF), v_dtype=F16)
 
 
+@pytest.mark.parametrize("T,v_dtype", [(1, F32), (2, F32), (2, BF16)])
+def test_1x1_of_up_to_two_timesteps_needs_no_copy(hip_ops, snnf_lib, T, v_dtype):
+    """Layers that are on this route only where the kernel reads their frames ask for a token, not for the room of a copy, and leave it as it is."""
+    from triton_snn_fusion_amd import _lib
+    from triton_snn_fusion_amd.runtime import hip_convlif_backend as CB
+    g = gen(9385)
+    N, Cin, Cout, H, W, code = 9, 144, 104, 10, 54, _lib.dtype_code(BF16)
+    x = [spikes((N, Cin, H, W), 0.25, g) for _ in range(T)]
+    xs = [dev(t, BF16) for t in x]
+    w, b = q(torch.randn(Cout, Cin, 1, 1, generator=g) * 2.0 * (2.0 / Cin) ** 0.5, BF16), q(torch.randn(Cout, generator=g) * 0.1, BF16)
+    packed = CB._packed_weight(dev(w, BF16), dev(b, BF16), BF16)
+    need = snnf_lib.snnf_conv_lif_scratch_bytes(T, N, Cin, H, W, code, Cout, 1, 1, 1, 1, 0, 0, _lib.dtype_code(v_dtype), 0)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert need == 16 * T
+    room = torch.full((max(need, 16) + 4096,), 171, dtype=torch.uint8, device=DEV)
+    sp, v = torch.empty(T, N, Cout, H, W, device=DEV, dtype=BF16), torch.empty(N, Cout, H, W, device=DEV, dtype=v_dtype)
+    _lib.check("ws", snnf_lib.snnf_conv_lif_ws(_lib.step_pointers(xs), None, T, N, Cin, H, W, code, packed.data_ptr(), Cout, 1, 1, 1, 1, 0, 0, None, _lib.dtype_code(v_dtype),
+                                               sp.data_ptr(), int(sp.stride(0)), v.data_ptr(), *LIF, room.data_ptr(), need, _lib.current_stream(sp.device)))
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert CB.last_conv_plan().get("reads") == "frames"
+    assert bool((room == 171).all())
+    check(sp, v, O.temporal_conv_lif(x, w, b, torch.tensor(0.0), (1, 1), (0, 0), (1, 1), 1, *LIF), v_dtype=v_dtype)
+
+
 @pytest.mark.parametrize("N,H", [(8, 32), (1, 12)])      # tiles, few pixels
 def test_spikes_over_the_inputs(hip_ops, snnf_lib, N, H):
     """Inputs that the spikes are written over are copied first."""

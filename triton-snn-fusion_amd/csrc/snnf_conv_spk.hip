@@ -546,7 +546,7 @@ struct KeptPlan {
     bool few_steps;                                    // the kernel for few pixels reads the dense frames itself (`few_reads_steps`)
     BlockedPlan steps;                                 // of the kernel on the dense frames themselves, where the dense epilogue applies (see `reads_steps`; grid 0: never)
     char steps_text[256];
-    bool steps_only;                                   // a call that doesn't read its frames stays on the dense kernels
+    bool steps_only;                                   // a call that doesn't read its frames stays on the dense kernels (one window)
 };
 struct Route { bool taken; DenseFamily family; std::shared_ptr<const KeptPlan> kept; };
 std::mutex routes_mutex;
@@ -607,7 +607,7 @@ Route blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, 
                 }
             }
             kept->steps_only = weigh < 0.0;
-            if (kept->steps_only && kept->steps.grid == 0) route.taken = false;
+            if (kept->steps_only && (kept->steps.grid == 0 || kept->steps.windows > 1)) route.taken = false;
             else route.kept = kept;
         }
     }
@@ -623,12 +623,22 @@ int64_t carried_membrane(const Route& r, int v_dtype, int N, int H, int W, int C
     return static_cast<int64_t>(N) * Cout * ((H + 2 * pad_h - KH) / stride_h + 1) * ((W + 2 * pad_w - KW) / stride_w + 1);
 }
 
+// The scratch memory of a layer. A kernel that always reads the frames itself needs none: a token asks for the route.
+RouteSpace scratch_space(const Route& r, int T, int N, int Cin, int H, int W, int x_dtype, int v_dtype, bool neuron, int Cout, int KH, int KW, int stride_h, int stride_w, int pad_h, int pad_w) {
+    if (!r.kept->steps_only) return route_space(T, N, Cin, H, W, x_dtype == SNNF_F32, neuron ? carried_membrane(r, v_dtype, N, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w) : 0);
+    RouteSpace token = {};
+    token.step = 16;
+    token.total = token.carry = static_cast<size_t>(T) * token.step;
+    return token;
+}
+
 // A call on dense tensors that runs here: its inputs, which are brought into C8 first (null: a frame, which is read as it is), and its plan.
 struct DenseRoute {
     const void* const* xs;
     const KeptPlan* kept;
     RouteSpace space;
     int v_dtype;
+    bool apart;                                        // the call writes nothing where its inputs lie, so that the kernel may read them as they are
 };
 
 }  // namespace
@@ -711,7 +721,7 @@ extern "C" size_t snnf_conv_lif_scratch_bytes(int T, int N, int Cin, int H, int 
     using namespace snnf;
     const Route route = blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residual != 0, true);
     if (!route.taken) return 0;
-    return route_space(T, N, Cin, H, W, x_dtype == SNNF_F32, carried_membrane(route, v_dtype, N, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w)).total;
+    return scratch_space(route, T, N, Cin, H, W, x_dtype, v_dtype, true, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w).total;
 }
 
 extern "C" size_t snnf_conv_bias_workspace_bytes(int T, int N, int Cin, int H, int W, int x_dtype, int Cout, int KH, int KW, int stride_h,
@@ -753,7 +763,7 @@ int run_blocked_route(const void* const* xs, const void* const* residuals, int T
     if (neuron && takes_frame(shared, T, Cin, x_dtype, v_dtype, residuals != nullptr, make_lif_params(v_threshold, v_reset, tau))) {
         const Route frame = blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, false, true, true);
         if (!frame.taken) return SNNF_ERR_UNSUPPORTED;
-        const DenseRoute route = {nullptr, frame.kept.get(), RouteSpace{}, v_dtype};
+        const DenseRoute route = {nullptr, frame.kept.get(), RouteSpace{}, v_dtype, false};
         return conv_lif_blocked_impl("snnf_conv_lif", xs, SNNF_LAYOUT_NCHW, nullptr, SNNF_LAYOUT_NCHW, T, N, Cin, H, W, x_dtype, packed_weight, Cout, KH, KW, stride_h, stride_w,
                                      pad_h, pad_w, v_init, out, SNNF_LAYOUT_NCHW, out_step_stride * dtype_size(x_dtype), v_out, 1, v_threshold, v_reset, tau, stream, nullptr,
                                      false, &route);
@@ -761,13 +771,20 @@ int run_blocked_route(const void* const* xs, const void* const* residuals, int T
     if (workspace == nullptr || !aligned_to(workspace, 16) || shared) return SNNF_ERR_UNSUPPORTED;   // one frame for all timesteps is convolved once on the dense kernels too
     const Route taken = blocked_route(T, N, Cin, H, W, x_dtype, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_dtype, residuals != nullptr, neuron != 0);
     if (!taken.taken) return SNNF_ERR_UNSUPPORTED;
-    if (taken.kept->steps_only && !dense_epilogue_neuron(make_lif_params(v_threshold, v_reset, tau))) return SNNF_ERR_UNSUPPORTED;
-    const RouteSpace space = route_space(T, N, Cin, H, W, x_dtype == SNNF_F32,
-                                         neuron ? carried_membrane(taken, v_dtype, N, H, W, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w) : 0);
+    const RouteSpace space = scratch_space(taken, T, N, Cin, H, W, x_dtype, v_dtype, neuron != 0, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w);
     if (workspace_bytes < space.total) return SNNF_ERR_UNSUPPORTED;
+    const int size = dtype_size(x_dtype);
+    const auto to = reinterpret_cast<uintptr_t>(out), v = reinterpret_cast<uintptr_t>(v_out);
+    const uintptr_t neurons = static_cast<uintptr_t>(N) * Cout * ((H + 2 * pad_h - KH) / stride_h + 1) * ((W + 2 * pad_w - KW) / stride_w + 1);
+    const uintptr_t to_end = to + (static_cast<uintptr_t>(T - 1) * static_cast<uintptr_t>(out_step_stride) + neurons) * size;
+    const bool apart = std::all_of(xs, xs + T, [&](const void* x) {
+        const auto in = reinterpret_cast<uintptr_t>(x), in_end = in + static_cast<uintptr_t>(N) * Cin * H * W * size;
+        return aligned_to(x, size) && (in >= to_end || to >= in_end) && (v_out == nullptr || in >= v + neurons * 4 || v >= in_end);
+    });
+    if (taken.kept->steps_only && !(apart && dense_epilogue_neuron(make_lif_params(v_threshold, v_reset, tau)))) return SNNF_ERR_UNSUPPORTED;
     const void* inner[SNNF_MAX_T_PER_LAUNCH];
     for (int t = 0; t < T; ++t) inner[t] = static_cast<const char*>(workspace) + t * space.step;
-    const DenseRoute route = {xs, taken.kept.get(), space, v_dtype};
+    const DenseRoute route = {xs, taken.kept.get(), space, v_dtype, apart};
     return conv_lif_blocked_impl(neuron ? "snnf_conv_lif" : "snnf_conv_bias", inner, SNNF_LAYOUT_C8, residuals, SNNF_LAYOUT_NCHW, T, N, Cin, H, W, x_dtype,
                                  packed_weight, Cout, KH, KW, stride_h, stride_w, pad_h, pad_w, v_init, out, SNNF_LAYOUT_NCHW, out_step_stride * dtype_size(x_dtype), v_out,
                                  neuron, v_threshold, v_reset, tau, stream, nullptr, false, &route);
@@ -865,18 +882,12 @@ int conv_lif_blocked_impl(const char* who, const void* const* xs, int x_layout, 
                                                          v_init != nullptr, v_out != nullptr, pool2, sc, split}, made); rc != SNNF_OK)
             return rc;
     }
-    // (Of a dense call xs are the C8 buffers; a wave's K, stages and sums don't depend on which of the two it reads.)
+    // (Of a dense call xs are the C8 buffers. The plan of the frames is one of its own: its patches, stages and shares of K can be others than the copy's, and fp32's low terms follow a wave's own stages,
+    // so the order of a sum's additions can depend on whether the call may read them as they are.)
     const LifParams lif_params = make_lif_params(v_threshold, v_reset, tau);
     const bool usual = dense_epilogue_neuron(lif_params);
     // (Frames that the call writes to, spikes or membrane, are copied first.)
-    const auto apart = [&](const void* x) {
-        const auto in = reinterpret_cast<uintptr_t>(x), to = reinterpret_cast<uintptr_t>(out), v = reinterpret_cast<uintptr_t>(v_out);
-        const uintptr_t in_end = in + static_cast<uintptr_t>(N) * Cin * H * W * dtype_size(x_dtype);
-        const uintptr_t neurons = static_cast<uintptr_t>(N) * Cout * ((H + 2 * pad_h - KH) / stride_h + 1) * ((W + 2 * pad_w - KW) / stride_w + 1);
-        const uintptr_t to_end = to + static_cast<uintptr_t>(T - 1) * static_cast<uintptr_t>(out_step_stride) + neurons * dtype_size(x_dtype);
-        return aligned_to(x, dtype_size(x_dtype)) && (in >= to_end || to >= in_end) && (v_out == nullptr || in >= v + neurons * 4 || v >= in_end);
-    };
-    const bool frames = dense != nullptr && dense->xs != nullptr && std::all_of(dense->xs, dense->xs + T, apart);
+    const bool frames = dense != nullptr && dense->xs != nullptr && dense->apart;
     const bool steps = frames && dense->kept->steps.grid > 0 && usual && v_out != nullptr &&
                        (dense->kept->steps.windows == 1 || dense->v_dtype == SNNF_F32 || x_dtype == SNNF_F32 || dense->space.total > dense->space.carry);
     const bool few_steps = frames && dense->kept->few_steps;
