@@ -42,6 +42,24 @@ def test_membrane_passes_from_window_to_window(snnf_lib, Cin, Cout, H, W, N, T, 
     check(B.to_dense(out), v, ref, what=f"{Cin}->{Cout} {H}x{W} T={T}")
 
 
+@pytest.mark.parametrize("Cin,Cout,H,W,N,window", [
+    (16, 96, 40, 40, 46, 4),      # a wave per tile: windows of four, four and one
+    (24, 120, 58, 58, 13, 4),
+    (48, 96, 14, 14, 4, 3),       # waves that share a tile: three of three
+])
+def test_nine_steps_of_1x1(snnf_lib, Cin, Cout, H, W, N, window):
+    from triton_snn_fusion_amd.runtime import hip_blocked_backend as B
+    g = gen(7100 + Cin)
+    x = torch.stack([spikes((N, Cin, H, W), 0.25, g) for _ in range(9)])
+    w, b = q(torch.randn(Cout, Cin, 1, 1, generator=g) * 2.0 * (2.0 / Cin) ** 0.5, BF16), q(torch.randn(Cout, generator=g) * 0.1, BF16)
+    ref = O.temporal_conv_lif(list(x), w, b, torch.tensor(0.0), (1, 1), (0, 0), (1, 1), 1, *LIF)
+    out, v = B.conv_lif_blocked(B.from_dense(dev(x, BF16), B.BITS), dev(w, BF16), dev(b, BF16), [1, 1], [0, 0], LIF, out_layout=B.BITS, want_v=True)
+    plan = B.last_conv_plan()
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert int(plan["window"]) == window, plan
+    check(B.to_dense(out), v, ref, what=f"{Cin}->{Cout} {H}x{W} T=9")
+
+
 SOFT = (1.0, -1.0, 2.0)
 
 

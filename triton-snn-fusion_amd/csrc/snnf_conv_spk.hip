@@ -252,7 +252,7 @@ struct BlockedPlan {
 };
 
 // Everything that decides whether and how the kernel runs a call; nothing is enqueued. `window`: all timesteps in one window of so many (0: windows of up to four).
-int plan_window(const char* who, const BlockedCall& c, BlockedPlan& p, int window) {
+int plan_window(const char* who, const BlockedCall& c, BlockedPlan& p, int window, bool may_three = true) {
     const int T = c.T, N = c.N, Cin = c.Cin, H = c.H, W = c.W, Cout = c.Cout, KH = c.KH, KW = c.KW;
     const int stride_h = c.stride_h, stride_w = c.stride_w, pad_h = c.pad_h, pad_w = c.pad_w;
     const bool shared = c.shared, neuron = c.neuron, pool2 = c.pool2;
@@ -291,7 +291,7 @@ int plan_window(const char* who, const BlockedCall& c, BlockedPlan& p, int windo
     // Where four don't fit, three only do with few pixels a tile, and two it is (160 -> 40 7x7 stride 2 at 21^2 x 29, T = 6 in patches of 11 x 1 77 us, of 2 x 11 55).
     int& tt = p.tt;
     SpkPlan fours;
-    const bool three = !shared && !pool2 && threes(T) && plan_spk(g, 4, fours);
+    const bool three = may_three && !shared && !pool2 && threes(T) && plan_spk(g, 4, fours);
     tt = window > 0 ? window : (shared || T == 1 ? 1 : (T == 2 ? 2 : (three ? 3 : 4)));
     TunedPlan tuned = {0, 0, 0};
     if (!c.split) {   // (measured on 16-bit activations)
@@ -455,6 +455,14 @@ int plan_window(const char* who, const BlockedCall& c, BlockedPlan& p, int windo
 // at 7^2 x 7, T = 8 23.2 / 26.8): nothing is multiplied for steps beyond T, and the activations of a narrow tile come from LDS at its full rate.
 int plan_blocked(const char* who, const BlockedCall& c, BlockedPlan& p) {
     if (const int rc = plan_window(who, c, p, 0); rc != SNNF_OK) return rc;
+    // Nine timesteps of a 1x1 layer on bits, a wave to a tile: windows of four, four and one. A window of three takes as long to set up as one of four, and the last one of a single step has next to no
+    // epilogue (us, three / four, 16 -> 320 at 96^2 x 2 49.5 / 44.8, 24 -> 320 at 111 x 9 x 25 91.8 / 84.4, 64 -> 64 at 96^2 x 8 with a residual 57.1 / 53.4, 96 -> 192 the same; of 64 layers the mean 0.98, where waves
+    // share a tile 49 of 1.10).
+    if (c.T > 6 && p.tt == 3 && p.g.taps == 1 && p.g.C8in <= 8 && p.wk_log2 == 0 && c.out_layout == SNNF_LAYOUT_BITS && !p.tuned_patch && !p.tuned_split) {
+        BlockedPlan four;
+        if (plan_window(who, c, four, 0, false) == SNNF_OK) p = four;
+        return SNNF_OK;
+    }
     if ((c.T != 5 && c.T != 6) || c.shared || c.split || c.shortcut != nullptr || p.tt != 3 || p.few || p.tuned_patch || p.tuned_split || p.g.tap_pairs || !p.g.narrow ||
         p.wk_log2 == 0 || ((p.g.taps * p.g.C8in / 2) >> p.wk_log2) > 16) return SNNF_OK;
     BlockedPlan one;
