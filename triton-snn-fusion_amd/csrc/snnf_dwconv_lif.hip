@@ -616,8 +616,10 @@ int launch_rows(const StepPtrs& xs, const StepPtrs& res, int has_res, int T, con
 }
 
 // Which calls the kernel of any rows takes (see there). Odd rows start between dwords, where a 16-byte access takes longer than on even ones, and the time per step counts for more the more
-// there are: us, in LDS / here, 224 channels at 49 x W x 25, T = 1, 4, 8: W = 9 17.1 / 10.6, 22.4 / 27.2, 31.5 / 48.6, 13 30.5 / 11.3, 40.6 / 27.7, 59.6 / 49.3, 17 30.6 / 14.5, 40.6 / 37.5, 59.7 / 68.7,
-// 21 42.8 / 14.9, 54.8 / 37.9, 74.5 / 69.6; 10 17.2 / 8.4, 23.1 / 16.9, 33.1 / 26.8, 18 30.6 / 11.6, 40.5 / 22.7, 59.6 / 37.2. Small launches of odd rows gain up to two steps (64 at 17^2 x 4 3.6 / 3.3, 4.9 / 5.2, 6.5 / 7.6).
+// there are; a residual makes the way through LDS the longer one. us, in LDS / here, tensors from memory: 387 channels at 73 x W x 3, W = 73, T = 1 40.3 / 21.8, 2 46.3 / 34.2, 3 52.3 / 46.2, 4 58.2 / 57.5,
+// 5 65.3 / 69.0, 6 72.8 / 81.0, 8 86.8 / 103.5, W = 74, T = 5 72.0 / 50.8. Of 300 drawn layers of odd rows: up to two steps 1.39 in the mean, the smallest 0.96; three and four, from 20 k and 32 k strips of
+// eight on, 1.15 (four lose up to a twentieth), from 10 k to 32 k 0.91 to 1.02; five and six in rows of 80 elements and more 1.0 to 1.3, of fewer 0.86 to 1.1, eight 0.73 to 1.0; with a residual
+// 1.04 to 1.9 at any number of steps, in rows of nine 0.88.
 // Calls that write over what they read (a membrane in place, spikes over the residuals) stay in LDS, where every output has one owner.
 bool takes_rows(const StepPtrs& xs, const StepPtrs& res, int has_res, int T, const DwGeom& g, const void* v_init, int vsize, const void* spikes, int64_t spike_step_stride,
                 const void* v_out) {
@@ -634,7 +636,9 @@ bool takes_rows(const StepPtrs& xs, const StepPtrs& res, int has_res, int T, con
     for (int t = 0; t < T; ++t)
         if (written(xs.p[t], 2) || (has_res && written(res.p[t], 2))) return false;
     if (g.W % 2 == 0 || T <= 2) return true;
-    return static_cast<int64_t>(g.planes) * g.H * ((g.W + 7) / 8) >= 20000 && g.W >= (T <= 4 ? 11 : 21);
+    const int64_t strips = static_cast<int64_t>(g.planes) * g.H * ((g.W + 7) / 8);
+    if (has_res) return strips >= 20000 && g.W >= (T <= 4 ? 11 : 21);
+    return strips >= (T == 3 ? 20000 : 32000) && g.W >= (T <= 4 ? 11 : 80) && T <= 6;
 }
 
 // ---------------------------------------------------------------------------------------------------------------
