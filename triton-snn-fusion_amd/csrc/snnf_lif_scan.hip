@@ -8,10 +8,12 @@ namespace snnf {
 namespace {
 
 constexpr int kThreads = 256;
-// Timesteps in flight where their number is no constant: four of them, or (TC < 0) each stored before the next is loaded, which fp32 tensors that stream from memory prefer: they have
-// enough waves to overlap (2 M neurons, T = 3 10.1 us, four in flight 10.8; T = 16 51.4 / 53.0; but 200 k neurons, T = 16 12.6 -> 5.8, bf16 13.4 -> 6.1, 2 M neurons in bf16 30.0 -> 25.0).
+// Timesteps in flight where their number is no constant: four of them, or (TC < 0) each stored before the next is loaded, which whole vectors that stream from memory prefer: they have
+// enough waves to overlap (us, each / four, 16 bits, T = 5 3.2 M neurons 18.9 / 20.2, 6.4 M 32.5 / 34.2, T = 3 12.8 M 42.0 / 45.5, fp32 T = 16 2 M 51.4 / 53.0; but 16 bits, T = 16 0.2 M 13.4 / 6.1, and
+// single elements, T = 6 2.9 M 38.9 / 25.2). The line lies where the frame of a step has 3 MB: fp32 0.4 to 0.7 M neurons gain 1.05 to 1.16 from four in flight, 0.75 to 2 M lose 0.92 to 0.98, 16 bits from 0.7 to 1 M
+// 1.04 to 1.26, 1 to 1.5 M 0.97 to 1.02, 1.5 to 8 M 0.88 to 1.0.
 constexpr int kInFlight = 4;
-constexpr int64_t kStreamNeurons = 1 << 20;
+constexpr int64_t kStreamBytes = 3 << 20;
 
 // One thread owns VEC consecutive neurons; every load/store of a thread is one 16-byte (or narrower, VEC == 1)
 // transaction, so a 64-lane wave moves 1 KiB per instruction.
@@ -93,8 +95,13 @@ int launch_lif_scan(const StepPtrs& xs, int T, int64_t numel, const void* v_init
         case 4: go(std::integral_constant<int, 4>{}); break;
         case 8: go(std::integral_constant<int, 8>{}); break;
         default:
-            if (sizeof(XT) == 4 && numel >= kStreamNeurons) go(std::integral_constant<int, -1>{});
-            else go(std::integral_constant<int, 0>{});
+            if constexpr (VEC > 1) {
+                if (numel * static_cast<int64_t>(sizeof(XT)) >= kStreamBytes) {
+                    go(std::integral_constant<int, -1>{});
+                    break;
+                }
+            }
+            go(std::integral_constant<int, 0>{});
     }
     return check_launch("snnf_lif_scan");
 }
