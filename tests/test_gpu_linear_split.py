@@ -88,6 +88,20 @@ def test_layers_whose_tiles_fill_the_chip_do_not_split(snnf_lib):
     assert int(snnf_lib.snnf_linear_lif_workspace_bytes(2, 16, 4096, 4096)) == 0       # one or two timesteps: the kernel without staging
 
 
+@pytest.mark.parametrize("T,M,Fin,Fout,dtype", [(2, 16, 25088, 100, BF16), (1, 40, 8192, 64, BF16), (2, 5, 4096, 80, F32)])
+def test_one_and_two_timesteps_leave_a_workspace_alone(snnf_lib, T, M, Fin, Fout, dtype):
+    """They are asked none for, so that one which a call brings all the same need not be zero."""
+    from triton_snn_fusion_amd import _lib
+    assert int(snnf_lib.snnf_linear_lif_workspace_bytes(T, M, Fin, Fout)) == 0
+    x, w, b, _ = _inputs(T, M, Fin, Fout, dtype, F32, False, 7300 + T)
+    dx, dw, db = x.to(DEV, dtype), w.to(DEV, dtype), b.to(DEV, dtype)
+    ws = torch.full((1 << 22,), 1, dtype=torch.uint8, device=DEV)
+    s, v = _call(snnf_lib, _lib, dx, dw, db, None, F32, ws)
+    s_none, v_none = _call(snnf_lib, _lib, dx, dw, db, None, F32, None)
+    assert torch.equal(s, s_none) and torch.equal(v, v_none) and bool((ws == 1).all())
+    check(s, v, O.temporal_linear_lif(x, w, b, torch.tensor(0.0), *LIF), what=f"linear {Fin}->{Fout} T={T}")
+
+
 def test_split_k_windows_chain_like_one_long_call(hip_ops):
     """Two calls of 16 timesteps, the second starting from the first one's membrane, equal one call of 32 timesteps (which
     the library runs as two windows of 16) bit for bit; all of them split, the operator API allocates the workspace."""

@@ -728,7 +728,8 @@ int launch_tt(bool aligned, const LinWorkspace& ws, const StepPtrs& xs, const Li
             if (aligned && g.T <= 2 && takes_direct(g))
                 return g.T == 1 ? launch_direct<XT, VT, 1>(xs, g, W, bias, v_init, spikes, v_out, lif, stream) : launch_direct<XT, VT, 2>(xs, g, W, bias, v_init, spikes, v_out, lif, stream);
         }
-        if (g.T <= 2) return launch_staged_tt<XT, VT, 1, kTileM>(ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
+        // One or two timesteps are asked no workspace for, and what a call brings all the same may not be zero: K is not split.
+        if (g.T <= 2) return launch_staged_tt<XT, VT, 1, kTileM>(LinWorkspace{nullptr, 0}, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
         // Two feature fragments per workgroup (half the activation traffic) when that still leaves at least 128 workgroups.
         const bool half_rows = linear_half_row_tiles(ws, g);
         const int tm = half_rows ? 8 : kTileM;
@@ -761,7 +762,7 @@ int launch_bits(const LinWorkspace& ws, const StepPtrs& xs, const LinGeom& g, co
 
 extern "C" size_t snnf_linear_lif_workspace_bytes(int T, int M, int Fin, int Fout) {
     using namespace snnf;
-    if (T < 3 || M < 1 || Fin < 1 || Fout < 1) return 0;      // one or two timesteps run on the kernel without staging
+    if (T < 3 || M < 1 || Fin < 1 || Fout < 1) return 0;      // one or two timesteps don't split (see launch_tt)
     int tt = 4;
     while (tt < T && tt < SNNF_MAX_T_PER_LAUNCH) tt *= 2;
     const int64_t m_tiles = (M + kTileM - 1) / kTileM;
