@@ -474,6 +474,15 @@ def test_which_layers_of_whole_tiles_move(snnf_lib, layer, moves):
     assert asked == (T * N * Cin * H * H * 2 if moves else 0)
 
 
+@pytest.mark.parametrize("T,Fin", [(1, 4095), (2, 4095), (4, 4095), (1, 5)])
+def test_batches_beyond_the_grid_of_linear_layers_are_refused(snnf_lib, T, Fin):
+    """65535 tiles of 16 rows, whatever the rows of a kernel's tiles. (Nothing is enqueued: the pointers are never followed.)"""
+    steps = (ctypes.c_void_p * T)(*([4096] * T))
+    rc = snnf_lib.snnf_linear_lif(steps, T, 65535 * 16 + 1, Fin, Fin, _lib.SNNF_BF16, 4096, None, 64, _lib.SNNF_BF16, None, _lib.SNNF_F32, 4096, 1 << 40, 4096, 1.0, 0.0, 2.0, None)
+    assert rc == snnf_lib.snnf_linear_lif(steps, T, 1 << 30, Fin, Fin, _lib.SNNF_BF16, 4096, None, 64, _lib.SNNF_BF16, None, _lib.SNNF_F32, 4096, 1 << 40, 4096, 1.0, 0.0, 2.0, None)
+    assert rc != 0 and b"too large" in snnf_lib.snnf_last_error()
+
+
 def test_a_tuned_plan_is_seen_by_a_remembered_route(snnf_lib):
     """A 7x7 layer whose planned stages of four channel groups hold more steps than the table, and stages of two do not."""
     layer = (2, 2, 372, 5, 5, 384, 7, 7, 1, 1, 3, 3)

@@ -632,7 +632,7 @@ template <typename XT, typename VT, int TT, int OCF, int TM = kTileM, int SLABK 
 int launch_staged(const LinWorkspace& ws, const StepPtrs& xs, const LinGeom& g, const void* W, const void* bias, const void* v_init, void* spikes,
                   void* v_out, const LifParams& lif, hipStream_t stream) {
     dim3 grid((g.Fout + OCF * kTileOC - 1) / (OCF * kTileOC), (g.M + TM - 1) / TM);
-    if (grid.y > 65535) return fail(SNNF_ERR_UNSUPPORTED, "snnf_linear_lif: M=%d too large", g.M);
+    if (grid.y > 65535 || (g.M + kTileM - 1) / kTileM > 65535) return fail(SNNF_ERR_UNSUPPORTED, "snnf_linear_lif: M=%d too large", g.M);
     const int unit_slabs = (g.Fin + SLABK - 1) / SLABK;
     const int64_t tiles = static_cast<int64_t>(grid.x) * grid.y;
     const size_t part_bytes = static_cast<size_t>(TT) * OCF * kTileOC * TM * sizeof(float);
