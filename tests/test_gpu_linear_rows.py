@@ -58,3 +58,12 @@ def test_rows_of_any_length(snnf_lib, T, M, Fin, Fout, pad, dtype, shift):
 def test_one_and_two_steps_on_either_side_of_the_line(snnf_lib, T, M, Fin, Fout):
     """K just above multiples of 1024 and of 512, which the two kernels for one and two timesteps of aligned rows go over in rounds and in passes."""
     test_rows_of_any_length(snnf_lib, T, M, Fin, Fout, 0, BF16, 0)
+
+
+@pytest.mark.parametrize("T,M,Fin,Fout,dtype", [
+    (4, 40, 616, 256, BF16), (4, 20, 640, 64, F32),       # three slabs of 256 in a ring of four
+    (4, 200, 368, 650, F16), (8, 100, 240, 256, BF16),    # of 128; one in a ring of two
+])
+def test_one_slab_short_of_the_ring(snnf_lib, T, M, Fin, Fout, dtype):
+    """(Whole rows: 16-bit tensors walk the ring all the same, fp32 tensors the slabs that are there.)"""
+    test_rows_of_any_length(snnf_lib, T, M, Fin, Fout, 0, dtype, 0)

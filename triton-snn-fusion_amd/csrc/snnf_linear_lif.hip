@@ -612,7 +612,13 @@ template <typename XT, typename VT, int TT, int OCF, bool DB, int SLABK, int TM,
 int launch_staged_db(dim3 grid, int slabs_per_part, const LinWorkspace& ws, const StepPtrs& xs, const LinGeom& g, const void* W, const void* bias,
                      const void* v_init, void* spikes, void* v_out, const LifParams& lif, hipStream_t stream) {
     if constexpr (!XBITS && !SBITS) {
-        if ((g.Fin & 7) != 0 || slabs_per_part < StagedShape<TT, OCF, SLABK, TM, sizeof(XT) == 4 ? 2 : 1>::RING)
+        // (16-bit tensors one slab short of the ring walk it whole all the same, us, short / whole: 4 x 40, 616 -> 256 5.96 / 5.27, 4 x 200, 368 -> 2566 29.7 / 22.7, 8 x 100, 240 -> 256 5.95 / 5.44, 45 layers 1.06
+        // in the mean. Two short, 4 x 40, 440 -> 256, they are the same; a ring of two slabs of 128, of which there is one, loses, 5 x 59, 80 -> 2402 9.4 / 10.5, and so do fp32 tensors, 4 x 5, 768 -> 713 6.9 / 7.4. Where workgroups share
+        // a compute unit, of which fewer fit with this kernel's registers, one slab gains, 4 x 148, 64 -> 1304 9.5 / 11.3, and two lose, 4 x 100, 208 -> 4096 15.9 / 13.4, 39 layers 1.04 in the mean.)
+        constexpr int RING = StagedShape<TT, OCF, SLABK, TM, sizeof(XT) == 4 ? 2 : 1>::RING;
+        constexpr bool kWhole = sizeof(XT) == 2 && (RING > 2 || SLABK > kSlabK);
+        constexpr int kShort = kWhole ? RING - 1 : RING;
+        if ((g.Fin & 7) != 0 || slabs_per_part < (DB || sizeof(XT) == 4 ? kShort : std::min(kShort, 2)))
             return launch_staged_form<XT, VT, TT, OCF, DB, SLABK, TM, true>(grid, slabs_per_part, ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
     }
     return launch_staged_form<XT, VT, TT, OCF, DB, SLABK, TM, false, XBITS, SBITS>(grid, slabs_per_part, ws, xs, g, W, bias, v_init, spikes, v_out, lif, stream);
