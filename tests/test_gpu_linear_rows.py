@@ -67,3 +67,25 @@ def test_one_and_two_steps_on_either_side_of_the_line(snnf_lib, T, M, Fin, Fout)
 def test_one_slab_short_of_the_ring(snnf_lib, T, M, Fin, Fout, dtype):
     """(Whole rows: 16-bit tensors walk the ring all the same, fp32 tensors the slabs that are there.)"""
     test_rows_of_any_length(snnf_lib, T, M, Fin, Fout, 0, dtype, 0)
+
+
+@pytest.mark.parametrize("dtype,Fin", [(BF16, 25085), (F16, 4001)])
+def test_rows_of_eight_timesteps_round_like_those_of_four(snnf_lib, dtype, Fin):
+    """Both add K in eight chains, so that the root mean square of what a membrane is off by, which eight timesteps halve and add to like four, is about the same (with half as many chains 1.3 to
+    1.45 times as large). 16 rows x 192 features: two such values of equal chains lie within a twentieth or so of each other."""
+    from triton_snn_fusion_amd import _lib
+    M, Fout, code, off = 16, 192, _lib.dtype_code(dtype), {}
+    g = torch.Generator(device=DEV)
+    g.manual_seed(5360)
+    w = (torch.randn(Fout, Fin, generator=g, device=DEV) / Fin ** 0.5).to(dtype)
+    for T in (4, 8):
+        x = torch.randn(T, M, Fin, generator=g, device=DEV).to(dtype)
+        s, v = torch.empty(T, M, Fout, device=DEV, dtype=dtype), torch.empty(M, Fout, device=DEV)
+        _lib.check("linear", snnf_lib.snnf_linear_lif(
+            _lib.step_pointers(list(x)), T, M, Fin, Fin, code, w.data_ptr(), None, Fout, code, None, _lib.dtype_code(torch.float32), s.data_ptr(), M * Fout, v.data_ptr(), 1e30, 0.0, 2.0,
+            _lib.current_stream(s.device)))
+        exact = torch.zeros(M, Fout, dtype=torch.float64, device=DEV)
+        for t in range(T):
+            exact += (x[t].double() @ w.double().t().contiguous() - exact) / 2
+        off[T] = float((v.double() - exact).pow(2).mean().sqrt())
+    assert 0.0 < off[8] < 1.15 * off[4], off

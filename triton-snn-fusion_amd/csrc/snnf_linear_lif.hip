@@ -272,8 +272,9 @@ template <int TT, int OCF, int SLABK, int TM, int PLANES> struct StagedShape {
 // stride is in bytes), expanded to 0 / 1 operands where a slab is parked. SBITS: the spikes leave as bits in the same form
 // ([T][M][Fout / 8] bytes, the step stride in bytes) instead of elements. Both are the internal layouts of a network executor
 // (a convolution on a plane of a few pixels is this matrix product, see snnf_linear_lif_bits).
+// (Two workgroups to a compute unit, four waves to a SIMD, where the second chain of sums would just take the registers of one.)
 template <typename XT, typename VT, int TT, int OCF, bool DB, int SLABK, int TM, bool SPECIAL, bool XBITS = false, bool SBITS = false>
-__global__ __launch_bounds__(kStagedWaves * 64) void linear_lif_staged_kernel(StepPtrs xs, LinGeom g, const XT* __restrict__ W,
+__global__ __launch_bounds__(kStagedWaves * 64, !DB && SPECIAL && sizeof(XT) == 2 && TT == 8 && OCF == 1 ? 4 : 2) void linear_lif_staged_kernel(StepPtrs xs, LinGeom g, const XT* __restrict__ W,
                                                                               const XT* __restrict__ bias,
                                                                               const VT* __restrict__ v_start, XT* __restrict__ spikes,
                                                                               VT* __restrict__ v_store, LifParams lif,
@@ -336,16 +337,23 @@ __global__ __launch_bounds__(kStagedWaves * 64) void linear_lif_staged_kernel(St
             ptr = W + static_cast<int64_t>(min(oc0 + r - TT * TM, g.Fout - 1)) * g.Fin;
         }
         item_row[j] = ptr;
-        item_dst[j] = static_cast<uint32_t>(r * kSlabPitch + octet * 16);
+        // (Of items that are not live it is never used; where the registers are short the places are offsets from the first one's. In the kernel of whole rows that
+        // takes longer: 5 x 3, 328 -> 449 4.6 -> 5.3 us.)
+        item_dst[j] = static_cast<uint32_t>((SPECIAL ? row : r) * kSlabPitch + octet * 16);
     }
 
     const int tg = wave % SH::TG;
     const int kp = wave / SH::TG;
-    f32x4 acc[OCF][SH::TPW];
+    // Rows that end inside an octet add their K steps in as many chains as a kernel of eight waves (beyond 8 timesteps four) that splits K among them all: two by turns where fewer share it.
+    // (Root mean square of what the sums of normal numbers are off by, against 64 bits, 8 x 16 rows, 25085 -> 96 in bf16: one chain 2.9e-7, two 2.0e-7.)
+    constexpr int CHAINS = SPECIAL && sizeof(XT) == 2 && SH::KSPLIT < (TT <= 8 ? 8 : 4) ? 2 : 1;
+    f32x4 acc[CHAINS][OCF][SH::TPW];
 #pragma unroll
-    for (int f = 0; f < OCF; ++f)
+    for (int c = 0; c < CHAINS; ++c)
 #pragma unroll
-        for (int u = 0; u < SH::TPW; ++u) acc[f][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int f = 0; f < OCF; ++f)
+#pragma unroll
+            for (int u = 0; u < SH::TPW; ++u) acc[c][f][u] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     // RING slabs ahead in registers: a slab's loads have the time of RING - 1 other slabs to arrive, so the loop runs at
     // the rate of its LDS traffic and barriers instead of one memory latency per slab. Every load is unconditional and
@@ -418,7 +426,7 @@ __global__ __launch_bounds__(kStagedWaves * 64) void linear_lif_staged_kernel(St
                 }
             }
     };
-    auto multiply = [&](const unsigned char* buf) __attribute__((always_inline)) {
+    auto multiply = [&](const unsigned char* buf, int r) __attribute__((always_inline)) {
         constexpr int OWN = SLABK / 32 / SH::KSPLIT;
         constexpr int P = sizeof(XT) == 4 ? 2 : 1;
         constexpr int TOGETHER = P == 1 ? 4 : (SH::ITEMS > 5 ? 1 : 2);      // (registers)
@@ -448,7 +456,10 @@ __global__ __launch_bounds__(kStagedWaves * 64) void linear_lif_staged_kernel(St
 #pragma unroll
                         for (int u = 0; u < SH::TPW; ++u)
 #pragma unroll
-                            for (int f = 0; f < OCF; ++f) acc[f][u] = mfma16<XT>(a[i][term == 1 ? 1 : 0][f], b[i][term == 2 ? 1 : 0][u], acc[f][u]);
+                            for (int f = 0; f < OCF; ++f) {
+                                f32x4& sum = acc[(r * OWN + i0 + i) % CHAINS][f][u];
+                                sum = mfma16<XT>(a[i][term == 1 ? 1 : 0][f], b[i][term == 2 ? 1 : 0][u], sum);
+                            }
                 }
             }
         }
@@ -463,7 +474,7 @@ __global__ __launch_bounds__(kStagedWaves * 64) void linear_lif_staged_kernel(St
                 unsigned char* buf = staged_lds + (DB ? (r & 1) * SH::slab_bytes : 0);
                 park(r, buf);
                 __syncthreads();
-                multiply(buf);
+                multiply(buf, r);
                 if (!DB) __syncthreads();
             }
         }
@@ -475,7 +486,7 @@ __global__ __launch_bounds__(kStagedWaves * 64) void linear_lif_staged_kernel(St
             park(r, buf);
             __syncthreads();
             fetch(slab + RING, r);
-            multiply(buf);
+            multiply(buf, r);
             if (!DB) __syncthreads();
         }
     }
@@ -491,8 +502,22 @@ __global__ __launch_bounds__(kStagedWaves * 64) void linear_lif_staged_kernel(St
         for (int f = 0; f < OCF; ++f)
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                partial[((kp * SH::FRAGS + tg * SH::TPW + u) * 16 + (lane & 15)) * SH::PITCH + f * kTileOC + (lane >> 4) * 4 + r] = acc[f][u][r];
+                partial[((kp * SH::FRAGS + tg * SH::TPW + u) * 16 + (lane & 15)) * SH::PITCH + f * kTileOC + (lane >> 4) * 4 + r] = CHAINS == 2 ? acc[0][f][u][r] + acc[CHAINS - 1][f][u][r] : acc[0][f][u][r];
     __syncthreads();
+
+    // The sums of the waves in the order of their K steps (in pairs where the kernel of one and two timesteps and of any rows has them so).
+    auto waves_sum = [&](int t, int slot) __attribute__((always_inline)) -> float {
+        constexpr int TOGETHER = TT <= 2 || SPECIAL ? 2 : 1;
+        static_assert(SH::KSPLIT % 2 == 0, "pairs of waves");
+        float sum = 0.0f;
+#pragma unroll
+        for (int w = 0; w < SH::KSPLIT; w += TOGETHER) {
+            float part = partial[(w * TT + t) * SLAB_F + slot];
+            if (TOGETHER == 2) part += partial[((w + 1) * TT + t) * SLAB_F + slot];
+            sum += part;
+        }
+        return sum;
+    };
 
     // K split over workgroups: every workgroup of a tile leaves its sums in the workspace and counts itself in; the one
     // that arrives last adds all parts in the order of their K ranges (so the result does not depend on who was last)
@@ -512,10 +537,7 @@ __global__ __launch_bounds__(kStagedWaves * 64) void linear_lif_staged_kernel(St
             const int slot = (e / TILE_OC) * SH::PITCH + e % TILE_OC;
 #pragma unroll
             for (int t = 0; t < TT; ++t) {
-                float sum = 0.0f;
-#pragma unroll
-                for (int w = 0; w < SH::KSPLIT; ++w) sum += partial[(w * TT + t) * SLAB_F + slot];
-                __hip_atomic_store(mine + t * OUTS + e, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(mine + t * OUTS + e, waves_sum(t, slot), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // this thread's partial sums have reached memory
@@ -545,10 +567,7 @@ __global__ __launch_bounds__(kStagedWaves * 64) void linear_lif_staged_kernel(St
             }
         } else {
 #pragma unroll
-            for (int t = 0; t < TT; ++t) {
-#pragma unroll
-                for (int w = 0; w < SH::KSPLIT; ++w) sum[t] += partial[(w * TT + t) * SLAB_F + slot];
-            }
+            for (int t = 0; t < TT; ++t) sum[t] = waves_sum(t, slot);
         }
         auto recurrence = [&](auto usual) __attribute__((always_inline)) {
 #pragma unroll
