@@ -193,6 +193,28 @@ def test_spikes_over_the_inputs(hip_ops, snnf_lib, N, H):
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and 0 < float(got[0][0].float().mean()) < 1
 
 
+@pytest.mark.parametrize("N,H", [(8, 32), (1, 12)])      # tiles, few pixels
+def test_inputs_right_behind_a_16bit_membrane_are_no_overlap(hip_ops, snnf_lib, N, H):
+    from triton_snn_fusion_amd import _lib
+    from triton_snn_fusion_amd.runtime import hip_convlif_backend as CB
+    g = gen(9396)
+    T, C, code = 4, 32, _lib.dtype_code(BF16)
+    n = N * C * H * H
+    x = torch.stack([spikes((N, C, H, H), 0.25, g) for _ in range(T)])
+    w, b = q(torch.randn(C, C, 3, 3, generator=g) * 0.2, BF16), q(torch.randn(C, generator=g) * 0.1, BF16)
+    packed = CB._packed_weight(dev(w, BF16), dev(b, BF16), BF16)
+    need = snnf_lib.snnf_conv_lif_scratch_bytes(T, N, C, H, H, code, C, 3, 3, 1, 1, 1, 1, code, 0)
+    both, room = torch.empty((T + 1) * n, device=DEV, dtype=BF16), torch.empty(need, dtype=torch.uint8, device=DEV)
+    v, xs = both[:n].view(N, C, H, H), both[n:].view(T, N, C, H, H)
+    xs.copy_(x)
+    sp = torch.empty(T, N, C, H, H, device=DEV, dtype=BF16)
+    _lib.check("ws", snnf_lib.snnf_conv_lif_ws(_lib.step_pointers(list(xs)), None, T, N, C, H, H, code, packed.data_ptr(), C, 3, 3, 1, 1, 1, 1, None, code, sp.data_ptr(),
+                                               int(sp.stride(0)), v.data_ptr(), *LIF, room.data_ptr(), need, _lib.current_stream(sp.device)))
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256 and N > 1:      # (the plan of few pixels names its frames either way)
+        assert CB.last_conv_plan().get("reads") == "frames"
+    check(sp, v, O.temporal_conv_lif(list(x), w, b, torch.tensor(0.0), (1, 1), (1, 1), (1, 1), 1, *LIF), v_dtype=BF16)
+
+
 def test_infinities_stay_in_their_windows(hip_ops, snnf_lib):
     """An infinity in the last channel of an image reaches its own windows and no neighbour's: pixels outside the image and channels beyond the last are zeros."""
     g = gen(9390)

@@ -787,7 +787,7 @@ int run_blocked_route(const void* const* xs, const void* const* residuals, int T
     const uintptr_t to_end = to + (static_cast<uintptr_t>(T - 1) * static_cast<uintptr_t>(out_step_stride) + neurons) * size;
     const bool apart = std::all_of(xs, xs + T, [&](const void* x) {
         const auto in = reinterpret_cast<uintptr_t>(x), in_end = in + static_cast<uintptr_t>(N) * Cin * H * W * size;
-        return aligned_to(x, size) && (in >= to_end || to >= in_end) && (v_out == nullptr || in >= v + neurons * 4 || v >= in_end);
+        return aligned_to(x, size) && (in >= to_end || to >= in_end) && (v_out == nullptr || in >= v + neurons * dtype_size(v_dtype) || v >= in_end);
     });
     if (taken.kept->steps_only && !(apart && dense_epilogue_neuron(make_lif_params(v_threshold, v_reset, tau)))) return SNNF_ERR_UNSUPPORTED;
     const void* inner[SNNF_MAX_T_PER_LAUNCH];
