@@ -489,14 +489,16 @@ bool fills_waves(const BlockedPlan& p, double weigh, int T, int Cout) {
 }
 
 // Whether the kernel reads the dense frames of a call itself (`p`) instead of a launch that brings them into C8 first (`copy`). That launch takes some 3 us and the time of the bytes it moves; without it
-// every tile assembles its halo from loads of two pixels of one channel, and `loads` of them for a compute unit take some 4.5 ns each, more from patches of short rows, and half as much again
-// where a wave has a tile of its own, all of whose stages then wait for them in turn; the longer a wave's matrix steps (`steps`, in hundreds), the later its staged vectors would have been missed.
-// Fitted to drawn layers whose frames come from memory, not from a cache: of 1263 in 16 bits this takes 733, at 1.195 in the mean (17 lose more than a twentieth, the worst 0.77); a line fitted to
-// frames in the caches took 948, 113 of which lost that much, down to 0.56, at 1.13. Of 766 in fp32, whose pairs take loads of 8 bytes and twice the rounding to two terms, 360, at 1.18 (5 lose
-// more than a twentieth, 0.90). us, copy / here, frames in the caches: T = 4 64 -> 64 at 32^2 x 8 14.6 / 11.5, 128 -> 128 at 20^2 x 7 16.0 / 12.1, 168 -> 56 1x1 at 36^2 x 4 17.0 / 9.8, 72 -> 104 at 27 x 35 x 5
+// every tile assembles its halo from loads of two pixels of one channel, `loads` of them for a compute unit. What they take goes with the lines that they touch: in long rows (up to 64 elements) a tile's
+// rows lie in lines of their own, which come from memory once if the frames are there and from a cache for every further tile of output channels; patches of short rows take more, 1x1 ones
+// of a few columns most, whose lines many tiles share, and a wave with a tile of its own waits for its stages in turn. The longer a wave's matrix steps (`steps`, in hundreds), the less of the copy's
+// time would have been seen. Fitted to drawn layers, both with frames from the caches, as the layer before leaves them, and from memory: of 1176 and 1229 in 16 bits this takes 793, at 1.25 in the mean
+// (7 lose more than a twentieth, the worst 0.86), and 815, at 1.18 (30, the worst 0.68); a line by loads and bytes alone took 892 (26, 0.71) and 937 (103, 0.56), at 1.22 and 1.14. fp32,
+// whose pairs take loads of 8 bytes and twice the rounding to two terms: of 672 and 766 332, at 1.23 (5 lose more than a twentieth), and 386, at 1.165 (15, the worst 0.77).
+// us, copy / here, T = 4, from the caches: 64 -> 64 at 32^2 x 8 14.6 / 11.5, 128 -> 128 at 28^2 x 16 36.1 / 34.0, at 20^2 x 7 16.0 / 12.1, 256 -> 256 at 14^2 x 16 30.5 / 27.7, 168 -> 56 1x1 at 36^2 x 4 17.0 / 9.8, 72 -> 104 at 27 x 35 x 5
 // with a residual, T = 6 28.4 / 25.0, 48 -> 18 1x1 at 9^2 x 9, T = 3 10.7 / 7.1, 88 -> 96 at 104^2 x 2 38.9 / 43.8, fp32 64 -> 64 at 32^2 x 8 16.1 / 14.7, 88 -> 88 at 20^2 x 9, T = 3 16.2 / 11.7, 256 -> 88 1x1 at
-// 8^2 x 16 with a residual 13.3 / 9.4, 128 -> 128 at 28^2 x 16 50.4 / 65.7; from memory: 488 -> 24 1x1 at 16 x 30 x 18, T = 8 64 / 114, 352 -> 24 at 76^2 x 3 with a residual 62 / 85, 400 -> 24 at
-// 27 x 79 x 2 25.4 / 33.0, fp32 424 -> 24 1x1 at 35^2 x 17, T = 5 90 / 117.
+// 8^2 x 16 with a residual 13.3 / 9.4, 128 -> 128 at 28^2 x 16 50.4 / 65.7; from memory: 128 -> 128 at 28^2 x 16 35.0 / 34.4, 488 -> 24 1x1 at 16 x 30 x 18, T = 8 64 / 114, 352 -> 24 at 76^2 x 3 with a residual 62 / 85,
+// 400 -> 24 at 27 x 79 x 2 25.4 / 33.0, fp32 424 -> 24 1x1 at 35^2 x 17, T = 5 90 / 117.
 // Halo rows of whole pairs can make the planner's choice another one. Where fewer waves then share a tile's K, or stages are shorter, the copy stays (7x7 stride 2 116 -> 72 at 34 x 27 x 25, T = 1, two waves for four
 // 25.7 / 40.1, 376 -> 32 at 40 x 54 x 12 with a residual 80 / 119; fp32 384 -> 19 1x1 at 69 x 33 x 5 with a residual, stages of four groups for eight, 37.2 / 48.8).
 // Strided layers of up to two channel groups are not among the measured and keep the copy, as do rows of one pixel, which have no pairs.
@@ -510,11 +512,10 @@ bool reads_steps(const BlockedPlan& p, const BlockedPlan& copy, int T, bool spli
     const double megabytes = static_cast<double>(g.N) * g.C8in * g.H * g.W * T * 16e-6;      // of one term
     const double shares = static_cast<double>(static_cast<int64_t>(g.n_items) << p.wk_log2) / (static_cast<double>(cus) * kSpkWaves);      // of tiles, to a wave
     const double steps = 0.01 * g.taps * g.C8in / 2.0 * p.tt * p.windows * (g.narrow ? 1 : 2) * std::max(std::ceil(shares) / (1 << p.wk_log2), 2.0 * shares / (1 << p.wk_log2));
-    // (1x1 in patches of a few columns: every line of the frames is read by many tiles, which the caches only hold for few bytes. 488 -> 24 at 16 x 30 x 18, T = 8, in columns of two 64 / 114 us, 336 -> 48 at 7 x 68 x 19,
-    // T = 8 61 / 93, 64 -> 23 at 54 x 97 x 5 24 / 28.)
-    if (!split && g.taps == 1 && g.PC <= 4 && megabytes > 8.0) return false;
-    if (split) return 3.0 + 0.176 * megabytes > loads * (0.0079 + (g.PC < 8 ? 0.0006 : 0.0) + (g.taps == 1 ? 0.0016 : 0.0)) + 0.33 * steps;
-    return 3.0 + 0.105 * megabytes > loads * (0.0045 + (p.wk_log2 == 0 ? 0.0028 : 0.0) + (g.PC < 8 ? 0.0007 : 0.0)) + 0.44 * steps;
+    if (split) return 3.0 + 0.25 * megabytes > loads * (0.0075 + (p.wk_log2 == 0 ? 0.0022 : 0.0) + (g.PC < 8 ? 0.0006 : 0.0) + (g.taps == 1 ? 0.0016 : 0.0)) + 0.3 * steps;
+    const bool strided = g.sh > 1 || g.sw > 1;
+    return 3.0 + megabytes * (0.74 - 0.37 / p.oc_tiles) > loads * (0.0031 + (p.wk_log2 == 0 ? 0.0031 : 0.0) + (g.PC < 8 ? 0.0019 : 0.0) + (g.taps == 1 && g.PC <= 4 ? 0.0073 : 0.0) -
+                                                                  (strided ? 0.0014 : 0.0) + 0.0075 * std::min(g.W, 64) / 64.0) + 0.37 * steps;
 }
 
 // The same for the kernel of few pixels: a workgroup's threads bring in its halo item by item, eight loads each, which takes what the copy does at some 2300 items of all timesteps.
