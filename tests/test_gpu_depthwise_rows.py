@@ -88,3 +88,24 @@ def test_outputs_over_what_is_read(hip_ops, snnf_lib, C, H, W, T, over):
         v.data_ptr(), *LIF, _lib.current_stream(sp.device)))
     assert torch.equal(sp.float().cpu(), ref[0]) and torch.equal(v.float().cpu(), q(ref[1], BF16))
     assert 0.0 < float(ref[0].mean()) < 1.0
+
+
+@pytest.mark.parametrize("N,C,H,W,T", [
+    (4, 125, 20, 11, 5),     # 20000 strips, the fewest of five steps that leave LDS
+    (2, 256, 64, 13, 8),     # 65536 strips: one workgroup to each compute unit
+    (1, 773, 53, 13, 6),     # more, and fewer than one and a half
+    (1, 771, 51, 23, 8),     # between one and a half and two
+    (1, 512, 33, 41, 7),     # long rows
+])
+def test_many_strips_of_odd_rows(hip_ops, snnf_lib, N, C, H, W, T):
+    from triton_snn_fusion_amd import _lib
+    g = gen(5300 + C + W + T)
+    w, b = torch.randint(-64, 65, (C, 1, 3, 3), generator=g) / 64.0, torch.randint(-16, 17, (C,), generator=g) / 64.0
+    x = torch.randint(-8, 9, (T, N, C, H, W), generator=g) / 4.0
+    ref = O.temporal_conv_lif(list(x), w, b, torch.tensor(0.0), (1, 1), (1, 1), (1, 1), C, *LIF)
+    xs, dw, db = dev(x, F16), dev(w, F16), dev(b, F16)
+    sp, v = torch.empty((T, N, C, H, W), dtype=F16, device=DEV), torch.empty((N, C, H, W), device=DEV)
+    _lib.check("dw", snnf_lib.snnf_dwconv3x3_lif(
+        _lib.step_pointers(list(xs)), None, T, N, C, H, W, 1, _lib.dtype_code(F16), dw.data_ptr(), db.data_ptr(), _lib.dtype_code(F16), None, _lib.dtype_code(F32),
+        sp.data_ptr(), int(sp.stride(0)), v.data_ptr(), *LIF, _lib.current_stream(sp.device)))
+    assert torch.equal(sp.float().cpu(), torch.as_tensor(ref[0])) and torch.equal(v.cpu(), ref[1])

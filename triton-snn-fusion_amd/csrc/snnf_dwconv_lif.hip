@@ -617,9 +617,11 @@ int launch_rows(const StepPtrs& xs, const StepPtrs& res, int has_res, int T, con
 
 // Which calls the kernel of any rows takes (see there). Odd rows start between dwords, where a 16-byte access takes longer than on even ones, and the time per step counts for more the more
 // there are; a residual makes the way through LDS the longer one. us, in LDS / here, tensors from memory: 387 channels at 73 x W x 3, W = 73, T = 1 40.3 / 21.8, 2 46.3 / 34.2, 3 52.3 / 46.2, 4 58.2 / 57.5,
-// 5 65.3 / 69.0, 6 72.8 / 81.0, 8 86.8 / 103.5, W = 74, T = 5 72.0 / 50.8. Of 300 drawn layers of odd rows: up to two steps 1.39 in the mean, the smallest 0.96; three and four, from 20 k and 32 k strips of
-// eight on, 1.15 (four lose up to a twentieth), from 10 k to 32 k 0.91 to 1.02; five and six in rows of 80 elements and more 1.0 to 1.3, of fewer 0.86 to 1.1, eight 0.73 to 1.0; with a residual
-// 1.04 to 1.9 at any number of steps, in rows of nine 0.88.
+// 5 65.3 / 69.0, 6 72.8 / 81.0, 8 86.8 / 103.5, W = 74, T = 5 72.0 / 50.8. From the caches this kernel gains more, so the lines lie where the
+// product of both gains is above one. 800 drawn layers of odd rows of three to twelve steps, LDS over here, from the caches / from memory, in the mean of those that the lines send here: T = 3 1.48 / 1.17,
+// 4 1.33 / 1.07, 5 1.28 / 1.02, 6 1.24 / 1.00, 7 1.17 / 0.97, 8 1.22 / 0.99 (the smallest 1.02 / 0.88), with a residual 1.26 to 1.5 / 1.2 to 1.4; of the others 1.00 to 1.10 / 0.88 to 1.00. From six steps on whole
+// rounds of a workgroup to each of the 256 compute units count: 8 steps, 65520 strips 1.47 / 1.09, 67200 0.91 / 0.82, 102816 1.39 / 1.19, 131040 1.38 / 1.17, 134904 0.90 / 0.85. Up to two steps 1.39 from
+// memory in the mean, the smallest 0.96.
 // Calls that write over what they read (a membrane in place, spikes over the residuals) stay in LDS, where every output has one owner.
 bool takes_rows(const StepPtrs& xs, const StepPtrs& res, int has_res, int T, const DwGeom& g, const void* v_init, int vsize, const void* spikes, int64_t spike_step_stride,
                 const void* v_out) {
@@ -638,7 +640,11 @@ bool takes_rows(const StepPtrs& xs, const StepPtrs& res, int has_res, int T, con
     if (g.W % 2 == 0 || T <= 2) return true;
     const int64_t strips = static_cast<int64_t>(g.planes) * g.H * ((g.W + 7) / 8);
     if (has_res) return strips >= 20000 && g.W >= (T <= 4 ? 11 : 21);
-    return strips >= (T == 3 ? 20000 : 32000) && g.W >= (T <= 4 ? 11 : 80) && T <= 6;
+    if (strips < (T <= 5 ? 20000 : 32000) || g.W < 11 || T > 8) return false;
+    constexpr int64_t kRound = 256 * kThreads;  // a workgroup to each compute unit
+    if (T == 3 || strips <= kRound) return true;
+    if (T >= 6 && g.W >= 13 && strips <= 2 * kRound && strips * 4 >= kRound * 6) return true;  // a second round that is half full
+    return T <= 7 && g.W >= (T <= 5 ? 15 : T == 6 ? 33 : 41);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
