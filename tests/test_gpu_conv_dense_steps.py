@@ -121,6 +121,28 @@ def test_layers_that_the_copy_is_faster_for(hip_ops, snnf_lib, Cin, Cout, H, W, 
     check(sp, v, ref, what=f"{Cin}->{Cout} {H}x{W} T={T}")
 
 
+@pytest.mark.parametrize("Cin,Cout,H,W,N,T,residual,dtype,route", [
+    (168, 104, 110, 58, 8, 1, True, BF16, None),      # no copy to fall back to: the dense kernel
+    (456, 86, 32, 83, 6, 2, False, F16, None),
+    (112, 24, 16, 57, 31, 4, False, BF16, "c8"),
+    (112, 24, 16, 57, 31, 4, False, F32, "c8"),
+])
+def test_large_frames_in_narrow_patches_of_1x1(hip_ops, snnf_lib, Cin, Cout, H, W, N, T, residual, dtype, route):
+    """Every tile of two or four columns would fetch whole lines, gone from the L2 caches before its neighbour's turn."""
+    from triton_snn_fusion_amd.runtime import hip_convlif_backend as CB
+    g = gen(9375 + Cin)
+    x, b = [spikes((N, Cin, H, W), 0.2, g) for _ in range(T)], torch.randint(-16, 17, (Cout,), generator=g) / 64.0
+    rs = [spikes((N, Cout, H, W), 0.2, g) for _ in range(T)] if residual else None
+    w = torch.randint(-64, 65, (Cout, Cin, 1, 1), generator=g) / 128.0      # (sums that are exact in any order)
+    sp, v = _run([dev(t, dtype) for t in x], [dev(t, dtype) for t in rs] if residual else None, dev(w, dtype), dev(b, dtype), torch.zeros((), device=DEV), 1, 0, LIF)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        plan = CB.last_conv_plan()
+        assert plan.get("reads") is None and plan.get("route") == route, plan
+    ref = O.temporal_conv_lif(x, w, b, torch.tensor(0.0), (1, 1), (0, 0), (1, 1), 1, *LIF, residuals=rs)
+    assert torch.equal(sp.float().cpu(), ref[0]) and 0.0 < float(ref[0].mean()) < 1.0
+    check(sp, v, ref, what=f"{Cin}->{Cout} {H}x{W} T={T}")
+
+
 @pytest.mark.parametrize("Cin,Cout,H,k,s,N,T", [
     (27, 328, 15, 7, 2, 5, 4),       # whose frames would take two windows where the copy takes one
     (72, 104, 27, 3, 1, 2, 6),       # two of each

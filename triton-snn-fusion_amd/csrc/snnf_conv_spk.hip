@@ -501,6 +501,10 @@ bool fills_waves(const BlockedPlan& p, double weigh, int T, int Cout) {
 // 400 -> 24 at 27 x 79 x 2 25.4 / 33.0, fp32 424 -> 24 1x1 at 35^2 x 17, T = 5 90 / 117.
 // Halo rows of whole pairs can make the planner's choice another one. Where fewer waves then share a tile's K, or stages are shorter, the copy stays (7x7 stride 2 116 -> 72 at 34 x 27 x 25, T = 1, two waves for four
 // 25.7 / 40.1, 376 -> 32 at 40 x 54 x 12 with a residual 80 / 119; fp32 384 -> 19 1x1 at 69 x 33 x 5 with a residual, stages of four groups for eight, 37.2 / 48.8).
+// 1x1 layers of many channels in patches of up to four columns of long rows touch a line of every channel and row for a pair or two of it. Where the frames are larger than the L2 caches hold beside each
+// other, the line is gone before the next tile asks for it, and the copy stays, or the dense kernel where the route has no copy (of 573 drawn 1x1 layers that go past the lines below ten are
+// stopped by this one, 0.80 in the mean: us, copy or dense / here, 168 -> 104 at 110 x 58 x 8 with a residual, T = 1 35.8 / 95.1, 456 -> 86 at 32 x 83 x 6, T = 2 31.3 / 54.7, 160 -> 29 at 67 x 52 x 18, T = 1 20.8 / 33.2,
+// 112 -> 24 at 16 x 57 x 31, T = 4 34.0 / 43.1, fp32 432 -> 30 at 80 x 52 x 18, T = 1 64 / 91; 7.5 MB, 306 -> 60 at 7 x 35 x 25, T = 2 16.4 / 10.7).
 // Strided layers of up to two channel groups are not among the measured and keep the copy, as do rows of one pixel, which have no pairs.
 bool reads_steps(const BlockedPlan& p, const BlockedPlan& copy, int T, bool split) {
     const SpkGeom& g = p.g;
@@ -512,6 +516,7 @@ bool reads_steps(const BlockedPlan& p, const BlockedPlan& copy, int T, bool spli
     const double megabytes = static_cast<double>(g.N) * g.C8in * g.H * g.W * T * 16e-6;      // of one term
     const double shares = static_cast<double>(static_cast<int64_t>(g.n_items) << p.wk_log2) / (static_cast<double>(cus) * kSpkWaves);      // of tiles, to a wave
     const double steps = 0.01 * g.taps * g.C8in / 2.0 * p.tt * p.windows * (g.narrow ? 1 : 2) * std::max(std::ceil(shares) / (1 << p.wk_log2), 2.0 * shares / (1 << p.wk_log2));
+    if (g.taps == 1 && g.PC <= 4 && g.W >= 20 && g.C8in >= 10 && megabytes * (split ? 2.0 : 1.0) > 8.0) return false;
     if (split) return 3.0 + 0.25 * megabytes > loads * (0.0075 + (p.wk_log2 == 0 ? 0.0022 : 0.0) + (g.PC < 8 ? 0.0006 : 0.0) + (g.taps == 1 ? 0.0016 : 0.0)) + 0.3 * steps;
     const bool strided = g.sh > 1 || g.sw > 1;
     return 3.0 + megabytes * (0.74 - 0.37 / p.oc_tiles) > loads * (0.0031 + (p.wk_log2 == 0 ? 0.0031 : 0.0) + (g.PC < 8 ? 0.0019 : 0.0) + (g.taps == 1 && g.PC <= 4 ? 0.0073 : 0.0) -
