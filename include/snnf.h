@@ -147,8 +147,9 @@ int snnf_pwconv_lif_rowbits(const void* const* xs_bits, int T, int N, int Cin, i
  *   out_sum : [N, K] x_dtype         v_out : [N, C, H, W] v_dtype
  *   workspace : at least snnf_lif_pool_linear_workspace_bytes(N, C) bytes of device memory, 16-byte aligned;
  *               it holds per-(n, c) spike counts between the two launches and needs no initialisation.
- * Tails as small as those at the end of a network (T * C * H * W of one sample at most 32 Ki, C % 8 == 0 and at most 2048,
- * C * H * W % 8 == 0, 16-byte aligned operands) run as ONE launch: a workgroup owns a sample and a range of classes, counts the
+ * Tails as small as those at the end of a network (C * H * W of one sample at most 8192 and T times that at most 32 Ki, C % 8 == 0
+ * and at most 2048, C * H * W % 8 == 0, 16-byte aligned operands, and classes that the workgroups of the batch go over in a few
+ * rounds: 64 samples of 1000 classes are too many) run as ONE launch: a workgroup owns a sample and a range of classes, counts the
  * sample's spikes per channel in LDS and multiplies its weight rows with them; the workspace is then not touched.
  * snnf_lif_pool_linear_launches() says which of the two forms a shape takes (1 or 2; 0 for invalid extents), assuming
  * aligned operands and a v_out that is not v_init (in place, a sample whose classes take several workgroups takes two launches).
@@ -245,12 +246,14 @@ int snnf_conv_lif(const void* const* xs, const void* const* residuals, int T,
                   float v_threshold, float v_reset, float tau, void* stream);
 
 /*
- * snnf_conv_lif with a caller-owned workspace, which lets the library bring the inputs into the channel-blocked layout
- * first and run the kernel of that layout on them. The reference has no counterpart (its Triton kernel reads NCHW,
+ * snnf_conv_lif with a caller-owned workspace, which lets the library run the kernel of the channel-blocked layout: on inputs
+ * that it brings into that layout first, or on the dense ones as they are where that is faster and the call writes nothing
+ * where they lie (the order of the additions can be another one then). The reference has no counterpart (its Triton kernel reads NCHW,
  * kernels/benchmark_conv_lif_temporal_general.py:629-676). Results are those of snnf_conv_lif up to the order of the fp32
  * additions.
  *   snnf_conv_lif_scratch_bytes : bytes with which this call takes that route (0: the call is snnf_conv_lif). A call whose
- *               timesteps all read one frame never takes it and needs none.
+ *               timesteps all read one frame never takes it and needs none. 16 bytes a timestep ask for a route that
+ *               always reads the dense inputs.
  *   snnf_conv_lif_workspace_bytes : the older question, which knows 16-bit activations beside an fp32 membrane only and answers 0 for every other
  *               call (that call then runs as snnf_conv_lif). Ask snnf_conv_lif_scratch_bytes instead.
  *   workspace : NULL (then this is snnf_conv_lif), or device memory, 16-byte aligned, contents undefined before and after.

@@ -135,7 +135,7 @@ __global__ __launch_bounds__(kColWaves * 64, 2) void conv_columns_kernel(const S
             if (c < left) (to + c * g.P)[o_at] = from_float<XT>(sum[c]);
     };
     if constexpr (SHARE) {
-        // [wave][fragment][quad][lane] sums; the wave f finishes fragment f, adding the parts in the order of K.
+        // [wave][fragment][quad][lane] sums; wave w finishes quad w of every fragment, adding the four parts in the order of K.
         __shared__ __align__(16) float parts[kColWaves * NF * 4 * 64 * 4];
 #pragma unroll
         for (int f = 0; f < NF; ++f)

@@ -193,7 +193,8 @@ bool takes_blocked_route(int T, int N, int Cin, int H, int W, int x_dtype, int C
         case DenseFamily::kTimeOuter: return !pointwise || static_cast<int64_t>(T) * N * (Cin + Cout) * plane <= (1 << 25);
         case DenseFamily::kPointwise: return plane % 64 != 0 || (Cout % 32 != 0 && outs <= (1 << 22));
         case DenseFamily::kMatrixMasked:
-            // One or two timesteps of a 1x1 layer of stride 1 move where the kernel reads the frames itself: 17 layers, 1.82 in the mean, one loses 10 % (us, dense / here, 360 -> 24 at 13 x 48 x 17, T = 2
+            // One or two timesteps of a 1x1 layer of stride 1 move where the kernel reads the frames itself: 410 drawn layers, 1.48 in the mean with frames from the caches, 1.35 from
+            // memory, 7 and 13 lose more than a twentieth, the worst 0.88 and 0.83 (us, dense / here, 360 -> 24 at 13 x 48 x 17, T = 2
             // 26.2 / 8.1, 136 -> 16 at 68 x 11 x 20, T = 1 13.1 / 7.2, 144 -> 205 at 12 x 54 x 28, T = 1 28.7 / 20.6, 216 -> 88 at 52^2 x 28, T = 2 55.4 / 61.8; of five that
             // keep the copy 464 -> 164 at 34 x 33 x 9, T = 1 21.3 / 34.1).
             if (pointwise && T <= 2 && outs > (1 << 17)) weigh = -1.0;

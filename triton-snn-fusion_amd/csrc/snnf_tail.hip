@@ -387,7 +387,8 @@ __global__ __launch_bounds__(kThreads) void count_linear_mm_kernel(const int* __
 constexpr int kOneMaxC = 2048;                    // channels of a sample whose counters fit the workgroup's LDS array
 constexpr int kOneMaxNeurons = 1024 * kVec;       // of a sample: one pass
 constexpr int64_t kOneMaxSampleWork = 32 * 1024;  // T * C * HW of one sample, at most: the pooling kernel of the two-launch path spreads more over many workgroups
-                                                  // (512 channels of 4x4 x 16, T = 8, 100 classes, one launch / two 8.3 / 8.2 us, 1000 classes 10.6 / 8.3)
+                                                  // (512 channels of 4x4 x 16, T = 8, 100 classes, one launch / two 8.3 / 8.2 us, 1000 classes 10.6 / 8.3;
+                                                  // 7x7 x 16, T = 4, 1000 classes, four passes in 4, 8, 16 and 32 class ranges 17.0, 14.9, 13.2 and 18.5 / 7.9, 10 classes 10.5 / 6.6)
 
 // out[n, k] = (Wt[k, :] . counts / HW + steps * bias[k]) * out_scale for the classes of this workgroup's range, from the
 // per-channel spike counts of sample n in LDS: kRowsPerWave rows per wave and pass, a lane takes 8 channels at a time.
